@@ -208,6 +208,16 @@ GS355_API int gs355_run(const gs355_frame *frame, const gs355_gaussians *g, void
 GS355_API int gs355_render(const gs355_frame *frame, const gs355_gaussians *g, void *workspace, size_t workspace_bytes,
                  int64_t n_cap, const gs355_outputs *out, void *stream);
 
+/* gs355_run over the vanilla model's stored parameters instead of their activated values
+ * (GaussianModel.forward, benchmarks/nerf/origin_gs/gs_model.py:112-228): g->shs is features_dc [P,1,3], features_rest
+ * the other coefficients [P,M-1,3] (NULL when frame->sh_coeffs = M = 1; M <= 16), g->scales holds logarithms,
+ * g->rotations unnormalised quaternions and g->opacities logits.  exp, q / max(|q|, 1e-12) and the logistic function
+ * are evaluated per Gaussian while it is preprocessed, with the rounding of the framework's elementwise operations:
+ * the frame is the one that the activated tensors give.  colors_precomp, cov3D_precomp and P_device are refused. */
+GS355_API int gs355_run_parameters(const gs355_frame *frame, const gs355_gaussians *g, const float *features_rest,
+                                   void *workspace, size_t workspace_bytes, int64_t n_cap, const gs355_outputs *out,
+                                   uint32_t stage_mask, void *stream);
+
 /* GaussianRasterizer.visible_filter: radii only (cull, covariance, radius,
  * non-empty tile rectangle); needs no workspace.  shs/colors/opacities of
  * `g` are ignored and may be NULL. */
@@ -301,6 +311,15 @@ GS355_API int gs355_backward_scratch_bytes(int32_t P, int64_t n_cap, size_t *byt
 GS355_API int gs355_render_backward(const gs355_frame *frame, const gs355_gaussians *g, const void *workspace,
                                     size_t workspace_bytes, int64_t n_cap, const gs355_backward_inputs *in,
                                     void *scratch, size_t scratch_bytes, const gs355_gradients *grads, void *stream);
+
+/* Backward pass of a frame rendered by gs355_run_parameters: gradients with respect to the stored parameters, the
+ * activations' derivatives included.  grads->shs receives that of features_dc [P,1,3], dL_dfeatures_rest (NULL = not
+ * wanted) that of features_rest; scales, rotations and opacities those of the logarithms, quaternions and logits. */
+GS355_API int gs355_render_parameters_backward(const gs355_frame *frame, const gs355_gaussians *g,
+                                               const float *features_rest, const void *workspace,
+                                               size_t workspace_bytes, int64_t n_cap, const gs355_backward_inputs *in,
+                                               void *scratch, size_t scratch_bytes, const gs355_gradients *grads,
+                                               float *dL_dfeatures_rest, void *stream);
 
 /* ---------------------------------------------------------------------------
  * Anchor decode for Scaffold-GS / Octree-GS: replaces AnchorDecoder.forward

@@ -29,7 +29,8 @@ DECODE_COUNT, DECODE_EMIT, DECODE_ALL = 1, 2, 3
 EXPORTS = ("gs355_version", "gs355_last_error", "gs355_workspace_layout", "gs355_run", "gs355_render",
            "gs355_visible_filter", "gs355_anchor_filter", "gs355_decode_scratch_bytes", "gs355_decode_count",
            "gs355_decode_count_static", "gs355_decode_emit", "gs355_decode_workspace_bytes", "gs355_decode",
-           "gs355_backward_scratch_bytes", "gs355_render_backward", "gs355_gather_scratch_bytes", "gs355_gather_rows")
+           "gs355_backward_scratch_bytes", "gs355_render_backward", "gs355_gather_scratch_bytes", "gs355_gather_rows",
+           "gs355_run_parameters", "gs355_render_parameters_backward")
 GATHER_MAX_ARRAYS, GATHER_MAX_ROW_BYTES = 8, 4096
 
 
@@ -221,6 +222,13 @@ def load() -> C.CDLL:
                                           C.POINTER(BackwardInputs), C.c_void_p, C.c_size_t, C.POINTER(Gradients),
                                           C.c_void_p]
     lib.gs355_render_backward.restype = C.c_int
+    lib.gs355_run_parameters.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_void_p, C.c_void_p, C.c_size_t,
+                                         C.c_int64, C.POINTER(Outputs), C.c_uint32, C.c_void_p]
+    lib.gs355_run_parameters.restype = C.c_int
+    lib.gs355_render_parameters_backward.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_void_p, C.c_void_p,
+                                                     C.c_size_t, C.c_int64, C.POINTER(BackwardInputs), C.c_void_p,
+                                                     C.c_size_t, C.POINTER(Gradients), C.c_void_p, C.c_void_p]
+    lib.gs355_render_parameters_backward.restype = C.c_int
     lib.gs355_gather_scratch_bytes.argtypes = [C.c_int32, C.POINTER(C.c_size_t)]
     lib.gs355_gather_scratch_bytes.restype = C.c_int
     lib.gs355_gather_rows.argtypes = [C.c_int32, C.c_void_p, C.c_int32, C.POINTER(GatherArray), C.c_void_p, C.c_void_p,

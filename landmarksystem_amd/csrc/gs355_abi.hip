@@ -149,6 +149,17 @@ int check_colour_inputs(const gs355_frame* f, const gs355_gaussians* g)
     return GS355_OK;
 }
 
+// (after check_geometry_inputs and check_colour_inputs)
+int check_parameters(const gs355_frame* f, const gs355_gaussians* g, const float* rest)
+{
+    if (g->P_device) return set_error(GS355_EINVAL, "stored parameters do not combine with a device-side Gaussian count");
+    if (g->P == 0) return GS355_OK;
+    if (!g->shs || !g->scales) return set_error(GS355_EINVAL, "stored parameters are SH coefficients, scales and rotations");
+    if (f->sh_coeffs > 16) return set_error(GS355_EINVAL, "stored parameters hold at most 16 SH coefficients (got %d)", f->sh_coeffs);
+    if (f->sh_coeffs > 1 && !rest) return set_error(GS355_EINVAL, "features_rest is NULL");
+    return GS355_OK;
+}
+
 FrameArgs make_args(const gs355_frame* f)
 {
     FrameArgs a;
@@ -188,8 +199,8 @@ int gs355_workspace_layout(int32_t P, int64_t n_cap, int32_t width, int32_t heig
     return make_layout(P, n_cap, width, height, out);
 }
 
-int gs355_run(const gs355_frame* frame, const gs355_gaussians* g, void* workspace, size_t workspace_bytes,
-              int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
+static int run_stages(const gs355_frame* frame, const gs355_gaussians* g, const ParameterArgs* par, void* workspace,
+                      size_t workspace_bytes, int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
 {
     int rc;
     if ((stage_mask & ~kKnownStages) != 0 || (stage_mask & ~kStageModifiers) == 0 ||
@@ -198,6 +209,7 @@ int gs355_run(const gs355_frame* frame, const gs355_gaussians* g, void* workspac
     if ((rc = check_frame(frame, true))) return rc;
     if ((rc = check_geometry_inputs(g))) return rc;
     if ((rc = check_colour_inputs(frame, g))) return rc;
+    if (par && (rc = check_parameters(frame, g, par->rest))) return rc;
     if (!out) return set_error(GS355_EINVAL, "outputs is NULL");
     if ((stage_mask & GS355_STAGE_PREPROCESS) && g->P > 0 && !out->radii)
         return set_error(GS355_EINVAL, "outputs.radii is NULL");
@@ -241,7 +253,7 @@ int gs355_run(const gs355_frame* frame, const gs355_gaussians* g, void* workspac
     const uint32_t cap = (uint32_t)n_cap;
 
     if (stage_mask & GS355_STAGE_PREPROCESS)
-        if ((rc = launch_preprocess(fa, *g, false, records, touched, rects, depth_bits, out->radii, s))) return rc;
+        if ((rc = launch_preprocess(fa, *g, par, false, records, touched, rects, depth_bits, out->radii, s))) return rc;
     if (stage_mask & GS355_STAGE_SCAN)
         if ((rc = launch_scan_offsets(touched, out->radii, g->P, g->P_device, offsets, scan_tmp, header,
                                       static_cast<gs355_header*>(out->header_copy), cap, s)))
@@ -287,6 +299,20 @@ int gs355_run(const gs355_frame* frame, const gs355_gaussians* g, void* workspac
     return GS355_OK;
 }
 
+int gs355_run(const gs355_frame* frame, const gs355_gaussians* g, void* workspace, size_t workspace_bytes,
+              int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
+{
+    return run_stages(frame, g, nullptr, workspace, workspace_bytes, n_cap, out, stage_mask, stream);
+}
+
+int gs355_run_parameters(const gs355_frame* frame, const gs355_gaussians* g, const float* features_rest, void* workspace,
+                         size_t workspace_bytes, int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
+{
+    ParameterArgs par;
+    par.rest = features_rest;
+    return run_stages(frame, g, &par, workspace, workspace_bytes, n_cap, out, stage_mask, stream);
+}
+
 int gs355_render(const gs355_frame* frame, const gs355_gaussians* g, void* workspace, size_t workspace_bytes,
                  int64_t n_cap, const gs355_outputs* out, void* stream)
 {
@@ -301,7 +327,7 @@ int gs355_visible_filter(const gs355_frame* frame, const gs355_gaussians* g, int
     if (g->P > 0 && !radii) return set_error(GS355_EINVAL, "radii is NULL");
     if (g->P_device) return set_error(GS355_EINVAL, "visible_filter does not take a device-side Gaussian count");
     const FrameArgs fa = make_args(frame);
-    return launch_preprocess(fa, *g, true, nullptr, nullptr, nullptr, nullptr, radii, static_cast<hipStream_t>(stream));
+    return launch_preprocess(fa, *g, nullptr, true, nullptr, nullptr, nullptr, nullptr, radii, static_cast<hipStream_t>(stream));
 }
 
 namespace {
@@ -332,14 +358,15 @@ int gs355_backward_scratch_bytes(int32_t P, int64_t n_cap, size_t* bytes)
     return GS355_OK;
 }
 
-int gs355_render_backward(const gs355_frame* frame, const gs355_gaussians* g, const void* workspace,
-                          size_t workspace_bytes, int64_t n_cap, const gs355_backward_inputs* in, void* scratch,
-                          size_t scratch_bytes, const gs355_gradients* grads, void* stream)
+static int render_backward(const gs355_frame* frame, const gs355_gaussians* g, const ParameterArgs* par,
+                           const void* workspace, size_t workspace_bytes, int64_t n_cap, const gs355_backward_inputs* in,
+                           void* scratch, size_t scratch_bytes, const gs355_gradients* grads, void* stream)
 {
     int rc;
     if ((rc = check_frame(frame, true))) return rc;
     if ((rc = check_geometry_inputs(g))) return rc;
     if ((rc = check_colour_inputs(frame, g))) return rc;
+    if (par && (rc = check_parameters(frame, g, par->rest))) return rc;
     if (g->P_device) return set_error(GS355_EINVAL, "the backward pass does not take a device-side Gaussian count");
     if (!in) return set_error(GS355_EINVAL, "backward inputs is NULL");
     if (!grads) return set_error(GS355_EINVAL, "gradients is NULL");
@@ -375,7 +402,25 @@ int gs355_render_backward(const gs355_frame* frame, const gs355_gaussians* g, co
                                   reinterpret_cast<const uint64_t*>(ws + L.rects), *in,
                                   reinterpret_cast<uint32_t*>(sc + B.first_key),
                                   reinterpret_cast<uint32_t*>(sc + B.scan_tmp),
-                                  reinterpret_cast<float*>(sc + B.key_grads), *grads, static_cast<hipStream_t>(stream));
+                                  reinterpret_cast<float*>(sc + B.key_grads), *grads, par, static_cast<hipStream_t>(stream));
+}
+
+int gs355_render_backward(const gs355_frame* frame, const gs355_gaussians* g, const void* workspace,
+                          size_t workspace_bytes, int64_t n_cap, const gs355_backward_inputs* in, void* scratch,
+                          size_t scratch_bytes, const gs355_gradients* grads, void* stream)
+{
+    return render_backward(frame, g, nullptr, workspace, workspace_bytes, n_cap, in, scratch, scratch_bytes, grads, stream);
+}
+
+int gs355_render_parameters_backward(const gs355_frame* frame, const gs355_gaussians* g, const float* features_rest,
+                                     const void* workspace, size_t workspace_bytes, int64_t n_cap,
+                                     const gs355_backward_inputs* in, void* scratch, size_t scratch_bytes,
+                                     const gs355_gradients* grads, float* dL_dfeatures_rest, void* stream)
+{
+    ParameterArgs par;
+    par.rest = features_rest;
+    par.d_rest = dL_dfeatures_rest;
+    return render_backward(frame, g, &par, workspace, workspace_bytes, n_cap, in, scratch, scratch_bytes, grads, stream);
 }
 
 int gs355_anchor_filter(const gs355_frame* frame, const gs355_gaussians* anchors, int32_t scale_stride,

@@ -287,15 +287,18 @@ __device__ __forceinline__ void sh_basis_grad(int deg, float x, float y, float z
 constexpr int kShStride = 52;  // floats per Gaussian in the SH staging area (16-B reads of 64 lanes on distinct banks)
 
 // kMode 0: SH blocks (if any) are read and written by their own lanes.  1 and 2: 16-coefficient blocks, 16-byte
-// aligned, staged through LDS; 2 also fetches the coefficients (needed for degree > 0 only).
-template <int kMode>
+// aligned, staged through LDS; 2 also fetches the coefficients (needed for degree > 0 only).  kStored: g holds the
+// vanilla model's stored parameters, and the gradients are theirs (activations' derivatives included); the rows of the
+// SH coefficients behind the first are then staged back to back, 3 (M - 1) floats each, as they lie in memory: a
+// wavefront's 64 rows start on a 256-B boundary whatever their length.
+template <int kMode, bool kStored>
 __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, gs355_gaussians g,
                                                                   const int32_t* __restrict__ radii,
                                                                   const float* __restrict__ records,
                                                                   const uint32_t* __restrict__ tiles_touched,
                                                                   const uint32_t* __restrict__ first_key,
                                                                   const float* __restrict__ key_grads,
-                                                                  gs355_gradients out)
+                                                                  gs355_gradients out, ParameterArgs par)
 {
     // Full 16-coefficient SH blocks travel through LDS: each wavefront moves the 12 KB of its 64 Gaussians'
     // coefficients (in) and coefficient gradients (out) with coalesced 16-B accesses; a lane works on its own row.
@@ -310,8 +313,9 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
     const size_t wave_first = (size_t)blockIdx.x * blockDim.x + (size_t)wave * 64;
     const int count = (int)min((size_t)64, (size_t)g.P > wave_first ? (size_t)g.P - wave_first : (size_t)0);
     constexpr bool staged = kMode != 0, fetch_sh = kMode == 2;
+    const int rest_row = 3 * (M - 1);  // floats per Gaussian in par.rest
     float4* __restrict__ mine = s_sh + (staged ? wave * 64 * (kShStride / 4) : 0);
-    float* __restrict__ my_row = reinterpret_cast<float*>(mine) + (staged ? lane * kShStride : 0);
+    float* __restrict__ my_row = reinterpret_cast<float*>(mine) + (staged ? lane * (kStored ? rest_row : kShStride) : 0);
 
     float dmean[3] = {0.f, 0.f, 0.f}, d2[3] = {0.f, 0.f, 0.f}, dscale[3] = {0.f, 0.f, 0.f};
     float drot[4] = {0.f, 0.f, 0.f, 0.f}, dcov[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, dcol[3] = {0.f, 0.f, 0.f};
@@ -372,14 +376,21 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
         // the kernel waits for memory, so the chain costs nothing in double and loses nothing.
         typedef double real;
         real S[6], s[3] = {0., 0., 0.}, q[4] = {0., 0., 0., 0.}, R[3][3] = {};
-        if (g.cov3D_precomp) {
+        float stored_q[4], norm = 1.f;
+        if (!kStored && g.cov3D_precomp) {
 #pragma unroll
             for (int k = 0; k < 6; ++k) S[k] = g.cov3D_precomp[6 * si + k];
         } else {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) s[k] = (real)f.scale_modifier * (real)g.scales[3 * si + k];
+            for (int k = 0; k < 3; ++k) {
+                const float v = g.scales[3 * si + k];
+                s[k] = (real)f.scale_modifier * (real)(kStored ? expf(v) : v);
+            }
 #pragma unroll
-            for (int k = 0; k < 4; ++k) q[k] = g.rotations[4 * si + k];
+            for (int k = 0; k < 4; ++k) stored_q[k] = g.rotations[4 * si + k];
+            if (kStored) norm = quaternion_norm(stored_q);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = kStored ? stored_q[k] / norm : stored_q[k];
             const real r = q[0], qx = q[1], qy = q[2], qz = q[3];
             R[0][0] = 1. - 2. * (qy * qy + qz * qz); R[0][1] = 2. * (qx * qy - r * qz); R[0][2] = 2. * (qx * qz + r * qy);
             R[1][0] = 2. * (qx * qy + r * qz); R[1][1] = 1. - 2. * (qx * qx + qz * qz); R[1][2] = 2. * (qy * qz - r * qx);
@@ -460,7 +471,7 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
         for (int k = 0; k < 3; ++k)
             dmean[k] += (float)(Vd[3 * k] * d_pvx + Vd[3 * k + 1] * d_pvy + Vd[3 * k + 2] * d_pvz);
 
-        if (g.cov3D_precomp) {
+        if (!kStored && g.cov3D_precomp) {
             dcov[0] = (float)dS[0][0]; dcov[1] = (float)(2. * dS[0][1]); dcov[2] = (float)(2. * dS[0][2]);
             dcov[3] = (float)dS[1][1]; dcov[4] = (float)(2. * dS[1][2]); dcov[5] = (float)dS[2][2];
         } else {
@@ -475,7 +486,7 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
                     ds += dL * R[a][k];
                     dR[a][k] = dL * s[k];
                 }
-                dscale[k] = (float)(ds * (real)f.scale_modifier);
+                dscale[k] = (float)(ds * (kStored ? s[k] : (real)f.scale_modifier));  // (d s / d log s = s)
             }
             const real r = q[0], qx = q[1], qy = q[2], qz = q[3];
             drot[0] = (float)(2. * (-qz * dR[0][1] + qy * dR[0][2] + qz * dR[1][0] - qx * dR[1][2] - qy * dR[2][0] + qx * dR[2][1]));
@@ -485,6 +496,17 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
                                     r * dR[2][0] + qz * dR[2][1] - 2. * qy * dR[2][2]));
             drot[3] = (float)(2. * (-2. * qz * dR[0][0] - r * dR[0][1] + qx * dR[0][2] + r * dR[1][0] - 2. * qz * dR[1][1] +
                                     qy * dR[1][2] + qx * dR[2][0] + qy * dR[2][1]));
+            if (kStored) {  // through q / max(|q|, 1e-12): the part along q drops out, unless the norm is the constant
+                const float along = norm > 1e-12f ? (float)(drot[0] * r + drot[1] * qx + drot[2] * qy + drot[3] * qz) : 0.f;
+                drot[0] = (drot[0] - (float)r * along) / norm;
+                drot[1] = (drot[1] - (float)qx * along) / norm;
+                drot[2] = (drot[2] - (float)qy * along) / norm;
+                drot[3] = (drot[3] - (float)qz * along) / norm;
+            }
+        }
+        if (kStored) {
+            const float o = logistic(g.opacities[si]);
+            dop = dop * ((1.0f - o) * o);
         }
 
         // ---- colour: view direction, SH basis and its gradient ----
@@ -506,7 +528,23 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
 
     // ---- SH coefficients: their part of the mean's gradient (through the view direction), and their own ----
     if (g.shs) {
-        if (fetch_sh) {
+        // kStored: the wavefront's rows as one run of float4, and the up to three floats behind the last whole one
+        const int run4 = kStored ? count * rest_row / 4 : 0, run_tail = kStored ? count * rest_row % 4 : 0;
+        const size_t run_first = wave_first * (size_t)rest_row;
+        if (fetch_sh && kStored) {
+            float4 sh_in[12];
+            const float4* __restrict__ src = reinterpret_cast<const float4*>(par.rest + run_first);
+            if (run4 > 0) {  // (uniform over the wavefront)
+#pragma unroll
+                for (int it = 0; it < 12; ++it)
+                    if (it * 64 < run4) sh_in[it] = src[min(it * 64 + lane, run4 - 1)];  // (uniform)
+#pragma unroll
+                for (int it = 0; it < 12; ++it)
+                    if (it * 64 + lane < run4) mine[it * 64 + lane] = sh_in[it];
+            }
+            if (lane < run_tail) reinterpret_cast<float*>(mine)[4 * run4 + lane] = par.rest[run_first + 4 * run4 + lane];
+            wave_lds_sync();
+        } else if (fetch_sh) {
             // coefficients of the wavefront's Gaussians: all loads in flight together, then into the rows (slots
             // past the last Gaussian re-read it)
             float4 sh_in[12];
@@ -524,12 +562,14 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
             wave_lds_sync();
         }
         if (alive && f.sh_degree > 0) {
-            const float* __restrict__ sh = staged ? my_row : g.shs + si * M * 3;
+            constexpr int kSkip = kStored ? 3 : 0;  // (the first coefficient is stored apart)
+            const float* __restrict__ sh = staged ? my_row : kStored ? par.rest + si * rest_row : g.shs + si * M * 3;
             float dn[3] = {0.f, 0.f, 0.f};
 #pragma unroll
             for (int k = 1; k < 16; ++k) {
                 if (k < K) {
-                    const float t = gcol[0] * sh[3 * k] + gcol[1] * sh[3 * k + 1] + gcol[2] * sh[3 * k + 2];
+                    const float* __restrict__ c = sh + (3 * k - kSkip);
+                    const float t = gcol[0] * c[0] + gcol[1] * c[1] + gcol[2] * c[2];
                     dn[0] += t * bx[k];
                     dn[1] += t * by[k];
                     dn[2] += t * bz[k];
@@ -540,7 +580,37 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
             dmean[1] += (dn[1] - ny * dot) * inv_len;
             dmean[2] += (dn[2] - nz * dot) * inv_len;
         }
-        if (out.shs) {
+        if (kStored) {
+            if (out.shs && valid)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) out.shs[3 * si + c] = alive ? b[0] * gcol[c] : 0.0f;
+            if (par.d_rest && staged) {
+                wave_lds_sync();  // rows were read above
+#pragma unroll
+                for (int k = 1; k < 16; ++k) {
+                    if (k < M) {
+                        const float bk = (alive && k < K) ? b[k] : 0.0f;
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) my_row[3 * (k - 1) + c] = bk * gcol[c];
+                    }
+                }
+                wave_lds_sync();
+                float4* __restrict__ dst = reinterpret_cast<float4*>(par.d_rest + run_first);
+#pragma unroll
+                for (int it = 0; it < 12; ++it)
+                    if (it * 64 + lane < run4) dst[it * 64 + lane] = mine[it * 64 + lane];
+                if (lane < run_tail) par.d_rest[run_first + 4 * run4 + lane] = reinterpret_cast<float*>(mine)[4 * run4 + lane];
+            } else if (par.d_rest && valid) {
+#pragma unroll
+                for (int k = 1; k < 16; ++k) {
+                    if (k < M) {
+                        const float bk = (alive && k < K) ? b[k] : 0.0f;
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) par.d_rest[si * rest_row + 3 * (k - 1) + c] = bk * gcol[c];
+                    }
+                }
+            }
+        } else if (out.shs) {
             if (staged) {
                 wave_lds_sync();  // rows were read above
 #pragma unroll
@@ -601,7 +671,7 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
                            const uint32_t* ranges, const uint32_t* values, const float* records,
                            const uint32_t* tiles_touched, const uint64_t* rects, const gs355_backward_inputs& in,
                            uint32_t* first_key, uint32_t* scan_tmp, float* key_grads, const gs355_gradients& out,
-                           hipStream_t s)
+                           const ParameterArgs* par, hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
     int rc = launch_exclusive_scan(tiles_touched, first_key, (size_t)g.P, scan_tmp, s);
@@ -614,15 +684,23 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     const bool staged = g.shs != nullptr && f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(g.shs) & 15u) == 0 &&
                         (out.shs == nullptr || (reinterpret_cast<uintptr_t>(out.shs) & 15u) == 0);
     const dim3 grid((g.P + 255) / 256), block(256);
-    if (!staged)
-        hipLaunchKernelGGL(preprocess_backward_kernel<0>, grid, block, 0, s, f, g, in.radii, records, tiles_touched,
-                           first_key, key_grads, out);
-    else if (f.sh_degree == 0)
-        hipLaunchKernelGGL(preprocess_backward_kernel<1>, grid, block, 0, s, f, g, in.radii, records, tiles_touched,
-                           first_key, key_grads, out);
-    else
-        hipLaunchKernelGGL(preprocess_backward_kernel<2>, grid, block, 0, s, f, g, in.radii, records, tiles_touched,
-                           first_key, key_grads, out);
+    auto launch = [&](auto kernel, const ParameterArgs& p) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, tiles_touched, first_key, key_grads, out, p);
+    };
+    if (par) {
+        if ((reinterpret_cast<uintptr_t>(par->rest) & 15u) != 0 || (reinterpret_cast<uintptr_t>(par->d_rest) & 15u) != 0)
+            launch(preprocess_backward_kernel<0, true>, *par);
+        else if (f.sh_degree == 0)
+            launch(preprocess_backward_kernel<1, true>, *par);
+        else
+            launch(preprocess_backward_kernel<2, true>, *par);
+    } else if (!staged) {
+        launch(preprocess_backward_kernel<0, false>, ParameterArgs());
+    } else if (f.sh_degree == 0) {
+        launch(preprocess_backward_kernel<1, false>, ParameterArgs());
+    } else {
+        launch(preprocess_backward_kernel<2, false>, ParameterArgs());
+    }
     GS355_CHECK_LAUNCH("preprocess backward");
     return GS355_OK;
 }

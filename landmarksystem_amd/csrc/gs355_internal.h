@@ -44,6 +44,13 @@ __device__ __forceinline__ int effective_count(const FrameArgs& f, int P)
     return n < (uint32_t)P ? (int)n : P;
 }
 
+// The stored parameters of the vanilla model in place of activated values (gs355_run_parameters): g.scales holds
+// logarithms, g.rotations unnormalised quaternions, g.opacities logits, g.shs the first SH coefficient [P,1,3].
+struct ParameterArgs {
+    const float* rest = nullptr;  // [P, M - 1, 3]
+    float* d_rest = nullptr;      // its gradient (backward pass)
+};
+
 // Extras of the radii-only preprocess when it serves the anchor prefilter (by-value kernel argument).
 struct FilterArgs {
     int32_t scale_stride = 3;   // floats between the scale rows
@@ -103,7 +110,8 @@ __device__ __forceinline__ float pair_exponent(float dx, float dy, float hx, flo
 constexpr float kAlphaCut = -7.99435329f;  // bits 0xc0ffd1be
 
 // stage launchers (each returns a gs355_status)
-int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, bool radii_only, float* records,
+// `par` (may be NULL): g holds stored parameters
+int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
                       uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, int32_t* radii, hipStream_t s);
 int launch_scan_offsets(const uint32_t* tiles_touched, const int32_t* radii, int32_t P, const uint32_t* p_device,
                         uint32_t* offsets, uint32_t* scan_tmp, gs355_header* header, gs355_header* header_copy, uint32_t n_cap, hipStream_t s);
@@ -122,7 +130,18 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
                            const uint32_t* ranges, const uint32_t* values, const float* records,
                            const uint32_t* tiles_touched, const uint64_t* rects, const gs355_backward_inputs& in,
                            uint32_t* first_key, uint32_t* scan_tmp, float* key_grads, const gs355_gradients& out,
-                           hipStream_t s);
+                           const ParameterArgs* par, hipStream_t s);
+
+// Activations of the stored parameters, each with the framework's own elementwise rounding (the caller is compiled
+// without contraction): the normalisation's sum of squares is taken pairwise, as its row reduction takes it.
+__device__ __forceinline__ float logistic(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+__device__ __forceinline__ float quaternion_norm(const float q[4])
+{
+#pragma clang fp contract(off)
+    const float n = sqrtf((q[0] * q[0] + q[1] * q[1]) + (q[2] * q[2] + q[3] * q[3]));
+    return n < 1e-12f ? 1e-12f : n;  // (NaN stays NaN)
+}
 
 // Number of lanes below this one that `mask` (uniform over the wavefront) holds: the hardware's masked bit count.
 __device__ __forceinline__ uint32_t lanes_below_in(uint64_t mask)

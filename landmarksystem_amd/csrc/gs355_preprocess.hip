@@ -154,6 +154,57 @@ __device__ __forceinline__ void sh_colour_of_entries(float4* __restrict__ mine, 
     }
 }
 
+// sh_colour_of_entries over the split storage of the stored parameters: the first coefficient (12 B per Gaussian) is
+// read by the entry's own lane, the other fifteen (45 floats per Gaussian, dword-aligned) with 16-B loads all the
+// same: a Gaussian's row starts (row & 3) floats behind a 16-B boundary and always spans twelve aligned 16-B chunks.
+// The chunks land in the staging row as they are, so the coefficients of entry e start at float (row & 3) of its
+// row; with the rows' stride of 52 floats consecutive Gaussians then sit an odd number of banks apart.  `n_floats`:
+// 45 P.  The last chunk of the last row may reach past the array: it is pulled back inside, and that row's last
+// floats are fetched by its own lane.
+template <int kLoads>
+__device__ __forceinline__ void sh_colour_of_split_entries(float4* __restrict__ mine, const float* __restrict__ dc,
+                                                           const float* __restrict__ rest, size_t n_floats,
+                                                           size_t group_first, const uint8_t* __restrict__ owner,
+                                                           int first_entry, int count, int lane, int degree,
+                                                           const float* campos)
+{
+    float4 v[kLoads];
+    int dst[kLoads];
+    const size_t last_chunk = n_floats / 4 - 1;  // (a row alone is eleven chunks)
+#pragma unroll
+    for (int it = 0; it < kLoads; ++it) {
+        const int q4 = it * 64 + lane;
+        const int e = min(q4 / 12, count - 1), m = q4 % 12;
+        const size_t first = (group_first + owner[first_entry + e]) * 45;
+        typedef float f4v __attribute__((ext_vector_type(4)));
+        const size_t chunk = min(first / 4 + m, last_chunk);
+        const f4v t = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(rest) + chunk);
+        v[it] = make_float4(t.x, t.y, t.z, t.w);
+        dst[it] = e * (kShStride / 4) + m;
+    }
+    const size_t row = group_first + owner[first_entry + min(lane, count - 1)];
+    float first_coeff[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) first_coeff[c] = __builtin_nontemporal_load(&dc[3 * row + c]);
+#pragma unroll
+    for (int it = 0; it < kLoads; ++it) mine[dst[it]] = v[it];
+    wave_lds_sync();
+    if (lane < count) {
+        float* __restrict__ slot = reinterpret_cast<float*>(mine) + lane * kShStride;
+        float* __restrict__ coeffs = slot + (int)(row & 3);
+        if ((row + 1) * 45 > 4 * (last_chunk + 1))  // the array's last row, where its length is no multiple of four
+            for (int k = (int)(4 * (last_chunk + 1) - row * 45); k < 45; ++k) coeffs[k] = rest[row * 45 + k];
+        float b[16], rgb[3] = {0.f, 0.f, 0.f};
+        sh_basis(degree, slot[48] - campos[0], slot[49] - campos[1], slot[50] - campos[2], b);
+        const int terms = (degree + 1) * (degree + 1);
+        sh_accumulate<0, 1>(terms, first_coeff, b, rgb);
+        sh_accumulate<1, 15>(terms, coeffs, b, rgb);
+        sh_finish(rgb);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) slot[48 + c] = rgb[c];
+    }
+}
+
 // Octree-GS level-of-detail test of one anchor, in the reference's order of fp32 operations
 // (octreegs_encoding.py:251-264).
 __device__ __forceinline__ bool lod_keeps(const gs355_anchor_lod& l, float log2_fork, int i, float x, float y, float z,
@@ -169,8 +220,11 @@ __device__ __forceinline__ bool lod_keeps(const gs355_anchor_lod& l, float log2_
     return level <= r;
 }
 
-template <bool kRadiiOnly>
-__global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaussians g, FilterArgs fx,
+// kStored: g holds the vanilla model's stored parameters, activated here (the activated copies would cost a pass over
+// memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
+// front of a kernel of 0.3 ms).
+template <bool kRadiiOnly, bool kStored>
+__global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaussians g, ParameterArgs par, FilterArgs fx,
                                                          float* __restrict__ records,
                                                          uint32_t* __restrict__ tiles_touched,
                                                          uint64_t* __restrict__ rects,
@@ -209,7 +263,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
             gated = !lod_keeps(fx.lod, fx.log2_fork, i, x, y, z, f.campos);
             if (fx.lod_mask) fx.lod_mask[i] = gated ? 0 : 1;
         }
-        if (g.cov3D_precomp) {
+        if (!kStored && g.cov3D_precomp) {
 #pragma unroll
             for (int k = 0; k < 6; ++k) cov[k] = g.cov3D_precomp[6 * (size_t)i + k];
         } else {
@@ -232,7 +286,14 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         const float inv_w = 1.0f / (hw + 0.0000001f);
         const float ndc_x = hx * inv_w, ndc_y = hy * inv_w;
 
-        if (!g.cov3D_precomp) covariance3d(scale, f.scale_modifier, quat, cov);
+        if (kStored) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) scale[k] = expf(scale[k]);
+            const float norm = quaternion_norm(quat);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) quat[k] = quat[k] / norm;
+        }
+        if (kStored || !g.cov3D_precomp) covariance3d(scale, f.scale_modifier, quat, cov);
 
         // EWA splatting: Jacobian of the perspective projection at the
         // (frustum-clamped) view-space mean, times the world->view rotation.
@@ -291,10 +352,11 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         rects[i] = rect_packed;
     }
     const bool alive = radius > 0;
+    if (kStored && alive) opacity = logistic(opacity);
 
     // ---- colour ----
     float rgb[3] = {0.f, 0.f, 0.f};
-    if (g.colors_precomp) {
+    if (!kStored && g.colors_precomp) {
         if (alive) {
             rgb[0] = g.colors_precomp[3 * (size_t)i];
             rgb[1] = g.colors_precomp[3 * (size_t)i + 1];
@@ -306,7 +368,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         // however many Gaussians were culled.  Other block sizes: every survivor fetches its own block.  Same
         // values and the same order of additions either way.
         const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        const bool packed = f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(g.shs) & 15u) == 0;  // uniform
+        const bool packed = f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(kStored ? par.rest : g.shs) & 15u) == 0;  // uniform
         if (packed) {
             const uint64_t m = __ballot(alive);
             if (lane == 0) s_alive[wave] = __popcll(m);
@@ -333,7 +395,18 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
                 float4* __restrict__ rows = s_sh + first_entry * (kShStride / 4);
                 const size_t group_first = (size_t)blockIdx.x * blockDim.x;
                 const int count = min(share, total - first_entry);
-                if (count <= 16)  // uniform: fewer survivors, fewer load rounds
+                if (kStored) {
+                    const size_t n_floats = (size_t)g.P * 45;
+                    if (count <= 16)
+                        sh_colour_of_split_entries<3>(rows, g.shs, par.rest, n_floats, group_first, s_owner, first_entry, count,
+                                                      lane, f.sh_degree, f.campos);
+                    else if (count <= 32)
+                        sh_colour_of_split_entries<6>(rows, g.shs, par.rest, n_floats, group_first, s_owner, first_entry, count,
+                                                      lane, f.sh_degree, f.campos);
+                    else
+                        sh_colour_of_split_entries<12>(rows, g.shs, par.rest, n_floats, group_first, s_owner, first_entry,
+                                                       count, lane, f.sh_degree, f.campos);
+                } else if (count <= 16)  // uniform: fewer survivors, fewer load rounds
                     sh_colour_of_entries<3>(rows, g.shs, group_first, s_owner, first_entry, count, lane, f.sh_degree, f.campos);
                 else if (count <= 32)
                     sh_colour_of_entries<6>(rows, g.shs, group_first, s_owner, first_entry, count, lane, f.sh_degree, f.campos);
@@ -348,7 +421,13 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         } else if (alive) {
             float b[16];
             sh_basis(f.sh_degree, x - f.campos[0], y - f.campos[1], z - f.campos[2], b);
-            sh_accumulate<0, 16>((f.sh_degree + 1) * (f.sh_degree + 1), g.shs + (size_t)i * f.sh_coeffs * 3, b, rgb);
+            const int terms = (f.sh_degree + 1) * (f.sh_degree + 1);
+            if (kStored) {
+                sh_accumulate<0, 1>(terms, g.shs + (size_t)i * 3, b, rgb);
+                sh_accumulate<1, 15>(terms, par.rest + (size_t)i * (f.sh_coeffs - 1) * 3, b, rgb);
+            } else {
+                sh_accumulate<0, 16>(terms, g.shs + (size_t)i * f.sh_coeffs * 3, b, rgb);
+            }
             sh_finish(rgb);
         }
     }
@@ -441,18 +520,21 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
 
 }  // namespace
 
-int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, bool radii_only, float* records,
+int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
                       uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, int32_t* radii, hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
     const dim3 block(256), grid((g.P + 255) / 256);
     const FilterArgs none;
     if (radii_only)
-        hipLaunchKernelGGL(preprocess_kernel<true>, grid, block, 0, s, f, g, none, records, tiles_touched, rects,
-                           depth_bits, radii);
+        hipLaunchKernelGGL((preprocess_kernel<true, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
+                           tiles_touched, rects, depth_bits, radii);
+    else if (par)
+        hipLaunchKernelGGL((preprocess_kernel<false, true>), grid, block, 0, s, f, g, *par, none, records, tiles_touched,
+                           rects, depth_bits, radii);
     else
-        hipLaunchKernelGGL(preprocess_kernel<false>, grid, block, 0, s, f, g, none, records, tiles_touched, rects,
-                           depth_bits, radii);
+        hipLaunchKernelGGL((preprocess_kernel<false, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
+                           tiles_touched, rects, depth_bits, radii);
     GS355_CHECK_LAUNCH("preprocess");
     return GS355_OK;
 }
@@ -460,8 +542,8 @@ int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, bool radii_o
 int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const FilterArgs& x, int32_t* radii, hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
-    hipLaunchKernelGGL(preprocess_kernel<true>, dim3((g.P + 255) / 256), dim3(256), 0, s, f, g, x, (float*)nullptr,
-                       (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, radii);
+    hipLaunchKernelGGL((preprocess_kernel<true, false>), dim3((g.P + 255) / 256), dim3(256), 0, s, f, g, ParameterArgs(), x,
+                       (float*)nullptr, (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, radii);
     GS355_CHECK_LAUNCH("anchor filter");
     return GS355_OK;
 }

@@ -262,6 +262,29 @@ class GaussianModel(nn.Module):
                                                rotations=rotations, cov3D_precomp=cov3D_precomp)
         return radii_pure > 0
 
+    def _screenspace_points(self):
+        self.viewspace_points = None
+        if self.training and torch.is_grad_enabled():
+            # (a leaf: .grad receives the rasterizer's gradient as it is)
+            self.viewspace_points = torch.zeros_like(self._xyz, requires_grad=True)
+        return self.viewspace_points
+
+    _parameter_getters = ("get_xyz", "get_scaling", "get_rotation", "get_opacity", "get_features")
+
+    def _renders_parameters(self):
+        """Whether the frame can be taken from the stored parameters, activated inside the kernels: nothing is cached
+        (a serving model keeps its activated tensors), no getter is overridden, and the tensors are as the kernels
+        read them.  The activated copies cost five passes over the scene per frame (2.6 of the 5.7 ms of a training
+        step at 6M Gaussians, most of it joining the SH coefficients and splitting their gradient)."""
+        if (self.act_cache and not self.training) or self.compute_cov3D_python:
+            return False
+        if any(getattr(type(self), n) is not getattr(GaussianModel, n) for n in self._parameter_getters):
+            return False
+        P, rest = self._xyz.shape[0], self._features_rest
+        return (P > 0 and rest.dim() == 3 and rest.shape[1] <= 15 and tuple(self._features_dc.shape) == (P, 1, 3)
+                and all(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.shape[0] == P
+                        for t in (self._xyz, self._features_dc, rest, self._scaling, self._rotation, self._opacity)))
+
     def forward(self, viewpoint_camera, scaling_modifier=1.0, override_color=None, render_exclude_filter=None):
         """origin_gs/gs_model.py:112-228.  Under torch.no_grad() (the inference engine) this is the plain frame.
         In training mode with gradients enabled every Gaussian is rendered (no gather), the frame is
@@ -276,6 +299,13 @@ class GaussianModel(nn.Module):
                 voxel_visible_mask = voxel_visible_mask & render_exclude_filter
         self.renderer.raster_settings = _settings(viewpoint_camera, self.background, scaling_modifier,
                                                   self.active_sh_degree)
+        if fused and override_color is None and self._renders_parameters():
+            means2D = self._screenspace_points()
+            rendered_image, radii, _ = self.renderer.forward_parameters(
+                self._xyz, means2D, self._features_dc, self._features_rest, self._opacity, self._scaling, self._rotation)
+            self._radii_all, self._visibility_filter = radii, None
+            self._radii = radii if self.training else None
+            return rendered_image
         means3D, opacity = self.get_xyz, self.get_opacity
         scales = rotations = cov3D_precomp = shs = colors_precomp = None
         if self.compute_cov3D_python:
@@ -289,11 +319,7 @@ class GaussianModel(nn.Module):
             # origin_gs/gs_model.py:184-193, or its rasterizer); here the preprocess kernel evaluates the same
             # expression, clamp_min(eval_sh + 0.5, 0), for either setting
             shs = self.get_features
-        screenspace_points = None
-        if self.training and torch.is_grad_enabled():
-            screenspace_points = torch.zeros_like(means3D, requires_grad=True) + 0
-            screenspace_points.retain_grad()
-        self.viewspace_points = screenspace_points
+        screenspace_points = self._screenspace_points()
         if fused:
             rendered_image, radii, _ = self.renderer(
                 means3D=means3D, means2D=screenspace_points, shs=shs, colors_precomp=colors_precomp, opacities=opacity,

@@ -126,10 +126,13 @@ class FrameInputs:
     """The tensors of one rasterizer call, validated and marshalled."""
 
     def __init__(self, settings, means3D, opacities=None, shs=None, colors_precomp=None, scales=None, rotations=None,
-                 cov3D_precomp=None, need_colour: bool = True, count: Optional[torch.Tensor] = None):
+                 cov3D_precomp=None, need_colour: bool = True, count: Optional[torch.Tensor] = None,
+                 features_rest: Optional[torch.Tensor] = None):
         """`count`: optional one-element int32 tensor on the device holding the number of Gaussians (the anchor
         decode leaves it there); the tensors are then sized for a capacity and only the first `count` rows are
-        rendered, without the host ever reading the number."""
+        rendered, without the host ever reading the number.
+        `features_rest` ([P, M - 1, 3]): the tensors are the vanilla model's stored parameters (shs = features_dc
+        [P, 1, 3], scales = logarithms, rotations unnormalised, opacities = logits), activated by the kernels."""
         if need_colour:
             if (shs is None and colors_precomp is None) or (shs is not None and colors_precomp is not None):
                 raise Exception("Please provide excatly one of either SHs or precomputed colors!")
@@ -156,6 +159,14 @@ class FrameInputs:
             if self.shs.dim() != 3 or self.shs.shape[0] != P or self.shs.shape[2] != 3:
                 raise ValueError("shs must have shape [P, M, 3], got %s" % (tuple(self.shs.shape),))
             sh_coeffs = int(self.shs.shape[1])
+        self.features_rest = None
+        if features_rest is not None:
+            if self.shs is None or sh_coeffs != 1 or scales is None or count is not None:
+                raise ValueError("stored parameters are features_dc [P, 1, 3], features_rest, scales and rotations")
+            self.features_rest = _dev_f32(features_rest, dev, "features_rest")
+            if self.features_rest.dim() != 3 or self.features_rest.shape[0] != P or self.features_rest.shape[2] != 3:
+                raise ValueError("features_rest must have shape [P, M - 1, 3], got %s" % (tuple(features_rest.shape),))
+            sh_coeffs = 1 + int(self.features_rest.shape[1])
 
         s = settings
         self.width, self.height = int(s.image_width), int(s.image_height)
@@ -291,8 +302,12 @@ def run_stages(inputs: FrameInputs, outputs: FrameOutputs, ws: Workspace, n_cap:
     """Enqueue the selected stages over `ws`; returns the layout used."""
     layout = ws.ensure(inputs.P, n_cap, inputs.width, inputs.height)
     stream = torch.cuda.current_stream(inputs.device).cuda_stream
-    rc = _lib.load().gs355_run(C.byref(inputs.frame), C.byref(inputs.gaussians), ws.buffer.data_ptr(),
-                               ws.buffer.numel(), int(n_cap), C.byref(outputs.c), int(stage_mask), stream)
+    frame, gaussians = C.byref(inputs.frame), C.byref(inputs.gaussians)
+    rest = (ws.buffer.data_ptr(), ws.buffer.numel(), int(n_cap), C.byref(outputs.c), int(stage_mask), stream)
+    if inputs.features_rest is None:
+        rc = _lib.load().gs355_run(frame, gaussians, *rest)
+    else:
+        rc = _lib.load().gs355_run_parameters(frame, gaussians, _ptr(inputs.features_rest), *rest)
     _lib.check(rc)
     return layout
 
@@ -364,6 +379,7 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
 
 
 GRAD_NAMES = ("means3D", "means2D", "shs", "colors_precomp", "opacities", "scales", "rotations", "cov3D_precomp")
+PARAMETER_GRAD_NAMES = ("means3D", "means2D", "shs", "features_rest", "opacities", "scales", "rotations")
 
 
 def render_backward(inputs: FrameInputs, out: FrameOutputs, workspace: torch.Tensor, dL_dimage: torch.Tensor,
@@ -372,11 +388,12 @@ def render_backward(inputs: FrameInputs, out: FrameOutputs, workspace: torch.Ten
     """Gradients of a frame rendered by `render` (gs355_render_backward).  `workspace` is the device buffer that
     frame was rendered in, untouched since; `out` its outputs.  Returns contiguous fp32 tensors for the names in
     `want` whose inputs were given: means3D [P,3], means2D [P,3], shs [P,M,3] / colors_precomp [P,3], opacities [P],
-    scales [P,3], rotations [P,4] / cov3D_precomp [P,6]."""
+    scales [P,3], rotations [P,4] / cov3D_precomp [P,6]; of a frame over stored parameters (PARAMETER_GRAD_NAMES) those of
+    the parameters: shs = features_dc [P,1,3], features_rest [P,M-1,3], logarithms, quaternions and logits."""
     dev, P, H, W = inputs.device, inputs.P, inputs.height, inputs.width
     given = {"means3D": inputs.means3D, "means2D": inputs.means3D, "shs": inputs.shs,
              "colors_precomp": inputs.colors_precomp, "opacities": inputs.opacities, "scales": inputs.scales,
-             "rotations": inputs.rotations, "cov3D_precomp": inputs.cov3D_precomp}
+             "rotations": inputs.rotations, "cov3D_precomp": inputs.cov3D_precomp, "features_rest": inputs.features_rest}
     grads = {n: torch.empty_like(given[n]) for n in want if given[n] is not None}
     gi = _dev_f32(dL_dimage, dev, "dL_dimage", (3, H, W))
     gd = _dev_f32(dL_ddepth, dev, "dL_ddepth", (H, W))
@@ -390,7 +407,12 @@ def render_backward(inputs: FrameInputs, out: FrameOutputs, workspace: torch.Ten
     _lib.check(_lib.load().gs355_backward_scratch_bytes(P, int(out.key_capacity), C.byref(need)))
     scratch = torch.empty(need.value // 4, dtype=torch.float32, device=dev)
     stream = torch.cuda.current_stream(dev).cuda_stream
-    _lib.check(_lib.load().gs355_render_backward(C.byref(inputs.frame), C.byref(inputs.gaussians), workspace.data_ptr(),
-                                                 workspace.numel(), int(out.key_capacity), C.byref(b),
-                                                 scratch.data_ptr(), scratch.numel() * 4, C.byref(g), stream))
+    frame, gaussians = C.byref(inputs.frame), C.byref(inputs.gaussians)
+    rest = (workspace.data_ptr(), workspace.numel(), int(out.key_capacity), C.byref(b), scratch.data_ptr(),
+            scratch.numel() * 4, C.byref(g))
+    if inputs.features_rest is None:
+        _lib.check(_lib.load().gs355_render_backward(frame, gaussians, *rest, stream))
+    else:
+        _lib.check(_lib.load().gs355_render_parameters_backward(frame, gaussians, _ptr(inputs.features_rest), *rest,
+                                                                _ptr(grads.get("features_rest")), stream))
     return grads

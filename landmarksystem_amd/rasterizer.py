@@ -53,6 +53,8 @@ class GaussianRasterizationSettings(NamedTuple):
     debug: bool
 
 
+_RENDER_AGAIN = ("the rasterizer's backward pass ran already for this frame: its workspace is released after the first "
+                 "backward pass (retain_graph=True cannot replay it); render the frame again")
 _INPUT_NAMES = ("means3D", "means2D", "opacities", "shs", "colors_precomp", "scales", "rotations", "cov3D_precomp")
 
 
@@ -92,9 +94,7 @@ class _RasterizeGaussians(torch.autograd.Function):
         if g_image is None and g_depth is None and g_alpha is None:
             return (None,) * 9
         if ctx.workspace is None:
-            raise RuntimeError("the rasterizer's backward pass ran already for this frame: its workspace is released "
-                               "after the first backward pass (retain_graph=True cannot replay it); render the frame "
-                               "again")
+            raise RuntimeError(_RENDER_AGAIN)
         inputs = pipeline.FrameInputs(ctx.settings, means3D, opacities=opacities, shs=shs,
                                       colors_precomp=colors_precomp, scales=scales, rotations=rotations,
                                       cov3D_precomp=cov3D_precomp)
@@ -114,6 +114,43 @@ class _RasterizeGaussians(torch.autograd.Function):
                 g = g.reshape(shape).to(dtype)
             result.append(g)
         return tuple(result)
+
+
+class _RasterizeParameters(torch.autograd.Function):
+    """The same frame from the vanilla model's stored parameters: the kernels activate them on the way in and carry the
+    gradients through the activations on the way out, so neither the activated tensors nor their gradients exist."""
+
+    @staticmethod
+    def forward(ctx, settings, xyz, means2D, features_dc, features_rest, opacity, scaling, rotation):
+        inputs = pipeline.FrameInputs(settings, xyz, opacities=opacity, shs=features_dc, scales=scaling,
+                                      rotations=rotation, features_rest=features_rest)
+        ws = pipeline.default_workspace(inputs.device)
+        out = pipeline.render(inputs, ws=ws)
+        ctx.workspace, ws.buffer = ws.buffer, None  # as in _RasterizeGaussians
+        ctx.settings, ctx.key_capacity = settings, out.key_capacity
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(xyz, features_dc, features_rest, opacity, scaling, rotation, out.image, out.depth,
+                              out.alpha, out.radii)
+        ctx.mark_non_differentiable(out.radii)
+        return out.image, out.radii, out.depth, out.alpha
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g_image, _g_radii, g_depth, g_alpha):
+        xyz, features_dc, features_rest, opacity, scaling, rotation, image, depth, alpha, radii = ctx.saved_tensors
+        if g_image is None and g_depth is None and g_alpha is None:
+            return (None,) * 8
+        if ctx.workspace is None:
+            raise RuntimeError(_RENDER_AGAIN)
+        out = SimpleNamespace(image=image, depth=depth, alpha=alpha, radii=radii, key_capacity=ctx.key_capacity)
+        inputs = pipeline.FrameInputs(ctx.settings, xyz, opacities=opacity, shs=features_dc, scales=scaling,
+                                      rotations=rotation, features_rest=features_rest)
+        names = ("means3D", "means2D", "shs", "features_rest", "opacities", "scales", "rotations")
+        want = [n for n, needed in zip(names, ctx.needs_input_grad[1:]) if needed]
+        grads = pipeline.render_backward(inputs, out, ctx.workspace, torch.zeros_like(image) if g_image is None else g_image,
+                                         g_depth, g_alpha, want=want)
+        ctx.workspace = None
+        return (None,) + tuple(grads.get(n) for n in names)
 
 
 class GaussianRasterizer(nn.Module):
@@ -154,6 +191,21 @@ class GaussianRasterizer(nn.Module):
         inputs = pipeline.FrameInputs(self.raster_settings, means3D, opacities=opacities, shs=shs,
                                       colors_precomp=colors_precomp, scales=scales, rotations=rotations,
                                       cov3D_precomp=cov3D_precomp, count=count)
+        out = pipeline.render(inputs)
+        self.last_depth, self.last_alpha, self.last_num_keys = out.depth, out.alpha, out.num_keys
+        return out.image, out.radii, out.depth
+
+    def forward_parameters(self, xyz, means2D, features_dc, features_rest, opacity, scaling, rotation):
+        """forward() of GaussianModel's stored parameters (fp32, contiguous, on the GPU): what
+        forward(xyz, means2D, sigmoid(opacity), cat(features_dc, features_rest), scales=exp(scaling),
+        rotations=normalize(rotation)) returns, and its gradients, without the activated tensors."""
+        tensors = (xyz, means2D, features_dc, features_rest, opacity, scaling, rotation)
+        if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors):
+            image, radii, depth, alpha = _RasterizeParameters.apply(self.raster_settings, *tensors)
+            self.last_depth, self.last_alpha, self.last_num_keys = depth, alpha, 0
+            return image, radii, depth
+        inputs = pipeline.FrameInputs(self.raster_settings, xyz, opacities=opacity, shs=features_dc, scales=scaling,
+                                      rotations=rotation, features_rest=features_rest)
         out = pipeline.render(inputs)
         self.last_depth, self.last_alpha, self.last_num_keys = out.depth, out.alpha, out.num_keys
         return out.image, out.radii, out.depth

@@ -1,0 +1,66 @@
+"""Frames and gradients taken from GaussianModel's stored parameters inside the kernels, against the same frame over the
+activated tensors (whose own parity with the oracle the other tests hold)."""
+import pytest
+import torch
+
+from landmarksystem_amd import GaussianRasterizer, scenes
+from landmarksystem_amd.models import GaussianModel
+from tests.helpers import settings_for
+from tests.test_gpu_backward import assert_grad_close
+
+pytestmark = pytest.mark.gpu
+
+
+# counts around the staging's wavefront and workgroup, and rows of 45 floats whose total is no multiple of four
+@pytest.mark.parametrize("P,degree,active", [(1, 3, 3), (2, 3, 3), (63, 0, 0), (65, 1, 1), (257, 2, 2), (258, 3, 1),
+                                             (1003, 3, 3), (30_001, 3, 3), (4096, 3, 0)])
+def test_stored_parameters_render_as_activated_ones(gpu_device, P, degree, active):
+    scene = scenes.tiny_scene(P=P, width=150, height=97, sh_degree=degree, log_scale_mean=-2.5)
+    g = torch.Generator().manual_seed(P)
+    rot = scene.rotations * (0.2 + 2.0 * torch.rand(P, 1, generator=g))
+    if P > 2:
+        rot[1] = 0.0  # (the normalisation's floor)
+    model = GaussianModel.from_activated(scene.means3D, scene.scales, rot, scene.opacities, scene.shs, sh_degree=degree)
+    model = model.to(gpu_device).train()
+    leaves = dict(means3D=model._xyz, shs=model._features_dc, features_rest=model._features_rest,
+                  opacities=model._opacity, scales=model._scaling, rotations=model._rotation)
+    for p in leaves.values():
+        p.requires_grad_(True)
+    model.active_sh_degree = active
+    r = GaussianRasterizer(settings_for(scene, gpu_device, sh_degree=active))
+    weights = torch.randn(3, 97, 150, generator=g).to(gpu_device)
+    results = []
+    for stored in (True, False):
+        means2D = torch.zeros(P, 3, device=gpu_device, requires_grad=True)
+        for p in leaves.values():
+            p.grad = None
+        if stored:
+            image, radii, depth = r.forward_parameters(model._xyz, means2D, model._features_dc, model._features_rest,
+                                                       model._opacity, model._scaling, model._rotation)
+        else:
+            image, radii, depth = r(means3D=model.get_xyz, means2D=means2D, shs=model.get_features,
+                                    opacities=model.get_opacity, scales=model.get_scaling, rotations=model.get_rotation)
+        (image * weights + depth * 0.1).sum().backward()
+        results.append((image.detach(), radii, depth.detach(),
+                        {n: p.grad.cpu().numpy() for n, p in dict(leaves, means2D=means2D).items()}))
+    (image_s, radii_s, depth_s, grads_s), (image_a, radii_a, depth_a, grads_a) = results
+    assert torch.equal(radii_s, radii_a) and torch.equal(image_s, image_a) and torch.equal(depth_s, depth_a)
+    for name, want in grads_a.items():
+        assert grads_s[name].shape == want.shape
+        if want.size:
+            assert_grad_close(grads_s[name], want, name)
+
+
+def test_training_model_takes_the_stored_parameters(gpu_device):
+    scene = scenes.tiny_scene(P=500, width=80, height=64, sh_degree=2)
+    model = GaussianModel.from_activated(scene.means3D, scene.scales, scene.rotations, scene.opacities, scene.shs,
+                                         sh_degree=2).to(gpu_device).train()
+    for p in model.parameters():
+        p.requires_grad_(True)
+    assert model._renders_parameters()
+    image = model(scene.camera)
+    image.sum().backward()
+    assert model.viewspace_points.grad.shape == model._xyz.shape and model.radii.shape == (500,)
+    model.compute_cov3D_python = True  # (the activated tensors again)
+    assert not model._renders_parameters()
+    assert torch.allclose(model(scene.camera), image, atol=1e-4)
