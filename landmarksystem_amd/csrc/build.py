@@ -36,7 +36,8 @@ SOURCES = [
     ("gs355_gather.hip", []),
     ("gs355_decode.hip", []),
     ("gs355_blend.hip", []),
-    ("gs355_backward.hip", []),
+    # (matrix results in ordinary registers: the blend's backward reads them with vector instructions right away)
+    ("gs355_backward.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form"]),
 ]
 
 

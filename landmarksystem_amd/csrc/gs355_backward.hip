@@ -9,9 +9,9 @@
 //                    prefix P_i = sum_{j<=i} w_j f_j and R = out_pixel . dL/dpixel - T_final dL/dalpha_out (all
 //                    known from the forward outputs), dL/dalpha_i = T_i f_i - (R - P_i) / (1 - alpha_i): no
 //                    division by a transmittance and no second, reversed walk.  Per-pair contributions are summed
-//                    over the 16 pixels of a block by lane exchanges inside the 16-lane row, added to the staged
-//                    Gaussian's accumulators in LDS (one LDS atomic per step: LDS float atomics are slow), and
-//                    written once per batch of 128 as one 48-byte record per (tile, Gaussian) key.  No global
+//                    over the 16 pixels of a block four list entries at a time, added to the wavefront's own sums of
+//                    the staged Gaussians in LDS (no atomics), and written once per batch of 64 as one 48-byte
+//                    record per (tile, Gaussian) key.  No global
 //                    atomics (they cost more than the rest of the kernel): the records of a Gaussian are
 //                    consecutive, in the order its tile rectangle is walked, and the next kernel sums them in
 //                    that order, so gradients are identical from run to run.
@@ -25,7 +25,6 @@ namespace gs355 {
 
 namespace {
 
-constexpr int kGradFloats = 10;  // accumulators per staged Gaussian in LDS
 constexpr int kKeyFloats = GS355_KEY_GRAD_FLOATS;  // per-key record: dpx, dpy, dconic xyz, dopacity, drgb, ddepth, 2 unused
 
 // Record slot of the key (tile, Gaussian): the Gaussian's keys in the order its tile rectangle is walked
@@ -36,81 +35,46 @@ __device__ __forceinline__ uint32_t key_slot(uint32_t first, uint64_t rect, int 
     return first + (uint32_t)((tile_y - y0) * (x1 - x0) + (tile_x - x0));
 }
 
-template <int kCtrl>
-__device__ __forceinline__ float dpp(float v)
+// Value of lane `kLane` of each quad of lanes, in all four of them.
+template <int kLane>
+__device__ __forceinline__ float quad_lane(float v)
 {
+    constexpr int kCtrl = kLane * 0x55;  // quad_perm [k, k, k, k]
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
 }
 
-// Two values reduced over a lane pair in one exchange: the lane with `upper` clear keeps a, the other keeps b,
-// each adds its partner's copy of the value it keeps.
-template <int kCtrl>
-__device__ __forceinline__ float keep_one_of_two(float a, float b, bool upper)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+// Sums over the four 16-lane rows, two values at a time: after the swap of lane halves (kLanes = 32) or of neighbouring
+// rows (16) one register holds the first value's two parts where the other holds the second's, and one addition
+// leaves the first value's partial sum in the lower half (even rows), the second's in the upper (odd rows).
+template <int kLanes>
+__device__ __forceinline__ float add_halves(float a, float b)
 {
-    const float send = upper ? a : b, keep = upper ? b : a;
-    return keep + dpp<kCtrl>(send);
+    const unsigned ua = (unsigned)__float_as_int(a), ub = (unsigned)__float_as_int(b);
+    u32x2 r;
+    if (kLanes == 32) r = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
+    else r = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+    return __int_as_float((int)r.x) + __int_as_float((int)r.y);
 }
 
-struct PixelGrad {
-    float g0, g1, g2, g3;  // dL/d(r, g, b, depth) of this pixel
-    float R;               // out . g - T_final * dL/dalpha_out
-};
-
-// One 16-lane row evaluates staged Gaussian `a, b, c` on its 16 pixels.  Returns false if no lane of the wavefront
-// blended its pair; otherwise lane s < 10 of each row returns in `sum` the row's total of accumulator s:
-// the moments of dL/dpower over the pixel offsets (dpow dx, dpow dy, dpow dx^2, dpow dx dy, dpow dy^2),
-// dL/dopacity, dL/d(r, g, b, depth).  T carries the forward blend's state (sign = finished).
-// b.y is log2(opacity): opacity * exp(power) is evaluated exactly as the forward blend evaluates it (one multiply-add
-// into the hardware exp2, decided on the exponent before the exp2), so both passes take the same decisions.  The
-// opacity's accumulator receives sum(dL/dpower) = opacity * dL/dopacity; the caller divides once per Gaussian.
-__device__ __forceinline__ bool backward_one(float& T, float& prefix, const PixelGrad& pg, float pxf, float pyf,
-                                             const float4 a, const float4 b, const float4 c, bool enabled, int sub,
-                                             float& sum)
-{
-    const float dx = a.x - pxf, dy = a.y - pyf;
-    const float power = pair_exponent(dx, dy, a.z, a.w, b.x);  // a.z, a.w, b.x = -conic_x / 2, -conic_y, -conic_z / 2
-    const float t = __builtin_fmaf(power, 1.4426950408889634f, b.y);
-    const bool accept = enabled && !(power > 0.0f || t < kAlphaCut);  // the forward blend's decision, on the exponent
-    if (__ballot(accept) == 0ull) return false;
-    const float raw = __builtin_amdgcn_exp2f(t);  // opacity * exp(power)
-    const float alpha = fminf(0.99f, raw);
-    const float test_T = __builtin_fmaf(-alpha, T, T);  // T - alpha T, as the forward blend forms it
-    const bool hit = accept && test_T >= 0.0001f;
-    if (accept && !hit && T > 0.0f) T = -T;
-    if (__ballot(hit) == 0ull) return false;
-    float w = 0.0f, dpow = 0.0f;
-    if (hit) {
-        w = alpha * T;
-        const float fg = b.z * pg.g0 + b.w * pg.g1 + c.x * pg.g2 + c.y * pg.g3;
-        prefix += w * fg;
-        const float dalpha = T * fg - (pg.R - prefix) * __builtin_amdgcn_rcpf(1.0f - alpha);
-        dpow = raw * dalpha;  // the gradient passes through min(0.99, .) unchanged
-        T = test_T;
-    }
-    const float dop = dpow;  // (times 1 / opacity, once per Gaussian, when the batch's sums are turned into records)
-    const float mx = dpow * dx, my = dpow * dy;
-    // ten sums over the row's 16 lanes, transposed as they are reduced: after the exchanges inside lane pairs and
-    // quads a lane holds one of four (then two) values, the quads' partial sums are rotated together, and lane s
-    // ends with the total of value s
-    const bool b0 = (sub & 1) != 0, b1 = (sub & 2) != 0;
-    const float u0 = keep_one_of_two<0xB1>(mx, my, b0);            // quad_perm [1,0,3,2]
-    const float u1 = keep_one_of_two<0xB1>(mx * dx, mx * dy, b0);
-    const float u2 = keep_one_of_two<0xB1>(my * dy, dop, b0);
-    const float u3 = keep_one_of_two<0xB1>(w * pg.g0, w * pg.g1, b0);
-    const float u4 = keep_one_of_two<0xB1>(w * pg.g2, w * pg.g3, b0);
-    float t0 = keep_one_of_two<0x4E>(u0, u1, b1);                  // quad_perm [2,3,0,1]: value 2 b1 + b0
-    float t1 = keep_one_of_two<0x4E>(u2, u3, b1);                  // value 4 + 2 b1 + b0
-    float t2 = u4 + dpp<0x4E>(u4);                                 // value 8 + b0
-    t0 += dpp<0x124>(t0);                                          // row_ror:4
-    t1 += dpp<0x124>(t1);
-    t2 += dpp<0x124>(t2);
-    t0 += dpp<0x128>(t0);                                          // row_ror:8
-    t1 += dpp<0x128>(t1);
-    t2 += dpp<0x128>(t2);
-    sum = sub < 4 ? t0 : sub < 8 ? t1 : t2;
-    return true;
-}
-
+// Lane layout of a wavefront's 8x8 quadrant: lane = 16 q + 4 b + i is pixel i of row q of the 4x4 block b.  Per step a
+// block's pixels produce two values each, d = dL/dpower and w = alpha T, and ten sums over the sixteen pixels are wanted:
+// the moments of d over the offsets from the splat's centre, and w against the four channels of dL/dpixel.  Four steps
+// are reduced together:
+//   - a matrix instruction per value and step (4x4x1, sixteen blocks of four lanes, K = 1; value times a one-hot row)
+//     hands step s's four values of a quad to the quad's lane s, so that lane (q, b, s) holds row q of step s in four
+//     registers: a transposition for eight cycles each;
+//   - the sums over a row are then additions inside a lane, every one serving four steps;
+//   - the sums over the rows pair up values through lane swaps (add_halves): ten values, sixteen instructions, and each
+//     row ends with the totals of its own two or three.
+// Reducing each step by itself with lane exchanges took 53 vector instructions per step, more than the gradient
+// arithmetic; this takes about 20.  Blend backward at 6M Gaussians / 1080p: 1.34 -> 1.25 ms, 622M -> 491M vector
+// instructions, LDS pipe 73 -> 37 % busy.  Larger matrix instructions do not pay for the sums (1.45 ms): fp32 ones
+// occupy the SIMD like the vector instructions they replace.
+// kDepth: a gradient arrives for the depth plane.
+template <bool kDepth>
 __global__ __launch_bounds__(256) void blend_backward_kernel(
     FrameArgs f, const gs355_header* __restrict__ header, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ values, const float* __restrict__ records, const float* __restrict__ image,
@@ -118,80 +82,94 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     const float* __restrict__ g_depth, const float* __restrict__ g_alpha, const uint64_t* __restrict__ rects,
     const uint32_t* __restrict__ first_key, float* __restrict__ key_grads)
 {
-    // staged Gaussians per round: 128 (13 KB of LDS per workgroup) leaves the register file as the limit on resident
-    // wavefronts; 256 measured 2 % slower
-    constexpr int kBatch = 128;
-    __shared__ float4 s_a[kBatch];  // px, py, -conic_x / 2, -conic_y   (rescaled as the forward blend stages them)
-    __shared__ float4 s_b[kBatch];  // -conic_z / 2, log2(opacity), r, g
-    __shared__ float4 s_c[kBatch];  // b, depth, reach_x, reach_y
-    __shared__ float s_grad[kBatch * kGradFloats];
+    // staged Gaussians per round, four threads each (96 and 128 measured 1 and 9 % slower: fewer resident workgroups)
+    constexpr int kBatch = 64;
+    // (entry kBatch: the null record, zero conic and log2(opacity) = -inf, which no pixel accepts; nothing reads its sums)
+    __shared__ float4 s_a[kBatch + 1];  // px, py, -conic_x / 2, -conic_y   (rescaled as the forward blend stages them)
+    __shared__ float4 s_b[kBatch + 1];  // -conic_z / 2, log2(opacity), r, g
+    __shared__ float4 s_c[kBatch + 1];  // b, depth, reach_x, reach_y
+    // Sums of each wavefront: of d, d dx | d dy, d dy^2 | d dx dy, green | red, blue | d dx^2, depth.  A wavefront owns
+    // its sums and serves its four blocks one after the other, so plain reads and writes do: float atomics on sums
+    // shared by the workgroup take almost two cycles per lane of the CU's one LDS pipe, which bounded the kernel
+    // (LDS pipe busy 73 %, whatever the vector instructions were reduced to).
+    __shared__ float2 s_sum[4][kBatch + 1][5];
+    __shared__ uint32_t s_slot[kBatch];  // where each staged Gaussian's record goes
     __shared__ uint32_t s_wave_done[4];
-    __shared__ uint8_t s_list[4][4][kBatch + 4];
+    __shared__ __align__(4) uint8_t s_list[4][4][kBatch + 8];
 
     if (header->overflow) return;
     const int tile = blockIdx.x;
     const int tile_x = tile % f.grid_x, tile_y = tile / f.grid_x;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int group = lane >> 4, sub = lane & 15;
+    const int row = lane >> 4, group = (lane >> 2) & 3, sub = lane & 3;
     const int qx0 = tile_x * kTile + (wave & 1) * 8, qy0 = tile_y * kTile + (wave >> 1) * 8;
-    const int px = qx0 + (group & 1) * 4 + (sub & 3), py = qy0 + (group >> 1) * 4 + (sub >> 2);
+    const int px = qx0 + (group & 1) * 4 + sub, py = qy0 + (group >> 1) * 4 + row;
     const bool inside = px < f.W && py < f.H;
     const float pxf = (float)px, pyf = (float)py;
     const float x_lo0 = (float)qx0, x_hi0 = (float)(qx0 + 3), x_lo1 = (float)(qx0 + 4), x_hi1 = (float)(qx0 + 7);
     const float y_lo0 = (float)qy0, y_hi0 = (float)(qy0 + 3), y_lo1 = (float)(qy0 + 4), y_hi1 = (float)(qy0 + 7);
+    constexpr uint64_t kBlockLanes = 0x000F000F000F000Full;  // block 0's lanes: four of each row
 
-    PixelGrad pg = {0.f, 0.f, 0.f, 0.f, 0.f};
+    float g0 = 0.f, g1 = 0.f, g2 = 0.f, g3 = 0.f;  // dL/d(r, g, b, depth) of this pixel
+    float R = 0.f;                                 // out . g - T_final * dL/dalpha_out
     if (inside) {
         const size_t plane = (size_t)f.W * f.H;
         const size_t o = (size_t)py * f.W + px;
-        pg.g0 = g_image[o];
-        pg.g1 = g_image[plane + o];
-        pg.g2 = g_image[2 * plane + o];
-        pg.R = image[o] * pg.g0 + image[plane + o] * pg.g1 + image[2 * plane + o] * pg.g2;
-        if (g_depth) {
-            pg.g3 = g_depth[o];
-            pg.R += out_depth[o] * pg.g3;
+        g0 = g_image[o];
+        g1 = g_image[plane + o];
+        g2 = g_image[2 * plane + o];
+        R = image[o] * g0 + image[plane + o] * g1 + image[2 * plane + o] * g2;
+        if (kDepth) {
+            g3 = g_depth[o];
+            R += out_depth[o] * g3;
         }
-        if (g_alpha) pg.R -= (1.0f - out_alpha[o]) * g_alpha[o];
+        if (g_alpha) R -= (1.0f - out_alpha[o]) * g_alpha[o];
     }
-
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    // 1 in the lanes of a constant mask (one instruction, and no register held for it)
+    auto ones = [](uint64_t lanes) { return __builtin_amdgcn_inverse_ballot_w64(lanes) ? 1.0f : 0.0f; };
+    // staging: thread 4 k + part brings part `part` of the batch's Gaussian k (part 3: the slot of its record), and later
+    // writes a third of its record
+    const int staged = tid >> 2, part = tid & 3;
     const uint32_t lo = ranges[2 * tile], hi = ranges[2 * tile + 1];
     float T = inside ? 1.0f : -1.0f, prefix = 0.0f;
+    if (tid < 3)
+        (tid == 0 ? s_a : tid == 1 ? s_b : s_c)[kBatch] = make_float4(0.f, tid == 1 ? -__builtin_inff() : 0.f, 0.f, 0.f);
+
+    for (int k = tid; k < 4 * (kBatch + 1) * 5; k += 256) (&s_sum[0][0][0])[k] = make_float2(0.f, 0.f);
 
     uint32_t base = lo;
     for (; base < hi; base += kBatch) {
-        const bool wave_done = __ballot(T > 0.0f) == 0ull;
+        const uint64_t live = __ballot(T > 0.0f);
+        const bool wave_done = live == 0ull;
         if (lane == 0) s_wave_done[wave] = wave_done ? 1u : 0u;
-        const uint32_t j = base + tid;
-        const bool staging = tid < kBatch && j < hi;  // this thread stages (and later writes the record of) a Gaussian
-        uint32_t slot = 0;
-        if (staging) {
-            const uint32_t g = values[j];
-            const float4* __restrict__ rec = reinterpret_cast<const float4*>(records + (size_t)g * kRecordFloats);
-            const float4 r0 = rec[0], r1 = rec[1];
-            const float opacity = r1.y < 0.0f ? 0.0f : r1.y;  // as the forward blend: a negative opacity never blends
-            s_a[tid] = make_float4(r0.x, r0.y, -0.5f * r0.z, -r0.w);
-            s_b[tid] = make_float4(-0.5f * r1.x, __builtin_amdgcn_logf(opacity), r1.z, r1.w);
-            s_c[tid] = rec[2];
-            slot = key_slot(first_key[g], rects[g], tile_x, tile_y);
-        }
-        if (tid < kBatch) {
-            float2* __restrict__ row = reinterpret_cast<float2*>(s_grad + tid * kGradFloats);
-#pragma unroll
-            for (int k = 0; k < kGradFloats / 2; ++k) row[k] = make_float2(0.f, 0.f);
+        const int count = (int)min((uint32_t)kBatch, hi - base);
+        if (staged < count) {
+            const uint32_t g = values[base + staged];
+            if (part == 3) {
+                s_slot[staged] = key_slot(first_key[g], rects[g], tile_x, tile_y);
+            } else {
+                float4 v = reinterpret_cast<const float4*>(records + (size_t)g * kRecordFloats)[part];
+                if (part == 0) {
+                    v.z *= -0.5f;
+                    v.w = -v.w;
+                } else if (part == 1) {  // (as the forward blend: a negative opacity never blends)
+                    v.x *= -0.5f;
+                    v.y = __builtin_amdgcn_logf(v.y < 0.0f ? 0.0f : v.y);
+                }
+                (part == 0 ? s_a : part == 1 ? s_b : s_c)[staged] = v;
+            }
         }
         __syncthreads();
         if ((s_wave_done[0] & s_wave_done[1] & s_wave_done[2] & s_wave_done[3]) != 0u) break;
-        const int count = (int)min((uint32_t)kBatch, hi - base);
         if (!wave_done) {
             // ---- lists: which staged Gaussians reach which 4x4 block (lane = Gaussian), as the forward blend ----
             uint32_t len[4] = {0u, 0u, 0u, 0u};
-            for (int chunk = 0; chunk < count; chunk += 64) {
+            {
                 // lane masks straight from the comparisons, combined in scalar registers (as the forward blend)
-                const int k = chunk + lane;  // < kBatch: slots past `count` hold older records, masked by `valid`
-                const uint64_t valid = __ballot(k < count);
-                const float4 a = s_a[k];
-                const float4 c = s_c[k];
+                const uint64_t valid = __ballot(lane < count);  // (slots past `count` hold older records)
+                const float4 a = s_a[lane];
+                const float4 c = s_c[lane];
                 const float bx_lo = a.x - c.z, bx_hi = a.x + c.z, by_lo = a.y - c.w, by_hi = a.y + c.w;
                 const uint64_t in_x0 = __ballot(bx_hi >= x_lo0) & __ballot(bx_lo <= x_hi0) & valid;
                 const uint64_t in_x1 = __ballot(bx_hi >= x_lo1) & __ballot(bx_lo <= x_hi1) & valid;
@@ -199,40 +177,132 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
                 const uint64_t in_y1 = __ballot(by_hi >= y_lo1) & __ballot(by_lo <= y_hi1);
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
+                    if ((live & (kBlockLanes << (4 * b))) == 0ull) continue;  // (all of the block's pixels have finished)
                     const uint64_t m = ((b & 1) ? in_x1 : in_x0) & ((b >> 1) ? in_y1 : in_y0);
-                    if (__builtin_amdgcn_inverse_ballot_w64(m)) s_list[wave][b][len[b] + lanes_below_in(m)] = (uint8_t)k;
-                    len[b] += (uint32_t)__popcll(m);
+                    if (__builtin_amdgcn_inverse_ballot_w64(m)) s_list[wave][b][lanes_below_in(m)] = (uint8_t)lane;
+                    len[b] = (uint32_t)__popcll(m);
                 }
             }
+            const uint32_t longest = (uint32_t)__builtin_amdgcn_readfirstlane(
+                (int)max(max(len[0], len[1]), max(len[2], len[3])));
+            const uint32_t quads = (longest + 3u) / 4u;
+#pragma unroll
+            for (int b = 0; b < 4; ++b)  // padded with the null record to the common length
+                if (len[b] + (uint32_t)lane < quads * 4u) s_list[wave][b][len[b] + (uint32_t)lane] = (uint8_t)kBatch;
             wave_lds_sync();
-            const uint32_t my_len = group == 0 ? len[0] : group == 1 ? len[1] : group == 2 ? len[2] : len[3];
-            const uint32_t longest = max(max(len[0], len[1]), max(len[2], len[3]));
-            const uint8_t* __restrict__ mine = s_list[wave][group];
-            uint32_t k_next = mine[0];
-            for (uint32_t i = 0; i < longest; ++i) {
-                const uint32_t kk = k_next;
-                k_next = mine[i + 1];
-                float sum;
-                if (backward_one(T, prefix, pg, pxf, pyf, s_a[kk], s_b[kk], s_c[kk], i < my_len, sub, sum)) {
-                    // lane s of each row adds accumulator s of the row's Gaussian
-                    if (sub < 10 && i < my_len && sum != 0.0f) atomicAdd(&s_grad[kk * kGradFloats + sub], sum);
+            const uint32_t* __restrict__ mine = reinterpret_cast<const uint32_t*>(s_list[wave][group]);
+            uint32_t next = mine[0];  // read ahead by one round (rounds past the end are never used)
+            for (uint32_t i = 0; i < quads; ++i) {
+                const uint32_t entries = next;
+                next = mine[i + 1];
+                float d[4], w[4];
+                uint64_t any = 0ull;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    // One entry per block.  b.y is log2(opacity): opacity * exp(power) is evaluated exactly as the
+                    // forward blend evaluates it (decided on the exponent before the exp2), so both passes take the
+                    // same decisions.  T carries the forward blend's state (sign = finished).
+                    d[s] = w[s] = 0.0f;
+                    const uint32_t k = (entries >> (8 * s)) & 0xFFu;
+                    const float4 a = s_a[k], b = s_b[k];
+                    const float dx = a.x - pxf, dy = a.y - pyf;
+                    const float power = pair_exponent(dx, dy, a.z, a.w, b.x);
+                    const float t = __builtin_fmaf(power, 1.4426950408889634f, b.y);
+                    const uint64_t accept = __ballot(!(power > 0.0f)) & __ballot(!(t < kAlphaCut));
+                    if (accept != 0ull) {
+                        const float raw = __builtin_amdgcn_exp2f(t);  // opacity * exp(power)
+                        const float alpha = fminf(0.99f, raw);
+                        const float test_T = __builtin_fmaf(-alpha, T, T);  // T - alpha T, as the forward blend forms it
+                        const uint64_t hit = accept & __ballot(test_T >= 0.0001f);
+                        if (__builtin_amdgcn_inverse_ballot_w64(accept & ~hit)) T = -fabsf(T);
+                        any |= hit;
+                        if (__builtin_amdgcn_inverse_ballot_w64(hit)) {
+                            const float2 c = *reinterpret_cast<const float2*>(&s_c[k]);
+                            w[s] = alpha * T;
+                            float fg = b.z * g0 + b.w * g1 + c.x * g2;
+                            if (kDepth) fg = __builtin_fmaf(c.y, g3, fg);
+                            prefix = __builtin_fmaf(w[s], fg, prefix);
+                            const float dalpha = T * fg - (R - prefix) * __builtin_amdgcn_rcpf(1.0f - alpha);
+                            d[s] = raw * dalpha;  // the gradient passes through min(0.99, .) unchanged
+                            T = test_T;
+                        }
+                    }
+                }
+                if (any != 0ull) {
+                    f32x4 D = zero4, W = zero4;  // lane (q, b, s): d and w of the row's pixels at step s
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const float one_hot = ones(0x1111111111111111ull << s);
+                        D = __builtin_amdgcn_mfma_f32_4x4x1f32(d[s], one_hot, D, 0, 0, 0);
+                        W = __builtin_amdgcn_mfma_f32_4x4x1f32(w[s], one_hot, W, 0, 0, 0);
+                    }
+                    const uint32_t k = (entries >> (8 * sub)) & 0xFFu;  // the column's entry
+                    const float2 at = *reinterpret_cast<const float2*>(&s_a[k]);
+                    const float ax = at.x - (pxf - (float)sub), dy = at.y - pyf;  // from the row's first pixel
+                    const float ax1 = ax - 1.0f, ax2 = ax - 2.0f, ax3 = ax - 3.0f;
+                    const float u0 = D[0] * ax, u1 = D[1] * ax1, u2 = D[2] * ax2, u3 = D[3] * ax3;
+                    const float m = (D[0] + D[1]) + (D[2] + D[3]);                    // sum d
+                    const float mx = (u0 + u1) + (u2 + u3);                           // sum d dx
+                    const float mxx = __builtin_fmaf(u3, ax3, __builtin_fmaf(u2, ax2, __builtin_fmaf(u1, ax1, u0 * ax)));
+                    const float my = dy * m, myy = dy * my, mxy = dy * mx;
+                    auto against = [&](float g) {  // the row's w against one channel of its pixels' gradients
+                        const f32x4 G = __builtin_amdgcn_mfma_f32_4x4x1f32(g, 1.0f, zero4, 0, 0, 0);
+                        return __builtin_fmaf(W[3], G[3], __builtin_fmaf(W[2], G[2], __builtin_fmaf(W[1], G[1], W[0] * G[0])));
+                    };
+                    const float red = against(g0), green = against(g1), blue = against(g2);
+                    // rows 0..3 end with (sum d, d dy, d dx dy, red), (d dx, d dy^2, green, blue), (d dx^2, depth)
+                    const float sum_a = add_halves<16>(add_halves<32>(m, mxy), add_halves<32>(my, red));
+                    const float sum_b = add_halves<16>(add_halves<32>(mx, green), add_halves<32>(myy, blue));
+                    float sum_c = add_halves<16>(mxx, kDepth ? against(g3) : mxx);
+                    sum_c = add_halves<32>(sum_c, sum_c);
+                    float2* __restrict__ sums = s_sum[wave][k];
+                    float* __restrict__ last = reinterpret_cast<float*>(sums + 4) + (row & 1);
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {  // (two blocks may hold the same entry)
+                        if ((any & (kBlockLanes << (4 * b))) == 0ull) continue;  // (uniform: nothing blended in the block)
+                        if (group == b) {
+                            const float2 v = sums[row];
+                            const float l = *last;
+                            sums[row] = make_float2(v.x + sum_a, v.y + sum_b);
+                            if (row < 2) *last = l + sum_c;
+                        }
+                        wave_lds_sync();
+                    }
                 }
                 if (__ballot(T > 0.0f) == 0ull) break;
             }
         }
         __syncthreads();
         // ---- this batch's records: the moments turned into gradients of position and conic ----
-        if (staging) {
-            const float* __restrict__ m = s_grad + tid * kGradFloats;
-            const float4 a = s_a[tid];
-            const float hz = s_b[tid].x;
-            const float inv_opacity = __builtin_amdgcn_exp2f(-s_b[tid].y);  // s_b.y = log2(opacity)
-            float4* __restrict__ dst = reinterpret_cast<float4*>(key_grads + (size_t)slot * kKeyFloats);
-            // d power / d centre = -(conic_x dx + conic_y dy, conic_z dy + conic_y dx), with conic_x = -2 a.z etc.
-            dst[0] = make_float4(2.0f * a.z * m[0] + a.w * m[1], 2.0f * hz * m[1] + a.w * m[0], -0.5f * m[2], -m[3]);
-            // m[5] = sum of opacity * dL/dopacity over the tile's pixels (zero, not 0 * inf, for a Gaussian that never blended)
-            dst[1] = make_float4(-0.5f * m[4], m[5] != 0.0f ? m[5] * inv_opacity : 0.0f, m[6], m[7]);
-            dst[2] = make_float4(m[8], m[9], 0.f, 0.f);
+        float2 m = make_float2(0.f, 0.f);
+        float l = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            float2* __restrict__ sums = s_sum[w][staged];
+            const float2 v = sums[part];
+            m = make_float2(m.x + v.x, m.y + v.y);
+            sums[part] = make_float2(0.f, 0.f);
+            if (part < 2) {
+                float* __restrict__ last = reinterpret_cast<float*>(sums + 4) + part;
+                l += *last;
+                *last = 0.f;
+            }
+        }
+        const float M = quad_lane<0>(m.x), my = quad_lane<1>(m.x), mxy = quad_lane<2>(m.x), red = quad_lane<3>(m.x);
+        const float green = quad_lane<2>(m.y), blue = quad_lane<3>(m.y), depth = quad_lane<1>(l);
+        if (staged < count && part < 3) {
+            const float hx = s_a[staged].z, ny = s_a[staged].w, hz = s_b[staged].x;
+            float4 v;
+            // d power / d centre = -(conic_x dx + conic_y dy, conic_z dy + conic_y dx), with conic_x = -2 hx etc.
+            if (part == 0)
+                v = make_float4(2.0f * hx * m.y + ny * my, 2.0f * hz * my + ny * m.y, -0.5f * l, -mxy);
+            else if (part == 1)
+                // M = sum of opacity * dL/dopacity over the tile's pixels (zero, not 0 * inf, for a Gaussian that never
+                // blended)
+                v = make_float4(-0.5f * m.y, M != 0.0f ? M * __builtin_amdgcn_exp2f(-s_b[staged].y) : 0.0f, red, green);
+            else
+                v = make_float4(blue, kDepth ? depth : 0.0f, 0.f, 0.f);
+            reinterpret_cast<float4*>(key_grads + (size_t)s_slot[staged] * kKeyFloats)[part] = v;
         }
     }
     // keys the tile never reached (every pixel finished before them) contribute nothing: every record is written
@@ -677,9 +747,14 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     int rc = launch_exclusive_scan(tiles_touched, first_key, (size_t)g.P, scan_tmp, s);
     if (rc) return rc;
     const int tiles = f.grid_x * f.grid_y;
-    hipLaunchKernelGGL(blend_backward_kernel, dim3(tiles), dim3(256), 0, s, f, header, ranges, values, records,
-                       in.image, in.depth, in.alpha, in.dL_dimage, in.dL_ddepth, in.dL_dalpha, rects, first_key,
-                       key_grads);
+    auto blend = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(tiles), dim3(256), 0, s, f, header, ranges, values, records, in.image, in.depth,
+                           in.alpha, in.dL_dimage, in.dL_ddepth, in.dL_dalpha, rects, first_key, key_grads);
+    };
+    if (in.dL_ddepth)
+        blend(blend_backward_kernel<true>);
+    else
+        blend(blend_backward_kernel<false>);
     GS355_CHECK_LAUNCH("blend backward");
     const bool staged = g.shs != nullptr && f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(g.shs) & 15u) == 0 &&
                         (out.shs == nullptr || (reinterpret_cast<uintptr_t>(out.shs) & 15u) == 0);
