@@ -356,6 +356,118 @@ __device__ __forceinline__ void sh_basis_grad(int deg, float x, float y, float z
 
 constexpr int kShStride = 52;  // floats per Gaussian in the SH staging area (16-B reads of 64 lanes on distinct banks)
 
+// A Gaussian's keys are consecutive records; they are added in a fixed order, so the result does not vary between runs.
+// Up to kSerialRecords of them are added by the Gaussian's own lane, four requested at a time (indices past the last
+// one re-read it and are not added).  A Gaussian of more keys would keep its whole wavefront waiting for one lane's
+// chain of requests (a splat of an early training step covers hundreds of tiles: 245 us of kernel for 100k Gaussians,
+// 112 with this), so those are served by all lanes, four Gaussians at a time: sixteen lanes take one, three per record
+// (48 bytes), five records side by side and four such rounds in flight, and the partial sums meet in LDS.
+constexpr uint32_t kSerialRecords = 8;
+// Scenes of few Gaussians leave most of the chip idle even so (a wavefront per 64 Gaussians): up to this many, a kernel
+// of its own gives every Gaussian of more than kSerialRecords keys a wavefront and leaves the sum in its first record
+// (100k Gaussians: 112 -> 67 us for both kernels).  Beyond, the launch of a wavefront per Gaussian costs more.
+constexpr int kSumAheadMax = 1 << 18;
+constexpr int kPartials = 4 * 15;  // float4 of LDS per wavefront
+
+__device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+
+__device__ __forceinline__ void sum_records(const float* __restrict__ key_grads, uint32_t n, uint32_t first,
+                                            float4* __restrict__ partial, float4& A0, float4& A1, float4& A2)
+{
+    const int lane = threadIdx.x & 63, group = lane >> 4, sub = lane & 15;
+    const float4* __restrict__ records = reinterpret_cast<const float4*>(key_grads);
+    A0 = A1 = A2 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (n <= kSerialRecords) {
+        const float4* __restrict__ rec = records + (size_t)first * (kKeyFloats / 4);
+        for (uint32_t k0 = 0; k0 < n; k0 += 4) {
+            float4 r[4][3];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const size_t k = min(k0 + (uint32_t)u, n - 1);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) r[u][q] = rec[3 * k + q];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (k0 + (uint32_t)u < n) {
+                    A0 = add4(A0, r[u][0]);
+                    A1 = add4(A1, r[u][1]);
+                    A2 = add4(A2, r[u][2]);
+                }
+            }
+        }
+    }
+    uint64_t left = __ballot(n > kSerialRecords);
+    const int slot = sub / 3, part = sub % 3;  // (lane 15 of a group has no part)
+    while (left != 0ull) {
+        int lane_of[4], mine = -1;  // the lanes whose Gaussians the four groups take
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            lane_of[g] = left != 0ull ? (int)__ffsll((unsigned long long)left) - 1 : -1;
+            left &= left - 1ull;  // (0 stays 0)
+            mine = group == g ? lane_of[g] : mine;
+        }
+        const uint32_t n_of = (uint32_t)__shfl((int)n, max(mine, 0), 64);
+        const uint32_t first_of = (uint32_t)__shfl((int)first, max(mine, 0), 64);
+        const uint32_t n_mine = mine < 0 || sub == 15 ? 0u : n_of;
+        const float4* __restrict__ rec = records + (size_t)first_of * (kKeyFloats / 4) + part;
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (uint32_t k0 = (uint32_t)slot; k0 < n_mine; k0 += 20) {
+            float4 r[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) r[u] = rec[3 * (size_t)min(k0 + 5u * (uint32_t)u, n_mine - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k0 + 5u * (uint32_t)u < n_mine) sum = add4(sum, r[u]);
+        }
+        if (sub < 15) partial[15 * group + sub] = sum;
+        wave_lds_sync();
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (lane != lane_of[g]) continue;
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                A0 = add4(A0, partial[15 * g + 3 * k]);
+                A1 = add4(A1, partial[15 * g + 3 * k + 1]);
+                A2 = add4(A2, partial[15 * g + 3 * k + 2]);
+            }
+        }
+        wave_lds_sync();
+    }
+}
+
+// Sixteen records side by side, three lanes each, three such rounds in flight; the first record is overwritten once all
+// of them have been read (its new value depends on every one).
+__global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __restrict__ radii,
+                                                        const uint32_t* __restrict__ tiles_touched,
+                                                        const uint32_t* __restrict__ first_key, float* key_grads)
+{
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= P) return;
+    const uint32_t n = radii[i] > 0 ? tiles_touched[i] : 0u;
+    if (n <= kSerialRecords) return;  // (uniform over the wavefront)
+    const int slot = lane / 3, part = lane % 3;
+    float4* rec = reinterpret_cast<float4*>(key_grads) + (size_t)first_key[i] * (kKeyFloats / 4) + part;
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (slot < 16) {
+        for (uint32_t k0 = (uint32_t)slot; k0 < n; k0 += 48) {
+            float4 r[3];
+#pragma unroll
+            for (int u = 0; u < 3; ++u) r[u] = rec[3 * (size_t)min(k0 + 16u * (uint32_t)u, n - 1)];
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (k0 + 16u * (uint32_t)u < n) sum = add4(sum, r[u]);
+        }
+    }
+#pragma unroll
+    for (int d = 24; d >= 3; d >>= 1) {
+        const float4 other = make_float4(__shfl_down(sum.x, d, 64), __shfl_down(sum.y, d, 64), __shfl_down(sum.z, d, 64),
+                                         __shfl_down(sum.w, d, 64));
+        sum = add4(sum, other);  // (lanes past the last slot hold zeros; sums other than the first slot's are not used)
+    }
+    if (slot == 0) rec[0] = sum;
+}
+
 // kMode 0: SH blocks (if any) are read and written by their own lanes.  1 and 2: 16-coefficient blocks, 16-byte
 // aligned, staged through LDS; 2 also fetches the coefficients (needed for degree > 0 only).  kStored: g holds the
 // vanilla model's stored parameters, and the gradients are theirs (activations' derivatives included); the rows of the
@@ -368,11 +480,11 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
                                                                   const uint32_t* __restrict__ tiles_touched,
                                                                   const uint32_t* __restrict__ first_key,
                                                                   const float* __restrict__ key_grads,
-                                                                  gs355_gradients out, ParameterArgs par)
+                                                                  gs355_gradients out, ParameterArgs par, bool summed)
 {
     // Full 16-coefficient SH blocks travel through LDS: each wavefront moves the 12 KB of its 64 Gaussians'
     // coefficients (in) and coefficient gradients (out) with coalesced 16-B accesses; a lane works on its own row.
-    __shared__ float4 s_sh[kMode == 0 ? 1 : 4 * 64 * kShStride / 4];
+    __shared__ float4 s_sh[kMode == 0 ? 4 * kPartials : 4 * 64 * kShStride / 4];
 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < g.P;
@@ -384,7 +496,7 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
     const int count = (int)min((size_t)64, (size_t)g.P > wave_first ? (size_t)g.P - wave_first : (size_t)0);
     constexpr bool staged = kMode != 0, fetch_sh = kMode == 2;
     const int rest_row = 3 * (M - 1);  // floats per Gaussian in par.rest
-    float4* __restrict__ mine = s_sh + (staged ? wave * 64 * (kShStride / 4) : 0);
+    float4* __restrict__ mine = s_sh + wave * (staged ? 64 * (kShStride / 4) : kPartials);
     float* __restrict__ my_row = reinterpret_cast<float*>(mine) + (staged ? lane * (kStored ? rest_row : kShStride) : 0);
 
     float dmean[3] = {0.f, 0.f, 0.f}, d2[3] = {0.f, 0.f, 0.f}, dscale[3] = {0.f, 0.f, 0.f};
@@ -394,33 +506,14 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
     float nx = 0.f, ny = 0.f, nz = 0.f, inv_len = 0.f;
     float bx[16], by[16], bz[16];
     int K = 0;
+    uint32_t n_keys = alive ? tiles_touched[si] : 0u;
+    const uint32_t first_record = alive ? first_key[si] : 0u;
+    if (summed && n_keys > kSerialRecords) n_keys = 1u;  // (sum_large_kernel has added them into the first)
+    float4 A0, A1, A2;
+    sum_records(key_grads, n_keys, first_record, mine, A0, A1, A2);
     if (alive) {
         const float* __restrict__ V = f.viewmatrix;
         const float* __restrict__ Pm = f.projmatrix;
-        // the Gaussian's keys are consecutive records; summed in order, so the result does not vary between runs.
-        // Four records are requested at a time (indices past the last one re-read it and are not added).
-        float4 A0 = make_float4(0.f, 0.f, 0.f, 0.f), A1 = A0, A2 = A0;
-        {
-            const float4* __restrict__ rec = reinterpret_cast<const float4*>(key_grads + (size_t)first_key[si] * kKeyFloats);
-            const uint32_t n = tiles_touched[si];
-            for (uint32_t k0 = 0; k0 < n; k0 += 4) {
-                float4 r[4][3];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const size_t k = min(k0 + (uint32_t)u, n - 1);
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) r[u][q] = rec[3 * k + q];
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (k0 + (uint32_t)u < n) {
-                        A0.x += r[u][0].x; A0.y += r[u][0].y; A0.z += r[u][0].z; A0.w += r[u][0].w;
-                        A1.x += r[u][1].x; A1.y += r[u][1].y; A1.z += r[u][1].z; A1.w += r[u][1].w;
-                        A2.x += r[u][2].x; A2.y += r[u][2].y;
-                    }
-                }
-            }
-        }
         const float g_px = A0.x, g_py = A0.y, gA = A0.z, gB = A0.w, gC = A1.x;
         dop = A1.y;
         dcol[0] = A1.z; dcol[1] = A1.w; dcol[2] = A2.x;
@@ -759,8 +852,15 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     const bool staged = g.shs != nullptr && f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(g.shs) & 15u) == 0 &&
                         (out.shs == nullptr || (reinterpret_cast<uintptr_t>(out.shs) & 15u) == 0);
     const dim3 grid((g.P + 255) / 256), block(256);
+    const bool summed = g.P <= kSumAheadMax;
+    if (summed) {
+        hipLaunchKernelGGL(sum_large_kernel, dim3((g.P + 3) / 4), dim3(256), 0, s, g.P, in.radii, tiles_touched, first_key,
+                           key_grads);
+        GS355_CHECK_LAUNCH("record sums");
+    }
     auto launch = [&](auto kernel, const ParameterArgs& p) {
-        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, tiles_touched, first_key, key_grads, out, p);
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, tiles_touched, first_key, key_grads, out, p,
+                           summed);
     };
     if (par) {
         if ((reinterpret_cast<uintptr_t>(par->rest) & 15u) != 0 || (reinterpret_cast<uintptr_t>(par->d_rest) & 15u) != 0)
