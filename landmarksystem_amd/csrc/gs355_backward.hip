@@ -474,7 +474,7 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __
 // SH coefficients behind the first are then staged back to back, 3 (M - 1) floats each, as they lie in memory: a
 // wavefront's 64 rows start on a 256-B boundary whatever their length.
 template <int kMode, bool kStored>
-__global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, gs355_gaussians g,
+__global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kernel(FrameArgs f, gs355_gaussians g,
                                                                   const int32_t* __restrict__ radii,
                                                                   const float* __restrict__ records,
                                                                   const uint32_t* __restrict__ tiles_touched,
@@ -484,7 +484,12 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
 {
     // Full 16-coefficient SH blocks travel through LDS: each wavefront moves the 12 KB of its 64 Gaussians'
     // coefficients (in) and coefficient gradients (out) with coalesced 16-B accesses; a lane works on its own row.
-    __shared__ float4 s_sh[kMode == 0 ? 4 * kPartials : 4 * 64 * kShStride / 4];
+    // (kStored: rows of at most 45 floats back to back, filled by whole-wavefront copies of 1 KB, twelve at most)
+    constexpr int kWaveRows = kMode == 0 ? 0 : kStored ? 12 * 64 : 64 * kShStride / 4;  // float4 per wavefront
+    // the partial record sums have their place behind the rows where those may be in flight, else inside them
+    constexpr int kPartialsAt = kStored ? kWaveRows : 0;
+    constexpr int kWaveLds = kPartialsAt + kPartials > kWaveRows ? kPartialsAt + kPartials : kWaveRows;
+    __shared__ float4 s_sh[4 * kWaveLds];
 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < g.P;
@@ -496,21 +501,54 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
     const int count = (int)min((size_t)64, (size_t)g.P > wave_first ? (size_t)g.P - wave_first : (size_t)0);
     constexpr bool staged = kMode != 0, fetch_sh = kMode == 2;
     const int rest_row = 3 * (M - 1);  // floats per Gaussian in par.rest
-    float4* __restrict__ mine = s_sh + wave * (staged ? 64 * (kShStride / 4) : kPartials);
+    float4* __restrict__ mine = s_sh + wave * kWaveLds;
     float* __restrict__ my_row = reinterpret_cast<float*>(mine) + (staged ? lane * (kStored ? rest_row : kShStride) : 0);
 
     float dmean[3] = {0.f, 0.f, 0.f}, d2[3] = {0.f, 0.f, 0.f}, dscale[3] = {0.f, 0.f, 0.f};
     float drot[4] = {0.f, 0.f, 0.f, 0.f}, dcov[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, dcol[3] = {0.f, 0.f, 0.f};
     float dop = 0.f;
-    float b[16], gcol[3] = {0.f, 0.f, 0.f};
+    float gcol[3] = {0.f, 0.f, 0.f};
     float nx = 0.f, ny = 0.f, nz = 0.f, inv_len = 0.f;
-    float bx[16], by[16], bz[16];
     int K = 0;
     uint32_t n_keys = alive ? tiles_touched[si] : 0u;
     const uint32_t first_record = alive ? first_key[si] : 0u;
     if (summed && n_keys > kSerialRecords) n_keys = 1u;  // (sum_large_kernel has added them into the first)
+    // kStored: the wavefront's rows as one run of float4, and the up to three floats behind the last whole one.  They
+    // travel from memory to LDS without passing through registers, requested before anything else is waited for: held
+    // in registers the 48 of them left two wavefronts per SIMD, requested later their latency came on top of the
+    // records' (6M Gaussians: 1.10 -> 0.76 ms, 3.5 GB at the rate of a large copy).
+    const int run4 = kStored ? count * rest_row / 4 : 0, run_tail = kStored ? count * rest_row % 4 : 0;
+    const size_t run_first = wave_first * (size_t)rest_row;
+    float tail = 0.f;
+    if (fetch_sh && kStored) {
+        typedef __attribute__((address_space(1))) const void global_void;
+        typedef __attribute__((address_space(3))) void lds_void;
+        const float4* src = reinterpret_cast<const float4*>(par.rest + run_first);
+#pragma unroll
+        for (int it = 0; it < 12; ++it)
+            if (it * 64 + lane < run4)  // (lane l of a copy writes float4 l behind the uniform LDS address)
+                __builtin_amdgcn_global_load_lds((global_void*)(src + it * 64 + lane), (lds_void*)(mine + it * 64), 16, 0, 0);
+        if (lane < run_tail) tail = par.rest[run_first + 4 * run4 + lane];
+    }
+    // the Gaussian's own inputs are requested before its records are waited for, too
+    float in_mean[3] = {0.f, 0.f, 0.f}, in_scale[3] = {0.f, 0.f, 0.f}, in_rot[4] = {0.f, 0.f, 0.f, 0.f};
+    float in_opacity = 0.f, in_rgb[3] = {0.f, 0.f, 0.f};
+    if (alive) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) in_mean[k] = g.means3D[3 * si + k];
+        if (kStored || !g.cov3D_precomp) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) in_scale[k] = g.scales[3 * si + k];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) in_rot[k] = g.rotations[4 * si + k];
+        }
+        if (kStored) in_opacity = g.opacities[si];
+        if (g.shs)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) in_rgb[c] = records[si * kRecordFloats + 6 + c];
+    }
     float4 A0, A1, A2;
-    sum_records(key_grads, n_keys, first_record, mine, A0, A1, A2);
+    sum_records(key_grads, n_keys, first_record, mine + kPartialsAt, A0, A1, A2);
     if (alive) {
         const float* __restrict__ V = f.viewmatrix;
         const float* __restrict__ Pm = f.projmatrix;
@@ -518,7 +556,7 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
         dop = A1.y;
         dcol[0] = A1.z; dcol[1] = A1.w; dcol[2] = A2.x;
         const float g_depth = A2.y;
-        const float x = g.means3D[3 * si], y = g.means3D[3 * si + 1], z = g.means3D[3 * si + 2];
+        const float x = in_mean[0], y = in_mean[1], z = in_mean[2];
 
         // ---- pixel position ----
         const float phx = Pm[0] * x + Pm[4] * y + Pm[8] * z + Pm[12];
@@ -539,21 +577,19 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
         // the kernel waits for memory, so the chain costs nothing in double and loses nothing.
         typedef double real;
         real S[6], s[3] = {0., 0., 0.}, q[4] = {0., 0., 0., 0.}, R[3][3] = {};
-        float stored_q[4], norm = 1.f;
+        float norm = 1.f;
         if (!kStored && g.cov3D_precomp) {
 #pragma unroll
             for (int k = 0; k < 6; ++k) S[k] = g.cov3D_precomp[6 * si + k];
         } else {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const float v = g.scales[3 * si + k];
+                const float v = in_scale[k];
                 s[k] = (real)f.scale_modifier * (real)(kStored ? expf(v) : v);
             }
+            if (kStored) norm = quaternion_norm(in_rot);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) stored_q[k] = g.rotations[4 * si + k];
-            if (kStored) norm = quaternion_norm(stored_q);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) q[k] = kStored ? stored_q[k] / norm : stored_q[k];
+            for (int k = 0; k < 4; ++k) q[k] = kStored ? in_rot[k] / norm : in_rot[k];
             const real r = q[0], qx = q[1], qy = q[2], qz = q[3];
             R[0][0] = 1. - 2. * (qy * qy + qz * qz); R[0][1] = 2. * (qx * qy - r * qz); R[0][2] = 2. * (qx * qz + r * qy);
             R[1][0] = 2. * (qx * qy + r * qz); R[1][1] = 1. - 2. * (qx * qx + qz * qz); R[1][2] = 2. * (qy * qz - r * qx);
@@ -668,7 +704,7 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
             }
         }
         if (kStored) {
-            const float o = logistic(g.opacities[si]);
+            const float o = logistic(in_opacity);
             dop = dop * ((1.0f - o) * o);
         }
 
@@ -679,33 +715,19 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
             nx = dirx * inv_len;
             ny = diry * inv_len;
             nz = dirz * inv_len;
-            sh_basis_grad(f.sh_degree, nx, ny, nz, b, bx, by, bz);
             K = (f.sh_degree + 1) * (f.sh_degree + 1);
             // the forward pass clamped the colour at zero: a zero in the record means no gradient
-            const float* __restrict__ rec = records + si * kRecordFloats;
-            gcol[0] = rec[6] > 0.0f ? dcol[0] : 0.0f;
-            gcol[1] = rec[7] > 0.0f ? dcol[1] : 0.0f;
-            gcol[2] = rec[8] > 0.0f ? dcol[2] : 0.0f;
+            gcol[0] = in_rgb[0] > 0.0f ? dcol[0] : 0.0f;
+            gcol[1] = in_rgb[1] > 0.0f ? dcol[1] : 0.0f;
+            gcol[2] = in_rgb[2] > 0.0f ? dcol[2] : 0.0f;
         }
     }
 
     // ---- SH coefficients: their part of the mean's gradient (through the view direction), and their own ----
     if (g.shs) {
-        // kStored: the wavefront's rows as one run of float4, and the up to three floats behind the last whole one
-        const int run4 = kStored ? count * rest_row / 4 : 0, run_tail = kStored ? count * rest_row % 4 : 0;
-        const size_t run_first = wave_first * (size_t)rest_row;
         if (fetch_sh && kStored) {
-            float4 sh_in[12];
-            const float4* __restrict__ src = reinterpret_cast<const float4*>(par.rest + run_first);
-            if (run4 > 0) {  // (uniform over the wavefront)
-#pragma unroll
-                for (int it = 0; it < 12; ++it)
-                    if (it * 64 < run4) sh_in[it] = src[min(it * 64 + lane, run4 - 1)];  // (uniform)
-#pragma unroll
-                for (int it = 0; it < 12; ++it)
-                    if (it * 64 + lane < run4) mine[it * 64 + lane] = sh_in[it];
-            }
-            if (lane < run_tail) reinterpret_cast<float*>(mine)[4 * run4 + lane] = par.rest[run_first + 4 * run4 + lane];
+            if (lane < run_tail) reinterpret_cast<float*>(mine)[4 * run4 + lane] = tail;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies have landed
             wave_lds_sync();
         } else if (fetch_sh) {
             // coefficients of the wavefront's Gaussians: all loads in flight together, then into the rows (slots
@@ -724,6 +746,10 @@ __global__ __launch_bounds__(256) void preprocess_backward_kernel(FrameArgs f, g
             }
             wave_lds_sync();
         }
+        // (the basis is evaluated after the coefficients have arrived: its 64 values held across the wait would cost a
+        // wavefront per SIMD)
+        float b[16], bx[16], by[16], bz[16];
+        sh_basis_grad(f.sh_degree, nx, ny, nz, b, bx, by, bz);
         if (alive && f.sh_degree > 0) {
             constexpr int kSkip = kStored ? 3 : 0;  // (the first coefficient is stored apart)
             const float* __restrict__ sh = staged ? my_row : kStored ? par.rest + si * rest_row : g.shs + si * M * 3;
