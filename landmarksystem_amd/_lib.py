@@ -25,12 +25,14 @@ PIPELINE_FAST = STAGE_PREPROCESS | STAGE_TILE_COUNT | STAGE_TILE_SCATTER | STAGE
 MAX_FAST_TILES = 36000 * 16  # limits of the tile-bucketed stages (the classic stages have neither)
 MAX_FAST_GAUSSIANS = 1 << 28
 DECODE_COUNT, DECODE_EMIT, DECODE_ALL = 1, 2, 3
+TRAIN_ROWS, TRAIN_INPUTS, TRAIN_COUNT, TRAIN_EMIT = 1, 2, 4, 8
 
 EXPORTS = ("gs355_version", "gs355_last_error", "gs355_workspace_layout", "gs355_run", "gs355_render",
            "gs355_visible_filter", "gs355_anchor_filter", "gs355_decode_scratch_bytes", "gs355_decode_count",
            "gs355_decode_count_static", "gs355_decode_emit", "gs355_decode_workspace_bytes", "gs355_decode",
            "gs355_backward_scratch_bytes", "gs355_render_backward", "gs355_gather_scratch_bytes", "gs355_gather_rows",
-           "gs355_run_parameters", "gs355_render_parameters_backward")
+           "gs355_run_parameters", "gs355_render_parameters_backward", "gs355_decode_train_bytes", "gs355_decode_train",
+           "gs355_decode_train_backward")
 GATHER_MAX_ARRAYS, GATHER_MAX_ROW_BYTES = 8, 4096
 
 
@@ -148,6 +150,20 @@ class Decoded(C.Structure):
                 ("neural_opacity", C.c_void_p), ("mask", C.c_void_p)]
 
 
+class TrainRows(C.Structure):
+    _fields_ = [("num_visible", C.c_int32), ("compact_feat", C.c_int32), ("with_dist", C.c_void_p), ("without", C.c_void_p),
+                ("hidden", C.c_void_p * 3), ("pre", C.c_void_p * 3)]
+
+
+class DecodeCotangents(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("xyz", "color", "opacity", "scaling", "rot", "neural_opacity")]
+
+
+class DecodeGradients(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("anchor", "feat", "offset", "scaling")] + [
+        (n, C.c_void_p * 3) for n in ("w0", "b0", "w1", "b1")]
+
+
 class AnchorLod(C.Structure):
     _fields_ = [("level", C.c_void_p), ("extra_level", C.c_void_p), ("voxel_size", C.c_float),
                 ("standard_dist", C.c_float), ("fork", C.c_float), ("resolution_scale", C.c_float),
@@ -216,6 +232,15 @@ def load() -> C.CDLL:
     lib.gs355_decode.argtypes = [C.POINTER(Decoder), C.POINTER(Anchors), C.c_int64, C.POINTER(Decoded), C.c_void_p,
                                  C.c_size_t, C.c_uint32, C.c_void_p]
     lib.gs355_decode.restype = C.c_int
+    lib.gs355_decode_train_bytes.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+    lib.gs355_decode_train_bytes.restype = C.c_int
+    lib.gs355_decode_train.argtypes = [C.POINTER(Decoder), C.POINTER(Anchors), C.POINTER(TrainRows), C.c_int64,
+                                       C.POINTER(Decoded), C.c_void_p, C.c_size_t, C.c_uint32, C.c_void_p]
+    lib.gs355_decode_train.restype = C.c_int
+    lib.gs355_decode_train_backward.argtypes = [C.POINTER(Decoder), C.POINTER(Anchors), C.POINTER(TrainRows), C.c_void_p, C.c_size_t,
+                                                C.POINTER(DecodeCotangents), C.POINTER(DecodeGradients), C.c_void_p,
+                                                C.c_size_t, C.c_void_p]
+    lib.gs355_decode_train_backward.restype = C.c_int
     lib.gs355_backward_scratch_bytes.argtypes = [C.c_int32, C.c_int64, C.POINTER(C.c_size_t)]
     lib.gs355_backward_scratch_bytes.restype = C.c_int
     lib.gs355_render_backward.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_void_p, C.c_size_t, C.c_int64,

@@ -34,6 +34,7 @@ from typing import NamedTuple, Optional
 
 import torch
 from torch import nn
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 
@@ -95,6 +96,97 @@ class _TallLinear(torch.autograd.Function):
                 dw += dy[whole:].t() @ x[whole:]
         db = dy.sum(dim=0) if ctx.needs_input_grad[2] else None
         return dx, dw, db
+
+
+class _DecodeTrain(torch.autograd.Function):
+    """The training decode around its matrix products (gs355_decode_train) with its whole backward pass in the kernels
+    (gs355_decode_train_backward): differentiable with respect to anchors, features, offsets, scales and the heads'
+    parameters.  The products going forward are the module's own (torch.addmm), so the Gaussians are bit for bit those
+    of its statements.  Workspace, input rows, hidden units and pre-activations live until the graph is dropped."""
+
+    @staticmethod
+    def forward(ctx, decoder, camera_center, visible, level, compact_feat, anchor, feat, offset, scaling, *params):
+        dev, A, n = anchor.device, anchor.shape[0], decoder.n_offsets
+        lib = _lib.load()
+        stream = torch.cuda.current_stream(dev)
+        dec, an = decoder._train_structs(camera_center, visible, level, anchor, feat, offset, scaling, params)
+        need, scratch = C.c_size_t(), C.c_size_t()
+        _lib.check(lib.gs355_decode_train_bytes(A, 0, n, C.byref(need), C.byref(scratch)))
+        f = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)  # noqa: E731
+        ws = torch.empty(need.value, dtype=torch.uint8, device=dev)
+        if decoder._host_count is None:
+            decoder._host_count = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+        counts = decoder._host_count  # (pinned: the kernels' stores land there, nothing is copied)
+        o, rows = _lib.Decoded(), _lib.TrainRows()
+        o.count, o.num_visible = counts.data_ptr(), counts.data_ptr() + 4
+
+        def run(phase, capacity=0):
+            _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), capacity, C.byref(o),
+                                              ws.data_ptr(), ws.numel(), phase, stream.cuda_stream))
+
+        run(_lib.TRAIN_ROWS)
+        stream.synchronize()
+        V = int(counts[1])
+        widths = [params[4 * j].shape[1] for j in range(3)]
+        with_dist = f(V, 36) if 36 in widths else None
+        without = f(V, 35) if 35 in widths else None
+        rows.num_visible, rows.compact_feat = V, 1 if compact_feat else 0
+        rows.with_dist = None if with_dist is None else with_dist.data_ptr()
+        rows.without = None if without is None else without.data_ptr()
+        run(_lib.TRAIN_INPUTS)
+        hidden, pre = [], []
+        for j in range(3):
+            w0, b0, w1, b1 = params[4 * j:4 * j + 4]
+            hidden.append(torch.addmm(b0, with_dist if widths[j] == 36 else without, w0.t()).relu_())
+            pre.append(torch.addmm(b1, hidden[j], w1.t()))
+            rows.hidden[j], rows.pre[j] = hidden[j].data_ptr(), pre[j].data_ptr()
+            if j == 0:  # (the number of Gaussians is on its way while the other heads run)
+                run(_lib.TRAIN_COUNT)
+                counted = torch.cuda.Event()
+                counted.record(stream)
+        counted.synchronize()
+        G = int(counts[0])
+        out = (f(G, 3), f(G, 3), f(G, 1), f(G, 3), f(G, 4), f(V * n, 1), torch.empty(V * n, dtype=torch.bool, device=dev))
+        if G > 0:
+            o.xyz, o.color, o.opacity, o.scaling, o.rot = (t.data_ptr() for t in out[:5])
+        o.neural_opacity, o.mask = out[5].data_ptr(), out[6].data_ptr()
+        run(_lib.TRAIN_EMIT, G)
+        ctx.decoder, ctx.num_visible, ctx.workspace, ctx.compact_feat = decoder, V, ws, compact_feat
+        ctx.rows = (with_dist, without, hidden, pre)
+        ctx.save_for_backward(camera_center, visible, level, anchor, feat, offset, scaling, *params)
+        ctx.mark_non_differentiable(out[6])
+        ctx.set_materialize_grads(False)
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural, _g_mask):
+        camera_center, visible, level, anchor, feat, offset, scaling, *params = ctx.saved_tensors
+        dev, A, V = anchor.device, anchor.shape[0], ctx.num_visible
+        lib = _lib.load()
+        ptr = lambda t: None if t is None or t.numel() == 0 else t.data_ptr()  # noqa: E731
+        dec, an = ctx.decoder._train_structs(camera_center, visible, level, anchor, feat, offset, scaling, params)
+        with_dist, without, hidden, pre = ctx.rows
+        rows = _lib.TrainRows(V, 1 if ctx.compact_feat else 0, ptr(with_dist), ptr(without))
+        for j in range(3):
+            rows.hidden[j], rows.pre[j] = ptr(hidden[j]), ptr(pre[j])
+        given = [None if g is None else g.contiguous() for g in (g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural)]
+        cot = _lib.DecodeCotangents(*[ptr(g) for g in given])
+        # (anchors that were not decoded have no gradient: their rows stay zero)
+        new = torch.empty_like if V == A else torch.zeros_like
+        wanted = ctx.needs_input_grad[5:]
+        grads = [new(t) if w else None for t, w in zip((anchor, feat, offset, scaling), wanted)]
+        grads += [torch.empty_like(p) if w else None for p, w in zip(params, wanted[4:])]
+        out = _lib.DecodeGradients(*[ptr(t) for t in grads[:4]])
+        for j in range(3):
+            out.w0[j], out.b0[j], out.w1[j], out.b1[j] = (ptr(t) for t in grads[4 + 4 * j:8 + 4 * j])
+        need, scratch_bytes = C.c_size_t(), C.c_size_t()
+        _lib.check(lib.gs355_decode_train_bytes(A, V, ctx.decoder.n_offsets, C.byref(need), C.byref(scratch_bytes)))
+        scratch = torch.empty(scratch_bytes.value // 4, dtype=torch.float32, device=dev)
+        _lib.check(lib.gs355_decode_train_backward(C.byref(dec), C.byref(an), C.byref(rows), ctx.workspace.data_ptr(),
+                                                   ctx.workspace.numel(), C.byref(cot), C.byref(out), scratch.data_ptr(),
+                                                   scratch.numel() * 4, torch.cuda.current_stream(dev).cuda_stream))
+        return (None, None, None, None, None, *grads)
 
 
 def _mlp(seq, x):
@@ -296,12 +388,58 @@ class FusedAnchorDecoder(nn.Module):
         with torch.no_grad():
             return self._forward_kernels(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
 
+    def _head_parameters(self):
+        return [t for m in (self.mlp_opacity, self.mlp_cov, self.mlp_color)
+                for t in (m[0].weight, m[0].bias, m[2].weight, m[2].bias)]
+
+    def _train_structs(self, camera_center, visible, level, anchor, feat, offset, scaling, params):
+        d = _lib.Decoder()
+        d.feat_dim, d.n_offsets = self.feat_dim, self.n_offsets
+        for j in range(3):
+            w0, b0, w1, b1 = params[4 * j:4 * j + 4]
+            d.in_dim[j] = w0.shape[1]
+            d.w0[j], d.b0[j], d.w1[j], d.b1[j] = w0.data_ptr(), b0.data_ptr(), w1.data_ptr(), b1.data_ptr()
+        d.add_level = 1 if self.add_level else 0
+        an = _lib.Anchors()
+        an.A = anchor.shape[0]
+        an.anchor, an.feat, an.offset, an.scaling = (t.data_ptr() for t in (anchor, feat, offset, scaling))
+        an.campos, an.visible_mask = camera_center.data_ptr(), visible.data_ptr()
+        an.level = None if level is None else level.data_ptr()
+        return d, an
+
+    def _bank_mix(self, feat, view, level):
+        """The feature bank (anchor_decoder.py:163-177): a softmax-weighted mix of strided copies of the features."""
+        w = _mlp(self.mlp_feature_bank, view if level is None else torch.cat([view, level], dim=1))  # softmax inside
+        return feat[:, ::4].repeat(1, 4) * w[:, 0:1] + feat[:, ::2].repeat(1, 2) * w[:, 1:2] + feat * w[:, 2:3]
+
     def _forward_differentiable(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level):
-        """The statements of the reference module (anchor_decoder.py:147-242) as torch operations, for autograd:
-        same 7-tuple, the training by-products always present."""
+        """The training decode: same 7-tuple, the training by-products always present.  In the kernels, forward and
+        backward, where every tensor is as they read it (fp32, contiguous, on one GPU; camera and level not
+        differentiated); else the statements of the reference module as torch operations."""
         level = self._check_level(level, anchor.shape[0])
         if visible_mask is None:
             visible_mask = torch.ones(anchor.shape[0], dtype=torch.bool, device=anchor.device)
+        params = self._head_parameters()
+        dev = anchor.device
+        camera_center = camera_center.to(dev)
+        tensors = [anchor, anchor_feat, offset, scaling, camera_center] + params + ([] if level is None else [level])
+        if (dev.type == "cuda" and anchor.shape[0] > 0 and visible_mask.dtype == torch.bool and visible_mask.device == dev
+                and all(t.device == dev and t.dtype == torch.float32 and t.is_contiguous() for t in tensors)
+                and anchor_feat.data_ptr() % 16 == 0 and not camera_center.requires_grad
+                and not (level is not None and level.requires_grad)):
+            feat = anchor_feat
+            if self.use_feat_bank:  # (mixed features of the visible anchors, one row each)
+                rows = visible_mask.nonzero(as_tuple=True)[0]
+                view = anchor.index_select(0, rows) - camera_center
+                view = view / view.norm(dim=1, keepdim=True)
+                feat = self._bank_mix(anchor_feat.index_select(0, rows), view,
+                                      None if level is None else level.reshape(-1, 1).index_select(0, rows))
+            return _DecodeTrain.apply(self, camera_center, visible_mask.contiguous(), level, self.use_feat_bank, anchor,
+                                      feat, offset, scaling, *params)
+        return self._forward_torch(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
+
+    def _forward_torch(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level):
+        """The statements of the reference module (anchor_decoder.py:147-242) as torch operations, for autograd."""
         # Rows are selected with index_select over index lists computed once, not with boolean masks: the results
         # are the same tensors, but the backward of a boolean-mask index is a sorting index_put (3.7 ms per step at
         # 500k anchors), that of index_select an index_add.
@@ -312,8 +450,7 @@ class FusedAnchorDecoder(nn.Module):
         view = view / dist
         lvl = level.reshape(-1, 1).index_select(0, rows).to(feat.dtype) if level is not None else None
         if self.use_feat_bank:
-            w = _mlp(self.mlp_feature_bank, view if lvl is None else torch.cat([view, lvl], dim=1))  # softmax inside
-            feat = feat[:, ::4].repeat(1, 4) * w[:, 0:1] + feat[:, ::2].repeat(1, 2) * w[:, 1:2] + feat * w[:, 2:3]
+            feat = self._bank_mix(feat, view, lvl)
         if lvl is not None:  # (:181-182: both inputs become [feat | view | level])
             with_dist = without = torch.cat([feat, view, lvl], dim=1)
         else:

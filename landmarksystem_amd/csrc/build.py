@@ -35,6 +35,7 @@ SOURCES = [
     ("gs355_bin.hip", []),
     ("gs355_gather.hip", []),
     ("gs355_decode.hip", []),
+    ("gs355_decode_train.hip", ["-ffp-contract=off"]),
     ("gs355_blend.hip", []),
     # (matrix results in ordinary registers: the blend's backward reads them with vector instructions right away)
     ("gs355_backward.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form"]),

@@ -699,7 +699,7 @@ struct DecodeLaunch {
     DecodeArgs args;
 };
 
-static int fill_args(const gs355_decoder* dec, const gs355_anchors* an, bool allow_bank, DecodeArgs* out)
+int check_decoder(const gs355_decoder* dec, const gs355_anchors* an)
 {
     if (!dec || !an) return set_error(GS355_EINVAL, "decoder / anchors is NULL");
     if (dec->feat_dim != kFeat)
@@ -722,7 +722,6 @@ static int fill_args(const gs355_decoder* dec, const gs355_anchors* an, bool all
             return set_error(GS355_EINVAL, "head %d: weight or bias pointer is NULL", j);
     }
     if (dec->bank_in_dim != 0) {
-        if (!allow_bank) return set_error(GS355_EINVAL, "the feature bank is supported by gs355_decode only");
         if (dec->bank_in_dim != 3 && dec->bank_in_dim != 4)
             return set_error(GS355_EINVAL, "bank_in_dim must be 0, 3 or 4 (got %d)", dec->bank_in_dim);
         if (!dec->bank_w0 || !dec->bank_b0 || !dec->bank_w1 || !dec->bank_b1)
@@ -734,6 +733,15 @@ static int fill_args(const gs355_decoder* dec, const gs355_anchors* an, bool all
         return set_error(GS355_EINVAL, "anchors.level is NULL but the decoder takes the level as an input");
     if (an->A > 0 && (reinterpret_cast<uintptr_t>(an->feat) & 15u) != 0)
         return set_error(GS355_EINVAL, "anchor features must be 16-byte aligned");
+    return GS355_OK;
+}
+
+static int fill_args(const gs355_decoder* dec, const gs355_anchors* an, bool allow_bank, DecodeArgs* out)
+{
+    if (dec && dec->bank_in_dim != 0 && !allow_bank)
+        return set_error(GS355_EINVAL, "the feature bank is supported by gs355_decode only");
+    const int rc = check_decoder(dec, an);
+    if (rc) return rc;
     DecodeArgs a;
     a.A = an->A;
     a.n = dec->n_offsets;
@@ -758,6 +766,14 @@ static int fill_args(const gs355_decoder* dec, const gs355_anchors* an, bool all
     a.neural_opacity = nullptr;
     a.kept_mask = nullptr;
     *out = a;
+    return GS355_OK;
+}
+
+int launch_run_scan(const uint2* totals, uint2* base, uint32_t runs, uint32_t* num_emitted, uint32_t* num_visible,
+                    hipStream_t s)
+{
+    hipLaunchKernelGGL(run_scan_kernel, dim3(1), dim3(1024), 0, s, totals, base, runs, num_emitted, num_visible);
+    GS355_CHECK_LAUNCH("decode: run scan");
     return GS355_OK;
 }
 
@@ -994,9 +1010,7 @@ int gs355_decode(const gs355_decoder* dec, const gs355_anchors* an, int64_t capa
         a.run_totals = reinterpret_cast<uint2*>(ws + L.run_totals);
         launch_decode(true, 1024, s, a, nullptr, nullptr, 0u, nullptr);
         GS355_CHECK_LAUNCH("decode: count");
-        hipLaunchKernelGGL(run_scan_kernel, dim3(1), dim3(1024), 0, s, a.run_totals, run_base, runs, out->count,
-                           out->num_visible);
-        GS355_CHECK_LAUNCH("decode: run scan");
+        if ((rc = launch_run_scan(a.run_totals, run_base, runs, out->count, out->num_visible, s))) return rc;
     }
     if (!do_emit) return GS355_OK;
     if (capacity == 0 && !out->neural_opacity && !out->mask) return GS355_OK;

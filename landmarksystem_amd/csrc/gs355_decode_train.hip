@@ -1,0 +1,755 @@
+// The anchor decode as training differentiates it (landmark/nerf_components/model_components/fields/
+// anchor_decoder.py:147-242 under autograd; benchmarks/nerf/scaffold_gs/gs_trainer.py): everything around the heads'
+// matrix products going forward, and all of it going back, in fp32.
+//
+//   rows      visible anchors per run of 128 and (scan) their ranks
+//   inputs    the list of visible anchors and the heads' input rows [feat | view | dist or level]
+//   (caller)  the heads' products, hidden = relu(W0 x + b0) and W1 hidden + b1
+//   count     kept offsets (opacity pre-activation > 0) per group of 32 rows and (scan) their output slots
+//   emit      activations and compaction of the kept offsets
+//   items     backward: cotangents of the outputs to those of the pre-activations, gradients of offsets and scales
+//   layers    backward: a wavefront takes 32 rows at a time back through the layers to the features (and view directions),
+//             the products of the weight gradients accumulated in registers over all of its tiles
+//   sum       the workgroups' weight gradients added up in a fixed order
+//
+// The forward products stay with the caller because a scene's opacities saturate: an anchor far from the camera has
+// pre-activations of a hundred, and one more rounding in them moves the few unsaturated Gaussians across the rasterizer's
+// thresholds.  Every operation here rounds as the framework's own does (this file is compiled without contraction), so
+// the Gaussians are bit for bit those of the module's statements.
+//
+// Backward, everything is transposed as in the inference decode: weights are the left operand of v_mfma_f32_32x32x2_f32
+// (rows = units), anchors the columns, and the accumulator of one layer (lane = anchor, registers = units
+// 8 b + 4 half + t) is the next product's right operand register by register, the weights being read in that order.  One
+// matrix instruction takes 64 cycles, so its left operand comes from LDS, one dword per lane, rows of odd stride.
+//
+// As torch operations the backward pass alone was some thirty launches of skinny matrix products, index and reduction
+// kernels.  At 200k anchors with ten offsets, most of them visible, a training step at 1080p went from 3.01 to 1.59 ms.
+#include "gs355_internal.h"
+
+namespace gs355 {
+
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+constexpr int kFeat = 32;
+constexpr int kRun = 128;           // anchors per run, as in the inference decode
+constexpr int kW0Stride = 37;       // 36 inputs (35-wide heads: zero weight) and, in gradients, the bias
+constexpr int kW1Stride = 33;       // 32 hidden units and, in gradients, the bias
+constexpr int kRows = 112;          // outputs of the three heads, 11 n <= 110, padded
+constexpr int kGroup = 32;          // rows per group of the kept offsets
+constexpr int kMaxOffsets = 10;
+
+struct TrainArgs {
+    int A, n;
+    uint32_t V;            // rows (visible anchors)
+    int in_dim[3];
+    const float* anchor;
+    const float* feat;     // [A,32], or [V,32] with compact_feat
+    const float* offset;
+    const float* scaling;
+    const uint8_t* visible;
+    const float* campos;
+    const float* level;    // replaces the distance
+    int compact_feat;
+    const float* w0[3];
+    const float* w1[3];
+    float* with_dist;      // [V,36] input rows, or NULL
+    float* without;        // [V,35] input rows, or NULL
+    const float* hidden[3];  // [V,32]
+    const float* pre[3];     // [V,n] [V,7n] [V,3n] pre-activations
+};
+
+// The heads' weights in LDS (and, in the same shape, a workgroup's gradients of them with the biases' in the last
+// columns).  Outputs are numbered through the heads: opacity [0, n), covariance [n, 8 n), colour [8 n, 11 n).
+struct HeadParameters {
+    float w0[3][32 * kW0Stride];
+    float w1[kRows * kW1Stride];
+};
+constexpr int kGradFloats = 3 * 32 * kW0Stride + kRows * kW1Stride;
+
+__device__ __forceinline__ int head_of(int o, int n) { return o < n ? 0 : o < 8 * n ? 1 : 2; }
+__device__ __forceinline__ int head_base(int j, int n) { return j == 0 ? 0 : j == 1 ? n : 8 * n; }
+__device__ __forceinline__ int head_outputs(int j, int n) { return j == 0 ? n : j == 1 ? 7 * n : 3 * n; }
+
+__device__ __forceinline__ void load_parameters(HeadParameters& s, const TrainArgs& d)
+{
+    const int threads = blockDim.x;
+    for (int i = threadIdx.x; i < 3 * 32 * kW0Stride; i += threads) {
+        const int j = i / (32 * kW0Stride), r = i % (32 * kW0Stride) / kW0Stride, c = i % kW0Stride;
+        s.w0[j][r * kW0Stride + c] = c < d.in_dim[j] ? d.w0[j][r * d.in_dim[j] + c] : 0.0f;
+    }
+    for (int i = threadIdx.x; i < kRows * kW1Stride; i += threads) {
+        const int o = i / kW1Stride, c = i % kW1Stride, j = head_of(o, d.n);
+        s.w1[i] = o < 11 * d.n && c < kFeat ? d.w1[j][(o - head_base(j, d.n)) * kFeat + c] : 0.0f;
+    }
+}
+
+__device__ __forceinline__ floatx16 mfma(float a, float b, floatx16 c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+// Unit held by register v of an accumulator.
+__device__ __forceinline__ int unit_of(int v, int half) { return 8 * (v >> 2) + 4 * half + (v & 3); }
+
+// View direction and distance of an anchor; the norm adds its squares as the framework's row reduction does.
+__device__ __forceinline__ float view_of(const TrainArgs& d, size_t a, float view[3])
+{
+    const float v[3] = {d.anchor[3 * a] - d.campos[0], d.anchor[3 * a + 1] - d.campos[1], d.anchor[3 * a + 2] - d.campos[2]};
+    const float dist = sqrtf((v[0] * v[0] + v[2] * v[2]) + v[1] * v[1]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) view[k] = v[k] / dist;
+    return dist;
+}
+
+// Positions (within the run) of a run's visible anchors, in order; returns their number.
+__device__ __forceinline__ int list_visible(const TrainArgs& d, int run, int lane, uint8_t* __restrict__ list)
+{
+    const int a0 = run * kRun + lane, a1 = a0 + 64;
+    const bool v0 = a0 < d.A && d.visible[a0] != 0, v1 = a1 < d.A && d.visible[a1] != 0;
+    const uint64_t m0 = __ballot(v0), m1 = __ballot(v1);
+    const int n0 = __popcll(m0);
+    if (v0) list[lanes_below_in(m0)] = (uint8_t)lane;
+    if (v1) list[n0 + lanes_below_in(m1)] = (uint8_t)(64 + lane);
+    wave_lds_sync();
+    return n0 + __popcll(m1);
+}
+
+__global__ __launch_bounds__(256) void train_rows_kernel(TrainArgs d, uint2* __restrict__ run_totals, int runs)
+{
+    const int run = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (run >= runs) return;
+    const int a0 = run * kRun + lane, a1 = a0 + 64;
+    const int nvis = __popcll(__ballot(a0 < d.A && d.visible[a0] != 0)) + __popcll(__ballot(a1 < d.A && d.visible[a1] != 0));
+    if (lane == 0) run_totals[run] = make_uint2(0u, (uint32_t)nvis);
+}
+
+// A wavefront lists its run's visible anchors and writes their input rows, four lanes per row.
+__global__ __launch_bounds__(256) void train_inputs_kernel(TrainArgs d, const uint2* __restrict__ run_base, int runs,
+                                                           uint32_t* __restrict__ rows)
+{
+    __shared__ uint8_t s_list[4][kRun];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, run = blockIdx.x * 4 + wave;
+    if (run >= runs) return;
+    const int nvis = list_visible(d, run, lane, s_list[wave]);
+    const uint32_t rank = run_base[run].y;
+    const int part = lane & 3;
+    for (int i = lane >> 2; i < nvis; i += 16) {
+        const size_t a = (size_t)run * kRun + s_list[wave][i], r = (size_t)rank + i;
+        const float4* __restrict__ f4 = reinterpret_cast<const float4*>(d.feat + (d.compact_feat ? r : a) * kFeat) + 2 * part;
+        const float4 f0 = f4[0], f1 = f4[1];
+        float extra[4];
+        if (part == 0) {
+            rows[r] = (uint32_t)a;
+            extra[3] = view_of(d, a, extra);
+            if (d.level) extra[3] = d.level[a];
+        }
+        if (d.with_dist) {  // (rows of 144 B)
+            float4* __restrict__ x = reinterpret_cast<float4*>(d.with_dist + r * 36);
+            x[2 * part] = f0;
+            x[2 * part + 1] = f1;
+            if (part == 0) x[8] = make_float4(extra[0], extra[1], extra[2], extra[3]);
+        }
+        if (d.without) {
+            float* __restrict__ x = d.without + r * 35 + 8 * part;
+            x[0] = f0.x, x[1] = f0.y, x[2] = f0.z, x[3] = f0.w, x[4] = f1.x, x[5] = f1.y, x[6] = f1.z, x[7] = f1.w;
+            if (part == 0)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) x[32 + k] = extra[k];
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void train_count_kernel(TrainArgs d, uint2* __restrict__ totals, uint32_t groups)
+{
+    const uint32_t group = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (group >= groups) return;
+    const size_t first = (size_t)group * kGroup * d.n, end = min((size_t)d.V * d.n, first + (size_t)kGroup * d.n);
+    uint32_t kept = 0;
+    for (size_t i = first; i < end; i += 64) {  // uniform
+        const size_t k = i + lane;
+        kept += (uint32_t)__popcll(__ballot(k < end && d.pre[0][min(k, end - 1)] > 0.0f));
+    }
+    if (lane == 0) totals[group] = make_uint2(kept, 0u);
+}
+
+// The items (row, offset) of a group of 32 rows, row-major (the output order), two per thread of a workgroup of 256: the
+// first output slots of the workgroup's four wavefronts in either round.
+struct GroupItems {
+    int count;             // of the group
+    uint32_t slot[2];      // this thread's, were its item kept
+    bool kept[2];
+    float pre[2];          // opacity pre-activations
+};
+__device__ __forceinline__ void group_items(const TrainArgs& d, uint32_t group, uint32_t first_slot, GroupItems& g)
+{
+    __shared__ uint32_t s_kept[2][4];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const size_t row0 = (size_t)group * kGroup;
+    g.count = (int)min((size_t)kGroup, (size_t)d.V - row0) * d.n;
+    uint64_t mask[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int it = 256 * i + (int)threadIdx.x;
+        g.pre[i] = d.pre[0][row0 * d.n + min(it, g.count - 1)];
+        g.kept[i] = it < g.count && g.pre[i] > 0.0f;
+        mask[i] = __ballot(g.kept[i]);
+        if (lane == 0) s_kept[i][wave] = (uint32_t)__popcll(mask[i]);
+    }
+    __syncthreads();
+    uint32_t slot = first_slot;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        for (int w = 0; w < 4; ++w) {
+            if (w == wave) g.slot[i] = slot + lanes_below_in(mask[i]);
+            slot += s_kept[i][w];
+        }
+    }
+}
+
+// One workgroup per group, an item per thread and round.  Memory-bound: some 130 MB at 200k anchors in 54 us.
+__global__ __launch_bounds__(256) void train_emit_kernel(TrainArgs d, const uint2* __restrict__ base, uint32_t capacity,
+                                                         gs355_decoded out, const uint32_t* __restrict__ rows)
+{
+    const int n = d.n, inv_n = (65536 + n - 1) / n;  // item / n == (item * inv_n) >> 16 for item < 32 n
+    const size_t row0 = (size_t)blockIdx.x * kGroup;
+    GroupItems g;
+    group_items(d, blockIdx.x, base[blockIdx.x].x, g);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int it = 256 * i + (int)threadIdx.x;
+        if (it >= g.count) continue;
+        const int rl = (it * inv_n) >> 16, m = it - rl * n;
+        const size_t item = row0 * n + it, pos = g.slot[i];
+        const float t = tanhf(g.pre[i]);
+        out.neural_opacity[item] = t;
+        out.mask[item] = g.kept[i] ? 1 : 0;
+        if (!g.kept[i] || pos >= capacity) continue;  // (the second cannot happen: capacity comes from the count pass)
+        const size_t a = rows[row0 + rl];
+        const float* __restrict__ c7 = d.pre[1] + 7 * item;
+        const float* __restrict__ c3 = d.pre[2] + 3 * item;
+        out.opacity[pos] = t;
+        const float q[4] = {c7[3], c7[4], c7[5], c7[6]};
+        const float norm = quaternion_norm(q);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            out.color[3 * pos + k] = logistic(c3[k]);
+            out.scaling[3 * pos + k] = d.scaling[6 * a + 3 + k] * logistic(c7[k]);
+            out.xyz[3 * pos + k] = d.anchor[3 * a + k] + d.offset[(a * n + m) * 3 + k] * d.scaling[6 * a + k];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) out.rot[4 * pos + k] = q[k] / norm;
+    }
+}
+
+// Cotangents of the outputs to those of the pre-activations (`d_pre`, shaped as d.pre), and what does not go through the
+// heads: gradients of offsets and scales, and the anchors' part through the Gaussians' positions.  A row's sums over its
+// offsets are taken in their order from LDS.  Memory-bound: some 210 MB at 200k anchors in 57 us (inside the kernel below,
+// a wavefront at a time, it was most of 389 us).
+__global__ __launch_bounds__(256) void train_items_kernel(TrainArgs d, const uint2* __restrict__ base,
+                                                          const uint32_t* __restrict__ rows, gs355_decode_cotangents g,
+                                                          gs355_decode_gradients out, float* __restrict__ d_op,
+                                                          float* __restrict__ d_cov, float* __restrict__ d_col)
+{
+    __shared__ float s_part[kGroup * kMaxOffsets][9];  // an item's share of d scaling (6) and d anchor (3)
+    const int n = d.n, inv_n = (65536 + n - 1) / n;
+    const size_t row0 = (size_t)blockIdx.x * kGroup;
+    GroupItems items;
+    group_items(d, blockIdx.x, base[blockIdx.x].x, items);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int it = 256 * i + (int)threadIdx.x;
+        if (it >= items.count) continue;
+        const int rl = (it * inv_n) >> 16, m = it - rl * n;
+        const size_t item = row0 * n + it, pos = items.slot[i], a = rows[row0 + rl];
+        float dt = g.neural_opacity ? g.neural_opacity[item] : 0.0f;
+        float c7[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, c3[3] = {0.f, 0.f, 0.f}, d_off[3] = {0.f, 0.f, 0.f};
+        float part[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (items.kept[i]) {
+            if (g.opacity) dt += g.opacity[pos];
+            float sc[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) sc[k] = d.scaling[6 * a + k];
+#pragma unroll
+            for (int k = 0; k < 7; ++k) c7[k] = d.pre[1][7 * item + k];
+            const float q[4] = {c7[3], c7[4], c7[5], c7[6]};
+            const float norm = quaternion_norm(q);
+            float d_q[4] = {0.f, 0.f, 0.f, 0.f};
+            if (g.rot) {
+                float along = 0.0f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    d_q[k] = g.rot[4 * pos + k];
+                    along += d_q[k] * (q[k] / norm);
+                }
+                if (!(norm > 1e-12f)) along = 0.0f;  // (the norm is a constant there)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) d_q[k] = (d_q[k] - (q[k] / norm) * along) / norm;
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float sig = logistic(c7[k]), colour = logistic(d.pre[2][3 * item + k]);
+                const float d_s = g.scaling ? g.scaling[3 * pos + k] : 0.0f;
+                const float d_c = g.color ? g.color[3 * pos + k] : 0.0f;
+                const float d_x = g.xyz ? g.xyz[3 * pos + k] : 0.0f;
+                part[k] = d_x * d.offset[(a * n + m) * 3 + k];
+                part[3 + k] = d_s * sig;
+                part[6 + k] = d_x;
+                d_off[k] = d_x * sc[k];
+                c7[k] = d_s * sc[3 + k] * (1.0f - sig) * sig;
+                c3[k] = d_c * (1.0f - colour) * colour;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) c7[3 + k] = d_q[k];
+        }
+        const float t = tanhf(items.pre[i]);
+        d_op[item] = dt * (1.0f - t * t);
+#pragma unroll
+        for (int k = 0; k < 7; ++k) d_cov[7 * item + k] = c7[k];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) d_col[3 * item + k] = c3[k];
+        if (out.offset)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) out.offset[(a * n + m) * 3 + k] = d_off[k];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s_part[it][k] = part[k];
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < 9 * (items.count / n); k += 256) {
+        const int rl = k / 9, c = k % 9;
+        float sum = 0.0f;
+        for (int m = 0; m < n; ++m) sum += s_part[rl * n + m][c];
+        const size_t a = rows[row0 + rl];
+        if (c < 6 && out.scaling) out.scaling[6 * a + c] = sum;
+        if (c >= 6 && out.anchor) out.anchor[3 * a + c - 6] = sum;  // (train_layers_kernel adds the view's part)
+    }
+}
+
+constexpr int kBackwardWaves = 4;      // one per SIMD: 176 registers of weight gradients and as many again
+constexpr int kBackwardMaxGroups = 256;
+constexpr int kTilePre = kGroup * 11 * kMaxOffsets;  // floats of a tile's pre-activation gradients
+
+// `count` floats from memory to LDS, both 16-B aligned, without passing through registers; the last few of a count that is
+// no multiple of four are copied one by one.
+__device__ __forceinline__ void copy_to_lds(const float* src, float* dst, int count, int lane)
+{
+    typedef __attribute__((address_space(1))) const void global_void;
+    typedef __attribute__((address_space(3))) void lds_void;
+    for (int i = 0; i < count / 4; i += 64)  // uniform
+        if (i + lane < count / 4)            // (lane l of a copy writes float4 l behind the uniform LDS address)
+            __builtin_amdgcn_global_load_lds((global_void*)(src + 4 * (i + lane)), (lds_void*)(dst + 4 * i), 16, 0, 0);
+    if (lane < (count & 3)) dst[(count & ~3) + lane] = src[(count & ~3) + lane];
+}
+
+// A wavefront keeps all 11 blocks of 32 x 32 weight gradients in registers, so there is one wavefront per SIMD and a
+// workgroup per compute unit, each with its own quarter of the LDS for the tile's rows; tiles come from memory straight to
+// LDS.  146 us at 200k anchors (37 us of matrix instructions; the rest is the wait for a tile's rows, which one wavefront
+// per SIMD does not hide).
+// kAnchor: the anchors' own gradient is wanted (the layers are then also walked back to view direction and distance).
+// kOffsets: offsets per anchor, or 0 (d.n).  Ten, the decoder's default, has its loops unrolled: with the count a variable,
+// the kernel does not fit its registers.
+template <bool kAnchor, int kOffsets>
+__global__ __launch_bounds__(64 * kBackwardWaves) void train_layers_kernel(
+    TrainArgs d, const uint32_t* __restrict__ rows, const float* __restrict__ d_op, const float* __restrict__ d_cov,
+    const float* __restrict__ d_col, gs355_decode_gradients out, float* __restrict__ partials)
+{
+    __shared__ HeadParameters s;
+    __shared__ __align__(16) float s_pre[kBackwardWaves][kTilePre];       // gradients of the pre-activations, head by head as in memory
+    __shared__ __align__(16) float s_in[kBackwardWaves][kGroup * 36];     // input rows
+    __shared__ __align__(16) float s_hidden[kBackwardWaves][kGroup * 32];  // one head's hidden units, by row
+    __shared__ float s_unit[kBackwardWaves][kGroup * kW1Stride];          // ... and their gradients
+    load_parameters(s, d);
+    __syncthreads();
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
+    const int n = kOffsets ? kOffsets : d.n, outputs = 11 * n;
+    const int width = d.with_dist ? 36 : 35;
+    const float* const input_rows = d.with_dist ? d.with_dist : d.without;
+    float* const pre = s_pre[wave];
+    float* const input = s_in[wave];
+    float* const hidden = s_hidden[wave];
+    float* const unit = s_unit[wave];
+
+    floatx16 grad1[5] = {}, grad0[6] = {};  // dW1: opacity | covariance x 3 | colour; dW0: features, extras + bias per head
+    float bias1[2] = {0.f, 0.f};            // db1 of outputs lane and 64 + lane
+    const uint32_t tiles = (d.V + kGroup - 1) / kGroup;
+    for (uint32_t tile = blockIdx.x * kBackwardWaves + wave; tile < tiles; tile += gridDim.x * kBackwardWaves) {
+        const uint32_t row0 = tile * kGroup, r = min(row0 + (uint32_t)col, d.V - 1);
+        const bool live = row0 + (uint32_t)col < d.V;
+        const int tile_rows = (int)min((uint32_t)kGroup, d.V - row0);
+        if (tile_rows < kGroup) {  // (rows that do not exist: zeros)
+            for (int i = lane; i < kGroup * outputs; i += 64) pre[i] = 0.0f;
+            for (int i = lane; i < kGroup * width; i += 64) input[i] = 0.0f;
+            for (int i = lane; i < kGroup * kFeat; i += 64) hidden[i] = 0.0f;
+            wave_lds_sync();
+        }
+        copy_to_lds(d_op + (size_t)row0 * n, pre, tile_rows * n, lane);
+        copy_to_lds(d_cov + (size_t)row0 * 7 * n, pre + kGroup * n, tile_rows * 7 * n, lane);
+        copy_to_lds(d_col + (size_t)row0 * 3 * n, pre + kGroup * 8 * n, tile_rows * 3 * n, lane);
+        copy_to_lds(input_rows + (size_t)row0 * width, input, tile_rows * width, lane);
+        copy_to_lds(d.hidden[0] + (size_t)row0 * kFeat, hidden, tile_rows * kFeat, lane);
+        floatx16 d_feat = {}, d_extra = {};
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int base = head_base(j, n), count = head_outputs(j, n);
+            float relu[16];  // the hidden units of this lane's row, in accumulator order (only their sign is used)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const float4 v = reinterpret_cast<const float4*>(d.hidden[j] + (size_t)r * kFeat)[2 * b + half];
+                relu[4 * b] = v.x, relu[4 * b + 1] = v.y, relu[4 * b + 2] = v.z, relu[4 * b + 3] = v.w;
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies have landed
+            wave_lds_sync();
+            // the head's gradients: row stride `count`, conflict-free for the counts of ten offsets (twice an odd number)
+            const float* const g = pre + kGroup * base;
+            floatx16 dh = {};
+            {
+                const float* const w1 = s.w1 + base * kW1Stride + col;  // transposed: this lane's hidden unit
+                const int steps = (count + 1) / 2;
+                constexpr int kUnroll = kOffsets ? 35 : 1;
+#pragma unroll kUnroll
+                for (int k = 0; k < steps; ++k) {
+                    const int o = 2 * k + half;
+                    const bool in_head = kOffsets ? true : o < count;  // (the counts of ten offsets are even)
+                    dh = mfma(w1[(in_head ? o : 0) * kW1Stride], in_head ? g[col * count + o] : 0.0f, dh);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                dh[v] = relu[v] > 0.0f ? dh[v] : 0.0f;
+                unit[col * kW1Stride + unit_of(v, half)] = dh[v];
+            }
+            // dW1 and db1: products over the tile's rows
+#pragma unroll
+            for (int q = 0; q < (j == 1 ? 3 : 1); ++q) {
+                if (32 * q >= count) break;  // uniform
+                const int o = min(32 * q + col, count - 1);  // (rows past the head's last output are not used)
+                floatx16& acc = grad1[j == 0 ? 0 : j == 1 ? 1 + q : 4];
+#pragma unroll
+                for (int k = 0; k < 16; ++k)
+                    acc = mfma(g[(2 * k + half) * count + o], hidden[(2 * k + half) * kFeat + col], acc);
+            }
+            {
+                const int o0 = lane - base, o1 = 64 + lane - base;
+                if (o0 >= 0 && o0 < count)
+#pragma unroll 8
+                    for (int k = 0; k < kGroup; ++k) bias1[0] += g[k * count + o0];
+                if (o1 >= 0 && o1 < count)
+#pragma unroll 8
+                    for (int k = 0; k < kGroup; ++k) bias1[1] += g[k * count + o1];
+            }
+            wave_lds_sync();
+            if (j < 2) copy_to_lds(d.hidden[j + 1] + (size_t)row0 * kFeat, hidden, tile_rows * kFeat, lane);
+            // back to the inputs, and dW0
+            const float* const w0 = s.w0[j];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) d_feat = mfma(w0[unit_of(v, half) * kW0Stride + col], dh[v], d_feat);
+            if (kAnchor) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    d_extra = mfma(w0[unit_of(v, half) * kW0Stride + 32 + min(col, 4)], dh[v], d_extra);  // (rows past 3: unused)
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const float left = unit[(2 * k + half) * kW1Stride + col];
+                const float* const x = input + (2 * k + half) * width;
+                // columns 32 .. 35 (34): view and distance; then the constant one of the bias
+                const float extra = x[min(32 + col, width - 1)];
+                grad0[2 * j] = mfma(left, x[col], grad0[2 * j]);
+                grad0[2 * j + 1] = mfma(left, col < width - 32 ? extra : 1.0f, grad0[2 * j + 1]);
+            }
+            wave_lds_sync();
+        }
+        if (live && out.feat) {
+            float4* const dst = reinterpret_cast<float4*>(out.feat + (d.compact_feat ? (size_t)r : (size_t)rows[r]) * kFeat);
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                dst[2 * b + half] = make_float4(d_feat[4 * b], d_feat[4 * b + 1], d_feat[4 * b + 2], d_feat[4 * b + 3]);
+        }
+        if (kAnchor && live && half == 0) {  // rows 0..3 of d_extra: view direction, distance (or level)
+            const size_t a = rows[r];
+            float view[3];
+            const float dist = view_of(d, a, view);
+            const float along = view[0] * d_extra[0] + view[1] * d_extra[1] + view[2] * d_extra[2];
+            const float d_dist = d.level ? 0.0f : d_extra[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                out.anchor[3 * a + k] += (d_extra[k] - view[k] * along) / dist + d_dist * view[k];
+        }
+    }
+
+    // ---- the workgroup's weight gradients, its wavefronts one after the other, over the parameters' LDS ----
+    __syncthreads();
+    float* const sums0 = s.w0[0];
+    float* const sums1 = s.w1;
+    for (int i = threadIdx.x; i < 3 * 32 * kW0Stride; i += blockDim.x) sums0[i] = 0.0f;
+    for (int i = threadIdx.x; i < kRows * kW1Stride; i += blockDim.x) sums1[i] = 0.0f;
+    for (int w = 0; w < kBackwardWaves; ++w) {
+        __syncthreads();
+        if (wave != w) continue;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int base = head_base(j, n), count = head_outputs(j, n);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                float* const dst = s.w0[j] + unit_of(v, half) * kW0Stride;
+                dst[col] += grad0[2 * j][v];
+                if (col < width - 32) dst[32 + col] += grad0[2 * j + 1][v];
+                else if (col == width - 32) dst[36] += grad0[2 * j + 1][v];  // (the bias keeps its column)
+            }
+#pragma unroll
+            for (int q = 0; q < (j == 1 ? 3 : 1); ++q)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int o = 32 * q + unit_of(v, half);
+                    if (o < count) sums1[(base + o) * kW1Stride + col] += grad1[j == 0 ? 0 : j == 1 ? 1 + q : 4][v];
+                }
+        }
+        if (lane < outputs) sums1[lane * kW1Stride + 32] += bias1[0];
+        if (64 + lane < outputs) sums1[(64 + lane) * kW1Stride + 32] += bias1[1];
+    }
+    __syncthreads();
+    float* const to = partials + (size_t)blockIdx.x * kGradFloats;
+    for (int i = threadIdx.x; i < 3 * 32 * kW0Stride; i += blockDim.x) to[i] = sums0[i];
+    for (int i = threadIdx.x; i < kRows * kW1Stride; i += blockDim.x) to[3 * 32 * kW0Stride + i] = sums1[i];
+}
+
+// Sixty-four elements of the weight gradients per workgroup, the workgroups' contributions split over 16 wavefronts.
+__global__ __launch_bounds__(1024) void train_sum_kernel(TrainArgs d, const float* __restrict__ partials, int groups,
+                                                         gs355_decode_gradients out)
+{
+    __shared__ float s_sum[16][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = blockIdx.x * 64 + lane;
+    float sum = 0.0f;
+    if (i < kGradFloats)
+#pragma unroll 4
+        for (int g = wave; g < groups; g += 16) sum += partials[(size_t)g * kGradFloats + i];
+    s_sum[wave][lane] = sum;
+    __syncthreads();
+    if (wave != 0 || i >= kGradFloats) return;
+    sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) sum += s_sum[w][lane];
+    if (i < 3 * 32 * kW0Stride) {
+        const int j = i / (32 * kW0Stride), unit = i % (32 * kW0Stride) / kW0Stride, c = i % kW0Stride;
+        if (c < d.in_dim[j]) {
+            if (out.w0[j]) out.w0[j][unit * d.in_dim[j] + c] = sum;
+        } else if (c == 36 && out.b0[j]) {
+            out.b0[j][unit] = sum;
+        }
+        return;
+    }
+    const int k = i - 3 * 32 * kW0Stride, o = k / kW1Stride, c = k % kW1Stride;
+    if (o >= 11 * d.n) return;
+    const int j = head_of(o, d.n), at = o - head_base(j, d.n);
+    if (c < kFeat) {
+        if (out.w1[j]) out.w1[j][at * kFeat + c] = sum;
+    } else if (out.b1[j]) {
+        out.b1[j][at] = sum;
+    }
+}
+
+// Workspace kept from the forward to the backward pass: totals and bases (of the runs, then of the groups of rows), the
+// list of visible anchors.
+struct TrainLayout {
+    size_t totals, base, rows, total;
+};
+TrainLayout train_layout(int32_t A)
+{
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    const size_t groups = ((size_t)A + kGroup - 1) / kGroup;  // (at least as many as runs)
+    TrainLayout L;
+    L.totals = 0;
+    L.base = up(groups * sizeof(uint2) + 8);
+    L.rows = L.base + up(groups * sizeof(uint2) + 8);
+    L.total = L.rows + up((size_t)A * sizeof(uint32_t) + 4);
+    return L;
+}
+
+// Scratch of the backward pass: gradients of the pre-activations (each head's 256-byte aligned), then the workgroups'
+// weight gradients.
+struct TrainScratch {
+    size_t d_pre[3], partials, total;
+};
+
+int backward_groups(int32_t V);
+TrainScratch train_scratch(int32_t V, int n)
+{
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    TrainScratch t;
+    size_t off = 0;
+    for (int j = 0; j < 3; ++j) {
+        t.d_pre[j] = off;
+        off += up((size_t)V * (j == 0 ? 1 : j == 1 ? 7 : 3) * n * sizeof(float));
+    }
+    t.partials = off;
+    t.total = off + (size_t)backward_groups(V) * kGradFloats * sizeof(float);
+    return t;
+}
+
+int backward_groups(int32_t V) { return min(kBackwardMaxGroups, max(1, ((V + 31) / 32 + kBackwardWaves - 1) / kBackwardWaves)); }
+
+int train_args(const gs355_decoder* dec, const gs355_anchors* an, const gs355_train_rows* rows, const void* workspace,
+               size_t workspace_bytes, TrainArgs* out)
+{
+    const int rc = check_decoder(dec, an);
+    if (rc) return rc;
+    if (!rows) return set_error(GS355_EINVAL, "rows is NULL");
+    if (dec->bank_in_dim != 0)
+        return set_error(GS355_EINVAL, "the differentiable decode takes mixed features: the feature bank is the caller's");
+    if (rows->num_visible < 0 || rows->num_visible > an->A)
+        return set_error(GS355_EINVAL, "num_visible must be in [0, A] (got %d)", rows->num_visible);
+    if (an->A > 0) {
+        if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
+            return set_error(GS355_EINVAL, "workspace must be given and 256-byte aligned");
+        const TrainLayout L = train_layout(an->A);
+        if (workspace_bytes < L.total)
+            return set_error(GS355_ENOSPC, "decode workspace has %zu bytes, %zu needed", workspace_bytes, L.total);
+    }
+    TrainArgs a;
+    a.A = an->A;
+    a.n = dec->n_offsets;
+    a.V = (uint32_t)rows->num_visible;
+    a.anchor = an->anchor;
+    a.feat = an->feat;
+    a.offset = an->offset;
+    a.scaling = an->scaling;
+    a.visible = an->visible_mask;
+    a.campos = an->campos;
+    a.level = dec->add_level ? an->level : nullptr;
+    a.compact_feat = rows->compact_feat;
+    for (int j = 0; j < 3; ++j) {
+        a.in_dim[j] = dec->in_dim[j];
+        a.w0[j] = dec->w0[j];
+        a.w1[j] = dec->w1[j];
+        a.hidden[j] = rows->hidden[j];
+        a.pre[j] = rows->pre[j];
+    }
+    a.with_dist = rows->with_dist;
+    a.without = rows->without;
+    *out = a;
+    return GS355_OK;
+}
+
+}  // namespace
+
+}  // namespace gs355
+
+using namespace gs355;
+
+extern "C" {
+
+int gs355_decode_train_bytes(int32_t A, int32_t num_visible, int32_t n_offsets, size_t* workspace, size_t* scratch)
+{
+    if (!workspace || !scratch) return set_error(GS355_EINVAL, "workspace / scratch is NULL");
+    if (A < 0 || num_visible < 0 || num_visible > A)
+        return set_error(GS355_EINVAL, "A and num_visible out of range (got %d, %d)", A, num_visible);
+    if (n_offsets < 1 || n_offsets > kMaxOffsets)
+        return set_error(GS355_EINVAL, "anchor decode supports 1..10 offsets per anchor (got %d)", n_offsets);
+    *workspace = train_layout(A).total;
+    *scratch = train_scratch(num_visible, n_offsets).total;
+    return GS355_OK;
+}
+
+int gs355_decode_train(const gs355_decoder* dec, const gs355_anchors* an, const gs355_train_rows* rows, int64_t capacity,
+                       const gs355_decoded* out, void* workspace, size_t workspace_bytes, uint32_t phase, void* stream)
+{
+    TrainArgs a;
+    int rc = train_args(dec, an, rows, workspace, workspace_bytes, &a);
+    if (rc) return rc;
+    if (capacity < 0 || capacity > 0xFFFFFFFFll)
+        return set_error(GS355_EINVAL, "capacity must be in [0, 2^32) (got %lld)", (long long)capacity);
+    if (!out) return set_error(GS355_EINVAL, "decoded outputs is NULL");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    char* ws = static_cast<char*>(workspace);
+    const TrainLayout L = train_layout(a.A);
+    const int runs = (a.A + kRun - 1) / kRun;
+    const uint32_t groups = (a.V + kGroup - 1) / kGroup;
+    uint2* totals = reinterpret_cast<uint2*>(ws + L.totals);
+    uint2* base = reinterpret_cast<uint2*>(ws + L.base);
+    uint32_t* list = reinterpret_cast<uint32_t*>(ws + L.rows);
+    switch (phase) {
+        case GS355_TRAIN_ROWS:
+            if (!out->num_visible) return set_error(GS355_EINVAL, "num_visible is NULL");
+            if (runs > 0) hipLaunchKernelGGL(train_rows_kernel, dim3((runs + 3) / 4), dim3(256), 0, s, a, totals, runs);
+            GS355_CHECK_LAUNCH("decode train: rows");
+            return launch_run_scan(totals, base, (uint32_t)runs, nullptr, out->num_visible, s);
+        case GS355_TRAIN_INPUTS:
+            if (a.V == 0) return GS355_OK;
+            if (!a.with_dist && !a.without) return set_error(GS355_EINVAL, "with_dist and without are NULL");
+            if ((reinterpret_cast<uintptr_t>(a.with_dist) & 15u) != 0)
+                return set_error(GS355_EINVAL, "with_dist must be 16-byte aligned");
+            hipLaunchKernelGGL(train_inputs_kernel, dim3((runs + 3) / 4), dim3(256), 0, s, a, base, runs, list);
+            GS355_CHECK_LAUNCH("decode train: inputs");
+            return GS355_OK;
+        case GS355_TRAIN_COUNT:
+            if (!out->count) return set_error(GS355_EINVAL, "count is NULL");
+            if (a.V > 0 && !a.pre[0]) return set_error(GS355_EINVAL, "the opacity pre-activations are NULL");
+            if (groups > 0) hipLaunchKernelGGL(train_count_kernel, dim3((groups + 3) / 4), dim3(256), 0, s, a, totals, groups);
+            GS355_CHECK_LAUNCH("decode train: count");
+            return launch_run_scan(totals, base, groups, out->count, nullptr, s);
+        case GS355_TRAIN_EMIT:
+            if (a.V == 0) return GS355_OK;
+            if (!a.pre[0] || !a.pre[1] || !a.pre[2]) return set_error(GS355_EINVAL, "pre-activations must all be non-NULL");
+            if (!out->neural_opacity || !out->mask ||
+                (capacity > 0 && (!out->xyz || !out->color || !out->opacity || !out->scaling || !out->rot)))
+                return set_error(GS355_EINVAL, "decoded outputs must all be non-NULL");
+            hipLaunchKernelGGL(train_emit_kernel, dim3(groups), dim3(256), 0, s, a, base, (uint32_t)capacity, *out, list);
+            GS355_CHECK_LAUNCH("decode train: emit");
+            return GS355_OK;
+        default: return set_error(GS355_EINVAL, "phase must be one of GS355_TRAIN_* (got 0x%x)", phase);
+    }
+}
+
+int gs355_decode_train_backward(const gs355_decoder* dec, const gs355_anchors* an, const gs355_train_rows* rows,
+                                const void* workspace, size_t workspace_bytes, const gs355_decode_cotangents* cotangents,
+                                const gs355_decode_gradients* grads, void* scratch, size_t scratch_bytes, void* stream)
+{
+    TrainArgs a;
+    int rc = train_args(dec, an, rows, workspace, workspace_bytes, &a);
+    if (rc) return rc;
+    if (!cotangents || !grads) return set_error(GS355_EINVAL, "cotangents / gradients is NULL");
+    for (int j = 0; j < 3; ++j)
+        if (a.V > 0 && (!a.pre[j] || !a.hidden[j] || (reinterpret_cast<uintptr_t>(a.hidden[j]) & 15u) != 0))
+            return set_error(GS355_EINVAL, "head %d: hidden (16-byte aligned) and pre-activations are needed", j);
+    if (a.V > 0 && !a.with_dist && !a.without) return set_error(GS355_EINVAL, "with_dist and without are NULL");
+    if (grads->feat && (reinterpret_cast<uintptr_t>(grads->feat) & 15u) != 0)
+        return set_error(GS355_EINVAL, "the gradient of the features must be 16-byte aligned");
+    const int workgroups = backward_groups(rows->num_visible);
+    const TrainScratch S = train_scratch(rows->num_visible, a.n);
+    if (!scratch || (reinterpret_cast<uintptr_t>(scratch) & 255u) != 0 || scratch_bytes < S.total)
+        return set_error(GS355_ENOSPC, "decode backward scratch: %zu bytes given, %zu needed, 256-byte aligned", scratch_bytes,
+                         S.total);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const TrainLayout L = train_layout(a.A);
+    const char* ws = static_cast<const char*>(workspace);
+    char* sc = static_cast<char*>(scratch);
+    const uint32_t* list = reinterpret_cast<const uint32_t*>(ws + L.rows);
+    const uint2* base = reinterpret_cast<const uint2*>(ws + L.base);
+    float* d_pre[3];
+    for (int j = 0; j < 3; ++j) d_pre[j] = reinterpret_cast<float*>(sc + S.d_pre[j]);
+    float* partials = reinterpret_cast<float*>(sc + S.partials);
+    if (a.V > 0) {
+        hipLaunchKernelGGL(train_items_kernel, dim3((a.V + kGroup - 1) / kGroup), dim3(256), 0, s, a, base, list, *cotangents,
+                           *grads, d_pre[0], d_pre[1], d_pre[2]);
+        GS355_CHECK_LAUNCH("decode train: items");
+    }
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(64 * kBackwardWaves), 0, s, a, list, d_pre[0], d_pre[1], d_pre[2],
+                           *grads, partials);
+    };
+    if (grads->anchor) {
+        if (a.n == 10) launch(train_layers_kernel<true, 10>);
+        else launch(train_layers_kernel<true, 0>);
+    } else {
+        if (a.n == 10) launch(train_layers_kernel<false, 10>);
+        else launch(train_layers_kernel<false, 0>);
+    }
+    GS355_CHECK_LAUNCH("decode train: layers");
+    hipLaunchKernelGGL(train_sum_kernel, dim3((kGradFloats + 63) / 64), dim3(1024), 0, s, a, partials, workgroups, *grads);
+    GS355_CHECK_LAUNCH("decode train: weight gradients");
+    return GS355_OK;
+}
+
+}  // extern "C"

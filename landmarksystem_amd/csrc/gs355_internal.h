@@ -196,6 +196,11 @@ constexpr int kListHeader = 8;
 int launch_tile_sort(const gs355_header* header, int tiles, const uint32_t* ranges, uint32_t* lists,
                      uint64_t* buckets, uint64_t* out_keys, uint32_t* out_vals, uint32_t skip_classes, hipStream_t s);
 
+// anchor decode: argument checks, and the exclusive prefix of per-run (kept offsets, visible anchors) with the totals
+int check_decoder(const gs355_decoder* dec, const gs355_anchors* an);
+int launch_run_scan(const uint2* totals, uint2* base, uint32_t runs, uint32_t* num_emitted, uint32_t* num_visible,
+                    hipStream_t s);
+
 // row compaction by a byte mask (gs355_gather_rows); scratch: gather_scratch_words(P) words
 size_t gather_scratch_words(int32_t P);
 int launch_gather_rows(int32_t P, const uint8_t* mask, int32_t n_arrays, const gs355_gather_array* arrays,

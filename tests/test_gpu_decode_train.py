@@ -1,0 +1,74 @@
+"""The differentiable decode's kernels against the reference module's statements in float64 on the CPU: outputs and every
+gradient, at the edges of the tiles (32 visible anchors) and runs (128 anchors)."""
+import copy
+
+import pytest
+import torch
+
+from landmarksystem_amd.anchor_decoder import FusedAnchorDecoder
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, want, name):
+    if got is None or want is None:  # (no gradient and a gradient of zeros are the same answer)
+        assert all(t is None or float(t.abs().max()) == 0.0 for t in (got, want)), name
+        return
+    if want.numel() == 0:
+        return
+    scale = max(float(want.abs().max()), 1e-12)
+    err = float((got.cpu().double() - want).abs().max())
+    assert err <= 2e-5 * scale, (name, err, scale)
+
+
+@pytest.mark.parametrize("A,n,visible,dist,level,bank", [
+    (1, 10, 1.0, (True, True, True), False, False), (31, 1, 1.0, (True, True, True), False, False),
+    (33, 10, 1.0, (False, True, False), False, False), (127, 5, 0.5, (True, False, True), False, False),
+    (129, 7, 0.9, (False, False, False), True, False), (1000, 10, 0.3, (True, True, True), False, True),
+    (300, 3, 0.8, (False, False, False), True, True), (40_000, 10, 0.88, (True, True, True), False, False),
+    (64, 10, 0.0, (True, True, True), False, False)])
+def test_decode_and_gradients(gpu_device, A, n, visible, dist, level, bank):
+    g = torch.Generator().manual_seed(A + n)
+    dec = FusedAnchorDecoder(use_feat_bank=bank, add_opacity_dist=dist[0], add_cov_dist=dist[1], add_color_dist=dist[2],
+                             view_dim=3, feat_dim=32, n_offsets=n, add_level=level)
+    with torch.no_grad():
+        for p in dec.parameters():
+            p.copy_(torch.randn(p.shape, generator=g) * (p.shape[1] ** -0.5 if p.dim() == 2 else 0.1))
+    cam = torch.tensor([0.3, -4.0, 2.0])
+    vis = torch.rand(A, generator=g) < visible
+    lvl = torch.randint(0, 4, (A, 1), generator=g).float() if level else None
+    inputs = [torch.randn(A, 3, generator=g) * 3, torch.randn(A, 32, generator=g), torch.randn(A, n, 3, generator=g) * 0.1,
+              torch.exp(torch.randn(A, 6, generator=g) - 1)]
+    ref_dec = copy.deepcopy(dec).double().train()
+    ref_in = [t.double().requires_grad_(True) for t in inputs]
+    want = ref_dec._forward_torch(cam.double(), *ref_in, vis, None if lvl is None else lvl.double().reshape(-1))
+    dec = dec.to(gpu_device).train()
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in inputs]
+    got = dec(cam.to(gpu_device), *leaves, vis.to(gpu_device), None if lvl is None else lvl.to(gpu_device))
+    assert got[0].grad_fn is not None and "DecodeTrain" in type(got[0].grad_fn).__name__
+    assert torch.equal(got[6].cpu(), want[6])
+    names = ("xyz", "color", "opacity", "scaling", "rot", "neural_opacity")
+    weights = [torch.randn(t.shape, generator=g) for t in want[:6]]
+    for name, a, b in zip(names, got, want):
+        assert a.shape == b.shape
+        _close(a.detach(), b.detach(), name)
+    sum((t * w.to(gpu_device)).sum() for t, w in zip(got, weights)).backward()
+    sum((t * w.double()).sum() for t, w in zip(want, weights)).backward()
+    for name, a, b in zip(("anchor", "feat", "offset", "scaling"), leaves, ref_in):
+        _close(a.grad, b.grad, name)
+    for (name, a), b in zip(dec.named_parameters(), ref_dec.parameters()):
+        _close(a.grad, b.grad, name)
+    # only some outputs in the loss, anchors not differentiated
+    for p in list(dec.parameters()) + leaves:
+        p.grad = None
+    leaves[0].requires_grad_(False)
+    got = dec(cam.to(gpu_device), *leaves, vis.to(gpu_device), None if lvl is None else lvl.to(gpu_device))
+    for p in list(ref_dec.parameters()) + ref_in:
+        p.grad = None
+    want = ref_dec._forward_torch(cam.double(), *ref_in, vis, None if lvl is None else lvl.double().reshape(-1))
+    (got[1].square().sum() + got[4].sum()).backward()
+    (want[1].square().sum() + want[4].sum()).backward()
+    for name, a, b in zip(("feat", "offset", "scaling"), leaves[1:], ref_in[1:]):
+        _close(a.grad, b.grad, name)
+    for (name, a), b in zip(dec.named_parameters(), ref_dec.parameters()):
+        _close(a.grad, b.grad, name)
