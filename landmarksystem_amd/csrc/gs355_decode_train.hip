@@ -305,7 +305,8 @@ __global__ __launch_bounds__(256) void train_items_kernel(TrainArgs d, const uin
             for (int k = 0; k < 4; ++k) c7[3 + k] = d_q[k];
         }
         const float t = tanhf(items.pre[i]);
-        d_op[item] = dt * (1.0f - t * t);
+        // (fused: close to saturation t * t rounded by itself would be wrong by a good part of the difference)
+        d_op[item] = dt * __builtin_fmaf(-t, t, 1.0f);
 #pragma unroll
         for (int k = 0; k < 7; ++k) d_cov[7 * item + k] = c7[k];
 #pragma unroll
