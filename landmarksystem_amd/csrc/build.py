@@ -36,8 +36,8 @@ SOURCES = [
     ("gs355_gather.hip", []),
     ("gs355_decode.hip", []),
     ("gs355_decode_train.hip", ["-ffp-contract=off"]),
-    ("gs355_blend.hip", []),
-    # (matrix results in ordinary registers: the blend's backward reads them with vector instructions right away)
+    # (matrix results in ordinary registers: the blend and its backward read them with vector instructions right away)
+    ("gs355_blend.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form"]),
     ("gs355_backward.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form"]),
 ]
 
