@@ -143,10 +143,11 @@ __device__ __forceinline__ float quaternion_norm(const float q[4])
     return n < 1e-12f ? 1e-12f : n;  // (NaN stays NaN)
 }
 
-// Number of lanes below this one that `mask` (uniform over the wavefront) holds: the hardware's masked bit count.
-__device__ __forceinline__ uint32_t lanes_below_in(uint64_t mask)
+// `first` plus the number of lanes below this one that `mask` (uniform over the wavefront) holds: the hardware's masked
+// bit count.
+__device__ __forceinline__ uint32_t lanes_below_in(uint64_t mask, uint32_t first = 0u)
 {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, first));
 }
 
 // Orders one wavefront's LDS writes before its later LDS reads (and the reverse).  The hardware executes a

@@ -1,0 +1,51 @@
+"""The blend's culling of 4x4 pixel blocks on splats that bend its ellipse test (needles in every direction, splats of half
+a pixel, opacities at the 1/255 threshold) and its accumulation of colours that are not finite."""
+import math
+
+import pytest
+import torch
+
+from landmarksystem_amd import _lib, pipeline, scenes
+from tests.helpers import settings_for
+
+pytestmark = pytest.mark.gpu
+
+
+def _render(scene, device, ws, **kw):
+    inp = pipeline.FrameInputs(settings_for(scene, device), scene.means3D.to(device), opacities=scene.opacities.to(device),
+                               scales=scene.scales.to(device), rotations=scene.rotations.to(device),
+                               **(kw or dict(shs=scene.shs.to(device))))
+    return inp, pipeline.render(inp, ws=ws)
+
+
+@pytest.mark.parametrize("width,height,long_axis,short_axis,logit", [
+    (128, 96, 1.0, 0.002, 0.0), (129, 97, 4.0, 0.01, -4.0), (67, 131, 0.02, 0.02, 2.0), (256, 64, 30.0, 0.05, 1.0),
+    (96, 96, 0.3, 0.003, -5.4)])
+def test_ellipse_culling_is_result_neutral(gpu_device, width, height, long_axis, short_axis, logit):
+    g = torch.Generator().manual_seed(width + height)
+    scene = scenes.tiny_scene(P=6000, width=width, height=height, sh_degree=1, seed=width)
+    log = torch.randn(6000, 3, generator=g) * 0.5
+    scene.scales = torch.exp(log) * torch.tensor([long_axis, short_axis, short_axis])
+    scene.opacities = torch.sigmoid(torch.randn(6000, 1, generator=g) + logit)
+    ws = pipeline.Workspace(gpu_device)
+    inp, out = _render(scene, gpu_device, ws)
+    culled = [out.image.clone(), out.depth.clone(), out.alpha.clone()]
+    pipeline.run_stages(inp, out, ws, ws.key_capacity, _lib.STAGE_BLEND_PLAIN)
+    assert float(out.alpha.max()) > 0.05
+    for a, b in zip(culled, (out.image, out.depth, out.alpha)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("value", [math.inf, math.nan])
+def test_colours_that_are_not_finite_stay_with_their_pixels(gpu_device, value):
+    scene = scenes.tiny_scene(P=400, width=133, height=75, sh_degree=1, seed=3)
+    ws = pipeline.Workspace(gpu_device)
+    colours = torch.rand(400, 3, generator=torch.Generator().manual_seed(0)).to(gpu_device)
+    images = []
+    for c in (0.25, 0.75, value):
+        colours[17] = c
+        images.append(_render(scene, gpu_device, ws, colors_precomp=colours)[1].image.clone())
+    touched = images[0] != images[1]
+    assert 0 < int(touched.sum()) < touched.numel()
+    assert torch.equal(~torch.isfinite(images[2]), touched)
+    assert torch.equal(images[2][~touched], images[0][~touched])
