@@ -332,16 +332,16 @@ int gs355_visible_filter(const gs355_frame* frame, const gs355_gaussians* g, int
 
 namespace {
 struct BackwardScratch {
-    size_t first_key, scan_tmp, key_grads, total;
+    size_t record_slots, next_slot, key_grads, total;
 };
 BackwardScratch backward_scratch(int32_t P, int64_t n_cap)
 {
     BackwardScratch b;
     size_t off = 0;
-    b.first_key = off;
-    off = align_up(off + (size_t)P * sizeof(uint32_t) + 4);
-    b.scan_tmp = off;
-    off = align_up(off + scan_tmp_words((size_t)P) * sizeof(uint32_t));
+    b.record_slots = off;
+    off = align_up(off + (size_t)P * sizeof(uint2) + 4);
+    b.next_slot = off;
+    off = align_up(off + sizeof(uint32_t));
     b.key_grads = off;
     off = align_up(off + (size_t)n_cap * GS355_KEY_GRAD_FLOATS * sizeof(float) + 4);
     b.total = off;
@@ -398,10 +398,9 @@ static int render_backward(const gs355_frame* frame, const gs355_gaussians* g, c
                                   reinterpret_cast<const uint32_t*>(ws + L.ranges),
                                   reinterpret_cast<const uint32_t*>(ws + L.values[L.sorted_buffer]),
                                   reinterpret_cast<const float*>(ws + L.records),
-                                  reinterpret_cast<const uint32_t*>(ws + L.tiles_touched),
                                   reinterpret_cast<const uint64_t*>(ws + L.rects), *in,
-                                  reinterpret_cast<uint32_t*>(sc + B.first_key),
-                                  reinterpret_cast<uint32_t*>(sc + B.scan_tmp),
+                                  reinterpret_cast<uint2*>(sc + B.record_slots),
+                                  reinterpret_cast<uint32_t*>(sc + B.next_slot),
                                   reinterpret_cast<float*>(sc + B.key_grads), *grads, par, static_cast<hipStream_t>(stream));
 }
 

@@ -27,12 +27,65 @@ namespace {
 
 constexpr int kKeyFloats = GS355_KEY_GRAD_FLOATS;  // per-key record: dpx, dpy, dconic xyz, dopacity, drgb, ddepth, 2 unused
 
-// Record slot of the key (tile, Gaussian): the Gaussian's keys in the order its tile rectangle is walked
-// (row by row), after those of all Gaussians before it.
-__device__ __forceinline__ uint32_t key_slot(uint32_t first, uint64_t rect, int tile_x, int tile_y)
+// Where a Gaussian's records lie: those of its tile rectangle, row by row, from some first slot on.  The blend needs the
+// slot of one tile (tx, ty) per key: base + ty * width + tx with base = first - y0 * width - x0 (modulo 2^32), eight bytes
+// from one place (first slot and rectangle took two cache lines per key, of the four to five that a key costs: blend
+// backward 1109 -> 1013 us at 6M Gaussians, 1080p).
+struct RecordSlots {
+    uint32_t base, width;
+};
+struct RecordRun {
+    uint32_t first, n;
+};
+__device__ __forceinline__ uint32_t rect_width(uint64_t rect) { return ((uint32_t)(rect >> 32) & 0xffffu) - ((uint32_t)rect & 0xffffu); }
+__device__ __forceinline__ RecordRun record_run(RecordSlots s, uint64_t rect)
 {
-    const int x0 = (int)(rect & 0xffffu), y0 = (int)((rect >> 16) & 0xffffu), x1 = (int)((rect >> 32) & 0xffffu);
-    return first + (uint32_t)((tile_y - y0) * (x1 - x0) + (tile_x - x0));
+    const uint32_t x0 = (uint32_t)rect & 0xffffu, y0 = (uint32_t)(rect >> 16) & 0xffffu, y1 = (uint32_t)(rect >> 48);
+    return {s.base + y0 * s.width + x0, (y1 - y0) * s.width};
+}
+
+// Slots of all Gaussians: a workgroup adds up the rectangles of its 8192 Gaussians and takes that many slots from one
+// counter (1024 Gaussians per request: 73 us at 6M Gaussians, the requests being served one after the other).  Which
+// workgroup gets which slots varies between runs, the order of a Gaussian's own records does not, and nothing else enters
+// a sum.
+constexpr int kSlotItems = 8, kSlotThreads = 1024;
+__global__ __launch_bounds__(kSlotThreads) void record_slots_kernel(int P, const uint64_t* __restrict__ rects,
+                                                                    uint32_t* __restrict__ next,
+                                                                    RecordSlots* __restrict__ slots)
+{
+    __shared__ uint32_t s_wave[kSlotThreads / 64], s_first;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int first = (int)blockIdx.x * kSlotItems * kSlotThreads + (int)threadIdx.x;
+    uint64_t rect[kSlotItems];
+#pragma unroll
+    for (int k = 0; k < kSlotItems; ++k) rect[k] = first + k * kSlotThreads < P ? rects[first + k * kSlotThreads] : 0ull;
+    uint32_t sum = 0;
+#pragma unroll
+    for (int k = 0; k < kSlotItems; ++k) sum += record_run({0u, rect_width(rect[k])}, rect[k]).n;
+    uint32_t inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t up = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += up;
+    }
+    if (lane == 63) s_wave[wave] = inc;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kSlotThreads / 64; ++w) {
+        before += w < wave ? s_wave[w] : 0u;
+        all += s_wave[w];
+    }
+    if (threadIdx.x == 0) s_first = atomicAdd(next, all);
+    __syncthreads();
+    uint32_t at = s_first + before + inc - sum;
+#pragma unroll
+    for (int k = 0; k < kSlotItems; ++k) {
+        const uint32_t width = rect_width(rect[k]);
+        const RecordRun run = record_run({0u, width}, rect[k]);  // (its first: the slot of the rectangle's corner)
+        if (first + k * kSlotThreads < P) slots[first + k * kSlotThreads] = {at - run.first, width};
+        at += run.n;
+    }
 }
 
 // Value of lane `kLane` of each quad of lanes, in all four of them.
@@ -79,15 +132,15 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     FrameArgs f, const gs355_header* __restrict__ header, const uint32_t* __restrict__ ranges,
     const uint32_t* __restrict__ values, const float* __restrict__ records, const float* __restrict__ image,
     const float* __restrict__ out_depth, const float* __restrict__ out_alpha, const float* __restrict__ g_image,
-    const float* __restrict__ g_depth, const float* __restrict__ g_alpha, const uint64_t* __restrict__ rects,
-    const uint32_t* __restrict__ first_key, float* __restrict__ key_grads)
+    const float* __restrict__ g_depth, const float* __restrict__ g_alpha, const RecordSlots* __restrict__ slots,
+    float* __restrict__ key_grads)
 {
     // staged Gaussians per round, four threads each (96 and 128 measured 1 and 9 % slower: fewer resident workgroups)
     constexpr int kBatch = 64;
     // (entry kBatch: the null record, zero conic and log2(opacity) = -inf, which no pixel accepts; nothing reads its sums)
     __shared__ float4 s_a[kBatch + 1];  // px, py, -conic_x / 2, -conic_y   (rescaled as the forward blend stages them)
     __shared__ float4 s_b[kBatch + 1];  // -conic_z / 2, log2(opacity), r, g
-    __shared__ float4 s_c[kBatch + 1];  // b, depth, reach_x, reach_y
+    __shared__ float4 s_c[kBatch + 1];  // b, depth, mask of the blocks it can reach, unused
     // Sums of each wavefront: of d, d dx | d dy, d dy^2 | d dx dy, green | red, blue | d dx^2, depth.  A wavefront owns
     // its sums and serves its four blocks one after the other, so plain reads and writes do: float atomics on sums
     // shared by the workgroup take almost two cycles per lane of the CU's one LDS pipe, which bounded the kernel
@@ -106,8 +159,7 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     const int px = qx0 + (group & 1) * 4 + sub, py = qy0 + (group >> 1) * 4 + row;
     const bool inside = px < f.W && py < f.H;
     const float pxf = (float)px, pyf = (float)py;
-    const float x_lo0 = (float)qx0, x_hi0 = (float)(qx0 + 3), x_lo1 = (float)(qx0 + 4), x_hi1 = (float)(qx0 + 7);
-    const float y_lo0 = (float)qy0, y_hi0 = (float)(qy0 + 3), y_lo1 = (float)(qy0 + 4), y_hi1 = (float)(qy0 + 7);
+    const int first_bit = 8 * (wave >> 1) + 2 * (wave & 1);  // the quadrant's first block in a record's mask
     constexpr uint64_t kBlockLanes = 0x000F000F000F000Full;  // block 0's lanes: four of each row
 
     float g0 = 0.f, g1 = 0.f, g2 = 0.f, g3 = 0.f;  // dL/d(r, g, b, depth) of this pixel
@@ -146,19 +198,30 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
         const int count = (int)min((uint32_t)kBatch, hi - base);
         if (staged < count) {
             const uint32_t g = values[base + staged];
+            float4 v = reinterpret_cast<const float4*>(records + (size_t)g * kRecordFloats)[min(part, 2)];
             if (part == 3) {
-                s_slot[staged] = key_slot(first_key[g], rects[g], tile_x, tile_y);
-            } else {
-                float4 v = reinterpret_cast<const float4*>(records + (size_t)g * kRecordFloats)[part];
-                if (part == 0) {
-                    v.z *= -0.5f;
-                    v.w = -v.w;
-                } else if (part == 1) {  // (as the forward blend: a negative opacity never blends)
-                    v.x *= -0.5f;
-                    v.y = __builtin_amdgcn_logf(v.y < 0.0f ? 0.0f : v.y);
-                }
-                (part == 0 ? s_a : part == 1 ? s_b : s_c)[staged] = v;
+                const RecordSlots at = slots[g];
+                s_slot[staged] = at.base + (uint32_t)tile_y * at.width + (uint32_t)tile_x;
             }
+            // thread `part` tests the tile's block row `part`
+            const TileReach reach(quad_lane<0>(v.x), quad_lane<0>(v.y), quad_lane<0>(v.z), quad_lane<0>(v.w),
+                                  quad_lane<1>(v.x), quad_lane<2>(v.z), quad_lane<2>(v.w), (float)(tile_x * kTile),
+                                  (float)(tile_y * kTile));
+            const float row_mask = __uint_as_float(reach.row((float)part) << (4 * part));
+            const uint32_t mask = __float_as_uint(quad_lane<0>(row_mask)) | __float_as_uint(quad_lane<1>(row_mask)) |
+                                  __float_as_uint(quad_lane<2>(row_mask)) | __float_as_uint(quad_lane<3>(row_mask));
+            if (part == 0) {
+                v.z *= -0.5f;
+                v.w = -v.w;
+            } else if (part == 1) {  // (as the forward blend: a negative opacity never blends)
+                v.x *= -0.5f;
+                v.y = __builtin_amdgcn_logf(v.y < 0.0f ? 0.0f : v.y);
+            } else {
+                v.z = __uint_as_float(mask);
+            }
+            if (part < 3) (part == 0 ? s_a : part == 1 ? s_b : s_c)[staged] = v;
+        } else if (part == 2) {
+            s_c[staged].z = 0.0f;  // (no record: reaches no block)
         }
         __syncthreads();
         if ((s_wave_done[0] & s_wave_done[1] & s_wave_done[2] & s_wave_done[3]) != 0u) break;
@@ -166,19 +229,11 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
             // ---- lists: which staged Gaussians reach which 4x4 block (lane = Gaussian), as the forward blend ----
             uint32_t len[4] = {0u, 0u, 0u, 0u};
             {
-                // lane masks straight from the comparisons, combined in scalar registers (as the forward blend)
-                const uint64_t valid = __ballot(lane < count);  // (slots past `count` hold older records)
-                const float4 a = s_a[lane];
-                const float4 c = s_c[lane];
-                const float bx_lo = a.x - c.z, bx_hi = a.x + c.z, by_lo = a.y - c.w, by_hi = a.y + c.w;
-                const uint64_t in_x0 = __ballot(bx_hi >= x_lo0) & __ballot(bx_lo <= x_hi0) & valid;
-                const uint64_t in_x1 = __ballot(bx_hi >= x_lo1) & __ballot(bx_lo <= x_hi1) & valid;
-                const uint64_t in_y0 = __ballot(by_hi >= y_lo0) & __ballot(by_lo <= y_hi0);
-                const uint64_t in_y1 = __ballot(by_hi >= y_lo1) & __ballot(by_lo <= y_hi1);
+                const uint32_t reached = __float_as_uint(s_c[lane].z) >> first_bit;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
                     if ((live & (kBlockLanes << (4 * b))) == 0ull) continue;  // (all of the block's pixels have finished)
-                    const uint64_t m = ((b & 1) ? in_x1 : in_x0) & ((b >> 1) ? in_y1 : in_y0);
+                    const uint64_t m = __ballot((reached & (1u << (4 * (b >> 1) + (b & 1)))) != 0u);
                     if (__builtin_amdgcn_inverse_ballot_w64(m)) s_list[wave][b][lanes_below_in(m)] = (uint8_t)lane;
                     len[b] = (uint32_t)__popcll(m);
                 }
@@ -307,9 +362,9 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     }
     // keys the tile never reached (every pixel finished before them) contribute nothing: every record is written
     for (uint32_t j = base + tid; j < hi; j += 256) {
-        const uint32_t g = values[j];
-        float4* __restrict__ dst =
-            reinterpret_cast<float4*>(key_grads + (size_t)key_slot(first_key[g], rects[g], tile_x, tile_y) * kKeyFloats);
+        const RecordSlots at = slots[values[j]];
+        const uint32_t slot = at.base + (uint32_t)tile_y * at.width + (uint32_t)tile_x;
+        float4* __restrict__ dst = reinterpret_cast<float4*>(key_grads + (size_t)slot * kKeyFloats);
         dst[0] = dst[1] = dst[2] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
 }
@@ -439,15 +494,17 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
 // Sixteen records side by side, three lanes each, three such rounds in flight; the first record is overwritten once all
 // of them have been read (its new value depends on every one).
 __global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __restrict__ radii,
-                                                        const uint32_t* __restrict__ tiles_touched,
-                                                        const uint32_t* __restrict__ first_key, float* key_grads)
+                                                        const uint64_t* __restrict__ rects,
+                                                        const RecordSlots* __restrict__ slots, float* key_grads)
 {
     const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= P) return;
-    const uint32_t n = radii[i] > 0 ? tiles_touched[i] : 0u;
+    if (radii[i] <= 0) return;
+    const RecordRun run = record_run(slots[i], rects[i]);
+    const uint32_t n = run.n;
     if (n <= kSerialRecords) return;  // (uniform over the wavefront)
     const int slot = lane / 3, part = lane % 3;
-    float4* rec = reinterpret_cast<float4*>(key_grads) + (size_t)first_key[i] * (kKeyFloats / 4) + part;
+    float4* rec = reinterpret_cast<float4*>(key_grads) + (size_t)run.first * (kKeyFloats / 4) + part;
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
     if (slot < 16) {
         for (uint32_t k0 = (uint32_t)slot; k0 < n; k0 += 48) {
@@ -477,8 +534,8 @@ template <int kMode, bool kStored>
 __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kernel(FrameArgs f, gs355_gaussians g,
                                                                   const int32_t* __restrict__ radii,
                                                                   const float* __restrict__ records,
-                                                                  const uint32_t* __restrict__ tiles_touched,
-                                                                  const uint32_t* __restrict__ first_key,
+                                                                  const uint64_t* __restrict__ rects,
+                                                                  const RecordSlots* __restrict__ slots,
                                                                   const float* __restrict__ key_grads,
                                                                   gs355_gradients out, ParameterArgs par, bool summed)
 {
@@ -510,8 +567,8 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
     float gcol[3] = {0.f, 0.f, 0.f};
     float nx = 0.f, ny = 0.f, nz = 0.f, inv_len = 0.f;
     int K = 0;
-    uint32_t n_keys = alive ? tiles_touched[si] : 0u;
-    const uint32_t first_record = alive ? first_key[si] : 0u;
+    const RecordRun run = alive ? record_run(slots[si], rects[si]) : RecordRun{0u, 0u};
+    uint32_t n_keys = run.n;
     if (summed && n_keys > kSerialRecords) n_keys = 1u;  // (sum_large_kernel has added them into the first)
     // kStored: the wavefront's rows as one run of float4, and the up to three floats behind the last whole one.  They
     // travel from memory to LDS without passing through registers, requested before anything else is waited for: held
@@ -548,7 +605,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
             for (int c = 0; c < 3; ++c) in_rgb[c] = records[si * kRecordFloats + 6 + c];
     }
     float4 A0, A1, A2;
-    sum_records(key_grads, n_keys, first_record, mine + kPartialsAt, A0, A1, A2);
+    sum_records(key_grads, n_keys, run.first, mine + kPartialsAt, A0, A1, A2);
     if (alive) {
         const float* __restrict__ V = f.viewmatrix;
         const float* __restrict__ Pm = f.projmatrix;
@@ -858,17 +915,21 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
 
 int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const gs355_header* header,
                            const uint32_t* ranges, const uint32_t* values, const float* records,
-                           const uint32_t* tiles_touched, const uint64_t* rects, const gs355_backward_inputs& in,
-                           uint32_t* first_key, uint32_t* scan_tmp, float* key_grads, const gs355_gradients& out,
-                           const ParameterArgs* par, hipStream_t s)
+                           const uint64_t* rects, const gs355_backward_inputs& in, uint2* record_slots, uint32_t* next_slot,
+                           float* key_grads, const gs355_gradients& out, const ParameterArgs* par, hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
-    int rc = launch_exclusive_scan(tiles_touched, first_key, (size_t)g.P, scan_tmp, s);
+    int rc = launch_fill_u32(next_slot, 1, 0u, s);
     if (rc) return rc;
+    RecordSlots* slots = reinterpret_cast<RecordSlots*>(record_slots);
+    hipLaunchKernelGGL(record_slots_kernel, dim3((g.P + kSlotThreads * kSlotItems - 1) / (kSlotThreads * kSlotItems)),
+                       dim3(kSlotThreads), 0, s, g.P,
+                       rects, next_slot, slots);
+    GS355_CHECK_LAUNCH("record slots");
     const int tiles = f.grid_x * f.grid_y;
     auto blend = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(tiles), dim3(256), 0, s, f, header, ranges, values, records, in.image, in.depth,
-                           in.alpha, in.dL_dimage, in.dL_ddepth, in.dL_dalpha, rects, first_key, key_grads);
+                           in.alpha, in.dL_dimage, in.dL_ddepth, in.dL_dalpha, slots, key_grads);
     };
     if (in.dL_ddepth)
         blend(blend_backward_kernel<true>);
@@ -880,12 +941,12 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     const dim3 grid((g.P + 255) / 256), block(256);
     const bool summed = g.P <= kSumAheadMax;
     if (summed) {
-        hipLaunchKernelGGL(sum_large_kernel, dim3((g.P + 3) / 4), dim3(256), 0, s, g.P, in.radii, tiles_touched, first_key,
+        hipLaunchKernelGGL(sum_large_kernel, dim3((g.P + 3) / 4), dim3(256), 0, s, g.P, in.radii, rects, slots,
                            key_grads);
         GS355_CHECK_LAUNCH("record sums");
     }
     auto launch = [&](auto kernel, const ParameterArgs& p) {
-        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, tiles_touched, first_key, key_grads, out, p,
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, rects, slots, key_grads, out, p,
                            summed);
     };
     if (par) {

@@ -128,52 +128,13 @@ __device__ __forceinline__ void blend_one(PixelState& p, float pxf, float pyf, c
     }
 }
 
-// Which of a tile's sixteen 4x4 blocks (bit 4 row + column) the splat's alpha >= 1/255 ellipse can reach.  The record's
-// reach is the half-extent (Rx, Ry) of the ellipse's bounding box; with rho = -conic_y / sqrt(conic_x conic_z) the
-// ellipse's span at dy = Ry t is Rx (rho t +- sqrt((1 - rho^2)(1 - t^2))).  Over a row of blocks, t in [t0, t1], the upper
-// end is largest at t = rho pulled into the interval, the lower end smallest at -rho: two spans per block row instead of
-// the bounding box for all of them.  (A row beyond the ellipse gives sqrt(negative) = NaN, and no blocks.)
-// The reach contains the rounding of the exponent (gs355_preprocess); `slack` covers that its margin was added to Rx and Ry
-// separately, which bends t by up to 0.002 + 0.02 / Ry, and the rounding here.
-// With the bounding box alone 36 % of the list entries of a scene of large splats (21 % of small ones) reached no pixel.
-// About 115 vector instructions per 64 records and tile, against some 20 per list entry left out: blend 198 -> 161 us
-// (1M large splats, 1080p), 361 -> 334 us (6M), 969 -> 903 us (20M, 4K), 304 -> 290 us (500k anchors).
-__device__ __forceinline__ uint32_t block_mask(float px, float py, float qx, float qy, float qz, float reach_x, float reach_y,
-                                               float tile_x0, float tile_y0)
-{
-    const float inv_y = __builtin_amdgcn_rcpf(reach_y);
-    const float rho = fmaxf(-1.0f, fminf(1.0f, -qy * __builtin_amdgcn_rsqf(qx * qz)));
-    const float across = __builtin_amdgcn_sqrtf(fmaxf(0.0f, __builtin_fmaf(-rho, rho, 1.0f)) + 1e-5f);
-    const float slack = __builtin_fmaf(reach_x, __builtin_fmaf(0.02f, inv_y, 0.002f), 0.01f);
-    const float x = px - tile_x0, y = tile_y0 - py;
-    const float t_first = y * inv_y, t_step = 4.0f * inv_y, t_span = 3.0f * inv_y;
-    // block columns below n1 = trunc(right end + 1) and from n0 = trunc(left end + almost 1) on are reached
-    const float right = __builtin_fmaf(0.25f, x + slack, 1.0f), left = __builtin_fmaf(0.25f, x - slack, 0.2499f);
-    const float scale = 0.25f * reach_x;
-    uint32_t mask = 0u;
-#pragma unroll
-    for (int b = 3; b >= 0; --b) {
-        const float t0 = __builtin_fmaf((float)b, t_step, t_first), t1 = t0 + t_span;
-        const float up = __builtin_amdgcn_fmed3f(rho, t0, t1), down = __builtin_amdgcn_fmed3f(-rho, t0, t1);
-        const float half_up = __builtin_amdgcn_sqrtf(__builtin_fmaf(-up, up, 1.0f));
-        const float half_down = __builtin_amdgcn_sqrtf(__builtin_fmaf(-down, down, 1.0f));
-        const float hi = __builtin_fmaf(scale, __builtin_fmaf(rho, up, across * half_up), right);
-        const float lo = __builtin_fmaf(scale, __builtin_fmaf(rho, down, -(across * half_down)), left);
-        const uint32_t n1 = (uint32_t)__builtin_amdgcn_fmed3f(hi, 0.0f, 4.0f), n0 = (uint32_t)__builtin_amdgcn_fmed3f(lo, 0.0f, 4.0f);
-        mask = (mask << 4) | (((1u << n1) - 1u) & ~((1u << n0) - 1u));
-    }
-    if (!(reach_x < __builtin_inff())) mask = 0xFFFFu;  // never culled
-    if (reach_x < 0.0f) mask = 0u;                      // never visible
-    return mask;
-}
-
 using ListEntry = uint16_t;
 constexpr int kBatch = 256;            // records staged per round
 constexpr uint32_t kNullEntry = kBatch * 16;  // list entry of the null record (opacity 0: rejected by every pixel)
 constexpr int kListWords = kBatch + 8;  // entries per list: a batch, padded to a multiple of four, one round read ahead
 
 // kCull: staging a record also finds which of the tile's sixteen 4x4 blocks its
-// alpha >= 1/255 ellipse can reach (block_mask), and each wavefront appends the
+// alpha >= 1/255 ellipse can reach (TileReach), and each wavefront appends the
 // Gaussians that reach its four blocks, in depth order, to the blocks' lists.  A (block, Gaussian) pair
 // that is left out is one whose 16 pixels would all have taken the
 // `alpha < 1/255` branch, and every pixel still sees its Gaussians front to
@@ -192,7 +153,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
                                                     float* __restrict__ out_depth, float* __restrict__ out_alpha)
 {
     __shared__ float4 s_a[kBatch + 1];  // px, py, -conic_x / 2, -conic_y          (+ the null record)
-    __shared__ float4 s_b[kBatch + 1];  // -conic_z / 2, log2(opacity), block_mask, unused
+    __shared__ float4 s_b[kBatch + 1];  // -conic_z / 2, log2(opacity), mask of the blocks it can reach, unused
     __shared__ float4 s_c[kBatch + 1];  // r, g, b, depth
     __shared__ uint32_t s_wave_state[4];  // bit 0: all pixels of the wavefront finished; 1: it staged a channel that is not finite
     // per wavefront and 4x4 block: byte offsets of the staged records of the Gaussians that can reach the block
@@ -268,8 +229,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
             // a negative opacity gives a negative alpha, which every pixel rejects: log2(0) = -inf does the same
             const float log2o = __builtin_amdgcn_logf(r1.y < 0.0f ? 0.0f : r1.y);
             s_a[tid] = make_float4(r0.x, r0.y, -0.5f * r0.z, -r0.w);
-            const uint32_t mask = !kCull ? 0u : block_mask(r0.x, r0.y, r0.z, r0.w, r1.x, r2.z, r2.w, (float)(tile_x * kTile),
-                                                           (float)(tile_y * kTile));
+            uint32_t mask = 0u;
+            if (kCull) {
+                const TileReach reach(r0.x, r0.y, r0.z, r0.w, r1.x, r2.z, r2.w, (float)(tile_x * kTile), (float)(tile_y * kTile));
+#pragma unroll
+                for (int b = 3; b >= 0; --b) mask = (mask << 4) | reach.row((float)b);
+            }
             s_b[tid] = make_float4(-0.5f * r1.x, log2o, __uint_as_float(mask), 0.f);
             s_c[tid] = make_float4(r1.z, r1.w, r2.x, r2.y);
             // (the sum of the magnitudes overflows only where one of them is beyond 2^125: then the careful way is right too)
