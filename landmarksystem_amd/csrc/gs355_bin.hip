@@ -29,6 +29,45 @@ namespace {
 constexpr int kInlineTiles = 32;
 constexpr int kBinItems = 4;      // Gaussians per thread and round of the binning walk
 
+// Gaussians per slice: at most kBinMaxGroups slices, in whole rounds of a workgroup for large frames, in whole wavefronts
+// for small ones, so that a frame of a few thousand Gaussians is still spread over the chip.
+__host__ __device__ __forceinline__ int slice_size(int P, int groups)
+{
+    const int per = (P + groups - 1) / groups, unit = per > kBinThreads / 2 ? kBinThreads : 64;
+    const int whole = (per + unit - 1) / unit * unit;
+    return whole < 64 ? 64 : whole;
+}
+
+// A slice of at most half a workgroup's threads gives each of its Gaussians 2, 4, 8 or 16 lanes, which take the tiles of
+// its rectangle in turn: with a lane per Gaussian a slice of large splats is a chain of LDS requests as long as its
+// largest rectangle, on the few compute units that a small frame's slices occupy.  10k Gaussians at 256x256 (26 tiles
+// each): count 13.4 -> 4.7 us, scatter 29.0 -> 7.0 us.
+__device__ __forceinline__ int lanes_per_gaussian(int per_group)
+{
+    int lanes = 1;
+    while (lanes < 16 && 2 * lanes * per_group <= kBinThreads) lanes *= 2;
+    return lanes;
+}
+
+struct TileRect {
+    int x0, y0, width, area;
+    float inv_width;
+    __device__ __forceinline__ explicit TileRect(uint64_t r)
+        : x0((int)(r & 0xFFFF)), y0((int)((r >> 16) & 0xFFFF)), width((int)((r >> 32) & 0xFFFF) - x0),
+          area(width * ((int)(r >> 48) - y0)), inv_width(__builtin_amdgcn_rcpf((float)width))
+    {
+    }
+    // tile number e of the rectangle, row by row (the quotient by the reciprocal is off by one at most)
+    __device__ __forceinline__ int tile(int e, int grid_x) const
+    {
+        int row = (int)(((float)e + 0.5f) * inv_width);
+        int col = e - row * width;
+        if (col < 0) { --row; col += width; }
+        else if (col >= width) { ++row; col -= width; }
+        return (y0 + row) * grid_x + x0 + col;
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Counting.  Workgroup c owns Gaussians [c * per_group, (c+1) * per_group) and a private array of counters in LDS.
 //   up to kBinMaxTiles tiles:  one counter per tile; matrix[c][t] = pairs of this slice that fall in tile t.  No
@@ -47,10 +86,9 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
     __shared__ uint32_t s_queue[kBinItems * kBinThreads];
     __shared__ uint32_t s_nqueue, s_visible;
 
-    if (f.p_device) {  // the slices follow the device-side count: as many Gaussians per workgroup as on the host side
+    if (f.p_device) {  // the slices follow the device-side count
         P = effective_count(f, P);
-        per_group = (P + (int)gridDim.x - 1) / (int)gridDim.x;
-        per_group = max(kBinThreads, (per_group + kBinThreads - 1) / kBinThreads * kBinThreads);
+        per_group = slice_size(P, (int)gridDim.x);
     }
     const int T = f.grid_x * f.grid_y;
     const int counters = kWide ? (T + kCoarseTiles - 1) >> kCoarseShift : T;
@@ -61,64 +99,87 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
     const int g_end = min(P, g_begin + per_group);
     uint32_t visible = 0;
     auto add = [&](int t) { atomicAdd(&s_count[kWide ? t >> kCoarseShift : t], 1u); };
+    // large rectangles: one per wavefront at a time, 64 tiles per step (the sixteen wavefronts work on sixteen
+    // rectangles side by side; the whole workgroup on one rectangle left most of its threads idle)
+    auto walk_queue = [&]() {
+        const uint32_t nq = s_nqueue;
+        uint32_t k = (uint32_t)tid >> 6;
+        uint64_t next = k < nq ? rects[s_queue[k]] : 0ull;
+        while (k < nq) {
+            const TileRect q(next);
+            k += kBinThreads / 64;
+            if (k < nq) next = rects[s_queue[k]];
+            for (int e = tid & 63; e < q.area; e += 64) add(q.tile(e, f.grid_x));
+        }
+    };
 
-    // a thread's Gaussians of a round: their rectangles are requested together, and those of the next round before
-    // this round's are walked (a slice is a dozen rounds or more, each otherwise a memory latency plus its walk)
-    uint64_t ahead[kBinItems];
-#pragma unroll
-    for (int u = 0; u < kBinItems; ++u) ahead[u] = g_begin < g_end ? rects[min(g_begin + u * kBinThreads + tid, g_end - 1)] : 0ull;
-    for (int base = g_begin; base < g_end; base += kBinItems * kBinThreads) {
+    const int lanes = lanes_per_gaussian(per_group);
+    if (lanes > 1) {  // (uniform; a single round)
         if (tid == 0) s_nqueue = 0;
         __syncthreads();
-        uint64_t rr[kBinItems];
-#pragma unroll
-        for (int u = 0; u < kBinItems; ++u) rr[u] = ahead[u];
-        if (base + kBinItems * kBinThreads < g_end) {  // uniform
-#pragma unroll
-            for (int u = 0; u < kBinItems; ++u)
-                ahead[u] = rects[min(base + (kBinItems + u) * kBinThreads + tid, g_end - 1)];
-        }
-#pragma unroll
-        for (int u = 0; u < kBinItems; ++u) {
-            const int i = base + u * kBinThreads + tid;
-            if (i < g_end) {
-                const uint64_t r = rr[u];
-                const int x0 = (int)(r & 0xFFFF), y0 = (int)((r >> 16) & 0xFFFF), x1 = (int)((r >> 32) & 0xFFFF),
-                          y1 = (int)(r >> 48);
-                const int area = (x1 - x0) * (y1 - y0);
-                if (area > 0) {
-                    ++visible;
-                    if (area > kInlineTiles) {
-                        s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
-                    } else if (kWide) {  // a rectangle row: one request per coarse bin it crosses
-                        for (int ty = y0; ty < y1; ++ty) {
-                            int ta = ty * f.grid_x + x0;
-                            const int tb = ty * f.grid_x + x1;
-                            while (ta < tb) {
-                                const int stop = min(tb, ((ta >> kCoarseShift) + 1) << kCoarseShift);
-                                atomicAdd(&s_count[ta >> kCoarseShift], (uint32_t)(stop - ta));
-                                ta = stop;
-                            }
-                        }
-                    } else {
-                        for (int ty = y0; ty < y1; ++ty)
-                            for (int tx = x0; tx < x1; ++tx) add(ty * f.grid_x + tx);
-                    }
-                }
+        const int i = g_begin + tid / lanes, sub = tid % lanes;
+        if (i < g_end) {
+            const TileRect q(rects[i]);
+            if (sub == 0 && q.area > 0) ++visible;
+            if (q.area > kInlineTiles * lanes) {
+                if (sub == 0) s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
+            } else {
+                for (int e = sub; e < q.area; e += lanes) add(q.tile(e, f.grid_x));
             }
         }
         __syncthreads();
-        // large rectangles: one per wavefront at a time, 64 tiles per step (the sixteen wavefronts work on sixteen
-        // rectangles side by side; the whole workgroup on one rectangle left most of its threads idle)
-        const uint32_t nq = s_nqueue;
-        for (uint32_t k = (uint32_t)tid >> 6; k < nq; k += kBinThreads / 64) {
-            const uint64_t r = rects[s_queue[k]];
-            const int x0 = (int)(r & 0xFFFF), y0 = (int)((r >> 16) & 0xFFFF), x1 = (int)((r >> 32) & 0xFFFF),
-                      y1 = (int)(r >> 48);
-            const int w = x1 - x0, area = w * (y1 - y0);
-            for (int e = tid & 63; e < area; e += 64) add((y0 + e / w) * f.grid_x + x0 + e % w);
-        }
+        walk_queue();
         __syncthreads();
+    } else {
+        // a thread's Gaussians of a round: their rectangles are requested together, and those of the next round before
+        // this round's are walked (a slice is a dozen rounds or more, each otherwise a memory latency plus its walk)
+        uint64_t ahead[kBinItems];
+#pragma unroll
+        for (int u = 0; u < kBinItems; ++u) ahead[u] = g_begin < g_end ? rects[min(g_begin + u * kBinThreads + tid, g_end - 1)] : 0ull;
+        for (int base = g_begin; base < g_end; base += kBinItems * kBinThreads) {
+            if (tid == 0) s_nqueue = 0;
+            __syncthreads();
+            uint64_t rr[kBinItems];
+#pragma unroll
+            for (int u = 0; u < kBinItems; ++u) rr[u] = ahead[u];
+            if (base + kBinItems * kBinThreads < g_end) {  // uniform
+#pragma unroll
+                for (int u = 0; u < kBinItems; ++u)
+                    ahead[u] = rects[min(base + (kBinItems + u) * kBinThreads + tid, g_end - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < kBinItems; ++u) {
+                const int i = base + u * kBinThreads + tid;
+                if (i < g_end) {
+                    const uint64_t r = rr[u];
+                    const int x0 = (int)(r & 0xFFFF), y0 = (int)((r >> 16) & 0xFFFF), x1 = (int)((r >> 32) & 0xFFFF),
+                              y1 = (int)(r >> 48);
+                    const int area = (x1 - x0) * (y1 - y0);
+                    if (area > 0) {
+                        ++visible;
+                        if (area > kInlineTiles) {
+                            s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
+                        } else if (kWide) {  // a rectangle row: one request per coarse bin it crosses
+                            for (int ty = y0; ty < y1; ++ty) {
+                                int ta = ty * f.grid_x + x0;
+                                const int tb = ty * f.grid_x + x1;
+                                while (ta < tb) {
+                                    const int stop = min(tb, ((ta >> kCoarseShift) + 1) << kCoarseShift);
+                                    atomicAdd(&s_count[ta >> kCoarseShift], (uint32_t)(stop - ta));
+                                    ta = stop;
+                                }
+                            }
+                        } else {
+                            for (int ty = y0; ty < y1; ++ty)
+                                for (int tx = x0; tx < x1; ++tx) add(ty * f.grid_x + tx);
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            walk_queue();
+            __syncthreads();
+        }
     }
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) visible += __shfl_down(visible, d, 64);
@@ -171,8 +232,7 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
     if (header->overflow || header->num_keys < min_keys || header->num_keys >= max_keys) return;
     if (f.p_device) {
         P = effective_count(f, P);
-        per_group = (P + (int)gridDim.x - 1) / (int)gridDim.x;
-        per_group = max(kBinThreads, (per_group + kBinThreads - 1) / kBinThreads * kBinThreads);
+        per_group = slice_size(P, (int)gridDim.x);
     }
     constexpr int kSpan = 1 << kShift;
     const int T = f.grid_x * f.grid_y, bins = (T + kSpan - 1) >> kShift;
@@ -209,6 +269,46 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
         }
     };
 
+    auto emit_tile = [&](int t, uint64_t payload) {
+        dst[atomicAdd(&s_bin[t >> kShift], 1u)] = payload | (uint64_t)(t & (kSpan - 1));
+    };
+    auto payload_of = [&](uint32_t depth, uint32_t i) { return ((uint64_t)depth << 32) | ((uint64_t)i << kShift); };
+    // large rectangles: one per wavefront at a time, 64 tiles per step
+    auto walk_queue = [&]() {
+        const uint32_t nq = s_nqueue;
+        uint32_t k = wave, gi = k < nq ? s_queue[k] : 0u, depth = k < nq ? depth_bits[gi] : 0u;
+        uint64_t next = k < nq ? rects[gi] : 0ull;
+        while (k < nq) {
+            const TileRect q(next);
+            const uint64_t payload = payload_of(depth, gi);
+            k += kBinThreads / 64;
+            if (k < nq) {
+                gi = s_queue[k];
+                next = rects[gi];
+                depth = depth_bits[gi];
+            }
+            for (int e = lane; e < q.area; e += 64) emit_tile(q.tile(e, f.grid_x), payload);
+        }
+    };
+    const int lanes = lanes_per_gaussian(per_group);
+    if (lanes > 1) {  // (uniform; a single round, as in the count)
+        if (tid == 0) s_nqueue = 0;
+        __syncthreads();
+        const int i = g_begin + tid / lanes, sub = tid % lanes;
+        if (i < g_end) {
+            const TileRect q(rects[i]);
+            const uint64_t payload = payload_of(depth_bits[i], (uint32_t)i);
+            if (q.area > kInlineTiles * lanes) {
+                if (sub == 0) s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
+            } else {
+                for (int e = sub; e < q.area; e += lanes) emit_tile(q.tile(e, f.grid_x), payload);
+            }
+        }
+        __syncthreads();
+        walk_queue();
+        return;
+    }
+
     for (int first = g_begin; first < g_end; first += kBinItems * kBinThreads) {
         if (tid == 0) s_nqueue = 0;
         __syncthreads();
@@ -231,27 +331,13 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
                 if (area > kInlineTiles) {
                     s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
                 } else if (area > 0) {
-                    const uint64_t payload = ((uint64_t)dd[u] << 32) | ((uint64_t)(uint32_t)i << kShift);
+                    const uint64_t payload = payload_of(dd[u], (uint32_t)i);
                     for (int ty = y0; ty < y1; ++ty) emit_row(ty * f.grid_x + x0, ty * f.grid_x + x1, payload);
                 }
             }
         }
         __syncthreads();
-        // large rectangles: one per wavefront at a time, 64 tiles per step
-        const uint32_t nq = s_nqueue;
-        for (uint32_t k = wave; k < nq; k += kBinThreads / 64) {
-            const uint32_t gi = s_queue[k];
-            const uint64_t r = rects[gi];
-            const int x0 = (int)(r & 0xFFFF), y0 = (int)((r >> 16) & 0xFFFF), x1 = (int)((r >> 32) & 0xFFFF),
-                      y1 = (int)(r >> 48);
-            const int w = x1 - x0, area = w * (y1 - y0);
-            const uint64_t payload = ((uint64_t)depth_bits[gi] << 32) | ((uint64_t)gi << kShift);
-            for (int e = lane; e < area; e += 64) {
-                const int t = (y0 + e / w) * f.grid_x + x0 + e % w;
-                const uint32_t slot = atomicAdd(&s_bin[t >> kShift], 1u);
-                dst[slot] = payload | (uint64_t)(t & (kSpan - 1));
-            }
-        }
+        walk_queue();
         __syncthreads();
     }
 }
@@ -458,54 +544,45 @@ __global__ __launch_bounds__(kFineThreads) void fine_count_kernel(const gs355_he
 }
 
 // Exclusive prefix of every tile's counts over the slices (in place), the
-// tile's total and the total of the workgroup's tiles.  A workgroup covers 64 tiles; its four wavefronts take a
-// quarter of the slices each (loads of a thread are issued in batches, so many
-// are in flight), exchange their quarter sums through LDS and write the
-// prefixes shifted by the quarters before them.
-__global__ __launch_bounds__(256) void slice_prefix_kernel(uint32_t* __restrict__ matrix, int groups, int tiles,
-                                                           uint32_t* __restrict__ totals,
-                                                           uint64_t* __restrict__ block_sums,
-                                                           uint32_t* __restrict__ bin_sums,
-                                                           uint32_t* __restrict__ block_classes,
-                                                           uint32_t* __restrict__ list_counts)
+// tile's total and the total of the workgroup's tiles.  A workgroup covers 64 tiles; its sixteen wavefronts take a
+// sixteenth of the slices each, all requested at once and kept in registers, exchange their sums through LDS and write the
+// prefixes shifted by the wavefronts' before them.  (Four wavefronts that read their quarter twice, sixteen slices at a
+// time, were a chain of eight memory latencies: 9.7 us for 1700 tiles, as many as for 8160.)
+constexpr int kPrefixParts = 16;
+constexpr int kPrefixRows = kBinMaxGroups / kPrefixParts;
+__global__ __launch_bounds__(64 * kPrefixParts) void slice_prefix_kernel(uint32_t* __restrict__ matrix, int groups, int tiles,
+                                                                         uint32_t* __restrict__ totals,
+                                                                         uint64_t* __restrict__ block_sums,
+                                                                         uint32_t* __restrict__ bin_sums,
+                                                                         uint32_t* __restrict__ block_classes,
+                                                                         uint32_t* __restrict__ list_counts)
 {
-    __shared__ uint32_t s_part[4][64];
+    __shared__ uint32_t s_part[kPrefixParts][64];
     if (blockIdx.x == 0 && threadIdx.x < 4) list_counts[threadIdx.x] = 0u;  // filled by tile_publish_kernel
     const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
     const int t = blockIdx.x * 64 + lane;
-    const int per = (groups + 3) / 4;
-    const int c0 = min(part * per, groups), c1 = min(c0 + per, groups);
+    const int per = (groups + kPrefixParts - 1) / kPrefixParts;  // <= kPrefixRows
+    const int c0 = min(part * per, groups), rows = min(per, groups - c0);
     const bool live = t < tiles;
-    // pass 1: sum of this thread's quarter
-    uint32_t sum = 0;
-    for (int c = c0; c < c1 && live; c += 16) {
-        uint32_t v[16];
+    uint32_t* __restrict__ column = matrix + (size_t)c0 * tiles + t;
+    uint32_t v[kPrefixRows], sum = 0;
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = matrix[(size_t)min(c + k, c1 - 1) * tiles + t];
+    for (int k = 0; k < kPrefixRows; ++k) v[k] = live && k < rows ? column[(size_t)k * tiles] : 0u;
 #pragma unroll
-        for (int k = 0; k < 16; ++k) sum += c + k < c1 ? v[k] : 0u;
-    }
+    for (int k = 0; k < kPrefixRows; ++k) sum += v[k];
     s_part[part][lane] = sum;
     __syncthreads();
     uint32_t run = 0, total = 0;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const uint32_t v = s_part[p][lane];
-        if (p < part) run += v;
-        total += v;
+    for (int p = 0; p < kPrefixParts; ++p) {
+        const uint32_t n = s_part[p][lane];
+        if (p < part) run += n;
+        total += n;
     }
-    // pass 2: the quarter's values again (now cached), replaced by the running sum before them
-    for (int c = c0; c < c1 && live; c += 16) {
-        uint32_t v[16];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = matrix[(size_t)min(c + k, c1 - 1) * tiles + t];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            if (c + k < c1) {
-                matrix[(size_t)(c + k) * tiles + t] = run;
-                run += v[k];
-            }
-        }
+    for (int k = 0; k < kPrefixRows; ++k) {
+        if (live && k < rows) column[(size_t)k * tiles] = run;
+        run += v[k];
     }
     if (part == 0) {
         if (live) totals[t] = total;
@@ -535,9 +612,11 @@ __global__ __launch_bounds__(256) void slice_prefix_kernel(uint32_t* __restrict_
 // workgroup waits for another and no separate scan pass is launched.  Workgroup 0 also writes the frame header and
 // the work list of the scatter's second level: chunk_base[b] = chunks of kFineChunk pairs in the coarse bins before
 // b, chunk_base[bins] = all (`bin_pairs`, the pairs per bin, may be the same array).  With kTiles the wavefronts
-// publish tile bases, the scatter's cursors, the ranges and the lists of buckets too large for the small sorter
-// (`lists[0..3]` cleared by an earlier kernel); without, the columns are coarse bins and only their bases are
-// written.  `totals` and `tile_base` may be the same array.  `header_known`: second layout of a frame (by tile,
+// publish tile bases, the scatter's cursors, the ranges and the lists of buckets too large for the small sorter;
+// without, the columns are coarse bins and only their bases are written.  Where the buckets per size class were counted
+// by block (`block_classes`, a byte per class), a block's places in the lists follow from the blocks before it, as its
+// slots do; else they are requested from the lists' counters (`lists[0..3]` cleared by an earlier kernel), which costs
+// three dependent round trips to memory (9.1 us at 1080p against 5.1).  `totals` and `tile_base` may be the same array.  `header_known`: second layout of a frame (by tile,
 // after the one by coarse bin): the header stands, and nothing is done on overflow.
 template <bool kTiles>
 __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* totals, uint32_t tiles,
@@ -550,47 +629,46 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
                                                            const uint32_t* bin_pairs, int bins, uint32_t* chunk_base,
                                                            const uint32_t* __restrict__ block_classes)
 {
-    __shared__ uint64_t s_before[4], s_total[4];
-    __shared__ uint32_t s_vis[4], s_chunks[4], s_class[3];
+    __shared__ uint64_t s_before[4], s_total[4], s_class_before[4], s_class_total[4];
+    __shared__ uint32_t s_vis[4], s_chunks[4];
     if (header_known && header->overflow) return;
-    if (threadIdx.x < 3) s_class[threadIdx.x] = 0u;
-    __syncthreads();
+    // counts of the three classes, 21 bits each
+    auto classes_of = [&](uint32_t b) {
+        const uint32_t w = block_classes[b];
+        return (uint64_t)(w & 0xFFu) | ((uint64_t)((w >> 8) & 0xFFu) << 21) | ((uint64_t)((w >> 16) & 0xFFu) << 42);
+    };
+    auto class_count = [](uint64_t packed, int c) { return (uint32_t)(packed >> (21 * c)) & 0x1FFFFFu; };
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t first_block = blockIdx.x * 4u, block = first_block + (uint32_t)wave;
     {
-        uint64_t before = 0, total = 0;
+        uint64_t before = 0, total = 0, class_before = 0, class_total = 0;
         for (uint32_t b = threadIdx.x; b < n_blocks; b += 256u) {
             const uint64_t v = block_sums[b];
             total += v;
             before += b < first_block ? v : 0ull;
-        }
-        uint32_t vis = 0;
-        if (blockIdx.x == 0 && !header_known) {
-            for (int c = threadIdx.x; c < groups; c += 256) vis += group_visible[c];
-            // buckets per larger sorter size class, for the header (counted per block by the slice prefix)
             if (block_classes) {
-                uint32_t n1 = 0, n2 = 0, n3 = 0;
-                for (uint32_t b = threadIdx.x; b < n_blocks; b += 256u) {
-                    const uint32_t w = block_classes[b];
-                    n1 += w & 0xFFu;
-                    n2 += (w >> 8) & 0xFFu;
-                    n3 += (w >> 16) & 0xFFu;
-                }
-                if (n1) atomicAdd(&s_class[0], n1);
-                if (n2) atomicAdd(&s_class[1], n2);
-                if (n3) atomicAdd(&s_class[2], n3);
+                const uint64_t w = classes_of(b);
+                class_total += w;
+                class_before += b < first_block ? w : 0ull;
             }
         }
+        uint32_t vis = 0;
+        if (blockIdx.x == 0 && !header_known)
+            for (int c = threadIdx.x; c < groups; c += 256) vis += group_visible[c];
 #pragma unroll
         for (int d = 32; d > 0; d >>= 1) {
             before += __shfl_down(before, d, 64);
             total += __shfl_down(total, d, 64);
             vis += __shfl_down(vis, d, 64);
+            class_before += __shfl_down(class_before, d, 64);
+            class_total += __shfl_down(class_total, d, 64);
         }
         if (lane == 0) {
             s_before[wave] = before;
             s_total[wave] = total;
             s_vis[wave] = vis;
+            s_class_before[wave] = class_before;
+            s_class_total[wave] = class_total;
         }
     }
     __syncthreads();
@@ -602,13 +680,16 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         header->overflow = overflow ? 1u : 0u;
         header->num_visible = (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]);
         const bool counted = block_classes != nullptr;
-        for (int c = 0; c < 3; ++c) header->sort_class_count[c] = counted ? s_class[c] : 0xFFFFFFFFu;
+        const uint64_t in_class = (s_class_total[0] + s_class_total[1]) + (s_class_total[2] + s_class_total[3]);
+        for (int c = 0; c < 3; ++c) header->sort_class_count[c] = counted ? class_count(in_class, c) : 0xFFFFFFFFu;
+        if (counted && kTiles)
+            for (int c = 0; c < 3; ++c) lists[c] = class_count(in_class, c);
         if (header_copy) {  // (may be host memory: plain stores, complete when the kernel is)
             header_copy->num_keys_total = total;
             header_copy->num_keys = overflow ? n_cap : (uint32_t)total;
             header_copy->overflow = overflow ? 1u : 0u;
             header_copy->num_visible = (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]);
-            for (int c = 0; c < 3; ++c) header_copy->sort_class_count[c] = counted ? s_class[c] : 0xFFFFFFFFu;
+            for (int c = 0; c < 3; ++c) header_copy->sort_class_count[c] = counted ? class_count(in_class, c) : 0xFFFFFFFFu;
         }
     }
     if (overflow) return;  // later stages do nothing either
@@ -656,22 +737,29 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         ranges[2 * t + 1] = v ? first + v : 0u;
         tile_base[tiles + t] = first;  // the bucket's next free slot during the scatter
     }
-    // buckets beyond the smallest sorter's capacity go on the list of their size class (order within a list is free):
-    // one request per wavefront and class
+    // buckets beyond the smallest sorter's capacity go on the list of their size class (order within a list is free;
+    // without counts by block, one request per wavefront and class)
     int cls = -1;
     if (v > (uint32_t)kTileSortCap[3]) cls = -1;  // beyond the LDS sorters: sorted by its own workgroup of the class-0 kernel
     else if (v > (uint32_t)kTileSortCap[2]) cls = 2;
     else if (v > (uint32_t)kTileSortCap[1]) cls = 1;
     else if (v > (uint32_t)kTileSortCap[0]) cls = 0;
-    const uint64_t lanes_below = (1ull << lane) - 1ull;
+    uint64_t class_first = 0;
+    if (block_classes) {
+        class_first = (s_class_before[0] + s_class_before[1]) + (s_class_before[2] + s_class_before[3]);
+        for (int w = 0; w < wave; ++w) class_first += classes_of(first_block + (uint32_t)w);  // (earlier blocks exist)
+    }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < 3; ++c) {
         const uint64_t m = __ballot(cls == c);
         if (m == 0ull) continue;
-        uint32_t at = 0;
-        if (lane == __ffsll((unsigned long long)m) - 1) at = atomicAdd(&lists[c], (uint32_t)__popcll(m));
-        at = __shfl(at, __ffsll((unsigned long long)m) - 1, 64);
-        if (cls == c) lists[kListHeader + (size_t)c * tiles + at + (uint32_t)__popcll(m & lanes_below)] = t;
+        uint32_t at = class_count(class_first, c);
+        if (!block_classes) {
+            const int leader = __ffsll((unsigned long long)m) - 1;
+            if (lane == leader) at = atomicAdd(&lists[c], (uint32_t)__popcll(m));
+            at = __shfl(at, leader, 64);
+        }
+        if (cls == c) lists[kListHeader + (size_t)c * tiles + lanes_below_in(m, at)] = t;
     }
 }
 
@@ -1330,10 +1418,7 @@ __global__ __launch_bounds__(kT) void tile_sort_list_kernel(const gs355_header* 
 
 int bin_groups(int32_t P, int* per_group)
 {
-    // slices are multiples of the workgroup size so that every pass over a slice is full
-    int per = (P + kBinMaxGroups - 1) / kBinMaxGroups;
-    per = (per + kBinThreads - 1) / kBinThreads * kBinThreads;
-    if (per < kBinThreads) per = kBinThreads;
+    const int per = slice_size(P, kBinMaxGroups);
     *per_group = per;
     const int groups = (P + per - 1) / per;
     return groups < 1 ? 1 : groups;
@@ -1426,7 +1511,7 @@ int launch_tile_layout(int32_t P, uint32_t* matrix, const uint32_t* group_visibl
     uint32_t* block_classes = chunk_base + bins + 1;  // [ceil(tiles / 64)]
     if (tiles <= kBinMaxTiles) {
         // (the pairs of each coarse bin go to chunk_base, which the block scan turns into chunk bases in place)
-        hipLaunchKernelGGL(slice_prefix_kernel, dim3((tiles + 63) / 64), dim3(256), 0, s, matrix, groups, tiles,
+        hipLaunchKernelGGL(slice_prefix_kernel, dim3((tiles + 63) / 64), dim3(64 * kPrefixParts), 0, s, matrix, groups, tiles,
                            tile_base, blocks, chunk_base, block_classes, lists);
         GS355_CHECK_LAUNCH("bin: slice prefix");
         return launch_layout<true>(tile_base, tile_base, tiles, blocks, group_visible, groups, n_cap, header, header_copy, false, ranges,
@@ -1435,7 +1520,7 @@ int launch_tile_layout(int32_t P, uint32_t* matrix, const uint32_t* group_visibl
     // (both in the cursor half of tile_base, which the tile-level layout of launch_tile_scatter overwrites later)
     uint32_t* bin_base = tile_base + tiles;
     uint32_t* bin_pairs = bin_base + bins;
-    hipLaunchKernelGGL(slice_prefix_kernel, dim3((bins + 63) / 64), dim3(256), 0, s, matrix, groups, bins, bin_pairs,
+    hipLaunchKernelGGL(slice_prefix_kernel, dim3((bins + 63) / 64), dim3(64 * kPrefixParts), 0, s, matrix, groups, bins, bin_pairs,
                        blocks, (uint32_t*)nullptr, (uint32_t*)nullptr, lists);
     GS355_CHECK_LAUNCH("bin: slice prefix");
     return launch_layout<false>(bin_pairs, bin_base, bins, blocks, group_visible, groups, n_cap, header, header_copy, false, ranges,
