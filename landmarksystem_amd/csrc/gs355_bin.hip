@@ -947,17 +947,37 @@ __device__ __forceinline__ void write_sorted(const Buf cur, uint32_t n, uint32_t
 }
 
 // ---------------------------------------------------------------------------
-// In-LDS bucket sorter: kT threads, up to kT * kR pairs, every pass ranks the
-// whole bucket at once (each wavefront owns kR * 64 consecutive positions).
-// LDS holds the bucket once (depth bits, index: 8 B per pair) plus two 16-bit
-// permutations that ping-pong between passes (4 B per pair).
+// Lane exchanges inside the vector unit (no LDS): sums, minima and maxima over a wavefront.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t dpp(uint32_t absent, uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)absent, (int)v, kCtrl, kRows, 0xf, false);
+}
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, uint32_t neutral, Op op)  // inclusive
+{
+    v = op(v, dpp<0x111, 0xf>(neutral, v));  // row_shr 1, 2, 4, 8
+    v = op(v, dpp<0x112, 0xf>(neutral, v));
+    v = op(v, dpp<0x114, 0xf>(neutral, v));
+    v = op(v, dpp<0x118, 0xf>(neutral, v));
+    v = op(v, dpp<0x142, 0xa>(neutral, v));  // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
+    return op(v, dpp<0x143, 0xc>(neutral, v));
+}
+__device__ __forceinline__ uint32_t wave_sum_scan(uint32_t v)
+{
+    return wave_scan(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+}
+
+// In-LDS bucket sorter: kT threads, up to kT * kR pairs, kR of them held in each thread's registers.
+// The counting sort keeps the bucket in LDS once, as 64-bit pairs.  The radix passes it falls back to keep it as depth bits
+// and index (8 B per pair) plus two 16-bit permutations that ping-pong between passes (4 B per pair), every pass ranking
+// the whole bucket at once (each wavefront owns kR * 64 consecutive positions).
 template <int kT, int kR>
 struct LdsSorter {
     static constexpr int kW = kT / 64;
     static constexpr int kCap = kT * kR;
-    // fine bins per thread of the counting pass (measured at 1080p / 6M Gaussians, the two larger classes together:
-    // 1 / 2 / 3 / 4 bins = 0.169 / 0.155 / 0.147 / 0.145 ms)
-    static constexpr int kBinsPer = kT >= 512 ? 4 : 2;
+    // fine bins per thread of the counting pass: one 16-byte access
+    static constexpr int kBinsPer = 4;
     static constexpr int kB = kBinsPer * kT;                      // fine bins
     // counters: [kW][256] words for the radix passes, or the fine bins and 512 coarse words of the counting pass
     static constexpr int kCounterWords = kB + 512 > kW * 256 ? kB + 512 : kW * 256;
@@ -1103,136 +1123,105 @@ struct LdsSorter {
         return cur;
     }
 
-    // Fast path: one counting pass over a monotone map of the depth onto kT bins leaves a handful of pairs per
-    // bin; every pair then ranks itself among the members of its bin by (depth bits, index).  Bins are ordered and
-    // each bin is fully ordered, so the result is the exact total order whatever order the LDS atomics ran in.
+    // Fast path: one counting pass over a monotone map of the depth onto kB bins leaves a pair or two per bin; every pair
+    // then ranks itself among the members of its bin.  Bins are ordered and each bin is fully ordered, so the result is
+    // the exact total order by (depth bits, index) whatever order the LDS atomics ran in.
     // Depths along the rays of a tile cluster (most splats sit near the ground), so the map is adaptive: a
     // 256-bin histogram over [dmin, dmax] gives a piecewise-linear estimate of each pair's final position, and
-    // the bin is that position scaled to kT.  Returns the buffer holding the order, or -2 when some bin is still
-    // too full for this to pay: the caller then runs the radix passes.
+    // the bin is that position scaled to kB.  Positions are floats: conversion, multiplication and multiply-add round
+    // monotonically and a coarse bin's end is a whole number, so the map stays monotone.
+    // The pairs wait in registers, and pass through LDS three times as they are (to their bin, to its ranking readers, to
+    // their place): ten LDS accesses per pair.  Kept in LDS as separate words behind a permutation they took twenty (6M
+    // Gaussians, 1080p, 13.4M pairs: the four classes 17 + 51 + 80 + 20 us, now 15 + 36 + 61 + 11).
+    // Returns false when some bin is too full for this to pay (nothing but the counters has then been written): the caller
+    // runs the radix passes.
     static constexpr uint32_t kMaxBin = 256;
 
-    __device__ int bucket_sort(uint32_t n, uint32_t dmin, uint32_t dmax) const
+    __device__ bool counting_sort(const uint64_t (&v)[kR], uint32_t n, uint32_t dmin, uint32_t dmax) const
     {
         const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-        uint32_t* const count = &cnt[0][0];  // [kB] pairs per bin, then the bin's first slot
-        uint32_t* const coarse = count + kB;  // [256] pairs per coarse bin, then their exclusive prefix
+        uint32_t* const count = &cnt[0][0];                              // [kB] pairs per bin, then the bin's first slot
+        uint32_t* const coarse = count + kB;                             // [256] pairs per coarse bin
+        float2* const line = reinterpret_cast<float2*>(coarse);          // [256] pairs before it and in it (same words)
+        uint64_t* const pairs = reinterpret_cast<uint64_t*>(depth);      // [kCap]
         const uint32_t range = dmax - dmin;
-        if (range == 0) return -2;
-        // coarse(d) = floor((d - dmin) * 256 / (range + 1)) as the high word of a 32x32 multiply, whose low word is
-        // the position inside the coarse bin as a 0.32 fraction; a range below 256 gives every depth its own bin
-        const bool direct = range < 256u;
-        const uint32_t mult = direct ? 0u : (uint32_t)((256ull << 32) / ((uint64_t)range + 1ull));
-        // position -> bin: floor(pos * kB / n) for n > kB, else the position itself (one pair per bin)
-        const bool spread = n > (uint32_t)kB;
-        const uint32_t to_bin = spread ? (uint32_t)(((uint64_t)kB << 32) / (uint64_t)n) : 0u;
+        const float scale = 256.0f / ((float)range + 1.0f);
+        const float to_bin = n > (uint32_t)kB ? (float)kB / (float)n : 1.0f;
         // (the counters were cleared by the caller, before the barrier that made dmin and dmax known)
-        uint32_t cbin[kR], frac[kR];
+        float at[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t j = (uint32_t)r * kT + tid;
-            cbin[r] = 0;
-            frac[r] = 0;
-            if (j < n) {
-                const uint32_t rel = depth[j] - dmin;
-                const uint64_t wide = (uint64_t)rel * mult;
-                cbin[r] = direct ? rel : (uint32_t)(wide >> 32);
-                frac[r] = direct ? 0u : (uint32_t)wide;
-                atomicAdd(&coarse[cbin[r]], 1u);
-            }
+            at[r] = fminf((float)((uint32_t)(v[r] >> 32) - dmin) * scale, 255.99998f);
+            if ((uint32_t)r * kT + tid < n) atomicAdd(&coarse[(uint32_t)at[r]], 1u);
         }
         __syncthreads();
+        uint32_t own = 0, inc = 0;
         if (tid < 256) {  // exclusive scan of the coarse counts (wavefronts 0..3)
-            const uint32_t own = coarse[tid];
-            uint32_t inc = own;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const uint32_t up = __shfl_up(inc, d, 64);
-                if (lane >= d) inc += up;
-            }
+            own = coarse[tid];
+            inc = wave_sum_scan(own);
             if (lane == 63) flags[16 + wave] = inc;
-            // (a thread replaces the one count that only it has read) exclusive within the wavefront: the
-            // wavefronts' totals are added by whoever reads it, which saves a barrier
-            coarse[tid] = inc - own;
-            coarse[256 + tid] = own;
         }
         __syncthreads();
-        const uint32_t before1 = flags[16], before2 = before1 + flags[17], before3 = before2 + flags[18];
+        if (tid < 256) {
+            uint32_t before = inc - own;
+            for (int w = 0; w < wave; ++w) before += flags[16 + w];
+            line[tid] = make_float2((float)before, (float)own);
+        }
+        __syncthreads();
         uint32_t bin[kR], slot[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t j = (uint32_t)r * kT + tid;
-            bin[r] = 0;
-            slot[r] = 0;
-            if (j < n) {
-                const uint32_t cb = cbin[r];
-                const uint32_t before = cb >= 192u ? before3 : cb >= 128u ? before2 : cb >= 64u ? before1 : 0u;
-                const uint32_t pos = coarse[cb] + before + __umulhi(frac[r], coarse[256 + cb]);  // in [0, n)
-                bin[r] = min(spread ? __umulhi(pos, to_bin) : pos, (uint32_t)kB - 1u);
+            bin[r] = slot[r] = 0;
+            if ((uint32_t)r * kT + tid < n) {
+                const float2 l = line[(uint32_t)at[r]];
+                const float pos = __builtin_fmaf(__builtin_amdgcn_fractf(at[r]), l.y, l.x);  // in [0, n]
+                bin[r] = min((uint32_t)(pos * to_bin), (uint32_t)kB - 1u);
                 slot[r] = atomicAdd(&count[bin[r]], 1u);
             }
         }
         __syncthreads();
-        // exclusive scan of the kB bin counts (a thread owns kBinsPer consecutive bins); remember whether any bin
-        // is over-full
-        uint32_t mine[kBinsPer], c = 0;
-        bool overfull = false;
-#pragma unroll
-        for (int i = 0; i < kBinsPer; ++i) {
-            mine[i] = count[kBinsPer * tid + i];
-            c += mine[i];
-            overfull = overfull || mine[i] > kMaxBin;
-        }
-        uint32_t inc = c;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t up = __shfl_up(inc, d, 64);
-            if (lane >= d) inc += up;
-        }
+        // exclusive scan of the kB bin counts (a thread owns four consecutive bins)
+        uint4 mine = reinterpret_cast<const uint4*>(count)[tid];
+        const uint32_t c = (mine.x + mine.y) + (mine.z + mine.w);
+        inc = wave_sum_scan(c);
         if (lane == 63) flags[16 + wave] = inc;
-        if (overfull) flags[8] = 1;
+        if (max(max(mine.x, mine.y), max(mine.z, mine.w)) > kMaxBin) flags[8] = 1;
         __syncthreads();
         if (flags[8] != 0) {
             __syncthreads();
-            return -2;
+            return false;
         }
         uint32_t first = inc - c;
         for (int w = 0; w < wave; ++w) first += flags[16 + w];
-#pragma unroll
-        for (int i = 0; i < kBinsPer; ++i) {
-            count[kBinsPer * tid + i] = first;
-            first += mine[i];
-        }
+        const uint32_t f1 = first + mine.x, f2 = f1 + mine.y;
+        reinterpret_cast<uint4*>(count)[tid] = make_uint4(first, f1, f2, f2 + mine.z);
+        if (tid == 0) count[kB] = n;  // (over the coarse bins, which are done with)
         __syncthreads();
-        uint16_t* const P = perm(0);
+#pragma unroll
+        for (int r = 0; r < kR; ++r)
+            if ((uint32_t)r * kT + tid < n) pairs[count[bin[r]] + slot[r]] = v[r];
+        if (tid < 4) pairs[n + tid] = ~0ull;  // (the permutations' area follows)
+        __syncthreads();
+        // A pair's rank among the members of its bin, four at a time: what follows the bin is larger than all of them, so
+        // a bin of up to four needs no further test.
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t j = (uint32_t)r * kT + tid;
-            if (j < n) P[count[bin[r]] + slot[r]] = (uint16_t)j;
-        }
-        __syncthreads();
-        // every pair ranks itself among the members of its bin (independent reads, evenly spread over the
-        // threads whatever the bin sizes are) and takes the slot of that rank
-        uint16_t* const Q = perm(1);
+            if ((uint32_t)r * kT + tid < n) {
+                const uint32_t lo = count[bin[r]], hi = count[bin[r] + 1];
+                uint32_t rank = lo;
+                for (uint32_t q = lo; q < hi; q += 4) {
 #pragma unroll
-        for (int r = 0; r < kR; ++r) {
-            const uint32_t j = (uint32_t)r * kT + tid;
-            if (j < n) {
-                const uint32_t b = bin[r];
-                const uint32_t lo_slot = count[b];
-                const uint32_t hi_slot = b + 1 < (uint32_t)kB ? count[b + 1] : n;
-                const uint32_t md = depth[j], mi = index[j];
-                uint32_t rank = 0;
-                for (uint32_t q = lo_slot; q < hi_slot; ++q) {
-                    const uint32_t e = P[q];
-                    const uint32_t ed = depth[e], ei = index[e];
-                    rank += (ed < md || (ed == md && ei < mi)) ? 1u : 0u;
+                    for (uint32_t k = 0; k < 4; ++k) rank += pairs[q + k] < v[r] ? 1u : 0u;
                 }
-                Q[lo_slot + rank] = (uint16_t)j;
+                slot[r] = rank;
             }
         }
         __syncthreads();
-        return 1;
+#pragma unroll
+        for (int r = 0; r < kR; ++r)
+            if ((uint32_t)r * kT + tid < n) pairs[slot[r]] = v[r];
+        __syncthreads();
+        return true;
     }
 
     // A bucket on its way from memory: where it lies and this thread's pairs of it (requested, not yet used).
@@ -1264,57 +1253,73 @@ struct LdsSorter {
     {
         const uint32_t lo = f.lo, n = f.n, tile = f.tile;
         if (n == 0 || n > (uint32_t)kCap) return;  // uniform over the workgroup
-        if (threadIdx.x == 0) {
-            flags[11] = 0;
-            flags[12] = 0xFFFFFFFFu;
-            flags[13] = 0;
-            flags[14] = 0xFFFFFFFFu;
-        }
-        __syncthreads();
-        // depth bits that differ somewhere in the bucket = (OR of all) ^ (AND of all)
-        uint32_t any = 0, all = 0xFFFFFFFFu, dmin = 0xFFFFFFFFu, dmax = 0;
+        uint32_t dmin = 0xFFFFFFFFu, dmax = 0;
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t j = (uint32_t)r * kT + threadIdx.x;
-            if (j < n) {
+            if ((uint32_t)r * kT + threadIdx.x < n) {
                 const uint32_t dj = (uint32_t)(f.v[r] >> 32);
-                depth[j] = dj;
-                index[j] = (uint32_t)f.v[r];
-                any |= dj;
-                all &= dj;
                 dmin = min(dmin, dj);
                 dmax = max(dmax, dj);
             }
         }
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            any |= __shfl_xor(any, d, 64);
-            all &= __shfl_xor(all, d, 64);
-            dmin = min(dmin, (uint32_t)__shfl_xor(dmin, d, 64));
-            dmax = max(dmax, (uint32_t)__shfl_xor(dmax, d, 64));
-        }
-        if ((threadIdx.x & 63) == 0) {
-            atomicOr(&flags[11], any);
-            atomicAnd(&flags[14], all);
-            atomicMin(&flags[12], dmin);
-            atomicMax(&flags[13], dmax);
+        dmin = wave_scan(dmin, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return min(a, b); });
+        dmax = wave_scan(dmax, 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
+        const int wave = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) == 63) {
+            flags[16 + wave] = dmin;
+            flags[32 + wave] = dmax;
         }
         {  // the counting sort's counters, cleared here so that it needs no barrier of its own for it
-            uint32_t* const count = &cnt[0][0];
-#pragma unroll
-            for (int i = 0; i < kBinsPer; ++i) count[i * kT + threadIdx.x] = 0;
-            if (threadIdx.x < 256) count[kB + threadIdx.x] = 0;
+            uint4* const count = reinterpret_cast<uint4*>(&cnt[0][0]);
+            count[threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
+            if (threadIdx.x < 128) count[kT + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
             if (threadIdx.x == 0) flags[8] = 0;
         }
         __syncthreads();
-        int cur = bucket_sort(n, flags[12], flags[13]);
-        if (cur == -2) cur = sort(n, flags[11] ^ flags[14]);
-        for (uint32_t j = threadIdx.x; j < n; j += kT) {
-            const uint32_t e = cur < 0 ? j : (uint32_t)perm(cur)[j];
-            // (no later stage reads the sorted keys: a streaming store, which leaves the cache to the records the
-            // blend is about to gather)
-            __builtin_nontemporal_store(((uint64_t)tile << 32) | (uint64_t)depth[e], &out_keys[lo + j]);
-            out_vals[lo + j] = index[e];
+        dmin = 0xFFFFFFFFu;
+        dmax = 0;
+#pragma unroll
+        for (int w = 0; w < kW; ++w) {
+            dmin = min(dmin, flags[16 + w]);
+            dmax = max(dmax, flags[32 + w]);
+        }
+        if (counting_sort(f.v, n, dmin, dmax)) {
+            const uint64_t* const pairs = reinterpret_cast<const uint64_t*>(depth);
+            for (uint32_t j = threadIdx.x; j < n; j += kT) {
+                const uint64_t v = pairs[j];
+                // (no later stage reads the sorted keys: a streaming store, which leaves the cache to the records the
+                // blend is about to gather)
+                __builtin_nontemporal_store(((uint64_t)tile << 32) | (v >> 32), &out_keys[lo + j]);
+                out_vals[lo + j] = (uint32_t)v;
+            }
+        } else {
+            // depth bits that differ somewhere in the bucket: (OR of all) ^ (AND of all)
+            uint32_t any = 0, all = 0xFFFFFFFFu;
+            if (threadIdx.x == 0) {
+                flags[11] = 0;
+                flags[14] = 0xFFFFFFFFu;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                const uint32_t j = (uint32_t)r * kT + threadIdx.x;
+                if (j < n) {
+                    const uint32_t dj = (uint32_t)(f.v[r] >> 32);
+                    depth[j] = dj;
+                    index[j] = (uint32_t)f.v[r];
+                    any |= dj;
+                    all &= dj;
+                }
+            }
+            atomicOr(&flags[11], any);
+            atomicAnd(&flags[14], all);
+            __syncthreads();
+            const int cur = sort(n, flags[11] ^ flags[14]);
+            for (uint32_t j = threadIdx.x; j < n; j += kT) {
+                const uint32_t e = cur < 0 ? j : (uint32_t)perm(cur)[j];
+                __builtin_nontemporal_store(((uint64_t)tile << 32) | (uint64_t)depth[e], &out_keys[lo + j]);
+                out_vals[lo + j] = index[e];
+            }
         }
         __syncthreads();
     }
