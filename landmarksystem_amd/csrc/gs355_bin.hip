@@ -809,7 +809,7 @@ struct SortScratch {
 // (by_depth) or the index word.  Returns false (and moves nothing) when every
 // pair has the same digit.
 template <typename Src, typename Dst>
-__device__ bool radix_pass(const Src src, const Dst dst, uint32_t n, int shift, bool by_depth, const SortScratch sc)
+__device__ __forceinline__ bool radix_pass(const Src src, const Dst dst, uint32_t n, int shift, bool by_depth, const SortScratch sc)
 {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     sc.hist[tid] = 0;
@@ -898,7 +898,7 @@ __device__ bool radix_pass(const Src src, const Dst dst, uint32_t n, int shift, 
 // Sort n pairs held in buffer A (B is scratch of the same size) by
 // (depth bits, index).  Returns true if the result is in B.
 template <typename Buf>
-__device__ bool sort_pairs(const Buf A, const Buf B, uint32_t n, const SortScratch sc)
+__device__ __forceinline__ bool sort_pairs(const Buf A, const Buf B, uint32_t n, const SortScratch sc)
 {
     bool in_b = false;
     // depth passes; pairs of one tile rarely share depth bits, so the index
@@ -1002,7 +1002,7 @@ struct LdsSorter {
 
     // One stable pass.  `src` < 0: the input order is the identity.  Returns the
     // buffer holding the output order (unchanged when all digits are equal).
-    __device__ int pass(uint32_t n, int shift, bool by_depth, int src) const
+    __device__ __forceinline__ int pass(uint32_t n, int shift, bool by_depth, int src) const
     {
         const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
         for (int k = tid; k < kW * 256; k += kT) (&cnt[0][0])[k] = 0;
@@ -1080,7 +1080,7 @@ struct LdsSorter {
 
     // Sort the n loaded pairs by (depth bits, index); returns the buffer with
     // the final order.
-    __device__ int sort(uint32_t n, uint32_t varying) const
+    __device__ __forceinline__ int sort(uint32_t n, uint32_t varying) const
     {
         int cur = -1;
         // bytes of the depth word that are identical in every pair need no pass
@@ -1137,7 +1137,7 @@ struct LdsSorter {
     // runs the radix passes.
     static constexpr uint32_t kMaxBin = 256;
 
-    __device__ bool counting_sort(const uint64_t (&v)[kR], uint32_t n, uint32_t dmin, uint32_t dmax) const
+    __device__ __forceinline__ bool counting_sort(const uint64_t (&v)[kR], uint32_t n, uint32_t dmin, uint32_t dmax) const
     {
         const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
         uint32_t* const count = &cnt[0][0];                              // [kB] pairs per bin, then the bin's first slot
@@ -1249,7 +1249,7 @@ struct LdsSorter {
     }
 
     // Sorts the fetched bucket and writes it out; ends with a barrier.
-    __device__ void sort_fetched(const Fetched& f, uint64_t* __restrict__ out_keys, uint32_t* __restrict__ out_vals) const
+    __device__ __forceinline__ void sort_fetched(const Fetched& f, uint64_t* __restrict__ out_keys, uint32_t* __restrict__ out_vals) const
     {
         const uint32_t lo = f.lo, n = f.n, tile = f.tile;
         if (n == 0 || n > (uint32_t)kCap) return;  // uniform over the workgroup
@@ -1324,7 +1324,7 @@ struct LdsSorter {
         __syncthreads();
     }
 
-    __device__ void run(uint32_t tile, const uint32_t* __restrict__ ranges, const uint64_t* __restrict__ buckets,
+    __device__ __forceinline__ void run(uint32_t tile, const uint32_t* __restrict__ ranges, const uint64_t* __restrict__ buckets,
                         uint64_t* __restrict__ out_keys, uint32_t* __restrict__ out_vals) const
     {
         Fetched f;
@@ -1349,16 +1349,16 @@ __global__ __launch_bounds__(kT) void tile_sort_each_kernel(const gs355_header* 
 {
     extern __shared__ uint32_t s_dyn[];
     if (header->overflow) return;
-    static_assert(kT == kThreads, "the global-memory passes are written for kThreads threads");
     static_assert((256 + kWaves * 256 + 8) * sizeof(uint32_t) <= LdsSorter<kT, kR>::kBytes, "scratch of the global passes");
     const uint32_t tile = blockIdx.x;
     const uint32_t lo = ranges[2 * tile], n = ranges[2 * tile + 1] - lo;
     bool through_global = n > (uint32_t)kTileSortCap[3];
-    if (skip_classes != 0u && n > (uint32_t)kTileSortCap[0] && !through_global) {
+    if (skip_classes != 0u && n > (uint32_t)LdsSorter<kT, kR>::kCap && !through_global) {
         const int cls = n <= (uint32_t)kTileSortCap[1] ? 0 : n <= (uint32_t)kTileSortCap[2] ? 1 : 2;
         through_global = (skip_classes >> cls) & 1u;
     }
-    if (through_global) {  // (uniform over the workgroup)
+    if (through_global) {  // (uniform over the workgroup; passes of kThreads threads)
+        if (threadIdx.x >= kThreads) return;
         const SortScratch sc = {s_dyn, reinterpret_cast<uint32_t(*)[256]>(s_dyn + 256), s_dyn + 256 + kWaves * 256};
         const GlobalPairs A = {buckets + lo}, B = {out_keys + lo};
         const bool in_b = sort_pairs(A, B, n, sc);
@@ -1454,6 +1454,7 @@ static int allow_large_lds()
         (e = raise_lds_limit(scatter_kernel<0, false>, bin_bytes)) != hipSuccess ||
         (e = raise_lds_limit(scatter_kernel<kCoarseShift, true>, bin_bytes)) != hipSuccess ||
         (e = raise_lds_limit(tile_sort_list_1024x5_kernel, LdsSorter<1024, 5>::kBytes)) != hipSuccess ||
+        (e = raise_lds_limit(tile_sort_each_kernel<1024, 5>, LdsSorter<1024, 5>::kBytes)) != hipSuccess ||
         (e = raise_lds_limit(tile_sort_list_kernel<1024, 10, true>, LdsSorter<1024, 10>::kBytes)) != hipSuccess)
         return set_error(GS355_EHIP, "LDS limit of the binning / tile sort kernels: %s", hipGetErrorString(e));
     done[dev].store(1, std::memory_order_release);  // racing threads set the same values
@@ -1582,6 +1583,12 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
     return GS355_OK;
 }
 
+// Up to this many tiles the 5120-pair sorter takes the smaller buckets too, all of them side by side in one launch (two
+// workgroups of it fit a CU): 10k Gaussians at 256x256, three launches of 7 us each against 8.9 us.  Beyond, buckets of
+// small classes hold back too many threads in it: a 2048-pair sorter for the two smallest classes already took 21 us
+// against 19 at 2170 tiles, 53 against 24 at 8160.
+constexpr int kOneLaunchTiles = 512;
+
 int launch_tile_sort(const gs355_header* header, int tiles, const uint32_t* ranges, uint32_t* lists, uint64_t* buckets,
                      uint64_t* out_keys, uint32_t* out_vals, uint32_t skip_classes, hipStream_t s)
 {
@@ -1594,19 +1601,24 @@ int launch_tile_sort(const gs355_header* header, int tiles, const uint32_t* rang
     int rc;
     if ((rc = allow_large_lds())) return rc;
     const uint32_t* list0 = lists + kListHeader;
-    hipLaunchKernelGGL((tile_sort_each_kernel<256, 4>), dim3(tiles), dim3(256), S0::kBytes, s, header, ranges, buckets,
-                       out_keys, out_vals, skip_classes);
+    const bool one_launch = tiles <= kOneLaunchTiles;
+    if (one_launch)
+        hipLaunchKernelGGL((tile_sort_each_kernel<1024, 5>), dim3(tiles), dim3(1024), S2::kBytes, s, header, ranges, buckets,
+                           out_keys, out_vals, skip_classes);
+    else
+        hipLaunchKernelGGL((tile_sort_each_kernel<256, 4>), dim3(tiles), dim3(256), S0::kBytes, s, header, ranges, buckets,
+                           out_keys, out_vals, skip_classes);
     GS355_CHECK_LAUNCH("tile sort: class 0");
     // A launch per larger class, a workgroup per tile: those past the end of the class's list leave at once, which
     // costs nothing measurable (sizing the launch by the list's expected length changed no kernel's time).  The
     // largest class is the exception: a workgroup of it fills a CU, so its launch is the chip's size and strides.
     // (skip_classes: bit c set = the caller expects list c to be empty; the kernel above has sorted what is on it)
-    if (!(skip_classes & 1u)) {
+    if (!(skip_classes & 1u) && !one_launch) {
         hipLaunchKernelGGL((tile_sort_list_kernel<512, 4, false>), dim3(tiles), dim3(512), S1::kBytes, s, header, ranges,
                            list0, lists + 0, buckets, out_keys, out_vals);
         GS355_CHECK_LAUNCH("tile sort: class 1");
     }
-    if (!(skip_classes & 2u)) {
+    if (!(skip_classes & 2u) && !one_launch) {
         hipLaunchKernelGGL(tile_sort_list_1024x5_kernel, dim3(tiles), dim3(1024), S2::kBytes, s, header, ranges,
                            list0 + (size_t)tiles, lists + 1, buckets, out_keys, out_vals);
         GS355_CHECK_LAUNCH("tile sort: class 2");
