@@ -117,7 +117,8 @@ typedef struct gs355_header {
      * (1025..2048, 2049..5120, 5121..10240 pairs); 0xFFFFFFFF = not counted (scan stage, larger images).  What a
      * caller needs to choose GS355_STAGE_TILESORT_SKIP_* for the next frame. */
     uint32_t sort_class_count[3];
-    uint32_t reserved[8];
+    uint32_t ready;          /* set to 1 in a header copy, after everything else in it (in the workspace: not used) */
+    uint32_t reserved[7];
 } gs355_header;
 
 /* Byte offsets of every array inside the caller's workspace (each 256-byte
@@ -217,6 +218,16 @@ GS355_API int gs355_render(const gs355_frame *frame, const gs355_gaussians *g, v
 GS355_API int gs355_run_parameters(const gs355_frame *frame, const gs355_gaussians *g, const float *features_rest,
                                    void *workspace, size_t workspace_bytes, int64_t n_cap, const gs355_outputs *out,
                                    uint32_t stage_mask, void *stream);
+
+/* A frame from its preprocess stage to its blend stage in one call, and the wait for its header: enqueues `stage_mask`
+ * (which must hold the scan or the tile-count stage), has that stage store the header in out->header_copy, here pinned
+ * host memory that the GPU can write, and returns when it has, with the later stages still under way: the caller learns
+ * the key count and whether the frame overflowed its capacity.  The host watches the header's last word, so nothing is
+ * recorded on the stream between the stages.  stored_parameters = 0: as gs355_run (features_rest is ignored), else as
+ * gs355_run_parameters.  Not for a stream that is being captured. */
+GS355_API int gs355_render_frame(const gs355_frame *frame, const gs355_gaussians *g, int32_t stored_parameters,
+                                 const float *features_rest, void *workspace, size_t workspace_bytes, int64_t n_cap,
+                                 const gs355_outputs *out, uint32_t stage_mask, void *stream);
 
 /* GaussianRasterizer.visible_filter: radii only (cull, covariance, radius,
  * non-empty tile rectangle); needs no workspace.  shs/colors/opacities of

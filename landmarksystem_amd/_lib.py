@@ -32,7 +32,7 @@ EXPORTS = ("gs355_version", "gs355_last_error", "gs355_workspace_layout", "gs355
            "gs355_decode_count_static", "gs355_decode_emit", "gs355_decode_workspace_bytes", "gs355_decode",
            "gs355_backward_scratch_bytes", "gs355_render_backward", "gs355_gather_scratch_bytes", "gs355_gather_rows",
            "gs355_run_parameters", "gs355_render_parameters_backward", "gs355_decode_train_bytes", "gs355_decode_train",
-           "gs355_decode_train_backward")
+           "gs355_decode_train_backward", "gs355_render_frame")
 GATHER_MAX_ARRAYS, GATHER_MAX_ROW_BYTES = 8, 4096
 
 
@@ -82,7 +82,8 @@ class Header(C.Structure):
         ("overflow", C.c_uint32),
         ("num_visible", C.c_uint32),
         ("sort_class_count", C.c_uint32 * 3),
-        ("reserved", C.c_uint32 * 8),
+        ("ready", C.c_uint32),
+        ("reserved", C.c_uint32 * 7),
     ]
 
 
@@ -250,6 +251,9 @@ def load() -> C.CDLL:
     lib.gs355_run_parameters.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_void_p, C.c_void_p, C.c_size_t,
                                          C.c_int64, C.POINTER(Outputs), C.c_uint32, C.c_void_p]
     lib.gs355_run_parameters.restype = C.c_int
+    lib.gs355_render_frame.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_int32, C.c_void_p, C.c_void_p,
+                                       C.c_size_t, C.c_int64, C.POINTER(Outputs), C.c_uint32, C.c_void_p]
+    lib.gs355_render_frame.restype = C.c_int
     lib.gs355_render_parameters_backward.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_void_p, C.c_void_p,
                                                      C.c_size_t, C.c_int64, C.POINTER(BackwardInputs), C.c_void_p,
                                                      C.c_size_t, C.POINTER(Gradients), C.c_void_p, C.c_void_p]

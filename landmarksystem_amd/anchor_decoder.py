@@ -37,9 +37,12 @@ from torch import nn
 from torch.autograd.function import once_differentiable
 
 from . import _lib
+from .pipeline import _raw_stream
 
 
 def _f32c(t: torch.Tensor, device) -> torch.Tensor:
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous():
+        return t
     t = t.detach()
     if t.device != device:
         t = t.to(device)
@@ -185,7 +188,7 @@ class _DecodeTrain(torch.autograd.Function):
         scratch = torch.empty(scratch_bytes.value // 4, dtype=torch.float32, device=dev)
         _lib.check(lib.gs355_decode_train_backward(C.byref(dec), C.byref(an), C.byref(rows), ctx.workspace.data_ptr(),
                                                    ctx.workspace.numel(), C.byref(cot), C.byref(out), scratch.data_ptr(),
-                                                   scratch.numel() * 4, torch.cuda.current_stream(dev).cuda_stream))
+                                                   scratch.numel() * 4, _raw_stream(dev)))
         return (None, None, None, None, None, *grads)
 
 
@@ -260,8 +263,22 @@ class FusedAnchorDecoder(nn.Module):
         return d
 
     def _parameter_list(self):
-        mlps = [self.mlp_opacity, self.mlp_cov, self.mlp_color] + ([self.mlp_feature_bank] if self.use_feat_bank else [])
-        return [t for m in mlps for t in (m[0].weight, m[0].bias, m[2].weight, m[2].bias)]
+        return self._parameters_of(("mlp_opacity", "mlp_cov", "mlp_color") +
+                                   (("mlp_feature_bank",) if self.use_feat_bank else ()))
+
+    def _parameters_of(self, names):
+        """Weights and biases of the named heads' two layers.  Read from the modules' own tables: the attribute and index
+        lookups of nn.Module cost a microsecond each, and every frame asks for a dozen parameters."""
+        out = []
+        for name in names:
+            layers = self._modules[name]._modules
+            for layer in (layers["0"], layers["2"]):
+                p = layer._parameters
+                if "weight" in p and "bias" in p:
+                    out += (p["weight"], p["bias"])
+                else:  # (a reparametrised layer computes them)
+                    out += (layer.weight, layer.bias)
+        return out
 
     def _check_level(self, level, A):
         """The reference's behaviour for the level input (anchor_decoder.py:157-186): with add_level and a level
@@ -309,16 +326,18 @@ class FusedAnchorDecoder(nn.Module):
             f32 = tensors[1]
             self._feat_checked = (feat_key, bool(torch.equal(f32.half().float(), f32)))
         dec.fp32_features = 0 if self._feat_checked[1] else 1
-        need = C.c_size_t()
-        _lib.check(_lib.load().gs355_decode_workspace_bytes(A, self.n_offsets, 1 if self.use_feat_bank else 0,
-                                                            C.byref(need)))
         kept = self._kept(dev)
-        if kept.get("workspace") is None or kept["workspace"].numel() < need.value:
-            kept["workspace"] = torch.empty(max(need.value, 256), dtype=torch.uint8, device=dev)
+        if kept.get("anchors") != A:
+            need = C.c_size_t()
+            _lib.check(_lib.load().gs355_decode_workspace_bytes(A, self.n_offsets, 1 if self.use_feat_bank else 0,
+                                                                C.byref(need)))
+            if kept.get("workspace") is None or kept["workspace"].numel() < need.value:
+                kept["workspace"] = torch.empty(max(need.value, 256), dtype=torch.uint8, device=dev)
+            kept["anchors"] = A
         return dev, A, dec, an, tensors
 
     def _kept(self, dev):
-        key = (dev, torch.cuda.current_stream(dev).cuda_stream)
+        key = (dev, _raw_stream(dev))
         kept = self._per_stream.get(key)
         if kept is None:
             kept = self._per_stream[key] = {}
@@ -329,10 +348,9 @@ class FusedAnchorDecoder(nn.Module):
         return kept
 
     def _run(self, dec, an, capacity, o, phases, dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
         ws = self._kept(dev)["workspace"]
         _lib.check(_lib.load().gs355_decode(C.byref(dec), C.byref(an), int(capacity), C.byref(o), ws.data_ptr(),
-                                            ws.numel(), int(phases), stream))
+                                            ws.numel(), int(phases), _raw_stream(dev)))
 
     @torch.no_grad()
     def decode_on_device(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask=None, level=None,
@@ -389,8 +407,7 @@ class FusedAnchorDecoder(nn.Module):
             return self._forward_kernels(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
 
     def _head_parameters(self):
-        return [t for m in (self.mlp_opacity, self.mlp_cov, self.mlp_color)
-                for t in (m[0].weight, m[0].bias, m[2].weight, m[2].bias)]
+        return self._parameters_of(("mlp_opacity", "mlp_cov", "mlp_color"))
 
     def _train_structs(self, camera_center, visible, level, anchor, feat, offset, scaling, params):
         d = _lib.Decoder()

@@ -3,6 +3,7 @@
 // call sites: benchmarks/nerf/origin_gs/gs_model.py:211-220, 327-329).
 // Validation runs before any HIP call so that error paths are testable on a
 // machine without a GPU.
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -160,6 +161,24 @@ int check_parameters(const gs355_frame* f, const gs355_gaussians* g, const float
     return GS355_OK;
 }
 
+// Watches a header in host memory until its `ready` is set.  The stream is looked at once a millisecond: an error on it, or
+// its end without a header, ends the wait.
+int wait_for_header(volatile gs355_header* header, hipStream_t s)
+{
+    auto ready = [&]() { return __atomic_load_n(const_cast<uint32_t*>(&header->ready), __ATOMIC_ACQUIRE) != 0u; };
+    auto next_look = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+    for (uint32_t spins = 1;; ++spins) {
+        if (ready()) return GS355_OK;
+        __builtin_ia32_pause();
+        if ((spins & 255u) != 0u || std::chrono::steady_clock::now() < next_look) continue;
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipSuccess) return ready() ? GS355_OK : set_error(GS355_EHIP, "the frame ended without a header");
+        if (e != hipErrorNotReady) return set_error(GS355_EHIP, "waiting for the frame's header: %s", hipGetErrorString(e));
+        (void)hipGetLastError();  // (not-ready is no error of a later launch)
+        next_look = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+    }
+}
+
 FrameArgs make_args(const gs355_frame* f)
 {
     FrameArgs a;
@@ -311,6 +330,30 @@ int gs355_run_parameters(const gs355_frame* frame, const gs355_gaussians* g, con
     ParameterArgs par;
     par.rest = features_rest;
     return run_stages(frame, g, &par, workspace, workspace_bytes, n_cap, out, stage_mask, stream);
+}
+
+int gs355_render_frame(const gs355_frame* frame, const gs355_gaussians* g, int32_t stored_parameters,
+                       const float* features_rest, void* workspace, size_t workspace_bytes, int64_t n_cap,
+                       const gs355_outputs* out, uint32_t stage_mask, void* stream)
+{
+    constexpr uint32_t kFront = GS355_STAGE_PREPROCESS | GS355_STAGE_SCAN | GS355_STAGE_TILE_COUNT;
+    if (!out) return set_error(GS355_EINVAL, "outputs is NULL");
+    if (!out->header_copy) return set_error(GS355_EINVAL, "outputs.header_copy is NULL (the header is what the call waits for)");
+    if (!(stage_mask & (GS355_STAGE_SCAN | GS355_STAGE_TILE_COUNT)) || !(stage_mask & ~(kFront | kStageModifiers)))
+        return set_error(GS355_EINVAL, "stage_mask 0x%x is not a frame: it needs the scan or tile-count stage and later ones",
+                         stage_mask);
+    ParameterArgs par;
+    par.rest = features_rest;
+    const ParameterArgs* p = stored_parameters ? &par : nullptr;
+    gs355_outputs later = *out;
+    later.header_copy = nullptr;
+    volatile gs355_header* header = static_cast<volatile gs355_header*>(out->header_copy);
+    header->ready = 0u;
+    __atomic_thread_fence(__ATOMIC_SEQ_CST);
+    int rc = run_stages(frame, g, p, workspace, workspace_bytes, n_cap, out, stage_mask & kFront, stream);
+    if (!rc) rc = run_stages(frame, g, p, workspace, workspace_bytes, n_cap, &later, stage_mask & ~kFront, stream);
+    if (rc) return rc;
+    return wait_for_header(header, static_cast<hipStream_t>(stream));
 }
 
 int gs355_render(const gs355_frame* frame, const gs355_gaussians* g, void* workspace, size_t workspace_bytes,

@@ -684,12 +684,13 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         for (int c = 0; c < 3; ++c) header->sort_class_count[c] = counted ? class_count(in_class, c) : 0xFFFFFFFFu;
         if (counted && kTiles)
             for (int c = 0; c < 3; ++c) lists[c] = class_count(in_class, c);
-        if (header_copy) {  // (may be host memory: plain stores, complete when the kernel is)
+        if (header_copy) {
             header_copy->num_keys_total = total;
             header_copy->num_keys = overflow ? n_cap : (uint32_t)total;
             header_copy->overflow = overflow ? 1u : 0u;
             header_copy->num_visible = (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]);
             for (int c = 0; c < 3; ++c) header_copy->sort_class_count[c] = counted ? class_count(in_class, c) : 0xFFFFFFFFu;
+            mark_ready(header_copy);
         }
     }
     if (overflow) return;  // later stages do nothing either

@@ -209,6 +209,13 @@ __device__ __forceinline__ void wave_lds_sync()
 
 int launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s);
 
+// Marks a header copy as complete (it may be host memory that a host thread watches): everything stored in it before is
+// visible to whoever sees the mark.
+__device__ __forceinline__ void mark_ready(gs355_header* copy)
+{
+    __hip_atomic_store(&copy->ready, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // tile-bucketed path
 constexpr int kBinThreads = 1024;       // threads per binning workgroup
 constexpr int kBinMaxGroups = 256;      // binning workgroups (each owns a contiguous slice of the Gaussians)

@@ -574,8 +574,8 @@ class ScaffoldGS(nn.Module):
             rendered_image, radii, _ = self.renderer(
                 means3D=res.xyz, means2D=None, shs=None, colors_precomp=res.color, opacities=res.opacity,
                 scales=res.scaling, rotations=res.rot, cov3D_precomp=None, count=res.count)
-            self._visibility_filter, self._pending = None, (res, radii)
-            self.voxel_visible_mask = voxel_visible_mask
+            d = self.__dict__  # (plain attributes, set past nn.Module's search for parameters, buffers and modules)
+            d["_visibility_filter"], d["_pending"], d["voxel_visible_mask"] = None, (res, radii), voxel_visible_mask
             return rendered_image
         xyz, color, opacity, scaling, rot, _, _ = self.anchor_decoder(**decode)
         rendered_image, radii, _ = self.renderer(

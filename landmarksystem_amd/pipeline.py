@@ -24,6 +24,10 @@ def _dev_f32(t: Optional[torch.Tensor], device: torch.device, name: str, shape=N
         return None
     if not isinstance(t, torch.Tensor):
         raise TypeError("%s must be a torch.Tensor, got %r" % (name, type(t)))
+    # the usual case, tensors that are already as the kernels read them, is decided by four quick tests
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous() and (
+            shape is None or t.numel() == math.prod(shape)):
+        return t
     t = t.detach()
     if t.device != device:
         t = t.to(device)
@@ -36,7 +40,12 @@ def _dev_f32(t: Optional[torch.Tensor], device: torch.device, name: str, shape=N
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None or t.numel() == 0 else t.data_ptr()
+    return None if t is None else t.data_ptr()  # (0, a null pointer, for an empty tensor)
+
+
+def _raw_stream(device: torch.device) -> int:
+    """Handle of the current stream on `device`."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 class Workspace:
@@ -51,7 +60,8 @@ class Workspace:
         self.buffer: Optional[torch.Tensor] = None
         self.key_capacity = 0
         self.header_host = torch.zeros(8, dtype=torch.int64, pin_memory=True)
-        self.header_event = torch.cuda.Event()
+        self.header = _lib.Header.from_address(self.header_host.data_ptr())  # the same 64 bytes
+        self._layout = None  # (the sizes it was made for, the layout of the latest frame)
         self.frames = 0
         self.overflows = 0
         self.sort_mispredictions = 0  # frames with buckets in a sorter size class that was expected empty
@@ -60,7 +70,10 @@ class Workspace:
         self.sort_class_wait = [4, 4, 4]  # ... and how many of them it takes before the class's launch is left out
 
     def ensure(self, P: int, n_cap: int, width: int, height: int) -> "_lib.Layout":
-        layout = _lib.workspace_layout(P, n_cap, width, height)
+        sizes = (P, n_cap, width, height)
+        if self._layout is None or self._layout[0] != sizes:
+            self._layout = (sizes, _lib.workspace_layout(P, n_cap, width, height))
+        layout = self._layout[1]
         if self.buffer is None or self.buffer.numel() < layout.total_bytes:
             self.buffer = None  # release before growing
             self.buffer = torch.empty(int(layout.total_bytes * 1.1) + 4096, dtype=torch.uint8, device=self.device)
@@ -100,8 +113,8 @@ _workspaces: "OrderedDict[Tuple[int, int], Workspace]" = OrderedDict()
 
 
 def _workspace_key(device: torch.device, stream=None) -> Tuple[int, int]:
-    stream = stream if stream is not None else torch.cuda.current_stream(device)
-    return (device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream)
+    return (device.index if device.index is not None else torch.cuda.current_device(),
+            _raw_stream(device) if stream is None else stream.cuda_stream)
 
 
 def default_workspace(device: torch.device) -> Workspace:
@@ -175,20 +188,12 @@ class FrameInputs:
         self.campos = _dev_f32(s.campos, dev, "campos", (3,))
         self.bg = _dev_f32(s.bg, dev, "bg", (3,))
 
-        f = _lib.Frame()
-        f.image_width, f.image_height = self.width, self.height
-        f.tanfovx, f.tanfovy = float(s.tanfovx), float(s.tanfovy)
-        f.scale_modifier = float(s.scale_modifier)
-        f.sh_degree, f.sh_coeffs = int(s.sh_degree), sh_coeffs
-        f.viewmatrix, f.projmatrix = _ptr(self.viewmatrix), _ptr(self.projmatrix)
-        f.campos, f.bg = _ptr(self.campos), _ptr(self.bg)
-        self.frame = f
-
-        g = _lib.Gaussians()
-        g.P = P
-        g.means3D, g.shs, g.colors_precomp = _ptr(self.means3D), _ptr(self.shs), _ptr(self.colors_precomp)
-        g.opacities, g.scales, g.rotations = _ptr(self.opacities), _ptr(self.scales), _ptr(self.rotations)
-        g.cov3D_precomp = _ptr(self.cov3D_precomp)
+        # (fields in the structures' order)
+        self.frame = _lib.Frame(self.width, self.height, float(s.tanfovx), float(s.tanfovy), float(s.scale_modifier),
+                                int(s.sh_degree), sh_coeffs, _ptr(self.viewmatrix), _ptr(self.projmatrix),
+                                _ptr(self.campos), _ptr(self.bg))
+        g = _lib.Gaussians(P, _ptr(self.means3D), _ptr(self.shs), _ptr(self.colors_precomp), _ptr(self.opacities),
+                           _ptr(self.scales), _ptr(self.rotations), _ptr(self.cov3D_precomp))
         self.count = None
         if count is not None:
             if not (isinstance(count, torch.Tensor) and count.device == dev and count.numel() == 1
@@ -206,8 +211,8 @@ class FrameInputs:
 def visible_filter(inputs: FrameInputs) -> torch.Tensor:
     """radii int32[P] of the cull / covariance / radius / tile-rectangle test."""
     radii = torch.empty(inputs.P, dtype=torch.int32, device=inputs.device)
-    stream = torch.cuda.current_stream(inputs.device).cuda_stream
-    _lib.check(_lib.load().gs355_visible_filter(C.byref(inputs.frame), C.byref(inputs.gaussians), _ptr(radii), stream))
+    _lib.check(_lib.load().gs355_visible_filter(C.byref(inputs.frame), C.byref(inputs.gaussians), radii.data_ptr(),
+                                                _raw_stream(inputs.device)))
     return radii
 
 
@@ -243,7 +248,7 @@ def anchor_filter(settings, anchors: torch.Tensor, scaling: torch.Tensor, rotati
         lod_c = _lib.AnchorLod(_ptr(level), _ptr(extra), float(lod["voxel_size"]), float(lod["standard_dist"]),
                                float(lod["fork"]), float(lod["resolution_scale"]),
                                {"floor": 0, "round": 1, "ceil": 2}[lod["rounding"]], int(lod["max_level"]))
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _raw_stream(dev)
     _lib.check(_lib.load().gs355_anchor_filter(C.byref(f), C.byref(g), int(sc.shape[1]),
                                                C.byref(lod_c) if lod_c is not None else None, _ptr(mask),
                                                _ptr(visible), None, stream))
@@ -275,7 +280,7 @@ def gather_rows(mask: torch.Tensor, tensors):
     _lib.check(lib.gs355_gather_scratch_bytes(P, C.byref(need)))
     scratch = torch.empty(need.value // 8 + 1, dtype=torch.int64, device=dev)
     count = torch.empty(1, dtype=torch.int32, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _raw_stream(dev)
     _lib.check(lib.gs355_gather_rows(P, mask.contiguous().data_ptr() if P else None, len(given), arrays,
                                      count.data_ptr(), scratch.data_ptr(), scratch.numel() * 8, stream))
     n = int(count.item())  # the one wait: the caller's tensors are exactly sized, as after boolean indexing
@@ -290,9 +295,7 @@ class FrameOutputs:
         self.depth = torch.empty((1, H, W), dtype=torch.float32, device=dev) if want_depth else None
         self.alpha = torch.empty((1, H, W), dtype=torch.float32, device=dev) if want_alpha else None
         self.radii = torch.empty(inputs.P, dtype=torch.int32, device=dev)
-        o = _lib.Outputs()
-        o.image, o.depth, o.alpha, o.radii = _ptr(self.image), _ptr(self.depth), _ptr(self.alpha), _ptr(self.radii)
-        self.c = o
+        self.c = _lib.Outputs(self.image.data_ptr(), _ptr(self.depth), _ptr(self.alpha), self.radii.data_ptr())
         self.num_keys = 0
         self.num_visible = 0
         self.key_capacity = 0  # the capacity the frame was finally rendered with (what a backward pass must pass)
@@ -301,7 +304,7 @@ class FrameOutputs:
 def run_stages(inputs: FrameInputs, outputs: FrameOutputs, ws: Workspace, n_cap: int, stage_mask: int):
     """Enqueue the selected stages over `ws`; returns the layout used."""
     layout = ws.ensure(inputs.P, n_cap, inputs.width, inputs.height)
-    stream = torch.cuda.current_stream(inputs.device).cuda_stream
+    stream = _raw_stream(inputs.device)
     frame, gaussians = C.byref(inputs.frame), C.byref(inputs.gaussians)
     rest = (ws.buffer.data_ptr(), ws.buffer.numel(), int(n_cap), C.byref(outputs.c), int(stage_mask), stream)
     if inputs.features_rest is None:
@@ -320,7 +323,8 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
     The key count is only known on the device after the scan.  The kernel that
     computes it also stores the header in pinned host memory; the remaining stages
     are enqueued against the current capacity without waiting, and the host then
-    waits for that kernel only (the GPU keeps working on sort and blend).
+    watches that memory (the GPU keeps working on sort and blend).  All of it is
+    one native call.
     If the frame needed more keys than the capacity, it is redone once with
     the exact requirement plus headroom; capacity never shrinks."""
     ws = ws or default_workspace(inputs.device)
@@ -336,32 +340,28 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
         # no launch for a sorter size class that the last few frames left empty (a hint: the library sorts the
         # buckets of such a class all the same, but far slower than the launch costs, so a class that turns up
         # unexpectedly has to stay away four times as long before it is left out again)
-        skipped = [c for c in range(3) if ws.sort_class_idle[c] >= ws.sort_class_wait[c]]
+        idle, wait = ws.sort_class_idle, ws.sort_class_wait
+        skipped = [c for c in (0, 1, 2) if idle[c] >= wait[c]]
         for c in skipped:
             back |= _lib.STAGE_TILESORT_SKIP[c]
     else:  # beyond the bucketed stages' limits (images past 8K): classic duplicate / radix sort / ranges
         front = _lib.STAGE_PREPROCESS | _lib.STAGE_SCAN
         back = _lib.STAGE_DUPLICATE | _lib.STAGE_SORT | _lib.STAGE_RANGES | _lib.STAGE_BLEND
         skipped = []
+    header, render_frame, stream = ws.header, _lib.load().gs355_render_frame, _raw_stream(inputs.device)
+    out.c.header_copy = ws.header_host.data_ptr()
     for attempt in range(3):
         n_cap = ws.key_capacity
-        # the stage that produces the header also stores it in pinned host memory (no copy is enqueued)
-        out.c.header_copy = ws.header_host.data_ptr()
-        run_stages(inputs, out, ws, n_cap, front)
-        out.c.header_copy = None
-        ws.header_event.record(torch.cuda.current_stream(inputs.device))
-        run_stages(inputs, out, ws, n_cap, back)
-        ws.header_event.synchronize()
-        total = int(ws.header_host[0])
-        word1 = int(ws.header_host[1])
-        overflow = (word1 >> 32) & 0xFFFFFFFF
+        ws.ensure(inputs.P, n_cap, inputs.width, inputs.height)
+        _lib.check(render_frame(C.byref(inputs.frame), C.byref(inputs.gaussians), inputs.features_rest is not None,
+                                _ptr(inputs.features_rest), ws.buffer.data_ptr(), ws.buffer.numel(), n_cap,
+                                C.byref(out.c), front | back, stream))
+        total, overflow = header.num_keys_total, header.overflow
         out.num_keys = ws.last_num_keys = total
-        out.num_visible = int(ws.header_host[2]) & 0xFFFFFFFF
+        out.num_visible = header.num_visible
         ws.frames += 1
-        word3 = int(ws.header_host[3])
-        counts = ((int(ws.header_host[2]) >> 32) & 0xFFFFFFFF, word3 & 0xFFFFFFFF, (word3 >> 32) & 0xFFFFFFFF)
-        for c in range(3):  # (0xFFFFFFFF: this path does not count the classes)
-            ws.sort_class_idle[c] = ws.sort_class_idle[c] + 1 if counts[c] == 0 else 0
+        counts = tuple(header.sort_class_count)
+        ws.sort_class_idle = [0 if n else i + 1 for n, i in zip(counts, ws.sort_class_idle)]  # (0xFFFFFFFF: not counted)
         wrong = [c for c in skipped if counts[c] != 0]
         if wrong and not overflow:
             ws.sort_mispredictions += 1  # (the frame is right all the same: the library sorts such buckets the slow way)
@@ -406,7 +406,7 @@ def render_backward(inputs: FrameInputs, out: FrameOutputs, workspace: torch.Ten
     need = C.c_size_t(0)
     _lib.check(_lib.load().gs355_backward_scratch_bytes(P, int(out.key_capacity), C.byref(need)))
     scratch = torch.empty(need.value // 4, dtype=torch.float32, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _raw_stream(dev)
     frame, gaussians = C.byref(inputs.frame), C.byref(inputs.gaussians)
     rest = (workspace.data_ptr(), workspace.numel(), int(out.key_capacity), C.byref(b), scratch.data_ptr(),
             scratch.numel() * 4, C.byref(g))

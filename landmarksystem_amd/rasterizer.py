@@ -162,6 +162,11 @@ class GaussianRasterizer(nn.Module):
         self.last_alpha: Optional[torch.Tensor] = None
         self.last_num_keys = 0
 
+    def _keep(self, depth, alpha, num_keys):
+        # (plain attributes, set past nn.Module.__setattr__, which first looks for parameters, buffers and modules)
+        d = self.__dict__
+        d["last_depth"], d["last_alpha"], d["last_num_keys"] = depth, alpha, num_keys
+
     def visible_filter(self, means3D, scales=None, rotations=None, cov3D_precomp=None):
         """int32[P] screen-space radii; 0 for Gaussians that are culled or
         touch no tile.  Callers threshold with `> 0`."""
@@ -186,13 +191,13 @@ class GaussianRasterizer(nn.Module):
             if count is not None:
                 raise ValueError("a device-side Gaussian count cannot be combined with gradients")
             image, radii, depth, alpha = _RasterizeGaussians.apply(self.raster_settings, *tensors)
-            self.last_depth, self.last_alpha, self.last_num_keys = depth, alpha, 0
+            self._keep(depth, alpha, 0)
             return image, radii, depth
         inputs = pipeline.FrameInputs(self.raster_settings, means3D, opacities=opacities, shs=shs,
                                       colors_precomp=colors_precomp, scales=scales, rotations=rotations,
                                       cov3D_precomp=cov3D_precomp, count=count)
         out = pipeline.render(inputs)
-        self.last_depth, self.last_alpha, self.last_num_keys = out.depth, out.alpha, out.num_keys
+        self._keep(out.depth, out.alpha, out.num_keys)
         return out.image, out.radii, out.depth
 
     def forward_parameters(self, xyz, means2D, features_dc, features_rest, opacity, scaling, rotation):
@@ -202,10 +207,10 @@ class GaussianRasterizer(nn.Module):
         tensors = (xyz, means2D, features_dc, features_rest, opacity, scaling, rotation)
         if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors):
             image, radii, depth, alpha = _RasterizeParameters.apply(self.raster_settings, *tensors)
-            self.last_depth, self.last_alpha, self.last_num_keys = depth, alpha, 0
+            self._keep(depth, alpha, 0)
             return image, radii, depth
         inputs = pipeline.FrameInputs(self.raster_settings, xyz, opacities=opacity, shs=features_dc, scales=scaling,
                                       rotations=rotation, features_rest=features_rest)
         out = pipeline.render(inputs)
-        self.last_depth, self.last_alpha, self.last_num_keys = out.depth, out.alpha, out.num_keys
+        self._keep(out.depth, out.alpha, out.num_keys)
         return out.image, out.radii, out.depth
