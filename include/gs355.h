@@ -426,26 +426,24 @@ GS355_API int gs355_decode(const gs355_decoder *dec, const gs355_anchors *an, in
                            void *workspace, size_t workspace_bytes, uint32_t phases, void *stream);
 
 /* ---------------------------------------------------------------------------
- * The decode as training differentiates it (anchor_decoder.py:147-242 under autograd): everything around the heads'
- * matrix products going forward, which stay with the caller, and all of it going back, in fp32.  Four phases of
- * gs355_decode_train, one call each:
- *   ROWS    out->num_visible (device or pinned host memory); the caller reads it and sizes the rows
- *   INPUTS  the heads' input rows: rows->with_dist [V,36] = [feat | view | dist] (the level instead of the distance with
- *           add_level) and / or rows->without [V,35] = [feat | view].  The caller then computes, per head,
- *           hidden = relu(x w0^T + b0) [V,32] and pre = hidden w1^T + b1 [V,k]
- *   COUNT   out->count from the opacity pre-activations; the caller reads it and sizes the outputs
- *   EMIT    every field of `out` but those two
+ * The decode as training differentiates it (anchor_decoder.py:147-242 under autograd), forward and back, in fp32.  Two
+ * phases of gs355_decode_train, one call each:
+ *   HEADS   the heads' input rows, rows->with_dist [V,36] = [feat | view | dist] (the level instead of the distance with
+ *           add_level) and / or rows->without [V,35] = [feat | view], per head hidden = relu(x w0^T + b0) [V,32] and
+ *           pre = hidden w1^T + b1 [V,k], and the two counts out->num_visible (V) and out->count (device or pinned host
+ *           memory).  rows->num_visible says how many rows there is room for: the number of anchors, V not being known
+ *   EMIT    every field of `out` but the counts, which the caller has read to size them; rows->num_visible is V from here on
  * No feature bank: the caller mixes the features.  The workspace and the rows must stay as they are until the backward
  * pass has run.  Outputs of gs355_decode_train_bytes: bytes of the workspace and of the backward pass's scratch (both
  * 256-byte aligned). */
-enum { GS355_TRAIN_ROWS = 1, GS355_TRAIN_INPUTS = 2, GS355_TRAIN_COUNT = 4, GS355_TRAIN_EMIT = 8 };
+enum { GS355_TRAIN_HEADS = 1, GS355_TRAIN_EMIT = 2 };
 typedef struct gs355_train_rows {
-    int32_t num_visible;    /* V; unused by the ROWS phase */
+    int32_t num_visible;    /* V, or the rows there is room for (HEADS) */
     int32_t compact_feat;   /* 1: anchors.feat is [V,32], one row per visible anchor (mixed features) */
     float *with_dist;       /* [V,36], 16-byte aligned, or NULL */
     float *without;         /* [V,35] or NULL */
-    const float *hidden[3]; /* [V,32], 16-byte aligned (backward pass) */
-    const float *pre[3];    /* [V,n] [V,7n] [V,3n] (COUNT: the first) */
+    const float *hidden[3]; /* [V,32], 16-byte aligned; written by the HEADS phase, like the next */
+    const float *pre[3];    /* [V,n] [V,7n] [V,3n], 16-byte aligned */
 } gs355_train_rows;
 typedef struct gs355_decode_cotangents { /* of the outputs; any pointer may be NULL (zeros) */
     const float *xyz, *color, *opacity, *scaling, *rot; /* [G,3] [G,3] [G,1] [G,3] [G,4] */

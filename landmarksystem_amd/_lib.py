@@ -25,7 +25,7 @@ PIPELINE_FAST = STAGE_PREPROCESS | STAGE_TILE_COUNT | STAGE_TILE_SCATTER | STAGE
 MAX_FAST_TILES = 36000 * 16  # limits of the tile-bucketed stages (the classic stages have neither)
 MAX_FAST_GAUSSIANS = 1 << 28
 DECODE_COUNT, DECODE_EMIT, DECODE_ALL = 1, 2, 3
-TRAIN_ROWS, TRAIN_INPUTS, TRAIN_COUNT, TRAIN_EMIT = 1, 2, 4, 8
+TRAIN_HEADS, TRAIN_EMIT = 1, 2
 
 EXPORTS = ("gs355_version", "gs355_last_error", "gs355_workspace_layout", "gs355_run", "gs355_render",
            "gs355_visible_filter", "gs355_anchor_filter", "gs355_decode_scratch_bytes", "gs355_decode_count",

@@ -102,60 +102,53 @@ class _TallLinear(torch.autograd.Function):
 
 
 class _DecodeTrain(torch.autograd.Function):
-    """The training decode around its matrix products (gs355_decode_train) with its whole backward pass in the kernels
+    """The training decode (gs355_decode_train) with its whole backward pass in the kernels
     (gs355_decode_train_backward): differentiable with respect to anchors, features, offsets, scales and the heads'
-    parameters.  The products going forward are the module's own (torch.addmm), so the Gaussians are bit for bit those
-    of its statements.  Workspace, input rows, hidden units and pre-activations live until the graph is dropped."""
+    parameters.  Workspace, input rows, hidden units and pre-activations (968 bytes per anchor) live until the graph is
+    dropped."""
 
     @staticmethod
     def forward(ctx, decoder, camera_center, visible, level, compact_feat, anchor, feat, offset, scaling, *params):
         dev, A, n = anchor.device, anchor.shape[0], decoder.n_offsets
         lib = _lib.load()
-        stream = torch.cuda.current_stream(dev)
+        stream = _raw_stream(dev)
         dec, an = decoder._train_structs(camera_center, visible, level, anchor, feat, offset, scaling, params)
         need, scratch = C.c_size_t(), C.c_size_t()
         _lib.check(lib.gs355_decode_train_bytes(A, 0, n, C.byref(need), C.byref(scratch)))
         f = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)  # noqa: E731
-        ws = torch.empty(need.value, dtype=torch.uint8, device=dev)
         if decoder._host_count is None:
             decoder._host_count = torch.zeros(2, dtype=torch.int32, pin_memory=True)
         counts = decoder._host_count  # (pinned: the kernels' stores land there, nothing is copied)
-        o, rows = _lib.Decoded(), _lib.TrainRows()
-        o.count, o.num_visible = counts.data_ptr(), counts.data_ptr() + 4
-
-        def run(phase, capacity=0):
-            _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), capacity, C.byref(o),
-                                              ws.data_ptr(), ws.numel(), phase, stream.cuda_stream))
-
-        run(_lib.TRAIN_ROWS)
-        stream.synchronize()
-        V = int(counts[1])
-        widths = [params[4 * j].shape[1] for j in range(3)]
-        with_dist = f(V, 36) if 36 in widths else None
-        without = f(V, 35) if 35 in widths else None
-        rows.num_visible, rows.compact_feat = V, 1 if compact_feat else 0
-        rows.with_dist = None if with_dist is None else with_dist.data_ptr()
-        rows.without = None if without is None else without.data_ptr()
-        run(_lib.TRAIN_INPUTS)
-        hidden, pre = [], []
+        # one block: workspace, then the rows with and without distance, hidden units and pre-activations, room for every
+        # anchor (how many are visible is only known on the device); every part 256-byte aligned
+        widths = {params[4 * j].shape[1] for j in range(3)}
+        sizes = [need.value, A * 36 * 4 if 36 in widths else 0, A * 35 * 4 if 35 in widths else 0]
+        sizes += [A * 32 * 4] * 3 + [A * n * k * 4 for k in (1, 7, 3)]
+        offsets, total = [], 0
+        for size in sizes:
+            offsets.append(total)
+            total += (size + 255) // 256 * 256
+        block = torch.empty(total, dtype=torch.uint8, device=dev)
+        at = [block.data_ptr() + o for o in offsets]
+        rows = _lib.TrainRows(A, 1 if compact_feat else 0, at[1] if sizes[1] else None, at[2] if sizes[2] else None)
         for j in range(3):
-            w0, b0, w1, b1 = params[4 * j:4 * j + 4]
-            hidden.append(torch.addmm(b0, with_dist if widths[j] == 36 else without, w0.t()).relu_())
-            pre.append(torch.addmm(b1, hidden[j], w1.t()))
-            rows.hidden[j], rows.pre[j] = hidden[j].data_ptr(), pre[j].data_ptr()
-            if j == 0:  # (the number of Gaussians is on its way while the other heads run)
-                run(_lib.TRAIN_COUNT)
-                counted = torch.cuda.Event()
-                counted.record(stream)
-        counted.synchronize()
-        G = int(counts[0])
+            rows.hidden[j], rows.pre[j] = at[3 + j], at[6 + j]
+        o = _lib.Decoded()
+        o.num_visible = counts.data_ptr() + 4
+        o.count = counts.data_ptr()
+        _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), 0, C.byref(o), at[0], need.value,
+                                          _lib.TRAIN_HEADS, stream))
+        torch.cuda.current_stream(dev).synchronize()
+        G, V = counts.tolist()
+        rows.num_visible = V
         out = (f(G, 3), f(G, 3), f(G, 1), f(G, 3), f(G, 4), f(V * n, 1), torch.empty(V * n, dtype=torch.bool, device=dev))
         if G > 0:
             o.xyz, o.color, o.opacity, o.scaling, o.rot = (t.data_ptr() for t in out[:5])
         o.neural_opacity, o.mask = out[5].data_ptr(), out[6].data_ptr()
-        run(_lib.TRAIN_EMIT, G)
-        ctx.decoder, ctx.num_visible, ctx.workspace, ctx.compact_feat = decoder, V, ws, compact_feat
-        ctx.rows = (with_dist, without, hidden, pre)
+        _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), G, C.byref(o), at[0], need.value,
+                                          _lib.TRAIN_EMIT, stream))
+        ctx.structs = (dec, an, rows, at[0], need.value)  # (pointers into the saved tensors and the block)
+        ctx.block, ctx.n_offsets = block, n
         ctx.save_for_backward(camera_center, visible, level, anchor, feat, offset, scaling, *params)
         ctx.mark_non_differentiable(out[6])
         ctx.set_materialize_grads(False)
@@ -164,15 +157,11 @@ class _DecodeTrain(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural, _g_mask):
-        camera_center, visible, level, anchor, feat, offset, scaling, *params = ctx.saved_tensors
-        dev, A, V = anchor.device, anchor.shape[0], ctx.num_visible
+        _camera_center, _visible, _level, anchor, feat, offset, scaling, *params = ctx.saved_tensors
+        dec, an, rows, workspace, workspace_bytes = ctx.structs
+        dev, A, V = anchor.device, anchor.shape[0], rows.num_visible
         lib = _lib.load()
         ptr = lambda t: None if t is None or t.numel() == 0 else t.data_ptr()  # noqa: E731
-        dec, an = ctx.decoder._train_structs(camera_center, visible, level, anchor, feat, offset, scaling, params)
-        with_dist, without, hidden, pre = ctx.rows
-        rows = _lib.TrainRows(V, 1 if ctx.compact_feat else 0, ptr(with_dist), ptr(without))
-        for j in range(3):
-            rows.hidden[j], rows.pre[j] = ptr(hidden[j]), ptr(pre[j])
         given = [None if g is None else g.contiguous() for g in (g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural)]
         cot = _lib.DecodeCotangents(*[ptr(g) for g in given])
         # (anchors that were not decoded have no gradient: their rows stay zero)
@@ -184,11 +173,11 @@ class _DecodeTrain(torch.autograd.Function):
         for j in range(3):
             out.w0[j], out.b0[j], out.w1[j], out.b1[j] = (ptr(t) for t in grads[4 + 4 * j:8 + 4 * j])
         need, scratch_bytes = C.c_size_t(), C.c_size_t()
-        _lib.check(lib.gs355_decode_train_bytes(A, V, ctx.decoder.n_offsets, C.byref(need), C.byref(scratch_bytes)))
+        _lib.check(lib.gs355_decode_train_bytes(A, V, ctx.n_offsets, C.byref(need), C.byref(scratch_bytes)))
         scratch = torch.empty(scratch_bytes.value // 4, dtype=torch.float32, device=dev)
-        _lib.check(lib.gs355_decode_train_backward(C.byref(dec), C.byref(an), C.byref(rows), ctx.workspace.data_ptr(),
-                                                   ctx.workspace.numel(), C.byref(cot), C.byref(out), scratch.data_ptr(),
-                                                   scratch.numel() * 4, _raw_stream(dev)))
+        _lib.check(lib.gs355_decode_train_backward(C.byref(dec), C.byref(an), C.byref(rows), workspace, workspace_bytes,
+                                                   C.byref(cot), C.byref(out), scratch.data_ptr(), scratch.numel() * 4,
+                                                   _raw_stream(dev)))
         return (None, None, None, None, None, *grads)
 
 

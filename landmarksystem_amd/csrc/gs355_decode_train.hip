@@ -4,8 +4,8 @@
 //
 //   rows      visible anchors per run of 128 and (scan) their ranks
 //   inputs    the list of visible anchors and the heads' input rows [feat | view | dist or level]
-//   (caller)  the heads' products, hidden = relu(W0 x + b0) and W1 hidden + b1
-//   count     kept offsets (opacity pre-activation > 0) per group of 32 rows and (scan) their output slots
+//   heads     hidden = relu(W0 x + b0) and W1 hidden + b1, kept offsets (opacity pre-activation > 0) per group of 32 rows
+//             and (scan) their output slots
 //   emit      activations and compaction of the kept offsets
 //   items     backward: cotangents of the outputs to those of the pre-activations, gradients of offsets and scales
 //   layers    backward: a wavefront takes 32 rows at a time back through the layers to the features (and view directions),
@@ -42,7 +42,7 @@ constexpr int kMaxOffsets = 10;
 
 struct TrainArgs {
     int A, n;
-    uint32_t V;            // rows (visible anchors)
+    uint32_t V;            // rows (visible anchors; going through the heads: as many as there is room for)
     int in_dim[3];
     const float* anchor;
     const float* feat;     // [A,32], or [V,32] with compact_feat
@@ -53,7 +53,9 @@ struct TrainArgs {
     const float* level;    // replaces the distance
     int compact_feat;
     const float* w0[3];
+    const float* b0[3];
     const float* w1[3];
+    const float* b1[3];
     float* with_dist;      // [V,36] input rows, or NULL
     float* without;        // [V,35] input rows, or NULL
     const float* hidden[3];  // [V,32]
@@ -161,18 +163,164 @@ __global__ __launch_bounds__(256) void train_inputs_kernel(TrainArgs d, const ui
     }
 }
 
-__global__ __launch_bounds__(256) void train_count_kernel(TrainArgs d, uint2* __restrict__ totals, uint32_t groups)
+// The heads going forward: hidden = relu(W0 x + b0) and W1 hidden + b1 for every row, 32 rows (a group) per wavefront and
+// step, and the number of kept offsets per group.  Both layers are v_mfma_f32_16x16x4_f32 with the weights (left operand,
+// rows = units) in registers for the whole kernel and 16 rows as columns.  Each eight inputs are two steps, the even ones
+// and the odd ones (lane quarter q: input 2 q, then 2 q + 1), the last four of 36 one more, and the bias is added last:
+// the order in which the framework's fp32 linear layers add at these shapes, so that training sees the same bits whichever
+// evaluates them (a saturated opacity's gradient hangs on the last bits of its pre-activation; layers of thousands of
+// rows; with fewer it may split the sum).  The accumulator of the first layer (register r of lane quarter q = unit
+// 4 q + r) becomes the second's right operand by two lane exchanges per pair of registers.  Outputs pass through LDS so
+// that they leave in 16-byte stores (a row of 70 is not a multiple of that).
+// Six library products, three activations and a counting pass took 250 us at 200k anchors (176k of them visible, ten
+// offsets); this takes 66 us for the 170 MB it moves.
+// The rows are as many as the device-side count of visible anchors says, `visible_rows`: nothing is read back before the
+// number of kept offsets is.
+constexpr int kHeadBlocks = 8;                           // of 16 outputs: opacity 1, covariance up to 5, colour up to 2
+constexpr int kHeadOut = 16 * 11 * kMaxOffsets;          // floats of 16 rows' outputs
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void swap_lane_halves(float& a, float& b)
 {
-    const uint32_t group = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (group >= groups) return;
-    const size_t first = (size_t)group * kGroup * d.n, end = min((size_t)d.V * d.n, first + (size_t)kGroup * d.n);
-    uint32_t kept = 0;
-    for (size_t i = first; i < end; i += 64) {  // uniform
-        const size_t k = i + lane;
-        kept += (uint32_t)__popcll(__ballot(k < end && d.pre[0][min(k, end - 1)] > 0.0f));
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 r = __builtin_amdgcn_permlane32_swap((unsigned)__float_as_int(a), (unsigned)__float_as_int(b), false, false);
+    a = __int_as_float((int)r.x);
+    b = __int_as_float((int)r.y);
+}
+__device__ __forceinline__ void swap_lane_rows(float& a, float& b)
+{
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 r = __builtin_amdgcn_permlane16_swap((unsigned)__float_as_int(a), (unsigned)__float_as_int(b), false, false);
+    a = __int_as_float((int)r.x);
+    b = __int_as_float((int)r.y);
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_heads_kernel(
+    TrainArgs d, const uint32_t* __restrict__ visible_rows, uint32_t* __restrict__ visible_out, float* __restrict__ hidden0, float* __restrict__ hidden1, float* __restrict__ hidden2,
+    float* __restrict__ pre0, float* __restrict__ pre1, float* __restrict__ pre2, uint2* __restrict__ totals)
+{
+    __shared__ float s_b0[3][32];
+    __shared__ float s_b1[kHeadBlocks * 16];
+    __shared__ __align__(16) float s_out[4][kHeadOut];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, quarter = lane >> 4, col = lane & 15;
+    const int n = d.n;
+    const uint32_t groups = (d.V + kGroup - 1) / kGroup;  // that have a place in `totals`
+    const uint32_t V = min(*visible_rows, d.V);
+    if (visible_out && blockIdx.x == 0 && threadIdx.x == 0) *visible_out = V;
+    auto block_head = [](int blk) { return blk == 0 ? 0 : blk < 6 ? 1 : 2; };
+    auto block_first = [](int blk) { return blk == 0 ? 0 : blk < 6 ? 16 * (blk - 1) : 16 * (blk - 6); };  // output within its head
+    for (int i = threadIdx.x; i < 3 * 32; i += 256) s_b0[i / 32][i % 32] = d.b0[i / 32][i % 32];
+    for (int i = threadIdx.x; i < kHeadBlocks * 16; i += 256) {
+        const int j = block_head(i / 16), o = block_first(i / 16) + i % 16;
+        s_b1[i] = o < head_outputs(j, n) ? d.b1[j][o] : 0.0f;
     }
-    if (lane == 0) totals[group] = make_uint2(kept, 0u);
+    auto input_of = [&](int step) { return step < 8 ? 8 * (step / 2) + 2 * quarter + (step & 1) : 32 + quarter; };
+    float w0[3][2][9], w1[kHeadBlocks][8];  // lane (quarter, column i): unit 16 block + i, input_of(step)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                const int in = input_of(k);
+                w0[j][h][k] = in < d.in_dim[j] ? d.w0[j][(16 * h + col) * d.in_dim[j] + in] : 0.0f;
+            }
+#pragma unroll
+    for (int blk = 0; blk < kHeadBlocks; ++blk) {
+        const int j = block_head(blk), o = block_first(blk) + col;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w1[blk][k] = o < head_outputs(j, n) ? d.w1[j][o * kFeat + input_of(k)] : 0.0f;
+    }
+    __syncthreads();
+    float* const out = s_out[wave];
+    for (uint32_t tile = blockIdx.x * 4 + wave; tile < groups; tile += gridDim.x * 4) {
+        const uint32_t row0 = tile * kGroup;
+        if (row0 >= V) {  // (the scan goes over all places)
+            if (lane == 0) totals[tile] = make_uint2(0u, 0u);
+            continue;
+        }
+        uint32_t row[2];
+        float x[2][2][9];  // [without, with distance][16 rows][step]
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            row[h] = row0 + 16u * h + (uint32_t)col;
+            const size_t r = min(row[h], V - 1);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {  // (column 35 of a row of 35: any finite value, its weight is zero)
+                x[0][h][k] = d.without ? d.without[r * 35 + min(input_of(k), 34)] : 0.0f;
+                x[1][h][k] = d.with_dist ? d.with_dist[r * 36 + input_of(k)] : 0.0f;
+            }
+        }
+        uint32_t kept = 0;
+        float right[3][2][8];  // hidden units as the second layer's right operand
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const bool dist = d.in_dim[j] == 36;
+            floatx4 acc[2][2] = {};
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+                        acc[h][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[j][u][k], dist ? x[1][h][k] : x[0][h][k], acc[h][u], 0, 0, 0);
+            float* const dst = j == 0 ? hidden0 : j == 1 ? hidden1 : hidden2;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    float v[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float pre = acc[h][u][r] + s_b0[j][16 * u + 4 * quarter + r];
+                        v[r] = pre > 0.0f || pre != pre ? pre : 0.0f;  // (NaN stays)
+                    }
+                    if (row[h] < V)
+                        *reinterpret_cast<float4*>(dst + (size_t)row[h] * kFeat + 16 * u + 4 * quarter) =
+                            make_float4(v[0], v[1], v[2], v[3]);
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) {
+                        swap_lane_rows(v[r], v[r + 2]);
+                        swap_lane_halves(v[r], v[r + 2]);
+                        right[j][h][4 * u + r] = v[r];
+                        right[j][h][4 * u + 2 + r] = v[r + 2];
+                    }
+                }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int blk = 0; blk < kHeadBlocks; ++blk) {
+                const int j = block_head(blk), count = head_outputs(j, n), first = block_first(blk);
+                if (first >= count) continue;  // uniform
+                floatx4 acc = {};
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[blk][k], right[j][h][k], acc, 0, 0, 0);
+                float* const dst = out + 16 * head_base(j, n) + col * count;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int o = first + 4 * quarter + r;
+                    const float v = acc[r] + s_b1[16 * blk + 4 * quarter + r];
+                    if (o < count) dst[o] = v;
+                    if (blk == 0) kept += (uint32_t)__popcll(__ballot(o < count && row[h] < V && v > 0.0f));
+                }
+            }
+            wave_lds_sync();
+            const uint32_t first_row = row0 + 16u * h, rows = first_row < V ? min(16u, V - first_row) : 0u;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const int count = head_outputs(j, n), floats = (int)rows * count;
+                float* const dst = (j == 0 ? pre0 : j == 1 ? pre1 : pre2) + (size_t)first_row * count;
+                const float* const src = out + 16 * head_base(j, n);
+                for (int i = lane; i < floats / 4; i += 64)
+                    reinterpret_cast<float4*>(dst)[i] = reinterpret_cast<const float4*>(src)[i];
+                if (lane < (floats & 3)) dst[(floats & ~3) + lane] = src[(floats & ~3) + lane];
+            }
+            wave_lds_sync();
+        }
+        if (lane == 0) totals[tile] = make_uint2(kept, 0u);
+    }
 }
 
 // The items (row, offset) of a group of 32 rows, row-major (the output order), two per thread of a workgroup of 256: the
@@ -554,7 +702,7 @@ __global__ __launch_bounds__(1024) void train_sum_kernel(TrainArgs d, const floa
 // Workspace kept from the forward to the backward pass: totals and bases (of the runs, then of the groups of rows), the
 // list of visible anchors.
 struct TrainLayout {
-    size_t totals, base, rows, total;
+    size_t totals, visible, base, rows, total;
 };
 TrainLayout train_layout(int32_t A)
 {
@@ -562,6 +710,7 @@ TrainLayout train_layout(int32_t A)
     const size_t groups = ((size_t)A + kGroup - 1) / kGroup;  // (at least as many as runs)
     TrainLayout L;
     L.totals = 0;
+    L.visible = groups * sizeof(uint2);  // the number of rows, behind the totals
     L.base = up(groups * sizeof(uint2) + 8);
     L.rows = L.base + up(groups * sizeof(uint2) + 8);
     L.total = L.rows + up((size_t)A * sizeof(uint32_t) + 4);
@@ -623,7 +772,9 @@ int train_args(const gs355_decoder* dec, const gs355_anchors* an, const gs355_tr
     for (int j = 0; j < 3; ++j) {
         a.in_dim[j] = dec->in_dim[j];
         a.w0[j] = dec->w0[j];
+        a.b0[j] = dec->b0[j];
         a.w1[j] = dec->w1[j];
+        a.b1[j] = dec->b1[j];
         a.hidden[j] = rows->hidden[j];
         a.pre[j] = rows->pre[j];
     }
@@ -671,25 +822,35 @@ int gs355_decode_train(const gs355_decoder* dec, const gs355_anchors* an, const 
     uint2* base = reinterpret_cast<uint2*>(ws + L.base);
     uint32_t* list = reinterpret_cast<uint32_t*>(ws + L.rows);
     switch (phase) {
-        case GS355_TRAIN_ROWS:
-            if (!out->num_visible) return set_error(GS355_EINVAL, "num_visible is NULL");
+        case GS355_TRAIN_HEADS: {
+            if (!out->num_visible || !out->count) return set_error(GS355_EINVAL, "num_visible / count is NULL");
+            uint32_t* visible = reinterpret_cast<uint32_t*>(ws + L.visible);
+            if (groups > 0) {
+                if ((reinterpret_cast<uintptr_t>(a.with_dist) & 15u) != 0)
+                    return set_error(GS355_EINVAL, "with_dist must be 16-byte aligned");
+                for (int j = 0; j < 3; ++j)
+                    if (!a.hidden[j] || !a.pre[j] || ((reinterpret_cast<uintptr_t>(a.hidden[j]) | reinterpret_cast<uintptr_t>(a.pre[j])) & 15u) != 0 ||
+                        !a.b0[j] || !a.b1[j] || (a.in_dim[j] == 36 ? !a.with_dist : !a.without))
+                        return set_error(GS355_EINVAL, "head %d: input rows, biases, hidden and pre-activations (16-byte aligned) are needed", j);
+            } else {
+                visible = nullptr;
+            }
             if (runs > 0) hipLaunchKernelGGL(train_rows_kernel, dim3((runs + 3) / 4), dim3(256), 0, s, a, totals, runs);
             GS355_CHECK_LAUNCH("decode train: rows");
-            return launch_run_scan(totals, base, (uint32_t)runs, nullptr, out->num_visible, s);
-        case GS355_TRAIN_INPUTS:
-            if (a.V == 0) return GS355_OK;
-            if (!a.with_dist && !a.without) return set_error(GS355_EINVAL, "with_dist and without are NULL");
-            if ((reinterpret_cast<uintptr_t>(a.with_dist) & 15u) != 0)
-                return set_error(GS355_EINVAL, "with_dist must be 16-byte aligned");
-            hipLaunchKernelGGL(train_inputs_kernel, dim3((runs + 3) / 4), dim3(256), 0, s, a, base, runs, list);
-            GS355_CHECK_LAUNCH("decode train: inputs");
-            return GS355_OK;
-        case GS355_TRAIN_COUNT:
-            if (!out->count) return set_error(GS355_EINVAL, "count is NULL");
-            if (a.V > 0 && !a.pre[0]) return set_error(GS355_EINVAL, "the opacity pre-activations are NULL");
-            if (groups > 0) hipLaunchKernelGGL(train_count_kernel, dim3((groups + 3) / 4), dim3(256), 0, s, a, totals, groups);
-            GS355_CHECK_LAUNCH("decode train: count");
+            rc = launch_run_scan(totals, base, (uint32_t)runs, nullptr, visible ? visible : out->num_visible, s);
+            if (rc) return rc;
+            if (groups > 0) {
+                hipLaunchKernelGGL(train_inputs_kernel, dim3((runs + 3) / 4), dim3(256), 0, s, a, base, runs, list);
+                GS355_CHECK_LAUNCH("decode train: inputs");
+                float* const hidden[3] = {const_cast<float*>(a.hidden[0]), const_cast<float*>(a.hidden[1]), const_cast<float*>(a.hidden[2])};
+                float* const pre[3] = {const_cast<float*>(a.pre[0]), const_cast<float*>(a.pre[1]), const_cast<float*>(a.pre[2])};
+                // (two workgroups per compute unit: a wavefront's weights are 118 registers)
+                hipLaunchKernelGGL(train_heads_kernel, dim3(min((groups + 3u) / 4u, 512u)), dim3(256), 0, s, a, visible,
+                                   out->num_visible, hidden[0], hidden[1], hidden[2], pre[0], pre[1], pre[2], totals);
+                GS355_CHECK_LAUNCH("decode train: heads");
+            }
             return launch_run_scan(totals, base, groups, out->count, nullptr, s);
+        }
         case GS355_TRAIN_EMIT:
             if (a.V == 0) return GS355_OK;
             if (!a.pre[0] || !a.pre[1] || !a.pre[2]) return set_error(GS355_EINVAL, "pre-activations must all be non-NULL");
