@@ -258,6 +258,11 @@ GS355_API int gs355_anchor_filter(const gs355_frame *frame, const gs355_gaussian
                                   const gs355_anchor_lod *lod, uint8_t *lod_mask, uint8_t *visible, int32_t *radii,
                                   void *stream);
 
+/* The visibility test of gs355_anchor_filter over stored parameters, as training has them: anchors->scales holds
+ * logarithms, anchors->rotations unnormalised quaternions, activated as by gs355_run_parameters.  No level of detail. */
+GS355_API int gs355_anchor_filter_parameters(const gs355_frame *frame, const gs355_gaussians *anchors, int32_t scale_stride,
+                                             uint8_t *visible, void *stream);
+
 /* The eval-mode gather of the reference's vanilla model (benchmarks/nerf/origin_gs/gs_model.py:199-208: means3D,
  * shs, opacity, scales, rotations -- or override colours / covariances -- indexed by the prefilter's visible mask,
  * five boolean-index operations there) as one pass: the rows of up to GS355_GATHER_MAX_ARRAYS row-major arrays

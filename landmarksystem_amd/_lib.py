@@ -32,7 +32,7 @@ EXPORTS = ("gs355_version", "gs355_last_error", "gs355_workspace_layout", "gs355
            "gs355_decode_count_static", "gs355_decode_emit", "gs355_decode_workspace_bytes", "gs355_decode",
            "gs355_backward_scratch_bytes", "gs355_render_backward", "gs355_gather_scratch_bytes", "gs355_gather_rows",
            "gs355_run_parameters", "gs355_render_parameters_backward", "gs355_decode_train_bytes", "gs355_decode_train",
-           "gs355_decode_train_backward", "gs355_render_frame")
+           "gs355_decode_train_backward", "gs355_render_frame", "gs355_anchor_filter_parameters")
 GATHER_MAX_ARRAYS, GATHER_MAX_ROW_BYTES = 8, 4096
 
 
@@ -218,6 +218,8 @@ def load() -> C.CDLL:
     lib.gs355_anchor_filter.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_int32, C.POINTER(AnchorLod),
                                         C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.gs355_anchor_filter.restype = C.c_int
+    lib.gs355_anchor_filter_parameters.argtypes = [C.POINTER(Frame), C.POINTER(Gaussians), C.c_int32, C.c_void_p, C.c_void_p]
+    lib.gs355_anchor_filter_parameters.restype = C.c_int
     lib.gs355_decode_scratch_bytes.argtypes = [C.c_int32, C.POINTER(C.c_size_t)]
     lib.gs355_decode_scratch_bytes.restype = C.c_int
     lib.gs355_decode_count.argtypes = [C.POINTER(Decoder), C.POINTER(Anchors), C.c_void_p, C.c_void_p, C.c_void_p,

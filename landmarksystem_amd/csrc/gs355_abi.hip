@@ -494,6 +494,23 @@ int gs355_anchor_filter(const gs355_frame* frame, const gs355_gaussians* anchors
     return launch_anchor_filter(fa, *anchors, x, radii, static_cast<hipStream_t>(stream));
 }
 
+int gs355_anchor_filter_parameters(const gs355_frame* frame, const gs355_gaussians* anchors, int32_t scale_stride,
+                                   uint8_t* visible, void* stream)
+{
+    int rc;
+    if ((rc = check_frame(frame, false))) return rc;
+    if ((rc = check_geometry_inputs(anchors))) return rc;
+    if (scale_stride < 3) return set_error(GS355_EINVAL, "scale_stride must be >= 3 (got %d)", scale_stride);
+    if (anchors->P_device) return set_error(GS355_EINVAL, "the anchor filter does not take a device-side count");
+    if (anchors->P > 0 && !anchors->scales) return set_error(GS355_EINVAL, "stored parameters are scales and rotations");
+    if (anchors->P > 0 && !visible) return set_error(GS355_EINVAL, "visible is NULL");
+    FilterArgs x;
+    x.scale_stride = scale_stride;
+    x.stored = 1;
+    x.visible = visible;
+    return launch_anchor_filter(make_args(frame), *anchors, x, nullptr, static_cast<hipStream_t>(stream));
+}
+
 int gs355_gather_scratch_bytes(int32_t P, size_t* bytes)
 {
     if (P < 0) return set_error(GS355_EINVAL, "P must be >= 0 (got %d)", P);

@@ -54,6 +54,7 @@ struct ParameterArgs {
 // Extras of the radii-only preprocess when it serves the anchor prefilter (by-value kernel argument).
 struct FilterArgs {
     int32_t scale_stride = 3;   // floats between the scale rows
+    int32_t stored = 0;         // scales are logarithms, rotations unnormalised quaternions
     int32_t use_lod = 0;
     gs355_anchor_lod lod = {};
     float log2_fork = 1.0f;     // (float)log2((double)fork), as the reference's host-side math.log2(fork)

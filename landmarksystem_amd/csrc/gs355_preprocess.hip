@@ -542,8 +542,14 @@ int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const Parame
 int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const FilterArgs& x, int32_t* radii, hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
-    hipLaunchKernelGGL((preprocess_kernel<true, false>), dim3((g.P + 255) / 256), dim3(256), 0, s, f, g, ParameterArgs(), x,
-                       (float*)nullptr, (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, radii);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((g.P + 255) / 256), dim3(256), 0, s, f, g, ParameterArgs(), x, (float*)nullptr,
+                           (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, radii);
+    };
+    if (x.stored)
+        launch(preprocess_kernel<true, true>);
+    else
+        launch(preprocess_kernel<true, false>);
     GS355_CHECK_LAUNCH("anchor filter");
     return GS355_OK;
 }

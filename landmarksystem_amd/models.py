@@ -400,7 +400,9 @@ class ScaffoldGS(nn.Module):
         self.renderer = _placeholder_renderer(self.background)
         self._cache = {}
         self._visibility_filter = self.voxel_visible_mask = None
-        self._pending = None  # (decode result, radii sized for its capacity) of a frame whose count is still on the device
+        # (decode result, radii sized for its capacity) of a frame whose count is still on the device; (None, radii) of a
+        # training frame
+        self._pending = None
 
     # `visibility_filter` (bool[G] over the decoded Gaussians) is a by-product the reference leaves on the model.
     # A frame rendered without reading the number of Gaussians back derives it when it is asked for.
@@ -408,8 +410,9 @@ class ScaffoldGS(nn.Module):
     def visibility_filter(self):
         if self._visibility_filter is None and self._pending is not None:
             res, radii = self._pending
-            G, _ = self.anchor_decoder.read_counts(res)
-            self._visibility_filter = radii[:G] > 0
+            if res is not None:
+                radii = radii[:self.anchor_decoder.read_counts(res)[0]]
+            self._visibility_filter = radii > 0
             self._pending = None
         return self._visibility_filter
 
@@ -503,9 +506,13 @@ class ScaffoldGS(nn.Module):
             if mask is not None:
                 self._anchor_mask = mask
             return visible
+        subset = self._anchor_subset()
+        if self.fuse_prefilter and subset is None and self._filters_parameters():
+            from . import pipeline
+            return pipeline.anchor_filter(_settings(viewpoint_camera, self.background, scaling_modifier, 1), self._anchor,
+                                          self._scaling, self._rotation, stored=True)[0]
         rasterizer = GaussianRasterizer(raster_settings=_settings(viewpoint_camera, self.background,
                                                                   scaling_modifier, 1))
-        subset = self._anchor_subset()
         means3D, scales, rotations = self.get_anchor, self.get_scaling, self.get_rotation
         if subset is not None:
             means3D, scales, rotations = means3D[subset], scales[subset], rotations[subset]
@@ -516,6 +523,14 @@ class ScaffoldGS(nn.Module):
         visible_mask = subset.clone()
         visible_mask[subset] = radii_pure > 0
         return visible_mask
+
+    def _filters_parameters(self):
+        """Whether the prefilter can take the stored parameters (training: nothing is cached, and the activations ahead of
+        one small kernel were six launches)."""
+        if any(getattr(type(self), n) is not getattr(ScaffoldGS, n) for n in ("get_anchor", "get_scaling", "get_rotation")):
+            return False
+        return self._scaling.dim() == 2 and all(t.is_cuda and t.dtype == torch.float32
+                                                for t in (self._anchor, self._scaling, self._rotation))
 
     def _before_prefilter(self, viewpoint_camera):
         pass
@@ -545,16 +560,17 @@ class ScaffoldGS(nn.Module):
             camera_center=viewpoint_camera.camera_center, anchor=self.get_anchor, anchor_feat=self.get_anchor_feat,
             offset=self.get_offset, scaling=self.get_scaling, visible_mask=voxel_visible_mask,
             level=self._decoder_level())
-        screenspace_points = torch.zeros_like(xyz, requires_grad=True) + 0
-        if retain_grad and screenspace_points.requires_grad:  # (not under torch.no_grad())
-            screenspace_points.retain_grad()
+        screenspace_points = torch.zeros_like(xyz, requires_grad=torch.is_grad_enabled())
+        if not retain_grad:  # (with retain_grad a leaf, whose .grad receives the rasterizer's gradient as it is)
+            screenspace_points = screenspace_points + 0
         self.renderer.raster_settings = _settings(viewpoint_camera, self.background, scaling_modifier, 1)
         rendered_image, radii, _ = self.renderer(
             means3D=xyz, means2D=screenspace_points, shs=None, colors_precomp=color, opacities=opacity, scales=scaling,
             rotations=rot, cov3D_precomp=None)
-        self.viewspace_points = screenspace_points
-        self.visibility_filter, self.voxel_visible_mask = radii > 0, voxel_visible_mask
-        self.offset_selection_mask, self.opacity = mask, neural_opacity
+        d = self.__dict__  # (plain attributes, set past nn.Module's search for parameters, buffers and modules)
+        d["viewspace_points"], d["voxel_visible_mask"] = screenspace_points, voxel_visible_mask
+        d["_visibility_filter"], d["_pending"] = None, (None, radii)
+        d["offset_selection_mask"], d["opacity"] = mask, neural_opacity
         return rendered_image, scaling
 
     def _forward_frame(self, viewpoint_camera, scaling_modifier=1.0, render_exclude_filter=None):

@@ -216,12 +216,14 @@ def visible_filter(inputs: FrameInputs) -> torch.Tensor:
     return radii
 
 
-def anchor_filter(settings, anchors: torch.Tensor, scaling: torch.Tensor, rotations: torch.Tensor, lod=None):
+def anchor_filter(settings, anchors: torch.Tensor, scaling: torch.Tensor, rotations: torch.Tensor, lod=None,
+                  stored: bool = False):
     """The anchor-level visibility prefilter of Scaffold-GS / Octree-GS in one kernel (gs355_anchor_filter).
 
     `scaling` is the models' f32[A,6] (or [A,3]); its first three columns are read in place.  `lod`: None, or a dict
     with level f32[A], extra_level f32[A], voxel_size, standard_dist, fork, resolution_scale, rounding
-    ("floor" | "round" | "ceil") and max_level.  Returns (visible bool[A], lod_mask bool[A] or None)."""
+    ("floor" | "round" | "ceil") and max_level.  `stored` (without lod): scaling and rotations are the stored
+    parameters, logarithms and unnormalised quaternions.  Returns (visible bool[A], lod_mask bool[A] or None)."""
     if not anchors.is_cuda:
         raise ValueError("anchors must be a tensor on the GPU (the rasterizer has no CPU path)")
     dev, A = anchors.device, anchors.shape[0]
@@ -232,13 +234,16 @@ def anchor_filter(settings, anchors: torch.Tensor, scaling: torch.Tensor, rotati
     rot = _dev_f32(rotations, dev, "rotations", (A, 4))
     keep = [_dev_f32(settings.viewmatrix, dev, "viewmatrix", (16,)), _dev_f32(settings.projmatrix, dev, "projmatrix", (16,)),
             _dev_f32(settings.campos, dev, "campos", (3,))]
-    f = _lib.Frame()
-    f.image_width, f.image_height = int(settings.image_width), int(settings.image_height)
-    f.tanfovx, f.tanfovy, f.scale_modifier = float(settings.tanfovx), float(settings.tanfovy), float(settings.scale_modifier)
-    f.viewmatrix, f.projmatrix, f.campos = keep[0].data_ptr(), keep[1].data_ptr(), keep[2].data_ptr()
-    g = _lib.Gaussians()
-    g.P, g.means3D, g.scales, g.rotations = A, _ptr(means), _ptr(sc), _ptr(rot)
+    f = _lib.Frame(int(settings.image_width), int(settings.image_height), float(settings.tanfovx), float(settings.tanfovy),
+                   float(settings.scale_modifier), 0, 0, keep[0].data_ptr(), keep[1].data_ptr(), keep[2].data_ptr())
+    g = _lib.Gaussians(A, _ptr(means), None, None, None, _ptr(sc), _ptr(rot))
     visible = torch.empty(A, dtype=torch.bool, device=dev)
+    if stored:
+        if lod is not None:
+            raise ValueError("the level of detail takes activated scales and rotations")
+        _lib.check(_lib.load().gs355_anchor_filter_parameters(C.byref(f), C.byref(g), int(sc.shape[1]), visible.data_ptr(),
+                                                              _raw_stream(dev)))
+        return visible, None
     mask, lod_c = None, None
     if lod is not None:
         level = _dev_f32(lod["level"], dev, "level", (A,))
