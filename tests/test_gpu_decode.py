@@ -317,3 +317,38 @@ def test_model_frames_without_reading_the_gaussian_count_back(gpu_device):
         assert fused._pending is not None  # nothing was read back yet
         assert torch.equal(plain.visibility_filter, fused.visibility_filter) and fused._pending is None
         assert torch.equal(plain(scene.camera), fused(scene.camera))  # a second frame over the same buffers
+
+
+@pytest.mark.parametrize("A,frac", [(1, 1.0), (255, 1.0), (511, 0.7), (512, 0.5), (513, 1.0), (1025, 0.02)])
+def test_feature_bank_at_the_edges_of_its_tiles(gpu_device, A, frac):
+    """Anchor counts around the 512 anchors one workgroup of the feature bank packs, from one visible anchor up."""
+    sc = scenes.config5(A=A)
+    g = torch.Generator().manual_seed(A)
+    dec, mlp, bank = decoder_with(sc, gpu_device, g, True, False, (True, False, True))
+    vis = torch.rand(A, generator=g) < frac
+    vis[A - 1] = True
+    cam = sc.camera.camera_center
+    got = dec(camera_center=cam.to(gpu_device), anchor=sc.anchor.to(gpu_device), anchor_feat=sc.anchor_feat.to(gpu_device),
+              offset=sc.offset.to(gpu_device), scaling=sc.scaling.to(gpu_device), visible_mask=vis.to(gpu_device))
+    redo = lambda keep=None: ao.decode(cam, sc.anchor, sc.anchor_feat, sc.offset, sc.scaling, vis, mlp, sc.n_offsets,  # noqa: E731
+                                       add_dist=(True, False, True), keep_override=keep, bank=bank)
+    compare(got, redo(), redo)
+
+
+@pytest.mark.parametrize("A", [1_048_576, 1_048_577 + 128])
+def test_decode_runs_beyond_one_round_of_their_prefix(gpu_device, A):
+    """8192 runs of 128 anchors fill one round of the runs' prefix: visible anchors on both sides of that line give
+    the Gaussians that a decode of the visible anchors alone gives."""
+    sc = scenes.config5(A=A)
+    dec = build_decoder(sc, gpu_device)
+    vis = torch.zeros(A, dtype=torch.bool)
+    vis[1000:1040] = True
+    vis[A - 200:] = True
+    cam = sc.camera.camera_center.to(gpu_device)
+    t = [x.to(gpu_device) for x in (sc.anchor, sc.anchor_feat, sc.offset, sc.scaling)]
+    got = dec(cam, *t, vis.to(gpu_device))
+    few = [x[vis.to(gpu_device)].contiguous() for x in t]
+    want = dec(cam, *few, torch.ones(240, dtype=torch.bool, device=gpu_device))
+    assert want[0].shape[0] > 0
+    for name, a, b in zip(("xyz", "color", "opacity", "scaling", "rot"), got[:5], want[:5]):
+        assert torch.equal(a, b), name
