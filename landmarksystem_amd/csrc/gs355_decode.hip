@@ -24,12 +24,12 @@
 // operand; general fp32 weights and features, the four fp32-only inputs (view
 // direction, distance) and the hidden activations enter as hi + lo fp16
 // pairs (22 significant bits; the lo x lo products, 2^-22 of a term, are
-// left out), so the result carries fp32-level accuracy either way.  The low
-// parts of the weights live in LDS, their high parts in registers.
+// left out), so the result carries fp32-level accuracy either way.  A workgroup
+// keeps the weights' fragments, high and low parts, in LDS.
 //
-// Work follows the visible anchors: a wavefront takes runs of 128 consecutive
-// anchors, packs the visible ones (in order) into dense tiles of 32 and decodes
-// those only.
+// Work follows the visible anchors: the visible ones of every run of 128
+// consecutive anchors are packed (in order) into dense tiles of 32, and a
+// wavefront decodes one tile at a time.
 //
 // Output order is the reference's boolean-mask order: row-major over (visible
 // anchor, offset).  Two launches: count kept offsets per anchor (opacity head
@@ -67,7 +67,8 @@ struct DecodeArgs {
     // one-call decode (gs355_decode): the count pass leaves per-run totals behind, a one-workgroup scan turns
     // them into run bases, and the emit pass (which recomputes the opacity head: matrix instructions are cheap
     // here, registers and memory requests are not) places its Gaussians from those instead of per-anchor offsets
-    uint2* run_totals;       // [runs] (kept offsets, visible anchors) per run of kRun anchors, or NULL
+    uint2* run_totals;       // [runs] (kept offsets, visible anchors) per run of anchors, or NULL
+    uint2* run_tiles;        // [runs] kept offsets of the run before each of its four tiles, 16 bits each (with run_totals)
     const uint2* run_base;   // [runs] exclusive prefix of run_totals, or NULL
     float* neural_opacity;   // [A_vis * n] tanh of every pre-activation, in visible-anchor order, or NULL
     uint8_t* kept_mask;      // [A_vis * n] pre-activation > 0, or NULL
@@ -103,21 +104,14 @@ __device__ __forceinline__ half8_t to_half8(const float v[8])
 // operand: slots 0..3 hold columns ka..ka+3, slots 4..7 columns kb..kb+3 (zero outside the matrix).  Loads are
 // unconditional at clamped (in-range) positions and masked afterwards, so that none of them waits for another:
 // the fragments of a head are fetched with all loads in flight together.
-// `lo`: what the fp16 rounding of each entry left over, itself rounded to fp16.
-__device__ __forceinline__ half8_t weight_fragment(const float* __restrict__ w, int rows, int cols, int row, int ka,
-                                                   int kb, bool enable = true, bool lo = false)
+__device__ __forceinline__ void weight_values(const float* __restrict__ w, int rows, int cols, int row, int ka, int kb,
+                                              float v[8])
 {
-    float v[8];
     const int r = min(row, rows - 1);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = w[(size_t)r * cols + min((j < 4 ? ka : kb - 4) + j, cols - 1)];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (enable && row < rows && (j < 4 ? ka : kb - 4) + j < cols) ? v[j] : 0.0f;
-    if (lo) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] -= (float)(_Float16)v[j];
-    }
-    return to_half8(v);
+    for (int j = 0; j < 8; ++j) v[j] = (row < rows && (j < 4 ? ka : kb - 4) + j < cols) ? v[j] : 0.0f;
 }
 
 // Bias for an accumulator: register v = 4b + t holds row 8b + 4*half + t.  `bias` is the head's bias vector
@@ -126,92 +120,61 @@ __device__ __forceinline__ floatx16 bias_rows(const float* bias, int row0, int h
 {
     floatx16 c;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) c[v] = bias[row0 + 8 * (v >> 2) + 4 * half + (v & 3)];
+    for (int g = 0; g < 4; ++g) {
+        const float4 b = *reinterpret_cast<const float4*>(bias + row0 + 8 * g + 4 * half);
+        c[4 * g] = b.x, c[4 * g + 1] = b.y, c[4 * g + 2] = b.z, c[4 * g + 3] = b.w;
+    }
     return c;
 }
 
-// Weight fragments of one head, held in registers for the whole kernel.
+// Weight fragments of one head: an A operand's share for each lane.
 //   layer 1, k-steps 0 and 1: the 32 anchor features, slot j of half h <-> feature 16s + 8h + j
 //   layer 1, k-step 2:        the four fp32-only inputs twice on half 0 (slots 0..3 meet their hi parts, slots
-//                             4..7 their lo parts, both against W0[:, 32..35]); half 1 is zero
+//                             4..7 their lo parts, both against W0[:, 32..35]); half 1 meets zero inputs
 //   layer 2, k-step s:        slot j of half h <-> hidden unit 16s + 4h + j (j < 4) or 16s + 8 + 4h + (j - 4),
 //                             the units held by accumulator registers 8s..8s+7 of that lane
-template <int kTiles>
-struct HeadWeights {
-    half8_t w0[3];          // layer 1: [32 x in]
-    half8_t w1[kTiles][2];  // layer 2: [outputs x 32] in row tiles of 32
-};
+// Every wavefront needs the same fragments, so a workgroup keeps one copy in LDS, hi parts and, for weights that
+// fp16 cannot represent, lo parts: a head's fragments follow one another in the order w0[0..2], w1[0][0], w1[0][1],
+// w1[1][0], ..., 64 lanes each but for w0[2], whose half 1 never matters and reads half 0's 32.
+constexpr int kOpacityFrags = 0, kCovFrags = 288, kColourFrags = 832, kAllFrags = 1120;  // first lane entry of each head
 
-template <int kTiles>
-__device__ __forceinline__ void load_head(const DecodeArgs& d, int head, int outputs, int row, int half,
-                                          HeadWeights<kTiles>& w, bool lo = false)
+__device__ __forceinline__ int frag_entry(int f, int lane)  // f: 0..2 layer 1, 3.. layer 2
 {
-    const int in = d.in_dim[head];
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-        w.w0[s] = weight_fragment(d.w0[head], kFeat, in, row, 16 * s + 8 * half, 16 * s + 8 * half + 4, true, lo);
-    w.w0[2] = weight_fragment(d.w0[head], kFeat, in, row, 32, 32, half == 0, lo);
-#pragma unroll
-    for (int r = 0; r < kTiles; ++r)
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            w.w1[r][s] = weight_fragment(d.w1[head], outputs, kFeat, 32 * r + row, 16 * s + 4 * half,
-                                         16 * s + 8 + 4 * half, true, lo);
+    return f == 2 ? 128 + (lane & 31) : f < 2 ? 64 * f + lane : 160 + 64 * (f - 3) + lane;
 }
 
-// The low parts of a head's weight fragments, kept in LDS: [fragment][lane], fragments in the order w0[0..2],
-// w1[0][0], w1[0][1], w1[1][0], ...  Every wavefront holds the same fragments in its lanes, so the workgroup shares
-// one copy; `store_head_lo` is called by one wavefront per head.
-template <int kTiles>
-__device__ __forceinline__ void store_head_lo(const DecodeArgs& d, int head, int outputs, int row, int half, int lane,
-                                              half8_t (*dst)[64], bool lo = true)
+// One wavefront computes fragment f of a head and stores its hi parts and (`lo` not NULL) its lo parts.
+__device__ __forceinline__ void stage_fragment(const DecodeArgs& d, int head, int outputs, int f, int lane,
+                                               half8_t* __restrict__ hi, half8_t* __restrict__ lo)
 {
-    HeadWeights<kTiles> w;
-    load_head<kTiles>(d, head, outputs, row, half, w, lo);
-#pragma unroll
-    for (int s = 0; s < 3; ++s) dst[s][lane] = w.w0[s];
-#pragma unroll
-    for (int r = 0; r < kTiles; ++r)
-#pragma unroll
-        for (int s = 0; s < 2; ++s) dst[3 + 2 * r + s][lane] = w.w1[r][s];
-}
-
-// Store an accumulator's rows into the anchor's LDS row, head outputs at `base`.  Rows that do not exist
-// (>= outputs; their accumulators hold zeros: masked weights, zero bias) are stored too, all of them at row
-// `outputs` -- the first word after the head, which the stores that follow in program order overwrite (the next
-// head's first output, or the anchor's scaling) -- so that no store is predicated: 16 conditional stores cost five
-// instructions and a branch each.  A row tile that lies inside the head entirely takes constant offsets.
-__device__ __forceinline__ void store_rows(float* __restrict__ dst_anchor, int base, int outputs, int row0, int half,
-                                           const floatx16& c)
-{
-    float* __restrict__ dst = dst_anchor + base;
-    const int lane_row = row0 + 4 * half;
-    if (row0 + 32 <= outputs) {  // uniform
-#pragma unroll
-        for (int v = 0; v < 16; ++v) dst[lane_row + 8 * (v >> 2) + (v & 3)] = c[v];
-    } else {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) dst[min(lane_row + 8 * (v >> 2) + (v & 3), outputs)] = c[v];
+    const int row = lane & 31, half = lane >> 5;
+    float v[8];
+    if (f < 2) weight_values(d.w0[head], kFeat, d.in_dim[head], row, 16 * f + 8 * half, 16 * f + 8 * half + 4, v);
+    else if (f == 2) weight_values(d.w0[head], kFeat, d.in_dim[head], row, 32, 32, v);
+    else {
+        const int r = (f - 3) >> 1, s = (f - 3) & 1;
+        weight_values(d.w1[head], outputs, kFeat, 32 * r + row, 16 * s + 4 * half, 16 * s + 8 + 4 * half, v);
     }
+    half8_t h, l;
+    split_half8(v, h, l);
+    const int at = frag_entry(f, lane);
+    hi[at] = h;
+    if (lo) lo[at] = l;
 }
 
-// One head for one tile of 32 anchors: the kTiles accumulators of the second layer (rows = outputs
-// 32r + 8b + 4*half + t, column = this lane's anchor) go to the anchor's LDS row as soon as each is complete
-// (one accumulator live at a time).
-// `wlo`: the head's low weight fragments in LDS (kWLo), read right before their matrix instruction.
-// kWInLds: the weight fragments themselves are read from `whi` (same order as `wlo`) instead of `w`: the
-// covariance head's nine fragments would otherwise hold 36 registers for the whole kernel.
-template <int kTiles, bool kSplit, bool kWLo, bool kWInLds = false>
-__device__ __forceinline__ void run_head(const HeadWeights<kTiles>& w, const half8_t (*whi)[64],
-                                         const half8_t (*wlo)[64], int lane,
+// One head for one tile of 32 anchors; `store(r, c)` receives row tile r of its outputs (rows = outputs
+// 32r + 8b + 4*half + t, column = this lane's anchor), one accumulator live at a time.
+// `hi`, `lo`: the head's fragments in LDS, read right before their matrix instruction.
+template <int kTiles, bool kSplit, bool kWLo, class Store>
+__device__ __forceinline__ void run_head(const half8_t* __restrict__ hi, const half8_t* __restrict__ lo, int lane,
                                          const float* bias0, const float* bias1, const half8_t X[kSplit ? 5 : 3],
-                                         int half, float* __restrict__ dst_anchor, int base, int outputs)
+                                         int half, Store store)
 {
     // layer 1: hidden = W0 [32 x in] * X^T + b0  (X[3], X[4]: the low parts of features that fp16 cannot hold)
     floatx16 h = bias_rows(bias0, 0, half);
     half8_t w0[3];
 #pragma unroll
-    for (int s = 0; s < 3; ++s) w0[s] = kWInLds ? whi[s][lane] : w.w0[s];
+    for (int s = 0; s < 3; ++s) w0[s] = hi[frag_entry(s, lane)];
 #pragma unroll
     for (int s = 0; s < 3; ++s) h = __builtin_amdgcn_mfma_f32_32x32x16_f16(w0[s], X[s], h, 0, 0, 0);
     if constexpr (kSplit) {
@@ -220,7 +183,8 @@ __device__ __forceinline__ void run_head(const HeadWeights<kTiles>& w, const hal
     }
     if constexpr (kWLo) {  // low parts of the weights against the high parts of the inputs
 #pragma unroll
-        for (int s = 0; s < 3; ++s) h = __builtin_amdgcn_mfma_f32_32x32x16_f16(wlo[s][lane], X[s], h, 0, 0, 0);
+        for (int s = 0; s < 3; ++s)
+            h = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[frag_entry(s, lane)], X[s], h, 0, 0, 0);
     }
     // ReLU, then hi/lo split: registers 8s..8s+7 are the B operand of k-step s
     half8_t hh[2], hl[2];
@@ -237,12 +201,13 @@ __device__ __forceinline__ void run_head(const HeadWeights<kTiles>& w, const hal
         floatx16 c = bias_rows(bias1, 32 * r, half);
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            const half8_t w1 = kWInLds ? whi[3 + 2 * r + s][lane] : w.w1[r][s];
+            const half8_t w1 = hi[frag_entry(3 + 2 * r + s, lane)];
             c = __builtin_amdgcn_mfma_f32_32x32x16_f16(w1, hh[s], c, 0, 0, 0);
             c = __builtin_amdgcn_mfma_f32_32x32x16_f16(w1, hl[s], c, 0, 0, 0);
-            if constexpr (kWLo) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(wlo[3 + 2 * r + s][lane], hh[s], c, 0, 0, 0);
+            if constexpr (kWLo)
+                c = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[frag_entry(3 + 2 * r + s, lane)], hh[s], c, 0, 0, 0);
         }
-        store_rows(dst_anchor, base, outputs, 32 * r, half, c);
+        store(r, c);
     }
 }
 
@@ -253,56 +218,11 @@ __device__ __forceinline__ float fast_sigmoid(float x)
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
 }
 
-// Per-lane inputs of one tile of 32 anchors.
-template <bool kCountOnly>
-struct TileInputs {
-    float4 f[4] = {};          // features 16s + 8*half .. +7 in f[2s], f[2s+1], s = 0..1
-    float pos[3] = {0.f, 0.f, 0.f};
-    float sc3[3] = {0.f, 0.f, 0.f};
-    float extra = 0.f;  // the anchor's level when it replaces the distance
-    uint32_t first_slot = 0;
-    float ofv[kCountOnly ? 1 : 5][3] = {};
-};
-
-// A wavefront takes runs of kRun consecutive anchors, packs the visible ones (in order) into dense tiles of 32
-// and runs the MLPs on those only: the work follows the number of visible anchors, not of anchors.
-constexpr int kRun = 128;
-
-// kSplit: the features enter as hi + lo fp16 pairs (general fp32 features; two more matrix instructions per head).
-// kWLo: so do the weights (general fp32 weights; their low fragments take 19 KB of LDS in the emit pass, which
-// then runs three wavefronts per workgroup so that two workgroups still share a CU, held to 256 registers).
-constexpr int decode_waves(bool count_only, bool weights_lo) { return (weights_lo && !count_only) ? 3 : 4; }
-
-template <bool kCountOnly, bool kSplit, bool kWLo>
-__global__ __launch_bounds__((64 * decode_waves(kCountOnly, kWLo)), (!kCountOnly ? 2 : 4)) void decode_kernel(DecodeArgs d, uint32_t* __restrict__ counts,
-                                                     const uint32_t* __restrict__ offsets, uint32_t capacity,
-                                                     float* __restrict__ xyz, float* __restrict__ color,
-                                                     float* __restrict__ opacity, float* __restrict__ scaling_out,
-                                                     float* __restrict__ rot)
+// Biases of the three heads in LDS, zero-padded: b0 at [head*32], b1 of opacity / cov / colour at 96 / 128 / 224.
+__device__ __forceinline__ void stage_biases(const DecodeArgs& d, float* __restrict__ s_bias, int threads)
 {
-    // per wavefront: [32 anchors][stride] floats; stride odd -> conflict-free column access.  Emit pass: the
-    // 11n head outputs of an anchor, then its scaling (6), position (3) and first output slot (1).
-    constexpr int kStrideMax = kCountOnly ? 11 : 123;
-    constexpr int kListFloats = kCountOnly ? 0 : 160;  // 320 16-bit item numbers after the anchors' rows
-    constexpr int kRunFloats = kRun / 4;                // kRun 8-bit positions of the run's visible anchors
-    constexpr int kWaves = decode_waves(kCountOnly, kWLo);
-    __shared__ float s_out[kWaves][32 * kStrideMax + kListFloats + kRunFloats];
-
-    // biases of the three heads, zero-padded: b0 at [head*32], b1 of opacity / cov / colour at 96 / 128 / 224
-    __shared__ float s_bias[256];
-    // low parts of the weight fragments: opacity head 0..4, covariance 5..13, colour 14..18
-    __shared__ half8_t s_wlo[kWLo ? (kCountOnly ? 5 : 19) : 1][kWLo ? 64 : 1];
-    // the covariance head's weight fragments (0..8) and, where LDS has room for them beside the low parts, the
-    // colour head's (9..13), for the emit pass: read from here right before their matrix instruction instead of
-    // holding 36 + 20 registers for the whole kernel
-    constexpr bool kColourInLds = !kCountOnly && !kWLo;
-    __shared__ half8_t s_whi[kCountOnly ? 1 : (kColourInLds ? 14 : 9)][kCountOnly ? 1 : 64];
-    const half8_t (*const whi)[64] = reinterpret_cast<const half8_t (*)[64]>(s_whi);
-    const half8_t (*const wlo)[64] = reinterpret_cast<const half8_t (*)[64]>(s_wlo);
-
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
     const int n = d.n;
-    for (int t = threadIdx.x; t < 256; t += 64 * kWaves) {
+    for (int t = threadIdx.x; t < 256; t += threads) {
         float v = 0.0f;
         if (t < 96) v = d.b0[t >> 5][t & 31];
         else if (t < 128) v = (t - 96) < n ? d.b1[0][t - 96] : 0.0f;
@@ -310,275 +230,439 @@ __global__ __launch_bounds__((64 * decode_waves(kCountOnly, kWLo)), (!kCountOnly
         else v = (t - 224) < 3 * n ? d.b1[2][t - 224] : 0.0f;
         s_bias[t] = v;
     }
-    if constexpr (kWLo) {
-        if (wave == 0) store_head_lo<1>(d, 0, n, col, half, lane, s_wlo);
-        if constexpr (!kCountOnly) {
-            if (wave == 1) store_head_lo<3>(d, 1, 7 * n, col, half, lane, s_wlo + 5);
-            if (wave == 2) store_head_lo<1>(d, 2, 3 * n, col, half, lane, s_wlo + 14);
-        }
-    }
-    if constexpr (!kCountOnly) {
-        if (wave == kWaves - 1) store_head_lo<3>(d, 1, 7 * n, col, half, lane, s_whi, false);
-        if constexpr (kColourInLds) {
-            if (wave == kWaves - 2) store_head_lo<1>(d, 2, 3 * n, col, half, lane, s_whi + 9, false);
-        }
-    }
-    __syncthreads();
-    HeadWeights<1> w_op;
-    load_head<1>(d, 0, n, col, half, w_op);
-    const HeadWeights<3> w_cov = {};  // unused: read from s_whi
-    HeadWeights<1> w_col = {};
-    if (!kCountOnly && !kColourInLds) load_head<1>(d, 2, 3 * n, col, half, w_col);
-    const int stride = kCountOnly ? 11 : 11 * n + 13;
-    const int items = 32 * n;  // (anchor, offset) pairs of a tile: item = anchor_in_tile * n + offset
-    const int inv_n = (65536 + n - 1) / n;  // item / n == (item * inv_n) >> 16 for item < 32 n, n <= 10
-    const uint64_t lanes_below = (1ull << lane) - 1ull;
-    const int runs = (d.A + kRun - 1) / kRun;
-    float* __restrict__ mine = s_out[wave];
-    uint8_t* __restrict__ run_list = reinterpret_cast<uint8_t*>(mine + 32 * kStrideMax + kListFloats);
-    const float cx = d.campos[0], cy = d.campos[1], cz = d.campos[2];
+}
 
-    for (int run = blockIdx.x * kWaves + wave; run < runs; run += gridDim.x * kWaves) {
-      // positions (within the run) of its visible anchors, in order: lane covers anchors lane and 64 + lane
-      const int base = run * kRun;
-      const int a0 = base + lane, a1 = base + 64 + lane;
-      const bool v0 = a0 < d.A && d.visible[a0] != 0, v1 = a1 < d.A && d.visible[a1] != 0;
-      const uint64_t m0 = __ballot(v0), m1 = __ballot(v1);
-      const int n0 = __popcll(m0), nvis = n0 + __popcll(m1);
-      if (kCountOnly && counts) {  // anchors that are not decoded keep nothing
-          if (!v0 && a0 < d.A) counts[a0] = 0;
-          if (!v1 && a1 < d.A) counts[a1] = 0;
-      }
-      if (nvis == 0) {  // uniform
-          if (kCountOnly && d.run_totals && lane == 0) d.run_totals[run] = make_uint2(0u, 0u);
-          continue;
-      }
-      uint32_t run_kept = 0;  // count pass: this lane's share of the run's kept offsets
-      // emit pass of the one-call decode: the run's first output slot, advanced tile by tile (uniform), and the
-      // rank of its first visible anchor among all visible anchors
-      uint32_t run_slot = 0, run_rank = 0;
-      if (!kCountOnly && d.run_base) {
-          const uint2 rb = d.run_base[run];
-          run_slot = rb.x;
-          run_rank = rb.y;
-      }
-      if (v0) run_list[__popcll(m0 & lanes_below)] = (uint8_t)lane;
-      if (v1) run_list[n0 + __popcll(m1 & lanes_below)] = (uint8_t)(64 + lane);
-      wave_lds_sync();
-      // Everything a tile needs from global memory is requested before the first use, and without a
-      // condition: a lane without an anchor (or an item without one) reads anchor 0's data, which nothing uses
-      // (matrix columns are independent, and only items of visible anchors are ever emitted) -- conditional
-      // loads would each become a branch, and the values' first use would wait inside the condition.
-      // Features, position and level of the tile's anchors.
-      auto fetch_anchor = [&](int a, TileInputs<kCountOnly>& in) {
+// Anchors come in runs of kRun consecutive ones, whose visible ones are packed (in order) into dense tiles of 32; a
+// wavefront runs the MLPs on one tile at a time: the work follows the number of visible anchors, not of anchors.
+constexpr int kRun = 128, kRunTiles = kRun / 32;
+
+// A run's visible anchors as bits, and as a list of their positions within the run, in order.
+struct Visible {
+    uint64_t m0, m1;
+    __device__ __forceinline__ int count() const { return __popcll(m0) + __popcll(m1); }
+    __device__ __forceinline__ void pack(int lane, uint8_t* __restrict__ list) const
+    {
+        const uint64_t below = (1ull << lane) - 1ull;
+        if ((m0 >> lane) & 1ull) list[__popcll(m0 & below)] = (uint8_t)lane;
+        if ((m1 >> lane) & 1ull) list[__popcll(m0) + __popcll(m1 & below)] = (uint8_t)(64 + lane);
+    }
+};
+
+// The mask of a run's anchors, two a lane; requested well before it is looked at.
+struct VisibleBytes {
+    uint8_t b0 = 0, b1 = 0;
+    __device__ __forceinline__ void load(const DecodeArgs& d, int base, int lane)
+    {
+        b0 = base + lane < d.A ? d.visible[base + lane] : 0;
+        b1 = base + 64 + lane < d.A ? d.visible[base + 64 + lane] : 0;
+    }
+    __device__ __forceinline__ Visible look() const { return Visible{__ballot(b0 != 0), __ballot(b1 != 0)}; }
+};
+
+// Features, position and level of a tile's anchors.  Everything is requested without a condition: a lane without an
+// anchor reads anchor 0's data, which nothing uses (matrix columns are independent, and only items of visible anchors
+// are ever counted or emitted) -- conditional loads would each become a branch with its own wait.
+struct TileInputs {
+    float4 f[4];  // features 16s + 8*half .. +7 in f[2s], f[2s+1], s = 0..1
+    float pos[3];
+    float extra = 0.f;  // the anchor's level when it replaces the distance
+    __device__ __forceinline__ void load(const DecodeArgs& d, int a, int half)
+    {
         const float4* __restrict__ f4 = reinterpret_cast<const float4*>(d.feat + (size_t)a * kFeat);
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {  // features 16s + 8*half .. +7
-            in.f[2 * s] = f4[4 * s + 2 * half];
-            in.f[2 * s + 1] = f4[4 * s + 2 * half + 1];
+        for (int s = 0; s < 2; ++s) {
+            f[2 * s] = f4[4 * s + 2 * half];
+            f[2 * s + 1] = f4[4 * s + 2 * half + 1];
         }
 #pragma unroll
-        for (int k = 0; k < 3; ++k) in.pos[k] = d.anchor[3 * (size_t)a + k];
-        if (d.level) in.extra = d.level[a];
-      };
-      // The count pass has registers to spare and a run's tiles are otherwise a chain of memory latencies: it
-      // requests the next tile's inputs before it waits for the current tile's.
-      TileInputs<kCountOnly> ahead;
-      if constexpr (kCountOnly) fetch_anchor(col < nvis ? base + (int)run_list[col] : 0, ahead);
-      for (int first = 0; first < nvis; first += 32) {  // dense tiles of the run
-        const bool vis = first + col < nvis;  // lanes l and l+32 share entry first + l
-        const int a = vis ? base + (int)run_list[first + col] : 0;
-        const uint64_t any = __ballot(vis);  // bits l and l + 32 belong to entry l of the tile
-        TileInputs<kCountOnly> in;
-        if constexpr (kCountOnly) {
-            in = ahead;
-            if (first + 32 < nvis)  // uniform
-                fetch_anchor(first + 32 + col < nvis ? base + (int)run_list[first + 32 + col] : 0, ahead);
-        } else {
-            {  // as fetch_anchor, written out: through the lambda this pass spills three times as many registers
-                const float4* __restrict__ f4 = reinterpret_cast<const float4*>(d.feat + (size_t)a * kFeat);
+        for (int k = 0; k < 3; ++k) pos[k] = d.anchor[3 * (size_t)a + k];
+        if (d.level) extra = d.level[a];
+    }
+    // B operand: X^T, column = anchor; slots as described at the weight fragments
+    template <bool kSplit>
+    __device__ __forceinline__ void operand(const DecodeArgs& d, float cx, float cy, float cz, bool vis, int half,
+                                            half8_t X[kSplit ? 5 : 3]) const
+    {
+        float x8[8];
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    in.f[2 * s] = f4[4 * s + 2 * half];
-                    in.f[2 * s + 1] = f4[4 * s + 2 * half + 1];
+        for (int s = 0; s < 2; ++s) {
+            x8[0] = f[2 * s].x, x8[1] = f[2 * s].y, x8[2] = f[2 * s].z, x8[3] = f[2 * s].w;
+            x8[4] = f[2 * s + 1].x, x8[5] = f[2 * s + 1].y, x8[6] = f[2 * s + 1].z, x8[7] = f[2 * s + 1].w;
+            if constexpr (kSplit) split_half8(x8, X[s], X[3 + s]);  // the second: what the fp16 rounding left over
+            else X[s] = to_half8(x8);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x8[j] = 0.0f;
+        if (vis && half == 0) {
+            float vx = pos[0] - cx, vy = pos[1] - cy, vz = pos[2] - cz;
+            const float dist = sqrtf(vx * vx + vy * vy + vz * vz);
+            vx /= dist;
+            vy /= dist;
+            vz /= dist;
+            const float in4[4] = {vx, vy, vz, d.level ? extra : dist};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const _Float16 top = (_Float16)in4[t];
+                x8[t] = (float)top;
+                x8[4 + t] = in4[t] - (float)top;
+            }
+        }
+        X[2] = to_half8(x8);
+    }
+};
+
+// Which of its anchor's offsets this lane's opacity rows keep (bit m: offset m; the mask opacity > 0 is the sign of
+// the pre-activation: tanh is odd, monotone and tanh(x) = x for the smallest floats).  Rows that do not exist hold zero.
+__device__ __forceinline__ uint32_t kept_rows(const floatx16& c, bool vis, int half)
+{
+    uint32_t mask = 0;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) mask |= c[v] > 0.0f ? 1u << (8 * (v >> 2) + (v & 3)) : 0u;
+    return vis ? mask << (4 * half) : 0u;
+}
+
+// kSplit: the features enter as hi + lo fp16 pairs (general fp32 features; two more matrix instructions per head).
+// kWLo: so do the weights (general fp32 weights).
+// The count pass: the opacity head of every visible anchor and how many offsets it keeps.  Four wavefronts per SIMD;
+// a run's tiles are otherwise a chain of memory latencies, so the next tile's inputs are requested before the current
+// tile's are waited for, and the next run's mask before the run is walked.  While there are fewer runs than workgroups
+// (`shared_run`) the four wavefronts of a workgroup take a tile each of one run instead of a run each.
+constexpr int kCountWaves = 4;
+constexpr int kCountCap = 1024;  // workgroups: four per CU
+static_assert(kCountWaves == kRunTiles, "a workgroup's wavefronts share a run tile by tile");
+
+template <bool kSplit, bool kWLo>
+__global__ __launch_bounds__(64 * kCountWaves, 4) void decode_count_kernel(DecodeArgs d, uint32_t* __restrict__ counts,
+                                                                       int shared_run)
+{
+    __shared__ float s_bias[256];
+    __shared__ half8_t s_hi[kCovFrags];
+    __shared__ half8_t s_lo[kWLo ? kCovFrags : 1];
+    __shared__ uint8_t s_list[kCountWaves][kRun];
+    __shared__ uint32_t s_kept[kRunTiles];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
+    const int runs = (d.A + kRun - 1) / kRun;
+    const int step = shared_run ? gridDim.x : gridDim.x * kCountWaves;
+    int run = shared_run ? blockIdx.x : wave * gridDim.x + blockIdx.x;
+    const int first_entry = shared_run ? 32 * wave : 0, entry_step = shared_run ? kRun : 32;
+    VisibleBytes next;
+    if (run < runs) next.load(d, run * kRun, lane);
+    stage_biases(d, s_bias, 64 * kCountWaves);
+    for (int f = wave; f < 5; f += kCountWaves) stage_fragment(d, 0, d.n, f, lane, s_hi, kWLo ? s_lo : nullptr);
+    __syncthreads();
+    uint8_t* __restrict__ list = s_list[wave];
+    const float cx = d.campos[0], cy = d.campos[1], cz = d.campos[2];
+
+    for (; run < runs; run += step) {  // the same rounds for every wavefront where a run is shared
+        const Visible now = next.look();
+        const int base = run * kRun, nvis = now.count();
+        if (run + step < runs) next.load(d, base + step * kRun, lane);
+        now.pack(lane, list);
+        if (counts) {  // anchors that are not decoded keep nothing
+            if (!((now.m0 >> lane) & 1ull) && base + lane < d.A) counts[base + lane] = 0;
+            if (!((now.m1 >> lane) & 1ull) && base + 64 + lane < d.A) counts[base + 64 + lane] = 0;
+        }
+        wave_lds_sync();
+        uint32_t kept01 = 0, kept23 = 0;  // this lane's share of the kept offsets of the run's tiles, 16 bits each
+        TileInputs ahead;
+        int a_ahead = first_entry + col < nvis ? base + (int)list[first_entry + col] : 0;
+        if (first_entry < nvis) ahead.load(d, a_ahead, half);
+        for (int first = first_entry; first < nvis; first += entry_step) {  // dense tiles of the run
+            const bool vis = first + col < nvis;  // lanes l and l+32 share entry first + l
+            const TileInputs in = ahead;
+            const int a = a_ahead;
+            if (first + entry_step < nvis) {  // uniform
+                a_ahead = first + entry_step + col < nvis ? base + (int)list[first + entry_step + col] : 0;
+                ahead.load(d, a_ahead, half);
+            }
+            wave_lds_sync();  // the fragments are read again for every tile: kept across tiles they would spill
+            half8_t X[kSplit ? 5 : 3];
+            in.operand<kSplit>(d, cx, cy, cz, vis, half, X);
+            run_head<1, kSplit, kWLo>(s_hi, s_lo, lane, s_bias, s_bias + 96, X, half, [&](int, const floatx16& c) {
+                const uint32_t kept = (uint32_t)__popc(kept_rows(c, vis, half));
+                const uint32_t field = kept << (first & 32 ? 16 : 0);
+                (first & 64 ? kept23 : kept01) += field;
+                if (counts) {
+                    const uint32_t both = kept + (uint32_t)__shfl_xor((int)kept, 32, 64);
+                    if (half == 0 && vis) counts[a] = both;
                 }
+            });
+        }
+        if (d.run_totals) {
 #pragma unroll
-                for (int k = 0; k < 3; ++k) in.pos[k] = d.anchor[3 * (size_t)a + k];
-                if (d.level) in.extra = d.level[a];
+            for (int off = 32; off > 0; off >>= 1) {
+                kept01 += (uint32_t)__shfl_xor((int)kept01, off, 64);
+                kept23 += (uint32_t)__shfl_xor((int)kept23, off, 64);
             }
-            // half 0: scaling[0..2] (offset scale), half 1: scaling[3..5] (Gaussian scale)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) in.sc3[k] = d.scaling[6 * (size_t)a + 3 * half + k];
-            if (offsets) in.first_slot = offsets[a];  // entry 0's value is the tile's first output slot
-            // the learned offsets of the items this lane's position covers (item = entry * n + offset)
-            int item_anchor[5], item_offset[5];
-#pragma unroll
-            for (int r = 0; r < 5; ++r) {
-                const int it = min(r * 64 + lane, items - 1);
-                const int al = (it * inv_n) >> 16;
-                item_offset[r] = it - al * n;
-                item_anchor[r] = (int)run_list[min(first + al, nvis - 1)];
+            if (shared_run) {
+                if (lane == 0) s_kept[wave] = (wave & 2 ? kept23 : kept01) >> (wave & 1 ? 16 : 0);
+                __syncthreads();
+                kept01 = s_kept[0] | s_kept[1] << 16;
+                kept23 = s_kept[2] | s_kept[3] << 16;
+                __syncthreads();
             }
-#pragma unroll
-            for (int r = 0; r < 5; ++r) {
-                const float* __restrict__ of = d.offset + ((size_t)(base + item_anchor[r]) * n + item_offset[r]) * 3;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) in.ofv[r][k] = of[k];
+            if (lane == 0 && (!shared_run || wave == 0)) {
+                const uint32_t k0 = kept01 & 0xFFFFu, k1 = kept01 >> 16, k2 = kept23 & 0xFFFFu, k3 = kept23 >> 16;
+                d.run_totals[run] = make_uint2(k0 + k1 + k2 + k3, (uint32_t)nvis);
+                d.run_tiles[run] = make_uint2(k0 << 16, (k0 + k1) | (k0 + k1 + k2) << 16);
             }
         }
-        // B operand: X^T, column = anchor; slots as described at HeadWeights
+        wave_lds_sync();
+    }
+}
+
+// The emit pass: all heads, then the activations of the kept (anchor, offset) items on dense wavefronts of survivors.
+//
+// What bounds it is how many tiles are in flight: a tile is a chain of memory and matrix latencies.  With all 11n head
+// outputs of 32 anchors in LDS and part of the weights in registers a wavefront needed 27 KB and 256 registers: six
+// wavefronts per CU.  Colours and covariances now pass through the same 72 words per anchor one after the other, all
+// weights are shared through LDS, and the learned offsets are read for survivors only, so twelve wavefronts of 10 KB
+// and at most 168 registers fill a CU with one workgroup; an anchor's rows are a multiple of 16 bytes apart, so that
+// accumulators leave four rows at a time.
+//
+// A workgroup takes every gridDim.x-th run and its wavefronts deal out the tiles of those runs, not the runs: the
+// count pass left the visible anchors and the tiles' first slots of every run behind.  A wavefront requests the inputs of
+// its next tile before the current one's heads and turns them into matrix operands before the current one's stores: a wait for
+// them after the stores would be a wait for the stores as well.
+//
+// Measured (fp32 weights and features, n = 10): 500k visible anchors that keep 3.9M offsets, 358 MB in and out, 120 ->
+// 84 us; a million anchors behind a level-of-detail mask 59 -> 38 us; 60k anchors, where a wavefront has one tile, 31 -> 15.
+constexpr int kEmitWaves = 12;
+constexpr int kEmitCap = 256;  // workgroups: one per CU
+constexpr int kRowWords = 72;  // an anchor's words: first opacity, colour, offset scale, position; then covariance
+constexpr int kRowColour = 16, kRowExtra = 48;
+
+struct __align__(16) EmitWave {
+    float rows[32][kRowWords];
+    float scale[32][3];  // the anchor's Gaussian scale
+    uint16_t list[320];  // kept items, in order: 16 * entry + offset
+    uint8_t anchors[2][kRun];  // positions of the run's visible anchors: the current tile's run and the next tile's
+};
+
+// Rows 32r .. 32r + 31 of an accumulator to the anchor's words: groups of eight rows that hold an output.
+__device__ __forceinline__ void store_rows(float* __restrict__ dst, int r, int outputs, int half, const floatx16& c)
+{
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+        if (32 * r + 8 * g < outputs)  // uniform
+            *reinterpret_cast<float4*>(dst + 32 * r + 8 * g + 4 * half) =
+                make_float4(c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]);
+}
+
+template <bool kSplit, bool kWLo>
+__global__ __launch_bounds__(64 * kEmitWaves, 3) void decode_emit_kernel(DecodeArgs d, const uint32_t* __restrict__ offsets,
+                                                                      uint32_t capacity, float* __restrict__ xyz,
+                                                                      float* __restrict__ color, float* __restrict__ opacity,
+                                                                      float* __restrict__ scaling_out, float* __restrict__ rot)
+{
+    __shared__ EmitWave s_wave[kEmitWaves];
+    __shared__ float s_bias[256];
+    __shared__ half8_t s_hi[kAllFrags];
+    __shared__ half8_t s_lo[kWLo ? kAllFrags : 1];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
+    const int n = d.n;
+    const int runs = (d.A + kRun - 1) / kRun;
+    stage_biases(d, s_bias, 64 * kEmitWaves);
+    for (int f = wave; f < 19; f += kEmitWaves) {
+        const int head = f < 5 ? 0 : f < 14 ? 1 : 2;
+        const int at = head == 0 ? kOpacityFrags : head == 1 ? kCovFrags : kColourFrags;
+        stage_fragment(d, head, (head == 0 ? 1 : head == 1 ? 7 : 3) * n, f - (head == 0 ? 0 : head == 1 ? 5 : 14), lane, s_hi + at,
+                       kWLo ? s_lo + at : nullptr);
+    }
+    __syncthreads();
+    EmitWave& my = s_wave[wave];
+    const float cx = d.campos[0], cy = d.campos[1], cz = d.campos[2];
+
+    // 64 of the workgroup's runs at a time, a lane's worth each: run first_run + lane * gridDim.x
+    for (int first_run = blockIdx.x; first_run < runs; first_run += 64 * gridDim.x) {
+        const int my_run = first_run + lane * (int)gridDim.x;
+        uint32_t tiles = my_run < runs ? kRunTiles : 0;  // two-call decode: the visible anchors are not known here
+        uint2 run_base = make_uint2(0u, 0u), run_tiles = make_uint2(0u, 0u);
+        if (d.run_base && my_run < runs) {
+            tiles = (d.run_totals[my_run].y + 31u) >> 5;
+            run_base = d.run_base[my_run];
+            run_tiles = d.run_tiles[my_run];
+        }
+        uint32_t upto = tiles;
+#pragma unroll
+        for (int k = 1; k < 64; k <<= 1) {
+            const uint32_t u = (uint32_t)__shfl_up((int)upto, k, 64);
+            if (lane >= k) upto += u;
+        }
+        const int units = __builtin_amdgcn_readlane((int)upto, 63);
+        // unit u of these runs: tile `first / 32` of the run whose anchors start at `base`
+        auto locate = [&](int u, int& base, int& first, int& index) {
+            index = min(__popcll(__ballot((int)upto <= u)), 63);
+            base = (first_run + index * (int)gridDim.x) * kRun;
+            first = 32 * (u - __builtin_amdgcn_readlane((int)(upto - tiles), index));
+        };
+        TileInputs ahead;
+        float sc_ahead[3];  // half 0: scaling[0..2] (offset scale), half 1: scaling[3..5] (Gaussian scale)
+        auto fetch = [&](const uint8_t* __restrict__ anchors, int base, int first, int nvis) {
+            const int a = first + col < nvis ? base + (int)anchors[first + col] : 0;
+            ahead.load(d, a, half);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) sc_ahead[k] = d.scaling[6 * (size_t)a + 3 * half + k];
+        };
+        // the current tile, and the next: run, tile, visible anchors; `seen` is the next tile's
+        int base = 0, first = 0, index = 0, nvis = 0, base1 = 0, first1 = 0, index1 = 0;
+        Visible seen = {0ull, 0ull};
         half8_t X[kSplit ? 5 : 3];
-        const float ax = in.pos[0], ay = in.pos[1], az = in.pos[2];
-        {
-            float x8[8];
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                x8[0] = in.f[2 * s].x, x8[1] = in.f[2 * s].y, x8[2] = in.f[2 * s].z, x8[3] = in.f[2 * s].w;
-                x8[4] = in.f[2 * s + 1].x, x8[5] = in.f[2 * s + 1].y, x8[6] = in.f[2 * s + 1].z, x8[7] = in.f[2 * s + 1].w;
-                if constexpr (kSplit) split_half8(x8, X[s], X[3 + s]);  // the second: what the fp16 rounding left over
-                else X[s] = to_half8(x8);                               // all zero for an invisible anchor
+        if (wave < units) {
+            VisibleBytes bytes, bytes1;
+            locate(wave, base, first, index);
+            bytes.load(d, base, lane);
+            if (wave + kEmitWaves < units) {
+                locate(wave + kEmitWaves, base1, first1, index1);
+                bytes1.load(d, base1, lane);
             }
+            const Visible v = bytes.look();
+            nvis = v.count();
+            v.pack(lane, my.anchors[0]);
+            wave_lds_sync();
+            fetch(my.anchors[0], base, first, nvis);
+            seen = bytes1.look();
+            ahead.operand<kSplit>(d, cx, cy, cz, first + col < nvis, half, X);
+        }
+        int buffer = 0;
+        for (int unit = wave; unit < units; unit += kEmitWaves, buffer ^= 1) {
+            const bool vis = first + col < nvis;  // lanes l and l+32 share entry first + l
+            const uint8_t* __restrict__ anchors = my.anchors[buffer];
+            uint32_t slot, run_rank = 0;
+            if (offsets) {  // two-call decode: the first anchor's slot is the tile's (past the last tile: not used)
+                slot = first < nvis ? offsets[base + (int)anchors[first]] : 0u;
+            } else {  // the run's first slot and the kept items of the tiles before; the rank of its first visible anchor
+                const uint32_t before = first & 64 ? (uint32_t)__builtin_amdgcn_readlane((int)run_tiles.y, index)
+                                                   : (uint32_t)__builtin_amdgcn_readlane((int)run_tiles.x, index);
+                slot = (uint32_t)__builtin_amdgcn_readlane((int)run_base.x, index) + (first & 32 ? before >> 16 : before & 0xFFFFu);
+                run_rank = (uint32_t)__builtin_amdgcn_readlane((int)run_base.y, index);
+            }
+            {
+                float* __restrict__ extra = my.rows[col] + kRowExtra;
+                if (half == 0) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) x8[j] = 0.0f;
-            if (vis && half == 0) {
-                float vx = ax - cx, vy = ay - cy, vz = az - cz;
-                const float dist = sqrtf(vx * vx + vy * vy + vz * vz);
-                vx /= dist;
-                vy /= dist;
-                vz /= dist;
-                const float in4[4] = {vx, vy, vz, d.level ? in.extra : dist};
+                    for (int k = 0; k < 3; ++k) {
+                        extra[k] = sc_ahead[k];
+                        extra[3 + k] = ahead.pos[k];
+                    }
+                } else {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const _Float16 top = (_Float16)in4[t];
-                    x8[t] = (float)top;
-                    x8[4 + t] = in4[t] - (float)top;
+                    for (int k = 0; k < 3; ++k) my.scale[col][k] = sc_ahead[k];
                 }
             }
-            X[2] = to_half8(x8);
-        }
+            const int nvis1 = seen.count();
+            int base2 = 0, first2 = 0, index2 = 0;
+            VisibleBytes bytes;
+            if (unit + kEmitWaves < units) {  // uniform
+                seen.pack(lane, my.anchors[buffer ^ 1]);
+                wave_lds_sync();
+                fetch(my.anchors[buffer ^ 1], base1, first1, nvis1);
+                if (unit + 2 * kEmitWaves < units) {
+                    locate(unit + 2 * kEmitWaves, base2, first2, index2);
+                    bytes.load(d, base2, lane);
+                }
+            }
 
-        // ---- opacity head ----
-        // the mask opacity > 0 is the sign of the pre-activation (tanh is odd, monotone and tanh(x) = x for the
-        // smallest floats), so tanh itself is only evaluated for the offsets that are kept
-        run_head<1, kSplit, kWLo>(w_op, nullptr, wlo, lane, s_bias, s_bias + 96, X, half, mine + col * stride, 0, n);
-        if (kCountOnly) {
-            wave_lds_sync();
-            if (half == 0 && vis) {
-                uint32_t kept = 0;
-                for (int m = 0; m < n; ++m) kept += mine[col * stride + m] > 0.0f ? 1u : 0u;
-                if (counts) counts[a] = kept;
-                run_kept += kept;
+            // ---- opacity head; the kept items in the reference's order (anchor-major) ----
+            // tanh itself is only evaluated for the offsets that are kept
+            uint32_t mask = 0;
+            run_head<1, kSplit, kWLo>(s_hi + kOpacityFrags, s_lo + kOpacityFrags, lane, s_bias, s_bias + 96, X, half,
+                                      [&](int r, const floatx16& c) {
+                                          mask = kept_rows(c, vis, half);
+                                          store_rows(my.rows[col], r, n, half, c);
+                                      });
+            const uint32_t both = mask | (uint32_t)__shfl_xor((int)mask, 32, 64);
+            const uint32_t mine = (uint32_t)__popc(both);
+            uint32_t end = mine;  // inclusive prefix over the 32 anchors, the same in both halves
+            end += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)end, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+            end += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)end, 0x112, 0xf, 0xf, false);
+            end += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)end, 0x114, 0xf, 0xf, false);
+            end += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)end, 0x118, 0xf, 0xf, false);
+            end += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)end, 0x142, 0xa, 0xf, false);  // row_bcast 15
+            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)end, 31);
+            while (mask) {  // each half lists the rows it holds
+                const int m = __builtin_ctz(mask);
+                my.list[end - mine + (uint32_t)__popc(both & ((1u << m) - 1u))] = (uint16_t)(16 * col + m);
+                mask &= mask - 1u;
             }
             wave_lds_sync();
-            continue;
-        }
+            // Items are in output order and slots come from a prefix of the kept counts, so the survivors of a tile
+            // occupy consecutive output slots: lanes write consecutive addresses.
+            // The learned offset of the lane's next survivor is requested ahead of its use.
+            float of[3];
+            auto fetch_offset = [&](uint32_t s) {
+                const int it = (int)my.list[s < total ? s : 0];
+                const float* __restrict__ src =
+                    d.offset + ((size_t)(base + (int)anchors[first + (it >> 4)]) * n + (it & 15)) * 3;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) of[k] = src[k];
+            };
+            if (total > 0) fetch_offset(lane);
 
-        // ---- covariance and colour heads ----
-        run_head<3, kSplit, kWLo, true>(w_cov, whi, wlo + (kWLo ? 5 : 0), lane, s_bias + 32, s_bias + 128, X, half,
-                                        mine + col * stride, n, 7 * n);
-        run_head<1, kSplit, kWLo, kColourInLds>(w_col, whi + (kColourInLds ? 9 : 0), wlo + (kWLo ? 14 : 0), lane,
-                                                s_bias + 64, s_bias + 224, X, half, mine + col * stride, 8 * n, 3 * n);
-        {
-            float* __restrict__ extra = mine + col * stride + 11 * n;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) extra[3 * half + k] = in.sc3[k];
-            if (half == 0) {
-                extra[6] = ax;
-                extra[7] = ay;
-                extra[8] = az;
-                reinterpret_cast<uint32_t*>(extra)[9] = in.first_slot;
-            }
-        }
-        wave_lds_sync();
-
-        // ---- compact the kept (anchor, offset) items of the tile: about one in five survives the mask, and the
-        // activations below are the expensive part, so they run on dense wavefronts of survivors only ----
-        uint16_t* __restrict__ list = reinterpret_cast<uint16_t*>(mine + 32 * stride);  // [32 n] item numbers
-        uint32_t total = 0;
-        float pre[5];  // the items' opacity pre-activations, all requested before the first is looked at
-        bool exists[5];
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            const int it = min(r * 64 + lane, items - 1);
-            const int al = (it * inv_n) >> 16, m = it - al * n;
-            pre[r] = mine[al * stride + m];
-            exists[r] = r * 64 + lane < items && ((any >> al) & 1ull);
-        }
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            if (r * 64 >= items) break;  // uniform
-            const bool kept = exists[r] && pre[r] > 0.0f;
-            const uint64_t b = __ballot(kept);
-            if (kept) list[total + (uint32_t)__popcll(b & lanes_below)] = (uint16_t)(r * 64 + lane);
-            total += (uint32_t)__popcll(b);
-        }
-        wave_lds_sync();
-
-        // Items are numbered anchor-major and the slots come from an exclusive scan of the per-anchor counts, so
-        // the survivors of a tile occupy consecutive output slots from the slot of its first anchor: lanes write
-        // consecutive addresses.  No global reads in here: the learned offsets sit in registers of the lane that
-        // requested them (item = round * 64 + lane) and are fetched across lanes.
-        const uint32_t tile_slot = d.run_base ? run_slot : reinterpret_cast<const uint32_t*>(mine)[11 * n + 9];
-        run_slot += total;
-        // training-mode by-products: tanh of every pre-activation of the visible anchors and the mask, indexed by
-        // (visible anchor, offset): the tile's entries are the run's visible anchors first .. first + 31
-        if (d.neural_opacity || d.kept_mask) {
-            const size_t row0 = ((size_t)run_rank + (size_t)first) * (size_t)n;
-#pragma unroll
-            for (int r = 0; r < 5; ++r) {
-                const int it = r * 64 + lane;
-                if (it >= items) break;
-                const int al = (it * inv_n) >> 16, m = it - al * n;
-                if ((any >> al) & 1ull) {
-                    const float v = mine[al * stride + m];
+            // ---- colour head; opacity, colour and position of the survivors ----
+            run_head<1, kSplit, kWLo>(s_hi + kColourFrags, s_lo + (kWLo ? kColourFrags : 0), lane, s_bias + 64, s_bias + 224, X,
+                                      half, [&](int r, const floatx16& c) {
+                                          store_rows(my.rows[col] + kRowColour, r, 3 * n, half, c);
+                                      });
+            // the next tile's operands, before this tile's stores
+            half8_t X1[kSplit ? 5 : 3];
+            ahead.operand<kSplit>(d, cx, cy, cz, first1 + col < nvis1, half, X1);
+            seen = bytes.look();
+            wave_lds_sync();
+            // training-mode by-products: tanh of every pre-activation of the visible anchors and the mask, indexed by
+            // (visible anchor, offset): the tile's entries are the run's visible anchors first .. first + 31
+            if (d.neural_opacity || d.kept_mask) {
+                const size_t row0 = ((size_t)run_rank + (size_t)first) * (size_t)n;
+                const int inv_n = (65536 + n - 1) / n;  // item / n == (item * inv_n) >> 16 for item < 32 n, n <= 10
+                const int items = min(32, nvis - first) * n;
+                for (int it = lane; it < items; it += 64) {
+                    const int al = (it * inv_n) >> 16, m = it - al * n;
+                    const float v = my.rows[al][m];
                     if (d.neural_opacity) d.neural_opacity[row0 + (size_t)it] = tanhf(v);
                     if (d.kept_mask) d.kept_mask[row0 + (size_t)it] = v > 0.0f ? 1 : 0;
                 }
             }
-        }
-        for (uint32_t s0 = 0; s0 < total; s0 += 64) {  // uniform
-            const uint32_t s = s0 + lane;
-            const bool live = s < total;
-            const int it = live ? (int)list[s] : 0;
-            float off3[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-            for (int r = 0; r < 5; ++r) {
+            for (uint32_t s0 = 0; s0 < total; s0 += 64) {  // uniform
+                const uint32_t s = s0 + lane, pos = slot + s;
+                const float now_of[3] = {of[0], of[1], of[2]};
+                if (s0 + 64 < total) fetch_offset(s + 64);
+                if (s >= total || pos >= capacity) continue;  // the second cannot happen when capacity comes from the count pass
+                const int it = (int)my.list[s], m = it & 15;
+                const float* __restrict__ o = my.rows[it >> 4];
+                opacity[pos] = tanhf(o[m]);
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    const float got = __shfl(in.ofv[r][k], it & 63, 64);
-                    if ((it >> 6) == r) off3[k] = got;
+                    color[3 * (size_t)pos + k] = fast_sigmoid(o[kRowColour + 3 * m + k]);
+                    xyz[3 * (size_t)pos + k] = o[kRowExtra + 3 + k] + now_of[k] * o[kRowExtra + k];
                 }
             }
-            const uint32_t pos = tile_slot + s;
-            if (!live || pos >= capacity) continue;  // the second cannot happen when capacity comes from the count pass
-            const int al = (it * inv_n) >> 16, m = it - al * n;
-            const float* __restrict__ o = mine + al * stride;
-            const float* __restrict__ extra = o + 11 * n;
-            const float* __restrict__ c7 = o + n + 7 * m;
-            const float* __restrict__ c3 = o + 8 * n + 3 * m;
-            opacity[pos] = tanhf(o[m]);
+            wave_lds_sync();
+
+            // ---- covariance head, over the same words; scaling and rotation of the survivors ----
+            run_head<3, kSplit, kWLo>(s_hi + kCovFrags, s_lo + (kWLo ? kCovFrags : 0), lane, s_bias + 32, s_bias + 128, X, half,
+                                      [&](int r, const floatx16& c) { store_rows(my.rows[col], r, 7 * n, half, c); });
+            wave_lds_sync();
+            for (uint32_t s0 = 0; s0 < total; s0 += 64) {  // uniform
+                const uint32_t s = s0 + lane, pos = slot + s;
+                if (s >= total || pos >= capacity) continue;
+                const int it = (int)my.list[s];
+                const float* __restrict__ c7 = my.rows[it >> 4] + 7 * (it & 15);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                color[3 * (size_t)pos + k] = fast_sigmoid(c3[k]);
-                scaling_out[3 * (size_t)pos + k] = extra[3 + k] * fast_sigmoid(c7[k]);
-                xyz[3 * (size_t)pos + k] = extra[6 + k] + off3[k] * extra[k];
+                for (int k = 0; k < 3; ++k) scaling_out[3 * (size_t)pos + k] = my.scale[it >> 4][k] * fast_sigmoid(c7[k]);
+                const float q0 = c7[3], q1 = c7[4], q2 = c7[5], q3 = c7[6];
+                // q / max(|q|, 1e-12) with one reciprocal square root (1 ulp) instead of a root and four divisions
+                const float inv = __builtin_amdgcn_rsqf(fmaxf(q0 * q0 + q1 * q1 + q2 * q2 + q3 * q3, 1e-24f));
+                rot[4 * (size_t)pos + 0] = q0 * inv;
+                rot[4 * (size_t)pos + 1] = q1 * inv;
+                rot[4 * (size_t)pos + 2] = q2 * inv;
+                rot[4 * (size_t)pos + 3] = q3 * inv;
             }
-            const float q0 = c7[3], q1 = c7[4], q2 = c7[5], q3 = c7[6];
-            // q / max(|q|, 1e-12) with one reciprocal square root (1 ulp) instead of a root and four divisions
-            const float inv = __builtin_amdgcn_rsqf(fmaxf(q0 * q0 + q1 * q1 + q2 * q2 + q3 * q3, 1e-24f));
-            rot[4 * (size_t)pos + 0] = q0 * inv;
-            rot[4 * (size_t)pos + 1] = q1 * inv;
-            rot[4 * (size_t)pos + 2] = q2 * inv;
-            rot[4 * (size_t)pos + 3] = q3 * inv;
-        }
-        wave_lds_sync();
-      }
-      if (kCountOnly && d.run_totals) {  // the run's totals: kept offsets (summed over the lanes), visible anchors
-          uint32_t t = run_kept;
+            wave_lds_sync();
+            base = base1, first = first1, index = index1, nvis = nvis1;
+            base1 = base2, first1 = first2, index1 = index2;
 #pragma unroll
-          for (int off = 32; off > 0; off >>= 1) t += (uint32_t)__shfl_xor((int)t, off, 64);
-          if (lane == 0) d.run_totals[run] = make_uint2(t, (uint32_t)nvis);
-      }
+            for (int k = 0; k < (kSplit ? 5 : 3); ++k) X[k] = X1[k];
+        }
     }
 }
 
@@ -751,10 +835,6 @@ __global__ __launch_bounds__(256) void feature_bank_kernel(BankArgs k)
 
 }  // namespace
 
-struct DecodeLaunch {
-    DecodeArgs args;
-};
-
 int check_decoder(const gs355_decoder* dec, const gs355_anchors* an)
 {
     if (!dec || !an) return set_error(GS355_EINVAL, "decoder / anchors is NULL");
@@ -818,6 +898,7 @@ static int fill_args(const gs355_decoder* dec, const gs355_anchors* an, bool all
         a.b1[j] = dec->b1[j];
     }
     a.run_totals = nullptr;
+    a.run_tiles = nullptr;
     a.run_base = nullptr;
     a.neural_opacity = nullptr;
     a.kept_mask = nullptr;
@@ -833,47 +914,35 @@ int launch_run_scan(const uint2* totals, uint2* base, uint32_t runs, uint32_t* n
     return GS355_OK;
 }
 
-// Persistent workgroups (4 wavefronts, each walking runs of kRun anchors): at most `cap` of them, about what
-// the chip holds at once, so the weight fragments are fetched once per resident workgroup.
-static dim3 decode_grid(int A, int cap, int waves = 4)
+static uint32_t run_count(int A) { return (uint32_t)(((size_t)A + kRun - 1) / kRun); }
+
+// Launch the count or the emit pass in the variant the features and the weights need.
+// Persistent workgroups, at most what the chip holds at once: the weights are fetched once per resident workgroup.
+static void launch_count(hipStream_t s, const DecodeArgs& a, uint32_t* counts)
 {
-    const int runs = (A + kRun - 1) / kRun;
-    int blocks = (runs + waves - 1) / waves;
-    if (blocks > cap) blocks = cap;
-    if (blocks < 1) blocks = 1;
-    return dim3(blocks);
+    const uint32_t runs = run_count(a.A);
+    const int shared_run = runs <= (uint32_t)kCountCap ? 1 : 0;
+    const dim3 grid(runs < (uint32_t)kCountCap ? runs : (uint32_t)kCountCap), block(64 * kCountWaves);
+#define GS355_COUNT(S, W) hipLaunchKernelGGL((decode_count_kernel<S, W>), grid, block, 0, s, a, counts, shared_run)
+    if (a.split_feat && a.weights_lo) GS355_COUNT(true, true);
+    else if (a.split_feat) GS355_COUNT(true, false);
+    else if (a.weights_lo) GS355_COUNT(false, true);
+    else GS355_COUNT(false, false);
+#undef GS355_COUNT
 }
 
-// Launch the count or the emit pass in the variant the features and the weights need.  `cap`: most workgroups.
-template <bool kCountOnly, bool kSplit, bool kWLo>
-static void launch_variant(int cap, hipStream_t s, const DecodeArgs& a, uint32_t* counts, const uint32_t* offsets,
-                           uint32_t capacity, float* xyz, float* color, float* opacity, float* scaling, float* rot)
+static void launch_emit(hipStream_t s, const DecodeArgs& a, const uint32_t* offsets, uint32_t capacity, const gs355_decoded& o)
 {
-    constexpr int kWaves = decode_waves(kCountOnly, kWLo);
-    hipLaunchKernelGGL((decode_kernel<kCountOnly, kSplit, kWLo>), decode_grid(a.A, cap, kWaves), dim3(64 * kWaves), 0, s, a,
-                       counts, offsets, capacity, xyz, color, opacity, scaling, rot);
-}
-
-static void launch_decode(bool count_only, int cap, hipStream_t s, const DecodeArgs& a, uint32_t* counts,
-                          const uint32_t* offsets, uint32_t capacity, const gs355_decoded* out)
-{
-    float* xyz = out ? out->xyz : nullptr;
-    float* color = out ? out->color : nullptr;
-    float* opacity = out ? out->opacity : nullptr;
-    float* scaling = out ? out->scaling : nullptr;
-    float* rot = out ? out->rot : nullptr;
-#define GS355_DECODE_CASE(C, S, W)                                                                             \
-    if (count_only == C && (a.split_feat != 0) == S && (a.weights_lo != 0) == W)                               \
-        launch_variant<C, S, W>(cap, s, a, counts, offsets, capacity, xyz, color, opacity, scaling, rot);
-    GS355_DECODE_CASE(true, false, false)
-    GS355_DECODE_CASE(true, false, true)
-    GS355_DECODE_CASE(true, true, false)
-    GS355_DECODE_CASE(true, true, true)
-    GS355_DECODE_CASE(false, false, false)
-    GS355_DECODE_CASE(false, false, true)
-    GS355_DECODE_CASE(false, true, false)
-    GS355_DECODE_CASE(false, true, true)
-#undef GS355_DECODE_CASE
+    const uint32_t runs = run_count(a.A);
+    const dim3 grid(runs < (uint32_t)kEmitCap ? runs : (uint32_t)kEmitCap), block(64 * kEmitWaves);
+#define GS355_EMIT(S, W)                                                                                              \
+    hipLaunchKernelGGL((decode_emit_kernel<S, W>), grid, block, 0, s, a, offsets, capacity, o.xyz, o.color, o.opacity, \
+                       o.scaling, o.rot)
+    if (a.split_feat && a.weights_lo) GS355_EMIT(true, true);
+    else if (a.split_feat) GS355_EMIT(true, false);
+    else if (a.weights_lo) GS355_EMIT(false, true);
+    else GS355_EMIT(false, false);
+#undef GS355_EMIT
 }
 
 }  // namespace gs355
@@ -934,7 +1003,7 @@ int gs355_decode_count(const gs355_decoder* dec, const gs355_anchors* an, uint32
     if (scratch_bytes < need)
         return set_error(GS355_ENOSPC, "decode scratch has %zu bytes, %zu needed", scratch_bytes, need);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    launch_decode(true, 1024, s, a, counts, nullptr, 0u, nullptr);
+    launch_count(s, a, counts);
     GS355_CHECK_LAUNCH("decode: count");
     return launch_exclusive_scan(counts, offsets, (size_t)a.A, static_cast<uint32_t*>(scratch_buf), s);
 }
@@ -956,7 +1025,7 @@ int gs355_decode_count_static(const gs355_decoder* dec, const gs355_anchors* an,
     uint32_t* tmp = nullptr;
     if ((rc = static_scratch(&tmp))) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    launch_decode(true, 1024, s, a, counts, nullptr, 0u, nullptr);
+    launch_count(s, a, counts);
     GS355_CHECK_LAUNCH("decode: count");
     // the scan writes every block sum before it reads it: nothing in the array has to start at zero
     return launch_exclusive_scan(counts, offsets, (size_t)a.A, tmp, s);
@@ -975,23 +1044,25 @@ int gs355_decode_emit(const gs355_decoder* dec, const gs355_anchors* an, const u
     if (!out || !out->xyz || !out->color || !out->opacity || !out->scaling || !out->rot)
         return set_error(GS355_EINVAL, "decoded outputs must all be non-NULL");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    launch_decode(false, 512, s, a, nullptr, offsets, (uint32_t)capacity, out);
+    launch_emit(s, a, offsets, (uint32_t)capacity, *out);
     GS355_CHECK_LAUNCH("decode: emit");
     return GS355_OK;
 }
 
 namespace {
 struct FusedLayout {
-    size_t run_totals, run_base, mixed, total;
+    size_t run_totals, run_tiles, run_base, mixed, total;
 };
 FusedLayout fused_layout(int32_t A, int32_t n, bool bank)
 {
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-    const size_t runs = ((size_t)A + kRun - 1) / kRun;
+    const size_t runs = run_count(A);
     FusedLayout L;
     size_t off = 0;
     (void)n;
     L.run_totals = off;
+    off = up(off + runs * sizeof(uint2) + 8);
+    L.run_tiles = off;
     off = up(off + runs * sizeof(uint2) + 8);
     L.run_base = off;
     off = up(off + runs * sizeof(uint2) + 8);
@@ -1042,9 +1113,11 @@ int gs355_decode(const gs355_decoder* dec, const gs355_anchors* an, int64_t capa
         return GS355_OK;
     }
     char* ws = static_cast<char*>(workspace);
-    const uint32_t runs = (uint32_t)(((size_t)a.A + kRun - 1) / kRun);
+    const uint32_t runs = run_count(a.A);
     if (bank) a.feat = reinterpret_cast<float*>(ws + L.mixed);  // written by the count phase, read by both passes
     uint2* run_base = reinterpret_cast<uint2*>(ws + L.run_base);
+    a.run_totals = reinterpret_cast<uint2*>(ws + L.run_totals);
+    a.run_tiles = reinterpret_cast<uint2*>(ws + L.run_tiles);
     if (do_count) {
         if (bank) {
             BankArgs b;
@@ -1063,18 +1136,16 @@ int gs355_decode(const gs355_decoder* dec, const gs355_anchors* an, int64_t capa
             hipLaunchKernelGGL(feature_bank_kernel, dim3((a.A + kBankAnchors - 1) / kBankAnchors), dim3(256), 0, s, b);
             GS355_CHECK_LAUNCH("decode: feature bank");
         }
-        a.run_totals = reinterpret_cast<uint2*>(ws + L.run_totals);
-        launch_decode(true, 1024, s, a, nullptr, nullptr, 0u, nullptr);
+        launch_count(s, a, nullptr);
         GS355_CHECK_LAUNCH("decode: count");
         if ((rc = launch_run_scan(a.run_totals, run_base, runs, out->count, out->num_visible, s))) return rc;
     }
     if (!do_emit) return GS355_OK;
     if (capacity == 0 && !out->neural_opacity && !out->mask) return GS355_OK;
-    a.run_totals = nullptr;
     a.run_base = run_base;
     a.neural_opacity = out->neural_opacity;
     a.kept_mask = out->mask;
-    launch_decode(false, 512, s, a, nullptr, nullptr, (uint32_t)capacity, out);
+    launch_emit(s, a, nullptr, (uint32_t)capacity, *out);
     GS355_CHECK_LAUNCH("decode: emit");
     return GS355_OK;
 }

@@ -335,20 +335,21 @@ def test_feature_bank_at_the_edges_of_its_tiles(gpu_device, A, frac):
     compare(got, redo(), redo)
 
 
-@pytest.mark.parametrize("A", [1_048_576, 1_048_577 + 128])
-def test_decode_runs_beyond_one_round_of_their_prefix(gpu_device, A):
-    """8192 runs of 128 anchors fill one round of the runs' prefix: visible anchors on both sides of that line give
-    the Gaussians that a decode of the visible anchors alone gives."""
+@pytest.mark.parametrize("A", [129, 32_768, 32_769, 131_072, 131_073, 1_048_576, 1_048_705, 2_097_153])
+def test_decode_of_few_visible_anchors_among_many(gpu_device, A):
+    """Around the sizes where the split of the work changes (a run of 128 anchors per workgroup of the emit pass and of
+    the count pass, one round of the runs' prefix, 64 runs per workgroup): a few visible anchors near the ends give the
+    Gaussians that a decode of those anchors alone gives."""
     sc = scenes.config5(A=A)
     dec = build_decoder(sc, gpu_device)
     vis = torch.zeros(A, dtype=torch.bool)
-    vis[1000:1040] = True
-    vis[A - 200:] = True
+    vis[10:50] = True
+    vis[max(50, A - 200):] = True
     cam = sc.camera.camera_center.to(gpu_device)
     t = [x.to(gpu_device) for x in (sc.anchor, sc.anchor_feat, sc.offset, sc.scaling)]
     got = dec(cam, *t, vis.to(gpu_device))
     few = [x[vis.to(gpu_device)].contiguous() for x in t]
-    want = dec(cam, *few, torch.ones(240, dtype=torch.bool, device=gpu_device))
+    want = dec(cam, *few, torch.ones(int(vis.sum()), dtype=torch.bool, device=gpu_device))
     assert want[0].shape[0] > 0
     for name, a, b in zip(("xyz", "color", "opacity", "scaling", "rot"), got[:5], want[:5]):
         assert torch.equal(a, b), name
