@@ -62,10 +62,11 @@ class DeviceDecode(NamedTuple):
     counts: torch.Tensor
     neural_opacity: Optional[torch.Tensor]
     mask: Optional[torch.Tensor]
+    first_count: Optional[torch.Tensor] = None
 
     @property
     def count(self) -> torch.Tensor:  # int32[1]: what the rasterizer takes as its device-side Gaussian count
-        return self.counts[0:1]
+        return self.counts[0:1] if self.first_count is None else self.first_count
 
 
 class _TallLinear(torch.autograd.Function):
@@ -297,7 +298,9 @@ class FusedAnchorDecoder(nn.Module):
         level = self._check_level(level, A)
         if visible_mask is None:
             visible_mask = torch.ones(A, dtype=torch.bool, device=dev)
-        vis = visible_mask.to(device=dev, dtype=torch.bool).contiguous()
+        vis = visible_mask
+        if vis.dtype is not torch.bool or vis.device != dev or not vis.is_contiguous():
+            vis = vis.to(device=dev, dtype=torch.bool).contiguous()
         an = _lib.Anchors()
         tensors = [_f32c(anchor, dev), _f32c(anchor_feat, dev), _f32c(offset, dev), _f32c(scaling, dev),
                    _f32c(camera_center, dev), vis]
@@ -341,36 +344,36 @@ class FusedAnchorDecoder(nn.Module):
         _lib.check(_lib.load().gs355_decode(C.byref(dec), C.byref(an), int(capacity), C.byref(o), ws.data_ptr(),
                                             ws.numel(), int(phases), _raw_stream(dev)))
 
-    @torch.no_grad()
     def decode_on_device(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask=None, level=None,
                          want_training_outputs: bool = False, reuse_buffers: bool = False) -> DeviceDecode:
         """The whole decode enqueued on the current stream, nothing read back.  Outputs have room for
         A * n_offsets Gaussians; `counts` says how many are valid.  `reuse_buffers`: the outputs live in one block
         the decoder keeps and overwrites at its next call (a render loop that consumes them at once pays no
-        per-frame allocation of the capacity-sized block)."""
+        per-frame allocation of the capacity-sized block).  Nothing here is differentiated."""
         dev, A, dec, an, tensors = self._marshal(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
         n = self.n_offsets
         cap = A * n
         # one block for the five outputs (14 floats per Gaussian) and the two counters, carved into views
         kept = self._kept(dev)
         if reuse_buffers and kept.get("block") is not None and kept["block"][0] == cap:
-            res = kept["block"][1]
+            _, res, o = kept["block"]
         else:
             block = torch.empty(cap * 14 + 2, dtype=torch.float32, device=dev)
             cut = lambda first, width: block[first * cap:(first + width) * cap].view(cap, width)  # noqa: E731
-            res = DeviceDecode(cut(0, 3), cut(3, 3), cut(6, 1), cut(7, 3), cut(10, 4), block[cap * 14:].view(torch.int32),
-                               None, None)
-            kept["block"] = (cap, res) if reuse_buffers else None
+            counts = block[cap * 14:].view(torch.int32)
+            res = DeviceDecode(cut(0, 3), cut(3, 3), cut(6, 1), cut(7, 3), cut(10, 4), counts, None, None, counts[0:1])
+            o = _lib.Decoded()
+            if cap > 0:
+                o.xyz, o.color, o.opacity = res.xyz.data_ptr(), res.color.data_ptr(), res.opacity.data_ptr()
+                o.scaling, o.rot = res.scaling.data_ptr(), res.rot.data_ptr()
+            o.count, o.num_visible = counts.data_ptr(), counts.data_ptr() + 4
+            kept["block"] = (cap, res, o) if reuse_buffers else None
         if want_training_outputs:
             res = res._replace(neural_opacity=torch.empty((cap, 1), dtype=torch.float32, device=dev),
                                mask=torch.empty(cap, dtype=torch.bool, device=dev))
-        o = _lib.Decoded()
-        if cap > 0:
-            o.xyz, o.color, o.opacity = res.xyz.data_ptr(), res.color.data_ptr(), res.opacity.data_ptr()
-            o.scaling, o.rot = res.scaling.data_ptr(), res.rot.data_ptr()
-            if want_training_outputs:
+            o = _lib.Decoded.from_buffer_copy(o)
+            if cap > 0:
                 o.neural_opacity, o.mask = res.neural_opacity.data_ptr(), res.mask.data_ptr()
-        o.count, o.num_visible = res.counts.data_ptr(), res.counts.data_ptr() + 4
         self._run(dec, an, cap, o, _lib.DECODE_ALL, dev)
         del tensors  # torch's allocator keeps their memory alive for the work already enqueued on this stream
         return res

@@ -499,16 +499,18 @@ class ScaffoldGS(nn.Module):
 
     def prefilter_voxel(self, viewpoint_camera, scaling_modifier=1.0):
         if self.fuse_prefilter and not self.training:
-            from . import pipeline
-            visible, mask = pipeline.anchor_filter(
-                _settings(viewpoint_camera, self.background, scaling_modifier, 1), self.get_anchor, self.get_scaling,
-                self.get_rotation, self._lod(viewpoint_camera))
+            camera, view = self.__dict__.pop("_view", (None, None))  # (left by the frame that asks, for these settings)
+            if camera is viewpoint_camera and scaling_modifier == view.settings.scale_modifier:
+                settings = view.settings
+            else:
+                settings, view = _settings(viewpoint_camera, self.background, scaling_modifier, 1), None
+            visible, mask = pipeline.anchor_filter(settings, self.get_anchor, self.get_scaling, self.get_rotation,
+                                                   self._lod(viewpoint_camera), view=view)
             if mask is not None:
                 self._anchor_mask = mask
             return visible
         subset = self._anchor_subset()
         if self.fuse_prefilter and subset is None and self._filters_parameters():
-            from . import pipeline
             return pipeline.anchor_filter(_settings(viewpoint_camera, self.background, scaling_modifier, 1), self._anchor,
                                           self._scaling, self._rotation, stored=True)[0]
         rasterizer = GaussianRasterizer(raster_settings=_settings(viewpoint_camera, self.background,
@@ -546,6 +548,8 @@ class ScaffoldGS(nn.Module):
         the same values come from the kernels)."""
         if self.training:
             return self._forward_training(viewpoint_camera, scaling_modifier, retain_grad, render_exclude_filter)
+        if not torch.is_grad_enabled():
+            return self._forward_frame(viewpoint_camera, scaling_modifier, render_exclude_filter)
         with torch.no_grad():
             return self._forward_frame(viewpoint_camera, scaling_modifier, render_exclude_filter)
 
@@ -574,27 +578,35 @@ class ScaffoldGS(nn.Module):
         return rendered_image, scaling
 
     def _forward_frame(self, viewpoint_camera, scaling_modifier=1.0, render_exclude_filter=None):
-        viewpoint_camera = viewpoint_camera.to(self._anchor.device)
+        d = self.__dict__  # (plain attributes, set past nn.Module's search for parameters, buffers and modules)
+        anchor = self._anchor
+        viewpoint_camera = viewpoint_camera.to(anchor.device)
+        fused = self.fuse_prefilter and not self.training
+        settings, view = _settings(viewpoint_camera, self.background, scaling_modifier, 1), None
+        if fused:
+            view = pipeline.FrameView(settings, anchor.device)
+            d["_view"] = (viewpoint_camera, view)
         self._before_prefilter(viewpoint_camera)
         voxel_visible_mask = self.prefilter_voxel(viewpoint_camera)
         if render_exclude_filter is not None:
             voxel_visible_mask = voxel_visible_mask & render_exclude_filter
-        self.renderer.raster_settings = _settings(viewpoint_camera, self.background, scaling_modifier, 1)
+        renderer = self.renderer
+        renderer.__dict__["raster_settings"] = settings
         decode = dict(camera_center=viewpoint_camera.camera_center, anchor=self.get_anchor,
                       anchor_feat=self.get_anchor_feat, offset=self.get_offset, scaling=self.get_scaling,
                       visible_mask=voxel_visible_mask, level=self._decoder_level())
-        if self.fuse_prefilter and not self.training:
+        if fused:
             # nothing is read back: the decode leaves the number of Gaussians on the device, the rasterizer takes it
             # from there and works over tensors sized for the most the anchors can emit
             res = self.anchor_decoder.decode_on_device(**decode, reuse_buffers=True)
-            rendered_image, radii, _ = self.renderer(
+            renderer.__dict__["_view"] = view
+            rendered_image, radii, _ = renderer(
                 means3D=res.xyz, means2D=None, shs=None, colors_precomp=res.color, opacities=res.opacity,
                 scales=res.scaling, rotations=res.rot, cov3D_precomp=None, count=res.count)
-            d = self.__dict__  # (plain attributes, set past nn.Module's search for parameters, buffers and modules)
             d["_visibility_filter"], d["_pending"], d["voxel_visible_mask"] = None, (res, radii), voxel_visible_mask
             return rendered_image
         xyz, color, opacity, scaling, rot, _, _ = self.anchor_decoder(**decode)
-        rendered_image, radii, _ = self.renderer(
+        rendered_image, radii, _ = renderer(
             means3D=xyz, means2D=None, shs=None, colors_precomp=color, opacities=opacity, scales=scaling,
             rotations=rot, cov3D_precomp=None)
         self.visibility_filter, self.voxel_visible_mask = radii > 0, voxel_visible_mask

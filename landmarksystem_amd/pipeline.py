@@ -135,17 +135,36 @@ def release_workspace(device: torch.device, stream=None) -> None:
     _workspaces.pop(_workspace_key(device, stream), None)
 
 
+class FrameView:
+    """The settings of a frame (size, camera, background) as the kernels read them.  A frame over decoded anchors
+    uses them three times and marshals them once."""
+
+    __slots__ = ("settings", "viewmatrix", "projmatrix", "campos", "bg", "frame")
+
+    def __init__(self, s, dev: torch.device, sh_coeffs: int = 0, colour: bool = True):
+        self.settings = s
+        self.viewmatrix = _dev_f32(s.viewmatrix, dev, "viewmatrix", (16,))
+        self.projmatrix = _dev_f32(s.projmatrix, dev, "projmatrix", (16,))
+        self.campos = _dev_f32(s.campos, dev, "campos", (3,))
+        self.bg = _dev_f32(s.bg, dev, "bg", (3,)) if colour else None
+        # (fields in the structure's order)
+        self.frame = _lib.Frame(int(s.image_width), int(s.image_height), float(s.tanfovx), float(s.tanfovy),
+                                float(s.scale_modifier), int(s.sh_degree), sh_coeffs, _ptr(self.viewmatrix),
+                                _ptr(self.projmatrix), _ptr(self.campos), _ptr(self.bg))
+
+
 class FrameInputs:
     """The tensors of one rasterizer call, validated and marshalled."""
 
     def __init__(self, settings, means3D, opacities=None, shs=None, colors_precomp=None, scales=None, rotations=None,
                  cov3D_precomp=None, need_colour: bool = True, count: Optional[torch.Tensor] = None,
-                 features_rest: Optional[torch.Tensor] = None):
+                 features_rest: Optional[torch.Tensor] = None, view: Optional[FrameView] = None):
         """`count`: optional one-element int32 tensor on the device holding the number of Gaussians (the anchor
         decode leaves it there); the tensors are then sized for a capacity and only the first `count` rows are
         rendered, without the host ever reading the number.
         `features_rest` ([P, M - 1, 3]): the tensors are the vanilla model's stored parameters (shs = features_dc
-        [P, 1, 3], scales = logarithms, rotations unnormalised, opacities = logits), activated by the kernels."""
+        [P, 1, 3], scales = logarithms, rotations unnormalised, opacities = logits), activated by the kernels.
+        `view`: these settings, already marshalled for a call without spherical harmonics."""
         if need_colour:
             if (shs is None and colors_precomp is None) or (shs is not None and colors_precomp is not None):
                 raise Exception("Please provide excatly one of either SHs or precomputed colors!")
@@ -181,17 +200,11 @@ class FrameInputs:
                 raise ValueError("features_rest must have shape [P, M - 1, 3], got %s" % (tuple(features_rest.shape),))
             sh_coeffs = 1 + int(self.features_rest.shape[1])
 
-        s = settings
-        self.width, self.height = int(s.image_width), int(s.image_height)
-        self.viewmatrix = _dev_f32(s.viewmatrix, dev, "viewmatrix", (16,))
-        self.projmatrix = _dev_f32(s.projmatrix, dev, "projmatrix", (16,))
-        self.campos = _dev_f32(s.campos, dev, "campos", (3,))
-        self.bg = _dev_f32(s.bg, dev, "bg", (3,))
-
-        # (fields in the structures' order)
-        self.frame = _lib.Frame(self.width, self.height, float(s.tanfovx), float(s.tanfovy), float(s.scale_modifier),
-                                int(s.sh_degree), sh_coeffs, _ptr(self.viewmatrix), _ptr(self.projmatrix),
-                                _ptr(self.campos), _ptr(self.bg))
+        if view is None or view.settings is not settings or sh_coeffs != 0:
+            view = FrameView(settings, dev, sh_coeffs)
+        self.frame, self.viewmatrix, self.projmatrix, self.campos, self.bg = (view.frame, view.viewmatrix, view.projmatrix,
+                                                                              view.campos, view.bg)
+        self.width, self.height = view.frame.image_width, view.frame.image_height
         g = _lib.Gaussians(P, _ptr(self.means3D), _ptr(self.shs), _ptr(self.colors_precomp), _ptr(self.opacities),
                            _ptr(self.scales), _ptr(self.rotations), _ptr(self.cov3D_precomp))
         self.count = None
@@ -217,7 +230,7 @@ def visible_filter(inputs: FrameInputs) -> torch.Tensor:
 
 
 def anchor_filter(settings, anchors: torch.Tensor, scaling: torch.Tensor, rotations: torch.Tensor, lod=None,
-                  stored: bool = False):
+                  stored: bool = False, view: Optional[FrameView] = None):
     """The anchor-level visibility prefilter of Scaffold-GS / Octree-GS in one kernel (gs355_anchor_filter).
 
     `scaling` is the models' f32[A,6] (or [A,3]); its first three columns are read in place.  `lod`: None, or a dict
@@ -232,10 +245,9 @@ def anchor_filter(settings, anchors: torch.Tensor, scaling: torch.Tensor, rotati
     if sc.dim() != 2 or sc.shape[0] != A or sc.shape[1] < 3:
         raise ValueError("scaling must have shape [A, >=3], got %s" % (tuple(sc.shape),))
     rot = _dev_f32(rotations, dev, "rotations", (A, 4))
-    keep = [_dev_f32(settings.viewmatrix, dev, "viewmatrix", (16,)), _dev_f32(settings.projmatrix, dev, "projmatrix", (16,)),
-            _dev_f32(settings.campos, dev, "campos", (3,))]
-    f = _lib.Frame(int(settings.image_width), int(settings.image_height), float(settings.tanfovx), float(settings.tanfovy),
-                   float(settings.scale_modifier), 0, 0, keep[0].data_ptr(), keep[1].data_ptr(), keep[2].data_ptr())
+    if view is None or view.settings is not settings:
+        view = FrameView(settings, dev, colour=False)
+    f, keep = view.frame, [view]
     g = _lib.Gaussians(A, _ptr(means), None, None, None, _ptr(sc), _ptr(rot))
     visible = torch.empty(A, dtype=torch.bool, device=dev)
     if stored:

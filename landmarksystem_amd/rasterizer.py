@@ -195,7 +195,7 @@ class GaussianRasterizer(nn.Module):
             return image, radii, depth
         inputs = pipeline.FrameInputs(self.raster_settings, means3D, opacities=opacities, shs=shs,
                                       colors_precomp=colors_precomp, scales=scales, rotations=rotations,
-                                      cov3D_precomp=cov3D_precomp, count=count)
+                                      cov3D_precomp=cov3D_precomp, count=count, view=self.__dict__.pop("_view", None))
         out = pipeline.render(inputs)
         self._keep(out.depth, out.alpha, out.num_keys)
         return out.image, out.radii, out.depth
