@@ -491,38 +491,67 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
     }
 }
 
-// Sixteen records side by side, three lanes each, three such rounds in flight; the first record is overwritten once all
-// of them have been read (its new value depends on every one).
+// Sixteen records side by side, three lanes each, three such rounds per step; the first record is overwritten once all
+// of them have been read (its new value depends on every one).  A wavefront takes eight Gaussians and requests the next
+// step, of the same Gaussian or the next, before it adds the current one: with one Gaussian a wavefront, every one of them
+// waited for its rectangle and then for its records, 47 us for 100k Gaussians of some 20 records each; now 35 (18 is what
+// reading them takes).
+constexpr int kSumPerWave = 8;
 __global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __restrict__ radii,
                                                         const uint64_t* __restrict__ rects,
                                                         const RecordSlots* __restrict__ slots, float* key_grads)
 {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (i >= P) return;
-    if (radii[i] <= 0) return;
+    const int lane = threadIdx.x & 63, i0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kSumPerWave;
+    const int i = min(i0 + (lane & (kSumPerWave - 1)), P - 1);
+    const int32_t radius = radii[i];
     const RecordRun run = record_run(slots[i], rects[i]);
-    const uint32_t n = run.n;
-    if (n <= kSerialRecords) return;  // (uniform over the wavefront)
+    uint32_t left = (uint32_t)__ballot(lane < kSumPerWave && i0 + lane < P && radius > 0 && run.n > kSerialRecords);
+    if (left == 0u) return;
     const int slot = lane / 3, part = lane % 3;
-    float4* rec = reinterpret_cast<float4*>(key_grads) + (size_t)run.first * (kKeyFloats / 4) + part;
-    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (slot < 16) {
-        for (uint32_t k0 = (uint32_t)slot; k0 < n; k0 += 48) {
-            float4 r[3];
+    float4* const all = reinterpret_cast<float4*>(key_grads) + part;
+    uint32_t first = 0, n = 0, k0 = 0;  // the current step: records k0 .. k0 + 47 of the n from `first`
+    auto next = [&](uint32_t& f, uint32_t& m) {
+        const int l = __builtin_ctz(left);
+        left &= left - 1u;
+        f = (uint32_t)__builtin_amdgcn_readlane((int)run.first, l);
+        m = (uint32_t)__builtin_amdgcn_readlane((int)run.n, l);
+    };
+    auto request = [&](uint32_t f, uint32_t m, uint32_t k, float4 r[3]) {
 #pragma unroll
-            for (int u = 0; u < 3; ++u) r[u] = rec[3 * (size_t)min(k0 + 16u * (uint32_t)u, n - 1)];
-#pragma unroll
-            for (int u = 0; u < 3; ++u)
-                if (k0 + 16u * (uint32_t)u < n) sum = add4(sum, r[u]);
+        for (int u = 0; u < 3; ++u)
+            r[u] = all[((size_t)f + min(k + (uint32_t)slot + 16u * (uint32_t)u, m - 1)) * (kKeyFloats / 4)];
+    };
+    next(first, n);
+    float4 r[3], sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    request(first, n, k0, r);
+    for (;;) {  // (uniform; ends with the last Gaussian's last step)
+        const bool last = k0 + 48u >= n;
+        const bool more = !last || left != 0u;
+        uint32_t first1 = first, n1 = n, k1 = k0 + 48u;
+        float4 r1[3] = {};
+        if (last && more) {
+            next(first1, n1);
+            k1 = 0;
         }
-    }
+        if (more) request(first1, n1, k1, r1);
 #pragma unroll
-    for (int d = 24; d >= 3; d >>= 1) {
-        const float4 other = make_float4(__shfl_down(sum.x, d, 64), __shfl_down(sum.y, d, 64), __shfl_down(sum.z, d, 64),
-                                         __shfl_down(sum.w, d, 64));
-        sum = add4(sum, other);  // (lanes past the last slot hold zeros; sums other than the first slot's are not used)
+        for (int u = 0; u < 3; ++u)
+            if (slot < 16 && k0 + (uint32_t)slot + 16u * (uint32_t)u < n) sum = add4(sum, r[u]);
+        if (last) {
+#pragma unroll
+            for (int d = 24; d >= 3; d >>= 1) {
+                const float4 other = make_float4(__shfl_down(sum.x, d, 64), __shfl_down(sum.y, d, 64),
+                                                 __shfl_down(sum.z, d, 64), __shfl_down(sum.w, d, 64));
+                sum = add4(sum, other);  // (lanes past the last slot hold zeros; sums other than the first slot's are not used)
+            }
+            if (slot == 0) all[(size_t)first * (kKeyFloats / 4)] = sum;
+            sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        if (!more) break;
+        first = first1, n = n1, k0 = k1;
+#pragma unroll
+        for (int u = 0; u < 3; ++u) r[u] = r1[u];
     }
-    if (slot == 0) rec[0] = sum;
 }
 
 // kMode 0: SH blocks (if any) are read and written by their own lanes.  1 and 2: 16-coefficient blocks, 16-byte
@@ -941,8 +970,8 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     const dim3 grid((g.P + 255) / 256), block(256);
     const bool summed = g.P <= kSumAheadMax;
     if (summed) {
-        hipLaunchKernelGGL(sum_large_kernel, dim3((g.P + 3) / 4), dim3(256), 0, s, g.P, in.radii, rects, slots,
-                           key_grads);
+        hipLaunchKernelGGL(sum_large_kernel, dim3((g.P + 4 * kSumPerWave - 1) / (4 * kSumPerWave)), dim3(256), 0, s, g.P,
+                           in.radii, rects, slots, key_grads);
         GS355_CHECK_LAUNCH("record sums");
     }
     auto launch = [&](auto kernel, const ParameterArgs& p) {
