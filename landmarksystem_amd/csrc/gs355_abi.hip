@@ -218,8 +218,9 @@ int gs355_workspace_layout(int32_t P, int64_t n_cap, int32_t width, int32_t heig
     return make_layout(P, n_cap, width, height, out);
 }
 
-static int run_stages(const gs355_frame* frame, const gs355_gaussians* g, const ParameterArgs* par, void* workspace,
-                      size_t workspace_bytes, int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
+// Everything that can be wrong with a call that runs the stages `stage_mask`; leaves the workspace's layout in `layout`.
+static int check_stages(const gs355_frame* frame, const gs355_gaussians* g, const ParameterArgs* par, const void* workspace,
+                        size_t workspace_bytes, int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, gs355_layout* layout)
 {
     int rc;
     if ((stage_mask & ~kKnownStages) != 0 || (stage_mask & ~kStageModifiers) == 0 ||
@@ -233,8 +234,7 @@ static int run_stages(const gs355_frame* frame, const gs355_gaussians* g, const 
     if ((stage_mask & GS355_STAGE_PREPROCESS) && g->P > 0 && !out->radii)
         return set_error(GS355_EINVAL, "outputs.radii is NULL");
     if ((stage_mask & (GS355_STAGE_BLEND | GS355_STAGE_BLEND_PLAIN)) && !out->image) return set_error(GS355_EINVAL, "outputs.image is NULL");
-    gs355_layout L;
-    if ((rc = make_layout(g->P, n_cap, frame->image_width, frame->image_height, &L))) return rc;
+    if ((rc = make_layout(g->P, n_cap, frame->image_width, frame->image_height, layout))) return rc;
     if (stage_mask & (GS355_STAGE_TILE_COUNT | GS355_STAGE_TILE_SCATTER | GS355_STAGE_TILESORT)) {
         if ((int64_t)((frame->image_width + kTile - 1) / kTile) * ((frame->image_height + kTile - 1) / kTile) > kBinMaxTilesWide)
             return set_error(GS355_EINVAL, "the tile-bucketed stages support at most %d tiles; use the classic stages",
@@ -246,10 +246,17 @@ static int run_stages(const gs355_frame* frame, const gs355_gaussians* g, const 
     if (!workspace) return set_error(GS355_EINVAL, "workspace is NULL");
     if ((reinterpret_cast<uintptr_t>(workspace) & (kAlign - 1)) != 0)
         return set_error(GS355_EINVAL, "workspace must be 256-byte aligned");
-    if (workspace_bytes < L.total_bytes)
+    if (workspace_bytes < layout->total_bytes)
         return set_error(GS355_ENOSPC, "workspace has %zu bytes, %zu needed (P=%d, n_cap=%lld, %dx%d)", workspace_bytes,
-                         L.total_bytes, g->P, (long long)n_cap, frame->image_width, frame->image_height);
+                         layout->total_bytes, g->P, (long long)n_cap, frame->image_width, frame->image_height);
+    return GS355_OK;
+}
 
+// The stages of a call that check_stages accepted.
+static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, const ParameterArgs* par, void* workspace,
+                          const gs355_layout& L, int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
+{
+    int rc;
     char* ws = static_cast<char*>(workspace);
     auto* header = reinterpret_cast<gs355_header*>(ws + L.header);
     auto* records = reinterpret_cast<float*>(ws + L.records);
@@ -318,6 +325,14 @@ static int run_stages(const gs355_frame* frame, const gs355_gaussians* g, const 
     return GS355_OK;
 }
 
+static int run_stages(const gs355_frame* frame, const gs355_gaussians* g, const ParameterArgs* par, void* workspace,
+                      size_t workspace_bytes, int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
+{
+    gs355_layout L;
+    const int rc = check_stages(frame, g, par, workspace, workspace_bytes, n_cap, out, stage_mask, &L);
+    return rc ? rc : enqueue_stages(frame, g, par, workspace, L, n_cap, out, stage_mask, stream);
+}
+
 int gs355_run(const gs355_frame* frame, const gs355_gaussians* g, void* workspace, size_t workspace_bytes,
               int64_t n_cap, const gs355_outputs* out, uint32_t stage_mask, void* stream)
 {
@@ -345,14 +360,22 @@ int gs355_render_frame(const gs355_frame* frame, const gs355_gaussians* g, int32
     ParameterArgs par;
     par.rest = features_rest;
     const ParameterArgs* p = stored_parameters ? &par : nullptr;
+    // Both halves are checked before the first one is enqueued: from then on a store to the header is on its way, and a call
+    // that returned ahead of it would have it land in the next call's header, which would pass for that frame's.
+    gs355_layout L;
+    int rc = check_stages(frame, g, p, workspace, workspace_bytes, n_cap, out, stage_mask, &L);
+    if (rc) return rc;
     gs355_outputs later = *out;
     later.header_copy = nullptr;
     volatile gs355_header* header = static_cast<volatile gs355_header*>(out->header_copy);
     header->ready = 0u;
     __atomic_thread_fence(__ATOMIC_SEQ_CST);
-    int rc = run_stages(frame, g, p, workspace, workspace_bytes, n_cap, out, stage_mask & kFront, stream);
-    if (!rc) rc = run_stages(frame, g, p, workspace, workspace_bytes, n_cap, &later, stage_mask & ~kFront, stream);
-    if (rc) return rc;
+    rc = enqueue_stages(frame, g, p, workspace, L, n_cap, out, stage_mask & kFront, stream);
+    if (!rc) rc = enqueue_stages(frame, g, p, workspace, L, n_cap, &later, stage_mask & ~kFront, stream);
+    if (rc) {  // (a launch failed: what was enqueued before it ends first, for the same reason)
+        (void)hipStreamSynchronize(static_cast<hipStream_t>(stream));
+        return rc;
+    }
     return wait_for_header(header, static_cast<hipStream_t>(stream));
 }
 

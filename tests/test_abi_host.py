@@ -65,8 +65,8 @@ def test_workspace_layout_is_aligned_ordered_and_sized():
     assert L0.total_bytes > 0
 
 
-def _err(code_expected, fn, *args):
-    rc = fn(*args)
+def _err(code_expected, fn, *args, **kw):
+    rc = fn(*args, **kw)
     assert rc == code_expected, (rc, _lib.load().gs355_last_error())
     return _lib.load().gs355_last_error().decode()
 
@@ -153,6 +153,48 @@ def test_run_validates_before_any_hip_call():
     no_radii = _lib.Outputs()
     no_radii.image = 0x1000
     assert "radii is NULL" in _err(_lib.GS355_EINVAL, run, f, g, 0x1000, 1 << 30, 100, no_radii, _lib.STAGE_ALL)
+
+
+def test_render_frame_checks_everything_before_it_enqueues():
+    """What the later stages need is checked with the rest: an error behind the first launch would leave a store to the
+    header on its way, and the next call on the header would take it for its own.  (The header shows that nothing began.)"""
+    lib = _lib.load()
+    header = _lib.Header()
+    frame, g = _frame(), _gauss()
+    whole = _lib.PIPELINE_FAST
+
+    def outputs(**kw):
+        o = _lib.Outputs()
+        o.image = o.radii = 0x1000
+        o.header_copy = C.addressof(header)
+        for k, v in kw.items():
+            setattr(o, k, v)
+        return o
+
+    def call(o, mask=whole, g=g, stored=0, rest=None, nbytes=1 << 30, ws=0x1000):
+        header.ready = 7
+        rc = lib.gs355_render_frame(C.byref(frame), C.byref(g), stored, rest, ws, nbytes, 100, C.byref(o) if o else None, mask,
+                                    None)
+        assert header.ready == 7
+        return rc
+
+    assert "outputs is NULL" in _err(_lib.GS355_EINVAL, call, None)
+    assert "header_copy" in _err(_lib.GS355_EINVAL, call, outputs(header_copy=None))
+    assert "not a frame" in _err(_lib.GS355_EINVAL, call, outputs(), _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_COUNT)
+    assert "not a frame" in _err(_lib.GS355_EINVAL, call, outputs(), _lib.STAGE_PREPROCESS | _lib.STAGE_BLEND)
+    assert "stage_mask" in _err(_lib.GS355_EINVAL, call, outputs(), whole | 32768)
+    assert "stage_mask" in _err(_lib.GS355_EINVAL, call, outputs(),
+                                whole | _lib.STAGE_TILE_SCATTER_ONE_LEVEL | _lib.STAGE_TILE_SCATTER_TWO_LEVEL)
+    assert "image is NULL" in _err(_lib.GS355_EINVAL, call, outputs(image=None))
+    assert "radii is NULL" in _err(_lib.GS355_EINVAL, call, outputs(radii=None))
+    assert "workspace is NULL" in _err(_lib.GS355_EINVAL, call, outputs(), ws=None)
+    assert "bytes" in _err(_lib.GS355_ENOSPC, call, outputs(), nbytes=256)
+    # stored parameters: SH coefficients, scales and rotations, and a count that the host knows
+    assert "SH coefficients" in _err(_lib.GS355_EINVAL, call, outputs(), g=_gauss(shs=False, colors=True), stored=1)
+    assert "SH coefficients" in _err(_lib.GS355_EINVAL, call, outputs(), g=_gauss(sr=False, cov=True), stored=1)
+    on_device = _gauss()
+    on_device.P_device = 0x1000
+    assert "device-side" in _err(_lib.GS355_EINVAL, call, outputs(), g=on_device, stored=1)
 
 
 def test_render_backward_validates_before_any_hip_call():
