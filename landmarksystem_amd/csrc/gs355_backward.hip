@@ -19,6 +19,8 @@
 //                    mean; pixel position -> mean; colour -> SH coefficients and view direction -> mean.
 // min(0.99, opacity * G) passes the gradient unchanged, and the `means2D` gradient is in normalised device units
 // (pixel gradient times W/2, H/2), as the published backward pass of this rasterizer family does.
+#include <type_traits>
+
 #include "gs355_internal.h"
 
 namespace gs355 {
@@ -178,6 +180,7 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
         if (g_alpha) R -= (1.0f - out_alpha[o]) * g_alpha[o];
     }
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    const bool finite_g = __ballot(!(fabsf(g0) + fabsf(g1) + fabsf(g2) + fabsf(g3) < __builtin_inff())) == 0ull;
     // 1 in the lanes of a constant mask (one instruction, and no register held for it)
     auto ones = [](uint64_t lanes) { return __builtin_amdgcn_inverse_ballot_w64(lanes) ? 1.0f : 0.0f; };
     // staging: thread 4 k + part brings part `part` of the batch's Gaussian k (part 3: the slot of its record), and later
@@ -291,17 +294,34 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
                         D = __builtin_amdgcn_mfma_f32_4x4x1f32(d[s], one_hot, D, 0, 0, 0);
                         W = __builtin_amdgcn_mfma_f32_4x4x1f32(w[s], one_hot, W, 0, 0, 0);
                     }
+                    float m = (D[0] + D[1]) + (D[2] + D[3]);  // sum d
+                    // A d that is not finite times the zeros of the one-hot row is NaN in the quad's other columns, which
+                    // are other Gaussians, and every column's sum shows it: then the values change lanes by themselves.
+                    if (__ballot(!(fabsf(m) < __builtin_inff())) != 0ull) {
+                        auto from_lane = [&](auto lane) {  // (value by value: all sixteen at once cost a wavefront per SIMD)
+                            const float v[4] = {quad_lane<lane.value>(d[0]), quad_lane<lane.value>(d[1]),
+                                                quad_lane<lane.value>(d[2]), quad_lane<lane.value>(d[3])};
+                            return sub < 2 ? (sub == 0 ? v[0] : v[1]) : (sub == 2 ? v[2] : v[3]);
+                        };
+                        D[0] = from_lane(std::integral_constant<int, 0>{});
+                        D[1] = from_lane(std::integral_constant<int, 1>{});
+                        D[2] = from_lane(std::integral_constant<int, 2>{});
+                        D[3] = from_lane(std::integral_constant<int, 3>{});
+                        m = (D[0] + D[1]) + (D[2] + D[3]);
+                    }
                     const uint32_t k = (entries >> (8 * sub)) & 0xFFu;  // the column's entry
                     const float2 at = *reinterpret_cast<const float2*>(&s_a[k]);
                     const float ax = at.x - (pxf - (float)sub), dy = at.y - pyf;  // from the row's first pixel
                     const float ax1 = ax - 1.0f, ax2 = ax - 2.0f, ax3 = ax - 3.0f;
                     const float u0 = D[0] * ax, u1 = D[1] * ax1, u2 = D[2] * ax2, u3 = D[3] * ax3;
-                    const float m = (D[0] + D[1]) + (D[2] + D[3]);                    // sum d
                     const float mx = (u0 + u1) + (u2 + u3);                           // sum d dx
                     const float mxx = __builtin_fmaf(u3, ax3, __builtin_fmaf(u2, ax2, __builtin_fmaf(u1, ax1, u0 * ax)));
                     const float my = dy * m, myy = dy * my, mxy = dy * mx;
                     auto against = [&](float g) {  // the row's w against one channel of its pixels' gradients
-                        const f32x4 G = __builtin_amdgcn_mfma_f32_4x4x1f32(g, 1.0f, zero4, 0, 0, 0);
+                        f32x4 G = __builtin_amdgcn_mfma_f32_4x4x1f32(g, 1.0f, zero4, 0, 0, 0);
+                        if (!finite_g)  // (a pixel that rejected the Gaussian, w = 0, keeps its gradient to itself)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) G[i] = W[i] != 0.0f ? G[i] : 0.0f;
                         return __builtin_fmaf(W[3], G[3], __builtin_fmaf(W[2], G[2], __builtin_fmaf(W[1], G[1], W[0] * G[0])));
                     };
                     const float red = against(g0), green = against(g1), blue = against(g2);

@@ -304,3 +304,41 @@ def test_gradient_descent_through_the_model_fits_a_target(gpu_device):
         losses.append(float(loss.detach()))
     assert losses[-1] < 0.5 * losses[0], (losses[0], losses[-1])
     assert all(np.isfinite(losses))
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("where", ["colour", "cotangent"])
+def test_values_that_are_not_finite_reach_the_gaussians_of_their_pixels_only(gpu_device, where, value):
+    """A colour or a pixel's cotangent that is not finite: the gradients that the pixels concerned feed are not finite, all
+    others are the same bits as without it (four list entries share the reduction over a block's pixels)."""
+    scene = scenes.tiny_scene(P=400, width=133, height=75, sh_degree=0, seed=3)
+    colours = torch.rand(400, 3, generator=torch.Generator().manual_seed(0))
+    gi, gd, ga = cotangents(scene, 4)
+
+    def grads(colours, gi, gd=gd, ga=ga):
+        got, out = abi_backward(scene, gpu_device, gi, gd, ga, colors=colours)
+        return got, out.image.cpu()
+
+    want, image = grads(colours, gi)
+    bad_colours, bad_gi = colours.clone(), gi.clone()
+    if where == "colour":
+        bad_colours[17] = 2.0
+        touched = (grads(bad_colours, gi)[1] != image).any(dim=0)
+        bad_colours[17] = value
+    else:
+        touched = torch.zeros(75, 133, dtype=torch.bool)
+        touched[41, 70] = True
+        bad_gi[:, 41, 70] = value
+    assert 0 < int(touched.sum()) < touched.numel() // 2
+    # the Gaussians that blend in those pixels: the weights are positive, so a cotangent of ones leaves no gradient zero
+    zero = torch.zeros_like(gd)
+    there, _ = grads(colours, touched.float().expand(3, -1, -1).contiguous(), zero, zero)
+    concerned = there["colors_precomp"].any(axis=1)
+    assert 0 < concerned.sum() < 200
+    got, _ = grads(bad_colours, bad_gi)
+    for name in ("opacities", "means3D", "means2D", "scales") + (("colors_precomp",) if where == "cotangent" else ()):
+        finite = np.isfinite(got[name].reshape(400, -1))
+        assert not finite[concerned].all(axis=1).any(), name
+        assert finite[~concerned].all(), name
+    for name, value in got.items():
+        assert np.array_equal(value.reshape(400, -1)[~concerned], want[name].reshape(400, -1)[~concerned]), name
