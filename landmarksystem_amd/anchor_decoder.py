@@ -102,43 +102,75 @@ class _TallLinear(torch.autograd.Function):
         return dx, dw, db
 
 
+def _train_records(decoder, camera_center, visible, level, anchor, feat, offset, scaling, params):
+    """The gs355_decoder and gs355_anchors records of a training decode: pointers into these tensors."""
+    d = _lib.Decoder()
+    d.feat_dim, d.n_offsets = decoder.feat_dim, decoder.n_offsets
+    for j in range(3):
+        w0, b0, w1, b1 = params[4 * j:4 * j + 4]
+        d.in_dim[j] = w0.shape[1]
+        d.w0[j], d.b0[j], d.w1[j], d.b1[j] = w0.data_ptr(), b0.data_ptr(), w1.data_ptr(), b1.data_ptr()
+    d.add_level = 1 if decoder.add_level else 0
+    an = _lib.Anchors()
+    an.A = anchor.shape[0]
+    an.anchor, an.feat, an.offset, an.scaling = (t.data_ptr() for t in (anchor, feat, offset, scaling))
+    an.campos, an.visible_mask = camera_center.data_ptr(), visible.data_ptr()
+    an.level = None if level is None else level.data_ptr()
+    return d, an
+
+
+class _TrainBlock:
+    """Where things lie in the block that a training decode keeps for its backward pass: the kernels' workspace, the input
+    rows with and without the distance, hidden units and pre-activations of the three heads; every part 256-byte aligned.
+    `room`: the most rows (visible anchors) that fit."""
+
+    def __init__(self, A, room, n, widths, compact_feat):
+        need, scratch = C.c_size_t(), C.c_size_t()
+        _lib.check(_lib.load().gs355_decode_train_bytes(A, 0, n, C.byref(need), C.byref(scratch)))
+        sizes = [need.value, room * 36 * 4 if 36 in widths else 0, room * 35 * 4 if 35 in widths else 0]
+        sizes += [room * 32 * 4] * 3 + [room * n * k * 4 for k in (1, 7, 3)]
+        self.workspace_bytes, self.room, self.sizes, self.compact_feat = need.value, room, sizes, compact_feat
+        self.offsets, self.total = [], 0
+        for size in sizes:
+            self.offsets.append(self.total)
+            self.total += (size + 255) // 256 * 256
+
+    def rows(self, block, num_visible):
+        """The gs355_train_rows record of the block's parts, and the workspace's address."""
+        at = [block.data_ptr() + o for o in self.offsets]
+        rows = _lib.TrainRows(num_visible, 1 if self.compact_feat else 0, at[1] if self.sizes[1] else None,
+                              at[2] if self.sizes[2] else None)
+        for j in range(3):
+            rows.hidden[j], rows.pre[j] = at[3 + j], at[6 + j]
+        return rows, at[0]
+
+
 class _DecodeTrain(torch.autograd.Function):
     """The training decode (gs355_decode_train) with its whole backward pass in the kernels
     (gs355_decode_train_backward): differentiable with respect to anchors, features, offsets, scales and the heads'
     parameters.  Workspace, input rows, hidden units and pre-activations (968 bytes per anchor) live until the graph is
-    dropped."""
+    dropped.  Everything that the backward pass reads goes through save_for_backward and its pointers are taken there:
+    saved-tensor hooks (save_on_cpu, checkpointing) hand back other tensors than they were given."""
 
     @staticmethod
     def forward(ctx, decoder, camera_center, visible, level, compact_feat, anchor, feat, offset, scaling, *params):
         dev, A, n = anchor.device, anchor.shape[0], decoder.n_offsets
         lib = _lib.load()
         stream = _raw_stream(dev)
-        dec, an = decoder._train_structs(camera_center, visible, level, anchor, feat, offset, scaling, params)
-        need, scratch = C.c_size_t(), C.c_size_t()
-        _lib.check(lib.gs355_decode_train_bytes(A, 0, n, C.byref(need), C.byref(scratch)))
+        dec, an = _train_records(decoder, camera_center, visible, level, anchor, feat, offset, scaling, params)
         f = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)  # noqa: E731
         if decoder._host_count is None:
             decoder._host_count = torch.zeros(2, dtype=torch.int32, pin_memory=True)
         counts = decoder._host_count  # (pinned: the kernels' stores land there, nothing is copied)
-        # one block: workspace, then the rows with and without distance, hidden units and pre-activations, room for every
-        # anchor (how many are visible is only known on the device); every part 256-byte aligned
-        widths = {params[4 * j].shape[1] for j in range(3)}
-        sizes = [need.value, A * 36 * 4 if 36 in widths else 0, A * 35 * 4 if 35 in widths else 0]
-        sizes += [A * 32 * 4] * 3 + [A * n * k * 4 for k in (1, 7, 3)]
-        offsets, total = [], 0
-        for size in sizes:
-            offsets.append(total)
-            total += (size + 255) // 256 * 256
-        block = torch.empty(total, dtype=torch.uint8, device=dev)
-        at = [block.data_ptr() + o for o in offsets]
-        rows = _lib.TrainRows(A, 1 if compact_feat else 0, at[1] if sizes[1] else None, at[2] if sizes[2] else None)
-        for j in range(3):
-            rows.hidden[j], rows.pre[j] = at[3 + j], at[6 + j]
+        # room for every anchor: how many are visible is only known on the device
+        parts = _TrainBlock(A, A, n, {params[4 * j].shape[1] for j in range(3)}, compact_feat)
+        block = torch.empty(parts.total, dtype=torch.uint8, device=dev)
+        rows, workspace = parts.rows(block, parts.room)
         o = _lib.Decoded()
         o.num_visible = counts.data_ptr() + 4
         o.count = counts.data_ptr()
-        _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), 0, C.byref(o), at[0], need.value,
-                                          _lib.TRAIN_HEADS, stream))
+        _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), 0, C.byref(o), workspace,
+                                          parts.workspace_bytes, _lib.TRAIN_HEADS, stream))
         torch.cuda.current_stream(dev).synchronize()
         G, V = counts.tolist()
         rows.num_visible = V
@@ -146,11 +178,15 @@ class _DecodeTrain(torch.autograd.Function):
         if G > 0:
             o.xyz, o.color, o.opacity, o.scaling, o.rot = (t.data_ptr() for t in out[:5])
         o.neural_opacity, o.mask = out[5].data_ptr(), out[6].data_ptr()
-        _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), G, C.byref(o), at[0], need.value,
-                                          _lib.TRAIN_EMIT, stream))
-        ctx.structs = (dec, an, rows, at[0], need.value)  # (pointers into the saved tensors and the block)
-        ctx.block, ctx.n_offsets = block, n
-        ctx.save_for_backward(camera_center, visible, level, anchor, feat, offset, scaling, *params)
+        _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), G, C.byref(o), workspace,
+                                          parts.workspace_bytes, _lib.TRAIN_EMIT, stream))
+        # Camera, mask and level are not differentiated, and what a caller does to them after this is nothing to the
+        # gradients: the camera is copied, the kernels read neither mask nor level going back.
+        ctx.decoder, ctx.parts, ctx.num_visible = decoder, parts, V
+        ctx.visible, ctx.level = visible, level
+        saved = (camera_center.clone(), block, anchor, feat, offset, scaling, *params)
+        ctx.save_for_backward(*saved)
+        ctx.kinds = [(t.shape, t.dtype, t.device) for t in saved]
         ctx.mark_non_differentiable(out[6])
         ctx.set_materialize_grads(False)
         return out
@@ -158,8 +194,17 @@ class _DecodeTrain(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural, _g_mask):
-        _camera_center, _visible, _level, anchor, feat, offset, scaling, *params = ctx.saved_tensors
-        dec, an, rows, workspace, workspace_bytes = ctx.structs
+        saved = ctx.saved_tensors
+        if [(t.shape, t.dtype, t.device) for t in saved] != ctx.kinds:
+            raise RuntimeError("a tensor that the decode's backward pass reads has another shape, type or device than in its "
+                               "forward pass (its .data was replaced in between, or a saved-tensor hook changed it)")
+        saved = [t.contiguous() for t in saved]
+        # (kernels read 16 bytes at a time, the block's parts are laid out from 256-byte boundaries)
+        camera_center, block, anchor, feat, offset, scaling, *params = [t if t.data_ptr() % 256 == 0 or k not in (1, 3)
+                                                                        else t.clone() for k, t in enumerate(saved)]
+        parts = ctx.parts
+        dec, an = _train_records(ctx.decoder, camera_center, ctx.visible, ctx.level, anchor, feat, offset, scaling, params)
+        rows, workspace = parts.rows(block, ctx.num_visible)
         dev, A, V = anchor.device, anchor.shape[0], rows.num_visible
         lib = _lib.load()
         ptr = lambda t: None if t is None or t.numel() == 0 else t.data_ptr()  # noqa: E731
@@ -174,11 +219,11 @@ class _DecodeTrain(torch.autograd.Function):
         for j in range(3):
             out.w0[j], out.b0[j], out.w1[j], out.b1[j] = (ptr(t) for t in grads[4 + 4 * j:8 + 4 * j])
         need, scratch_bytes = C.c_size_t(), C.c_size_t()
-        _lib.check(lib.gs355_decode_train_bytes(A, V, ctx.n_offsets, C.byref(need), C.byref(scratch_bytes)))
+        _lib.check(lib.gs355_decode_train_bytes(A, V, ctx.decoder.n_offsets, C.byref(need), C.byref(scratch_bytes)))
         scratch = torch.empty(scratch_bytes.value // 4, dtype=torch.float32, device=dev)
-        _lib.check(lib.gs355_decode_train_backward(C.byref(dec), C.byref(an), C.byref(rows), workspace, workspace_bytes,
-                                                   C.byref(cot), C.byref(out), scratch.data_ptr(), scratch.numel() * 4,
-                                                   _raw_stream(dev)))
+        _lib.check(lib.gs355_decode_train_backward(C.byref(dec), C.byref(an), C.byref(rows), workspace,
+                                                   parts.workspace_bytes, C.byref(cot), C.byref(out), scratch.data_ptr(),
+                                                   scratch.numel() * 4, _raw_stream(dev)))
         return (None, None, None, None, None, *grads)
 
 
@@ -400,21 +445,6 @@ class FusedAnchorDecoder(nn.Module):
 
     def _head_parameters(self):
         return self._parameters_of(("mlp_opacity", "mlp_cov", "mlp_color"))
-
-    def _train_structs(self, camera_center, visible, level, anchor, feat, offset, scaling, params):
-        d = _lib.Decoder()
-        d.feat_dim, d.n_offsets = self.feat_dim, self.n_offsets
-        for j in range(3):
-            w0, b0, w1, b1 = params[4 * j:4 * j + 4]
-            d.in_dim[j] = w0.shape[1]
-            d.w0[j], d.b0[j], d.w1[j], d.b1[j] = w0.data_ptr(), b0.data_ptr(), w1.data_ptr(), b1.data_ptr()
-        d.add_level = 1 if self.add_level else 0
-        an = _lib.Anchors()
-        an.A = anchor.shape[0]
-        an.anchor, an.feat, an.offset, an.scaling = (t.data_ptr() for t in (anchor, feat, offset, scaling))
-        an.campos, an.visible_mask = camera_center.data_ptr(), visible.data_ptr()
-        an.level = None if level is None else level.data_ptr()
-        return d, an
 
     def _bank_mix(self, feat, view, level):
         """The feature bank (anchor_decoder.py:163-177): a softmax-weighted mix of strided copies of the features."""

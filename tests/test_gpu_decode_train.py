@@ -4,6 +4,7 @@ import copy
 
 import pytest
 import torch
+import torch.utils.checkpoint
 
 from landmarksystem_amd.anchor_decoder import FusedAnchorDecoder
 
@@ -72,3 +73,40 @@ def test_decode_and_gradients(gpu_device, A, n, visible, dist, level, bank):
         _close(a.grad, b.grad, name)
     for (name, a), b in zip(dec.named_parameters(), ref_dec.parameters()):
         _close(a.grad, b.grad, name)
+
+
+@pytest.mark.parametrize("how", ["save_on_cpu", "checkpoint"])
+@pytest.mark.parametrize("bank", [False, True])
+def test_gradients_under_saved_tensor_hooks(gpu_device, how, bank):
+    """Tensors that live elsewhere by the time of the backward pass (scales and camera are temporaries here): the same
+    gradients, bit for bit."""
+    g = torch.Generator().manual_seed(5)
+    dec = FusedAnchorDecoder(use_feat_bank=bank, add_opacity_dist=True, add_cov_dist=True, add_color_dist=True, view_dim=3,
+                             feat_dim=32, n_offsets=10).to(gpu_device).train()
+    cam = torch.tensor([0.3, -4.0, 2.0])
+    vis = (torch.rand(500, generator=g) < 0.7).to(gpu_device)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (
+        torch.randn(500, 3, generator=g) * 3, torch.randn(500, 32, generator=g), torch.randn(500, 10, 3, generator=g) * 0.1,
+        torch.randn(500, 6, generator=g) - 1)]
+
+    def decode(*t):
+        return dec(cam.to(gpu_device), t[0], t[1], t[2], torch.exp(t[3]), vis)[:6]
+
+    def gradients(run):
+        for p in leaves + list(dec.parameters()):
+            p.grad = None
+        out = run()
+        filler = [torch.full((500, 6), float("nan"), device=gpu_device) for _ in range(20)]  # takes what was freed
+        sum(t.square().sum() for t in out).backward()
+        del filler
+        return [p.grad.clone() for p in leaves + list(dec.parameters())]
+
+    def hooked():
+        if how == "checkpoint":
+            return torch.utils.checkpoint.checkpoint(decode, *leaves, use_reentrant=False)
+        with torch.autograd.graph.save_on_cpu():
+            return decode(*leaves)
+
+    want = gradients(lambda: decode(*leaves))
+    for a, b in zip(gradients(hooked), want):
+        assert torch.equal(a, b)
