@@ -199,9 +199,9 @@ class _DecodeTrain(torch.autograd.Function):
             raise RuntimeError("a tensor that the decode's backward pass reads has another shape, type or device than in its "
                                "forward pass (its .data was replaced in between, or a saved-tensor hook changed it)")
         saved = [t.contiguous() for t in saved]
-        # (kernels read 16 bytes at a time, the block's parts are laid out from 256-byte boundaries)
-        camera_center, block, anchor, feat, offset, scaling, *params = [t if t.data_ptr() % 256 == 0 or k not in (1, 3)
-                                                                        else t.clone() for k, t in enumerate(saved)]
+        camera_center, block, anchor, feat, offset, scaling, *params = saved
+        # (the block's parts lie at 256-byte boundaries from its start, feature rows are read 16 bytes at a time)
+        block, feat = (t if t.data_ptr() % to == 0 else t.clone() for t, to in ((block, 256), (feat, 16)))
         parts = ctx.parts
         dec, an = _train_records(ctx.decoder, camera_center, ctx.visible, ctx.level, anchor, feat, offset, scaling, params)
         rows, workspace = parts.rows(block, ctx.num_visible)
