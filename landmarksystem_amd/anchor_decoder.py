@@ -186,7 +186,7 @@ class _DecodeTrain(torch.autograd.Function):
         ctx.visible, ctx.level = visible, level
         saved = (camera_center.clone(), block, anchor, feat, offset, scaling, *params)
         ctx.save_for_backward(*saved)
-        ctx.kinds = [(t.shape, t.dtype, t.device) for t in saved]
+        ctx.shapes = [t.shape for t in saved]
         ctx.mark_non_differentiable(out[6])
         ctx.set_materialize_grads(False)
         return out
@@ -195,10 +195,12 @@ class _DecodeTrain(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural, _g_mask):
         saved = ctx.saved_tensors
-        if [(t.shape, t.dtype, t.device) for t in saved] != ctx.kinds:
+        device = ctx.visible.get_device()
+        if any(t.shape != shape or t.get_device() != device or t.dtype is not (torch.float32 if k != 1 else torch.uint8)
+               for k, (t, shape) in enumerate(zip(saved, ctx.shapes))):
             raise RuntimeError("a tensor that the decode's backward pass reads has another shape, type or device than in its "
                                "forward pass (its .data was replaced in between, or a saved-tensor hook changed it)")
-        saved = [t.contiguous() for t in saved]
+        saved = [t if t.is_contiguous() else t.contiguous() for t in saved]
         camera_center, block, anchor, feat, offset, scaling, *params = saved
         # (the block's parts lie at 256-byte boundaries from its start, feature rows are read 16 bytes at a time)
         block, feat = (t if t.data_ptr() % to == 0 else t.clone() for t, to in ((block, 256), (feat, 16)))
@@ -451,21 +453,45 @@ class FusedAnchorDecoder(nn.Module):
         w = _mlp(self.mlp_feature_bank, view if level is None else torch.cat([view, level], dim=1))  # softmax inside
         return feat[:, ::4].repeat(1, 4) * w[:, 0:1] + feat[:, ::2].repeat(1, 2) * w[:, 1:2] + feat * w[:, 2:3]
 
+    def _kernels_take(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level, params):
+        """Whether the training kernels read these tensors as the module's statements do: every one of the shape that the
+        kernels assume (they go by the number of anchors alone, rows of fixed widths), fp32, contiguous and on one device;
+        camera and level not differentiated.  The statements take more than that (masks of other lengths, scales of more
+        columns, heads of other widths) or refuse it themselves."""
+        A, n, dim, device, f32 = anchor.shape[0], self.n_offsets, self.feat_dim, anchor.get_device(), torch.float32
+        if (A == 0 or anchor.shape != (A, 3) or anchor_feat.shape != (A, dim) or offset.dim() == 0 or offset.shape[0] != A
+                or offset.numel() != A * n * 3 or scaling.shape != (A, 6) or visible_mask.shape != (A,)
+                or visible_mask.dtype is not torch.bool or visible_mask.get_device() != device
+                or (camera_center.shape != (3,) and camera_center.shape != (1, 3)) or camera_center.requires_grad
+                or (level is not None and level.requires_grad) or anchor_feat.data_ptr() % 16 != 0):
+            return False
+        wide = dim + 3 + (level is not None)
+        if any(t is None for t in params) or [t.shape for t in params] != [
+                (32, wide + bool(self.add_opacity_dist)), (32,), (n, 32), (n,),
+                (32, wide + bool(self.add_cov_dist)), (32,), (7 * n, 32), (7 * n,),
+                (32, wide + bool(self.add_color_dist)), (32,), (3 * n, 32), (3 * n,)]:
+            return False
+        tensors = [anchor, anchor_feat, offset, scaling, camera_center]
+        if level is not None:
+            tensors.append(level)
+        if any(t.is_inference() for t in tensors):  # (cannot be saved for the backward pass; the statements need not)
+            return False
+        for t in tensors + params:
+            if t.dtype is not f32 or t.get_device() != device or not t.is_contiguous():
+                return False
+        return True
+
     def _forward_differentiable(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level):
-        """The training decode: same 7-tuple, the training by-products always present.  In the kernels, forward and
-        backward, where every tensor is as they read it (fp32, contiguous, on one GPU; camera and level not
-        differentiated); else the statements of the reference module as torch operations."""
+        """The training decode: same 7-tuple, the training by-products always present.  On the GPU in the kernels, forward
+        and backward, where they can take the tensors (_kernels_take); else the statements of the reference module as
+        torch operations."""
         level = self._check_level(level, anchor.shape[0])
         if visible_mask is None:
             visible_mask = torch.ones(anchor.shape[0], dtype=torch.bool, device=anchor.device)
         params = self._head_parameters()
-        dev = anchor.device
-        camera_center = camera_center.to(dev)
-        tensors = [anchor, anchor_feat, offset, scaling, camera_center] + params + ([] if level is None else [level])
-        if (dev.type == "cuda" and anchor.shape[0] > 0 and visible_mask.dtype == torch.bool and visible_mask.device == dev
-                and all(t.device == dev and t.dtype == torch.float32 and t.is_contiguous() for t in tensors)
-                and anchor_feat.data_ptr() % 16 == 0 and not camera_center.requires_grad
-                and not (level is not None and level.requires_grad)):
+        camera_center = camera_center.to(anchor.device)
+        if anchor.is_cuda and self._kernels_take(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level,
+                                                 params):
             feat = anchor_feat
             if self.use_feat_bank:  # (mixed features of the visible anchors, one row each)
                 rows = visible_mask.nonzero(as_tuple=True)[0]
@@ -473,6 +499,7 @@ class FusedAnchorDecoder(nn.Module):
                 view = view / view.norm(dim=1, keepdim=True)
                 feat = self._bank_mix(anchor_feat.index_select(0, rows), view,
                                       None if level is None else level.reshape(-1, 1).index_select(0, rows))
+                feat = feat.float().contiguous()
             return _DecodeTrain.apply(self, camera_center, visible_mask.contiguous(), level, self.use_feat_bank, anchor,
                                       feat, offset, scaling, *params)
         return self._forward_torch(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
@@ -483,6 +510,11 @@ class FusedAnchorDecoder(nn.Module):
         # are the same tensors, but the backward of a boolean-mask index is a sorting index_put (3.7 ms per step at
         # 500k anchors), that of index_select an index_add.
         rows = visible_mask.nonzero(as_tuple=True)[0]
+        # (an index past the end is an error on the CPU and an assertion on the GPU: the rare call that can have one waits
+        # for the largest)
+        shortest = min(t.shape[0] for t in (anchor, anchor_feat, offset, scaling))
+        if shortest < visible_mask.shape[0] and rows.numel() and int(rows[-1]) >= shortest:
+            raise IndexError("anchor %d is visible, a tensor has %d rows" % (int(rows[-1]), shortest))
         a, feat, off, sc = (t.index_select(0, rows) for t in (anchor, anchor_feat, offset, scaling))
         view = a - camera_center.to(a.device)
         dist = view.norm(dim=1, keepdim=True)
@@ -499,12 +531,17 @@ class FusedAnchorDecoder(nn.Module):
         mask = (neural_opacity > 0.0).view(-1)
         kept = mask.nonzero(as_tuple=True)[0]
         owner = torch.div(kept, n, rounding_mode="floor")  # anchor (among the visible ones) of each kept offset
-        color = _mlp(self.mlp_color, with_dist if self.add_color_dist else without).reshape(-1, 3).index_select(0, kept)
-        cov = _mlp(self.mlp_cov, with_dist if self.add_cov_dist else without).reshape(-1, 7).index_select(0, kept)
+        off = off.reshape(-1, 3)
+        color = _mlp(self.mlp_color, with_dist if self.add_color_dist else without).reshape(-1, 3)
+        cov = _mlp(self.mlp_cov, with_dist if self.add_cov_dist else without).reshape(-1, 7)
+        shortest = min(t.shape[0] for t in (off, color, cov))
+        if shortest < mask.shape[0] and kept.numel() and int(kept[-1]) >= shortest:
+            raise IndexError("offset %d of the visible anchors is kept, a tensor has %d rows" % (int(kept[-1]), shortest))
+        color, cov = color.index_select(0, kept), cov.index_select(0, kept)
         sc_kept = sc.index_select(0, owner)
         scaling_out = sc_kept[:, 3:6] * torch.sigmoid(cov[:, 0:3])
         rot = torch.nn.functional.normalize(cov[:, 3:7])
-        xyz = a.index_select(0, owner) + off.reshape(-1, 3).index_select(0, kept) * sc_kept[:, 0:3]
+        xyz = a.index_select(0, owner) + off.index_select(0, kept) * sc_kept[:, 0:3]
         return xyz, color, neural_opacity.index_select(0, kept), scaling_out, rot, neural_opacity, mask
 
     def _forward_kernels(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask=None, level=None):

@@ -113,3 +113,76 @@ def test_camera_and_mask_may_change_after_the_forward_pass(recorder):
     visible.logical_not_()
     out[0].sum().backward()
     assert recorder.back.an.campos != camera.data_ptr()
+
+
+def _forms():
+    """name -> (what differs from the plain call: A = 7 anchors, n = 3 offsets; whether the kernels take it; whether the
+    module's statements do)"""
+    r = torch.Generator().manual_seed(1)
+    rand = lambda *s: torch.randn(*s, generator=r)  # noqa: E731
+    mask = torch.tensor([1, 0, 1, 1, 0, 1, 1], dtype=torch.bool)
+    return {
+        "plain": ({}, True, True),
+        "no mask": (dict(visible_mask=None), True, True),
+        "mask of bytes": (dict(visible_mask=mask.byte()), False, True),
+        "mask as a column": (dict(visible_mask=mask[:, None]), False, True),
+        "shorter mask": (dict(visible_mask=mask[:4]), False, True),
+        "longer mask, all of it past the end unset": (dict(visible_mask=torch.cat([mask, ~mask.new_ones(5)])), False, True),
+        "longer mask": (dict(visible_mask=torch.cat([mask, mask])), False, False),
+        "strided mask": (dict(visible_mask=mask.repeat_interleave(2)[::2]), True, True),
+        "camera as a row": (dict(camera_center=rand(1, 3)), True, True),
+        "camera of one number": (dict(camera_center=rand(1)), False, True),
+        "camera per visible anchor": (dict(camera_center=rand(5, 3)), False, True),
+        "differentiable camera": (dict(camera_center=rand(3).requires_grad_(True)), False, True),
+        "strided anchors": (dict(anchor=rand(3, 7).t()), False, True),
+        "anchors of four columns": (dict(anchor=rand(7, 4)), False, False),
+        "offsets as rows": (dict(offset=rand(7, 9)), True, True),
+        "fewer offsets": (dict(offset=rand(7, 1, 3)), False, False),
+        "more offsets": (dict(offset=rand(7, 5, 3)), False, True),
+        "offsets of fewer anchors": (dict(offset=rand(5, 3, 3)), False, False),
+        "scales of three columns": (dict(scaling=rand(7, 3).exp()), False, False),
+        "scales of eight columns": (dict(scaling=rand(7, 8).exp()), False, True),
+        "scales of fewer anchors": (dict(scaling=rand(3, 6).exp()), False, False),
+        "features of fewer anchors": (dict(anchor_feat=rand(6, 32)), False, False),
+        "features of more anchors": (dict(anchor_feat=rand(9, 32)), False, True),
+        "wider features": (dict(anchor_feat=rand(7, 64)), False, False),
+        "misaligned features": (dict(anchor_feat=rand(7 * 32 + 1)[1:].view(7, 32)), False, True),
+        "double features": (dict(anchor_feat=rand(7, 32).double()), False, False),
+        "head of another hidden width": (dict(hidden=48), False, True),
+        "head of another input width": (dict(inputs=40), False, False),
+        "head of more outputs": (dict(outputs=12), False, True),
+        "head of fewer outputs": (dict(outputs=6), False, False),
+    }
+
+
+@pytest.mark.parametrize("form", list(_forms()))
+def test_what_the_training_kernels_take(form):
+    """The kernels are chosen only for what they read as the module's statements do; the rest goes to the statements, which
+    take it or refuse it."""
+    change, kernels, statements = _forms()[form]
+    change = dict(change)
+    dec = decoder(n=3)
+    if "hidden" in change or "inputs" in change or "outputs" in change:
+        first = torch.nn.Linear(change.pop("inputs", 36), change.get("hidden", 32))
+        dec.mlp_color = torch.nn.Sequential(first, torch.nn.ReLU(True),
+                                            torch.nn.Linear(change.pop("hidden", 32), change.pop("outputs", 9)), torch.nn.Sigmoid())
+    with torch.no_grad():
+        dec.mlp_opacity[2].bias.fill_(2.0)  # (every offset is kept)
+    anchor, feat, offset, scaling = inputs(n=3)
+    call = dict(camera_center=torch.tensor([0.3, -4.0, 2.0]), anchor=anchor, anchor_feat=feat, offset=offset,
+                scaling=scaling.exp(), visible_mask=torch.tensor([1, 0, 1, 1, 0, 1, 1], dtype=torch.bool))
+    call.update(change)
+    mask = torch.ones(7, dtype=torch.bool) if call["visible_mask"] is None else call["visible_mask"]
+    takes = dec._kernels_take(*[call[k] for k in ("camera_center", "anchor", "anchor_feat", "offset", "scaling")],
+                              mask.contiguous() if mask.dim() == 1 else mask, None, dec._head_parameters())
+    assert takes == kernels
+    if not statements:
+        with pytest.raises((RuntimeError, IndexError)):
+            dec(**call)
+        return
+    got = dec(**call)
+    assert got[0].shape[0] == int(mask.sum()) * 3
+    if kernels:  # as the kernels read them: rows of the fixed widths, one after the other
+        rows = dict(camera_center=call["camera_center"].reshape(3), offset=call["offset"].reshape(7, 3, 3))
+        for a, b in zip(got, dec(**{**call, **rows})):
+            assert torch.equal(a, b)

@@ -110,3 +110,29 @@ def test_gradients_under_saved_tensor_hooks(gpu_device, how, bank):
     want = gradients(lambda: decode(*leaves))
     for a, b in zip(gradients(hooked), want):
         assert torch.equal(a, b)
+
+
+def test_tensors_of_other_shapes_take_the_statements(gpu_device):
+    """What the kernels would read past (a short mask, fewer scales or offsets) is refused on the host or evaluated as the
+    module's statements do, with their results."""
+    torch.manual_seed(0)
+    dec = FusedAnchorDecoder(use_feat_bank=False, add_opacity_dist=True, add_cov_dist=True, add_color_dist=True, view_dim=3,
+                             feat_dim=32, n_offsets=3).to(gpu_device).train()
+    with torch.no_grad():
+        dec.mlp_opacity[2].bias.fill_(2.0)
+    call = dict(camera_center=torch.tensor([0.3, -4.0, 2.0]), anchor=torch.randn(300, 3), anchor_feat=torch.randn(300, 32),
+                offset=torch.randn(300, 3, 3), scaling=torch.randn(300, 6).exp(), visible_mask=torch.rand(300) < 0.7)
+    call = {k: v.to(gpu_device) for k, v in call.items()}
+    whole = dec(**{**call, "visible_mask": call["visible_mask"] & (torch.arange(300, device=gpu_device) < 100)})
+    short = dec(**{**call, "visible_mask": call["visible_mask"][:100]})
+    assert "DecodeTrain" in type(whole[0].grad_fn).__name__ and "DecodeTrain" not in type(short[0].grad_fn).__name__
+    for a, b in zip(whole, short):
+        assert a.shape == b.shape and torch.allclose(a.float(), b.float(), rtol=1e-4, atol=1e-4)
+    for change in (dict(scaling=torch.ones(300, 3, device=gpu_device)), dict(offset=torch.zeros(300, 1, 3, device=gpu_device)),
+                   dict(anchor_feat=torch.zeros(120, 32, device=gpu_device))):
+        with pytest.raises((RuntimeError, IndexError)):
+            dec(**{**call, **change})
+    torch.cuda.synchronize()
+    dec.mlp_color = torch.nn.Sequential(torch.nn.Linear(36, 48), torch.nn.ReLU(True), torch.nn.Linear(48, 9),
+                                        torch.nn.Sigmoid()).to(gpu_device)
+    assert dec(**call)[1].shape == (int(call["visible_mask"].sum()) * 3, 3)
