@@ -35,6 +35,7 @@ from typing import NamedTuple, Optional
 import torch
 from torch import nn
 from torch.autograd.function import once_differentiable
+from torch.nn.modules import module as _module
 
 from . import _lib
 from .pipeline import _raw_stream
@@ -308,8 +309,8 @@ class FusedAnchorDecoder(nn.Module):
         lookups of nn.Module cost a microsecond each, and every frame asks for a dozen parameters."""
         out = []
         for name in names:
-            layers = self._modules[name]._modules
-            for layer in (layers["0"], layers["2"]):
+            layers = tuple(self._modules[name]._modules.values())
+            for layer in (layers[0], layers[2]):
                 p = layer._parameters
                 if "weight" in p and "bias" in p:
                     out += (p["weight"], p["bias"])
@@ -445,6 +446,29 @@ class FusedAnchorDecoder(nn.Module):
         with torch.no_grad():
             return self._forward_kernels(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
 
+    _HEAD_LAYERS = {"mlp_opacity": (nn.Linear, nn.ReLU, nn.Linear, nn.Tanh), "mlp_cov": (nn.Linear, nn.ReLU, nn.Linear),
+                    "mlp_color": (nn.Linear, nn.ReLU, nn.Linear, nn.Sigmoid)}
+
+    def _heads_as_built(self):
+        """Whether the heads are the layers that the constructor made and calling an activation would do nothing but
+        evaluate it: the kernels know neither a module that was put in its place nor a hook on it."""
+        if any((_module._global_forward_hooks, _module._global_forward_pre_hooks, _module._global_backward_hooks,
+                _module._global_backward_pre_hooks)):
+            return False
+        for name, kinds in self._HEAD_LAYERS.items():
+            head = self._modules[name]
+            layers = tuple(head._modules.values())
+            if type(head) is not nn.Sequential or len(layers) != len(kinds):
+                return False
+            for layer, kind in zip(layers, kinds):
+                if kind is nn.Linear:  # (weight and bias are read, the module is not called)
+                    if not isinstance(layer, nn.Linear):
+                        return False
+                elif (type(layer) is not kind or layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
+                      or layer._backward_pre_hooks or "forward" in layer.__dict__):
+                    return False
+        return True
+
     def _head_parameters(self):
         return self._parameters_of(("mlp_opacity", "mlp_cov", "mlp_color"))
 
@@ -483,15 +507,15 @@ class FusedAnchorDecoder(nn.Module):
 
     def _forward_differentiable(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level):
         """The training decode: same 7-tuple, the training by-products always present.  On the GPU in the kernels, forward
-        and backward, where they can take the tensors (_kernels_take); else the statements of the reference module as
-        torch operations."""
+        and backward, where the heads are what they evaluate (_heads_as_built) and they can take the tensors
+        (_kernels_take); else the statements of the reference module as torch operations."""
         level = self._check_level(level, anchor.shape[0])
         if visible_mask is None:
             visible_mask = torch.ones(anchor.shape[0], dtype=torch.bool, device=anchor.device)
-        params = self._head_parameters()
         camera_center = camera_center.to(anchor.device)
-        if anchor.is_cuda and self._kernels_take(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level,
-                                                 params):
+        params = self._head_parameters() if anchor.is_cuda and self._heads_as_built() else None
+        if params is not None and self._kernels_take(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level,
+                                                     params):
             feat = anchor_feat
             if self.use_feat_bank:  # (mixed features of the visible anchors, one row each)
                 rows = visible_mask.nonzero(as_tuple=True)[0]

@@ -1,5 +1,6 @@
 """Host side of the training decode, no GPU needed: what is handed to the library, which stands in as a recorder here."""
 import ctypes as C
+from collections import OrderedDict
 from types import SimpleNamespace
 
 import pytest
@@ -186,3 +187,46 @@ def test_what_the_training_kernels_take(form):
         rows = dict(camera_center=call["camera_center"].reshape(3), offset=call["offset"].reshape(7, 3, 3))
         for a, b in zip(got, dec(**{**call, **rows})):
             assert torch.equal(a, b)
+
+
+def test_heads_that_were_changed_take_the_statements():
+    """A hook on an activation, a module in its place or a head of other layers: the kernels know nothing of it."""
+    called = []
+    note = lambda *a: called.append(1)  # noqa: E731
+    changes = {
+        "forward hook": lambda d: d.mlp_opacity[1].register_forward_hook(note),
+        "forward pre-hook": lambda d: d.mlp_color[3].register_forward_pre_hook(note),
+        "backward hook": lambda d: d.mlp_color[3].register_full_backward_hook(note),
+        "backward pre-hook": lambda d: d.mlp_opacity[3].register_full_backward_pre_hook(note),
+        "own forward": lambda d: setattr(d.mlp_cov[1], "forward", torch.relu),
+        "another activation": lambda d: d.mlp_color.__setitem__(1, torch.nn.LeakyReLU()),
+        "one more layer": lambda d: d.mlp_cov.append(torch.nn.Tanh()),
+        "normalised hidden units": lambda d: setattr(d, "mlp_opacity", torch.nn.Sequential(
+            d.mlp_opacity[0], torch.nn.LayerNorm(32), torch.nn.ReLU(), d.mlp_opacity[2], torch.nn.Tanh())),
+        "hook on all modules": lambda d: torch.nn.modules.module.register_module_forward_hook(note),
+    }
+    for name, change in changes.items():
+        dec, leaves = decoder(n=3), inputs(n=3)
+        assert dec._heads_as_built()
+        handle = change(dec)
+        try:
+            assert not dec._heads_as_built(), name
+            called.clear()
+            out = dec(torch.tensor([0.3, -4.0, 2.0]), *leaves)
+            (out[1].sum() + out[5].sum()).backward()
+            assert bool(called) == ("hook" in name), name
+        finally:
+            if handle is not None and hasattr(handle, "remove"):
+                handle.remove()
+    dec = decoder(n=3)
+    dec.mlp_opacity[0].register_forward_hook(note)  # (the linear layers are not called, their parameters are read)
+    assert dec._heads_as_built()
+
+
+def test_parameters_are_found_by_place():
+    """Heads whose layers have names of their own."""
+    dec = decoder(n=3)
+    want = dec._head_parameters()
+    names = ("first", "relu", "second", "tanh")
+    dec.mlp_opacity = torch.nn.Sequential(OrderedDict(zip(names, dec.mlp_opacity)))
+    assert all(a is b for a, b in zip(dec._head_parameters(), want)) and dec._heads_as_built()

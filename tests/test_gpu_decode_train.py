@@ -136,3 +136,19 @@ def test_tensors_of_other_shapes_take_the_statements(gpu_device):
     dec.mlp_color = torch.nn.Sequential(torch.nn.Linear(36, 48), torch.nn.ReLU(True), torch.nn.Linear(48, 9),
                                         torch.nn.Sigmoid()).to(gpu_device)
     assert dec(**call)[1].shape == (int(call["visible_mask"].sum()) * 3, 3)
+
+
+def test_hooks_and_other_activations_are_not_passed_by(gpu_device):
+    torch.manual_seed(0)
+    dec = FusedAnchorDecoder(use_feat_bank=False, add_opacity_dist=True, add_cov_dist=True, add_color_dist=True, view_dim=3,
+                             feat_dim=32, n_offsets=3).to(gpu_device).train()
+    call = [t.to(gpu_device) for t in (torch.tensor([0.3, -4.0, 2.0]), torch.randn(200, 3), torch.randn(200, 32),
+                                       torch.randn(200, 3, 3), torch.randn(200, 6).exp())]
+    plain = dec(*call)
+    seen = []
+    handle = dec.mlp_color[3].register_forward_hook(lambda module, args, out: seen.append(out.shape))
+    hooked = dec(*call)
+    handle.remove()
+    assert seen == [(200, 9)] and torch.equal(hooked[6], plain[6]) and torch.allclose(hooked[1], plain[1], atol=1e-5)
+    dec.mlp_color[1] = torch.nn.LeakyReLU(0.5)
+    assert not torch.allclose(dec(*call)[1], plain[1], atol=1e-2)
