@@ -29,12 +29,12 @@ reference, whose fused decoder is an inference component and whose training
 runs the torch module.  The rasterizer behind it differentiates in HIP.
 """
 import ctypes as C
+import functools
 from collections import OrderedDict
 from typing import NamedTuple, Optional
 
 import torch
 from torch import nn
-from torch.autograd.function import once_differentiable
 from torch.nn.modules import module as _module
 
 from . import _lib
@@ -151,7 +151,10 @@ class _DecodeTrain(torch.autograd.Function):
     (gs355_decode_train_backward): differentiable with respect to anchors, features, offsets, scales and the heads'
     parameters.  Workspace, input rows, hidden units and pre-activations (968 bytes per anchor) live until the graph is
     dropped.  Everything that the backward pass reads goes through save_for_backward and its pointers are taken there:
-    saved-tensor hooks (save_on_cpu, checkpointing) hand back other tensors than they were given."""
+    saved-tensor hooks (save_on_cpu, checkpointing) hand back other tensors than they were given.
+
+    A backward pass that is itself differentiated (create_graph=True) or batched (is_grads_batched=True) takes the module's
+    statements from the visible anchors on, with the forward pass's choice of offsets."""
 
     @staticmethod
     def forward(ctx, decoder, camera_center, visible, level, compact_feat, anchor, feat, offset, scaling, *params):
@@ -182,9 +185,10 @@ class _DecodeTrain(torch.autograd.Function):
         _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), G, C.byref(o), workspace,
                                           parts.workspace_bytes, _lib.TRAIN_EMIT, stream))
         # Camera, mask and level are not differentiated, and what a caller does to them after this is nothing to the
-        # gradients: the camera is copied, the kernels read neither mask nor level going back.
+        # gradients: the camera is copied, the kernels read neither mask nor level going back (the statements do).
         ctx.decoder, ctx.parts, ctx.num_visible = decoder, parts, V
         ctx.visible, ctx.level = visible, level
+        ctx.versions = [_version(t) for t in (visible, level)]
         saved = (camera_center.clone(), block, anchor, feat, offset, scaling, *params)
         ctx.save_for_backward(*saved)
         ctx.shapes = [t.shape for t in saved]
@@ -193,8 +197,10 @@ class _DecodeTrain(torch.autograd.Function):
         return out
 
     @staticmethod
-    @once_differentiable
-    def backward(ctx, g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural, _g_mask):
+    def backward(ctx, *cotangents):
+        given = cotangents[:6]  # (the mask has none)
+        if torch.is_grad_enabled() or any(g is not None and _batched(g) for g in given):
+            return _DecodeTrain._backward_statements(ctx, given)
         saved = ctx.saved_tensors
         device = ctx.visible.get_device()
         if any(t.shape != shape or t.get_device() != device or t.dtype is not (torch.float32 if k != 1 else torch.uint8)
@@ -211,7 +217,7 @@ class _DecodeTrain(torch.autograd.Function):
         dev, A, V = anchor.device, anchor.shape[0], rows.num_visible
         lib = _lib.load()
         ptr = lambda t: None if t is None or t.numel() == 0 else t.data_ptr()  # noqa: E731
-        given = [None if g is None else g.contiguous() for g in (g_xyz, g_color, g_opacity, g_scaling, g_rot, g_neural)]
+        given = [None if g is None else g.contiguous() for g in given]
         cot = _lib.DecodeCotangents(*[ptr(g) for g in given])
         # (anchors that were not decoded have no gradient: their rows stay zero)
         new = torch.empty_like if V == A else torch.zeros_like
@@ -228,6 +234,52 @@ class _DecodeTrain(torch.autograd.Function):
                                                    parts.workspace_bytes, C.byref(cot), C.byref(out), scratch.data_ptr(),
                                                    scratch.numel() * 4, _raw_stream(dev)))
         return (None, None, None, None, None, *grads)
+
+    @staticmethod
+    def _backward_statements(ctx, given):
+        camera_center, block, *tensors = ctx.saved_tensors
+        visible, level = ctx.visible, ctx.level
+        if ctx.versions != [_version(t) for t in (visible, level)]:
+            raise RuntimeError("visible_mask or level was modified in place after the decode, and its gradients are to be "
+                               "differentiated")
+        decoder, parts = ctx.decoder, ctx.parts
+        opacities = block[parts.offsets[6]:][:ctx.num_visible * decoder.n_offsets * 4].view(torch.float32)
+        with torch.enable_grad():
+            # (aliases: features out of the bank depend on the anchors, and that part is not this function's)
+            anchor, feat, offset, scaling, *params = tensors = [t.view_as(t) for t in tensors]
+            rows = visible.nonzero(as_tuple=True)[0]
+            heads = [_Layers(params[4 * j:4 * j + 4], last) for j, last in enumerate((torch.tanh, None, torch.sigmoid))]
+            out = decoder._from_rows(camera_center, anchor.index_select(0, rows),
+                                     feat if parts.compact_feat else feat.index_select(0, rows),
+                                     offset.index_select(0, rows), scaling.index_select(0, rows),
+                                     None if level is None else level.reshape(-1, 1).index_select(0, rows), heads,
+                                     mixed=parts.compact_feat, mask=opacities > 0.0)
+            wanted = [t for t, w in zip(tensors, ctx.needs_input_grad[5:]) if w]
+            pairs = [(o, g) for o, g in zip(out, given) if g is not None and o.requires_grad]
+        grads = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], allow_unused=True,
+                                         create_graph=torch.is_grad_enabled()) if pairs else [None] * len(wanted))
+        return (None, None, None, None, None, *[next(grads) if w else None for w in ctx.needs_input_grad[5:]])
+
+
+def _batched(t):
+    """Whether t stands for a batch of tensors (vmap, is_grads_batched)."""
+    return torch._C._functorch.is_legacy_batchedtensor(t) or torch._C._functorch.is_batchedtensor(t)
+
+
+def _version(t):
+    return None if t is None or t.is_inference() else t._version
+
+
+class _Layers:
+    """A head by its parameters: Linear, ReLU, Linear and the activation `last`."""
+
+    def __init__(self, params, last):
+        self.params, self.last = params, last
+
+    def __call__(self, x):
+        w0, b0, w1, b1 = self.params
+        x = torch.addmm(b1, torch.relu(torch.addmm(b0, x, w0.t())), w1.t())
+        return x if self.last is None else self.last(x)
 
 
 def _mlp(seq, x):
@@ -540,24 +592,32 @@ class FusedAnchorDecoder(nn.Module):
         if shortest < visible_mask.shape[0] and rows.numel() and int(rows[-1]) >= shortest:
             raise IndexError("anchor %d is visible, a tensor has %d rows" % (int(rows[-1]), shortest))
         a, feat, off, sc = (t.index_select(0, rows) for t in (anchor, anchor_feat, offset, scaling))
+        lvl = level.reshape(-1, 1).index_select(0, rows).to(feat.dtype) if level is not None else None
+        heads = [functools.partial(_mlp, head) for head in (self.mlp_opacity, self.mlp_cov, self.mlp_color)]
+        return self._from_rows(camera_center, a, feat, off, sc, lvl, heads)
+
+    def _from_rows(self, camera_center, a, feat, off, sc, lvl, heads, mixed=False, mask=None):
+        """The statements from the rows of the visible anchors on.  `heads`: opacity, covariance and colour, callable;
+        `mixed`: the features come out of the feature bank; `mask`: the choice of offsets, where it was made before."""
+        mlp_opacity, mlp_cov, mlp_color = heads
         view = a - camera_center.to(a.device)
         dist = view.norm(dim=1, keepdim=True)
         view = view / dist
-        lvl = level.reshape(-1, 1).index_select(0, rows).to(feat.dtype) if level is not None else None
-        if self.use_feat_bank:
+        if self.use_feat_bank and not mixed:
             feat = self._bank_mix(feat, view, lvl)
         if lvl is not None:  # (:181-182: both inputs become [feat | view | level])
             with_dist = without = torch.cat([feat, view, lvl], dim=1)
         else:
             with_dist, without = torch.cat([feat, view, dist], dim=1), torch.cat([feat, view], dim=1)
         n = self.n_offsets
-        neural_opacity = _mlp(self.mlp_opacity, with_dist if self.add_opacity_dist else without).reshape(-1, 1)
-        mask = (neural_opacity > 0.0).view(-1)
+        neural_opacity = mlp_opacity(with_dist if self.add_opacity_dist else without).reshape(-1, 1)
+        if mask is None:
+            mask = (neural_opacity > 0.0).view(-1)
         kept = mask.nonzero(as_tuple=True)[0]
         owner = torch.div(kept, n, rounding_mode="floor")  # anchor (among the visible ones) of each kept offset
         off = off.reshape(-1, 3)
-        color = _mlp(self.mlp_color, with_dist if self.add_color_dist else without).reshape(-1, 3)
-        cov = _mlp(self.mlp_cov, with_dist if self.add_cov_dist else without).reshape(-1, 7)
+        color = mlp_color(with_dist if self.add_color_dist else without).reshape(-1, 3)
+        cov = mlp_cov(with_dist if self.add_cov_dist else without).reshape(-1, 7)
         shortest = min(t.shape[0] for t in (off, color, cov))
         if shortest < mask.shape[0] and kept.numel() and int(kept[-1]) >= shortest:
             raise IndexError("offset %d of the visible anchors is kept, a tensor has %d rows" % (int(kept[-1]), shortest))

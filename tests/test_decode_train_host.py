@@ -14,7 +14,7 @@ class Recorder:
     """The library's training calls: counts of `visible` rows and `kept` Gaussians, and the records of the backward call."""
 
     def __init__(self, visible, kept):
-        self.visible, self.kept, self.back, self.heads = visible, kept, None, []
+        self.visible, self.kept, self.back, self.heads, self.opacities = visible, kept, None, [], None
 
     def gs355_decode_train_bytes(self, A, num_visible, n, workspace, scratch):
         workspace._obj.value, scratch._obj.value = 1024, 1024
@@ -25,6 +25,8 @@ class Recorder:
             self.heads.append(rows._obj.num_visible)
             C.c_int32.from_address(out._obj.count).value = self.kept
             C.c_int32.from_address(out._obj.num_visible).value = self.visible
+            if self.opacities is not None:  # (pre-activations)
+                C.memmove(rows._obj.pre[0], self.opacities.data_ptr(), 4 * self.opacities.numel())
         return 0
 
     def gs355_decode_train_backward(self, dec, an, rows, workspace, nbytes, cot, grads, scratch, scratch_bytes, stream):
@@ -230,3 +232,52 @@ def test_parameters_are_found_by_place():
     names = ("first", "relu", "second", "tanh")
     dec.mlp_opacity = torch.nn.Sequential(OrderedDict(zip(names, dec.mlp_opacity)))
     assert all(a is b for a, b in zip(dec._head_parameters(), want)) and dec._heads_as_built()
+
+
+@pytest.mark.parametrize("bank", [False, True])
+def test_gradients_can_be_differentiated(recorder, bank):
+    """A penalty on a gradient: first and second derivatives of a backward pass under create_graph=True are the statements',
+    with the forward pass's choice of offsets."""
+    dec = decoder(n=3, use_feat_bank=bank).double()
+    leaves = [t.detach().double().requires_grad_(True) for t in inputs(n=3)]
+    camera, visible = torch.tensor([0.3, -4.0, 2.0]).double(), torch.tensor([1, 0, 1, 1, 0, 1, 1], dtype=torch.bool)
+    want = dec._forward_torch(camera, *leaves, visible, None)
+    recorder.kept, recorder.opacities = want[0].shape[0], torch.atanh(want[5].detach()).float().contiguous()
+    rows = visible.nonzero(as_tuple=True)[0]
+    feat = leaves[1]
+    if bank:
+        view = leaves[0].index_select(0, rows) - camera
+        feat = dec._bank_mix(feat.index_select(0, rows), view / view.norm(dim=1, keepdim=True), None)
+    got = _DecodeTrain.apply(dec, camera, visible, None, bank, leaves[0], feat, *leaves[2:], *dec._head_parameters())
+    weights = [torch.randn(t.shape).double() for t in want[:6]]  # (exact in the outputs' type)
+    params = leaves + list(dec.parameters())
+
+    def derivatives(out):
+        loss = sum((t.to(w) * w).sum() for t, w in zip(out, weights))
+        first = torch.autograd.grad(loss, params, create_graph=True, allow_unused=True)
+        second = torch.autograd.grad(sum(f.square().sum() for f in first if f is not None and f.requires_grad), params,
+                                     allow_unused=True)
+        return [torch.zeros_like(p) if g is None else g for p, g in zip(params * 2, first + second)]
+
+    for a, b in zip(derivatives(got), derivatives(want)):
+        assert torch.allclose(a, b, rtol=1e-9, atol=1e-9 * float(b.detach().abs().max()) + 1e-300)
+    assert recorder.back is None
+    # ... but not behind a mask that has changed since
+    got = _DecodeTrain.apply(dec, camera, visible, None, bank, leaves[0], feat, *leaves[2:], *dec._head_parameters())
+    visible.logical_not_()
+    with pytest.raises(RuntimeError, match="in place"):
+        derivatives(got)
+
+
+def test_batched_cotangents_take_the_statements(recorder):
+    dec, leaves = decoder(n=3), inputs(n=3)
+    for p in dec.parameters():
+        p.requires_grad_(False)
+    visible = torch.tensor([1, 0, 1, 1, 0, 1, 1], dtype=torch.bool)
+    want = dec._forward_torch(torch.zeros(3), *leaves, visible, None)
+    recorder.kept, recorder.opacities = want[0].shape[0], torch.atanh(want[5].detach()).contiguous()
+    got = apply(dec, leaves, visible)
+    cotangents = torch.randn(4, *want[3].shape)
+    for a, b in zip(torch.autograd.grad(got[3], leaves, cotangents, is_grads_batched=True, allow_unused=True),
+                    torch.autograd.grad(want[3], leaves, cotangents, is_grads_batched=True, allow_unused=True)):
+        assert (a is None) == (b is None) and (a is None or torch.allclose(a, b, rtol=1e-4, atol=1e-5))

@@ -152,3 +152,32 @@ def test_hooks_and_other_activations_are_not_passed_by(gpu_device):
     assert seen == [(200, 9)] and torch.equal(hooked[6], plain[6]) and torch.allclose(hooked[1], plain[1], atol=1e-5)
     dec.mlp_color[1] = torch.nn.LeakyReLU(0.5)
     assert not torch.allclose(dec(*call)[1], plain[1], atol=1e-2)
+
+
+@pytest.mark.parametrize("bank", [False, True])
+def test_a_penalty_on_a_gradient(gpu_device, bank):
+    """Second derivatives behind the kernels' forward pass, against the statements in float64 on the CPU.  The opacities are
+    kept away from zero, where the two could choose differently."""
+    g = torch.Generator().manual_seed(11)
+    dec = FusedAnchorDecoder(use_feat_bank=bank, add_opacity_dist=True, add_cov_dist=True, add_color_dist=True, view_dim=3,
+                             feat_dim=32, n_offsets=5).train()
+    with torch.no_grad():
+        dec.mlp_opacity[2].bias.copy_(torch.tensor([3.0, -3.0, 3.0, 3.0, -3.0]))
+        dec.mlp_opacity[2].weight.mul_(0.1)
+    cam, vis = torch.tensor([0.3, -4.0, 2.0]), torch.rand(150, generator=g) < 0.6
+    leaves = [torch.randn(150, 3, generator=g), torch.randn(150, 32, generator=g), torch.randn(150, 5, 3, generator=g),
+              torch.randn(150, 6, generator=g) * 0.3]
+
+    def second(dec, cam, leaves, vis):
+        leaves = [t.clone().requires_grad_(True) for t in leaves]
+        out = dec(cam, *leaves[:3], torch.exp(leaves[3]), vis)
+        first = torch.autograd.grad(sum(t.square().sum() for t in out[:5]), leaves, create_graph=True)
+        sum(f.square().sum() for f in first).backward()
+        return [t.grad for t in leaves] + [p.grad for p in dec.parameters()], out[0].grad_fn
+
+    want, _ = second(copy.deepcopy(dec).double(), cam.double(), [t.double() for t in leaves], vis)
+    got, fn = second(dec.to(gpu_device), cam.to(gpu_device), [t.to(gpu_device) for t in leaves], vis.to(gpu_device))
+    assert "DecodeTrain" in type(fn).__name__
+    for k, (a, b) in enumerate(zip(got, want)):
+        scale = float(b.abs().max())
+        assert float((a.cpu().double() - b).abs().max()) <= 1e-4 * scale, k  # (fp32, two passes of the products deep)
