@@ -55,6 +55,8 @@ class GaussianRasterizationSettings(NamedTuple):
 
 _RENDER_AGAIN = ("the rasterizer's backward pass ran already for this frame: its workspace is released after the first "
                  "backward pass (retain_graph=True cannot replay it); render the frame again")
+_OTHER_SCENE = ("the number of Gaussians is not that of the forward pass (%d, %d then): their tensors were replaced before the "
+                "backward pass")
 _INPUT_NAMES = ("means3D", "means2D", "opacities", "shs", "colors_precomp", "scales", "rotations", "cov3D_precomp")
 
 
@@ -98,6 +100,8 @@ class _RasterizeGaussians(torch.autograd.Function):
         inputs = pipeline.FrameInputs(ctx.settings, means3D, opacities=opacities, shs=shs,
                                       colors_precomp=colors_precomp, scales=scales, rotations=rotations,
                                       cov3D_precomp=cov3D_precomp)
+        if inputs.P != radii.shape[0]:  # (the kernels go by the workspace and radii of the forward pass)
+            raise RuntimeError(_OTHER_SCENE % (inputs.P, radii.shape[0]))
         if g_image is None:
             g_image = torch.zeros_like(image)
         want = [n for n in _INPUT_NAMES if needs[n]]
@@ -145,6 +149,8 @@ class _RasterizeParameters(torch.autograd.Function):
         out = SimpleNamespace(image=image, depth=depth, alpha=alpha, radii=radii, key_capacity=ctx.key_capacity)
         inputs = pipeline.FrameInputs(ctx.settings, xyz, opacities=opacity, shs=features_dc, scales=scaling,
                                       rotations=rotation, features_rest=features_rest)
+        if inputs.P != radii.shape[0]:
+            raise RuntimeError(_OTHER_SCENE % (inputs.P, radii.shape[0]))
         names = ("means3D", "means2D", "shs", "features_rest", "opacities", "scales", "rotations")
         want = [n for n, needed in zip(names, ctx.needs_input_grad[1:]) if needed]
         grads = pipeline.render_backward(inputs, out, ctx.workspace, torch.zeros_like(image) if g_image is None else g_image,

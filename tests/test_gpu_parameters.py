@@ -64,3 +64,19 @@ def test_training_model_takes_the_stored_parameters(gpu_device):
     model.compute_cov3D_python = True  # (the activated tensors again)
     assert not model._renders_parameters()
     assert torch.allclose(model(scene.camera), image, atol=1e-4)
+
+
+def test_parameters_replaced_before_the_backward_pass(gpu_device):
+    """Densification between the passes: the backward pass refuses a scene of another size (the workspace and the radii are
+    those of the forward pass)."""
+    scene = scenes.tiny_scene(P=500, width=80, height=64, sh_degree=2)
+    model = GaussianModel.from_activated(scene.means3D, scene.scales, scene.rotations, scene.opacities, scene.shs,
+                                         sh_degree=2).to(gpu_device).train()
+    for p in model.parameters():
+        p.requires_grad_(True)
+    image = model(scene.camera)
+    for p in (model._xyz, model._features_dc, model._features_rest, model._opacity, model._scaling, model._rotation):
+        p.data = torch.cat([p.data, p.data])
+    with pytest.raises(RuntimeError, match="number of Gaussians"):
+        image.sum().backward()
+    torch.cuda.synchronize()
