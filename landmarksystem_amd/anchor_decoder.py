@@ -30,6 +30,7 @@ runs the torch module.  The rasterizer behind it differentiates in HIP.
 """
 import ctypes as C
 import functools
+import threading
 from collections import OrderedDict
 from typing import NamedTuple, Optional
 
@@ -50,6 +51,21 @@ def _f32c(t: torch.Tensor, device) -> torch.Tensor:
     if t.dtype != torch.float32:
         t = t.float()
     return t.contiguous()
+
+
+_counts = threading.local()
+
+
+def _host_counts(dev: torch.device) -> torch.Tensor:
+    """Pinned int32[2] where the kernels of one call on `dev` leave their counts: this thread's own.  A call waits for them
+    before it returns or raises, so a thread has one such call under way at most; threads that share a decoder, or replicas of one,
+    have a buffer each."""
+    kept = _counts.__dict__
+    counts = kept.get(dev.index)
+    if counts is None:
+        with torch.inference_mode(False):
+            counts = kept[dev.index] = torch.zeros(2, dtype=torch.int32, device="cpu", pin_memory=True)
+    return counts
 
 
 class DeviceDecode(NamedTuple):
@@ -163,9 +179,7 @@ class _DecodeTrain(torch.autograd.Function):
         stream = _raw_stream(dev)
         dec, an = _train_records(decoder, camera_center, visible, level, anchor, feat, offset, scaling, params)
         f = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)  # noqa: E731
-        if decoder._host_count is None:
-            decoder._host_count = torch.zeros(2, dtype=torch.int32, pin_memory=True)
-        counts = decoder._host_count  # (pinned: the kernels' stores land there, nothing is copied)
+        counts = _host_counts(dev)  # (pinned: the kernels' stores land there, nothing is copied)
         # room for every anchor: how many are visible is only known on the device
         parts = _TrainBlock(A, A, n, {params[4 * j].shape[1] for j in range(3)}, compact_feat)
         block = torch.empty(parts.total, dtype=torch.uint8, device=dev)
@@ -173,9 +187,10 @@ class _DecodeTrain(torch.autograd.Function):
         o = _lib.Decoded()
         o.num_visible = counts.data_ptr() + 4
         o.count = counts.data_ptr()
-        _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), 0, C.byref(o), workspace,
-                                          parts.workspace_bytes, _lib.TRAIN_HEADS, stream))
+        rc = lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), 0, C.byref(o), workspace, parts.workspace_bytes,
+                                    _lib.TRAIN_HEADS, stream)
         torch.cuda.current_stream(dev).synchronize()
+        _lib.check(rc)
         G, V = counts.tolist()
         rows.num_visible = V
         out = (f(G, 3), f(G, 3), f(G, 1), f(G, 3), f(G, 4), f(V * n, 1), torch.empty(V * n, dtype=torch.bool, device=dev))
@@ -320,7 +335,6 @@ class FusedAnchorDecoder(nn.Module):
         # different streams may be in flight together): "workspace" of gs355_decode, "block" of reused outputs
         self._per_stream = OrderedDict()
         self._marshalled = None  # (key, gs355_decoder struct, the tensors it points at)
-        self._host_count: Optional[torch.Tensor] = None  # pinned landing place of the device-side counts
         self._feat_checked = None  # (identity of the last feature tensor, whether fp16 holds it exactly)
 
     # ---- marshalling -----------------------------------------------------------------------------------------
@@ -482,11 +496,10 @@ class FusedAnchorDecoder(nn.Module):
         """(G, visible anchors) from the device-side counters of a decode: one 8-byte copy to pinned memory, waited
         for.  `res`: a `decode_on_device` result or the int32[2] counter tensor."""
         counts = res.counts if isinstance(res, DeviceDecode) else res
-        if self._host_count is None:
-            self._host_count = torch.zeros(2, dtype=torch.int32, pin_memory=True)
-        self._host_count.copy_(counts, non_blocking=True)
+        host = _host_counts(counts.device)
+        host.copy_(counts, non_blocking=True)
         torch.cuda.current_stream(counts.device).synchronize()
-        return int(self._host_count[0]), int(self._host_count[1])
+        return int(host[0]), int(host[1])
 
     def forward(self, camera_center, anchor, anchor_feat, offset, scaling, visible_mask=None, level=None,
                 prog_ratio=None, transition_mask=None, appearance_code=None):
@@ -639,13 +652,13 @@ class FusedAnchorDecoder(nn.Module):
         dev, A, dec, an, tensors = self._marshal(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
         # the two counters go straight into pinned host memory (which the GPU addresses like its own): no copy is
         # enqueued, the host waits for the count phase and reads them
-        if self._host_count is None:
-            self._host_count = torch.zeros(2, dtype=torch.int32, pin_memory=True)
-        counts = self._host_count
+        counts = _host_counts(dev)
         o = _lib.Decoded()
         o.count, o.num_visible = counts.data_ptr(), counts.data_ptr() + 4
-        self._run(dec, an, 0, o, _lib.DECODE_COUNT, dev)
-        torch.cuda.current_stream(dev).synchronize()
+        try:
+            self._run(dec, an, 0, o, _lib.DECODE_COUNT, dev)
+        finally:
+            torch.cuda.current_stream(dev).synchronize()
         G, a_vis = int(counts[0]), int(counts[1])
         f = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)  # noqa: E731
         out = (f(G, 3), f(G, 3), f(G, 1), f(G, 3), f(G, 4))

@@ -1,5 +1,6 @@
 """Host side of the training decode, no GPU needed: what is handed to the library, which stands in as a recorder here."""
 import ctypes as C
+import threading
 from collections import OrderedDict
 from types import SimpleNamespace
 
@@ -15,6 +16,9 @@ class Recorder:
 
     def __init__(self, visible, kept):
         self.visible, self.kept, self.back, self.heads, self.opacities = visible, kept, None, [], None
+
+    def wait(self):
+        pass
 
     def gs355_decode_train_bytes(self, A, num_visible, n, workspace, scratch):
         workspace._obj.value, scratch._obj.value = 1024, 1024
@@ -39,7 +43,9 @@ def recorder(monkeypatch):
     lib = Recorder(visible=5, kept=11)
     monkeypatch.setattr(_lib, "load", lambda: lib)
     monkeypatch.setattr(anchor_decoder, "_raw_stream", lambda device: 0)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(synchronize=lambda: None))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(synchronize=lambda: lib.wait()))
+    zeros = torch.zeros
+    monkeypatch.setattr(torch, "zeros", lambda *a, pin_memory=False, **kw: zeros(*a, **kw))  # (no GPU to pin for)
     return lib
 
 
@@ -47,7 +53,6 @@ def decoder(n=10, **kw):
     torch.manual_seed(0)
     dec = FusedAnchorDecoder(**dict(dict(use_feat_bank=False, add_opacity_dist=True, add_cov_dist=True, add_color_dist=True,
                                          view_dim=3, feat_dim=32, n_offsets=n), **kw)).train()
-    dec._host_count = torch.zeros(2, dtype=torch.int32)
     return dec
 
 
@@ -281,3 +286,29 @@ def test_batched_cotangents_take_the_statements(recorder):
     for a, b in zip(torch.autograd.grad(got[3], leaves, cotangents, is_grads_batched=True, allow_unused=True),
                     torch.autograd.grad(want[3], leaves, cotangents, is_grads_batched=True, allow_unused=True)):
         assert (a is None) == (b is None) and (a is None or torch.allclose(a, b, rtol=1e-4, atol=1e-5))
+
+
+def test_threads_that_share_a_decoder_keep_their_counts(recorder, monkeypatch):
+    """Both calls have stored their counts before either reads its own (two streams, or replicas over one __dict__)."""
+    dec = decoder(n=3)
+    both, own = threading.Barrier(2), threading.local()
+    store = recorder.gs355_decode_train
+
+    def decode_train(dec, an, rows, capacity, out, *rest):
+        recorder.visible, recorder.kept = own.counts
+        return store(dec, an, rows, capacity, out, *rest)
+
+    monkeypatch.setattr(recorder, "gs355_decode_train", decode_train)
+    monkeypatch.setattr(recorder, "wait", lambda: both.wait(timeout=20))
+    shapes = {}
+
+    def train(visible, kept):
+        own.counts = (visible, kept)
+        shapes[visible] = [t.shape[0] for t in apply(dec, inputs(n=3))]
+
+    threads = [threading.Thread(target=train, args=a) for a in ((5, 11), (6, 13))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert shapes == {5: [11] * 5 + [15] * 2, 6: [13] * 5 + [18] * 2}
