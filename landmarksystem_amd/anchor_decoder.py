@@ -337,6 +337,10 @@ class FusedAnchorDecoder(nn.Module):
         self._marshalled = None  # (key, gs355_decoder struct, the tensors it points at)
         self._feat_checked = None  # (identity of the last feature tensor, whether fp16 holds it exactly)
 
+    def __getstate__(self):
+        """What a copy or a pickle takes along: not the buffers of past calls and the records of pointers into them."""
+        return dict(self.__dict__, _per_stream=OrderedDict(), _marshalled=None, _feat_checked=None)
+
     # ---- marshalling -----------------------------------------------------------------------------------------
     def _decoder_struct(self, device):
         """The gs355_decoder record of the current parameters, rebuilt only when a parameter was replaced, moved or

@@ -1,5 +1,7 @@
 """Host side of the training decode, no GPU needed: what is handed to the library, which stands in as a recorder here."""
+import copy
 import ctypes as C
+import pickle
 import threading
 from collections import OrderedDict
 from types import SimpleNamespace
@@ -312,3 +314,17 @@ def test_threads_that_share_a_decoder_keep_their_counts(recorder, monkeypatch):
     for t in threads:
         t.join()
     assert shapes == {5: [11] * 5 + [15] * 2, 6: [13] * 5 + [18] * 2}
+
+
+@pytest.mark.parametrize("make", [copy.deepcopy, lambda d: pickle.loads(pickle.dumps(d))])
+def test_copies_start_without_what_calls_left_behind(recorder, make):
+    """Buffers, records of pointers and pinned memory belong to the decoder that made them: a copy makes its own."""
+    dec = decoder(n=3)
+    apply(dec, inputs(n=3))
+    dec._per_stream[("stream",)] = dict(workspace=torch.zeros(4), block=(1, None, _lib.Decoded(1)))
+    dec._marshalled, dec._feat_checked = ("key", _lib.Decoder(), []), ("key", True)
+    twin = make(dec)
+    assert not twin._per_stream and twin._marshalled is None and twin._feat_checked is None
+    assert all(torch.equal(a, b) and a is not b for a, b in zip(dec.parameters(), twin.parameters()))
+    assert not any(isinstance(v, torch.Tensor) for v in twin.__dict__.values())
+    apply(twin, inputs(n=3))

@@ -1,5 +1,8 @@
 """GPU parity of the MFMA anchor decode (through gs355_decode_count / _emit)
 against the fp32 torch-CPU oracle of AnchorDecoder.forward."""
+import copy
+import pickle
+
 import numpy as np
 import pytest
 import torch
@@ -353,3 +356,18 @@ def test_decode_of_few_visible_anchors_among_many(gpu_device, A):
     assert want[0].shape[0] > 0
     for name, a, b in zip(("xyz", "color", "opacity", "scaling", "rot"), got[:5], want[:5]):
         assert torch.equal(a, b), name
+
+
+def test_a_copy_of_a_decoder_that_has_decoded(gpu_device):
+    """(nothing of the original's buffers, pinned memory or pointers)"""
+    torch.manual_seed(0)
+    dec = FusedAnchorDecoder(use_feat_bank=False, add_opacity_dist=True, add_cov_dist=True, add_color_dist=True, view_dim=3,
+                             feat_dim=32, n_offsets=10).to(gpu_device).eval()
+    call = [t.to(gpu_device) for t in (torch.tensor([0.3, -4.0, 2.0]), torch.randn(500, 3), torch.randn(500, 32),
+                                       torch.randn(500, 10, 3), torch.randn(500, 6).exp())]
+    with torch.no_grad():
+        want = dec(*call)
+        dec.decode_on_device(*call, reuse_buffers=True)
+        for twin in (copy.deepcopy(dec), pickle.loads(pickle.dumps(dec))):
+            for a, b in zip(twin(*call)[:5], want):
+                assert torch.equal(a, b)
