@@ -136,6 +136,13 @@ def _train_records(decoder, camera_center, visible, level, anchor, feat, offset,
     return d, an
 
 
+# The number of visible anchors is on the device until the heads are done: up to this many anchors there is room for every
+# one of them (63 MB), beyond, the visible ones are counted and waited for first, so that memory follows them (behind a
+# level-of-detail mask they may be few).  The second wait is about 5 % of a step at 5k and 60k anchors (952 -> 1004 us,
+# 989 -> 1068), 1 % or less from 200k on (1302 -> 1311).
+_ROOM_FOR_ALL = 1 << 16
+
+
 class _TrainBlock:
     """Where things lie in the block that a training decode keeps for its backward pass: the kernels' workspace, the input
     rows with and without the distance, hidden units and pre-activations of the three heads; every part 256-byte aligned.
@@ -165,9 +172,9 @@ class _TrainBlock:
 class _DecodeTrain(torch.autograd.Function):
     """The training decode (gs355_decode_train) with its whole backward pass in the kernels
     (gs355_decode_train_backward): differentiable with respect to anchors, features, offsets, scales and the heads'
-    parameters.  Workspace, input rows, hidden units and pre-activations (968 bytes per anchor) live until the graph is
-    dropped.  Everything that the backward pass reads goes through save_for_backward and its pointers are taken there:
-    saved-tensor hooks (save_on_cpu, checkpointing) hand back other tensors than they were given.
+    parameters.  Workspace, input rows, hidden units and pre-activations (968 bytes a row, 1108 with heads of both widths)
+    live until the graph is dropped.  Everything that the backward pass reads goes through save_for_backward and its
+    pointers are taken there: saved-tensor hooks (save_on_cpu, checkpointing) hand back other tensors than they were given.
 
     A backward pass that is itself differentiated (create_graph=True) or batched (is_grads_batched=True) takes the module's
     statements from the visible anchors on, with the forward pass's choice of offsets."""
@@ -180,18 +187,41 @@ class _DecodeTrain(torch.autograd.Function):
         dec, an = _train_records(decoder, camera_center, visible, level, anchor, feat, offset, scaling, params)
         f = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)  # noqa: E731
         counts = _host_counts(dev)  # (pinned: the kernels' stores land there, nothing is copied)
-        # room for every anchor: how many are visible is only known on the device
-        parts = _TrainBlock(A, A, n, {params[4 * j].shape[1] for j in range(3)}, compact_feat)
-        block = torch.empty(parts.total, dtype=torch.uint8, device=dev)
-        rows, workspace = parts.rows(block, parts.room)
         o = _lib.Decoded()
         o.num_visible = counts.data_ptr() + 4
         o.count = counts.data_ptr()
-        rc = lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), 0, C.byref(o), workspace, parts.workspace_bytes,
-                                    _lib.TRAIN_HEADS, stream)
+
+        def launch(room):
+            parts = _TrainBlock(A, room, n, {params[4 * j].shape[1] for j in range(3)}, compact_feat)
+            block = torch.empty(parts.total, dtype=torch.uint8, device=dev)
+            rows, workspace = parts.rows(block, room)
+            return parts, block, rows, workspace, lib.gs355_decode_train(
+                C.byref(dec), C.byref(an), C.byref(rows), 0, C.byref(o), workspace, parts.workspace_bytes, _lib.TRAIN_HEADS,
+                stream)
+
+        # How many rows there are is only known on the device, but for features out of the bank.
+        room = feat.shape[0] if compact_feat else A
+        if not compact_feat and A > _ROOM_FOR_ALL:
+            first = launch(0)  # (counts the visible anchors)
+            torch.cuda.current_stream(dev).synchronize()
+            _lib.check(first[-1])
+            room = int(counts[1])
+        parts, block, rows, workspace, rc = launch(room)
+        # Camera, mask and level are not differentiated, and what a caller does to them after this is nothing to the
+        # gradients: the camera is copied, the kernels read neither mask nor level going back (the statements do).
+        # (All of this while the heads are evaluated.)
+        ctx.decoder, ctx.parts, ctx.visible, ctx.level = decoder, parts, visible, level
+        ctx.versions = [_version(t) for t in (visible, level)]
+        saved = (camera_center.clone(), block, anchor, feat, offset, scaling, *params)
+        ctx.save_for_backward(*saved)
+        ctx.shapes = [t.shape for t in saved]
+        ctx.set_materialize_grads(False)
         torch.cuda.current_stream(dev).synchronize()
         _lib.check(rc)
         G, V = counts.tolist()
+        if V > room:
+            raise RuntimeError("%d anchors are visible, %d were a moment ago: the mask changed during the call" % (V, room))
+        ctx.num_visible = V
         rows.num_visible = V
         out = (f(G, 3), f(G, 3), f(G, 1), f(G, 3), f(G, 4), f(V * n, 1), torch.empty(V * n, dtype=torch.bool, device=dev))
         if G > 0:
@@ -199,16 +229,7 @@ class _DecodeTrain(torch.autograd.Function):
         o.neural_opacity, o.mask = out[5].data_ptr(), out[6].data_ptr()
         _lib.check(lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(rows), G, C.byref(o), workspace,
                                           parts.workspace_bytes, _lib.TRAIN_EMIT, stream))
-        # Camera, mask and level are not differentiated, and what a caller does to them after this is nothing to the
-        # gradients: the camera is copied, the kernels read neither mask nor level going back (the statements do).
-        ctx.decoder, ctx.parts, ctx.num_visible = decoder, parts, V
-        ctx.visible, ctx.level = visible, level
-        ctx.versions = [_version(t) for t in (visible, level)]
-        saved = (camera_center.clone(), block, anchor, feat, offset, scaling, *params)
-        ctx.save_for_backward(*saved)
-        ctx.shapes = [t.shape for t in saved]
         ctx.mark_non_differentiable(out[6])
-        ctx.set_materialize_grads(False)
         return out
 
     @staticmethod

@@ -139,6 +139,7 @@ __global__ __launch_bounds__(256) void train_inputs_kernel(TrainArgs d, const ui
     const int part = lane & 3;
     for (int i = lane >> 2; i < nvis; i += 16) {
         const size_t a = (size_t)run * kRun + s_list[wave][i], r = (size_t)rank + i;
+        if (r >= d.V) continue;  // (no room: the caller learns the number from the heads)
         const float4* __restrict__ f4 = reinterpret_cast<const float4*>(d.feat + (d.compact_feat ? r : a) * kFeat) + 2 * part;
         const float4 f0 = f4[0], f1 = f4[1];
         float extra[4];
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int n = d.n;
     const uint32_t groups = (d.V + kGroup - 1) / kGroup;  // that have a place in `totals`
     const uint32_t V = min(*visible_rows, d.V);
-    if (visible_out && blockIdx.x == 0 && threadIdx.x == 0) *visible_out = V;
+    if (visible_out && blockIdx.x == 0 && threadIdx.x == 0) *visible_out = *visible_rows;
     auto block_head = [](int blk) { return blk == 0 ? 0 : blk < 6 ? 1 : 2; };
     auto block_first = [](int blk) { return blk == 0 ? 0 : blk < 6 ? 16 * (blk - 1) : 16 * (blk - 6); };  // output within its head
     for (int i = threadIdx.x; i < 3 * 32; i += 256) s_b0[i / 32][i % 32] = d.b0[i / 32][i % 32];

@@ -328,3 +328,25 @@ def test_copies_start_without_what_calls_left_behind(recorder, make):
     assert all(torch.equal(a, b) and a is not b for a, b in zip(dec.parameters(), twin.parameters()))
     assert not any(isinstance(v, torch.Tensor) for v in twin.__dict__.values())
     apply(twin, inputs(n=3))
+
+
+@pytest.mark.parametrize("limit,compact,calls", [(7, False, [7]), (6, False, [0, 5]), (6, True, [5])])
+def test_room_for_rows(recorder, monkeypatch, limit, compact, calls):
+    """Room for every anchor up to a number of anchors, for the visible ones beyond (counted first, unless the features
+    come out of the bank, one row for each)."""
+    monkeypatch.setattr(anchor_decoder, "_ROOM_FOR_ALL", limit)
+    dec, leaves = decoder(), inputs()
+    feat = leaves[1][:5] if compact else leaves[1]
+    out = _DecodeTrain.apply(dec, torch.zeros(3), torch.arange(7) < 5, None, compact, leaves[0], feat, *leaves[2:],
+                             *dec._head_parameters())
+    assert recorder.heads == calls and out[5].shape[0] == 50
+    assert out[0].grad_fn.parts.room == calls[-1]
+
+
+def test_more_rows_than_room_are_refused(recorder, monkeypatch):
+    """(the mask changed while the call was under way; the kernels write no row past the room)"""
+    monkeypatch.setattr(recorder, "visible", 6)
+    dec, leaves = decoder(), inputs()
+    with pytest.raises(RuntimeError, match="visible"):
+        _DecodeTrain.apply(dec, torch.zeros(3), torch.arange(7) < 5, None, True, leaves[0], leaves[1][:5], *leaves[2:],
+                           *dec._head_parameters())

@@ -6,6 +6,7 @@ import pytest
 import torch
 import torch.utils.checkpoint
 
+from landmarksystem_amd import anchor_decoder
 from landmarksystem_amd.anchor_decoder import FusedAnchorDecoder
 
 pytestmark = pytest.mark.gpu
@@ -181,3 +182,26 @@ def test_a_penalty_on_a_gradient(gpu_device, bank):
     for k, (a, b) in enumerate(zip(got, want)):
         scale = float(b.abs().max())
         assert float((a.cpu().double() - b).abs().max()) <= 1e-4 * scale, k  # (fp32, two passes of the products deep)
+
+
+@pytest.mark.parametrize("A,visible", [(1, 1.0), (33, 0.5), (1000, 0.3), (300, 0.0), (5000, 0.9)])
+def test_rows_counted_first(gpu_device, monkeypatch, A, visible):
+    """Room for the visible anchors only: the same results, bit for bit, as with room for all."""
+    g = torch.Generator().manual_seed(A)
+    dec = FusedAnchorDecoder(use_feat_bank=False, add_opacity_dist=True, add_cov_dist=False, add_color_dist=True, view_dim=3,
+                             feat_dim=32, n_offsets=10).to(gpu_device).train()
+    vis = (torch.rand(A, generator=g) < visible).to(gpu_device)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (
+        torch.randn(A, 3, generator=g) * 3, torch.randn(A, 32, generator=g), torch.randn(A, 10, 3, generator=g),
+        torch.randn(A, 6, generator=g).exp())]
+    results = []
+    for limit in (1 << 30, 0):
+        monkeypatch.setattr(anchor_decoder, "_ROOM_FOR_ALL", limit)
+        for p in leaves + list(dec.parameters()):
+            p.grad = None
+        out = dec(torch.tensor([0.3, -4.0, 2.0], device=gpu_device), *leaves, vis)
+        assert out[0].grad_fn.parts.room == (A if limit else int(vis.sum()))
+        sum(t.square().sum() for t in out[:6]).backward()
+        results.append([t.detach() for t in out] + [p.grad for p in leaves + list(dec.parameters())])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
