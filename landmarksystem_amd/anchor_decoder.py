@@ -609,6 +609,8 @@ class FusedAnchorDecoder(nn.Module):
             feat = anchor_feat
             if self.use_feat_bank:  # (mixed features of the visible anchors, one row each)
                 rows = visible_mask.nonzero(as_tuple=True)[0]
+                if rows.shape[0] == 0:  # (no features to hand to the kernels)
+                    return self._forward_torch(camera_center, anchor, anchor_feat, offset, scaling, visible_mask, level)
                 view = anchor.index_select(0, rows) - camera_center
                 view = view / view.norm(dim=1, keepdim=True)
                 feat = self._bank_mix(anchor_feat.index_select(0, rows), view,

@@ -205,3 +205,14 @@ def test_rows_counted_first(gpu_device, monkeypatch, A, visible):
         results.append([t.detach() for t in out] + [p.grad for p in leaves + list(dec.parameters())])
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+def test_a_view_without_anchors_and_the_feature_bank(gpu_device):
+    dec = FusedAnchorDecoder(use_feat_bank=True, add_opacity_dist=True, add_cov_dist=True, add_color_dist=True, view_dim=3,
+                             feat_dim=32, n_offsets=10).to(gpu_device).train()
+    leaves = [torch.randn(s, device=gpu_device, requires_grad=True) for s in ((64, 3), (64, 32), (64, 10, 3), (64, 6))]
+    out = dec(torch.zeros(3, device=gpu_device), *leaves, torch.zeros(64, dtype=torch.bool, device=gpu_device))
+    assert [t.shape[0] for t in out] == [0] * 7
+    sum(t.sum() for t in out[:6]).backward()
+    for p in leaves[1:] + list(dec.parameters()):
+        assert p.grad is None or not p.grad.any()
