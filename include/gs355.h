@@ -436,7 +436,8 @@ GS355_API int gs355_decode(const gs355_decoder *dec, const gs355_anchors *an, in
  *   HEADS   the heads' input rows, rows->with_dist [V,36] = [feat | view | dist] (the level instead of the distance with
  *           add_level) and / or rows->without [V,35] = [feat | view], per head hidden = relu(x w0^T + b0) [V,32] and
  *           pre = hidden w1^T + b1 [V,k], and the two counts out->num_visible (V) and out->count (device or pinned host
- *           memory).  rows->num_visible says how many rows there is room for: the number of anchors, V not being known
+ *           memory).  rows->num_visible says how many rows there is room for (0: only V is counted); rows past it are
+ *           left out, and a V larger than it tells the caller that there was too little
  *   EMIT    every field of `out` but the counts, which the caller has read to size them; rows->num_visible is V from here on
  * No feature bank: the caller mixes the features.  The workspace and the rows must stay as they are until the backward
  * pass has run.  Outputs of gs355_decode_train_bytes: bytes of the workspace and of the backward pass's scratch (both

@@ -299,6 +299,111 @@ def _anchors(A=10, ptr=0x1000):
     return a
 
 
+def test_stored_parameters_are_validated_before_any_hip_call():
+    """gs355_run_parameters and its backward pass: SH coefficients, scales and rotations of a count that the host knows."""
+    lib = _lib.load()
+    out = _lib.Outputs()
+    out.image = out.radii = 0x1000
+    inputs = _lib.BackwardInputs(0x1000, 0x1000, 0x1000, 0x1000, 0x1000, 0x1000, 0x1000)
+    grads = _lib.Gradients()
+
+    def forward(f, g, rest):
+        return lib.gs355_run_parameters(C.byref(f), C.byref(g), rest, 0x1000, 1 << 30, 100, C.byref(out), _lib.PIPELINE_FAST, None)
+
+    def backward(f, g, rest):
+        return lib.gs355_render_parameters_backward(C.byref(f), C.byref(g), rest, 0x1000, 1 << 30, 100, C.byref(inputs), 0x1000,
+                                                    1 << 30, C.byref(grads), None, None)
+
+    on_device = _gauss()
+    on_device.P_device = 0x1000
+    for call in (forward, backward):
+        assert "device-side" in _err(_lib.GS355_EINVAL, call, _frame(), on_device, 0x1000)
+        assert "SH coefficients" in _err(_lib.GS355_EINVAL, call, _frame(), _gauss(shs=False, colors=True), None)
+        assert "SH coefficients" in _err(_lib.GS355_EINVAL, call, _frame(), _gauss(sr=False, cov=True), None)
+        assert "at most 16" in _err(_lib.GS355_EINVAL, call, _frame(deg=3, coeffs=25), _gauss(), 0x1000)
+        assert "features_rest is NULL" in _err(_lib.GS355_EINVAL, call, _frame(deg=1, coeffs=4), _gauss(), None)
+        assert "scale/rotation" in _err(_lib.GS355_EINVAL, call, _frame(), _gauss(sr=False), None)
+
+
+def test_anchor_filter_over_stored_parameters_validates():
+    lib = _lib.load()
+    call = lambda f, g, stride, visible: lib.gs355_anchor_filter_parameters(  # noqa: E731
+        C.byref(f) if f else None, C.byref(g) if g else None, stride, visible, None)
+    f, g = _frame(), _gauss(shs=False)
+    on_device = _gauss(shs=False)
+    on_device.P_device = 0x1000
+    assert "frame is NULL" in _err(_lib.GS355_EINVAL, call, None, g, 6, 0x1000)
+    assert "scale_stride" in _err(_lib.GS355_EINVAL, call, f, g, 2, 0x1000)
+    assert "device-side" in _err(_lib.GS355_EINVAL, call, f, on_device, 6, 0x1000)
+    assert "scales and rotations" in _err(_lib.GS355_EINVAL, call, f, _gauss(shs=False, sr=False, cov=True), 6, 0x1000)
+    assert "visible is NULL" in _err(_lib.GS355_EINVAL, call, f, g, 6, None)
+    assert call(f, _gauss(P=0, shs=False), 6, None) == 0  # nothing to do, nothing launched
+
+
+def test_training_decode_validates_before_any_hip_call():
+    lib = _lib.load()
+    need, scratch = C.c_size_t(), C.c_size_t()
+    nbytes = lambda *a: lib.gs355_decode_train_bytes(*a, C.byref(need), C.byref(scratch))  # noqa: E731
+    assert "out of range" in _err(_lib.GS355_EINVAL, nbytes, -1, 0, 10)
+    assert "out of range" in _err(_lib.GS355_EINVAL, nbytes, 10, 11, 10)
+    assert "1..10 offsets" in _err(_lib.GS355_EINVAL, nbytes, 10, 10, 11)
+    assert _err(_lib.GS355_EINVAL, lib.gs355_decode_train_bytes, 10, 10, 10, None, C.byref(scratch))
+    assert nbytes(1000, 1000, 10) == 0 and need.value >= 4 * 1000 and scratch.value >= 4 * 11 * 10 * 1000
+    whole, back = need.value, scratch.value
+    dec, an = _decoder(), _anchors(1000)
+
+    def rows(num_visible=1000, ptr=0x1000, **kw):
+        r = _lib.TrainRows(num_visible, 0, ptr, ptr)
+        for j in range(3):
+            r.hidden[j] = r.pre[j] = ptr
+        for k, v in kw.items():
+            setattr(r, k, v)
+        return r
+
+    out = _lib.Decoded(*[0x1000] * 9)
+
+    def train(dec=dec, an=an, r=None, capacity=0, out=out, ws=0x1000, size=whole, phase=_lib.TRAIN_HEADS):
+        return lib.gs355_decode_train(C.byref(dec), C.byref(an), C.byref(r or rows()), capacity, C.byref(out) if out else None,
+                                      ws, size, phase, None)
+
+    bank = _decoder()
+    bank.bank_in_dim, bank.bank_w0, bank.bank_b0, bank.bank_w1, bank.bank_b1 = 3, 0x1000, 0x1000, 0x1000, 0x1000
+    assert "feature bank" in _err(_lib.GS355_EINVAL, train, dec=bank)
+    assert "input width" in _err(_lib.GS355_EINVAL, train, dec=_decoder(in_dim=(36, 34, 36)))
+    assert "num_visible" in _err(_lib.GS355_EINVAL, train, r=rows(1001))
+    assert "num_visible" in _err(_lib.GS355_EINVAL, train, r=rows(-1))
+    assert "workspace" in _err(_lib.GS355_EINVAL, train, ws=None)
+    assert "aligned" in _err(_lib.GS355_EINVAL, train, ws=0x1010)
+    assert "needed" in _err(_lib.GS355_ENOSPC, train, size=whole - 1)
+    assert "capacity" in _err(_lib.GS355_EINVAL, train, capacity=-1)
+    assert "outputs is NULL" in _err(_lib.GS355_EINVAL, train, out=None)
+    assert "phase" in _err(_lib.GS355_EINVAL, train, phase=3)
+    assert "count is NULL" in _err(_lib.GS355_EINVAL, train, out=_lib.Decoded(*[0x1000] * 5))
+    assert "with_dist must be 16-byte aligned" in _err(_lib.GS355_EINVAL, train, r=rows(with_dist=0x1004))
+    assert "head 0" in _err(_lib.GS355_EINVAL, train, r=rows(with_dist=None))
+    assert "head 0" in _err(_lib.GS355_EINVAL, train, dec=_decoder(in_dim=(35, 36, 36)), r=rows(without=None))
+    misaligned = rows()
+    misaligned.pre[2] = 0x1008
+    assert "head 2" in _err(_lib.GS355_EINVAL, train, r=misaligned)
+    assert "non-NULL" in _err(_lib.GS355_EINVAL, train, out=_lib.Decoded(), phase=_lib.TRAIN_EMIT)
+    assert "non-NULL" in _err(_lib.GS355_EINVAL, train, r=rows(pre=(C.c_void_p * 3)()), phase=_lib.TRAIN_EMIT)
+
+    def backward(r=None, cot=_lib.DecodeCotangents(), grads=_lib.DecodeGradients(), ws=0x1000, sc=0x1000, size=back):
+        return lib.gs355_decode_train_backward(C.byref(dec), C.byref(an), C.byref(r or rows()), ws, whole,
+                                               C.byref(cot) if cot else None, C.byref(grads) if grads else None, sc, size, None)
+
+    assert "num_visible" in _err(_lib.GS355_EINVAL, backward, r=rows(1001))
+    assert "cotangents" in _err(_lib.GS355_EINVAL, backward, cot=None)
+    assert "gradients" in _err(_lib.GS355_EINVAL, backward, grads=None)
+    assert "head 1" in _err(_lib.GS355_EINVAL, backward, r=rows(hidden=(C.c_void_p * 3)(0x1000, 0x1004, 0x1000)))
+    assert "with_dist and without" in _err(_lib.GS355_EINVAL, backward, r=rows(with_dist=None, without=None))
+    assert "features must be 16-byte aligned" in _err(_lib.GS355_EINVAL, backward,
+                                                      grads=_lib.DecodeGradients(None, 0x1004, None, None))
+    assert "scratch" in _err(_lib.GS355_ENOSPC, backward, size=back - 1)
+    assert "scratch" in _err(_lib.GS355_ENOSPC, backward, sc=0x1010)
+    assert "workspace" in _err(_lib.GS355_EINVAL, backward, ws=None)
+
+
 def test_decode_validates_before_any_hip_call():
     lib = _lib.load()
     count = lambda d, a, c, o, s, n: lib.gs355_decode_count(C.byref(d), C.byref(a), c, o, s, n, None)  # noqa: E731

@@ -3,7 +3,7 @@ activated tensors (whose own parity with the oracle the other tests hold)."""
 import pytest
 import torch
 
-from landmarksystem_amd import GaussianRasterizer, scenes
+from landmarksystem_amd import GaussianRasterizer, pipeline, scenes
 from landmarksystem_amd.models import GaussianModel
 from tests.helpers import settings_for
 from tests.test_gpu_backward import assert_grad_close
@@ -80,3 +80,21 @@ def test_parameters_replaced_before_the_backward_pass(gpu_device):
     with pytest.raises(RuntimeError, match="number of Gaussians"):
         image.sum().backward()
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("A,columns", [(1, 6), (63, 3), (64, 6), (65, 4), (1023, 6), (100_001, 6)])
+def test_anchor_filter_over_stored_parameters(gpu_device, A, columns):
+    """gs355_anchor_filter_parameters against gs355_anchor_filter over the activated tensors: the same anchors, sizes down to
+    a pixel's (where the last bit of a scale decides) and quaternions down to zero among them."""
+    scene = scenes.tiny_scene(P=A, width=150, height=97, sh_degree=0)
+    g = torch.Generator().manual_seed(A)
+    anchors = (scene.means3D * 2.0).to(gpu_device)
+    scaling = (torch.randn(A, columns, generator=g) * 2.0 - 4.0).to(gpu_device)
+    rotation = (torch.randn(A, 4, generator=g) * torch.exp(torch.randn(A, 1, generator=g) * 4.0)).to(gpu_device)
+    if A > 2:
+        rotation[1], rotation[2] = 0.0, 1e-20
+    s = settings_for(scene, gpu_device)
+    stored, none = pipeline.anchor_filter(s, anchors, scaling, rotation, stored=True)
+    want, _ = pipeline.anchor_filter(s, anchors, torch.exp(scaling), torch.nn.functional.normalize(rotation))
+    assert none is None and torch.equal(stored, want)
+    assert A < 60 or 0 < int(want.sum()) < A
