@@ -21,12 +21,16 @@ number of Gaussians stays on the device; `forward` waits for that one number
 give its results their exact shapes, `decode_on_device` never waits.
 
 In training mode with gradients enabled and something to differentiate (a
-parameter or an input that requires grad: the training loops of benchmarks/nerf/scaffold_gs and
-octree_gs), `forward` evaluates the module's own statements
-(anchor_decoder.py:147-242) as torch operations on the GPU, so autograd
-reaches the MLPs, the features, the offsets and the scales -- as in the
-reference, whose fused decoder is an inference component and whose training
-runs the torch module.  The rasterizer behind it differentiates in HIP.
+parameter or an input that requires grad: the training loops of
+benchmarks/nerf/scaffold_gs and octree_gs), `forward` is one autograd function
+whose two directions run in kernels too (`gs355_decode_train` and its backward
+call, fp32), reaching the MLPs, the features, the offsets, the scales and the
+anchors.  The feature bank in front of it, heads that were changed (another
+activation, a hook on one), tensors of other shapes or types, and second
+derivatives are evaluated as the module's own statements
+(anchor_decoder.py:147-242) in torch operations -- as in the reference, whose
+fused decoder is an inference component and whose training runs the torch
+module.  The rasterizer behind it differentiates in HIP.
 """
 import ctypes as C
 import functools

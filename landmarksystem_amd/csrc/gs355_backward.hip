@@ -3,7 +3,8 @@
 // screen-space gradient of `means2D` feeds densification, landmark/nerf_components/model_components/fields/
 // encodings/gaussian_encoding.py:729-743).
 //
-// Two kernels over the forward pass's workspace (records, sorted values, ranges):
+// Kernels over the forward pass's workspace (records, sorted values, ranges), in their order:
+//   record_slots     where each Gaussian's records of the next kernel go: one per tile of its rectangle, side by side
 //   blend_backward   per 16x16 tile, the forward blend's walk repeated FRONT TO BACK with the same per-block
 //                    lists and the same per-pair decisions.  With f_i = colour_i . dL/dpixel, w_i = alpha_i T_i,
 //                    prefix P_i = sum_{j<=i} w_j f_j and R = out_pixel . dL/dpixel - T_final dL/dalpha_out (all
@@ -11,10 +12,10 @@
 //                    division by a transmittance and no second, reversed walk.  Per-pair contributions are summed
 //                    over the 16 pixels of a block four list entries at a time, added to the wavefront's own sums of
 //                    the staged Gaussians in LDS (no atomics), and written once per batch of 64 as one 48-byte
-//                    record per (tile, Gaussian) key.  No global
-//                    atomics (they cost more than the rest of the kernel): the records of a Gaussian are
-//                    consecutive, in the order its tile rectangle is walked, and the next kernel sums them in
-//                    that order, so gradients are identical from run to run.
+//                    record per (tile, Gaussian) key.  No global atomics (they cost more than the rest of the
+//                    kernel): the records of a Gaussian are consecutive, in the order its tile rectangle is
+//                    walked, and are summed in that order, so gradients are identical from run to run.
+//   sum_large        (scenes of up to 262144 Gaussians) the records of Gaussians of many tiles, summed by many lanes
 //   preprocess_backward  per Gaussian: conic -> 2-D covariance -> Jacobian / 3-D covariance -> scale, rotation,
 //                    mean; pixel position -> mean; colour -> SH coefficients and view direction -> mean.
 // min(0.99, opacity * G) passes the gradient unchanged, and the `means2D` gradient is in normalised device units

@@ -114,7 +114,10 @@ __device__ __forceinline__ void blend_one(PixelState& p, float pxf, float pyf, c
     const uint64_t finished = __ballot(p.T < p.limit);
     if (finished != 0ull) {  // (once in a pixel's life)
         if (__builtin_amdgcn_inverse_ballot_w64(finished)) {
-            p.last = p.T + w;  // (what T was, to its last bit or the one before)
+            // What T was, with one rounding more than the product's: T is below 0.01 here (1e-4 / (1 - 0.99)), so that is
+            // less than a hundredth of the last bit of alpha.  Keeping T itself is exact and costs a move per list entry
+            // (1M Gaussians at 1080p 447.6 -> 450.5 us, 20M at 4K 1718 -> 1724).
+            p.last = p.T + w;
             p.limit = -1.0f;
             w = p.T = 0.0f;
         }

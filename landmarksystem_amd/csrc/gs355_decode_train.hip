@@ -1,6 +1,6 @@
 // The anchor decode as training differentiates it (landmark/nerf_components/model_components/fields/
-// anchor_decoder.py:147-242 under autograd; benchmarks/nerf/scaffold_gs/gs_trainer.py): everything around the heads'
-// matrix products going forward, and all of it going back, in fp32.
+// anchor_decoder.py:147-242 under autograd; benchmarks/nerf/scaffold_gs/gs_trainer.py), forward and back, in fp32.  The
+// feature bank is the caller's: it hands over mixed features.
 //
 //   rows      visible anchors per run of 128 and (scan) their ranks
 //   inputs    the list of visible anchors and the heads' input rows [feat | view | dist or level]
@@ -12,10 +12,12 @@
 //             the products of the weight gradients accumulated in registers over all of its tiles
 //   sum       the workgroups' weight gradients added up in a fixed order
 //
-// The forward products stay with the caller because a scene's opacities saturate: an anchor far from the camera has
-// pre-activations of a hundred, and one more rounding in them moves the few unsaturated Gaussians across the rasterizer's
-// thresholds.  Every operation here rounds as the framework's own does (this file is compiled without contraction), so
-// the Gaussians are bit for bit those of the module's statements.
+// Going forward the heads add in the order in which the framework's fp32 linear layers add over some thousand rows, and
+// every operation around them rounds as the framework's own does (this file is compiled without contraction): a scene's
+// opacities saturate, an anchor far from the camera has pre-activations of a hundred, and one more rounding in them moves
+// the few unsaturated Gaussians across the rasterizer's thresholds.  With the library at hand the Gaussians of 5 000 to
+// 200 000 anchors are the statements' to the bit; with few rows, where it splits a sum, opacities differ by up to 1.2e-7
+// (1 and 880 rows).  Nothing relies on either: another library may add in another order.
 //
 // Backward, everything is transposed as in the inference decode: weights are the left operand of v_mfma_f32_32x32x2_f32
 // (rows = units), anchors the columns, and the accumulator of one layer (lane = anchor, registers = units
@@ -23,7 +25,8 @@
 // matrix instruction takes 64 cycles, so its left operand comes from LDS, one dword per lane, rows of odd stride.
 //
 // As torch operations the backward pass alone was some thirty launches of skinny matrix products, index and reduction
-// kernels.  At 200k anchors with ten offsets, most of them visible, a training step at 1080p went from 3.01 to 1.59 ms.
+// kernels.  A training step at 200k anchors with ten offsets, most of them visible, at 1080p: 3.48 ms with the statements
+// in both directions, 1.50 with these kernels (two runs of one side differ by 7 %).
 #include "gs355_internal.h"
 
 namespace gs355 {
@@ -168,9 +171,8 @@ __global__ __launch_bounds__(256) void train_inputs_kernel(TrainArgs d, const ui
 // step, and the number of kept offsets per group.  Both layers are v_mfma_f32_16x16x4_f32 with the weights (left operand,
 // rows = units) in registers for the whole kernel and 16 rows as columns.  Each eight inputs are two steps, the even ones
 // and the odd ones (lane quarter q: input 2 q, then 2 q + 1), the last four of 36 one more, and the bias is added last:
-// the order in which the framework's fp32 linear layers add at these shapes, so that training sees the same bits whichever
-// evaluates them (a saturated opacity's gradient hangs on the last bits of its pre-activation; layers of thousands of
-// rows; with fewer it may split the sum).  The accumulator of the first layer (register r of lane quarter q = unit
+// the order in which the framework's fp32 linear layers add over some thousand rows (see the top of this file; a saturated
+// opacity's gradient hangs on the last bits of its pre-activation).  The accumulator of the first layer (register r of lane quarter q = unit
 // 4 q + r) becomes the second's right operand by two lane exchanges per pair of registers.  Outputs pass through LDS so
 // that they leave in 16-byte stores (a row of 70 is not a multiple of that).
 // Six library products, three activations and a counting pass took 250 us at 200k anchors (176k of them visible, ten
@@ -498,8 +500,11 @@ __device__ __forceinline__ void copy_to_lds(const float* src, float* dst, int co
 // LDS.  146 us at 200k anchors (37 us of matrix instructions; the rest is the wait for a tile's rows, which one wavefront
 // per SIMD does not hide).
 // kAnchor: the anchors' own gradient is wanted (the layers are then also walked back to view direction and distance).
-// kOffsets: offsets per anchor, or 0 (d.n).  Ten, the decoder's default, has its loops unrolled: with the count a variable,
-// the kernel does not fit its registers.
+// kOffsets: offsets per anchor, or 0 (d.n).  Ten, the decoder's default, has its loops unrolled; with the count a variable
+// the compiler spills 16 registers (33 with kAnchor), and the kernel takes 185 us at ten offsets instead of 146 (206 and 162
+// with kAnchor; 200k anchors).  Any other count takes the variable one: 166 us at eight offsets (unrolled 134), 137 at four
+// (111), 175 at nine (whose odd counts an unrolled loop would have to guard).  A copy of the kernel for each of them would
+// take 25 to 32 us off a training step of more than a millisecond; only the default has one.
 template <bool kAnchor, int kOffsets>
 __global__ __launch_bounds__(64 * kBackwardWaves) void train_layers_kernel(
     TrainArgs d, const uint32_t* __restrict__ rows, const float* __restrict__ d_op, const float* __restrict__ d_cov,

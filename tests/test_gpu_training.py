@@ -1,8 +1,7 @@
-"""Training through the anchor decode (Scaffold-GS / Octree-GS): with gradients enabled the decoder evaluates the
-reference module's statements as torch operations (as the reference trains: its fused decoder is an inference
-component), the rasterizer behind it differentiates in HIP.  Checked: the differentiable path gives the kernels'
-Gaussians; its gradients equal those of the oracle's statements evaluated in float64; a short optimisation of a
-perturbed Scaffold-GS model against its own rendering reduces the loss."""
+"""Training through the anchor decode (Scaffold-GS / Octree-GS): with gradients enabled the decoder is an autograd function
+over the training kernels, the rasterizer behind it differentiates in HIP.  Checked: the differentiable path gives the
+inference kernels' Gaussians; its gradients equal those of the oracle's statements evaluated in float64; a short
+optimisation of a perturbed Scaffold-GS model against its own rendering reduces the loss."""
 import numpy as np
 import pytest
 import torch
