@@ -40,19 +40,20 @@ MFMA_F16_PEAK_TFLOPS = 2500.0
 COUNTER_TRAFFIC = {
     "source": "profiles/bench_c3_6M_1080p_hbm_traffic.txt",
     "workload": "configs[2]",
-    "bytes": {"blend": 1844.2e6, "preprocess": 1705.8e6, "keys_sort_ranges": 824.4e6},
-    # fp32 flops the blend kernel issues per launch (64 lanes x (2 FMA + MUL + ADD) wavefront instructions), from
+    "bytes": {"blend": 1847.2e6, "preprocess": 1705.8e6, "keys_sort_ranges": 824.7e6},
+    # fp32 flops the blend kernel issues per launch in vector instructions (64 lanes x (2 FMA + MUL + ADD) wavefront
+    # instructions; the four channels' accumulation is a matrix instruction and not among them), from
     # profiles/bench_c3_6M_1080p_valu_counters.txt
-    "blend_issued_flops": 10.31e9,
+    "blend_issued_flops": 6.86e9,
     "blend_issued_flops_source": "profiles/bench_c3_6M_1080p_valu_counters.txt",
-    "blend_valu_busy": 0.957,
+    "blend_valu_busy": 0.989,
 }
 
 # Same for `--config 5`: HBM bytes per launch of the two decode kernels (count + emit)
 COUNTER_TRAFFIC_C5 = {
     "source": "profiles/bench_c5_scaffold_500k_hbm_traffic.txt",
     "workload": "configs[4]",
-    "bytes": {"decode": 250.6e6},
+    "bytes": {"decode": 244.4e6},
 }
 
 
@@ -245,9 +246,10 @@ def raster_report(stage_ms, stats, P, tiles, npix, colour_bytes, pairs, counters
                         "valu_busy": counters.get("blend_valu_busy"), "traffic": traffic, "traffic_source": traffic_source,
                         "issued_flops_source": counters["blend_issued_flops_source"], "work_rate": work_rate,
                         "note": "achieved = fp32 flops the kernel ISSUED per launch (wavefront FMA / MUL / ADD instructions x "
-                                "64 lanes, FMA = 2; hardware counters of an earlier run of this workload, named above) / the "
-                                "launch time measured in this run.  peak = MI355X fp32 vector peak with packed FMA (157.3); "
-                                "this build issues unpacked fp32 only (packed fp32 is disabled on this pool), whose peak is "
+                                "64 lanes, FMA = 2, without the matrix instructions that accumulate the channels; hardware "
+                                "counters of an earlier run of this workload, named above) / the launch time measured in this "
+                                "run.  peak = MI355X fp32 vector peak with packed FMA (157.3); "
+                                "this build issues unpacked fp32 only (packed fp32 is left out), whose peak is "
                                 "78.6.  valu_busy = share of cycles the vector ALUs were issuing (same counter run): the "
                                 "kernel is bound by instruction issue, most of it compares, selects and address arithmetic"}
         else:

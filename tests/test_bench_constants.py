@@ -55,8 +55,9 @@ def test_quoted_decode_traffic_matches_the_profile_it_names():
     path = os.path.join(ROOT, table["source"])
     if not os.path.exists(path):
         pytest.skip("profiles/ is not part of this checkout")
-    # count + emit passes of the fp16-exact variant, which the named workload runs (<.., .., true> = fp32 weights)
-    mb = sum(v for k, v in traffic_table(path).items() if k.startswith("decode_kernel") and k.endswith("false>"))
+    # count + emit passes of the fp16-exact variant, which the named workload runs (<.., true> = fp32 weights)
+    mb = sum(v for k, v in traffic_table(path).items()
+             if k.startswith(("decode_count_kernel", "decode_emit_kernel")) and k.endswith("false>"))
     assert mb > 0 and abs(table["bytes"]["decode"] / 1e6 - mb) <= 0.002 * mb + 0.2, (table["bytes"]["decode"] / 1e6, mb)
 
 
