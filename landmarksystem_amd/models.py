@@ -586,8 +586,11 @@ class ScaffoldGS(nn.Module):
         if fused:
             view = pipeline.FrameView(settings, anchor.device)
             d["_view"] = (viewpoint_camera, view)
-        self._before_prefilter(viewpoint_camera)
-        voxel_visible_mask = self.prefilter_voxel(viewpoint_camera)
+        try:
+            self._before_prefilter(viewpoint_camera)
+            voxel_visible_mask = self.prefilter_voxel(viewpoint_camera)
+        finally:  # (a prefilter of another kind, or one that failed, has not taken it)
+            d.pop("_view", None)
         if render_exclude_filter is not None:
             voxel_visible_mask = voxel_visible_mask & render_exclude_filter
         renderer = self.renderer

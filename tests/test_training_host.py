@@ -1,4 +1,6 @@
 """Host-side pieces of the training path that need no GPU."""
+import copy
+
 import torch
 
 from landmarksystem_amd.anchor_decoder import _TallLinear, _mlp
@@ -29,3 +31,28 @@ def test_mlp_helper_follows_the_sequential_module():
     # a view whose rows are not contiguous
     wide = torch.randn(50, 70, dtype=torch.float64)
     assert torch.allclose(_mlp(seq, wide[:, ::2]), seq(wide[:, ::2].clone()), rtol=0, atol=1e-12)
+
+
+def test_a_frame_leaves_no_marshalled_settings_behind():
+    """The settings that a frame marshals for its prefilter are gone after it, also where the prefilter was another one or
+    failed: left on the model, the next direct call would take them for its own, and a copy of the model would hold
+    pointers."""
+    from landmarksystem_amd import scenes
+    from landmarksystem_amd.cameras import Camera
+    from landmarksystem_amd.models import ScaffoldGS
+
+    class Stop(Exception):
+        pass
+
+    class Other(ScaffoldGS):
+        def prefilter_voxel(self, viewpoint_camera, scaling_modifier=1.0):
+            raise Stop
+
+    model = Other.from_scene(scenes.config5(A=8)).eval()
+    camera = Camera.look_at([0.0, 0.0, 20.0], [0.0, 0.0, 0.0], [0.0, 1.0, 0.0], 32, 32, 1.0)
+    try:
+        model(camera)
+    except Stop:
+        pass
+    assert "_view" not in model.__dict__
+    copy.deepcopy(model)
