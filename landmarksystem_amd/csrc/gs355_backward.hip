@@ -50,18 +50,20 @@ __device__ __forceinline__ RecordRun record_run(RecordSlots s, uint64_t rect)
 // Slots of all Gaussians: a workgroup adds up the rectangles of its 8192 Gaussians and takes that many slots from one
 // counter (1024 Gaussians per request: 73 us at 6M Gaussians, the requests being served one after the other).  Which
 // workgroup gets which slots varies between runs, the order of a Gaussian's own records does not, and nothing else enters
-// a sum.
+// a sum.  A frame that overflowed its capacity has no records, and no room for them: no Gaussian has slots.
 constexpr int kSlotItems = 8, kSlotThreads = 1024;
-__global__ __launch_bounds__(kSlotThreads) void record_slots_kernel(int P, const uint64_t* __restrict__ rects,
+__global__ __launch_bounds__(kSlotThreads) void record_slots_kernel(int P, const gs355_header* __restrict__ header,
+                                                                    const uint64_t* __restrict__ rects,
                                                                     uint32_t* __restrict__ next,
                                                                     RecordSlots* __restrict__ slots)
 {
     __shared__ uint32_t s_wave[kSlotThreads / 64], s_first;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int first = (int)blockIdx.x * kSlotItems * kSlotThreads + (int)threadIdx.x;
+    const int end = header->overflow ? 0 : P;
     uint64_t rect[kSlotItems];
 #pragma unroll
-    for (int k = 0; k < kSlotItems; ++k) rect[k] = first + k * kSlotThreads < P ? rects[first + k * kSlotThreads] : 0ull;
+    for (int k = 0; k < kSlotItems; ++k) rect[k] = first + k * kSlotThreads < end ? rects[first + k * kSlotThreads] : 0ull;
     uint32_t sum = 0;
 #pragma unroll
     for (int k = 0; k < kSlotItems; ++k) sum += record_run({0u, rect_width(rect[k])}, rect[k]).n;
@@ -973,8 +975,7 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     if (rc) return rc;
     RecordSlots* slots = reinterpret_cast<RecordSlots*>(record_slots);
     hipLaunchKernelGGL(record_slots_kernel, dim3((g.P + kSlotThreads * kSlotItems - 1) / (kSlotThreads * kSlotItems)),
-                       dim3(kSlotThreads), 0, s, g.P,
-                       rects, next_slot, slots);
+                       dim3(kSlotThreads), 0, s, g.P, header, rects, next_slot, slots);
     GS355_CHECK_LAUNCH("record slots");
     const int tiles = f.grid_x * f.grid_y;
     auto blend = [&](auto kernel) {

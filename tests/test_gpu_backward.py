@@ -342,3 +342,24 @@ def test_values_that_are_not_finite_reach_the_gaussians_of_their_pixels_only(gpu
         assert finite[~concerned].all(), name
     for name, value in got.items():
         assert np.array_equal(value.reshape(400, -1)[~concerned], want[name].reshape(400, -1)[~concerned]), name
+
+
+def test_backward_of_a_frame_that_overflowed(gpu_device):
+    """A frame whose keys did not fit has no gradient records, and no room for them: every gradient is zero, nothing is read
+    or written past the scratch."""
+    scene = scenes.tiny_scene(P=3000, width=160, height=128, sh_degree=1, seed=2)
+    s = settings_for(scene, gpu_device)
+    inp = pipeline.FrameInputs(s, scene.means3D.to(gpu_device), opacities=scene.opacities.to(gpu_device),
+                               shs=scene.shs.to(gpu_device), scales=scene.scales.to(gpu_device),
+                               rotations=scene.rotations.to(gpu_device))
+    ws = pipeline.Workspace(gpu_device)
+    out = pipeline.render(inp, ws=ws)
+    image = torch.ones_like(out.image)
+    assert pipeline.render_backward(inp, out, ws.buffer, image)["opacities"].any()
+    few = out.num_keys // 4
+    layout = pipeline.run_stages(inp, out, ws, few, _lib.PIPELINE_FAST)
+    out.key_capacity = few
+    assert _lib.Header.from_buffer_copy(ws.view(layout, "header", 0, 0, 0).cpu().numpy()).overflow
+    grads = pipeline.render_backward(inp, out, ws.buffer, image)
+    torch.cuda.synchronize()
+    assert all(not g.any() for g in grads.values())
