@@ -1,9 +1,11 @@
 """Frames and gradients taken from GaussianModel's stored parameters inside the kernels, against the same frame over the
 activated tensors (whose own parity with the oracle the other tests hold)."""
+import ctypes as C
+
 import pytest
 import torch
 
-from landmarksystem_amd import GaussianRasterizer, pipeline, scenes
+from landmarksystem_amd import GaussianRasterizer, _lib, pipeline, scenes
 from landmarksystem_amd.models import GaussianModel
 from tests.helpers import settings_for
 from tests.test_gpu_backward import assert_grad_close
@@ -98,3 +100,35 @@ def test_anchor_filter_over_stored_parameters(gpu_device, A, columns):
     want, _ = pipeline.anchor_filter(s, anchors, torch.exp(scaling), torch.nn.functional.normalize(rotation))
     assert none is None and torch.equal(stored, want)
     assert A < 60 or 0 < int(want.sum()) < A
+
+
+@pytest.mark.parametrize("stored", [False, True])
+def test_frame_call_reports_an_overflow_and_is_repeated(gpu_device, stored):
+    """gs355_render_frame itself: too small a capacity comes back with the exact number of keys in the header, the same
+    call with that capacity renders the frame."""
+    scene = scenes.tiny_scene(P=3000, width=160, height=128, sh_degree=2, seed=2)
+    model = GaussianModel.from_activated(scene.means3D, scene.scales, scene.rotations, scene.opacities, scene.shs,
+                                         sh_degree=2).to(gpu_device)
+    s = settings_for(scene, gpu_device)
+    if stored:
+        inp = pipeline.FrameInputs(s, model._xyz, opacities=model._opacity, shs=model._features_dc, scales=model._scaling,
+                                   rotations=model._rotation, features_rest=model._features_rest)
+    else:
+        inp = pipeline.FrameInputs(s, model.get_xyz, opacities=model.get_opacity, shs=model.get_features,
+                                   scales=model.get_scaling, rotations=model.get_rotation)
+    want = pipeline.render(inp, ws=pipeline.Workspace(gpu_device))
+    ws, out = pipeline.Workspace(gpu_device), pipeline.FrameOutputs(inp)
+    out.c.header_copy = ws.header_host.data_ptr()
+
+    def call(n_cap):
+        ws.ensure(inp.P, n_cap, inp.width, inp.height)
+        _lib.check(_lib.load().gs355_render_frame(
+            C.byref(inp.frame), C.byref(inp.gaussians), int(stored), pipeline._ptr(inp.features_rest), ws.buffer.data_ptr(),
+            ws.buffer.numel(), n_cap, C.byref(out.c), _lib.PIPELINE_FAST, pipeline._raw_stream(gpu_device)))
+        h = ws.header
+        return h.ready, h.overflow, h.num_keys_total, h.num_visible
+
+    assert call(want.num_keys - 1) == (1, 1, want.num_keys, want.num_visible)
+    assert call(want.num_keys) == (1, 0, want.num_keys, want.num_visible)
+    for a, b in ((out.image, want.image), (out.depth, want.depth), (out.alpha, want.alpha), (out.radii, want.radii)):
+        assert torch.equal(a, b)
