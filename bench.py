@@ -126,12 +126,14 @@ def stage_breakdown(torch, pipeline, _lib, inp, n_cap, steps):
     out = pipeline.FrameOutputs(inp)
     # like render() on a steady stream of frames, the sort stage leaves out the launches of the sorter size classes
     # that this frame leaves empty (a hint to the library, read from the header the tile-count stage writes)
-    lay = pipeline.run_stages(inp, out, ws, n_cap, _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_COUNT)
+    front = _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_REACH  # (as render(): keys only for the tiles a splat reaches)
+    lay = pipeline.run_stages(inp, out, ws, n_cap, front | _lib.STAGE_TILE_COUNT)
     torch.cuda.synchronize()
     words = [int(w) for w in ws.view(lay, "header", inp.P, 0, inp.tiles)[:4].tolist()]
+    num_pairs = words[1] & 0xFFFFFFFF
     class_counts = ((words[2] >> 32) & 0xFFFFFFFF, words[3] & 0xFFFFFFFF, (words[3] >> 32) & 0xFFFFFFFF)
     skip = sum(m for m, c in zip(_lib.STAGE_TILESORT_SKIP, class_counts) if c == 0)
-    fast = [("preprocess", _lib.STAGE_PREPROCESS), ("tile_count", _lib.STAGE_TILE_COUNT),
+    fast = [("preprocess", front), ("tile_count", _lib.STAGE_TILE_COUNT),
             ("tile_scatter", _lib.STAGE_TILE_SCATTER), ("tile_sort", _lib.STAGE_TILESORT | skip),
             ("blend", _lib.STAGE_BLEND)]
     classic = [("scan", _lib.STAGE_SCAN), ("duplicate", _lib.STAGE_DUPLICATE), ("sort", _lib.STAGE_SORT),
@@ -143,7 +145,7 @@ def stage_breakdown(torch, pipeline, _lib, inp, n_cap, steps):
     ranges = ws.view(lay, "ranges", inp.P, 0, inp.tiles).cpu().numpy().view("uint32")
     stats = {"num_keys": int(hdr[0]), "num_visible": int(hdr[2]) & 0xFFFFFFFF,
              "range_sum": int((ranges[:, 1].astype("int64") - ranges[:, 0]).sum()), "sort_passes": int(lay.sort_passes),
-             "sort_class_buckets": list(class_counts)}
+             "sort_class_buckets": list(class_counts), "num_pairs": num_pairs}
     return ms, stats
 
 
@@ -220,6 +222,7 @@ def raster_report(stage_ms, stats, P, tiles, npix, colour_bytes, pairs, counters
     stages["preprocess_plus_sort"] = hbm(pre_sort_ms, work["preprocess"] + sort_bytes, counter_sum)
     stages["rates"] = {"gaussians_per_s_preprocess": round(P / stage_ms["preprocess"] * 1e3),
                        "sorted_keys_per_s": round(N / sort_ms * 1e3) if N else 0,
+                       "keys": N, "keys_in_reached_tiles": stats["num_pairs"],
                        "blend_frames_per_s": round(1e3 / stage_ms["blend"], 1)}
 
     # the dominant KERNEL: preprocess and blend are one kernel each; count / scatter / sort are groups of several
@@ -324,10 +327,13 @@ def cpu_pair_stats(scene, cam=None, colors_precomp=None, sh_degree=None, keep_fr
 
 def parity_leg(torch, pipeline, inp, ref):
     """The `parity` object: one frame through the product path (pipeline.render over a workspace of its own) against
-    the frame the C checker rendered from the same inputs: radii, key count, every sorted key and value and the
-    tile ranges bit for bit; image, depth and alpha as measured errors."""
+    the frame the C checker rendered from the same inputs: radii and key count bit for bit; image, depth and alpha as
+    measured errors.  The product path makes keys only for the tiles that a splat reaches, so every sorted key and value
+    and the tile ranges are compared, bit for bit, on the same stages run over whole rectangles, whose image has to be the
+    product path's."""
     import numpy as np
 
+    from landmarksystem_amd import _lib
     from oracle import compare
     ws = pipeline.Workspace(inp.device)
     out = pipeline.render(inp, ws=ws)
@@ -337,11 +343,14 @@ def parity_leg(torch, pipeline, inp, ref):
     take = lambda name, kind: ws.view(lay, name, inp.P, n, inp.tiles).cpu().numpy().view(kind)  # noqa: E731
     exact = {"radii": bool(np.array_equal(out.radii.cpu().numpy(), ref["radii"])),
              "num_keys": bool(n == ref["num_keys"])}
+    got = dict(image=out.image.cpu().numpy(), depth=out.depth.cpu().numpy(), alpha=out.alpha.cpu().numpy())
     if n == ref["num_keys"]:
+        pipeline.run_stages(inp, out, ws, out.key_capacity, _lib.PIPELINE_FAST)
+        torch.cuda.synchronize()
+        exact["image_of_whole_rectangles"] = bool(np.array_equal(out.image.cpu().numpy(), got["image"]))
         exact["sorted_keys"] = bool(np.array_equal(take("sorted_keys", np.uint64), ref["sorted_keys"]))
         exact["sorted_values"] = bool(np.array_equal(take("sorted_values", np.uint32), ref["sorted_values"]))
         exact["tile_ranges"] = bool(np.array_equal(take("ranges", np.uint32), ref["ranges"]))
-    got = dict(image=out.image.cpu().numpy(), depth=out.depth.cpu().numpy(), alpha=out.alpha.cpu().numpy())
     return compare.parity_object(got, ref, exact)
 
 

@@ -109,8 +109,9 @@ typedef struct gs355_outputs {
 /* Words of the workspace header (u32 unless noted), written by the scan stage (classic pipeline) or the
  * tile-count stage (fast pipeline). */
 typedef struct gs355_header {
-    uint64_t num_keys_total; /* exact number of (tile, Gaussian) keys the frame needs */
-    uint32_t num_keys;       /* min(num_keys_total, key capacity): what later stages process */
+    uint64_t num_keys_total; /* number of (tile, Gaussian) keys of the frame's tile rectangles: the capacity it needs */
+    uint32_t num_keys;       /* what later stages process: min(num_keys_total, key capacity), or with
+                              * GS355_STAGE_TILE_REACH the keys that were left (the capacity, if that was too small) */
     uint32_t overflow;       /* 1 if num_keys_total > key capacity (the frame must be redone with more) */
     uint32_t num_visible;    /* Gaussians with radius > 0 */
     /* Tile-count stage, images of at most 36000 tiles: buckets in each of the three larger sorter size classes
@@ -127,7 +128,9 @@ typedef struct gs355_layout {
     size_t header;        /* gs355_header */
     size_t records;       /* f32[P][12]: px, py, conic_x, conic_y, conic_z, opacity, r, g, b, depth, reach_x, reach_y */
     size_t tiles_touched; /* u32[P] */
-    size_t rects;         /* u16[P][4] tile rectangle (x0, y0, x1, y1), all zero when culled */
+    size_t rects;         /* u64[P]    tiles the Gaussian is blended in, zero when there are none: its tile rectangle
+                           * (u16 x0, y0, x1, y1), or with GS355_STAGE_TILE_REACH a part of it (TileRegion in
+                           * gs355_internal.h) */
     size_t depth_bits;    /* u32[P]    view depth as raw bits (written for survivors only) */
     size_t offsets;       /* u32[P]   inclusive prefix sum of tiles_touched */
     size_t scan_tmp;      /* u32[...] block sums of the scans */
@@ -141,7 +144,8 @@ typedef struct gs355_layout {
                            * then u64[ceil(tiles/64)], the first slot of each block of 64 tiles, and
                            * u32[ceil(tiles/16)+1], the work list of the scatter's second level, and
                            * u32[ceil(tiles/64)], buckets per larger sorter size class in each block of 64 tiles */
-    size_t bin_visible;   /* u32[slices]     visible Gaussians per slice */
+    size_t bin_visible;   /* {u64, u32, u32}[slices]  keys and visible Gaussians of each slice's share of what follows,
+                           * {u32, u32}[ceil(P/64)]   keys and visible Gaussians per 64 Gaussians */
     size_t tile_lists;    /* u32[8+4*tiles]  counts, work counters and lists of the buckets of each larger sorter size class */
     size_t total_bytes;
     int32_t unsorted_buffer; /* which keys/values buffer the duplicate stage writes (0) */
@@ -186,6 +190,12 @@ enum {
     GS355_STAGE_TILESORT_SKIP_1 = 4096,
     GS355_STAGE_TILESORT_SKIP_2 = 8192,
     GS355_STAGE_TILESORT_SKIP_3 = 16384,
+    /* Modifier of PREPROCESS, for the tile-bucketed stages: a Gaussian gets keys only for those tiles of its rectangle
+     * that its alpha >= 1/255 ellipse reaches.  The blend and the backward pass would take the `alpha < 1/255` branch for
+     * every pixel of the other tiles, so images and gradients are the same bits; sorted keys, values and ranges are those
+     * of the remaining keys.  num_keys_total, and with it the overflow of a capacity, still count whole rectangles.
+     * Refused together with a classic stage.  No effect beyond 32767 tiles along an axis. */
+    GS355_STAGE_TILE_REACH = 65536,
     GS355_PIPELINE_FAST = 1 | 128 | 512 | 256 | 32
 };
 

@@ -21,6 +21,7 @@ STAGE_TILE_SCATTER_TWO_LEVEL = 1024  # modifiers of STAGE_TILE_SCATTER: name the
 STAGE_TILE_SCATTER_ONE_LEVEL = 2048  # choose by the key count (which launches both)
 TWO_LEVEL_MIN_KEYS = 6 << 20         # the device's own threshold
 STAGE_TILESORT_SKIP = (4096, 8192, 16384)  # modifiers of STAGE_TILESORT: do not launch that size class's sorter
+STAGE_TILE_REACH = 65536  # modifier of STAGE_PREPROCESS: keys only for the tiles that a Gaussian's alpha >= 1/255 ellipse reaches
 PIPELINE_FAST = STAGE_PREPROCESS | STAGE_TILE_COUNT | STAGE_TILE_SCATTER | STAGE_TILESORT | STAGE_BLEND
 MAX_FAST_TILES = 36000 * 16  # limits of the tile-bucketed stages (the classic stages have neither)
 MAX_FAST_GAUSSIANS = 1 << 28

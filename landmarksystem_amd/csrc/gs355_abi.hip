@@ -29,10 +29,11 @@ namespace {
 constexpr size_t kAlign = 256;
 constexpr uint32_t kKnownStages = GS355_STAGE_ALL | GS355_STAGE_BLEND_PLAIN | GS355_STAGE_TILE_COUNT | GS355_STAGE_TILESORT | GS355_STAGE_TILE_SCATTER |
                                   GS355_STAGE_TILE_SCATTER_TWO_LEVEL | GS355_STAGE_TILE_SCATTER_ONE_LEVEL |
-                                  GS355_STAGE_TILESORT_SKIP_1 | GS355_STAGE_TILESORT_SKIP_2 | GS355_STAGE_TILESORT_SKIP_3;
+                                  GS355_STAGE_TILESORT_SKIP_1 | GS355_STAGE_TILESORT_SKIP_2 | GS355_STAGE_TILESORT_SKIP_3 |
+                                  GS355_STAGE_TILE_REACH;
 constexpr uint32_t kScatterModifiers = GS355_STAGE_TILE_SCATTER_TWO_LEVEL | GS355_STAGE_TILE_SCATTER_ONE_LEVEL;
 constexpr uint32_t kStageModifiers =
-    kScatterModifiers | GS355_STAGE_TILESORT_SKIP_1 | GS355_STAGE_TILESORT_SKIP_2 | GS355_STAGE_TILESORT_SKIP_3;
+    kScatterModifiers | GS355_STAGE_TILESORT_SKIP_1 | GS355_STAGE_TILESORT_SKIP_2 | GS355_STAGE_TILESORT_SKIP_3 | GS355_STAGE_TILE_REACH;
 constexpr int64_t kMaxKeys = (1ll << 32) - 1 - kSortTile;  // key slots are indexed with u32
 
 size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
@@ -93,7 +94,7 @@ int make_layout(int32_t P, int64_t n_cap, int32_t W, int32_t H, gs355_layout* L)
     L->ranges = take(tiles * 2 * sizeof(uint32_t));
     L->bin_matrix = take((tiles <= (size_t)kBinMaxTilesWide ? bin_matrix_words(tiles) : 0) * sizeof(uint32_t));
     L->tile_base = take((2 * tiles + 3 * ((tiles + 63) / 64) + (tiles + kCoarseTiles - 1) / kCoarseTiles + 1) * sizeof(uint32_t));
-    L->bin_visible = take((size_t)kBinMaxGroups * sizeof(uint32_t));
+    L->bin_visible = take((size_t)kBinMaxGroups * sizeof(SliceTotals) + wave_totals_count(P) * sizeof(uint2));
     L->tile_lists = take((kListHeader + 4 * tiles) * sizeof(uint32_t));
     L->total_bytes = off;
     L->sort_bits = 32 + ceil_log2((uint32_t)tiles);
@@ -198,6 +199,8 @@ FrameArgs make_args(const gs355_frame* f)
     a.campos = f->campos;
     a.bg = f->bg;
     a.p_device = nullptr;
+    a.plain_regions = a.grid_x > 32767 || a.grid_y > 32767;
+    a.tile_reach = 0;
     return a;
 }
 
@@ -226,6 +229,10 @@ static int check_stages(const gs355_frame* frame, const gs355_gaussians* g, cons
     if ((stage_mask & ~kKnownStages) != 0 || (stage_mask & ~kStageModifiers) == 0 ||
         (stage_mask & kScatterModifiers) == kScatterModifiers)
         return set_error(GS355_EINVAL, "stage_mask 0x%x selects no known stage", stage_mask);
+    if ((stage_mask & GS355_STAGE_TILE_REACH) &&
+        (stage_mask & (GS355_STAGE_SCAN | GS355_STAGE_DUPLICATE | GS355_STAGE_SORT | GS355_STAGE_RANGES)))
+        return set_error(GS355_EINVAL, "stage_mask 0x%x: the classic stages make the keys of whole rectangles (no TILE_REACH)",
+                         stage_mask);
     if ((rc = check_frame(frame, true))) return rc;
     if ((rc = check_geometry_inputs(g))) return rc;
     if ((rc = check_colour_inputs(frame, g))) return rc;
@@ -271,21 +278,23 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
     auto* ranges = reinterpret_cast<uint32_t*>(ws + L.ranges);
     auto* bin_matrix = reinterpret_cast<uint32_t*>(ws + L.bin_matrix);
     auto* tile_base = reinterpret_cast<uint32_t*>(ws + L.tile_base);
-    auto* bin_visible = reinterpret_cast<uint32_t*>(ws + L.bin_visible);
+    auto* slice_totals = reinterpret_cast<SliceTotals*>(ws + L.bin_visible);
+    auto* wave_totals = reinterpret_cast<uint2*>(slice_totals + kBinMaxGroups);
     auto* tile_lists = reinterpret_cast<uint32_t*>(ws + L.tile_lists);
     hipStream_t s = static_cast<hipStream_t>(stream);
     FrameArgs fa = make_args(frame);
     fa.p_device = g->P_device;
+    fa.tile_reach = (stage_mask & GS355_STAGE_TILE_REACH) && !fa.plain_regions;
     const uint32_t cap = (uint32_t)n_cap;
 
     if (stage_mask & GS355_STAGE_PREPROCESS)
-        if ((rc = launch_preprocess(fa, *g, par, false, records, touched, rects, depth_bits, out->radii, s))) return rc;
+        if ((rc = launch_preprocess(fa, *g, par, false, records, touched, rects, depth_bits, wave_totals, out->radii, s))) return rc;
     if (stage_mask & GS355_STAGE_SCAN)
         if ((rc = launch_scan_offsets(touched, out->radii, g->P, g->P_device, offsets, scan_tmp, header,
                                       static_cast<gs355_header*>(out->header_copy), cap, s)))
             return rc;
     if (stage_mask & GS355_STAGE_DUPLICATE)
-        if ((rc = launch_duplicate(fa, g->P, records, out->radii, offsets, header, keys[0], vals[0], s))) return rc;
+        if ((rc = launch_duplicate(fa, g->P, records, out->radii, offsets, header, keys[0], vals[0], rects, s))) return rc;
     if (stage_mask & GS355_STAGE_SORT)
         if ((rc = launch_sort(header, cap, L.sort_passes, keys[0], keys[1], vals[0], vals[1], hist, scan_tmp, s)))
             return rc;
@@ -295,15 +304,15 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
     const int tiles = fa.grid_x * fa.grid_y;
     uint64_t* buckets = keys[1 - L.sorted_buffer];
     if (stage_mask & GS355_STAGE_TILE_COUNT) {
-        if ((rc = launch_tile_count(fa, g->P, rects, bin_matrix, bin_visible, s))) return rc;
-        if ((rc = launch_tile_layout(g->P, bin_matrix, bin_visible, tiles, cap, header,
+        if ((rc = launch_tile_count(fa, g->P, rects, records, wave_totals, bin_matrix, slice_totals, s))) return rc;
+        if ((rc = launch_tile_layout(g->P, bin_matrix, slice_totals, tiles, cap, header,
                                      static_cast<gs355_header*>(out->header_copy), tile_base, ranges, tile_lists,
                                      s)))
             return rc;
     }
     if (stage_mask & GS355_STAGE_TILE_SCATTER)
         // (the buffer the sorted keys will go to is free until the sort: it holds the coarse level of the scatter)
-        if ((rc = launch_tile_scatter(fa, g->P, rects, depth_bits, header, bin_matrix, bin_visible, cap, tile_base, ranges,
+        if ((rc = launch_tile_scatter(fa, g->P, rects, records, depth_bits, header, bin_matrix, cap, tile_base, ranges,
                                       tile_lists, buckets, keys[L.sorted_buffer],
                                       (stage_mask & GS355_STAGE_TILE_SCATTER_TWO_LEVEL)   ? 2
                                       : (stage_mask & GS355_STAGE_TILE_SCATTER_ONE_LEVEL) ? 1
@@ -351,7 +360,7 @@ int gs355_render_frame(const gs355_frame* frame, const gs355_gaussians* g, int32
                        const float* features_rest, void* workspace, size_t workspace_bytes, int64_t n_cap,
                        const gs355_outputs* out, uint32_t stage_mask, void* stream)
 {
-    constexpr uint32_t kFront = GS355_STAGE_PREPROCESS | GS355_STAGE_SCAN | GS355_STAGE_TILE_COUNT;
+    constexpr uint32_t kFront = GS355_STAGE_PREPROCESS | GS355_STAGE_TILE_REACH | GS355_STAGE_SCAN | GS355_STAGE_TILE_COUNT;
     if (!out) return set_error(GS355_EINVAL, "outputs is NULL");
     if (!out->header_copy) return set_error(GS355_EINVAL, "outputs.header_copy is NULL (the header is what the call waits for)");
     if (!(stage_mask & (GS355_STAGE_SCAN | GS355_STAGE_TILE_COUNT)) || !(stage_mask & ~(kFront | kStageModifiers)))
@@ -393,7 +402,7 @@ int gs355_visible_filter(const gs355_frame* frame, const gs355_gaussians* g, int
     if (g->P > 0 && !radii) return set_error(GS355_EINVAL, "radii is NULL");
     if (g->P_device) return set_error(GS355_EINVAL, "visible_filter does not take a device-side Gaussian count");
     const FrameArgs fa = make_args(frame);
-    return launch_preprocess(fa, *g, nullptr, true, nullptr, nullptr, nullptr, nullptr, radii, static_cast<hipStream_t>(stream));
+    return launch_preprocess(fa, *g, nullptr, true, nullptr, nullptr, nullptr, nullptr, nullptr, radii, static_cast<hipStream_t>(stream));
 }
 
 namespace {

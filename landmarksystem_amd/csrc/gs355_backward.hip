@@ -4,7 +4,7 @@
 // encodings/gaussian_encoding.py:729-743).
 //
 // Kernels over the forward pass's workspace (records, sorted values, ranges), in their order:
-//   record_slots     where each Gaussian's records of the next kernel go: one per tile of its rectangle, side by side
+//   record_slots     where each Gaussian's records of the next kernel go: one per tile number of its region, side by side
 //   blend_backward   per 16x16 tile, the forward blend's walk repeated FRONT TO BACK with the same per-block
 //                    lists and the same per-pair decisions.  With f_i = colour_i . dL/dpixel, w_i = alpha_i T_i,
 //                    prefix P_i = sum_{j<=i} w_j f_j and R = out_pixel . dL/dpixel - T_final dL/dalpha_out (all
@@ -13,7 +13,7 @@
 //                    over the 16 pixels of a block four list entries at a time, added to the wavefront's own sums of
 //                    the staged Gaussians in LDS (no atomics), and written once per batch of 64 as one 48-byte
 //                    record per (tile, Gaussian) key.  No global atomics (they cost more than the rest of the
-//                    kernel): the records of a Gaussian are consecutive, in the order its tile rectangle is
+//                    kernel): the records of a Gaussian are consecutive, in the order its tile region is
 //                    walked, and are summed in that order, so gradients are identical from run to run.
 //   sum_large        (scenes of up to 262144 Gaussians) the records of Gaussians of many tiles, summed by many lanes
 //   preprocess_backward  per Gaussian: conic -> 2-D covariance -> Jacobian / 3-D covariance -> scale, rotation,
@@ -30,21 +30,24 @@ namespace {
 
 constexpr int kKeyFloats = GS355_KEY_GRAD_FLOATS;  // per-key record: dpx, dpy, dconic xyz, dopacity, drgb, ddepth, 2 unused
 
-// Where a Gaussian's records lie: those of its tile rectangle, row by row, from some first slot on.  The blend needs the
-// slot of one tile (tx, ty) per key: base + ty * width + tx with base = first - y0 * width - x0 (modulo 2^32), eight bytes
-// from one place (first slot and rectangle took two cache lines per key, of the four to five that a key costs: blend
+// Where a Gaussian's records lie: those of its tile region (TileRegion), by tile number, from some first slot on.  The blend
+// needs the slot of one tile (tx, ty) per key: base + ty * width + tx with base = first - y0 * width - x0 (modulo 2^32),
+// eight bytes from one place (first slot and rectangle took two cache lines per key, of the four to five that a key costs: blend
 // backward 1109 -> 1013 us at 6M Gaussians, 1080p).
 struct RecordSlots {
     uint32_t base, width;
 };
+// The records of a region: slot first + e for tile number e of n, of the tiles the region holds (the others have no key, and
+// their slots are not written).
 struct RecordRun {
-    uint32_t first, n;
+    uint32_t first, n, mask;
+    bool masked, spans;
+    __device__ __forceinline__ uint32_t keys() const { return masked ? (uint32_t)__popc(mask) : n; }  // (an upper bound with spans)
 };
-__device__ __forceinline__ uint32_t rect_width(uint64_t rect) { return ((uint32_t)(rect >> 32) & 0xffffu) - ((uint32_t)rect & 0xffffu); }
-__device__ __forceinline__ RecordRun record_run(RecordSlots s, uint64_t rect)
+__device__ __forceinline__ RecordRun record_run(RecordSlots s, const TileRegion& q)
 {
-    const uint32_t x0 = (uint32_t)rect & 0xffffu, y0 = (uint32_t)(rect >> 16) & 0xffffu, y1 = (uint32_t)(rect >> 48);
-    return {s.base + y0 * s.width + x0, (y1 - y0) * s.width};
+    if (s.width == 0u) return {0u, 0u, 0u, false, false};  // no tiles, or a frame that overflowed
+    return {s.base + (uint32_t)q.y0 * s.width + (uint32_t)q.x0, (uint32_t)q.area, q.mask, q.masked, q.spans};
 }
 
 // Slots of all Gaussians: a workgroup adds up the rectangles of its 8192 Gaussians and takes that many slots from one
@@ -52,7 +55,7 @@ __device__ __forceinline__ RecordRun record_run(RecordSlots s, uint64_t rect)
 // workgroup gets which slots varies between runs, the order of a Gaussian's own records does not, and nothing else enters
 // a sum.  A frame that overflowed its capacity has no records, and no room for them: no Gaussian has slots.
 constexpr int kSlotItems = 8, kSlotThreads = 1024;
-__global__ __launch_bounds__(kSlotThreads) void record_slots_kernel(int P, const gs355_header* __restrict__ header,
+__global__ __launch_bounds__(kSlotThreads) void record_slots_kernel(int P, bool plain, const gs355_header* __restrict__ header,
                                                                     const uint64_t* __restrict__ rects,
                                                                     uint32_t* __restrict__ next,
                                                                     RecordSlots* __restrict__ slots)
@@ -66,7 +69,7 @@ __global__ __launch_bounds__(kSlotThreads) void record_slots_kernel(int P, const
     for (int k = 0; k < kSlotItems; ++k) rect[k] = first + k * kSlotThreads < end ? rects[first + k * kSlotThreads] : 0ull;
     uint32_t sum = 0;
 #pragma unroll
-    for (int k = 0; k < kSlotItems; ++k) sum += record_run({0u, rect_width(rect[k])}, rect[k]).n;
+    for (int k = 0; k < kSlotItems; ++k) sum += (uint32_t)TileRegion(rect[k], plain).area;
     uint32_t inc = sum;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -86,8 +89,9 @@ __global__ __launch_bounds__(kSlotThreads) void record_slots_kernel(int P, const
     uint32_t at = s_first + before + inc - sum;
 #pragma unroll
     for (int k = 0; k < kSlotItems; ++k) {
-        const uint32_t width = rect_width(rect[k]);
-        const RecordRun run = record_run({0u, width}, rect[k]);  // (its first: the slot of the rectangle's corner)
+        const TileRegion q(rect[k], plain);
+        const uint32_t width = (uint32_t)q.width;
+        const RecordRun run = record_run({0u, width}, q);  // (its first: the slot of the region's corner)
         if (first + k * kSlotThreads < P) slots[first + k * kSlotThreads] = {at - run.first, width};
         at += run.n;
     }
@@ -442,32 +446,48 @@ constexpr int kShStride = 52;  // floats per Gaussian in the SH staging area (16
 // (48 bytes), five records side by side and four such rounds in flight, and the partial sums meet in LDS.
 constexpr uint32_t kSerialRecords = 8;
 // Scenes of few Gaussians leave most of the chip idle even so (a wavefront per 64 Gaussians): up to this many, a kernel
-// of its own gives every Gaussian of more than kSerialRecords keys a wavefront and leaves the sum in its first record
+// of its own gives every Gaussian of more than kSerialRecords keys a wavefront and leaves the sum in its first slot
 // (100k Gaussians: 112 -> 67 us for both kernels).  Beyond, the launch of a wavefront per Gaussian costs more.
 constexpr int kSumAheadMax = 1 << 18;
 constexpr int kPartials = 4 * 15;  // float4 of LDS per wavefront
 
+// (spans: how many of the tile numbers are keys is not known without evaluating them, and there are more than a few)
+__device__ __forceinline__ bool summed_ahead(const RecordRun& run) { return run.spans || run.keys() > kSerialRecords; }
+
+__device__ __forceinline__ TileSpans spans_of(const TileRegion& q, const float* __restrict__ splats, size_t i)
+{
+    TileSpans s;
+    if (q.spans) s = TileSpans(splats + i * kRecordFloats, q.x0, q.y0);
+    return s;
+}
+
 __device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 
-__device__ __forceinline__ void sum_records(const float* __restrict__ key_grads, uint32_t n, uint32_t first,
-                                            float4* __restrict__ partial, float4& A0, float4& A1, float4& A2)
+__device__ __forceinline__ void sum_records(const float* __restrict__ key_grads, const RecordRun run, uint64_t region, bool plain,
+                                            const float* __restrict__ splats, size_t index, float4* __restrict__ partial, float4& A0, float4& A1, float4& A2)
 {
     const int lane = threadIdx.x & 63, group = lane >> 4, sub = lane & 15;
     const float4* __restrict__ records = reinterpret_cast<const float4*>(key_grads);
     A0 = A1 = A2 = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (n <= kSerialRecords) {
-        const float4* __restrict__ rec = records + (size_t)first * (kKeyFloats / 4);
-        for (uint32_t k0 = 0; k0 < n; k0 += 4) {
+    const uint32_t n = run.n;
+    const bool serial = !summed_ahead(run);
+    if (serial) {
+        const float4* __restrict__ rec = records + (size_t)run.first * (kKeyFloats / 4);
+        const uint32_t keys = run.keys();
+        uint32_t left = run.masked ? run.mask : (1u << n) - 1u, last = 0;
+        for (uint32_t k0 = 0; k0 < keys; k0 += 4) {
             float4 r[4][3];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const size_t k = min(k0 + (uint32_t)u, n - 1);
+                last = left != 0u ? (uint32_t)__builtin_ctz(left) : last;
+                left &= left - 1u;  // (0 stays 0)
+                const size_t k = last;
 #pragma unroll
                 for (int q = 0; q < 3; ++q) r[u][q] = rec[3 * k + q];
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                if (k0 + (uint32_t)u < n) {
+                if (k0 + (uint32_t)u < keys) {
                     A0 = add4(A0, r[u][0]);
                     A1 = add4(A1, r[u][1]);
                     A2 = add4(A2, r[u][2]);
@@ -475,7 +495,7 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
             }
         }
     }
-    uint64_t left = __ballot(n > kSerialRecords);
+    uint64_t left = __ballot(!serial);
     const int slot = sub / 3, part = sub % 3;  // (lane 15 of a group has no part)
     while (left != 0ull) {
         int lane_of[4], mine = -1;  // the lanes whose Gaussians the four groups take
@@ -486,8 +506,17 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
             mine = group == g ? lane_of[g] : mine;
         }
         const uint32_t n_of = (uint32_t)__shfl((int)n, max(mine, 0), 64);
-        const uint32_t first_of = (uint32_t)__shfl((int)first, max(mine, 0), 64);
+        const uint32_t first_of = (uint32_t)__shfl((int)run.first, max(mine, 0), 64);
         const uint32_t n_mine = mine < 0 || sub == 15 ? 0u : n_of;
+        const uint64_t region_of = (uint64_t)__shfl((long long)region, max(mine, 0), 64);
+        const TileRegion q(region_of, plain);
+        const TileSpans spans = spans_of(q, splats, (size_t)__shfl((long long)index, max(mine, 0), 64));
+        auto held = [&](uint32_t k) {
+            if (k >= n_mine) return false;
+            int row, col;
+            q.place((int)k, row, col);
+            return q.holds((int)k, row, col, spans);
+        };
         const float4* __restrict__ rec = records + (size_t)first_of * (kKeyFloats / 4) + part;
         float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
         for (uint32_t k0 = (uint32_t)slot; k0 < n_mine; k0 += 20) {
@@ -496,7 +525,7 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
             for (int u = 0; u < 4; ++u) r[u] = rec[3 * (size_t)min(k0 + 5u * (uint32_t)u, n_mine - 1)];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                if (k0 + 5u * (uint32_t)u < n_mine) sum = add4(sum, r[u]);
+                if (held(k0 + 5u * (uint32_t)u)) sum = add4(sum, r[u]);
         }
         if (sub < 15) partial[15 * group + sub] = sum;
         wave_lds_sync();
@@ -517,24 +546,29 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
 // Sixteen records side by side, three lanes each, three such rounds per step; the first record is overwritten once all
 // of them have been read (its new value depends on every one).  A wavefront takes eight Gaussians and requests the next
 // step, of the same Gaussian or the next, before it adds the current one: with one Gaussian a wavefront, every one of them
-// waited for its rectangle and then for its records, 47 us for 100k Gaussians of some 20 records each; now 35 (18 is what
-// reading them takes).
+// waited for its rectangle and then for its records, 47 us for 100k Gaussians of some 20 records each; then 35 (18 was what
+// reading them took).  Regions leave out half of those records and the others are looked up in a span: 40.
 constexpr int kSumPerWave = 8;
-__global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __restrict__ radii,
+__global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const int32_t* __restrict__ radii,
+                                                        const float* __restrict__ splats,
                                                         const uint64_t* __restrict__ rects,
                                                         const RecordSlots* __restrict__ slots, float* key_grads)
 {
-    const int lane = threadIdx.x & 63, i0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kSumPerWave;
+    const int lane = threadIdx.x & 63;
+    const int i0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * kSumPerWave);
     const int i = min(i0 + (lane & (kSumPerWave - 1)), P - 1);
     const int32_t radius = radii[i];
-    const RecordRun run = record_run(slots[i], rects[i]);
-    uint32_t left = (uint32_t)__ballot(lane < kSumPerWave && i0 + lane < P && radius > 0 && run.n > kSerialRecords);
+    const uint64_t region = rects[i];
+    const RecordRun run = record_run(slots[i], TileRegion(region, plain));
+    uint32_t left = (uint32_t)__ballot(lane < kSumPerWave && i0 + lane < P && radius > 0 && summed_ahead(run));
     if (left == 0u) return;
     const int slot = lane / 3, part = lane % 3;
     float4* const all = reinterpret_cast<float4*>(key_grads) + part;
     uint32_t first = 0, n = 0, k0 = 0;  // the current step: records k0 .. k0 + 47 of the n from `first`
+    int from = 0, from1 = 0;            // its Gaussian's lane, the next step's
     auto next = [&](uint32_t& f, uint32_t& m) {
         const int l = __builtin_ctz(left);
+        from1 = l;
         left &= left - 1u;
         f = (uint32_t)__builtin_amdgcn_readlane((int)run.first, l);
         m = (uint32_t)__builtin_amdgcn_readlane((int)run.n, l);
@@ -545,6 +579,7 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __
             r[u] = all[((size_t)f + min(k + (uint32_t)slot + 16u * (uint32_t)u, m - 1)) * (kKeyFloats / 4)];
     };
     next(first, n);
+    from = from1;
     float4 r[3], sum = make_float4(0.f, 0.f, 0.f, 0.f);
     request(first, n, k0, r);
     for (;;) {  // (uniform; ends with the last Gaussian's last step)
@@ -557,9 +592,18 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __
             k1 = 0;
         }
         if (more) request(first1, n1, k1, r1);
+        const TileRegion q((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)region, from) |
+                               ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(region >> 32), from) << 32),
+                           plain);  // (uniform, and so are its spans)
+        const TileSpans spans = spans_of(q, splats, (size_t)(i0 + from));
 #pragma unroll
-        for (int u = 0; u < 3; ++u)
-            if (slot < 16 && k0 + (uint32_t)slot + 16u * (uint32_t)u < n) sum = add4(sum, r[u]);
+        for (int u = 0; u < 3; ++u) {
+            const uint32_t k = k0 + (uint32_t)slot + 16u * (uint32_t)u;
+            if (slot >= 16 || k >= n) continue;
+            int row, col;
+            q.place((int)k, row, col);
+            if (q.holds((int)k, row, col, spans)) sum = add4(sum, r[u]);
+        }
         if (last) {
 #pragma unroll
             for (int d = 24; d >= 3; d >>= 1) {
@@ -567,11 +611,12 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, const int32_t* __
                                                  __shfl_down(sum.z, d, 64), __shfl_down(sum.w, d, 64));
                 sum = add4(sum, other);  // (lanes past the last slot hold zeros; sums other than the first slot's are not used)
             }
+            // (into the slot of the region's first record; a mask's first tile may be past number 0)
             if (slot == 0) all[(size_t)first * (kKeyFloats / 4)] = sum;
             sum = make_float4(0.f, 0.f, 0.f, 0.f);
         }
         if (!more) break;
-        first = first1, n = n1, k0 = k1;
+        first = first1, n = n1, k0 = k1, from = from1;
 #pragma unroll
         for (int u = 0; u < 3; ++u) r[u] = r1[u];
     }
@@ -619,9 +664,9 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
     float gcol[3] = {0.f, 0.f, 0.f};
     float nx = 0.f, ny = 0.f, nz = 0.f, inv_len = 0.f;
     int K = 0;
-    const RecordRun run = alive ? record_run(slots[si], rects[si]) : RecordRun{0u, 0u};
-    uint32_t n_keys = run.n;
-    if (summed && n_keys > kSerialRecords) n_keys = 1u;  // (sum_large_kernel has added them into the first)
+    const uint64_t region = alive ? rects[si] : 0ull;
+    RecordRun run = record_run(slots[si], TileRegion(region, f.plain_regions));
+    if (summed && summed_ahead(run)) run = {run.first, 1u, 0u, false, false};  // (sum_large_kernel has added them into the first)
     // kStored: the wavefront's rows as one run of float4, and the up to three floats behind the last whole one.  They
     // travel from memory to LDS without passing through registers, requested before anything else is waited for: held
     // in registers the 48 of them left two wavefronts per SIMD, requested later their latency came on top of the
@@ -657,7 +702,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
             for (int c = 0; c < 3; ++c) in_rgb[c] = records[si * kRecordFloats + 6 + c];
     }
     float4 A0, A1, A2;
-    sum_records(key_grads, n_keys, run.first, mine + kPartialsAt, A0, A1, A2);
+    sum_records(key_grads, run, region, f.plain_regions, records, si, mine + kPartialsAt, A0, A1, A2);
     if (alive) {
         const float* __restrict__ V = f.viewmatrix;
         const float* __restrict__ Pm = f.projmatrix;
@@ -975,7 +1020,7 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     if (rc) return rc;
     RecordSlots* slots = reinterpret_cast<RecordSlots*>(record_slots);
     hipLaunchKernelGGL(record_slots_kernel, dim3((g.P + kSlotThreads * kSlotItems - 1) / (kSlotThreads * kSlotItems)),
-                       dim3(kSlotThreads), 0, s, g.P, header, rects, next_slot, slots);
+                       dim3(kSlotThreads), 0, s, g.P, (bool)f.plain_regions, header, rects, next_slot, slots);
     GS355_CHECK_LAUNCH("record slots");
     const int tiles = f.grid_x * f.grid_y;
     auto blend = [&](auto kernel) {
@@ -993,7 +1038,7 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     const bool summed = g.P <= kSumAheadMax;
     if (summed) {
         hipLaunchKernelGGL(sum_large_kernel, dim3((g.P + 4 * kSumPerWave - 1) / (4 * kSumPerWave)), dim3(256), 0, s, g.P,
-                           in.radii, rects, slots, key_grads);
+                           (bool)f.plain_regions, in.radii, records, rects, slots, key_grads);
         GS355_CHECK_LAUNCH("record sums");
     }
     auto launch = [&](auto kernel, const ParameterArgs& p) {

@@ -24,8 +24,8 @@ namespace gs355 {
 
 namespace {
 
-// splats touching more tiles than this are queued and expanded by a wavefront each (8 and 16 measured slower, 64 and
-// 128 the same)
+// whole rectangles of more tiles than this, and all regions with spans, are queued and expanded by a wavefront each (8 and 16
+// measured slower, 64 and 128 the same)
 constexpr int kInlineTiles = 32;
 constexpr int kBinItems = 4;      // Gaussians per thread and round of the binning walk
 
@@ -49,24 +49,52 @@ __device__ __forceinline__ int lanes_per_gaussian(int per_group)
     return lanes;
 }
 
-struct TileRect {
-    int x0, y0, width, area;
-    float inv_width;
-    __device__ __forceinline__ explicit TileRect(uint64_t r)
-        : x0((int)(r & 0xFFFF)), y0((int)((r >> 16) & 0xFFFF)), width((int)((r >> 32) & 0xFFFF) - x0),
-          area(width * ((int)(r >> 48) - y0)), inv_width(__builtin_amdgcn_rcpf((float)width))
-    {
+// A share of a region's tiles for each of `lanes` lanes (a power of two), this one the `sub`-th; `record`: the Gaussian's.
+// Of a region with spans a lane takes whole rows, or several lanes one where there are more lanes than rows: a row's span
+// costs some 30 instructions, too many to evaluate for every tile (100k large splats: count 24.3, scatter 27.0 us by tile, 12.2 and 18.0 by row).
+template <typename Visit>
+__device__ __forceinline__ void walk_region(const TileRegion& q, const float* __restrict__ record, int sub, int lanes, int grid_x,
+                                            Visit visit)
+{
+    if (q.spans) {
+        const TileSpans s(record, q.x0, q.y0);
+        const int rows = q.area / q.width;
+        int share = lanes;  // lanes per row
+        while (share > 1 && lanes < rows * share) share >>= 1;
+        for (int row = sub / share; row < rows; row += lanes / share) {
+            int first, end;
+            s.columns(row, q.width, first, end);
+            const int t = q.tile(row, 0, grid_x);
+            for (int col = first + sub % share; col < end; col += share) visit(t + col);
+        }
+    } else {
+        for (int e = sub; e < q.area; e += lanes) {
+            int row, col;
+            q.place(e, row, col);
+            if (!q.masked || ((q.mask >> e) & 1u) != 0u) visit(q.tile(row, col, grid_x));
+        }
     }
-    // tile number e of the rectangle, row by row (the quotient by the reciprocal is off by one at most)
-    __device__ __forceinline__ int tile(int e, int grid_x) const
-    {
-        int row = (int)(((float)e + 0.5f) * inv_width);
-        int col = e - row * width;
-        if (col < 0) { --row; col += width; }
-        else if (col >= width) { ++row; col -= width; }
-        return (y0 + row) * grid_x + x0 + col;
+}
+
+// The runs [ta, tb) of consecutive tiles of a masked or whole region, a row at a time (a row of a mask is one run: the
+// ellipse is convex).
+template <typename Visit>
+__device__ __forceinline__ void walk_rows(const TileRegion& q, int grid_x, Visit visit)
+{
+    int t = q.y0 * grid_x + q.x0;
+    if (q.masked) {
+        const uint32_t row_bits = (1u << q.width) - 1u;
+        for (uint32_t m = q.mask; m != 0u; m >>= q.width, t += grid_x) {
+            const uint32_t row = m & row_bits;
+            if (row != 0u) {
+                const int first = t + __builtin_ctz(row);
+                visit(first, first + __popc(row));
+            }
+        }
+    } else {
+        for (int e = 0; e < q.area; e += q.width, t += grid_x) visit(t, t + q.width);
     }
-};
+}
 
 // ---------------------------------------------------------------------------
 // Counting.  Workgroup c owns Gaussians [c * per_group, (c+1) * per_group) and a private array of counters in LDS.
@@ -79,37 +107,69 @@ struct TileRect {
 template <bool kWide>
 __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, int32_t P, int per_group,
                                                                  const uint64_t* __restrict__ rects,
+                                                                 const float* __restrict__ records,
+                                                                 const uint2* __restrict__ wave_totals, int n_totals,
                                                                  uint32_t* __restrict__ matrix,
-                                                                 uint32_t* __restrict__ group_visible)
+                                                                 SliceTotals* __restrict__ slice_totals)
 {
     extern __shared__ uint32_t s_count[];  // [tiles], or [coarse bins] when kWide
     __shared__ uint32_t s_queue[kBinItems * kBinThreads];
     __shared__ uint32_t s_nqueue, s_visible;
+    __shared__ unsigned long long s_keys;
 
     if (f.p_device) {  // the slices follow the device-side count
         P = effective_count(f, P);
         per_group = slice_size(P, (int)gridDim.x);
+        n_totals = (P + 63) / 64;
     }
     const int T = f.grid_x * f.grid_y;
     const int counters = kWide ? (T + kCoarseTiles - 1) >> kCoarseShift : T;
     const int tid = threadIdx.x, c = blockIdx.x;
     for (int t = tid; t < counters; t += kBinThreads) s_count[t] = 0u;
-    if (tid == 0) s_visible = 0;
+    if (tid == 0) {
+        s_visible = 0;
+        s_keys = 0;
+        s_nqueue = 0;
+    }
+    __syncthreads();
+    {  // this workgroup's share of the preprocess's totals (any split serves: the layout adds the shares up)
+        const int per = (n_totals + (int)gridDim.x - 1) / (int)gridDim.x, end = min(n_totals, (c + 1) * per);
+        unsigned long long keys = 0;
+        uint32_t visible = 0;
+        for (int k = c * per + tid; k < end; k += kBinThreads) {
+            const uint2 v = wave_totals[k];
+            keys += v.x;
+            visible += v.y;
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            keys += __shfl_down(keys, d, 64);
+            visible += __shfl_down(visible, d, 64);
+        }
+        if ((tid & 63) == 0 && visible) {
+            atomicAdd(&s_keys, keys);
+            atomicAdd(&s_visible, visible);
+        }
+    }
     const int g_begin = min(P, c * per_group);
     const int g_end = min(P, g_begin + per_group);
-    uint32_t visible = 0;
     auto add = [&](int t) { atomicAdd(&s_count[kWide ? t >> kCoarseShift : t], 1u); };
     // large rectangles: one per wavefront at a time, 64 tiles per step (the sixteen wavefronts work on sixteen
     // rectangles side by side; the whole workgroup on one rectangle left most of its threads idle)
     auto walk_queue = [&]() {
         const uint32_t nq = s_nqueue;
         uint32_t k = (uint32_t)tid >> 6;
-        uint64_t next = k < nq ? rects[s_queue[k]] : 0ull;
+        uint32_t gi = k < nq ? s_queue[k] : 0u;
+        uint64_t next = k < nq ? rects[gi] : 0ull;
         while (k < nq) {
-            const TileRect q(next);
+            const TileRegion q(next, f.plain_regions);
+            const float* __restrict__ record = records + (size_t)gi * kRecordFloats;
             k += kBinThreads / 64;
-            if (k < nq) next = rects[s_queue[k]];
-            for (int e = tid & 63; e < q.area; e += 64) add(q.tile(e, f.grid_x));
+            if (k < nq) {
+                gi = s_queue[k];
+                next = rects[gi];
+            }
+            walk_region(q, record, tid & 63, 64, f.grid_x, add);
         }
     };
 
@@ -119,12 +179,11 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
         __syncthreads();
         const int i = g_begin + tid / lanes, sub = tid % lanes;
         if (i < g_end) {
-            const TileRect q(rects[i]);
-            if (sub == 0 && q.area > 0) ++visible;
+            const TileRegion q(rects[i], f.plain_regions);
             if (q.area > kInlineTiles * lanes) {
                 if (sub == 0) s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
             } else {
-                for (int e = sub; e < q.area; e += lanes) add(q.tile(e, f.grid_x));
+                walk_region(q, records + (size_t)i * kRecordFloats, sub, lanes, f.grid_x, add);
             }
         }
         __syncthreads();
@@ -151,28 +210,21 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
             for (int u = 0; u < kBinItems; ++u) {
                 const int i = base + u * kBinThreads + tid;
                 if (i < g_end) {
-                    const uint64_t r = rr[u];
-                    const int x0 = (int)(r & 0xFFFF), y0 = (int)((r >> 16) & 0xFFFF), x1 = (int)((r >> 32) & 0xFFFF),
-                              y1 = (int)(r >> 48);
-                    const int area = (x1 - x0) * (y1 - y0);
-                    if (area > 0) {
-                        ++visible;
-                        if (area > kInlineTiles) {
-                            s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
-                        } else if (kWide) {  // a rectangle row: one request per coarse bin it crosses
-                            for (int ty = y0; ty < y1; ++ty) {
-                                int ta = ty * f.grid_x + x0;
-                                const int tb = ty * f.grid_x + x1;
+                    const TileRegion q(rr[u], f.plain_regions);
+                    if (q.area > (q.spans ? 0 : kInlineTiles)) {
+                        s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
+                    } else {
+                        walk_rows(q, f.grid_x, [&](int ta, int tb) {
+                            if (kWide) {  // one request per coarse bin the run crosses
                                 while (ta < tb) {
                                     const int stop = min(tb, ((ta >> kCoarseShift) + 1) << kCoarseShift);
                                     atomicAdd(&s_count[ta >> kCoarseShift], (uint32_t)(stop - ta));
                                     ta = stop;
                                 }
+                            } else {
+                                for (; ta < tb; ++ta) add(ta);
                             }
-                        } else {
-                            for (int ty = y0; ty < y1; ++ty)
-                                for (int tx = x0; tx < x1; ++tx) add(ty * f.grid_x + tx);
-                        }
+                        });
                     }
                 }
             }
@@ -181,13 +233,10 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
             __syncthreads();
         }
     }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) visible += __shfl_down(visible, d, 64);
-    if ((tid & 63) == 0 && visible) atomicAdd(&s_visible, visible);
     __syncthreads();
     uint32_t* __restrict__ row = matrix + (size_t)c * counters;
     for (int t = tid; t < counters; t += kBinThreads) row[t] = s_count[t];
-    if (tid == 0) group_visible[c] = s_visible;
+    if (tid == 0) slice_totals[c] = {(uint64_t)s_keys, s_visible, 0u};
 }
 
 // ---------------------------------------------------------------------------
@@ -217,6 +266,7 @@ constexpr uint32_t kTwoLevelMinKeys = 6u << 20;
 template <int kShift, bool kWide>
 __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32_t P, int per_group,
                                                               const uint64_t* __restrict__ rects,
+                                                              const float* __restrict__ records,
                                                               const uint32_t* __restrict__ depth_bits,
                                                               const gs355_header* __restrict__ header,
                                                               uint32_t min_keys, uint32_t max_keys,
@@ -279,7 +329,8 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
         uint32_t k = wave, gi = k < nq ? s_queue[k] : 0u, depth = k < nq ? depth_bits[gi] : 0u;
         uint64_t next = k < nq ? rects[gi] : 0ull;
         while (k < nq) {
-            const TileRect q(next);
+            const TileRegion q(next, f.plain_regions);
+            const float* __restrict__ record = records + (size_t)gi * kRecordFloats;
             const uint64_t payload = payload_of(depth, gi);
             k += kBinThreads / 64;
             if (k < nq) {
@@ -287,7 +338,7 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
                 next = rects[gi];
                 depth = depth_bits[gi];
             }
-            for (int e = lane; e < q.area; e += 64) emit_tile(q.tile(e, f.grid_x), payload);
+            walk_region(q, record, lane, 64, f.grid_x, [&](int t) { emit_tile(t, payload); });
         }
     };
     const int lanes = lanes_per_gaussian(per_group);
@@ -296,12 +347,13 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
         __syncthreads();
         const int i = g_begin + tid / lanes, sub = tid % lanes;
         if (i < g_end) {
-            const TileRect q(rects[i]);
+            const TileRegion q(rects[i], f.plain_regions);
             const uint64_t payload = payload_of(depth_bits[i], (uint32_t)i);
             if (q.area > kInlineTiles * lanes) {
                 if (sub == 0) s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
             } else {
-                for (int e = sub; e < q.area; e += lanes) emit_tile(q.tile(e, f.grid_x), payload);
+                walk_region(q, records + (size_t)i * kRecordFloats, sub, lanes, f.grid_x,
+                            [&](int t) { emit_tile(t, payload); });
             }
         }
         __syncthreads();
@@ -324,15 +376,12 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
         for (int u = 0; u < kBinItems; ++u) {
             const int i = first + u * kBinThreads + tid;
             if (i < g_end) {
-                const uint64_t r = rr[u];
-                const int x0 = (int)(r & 0xFFFF), y0 = (int)((r >> 16) & 0xFFFF), x1 = (int)((r >> 32) & 0xFFFF),
-                          y1 = (int)(r >> 48);
-                const int area = (x1 - x0) * (y1 - y0);
-                if (area > kInlineTiles) {
+                const TileRegion q(rr[u], f.plain_regions);
+                if (q.area > (q.spans ? 0 : kInlineTiles)) {
                     s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
-                } else if (area > 0) {
+                } else {
                     const uint64_t payload = payload_of(dd[u], (uint32_t)i);
-                    for (int ty = y0; ty < y1; ++ty) emit_row(ty * f.grid_x + x0, ty * f.grid_x + x1, payload);
+                    walk_rows(q, f.grid_x, [&](int ta, int tb) { emit_row(ta, tb, payload); });
                 }
             }
         }
@@ -608,8 +657,8 @@ __global__ __launch_bounds__(64 * kPrefixParts) void slice_prefix_kernel(uint32_
 
 // Layout of the buckets from the tiles' totals: one wavefront per block of 64 tiles, four per workgroup.  Every
 // workgroup adds up the block totals itself (a few hundred words, at most 9000): those before its own blocks give its
-// first slot, all of them the frame's key count, which decides overflow before anything is published — so no
-// workgroup waits for another and no separate scan pass is launched.  Workgroup 0 also writes the frame header and
+// first slot, all of them the number of pairs; the slices' totals are the frame's key count, which decides overflow before
+// anything is published — so no workgroup waits for another and no separate scan pass is launched.  Workgroup 0 also writes the frame header and
 // the work list of the scatter's second level: chunk_base[b] = chunks of kFineChunk pairs in the coarse bins before
 // b, chunk_base[bins] = all (`bin_pairs`, the pairs per bin, may be the same array).  With kTiles the wavefronts
 // publish tile bases, the scatter's cursors, the ranges and the lists of buckets too large for the small sorter;
@@ -621,7 +670,7 @@ __global__ __launch_bounds__(64 * kPrefixParts) void slice_prefix_kernel(uint32_
 template <bool kTiles>
 __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* totals, uint32_t tiles,
                                                            const uint64_t* __restrict__ block_sums, uint32_t n_blocks,
-                                                           const uint32_t* __restrict__ group_visible, int groups,
+                                                           const SliceTotals* __restrict__ slice_totals, int groups,
                                                            uint32_t n_cap, gs355_header* __restrict__ header,
                                                            gs355_header* __restrict__ header_copy, bool header_known,
                                                            uint32_t* tile_base,
@@ -629,7 +678,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
                                                            const uint32_t* bin_pairs, int bins, uint32_t* chunk_base,
                                                            const uint32_t* __restrict__ block_classes)
 {
-    __shared__ uint64_t s_before[4], s_total[4], s_class_before[4], s_class_total[4];
+    __shared__ uint64_t s_before[4], s_total[4], s_class_before[4], s_class_total[4], s_keys[4];
     __shared__ uint32_t s_vis[4], s_chunks[4];
     if (header_known && header->overflow) return;
     // counts of the three classes, 21 bits each
@@ -653,13 +702,20 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
             }
         }
         uint32_t vis = 0;
-        if (blockIdx.x == 0 && !header_known)
-            for (int c = threadIdx.x; c < groups; c += 256) vis += group_visible[c];
+        uint64_t keys = 0;
+        if (!header_known) {
+            for (int c = threadIdx.x; c < groups; c += 256) {
+                const SliceTotals v = slice_totals[c];
+                vis += v.visible;
+                keys += v.keys;
+            }
+        }
 #pragma unroll
         for (int d = 32; d > 0; d >>= 1) {
             before += __shfl_down(before, d, 64);
             total += __shfl_down(total, d, 64);
             vis += __shfl_down(vis, d, 64);
+            keys += __shfl_down(keys, d, 64);
             class_before += __shfl_down(class_before, d, 64);
             class_total += __shfl_down(class_total, d, 64);
         }
@@ -667,15 +723,17 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
             s_before[wave] = before;
             s_total[wave] = total;
             s_vis[wave] = vis;
+            s_keys[wave] = keys;
             s_class_before[wave] = class_before;
             s_class_total[wave] = class_total;
         }
     }
     __syncthreads();
     const uint64_t total = (s_total[0] + s_total[1]) + (s_total[2] + s_total[3]);
-    const bool overflow = total > (uint64_t)n_cap;
+    const uint64_t keys = (s_keys[0] + s_keys[1]) + (s_keys[2] + s_keys[3]);  // of whole rectangles: at least `total`
+    const bool overflow = keys > (uint64_t)n_cap;
     if (blockIdx.x == 0 && threadIdx.x == 0 && !header_known) {
-        header->num_keys_total = total;
+        header->num_keys_total = keys;
         header->num_keys = overflow ? n_cap : (uint32_t)total;
         header->overflow = overflow ? 1u : 0u;
         header->num_visible = (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]);
@@ -685,7 +743,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         if (counted && kTiles)
             for (int c = 0; c < 3; ++c) lists[c] = class_count(in_class, c);
         if (header_copy) {
-            header_copy->num_keys_total = total;
+            header_copy->num_keys_total = keys;
             header_copy->num_keys = overflow ? n_cap : (uint32_t)total;
             header_copy->overflow = overflow ? 1u : 0u;
             header_copy->num_visible = (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]);
@@ -1469,20 +1527,21 @@ static inline uint32_t* chunk_bases(uint32_t* tile_base, int tiles)
     return tile_base + 2 * (size_t)tiles + 2 * (size_t)((tiles + 63) / 64);
 }
 
-int launch_tile_count(const FrameArgs& f, int32_t P, const uint64_t* rects, uint32_t* matrix, uint32_t* group_visible,
-                      hipStream_t s)
+int launch_tile_count(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint2* wave_totals,
+                      uint32_t* matrix, SliceTotals* slice_totals, hipStream_t s)
 {
     int per_group;
     const int groups = bin_groups(P, &per_group);
-    const int T = f.grid_x * f.grid_y;
+    const int T = f.grid_x * f.grid_y, n_totals = (int)wave_totals_count(P);
     int rc = allow_large_lds();
     if (rc) return rc;
     if (T <= kBinMaxTiles)
         hipLaunchKernelGGL(tile_count_kernel<false>, dim3(groups), dim3(kBinThreads), (size_t)T * sizeof(uint32_t), s, f,
-                           P, per_group, rects, matrix, group_visible);
+                           P, per_group, rects, records, wave_totals, n_totals, matrix, slice_totals);
     else
         hipLaunchKernelGGL(tile_count_kernel<true>, dim3(groups), dim3(kBinThreads),
-                           (size_t)coarse_bins(T) * sizeof(uint32_t), s, f, P, per_group, rects, matrix, group_visible);
+                           (size_t)coarse_bins(T) * sizeof(uint32_t), s, f, P, per_group, rects, records, wave_totals, n_totals,
+                           matrix, slice_totals);
     GS355_CHECK_LAUNCH("bin: count");
     return GS355_OK;
 }
@@ -1492,13 +1551,13 @@ int launch_tile_count(const FrameArgs& f, int32_t P, const uint64_t* rects, uint
 // already write bases).
 template <bool kTiles>
 static int launch_layout(const uint32_t* totals, uint32_t* bases, int columns, const uint64_t* blocks,
-                         const uint32_t* group_visible, int groups, uint32_t n_cap, gs355_header* header,
+                         const SliceTotals* slice_totals, int groups, uint32_t n_cap, gs355_header* header,
                          gs355_header* header_copy, bool header_known, uint32_t* ranges, uint32_t* lists, const uint32_t* bin_pairs, int bins,
                          uint32_t* chunk_base, const uint32_t* block_classes, hipStream_t s)
 {
     const int n_blocks = (columns + 63) / 64;
     hipLaunchKernelGGL(tile_publish_kernel<kTiles>, dim3((n_blocks + 3) / 4), dim3(256), 0, s, totals, (uint32_t)columns,
-                       blocks, (uint32_t)n_blocks, group_visible, groups, n_cap, header, header_copy, header_known, bases, ranges, lists,
+                       blocks, (uint32_t)n_blocks, slice_totals, groups, n_cap, header, header_copy, header_known, bases, ranges, lists,
                        bin_pairs, bins, chunk_base, block_classes);
     GS355_CHECK_LAUNCH("bin: layout");
     return GS355_OK;
@@ -1507,7 +1566,7 @@ static int launch_layout(const uint32_t* totals, uint32_t* bases, int columns, c
 // Up to kBinMaxTiles tiles: everything the later stages need (tile bases, cursors, ranges, size-class lists,
 // header).  Beyond: the header and the coarse bins' bases (in tile_cursor[0, bins)); the per-tile layout follows
 // in launch_tile_scatter once the pairs of each bin can be counted by tile.
-int launch_tile_layout(int32_t P, uint32_t* matrix, const uint32_t* group_visible, int tiles, uint32_t n_cap,
+int launch_tile_layout(int32_t P, uint32_t* matrix, const SliceTotals* slice_totals, int tiles, uint32_t n_cap,
                        gs355_header* header, gs355_header* header_copy, uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, hipStream_t s)
 {
     int per_group;
@@ -1521,7 +1580,7 @@ int launch_tile_layout(int32_t P, uint32_t* matrix, const uint32_t* group_visibl
         hipLaunchKernelGGL(slice_prefix_kernel, dim3((tiles + 63) / 64), dim3(64 * kPrefixParts), 0, s, matrix, groups, tiles,
                            tile_base, blocks, chunk_base, block_classes, lists);
         GS355_CHECK_LAUNCH("bin: slice prefix");
-        return launch_layout<true>(tile_base, tile_base, tiles, blocks, group_visible, groups, n_cap, header, header_copy, false, ranges,
+        return launch_layout<true>(tile_base, tile_base, tiles, blocks, slice_totals, groups, n_cap, header, header_copy, false, ranges,
                                    lists, chunk_base, bins, chunk_base, block_classes, s);
     }
     // (both in the cursor half of tile_base, which the tile-level layout of launch_tile_scatter overwrites later)
@@ -1530,12 +1589,12 @@ int launch_tile_layout(int32_t P, uint32_t* matrix, const uint32_t* group_visibl
     hipLaunchKernelGGL(slice_prefix_kernel, dim3((bins + 63) / 64), dim3(64 * kPrefixParts), 0, s, matrix, groups, bins, bin_pairs,
                        blocks, (uint32_t*)nullptr, (uint32_t*)nullptr, lists);
     GS355_CHECK_LAUNCH("bin: slice prefix");
-    return launch_layout<false>(bin_pairs, bin_base, bins, blocks, group_visible, groups, n_cap, header, header_copy, false, ranges,
+    return launch_layout<false>(bin_pairs, bin_base, bins, blocks, slice_totals, groups, n_cap, header, header_copy, false, ranges,
                                 lists, bin_pairs, bins, chunk_base, nullptr, s);
 }
 
-int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const uint32_t* depth_bits,
-                        gs355_header* header, const uint32_t* matrix, const uint32_t* group_visible, uint32_t n_cap,
+int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint32_t* depth_bits,
+                        gs355_header* header, const uint32_t* matrix, uint32_t n_cap,
                         uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, uint64_t* buckets, uint64_t* coarse,
                         int levels, hipStream_t s)
 {
@@ -1552,19 +1611,19 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
         if (levels != 2) {
             min_keys = levels == 1 ? UINT32_MAX : kTwoLevelMinKeys;
             hipLaunchKernelGGL((scatter_kernel<0, false>), dim3(groups), dim3(kBinThreads), (size_t)T * sizeof(uint32_t), s,
-                               f, P, per_group, rects, depth_bits, header, 0u, min_keys, matrix, tile_base, buckets);
+                               f, P, per_group, rects, records, depth_bits, header, 0u, min_keys, matrix, tile_base, buckets);
             GS355_CHECK_LAUNCH("bin: scatter");
         }
         fine = levels != 1;
         if (fine) {
             hipLaunchKernelGGL((scatter_kernel<kCoarseShift, false>), dim3(groups), dim3(kBinThreads), coarse_lds, s, f, P,
-                               per_group, rects, depth_bits, header, min_keys, UINT32_MAX, matrix, tile_base, coarse);
+                               per_group, rects, records, depth_bits, header, min_keys, UINT32_MAX, matrix, tile_base, coarse);
             GS355_CHECK_LAUNCH("bin: coarse scatter");
         }
     } else {
         const uint32_t* bin_base = tile_cursor;  // (replaced by the tiles' cursors once the coarse level is done)
         hipLaunchKernelGGL((scatter_kernel<kCoarseShift, true>), dim3(groups), dim3(kBinThreads), coarse_lds, s, f, P,
-                           per_group, rects, depth_bits, header, 0u, UINT32_MAX, matrix, bin_base, coarse);
+                           per_group, rects, records, depth_bits, header, 0u, UINT32_MAX, matrix, bin_base, coarse);
         GS355_CHECK_LAUNCH("bin: coarse scatter");
         uint64_t* blocks = reinterpret_cast<uint64_t*>(tile_base + 2 * (size_t)T);
         if ((rc = launch_fill_u32(tile_base, (size_t)T, 0u, s))) return rc;
@@ -1572,7 +1631,7 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
         hipLaunchKernelGGL(fine_count_kernel, dim3(kFineGrid), dim3(kFineThreads), 0, s, header, bin_base, bins, T,
                            chunk_bases(tile_base, T), coarse, tile_base, blocks, lists);
         GS355_CHECK_LAUNCH("bin: fine count");
-        if ((rc = launch_layout<true>(tile_base, tile_base, T, blocks, group_visible, groups, n_cap, header, nullptr, true, ranges,
+        if ((rc = launch_layout<true>(tile_base, tile_base, T, blocks, (const SliceTotals*)nullptr, groups, n_cap, header, nullptr, true, ranges,
                                       lists, (const uint32_t*)nullptr, 0, (uint32_t*)nullptr, nullptr, s)))
             return rc;
     }

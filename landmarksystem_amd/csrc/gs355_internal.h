@@ -34,6 +34,8 @@ struct FrameArgs {  // by-value kernel argument
     const float* campos;
     const float* bg;
     const uint32_t* p_device;  // optional device-side number of Gaussians (gs355_gaussians.P_device)
+    int32_t plain_regions;  // the grid is too large for flags in the tile regions' words (TileRegion)
+    int32_t tile_reach;     // preprocess: a Gaussian's region is the tiles its alpha >= 1/255 ellipse reaches
 };
 
 // Number of Gaussians a kernel processes: the host's P, or the device-side count when there is one.
@@ -151,6 +153,103 @@ struct TileReach {
     }
 };
 
+// The columns of tiles that the splat's alpha >= 1/255 ellipse can reach, for one row of tiles at a time: TileReach's span
+// with tiles in the place of blocks (the same formula, and the same slack).  Rows and columns count from tile (x0, y0).
+// Contraction is off: the kernels that count, place and sum the pairs of large splats each evaluate this and have to agree.
+struct TileSpans {
+    float rho = 0.f, across = 0.f, slack = 0.f, rx = 0.f, x = 0.f, y = 0.f, inv_y = 0.f;
+
+    TileSpans() = default;
+    __device__ __forceinline__ TileSpans(float px, float py, float conic_x, float conic_y, float conic_z, float reach_x,
+                                         float reach_y, int x0, int y0)
+    {
+#pragma clang fp contract(off)
+        inv_y = __builtin_amdgcn_rcpf(reach_y);
+        rho = fmaxf(-1.0f, fminf(1.0f, -conic_y * __builtin_amdgcn_rsqf(conic_x * conic_z)));
+        across = __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - rho * rho) + 1e-5f);
+        slack = reach_x * (0.02f * inv_y + 0.002f) + 0.01f;
+        rx = reach_x;
+        x = px - (float)(x0 * kTile);
+        y = py - (float)(y0 * kTile);
+    }
+    // from a Gaussian's record
+    __device__ __forceinline__ TileSpans(const float* __restrict__ record, int x0, int y0)
+        : TileSpans(record[0], record[1], record[2], record[3], record[4], record[10], record[11], x0, y0)
+    {
+    }
+
+    // Integers in [0, n] around the pixel interval [lo, hi] from the corner: first tile that ends at or behind lo, one
+    // past the last that begins before or at hi (pixel centres are integers, a tile's last one is its first plus 15).
+    static __device__ __forceinline__ void tiles_of(float lo, float hi, int n, int& first, int& end)
+    {
+#pragma clang fp contract(off)
+        first = (int)__builtin_amdgcn_fmed3f(lo * 0.0625f + 0.0624f, 0.0f, (float)n);
+        end = (int)__builtin_amdgcn_fmed3f(hi * 0.0625f + 1.0f, 0.0f, (float)n);
+    }
+
+    // columns [first, end) of the `width` tiles of row `row` (first >= end: none)
+    __device__ __forceinline__ void columns(int row, int width, int& first, int& end) const
+    {
+#pragma clang fp contract(off)
+        const float top = (float)(row * kTile) - y;
+        const float t0 = __builtin_amdgcn_fmed3f(top * inv_y, -1.0f, 1.0f);
+        const float t1 = __builtin_amdgcn_fmed3f((top + (float)(kTile - 1)) * inv_y, -1.0f, 1.0f);
+        const float up = __builtin_amdgcn_fmed3f(rho, t0, t1), down = __builtin_amdgcn_fmed3f(-rho, t0, t1);
+        const float half_up = __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - up * up));
+        const float half_down = __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - down * down));
+        const float hi = x + (rx * (rho * up + across * half_up) + slack);
+        const float lo = x + (rx * (rho * down - across * half_down) - slack);
+        tiles_of(lo, hi, width, first, end);
+    }
+};
+
+// The tiles a Gaussian is blended in, as the word that the preprocess leaves per Gaussian (zero: none):
+//   whole     x0 | y0 << 16 | x1 << 32 | y1 << 48       every tile of the rectangle
+//   spans     the same with bit 47 set                  of the rectangle's tiles those inside the ellipse (TileSpans)
+//   masked    x0 | y0 << 16 | mask << 32 | (width - 1) << 60 | 1 << 63
+//                                                       of at most 28 tiles, at most 8 side by side, those in the mask
+// Tiles of a region are numbered row by row over its rectangle, from its first row with a tile to its last.  A grid of more
+// than 32767 tiles along an axis needs the flags' bits for coordinates: its regions are whole (`plain`).
+// 6M Gaussians at 1080p reach 73 % of their rectangles' tiles and nearly all of their regions are masked; of 1M large
+// splats 48 %, in spans a fifth.
+constexpr int kMaskTiles = 28, kMaskWidth = 8;
+struct TileRegion {
+    int x0, y0, width, area;  // area: tile numbers in use (of a masked region up to its last tile)
+    uint32_t mask;
+    bool masked, spans;
+
+    __device__ __forceinline__ TileRegion(uint64_t word, bool plain)
+    {
+        const uint32_t low = (uint32_t)word, high = (uint32_t)(word >> 32);
+        x0 = (int)(low & 0xFFFFu);
+        y0 = (int)(low >> 16);
+        masked = !plain && (high >> 31) != 0u;
+        spans = !plain && !masked && (high & 0x8000u) != 0u;
+        mask = masked ? high & ((1u << kMaskTiles) - 1u) : 0u;
+        const int x1 = (int)(high & (spans ? 0x7FFFu : 0xFFFFu)), y1 = (int)(high >> 16);
+        width = masked ? (int)((high >> 28) & 7u) + 1 : x1 - x0;
+        area = masked ? 32 - __clz((int)mask) : width * (y1 - y0);
+    }
+    // row and column of tile number e (the quotient by the reciprocal is off by one at most)
+    __device__ __forceinline__ void place(int e, int& row, int& col) const
+    {
+        row = (int)(((float)e + 0.5f) * __builtin_amdgcn_rcpf((float)width));
+        col = e - row * width;
+        if (col < 0) { --row; col += width; }
+        else if (col >= width) { ++row; col -= width; }
+    }
+    __device__ __forceinline__ int tile(int row, int col, int grid_x) const { return (y0 + row) * grid_x + x0 + col; }
+    // whether tile number e is one of the region's (`s`: of a region with spans)
+    __device__ __forceinline__ bool holds(int e, int row, int col, const TileSpans& s) const
+    {
+        if (masked) return ((mask >> e) & 1u) != 0u;
+        if (!spans) return true;
+        int first, end;
+        s.columns(row, width, first, end);
+        return col >= first && col < end;
+    }
+};
+
 // The hardware exp2 is monotone, so exp2(t) < 1/255 exactly when t < kAlphaCut, the smallest float whose exp2 reaches
 // 1/255 (found by running v_exp_f32 over every float between -8.2 and -7.8).  The blend (forward and backward) decides
 // on t = power * log2(e) + log2(opacity) and leaves the exp2 (a quarter-rate instruction) to the pairs that pass; the
@@ -161,12 +260,13 @@ constexpr float kAlphaCut = -7.99435329f;  // bits 0xc0ffd1be
 // stage launchers (each returns a gs355_status)
 // `par` (may be NULL): g holds stored parameters
 int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
-                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, int32_t* radii, hipStream_t s);
+                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, uint2* wave_totals, int32_t* radii,
+                      hipStream_t s);
 int launch_scan_offsets(const uint32_t* tiles_touched, const int32_t* radii, int32_t P, const uint32_t* p_device,
                         uint32_t* offsets, uint32_t* scan_tmp, gs355_header* header, gs355_header* header_copy, uint32_t n_cap, hipStream_t s);
 int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const FilterArgs& x, int32_t* radii, hipStream_t s);
 int launch_duplicate(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii,
-                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values,
+                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values, uint64_t* rects,
                      hipStream_t s);
 int launch_sort(const gs355_header* header, uint32_t n_cap, int passes, uint64_t* keys0, uint64_t* keys1,
                 uint32_t* vals0, uint32_t* vals1, uint32_t* hist, uint32_t* scan_tmp, hipStream_t s);
@@ -236,15 +336,23 @@ inline size_t bin_matrix_words(size_t tiles)
 // tile_base: u32[2][tiles] (bases, then the scatter's cursors), then u64[ceil(tiles / 64)] (bases of blocks of 64 tiles),
 // then u32[coarse bins + 1] (chunks of the second scatter level before each bin).  Beyond kBinMaxTiles tiles launch_tile_layout
 // publishes the header and the coarse bins' bases only; ranges, lists and tile bases follow in launch_tile_scatter.
-int launch_tile_count(const FrameArgs& f, int32_t P, const uint64_t* rects, uint32_t* matrix, uint32_t* group_visible,
-                      hipStream_t s);
-int launch_tile_layout(int32_t P, uint32_t* matrix, const uint32_t* group_visible, int tiles, uint32_t n_cap,
+// per slice, and before it per 64 Gaussians (the preprocess's wavefronts): keys of the whole rectangles, Gaussians with a
+// radius.  The frame's key count and its overflow go by the whole rectangles, so that a capacity that suffices for them
+// suffices whatever the regions leave out.
+struct SliceTotals {
+    uint64_t keys;
+    uint32_t visible, unused;
+};
+inline size_t wave_totals_count(int32_t P) { return ((size_t)P + 63) / 64; }
+int launch_tile_count(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint2* wave_totals,
+                      uint32_t* matrix, SliceTotals* slice_totals, hipStream_t s);
+int launch_tile_layout(int32_t P, uint32_t* matrix, const SliceTotals* slice_totals, int tiles, uint32_t n_cap,
                        gs355_header* header, gs355_header* header_copy, uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, hipStream_t s);
 // `coarse`: a second buffer of the buckets' size (first level of the two-level scatter).  `levels`: 1 or 2 = that
 // scatter whatever the frame holds, 0 = chosen on the device by the key count (both variants are launched); images
 // beyond kBinMaxTiles tiles always take two levels
-int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const uint32_t* depth_bits,
-                        gs355_header* header, const uint32_t* matrix, const uint32_t* group_visible, uint32_t n_cap,
+int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint32_t* depth_bits,
+                        gs355_header* header, const uint32_t* matrix, uint32_t n_cap,
                         uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, uint64_t* buckets, uint64_t* coarse,
                         int levels, hipStream_t s);
 // lists: u32[kListHeader + 4 * tiles]: the four class counts, four spare words, the four lists

@@ -117,93 +117,77 @@ constexpr int kShStride = 52;  // floats per Gaussian in the staging area
 // loads touch survivors' blocks only, however few of the 256 survived.  A row of the staging area holds an
 // entry's 48 coefficients and, in its 4 floats of padding, the Gaussian's position on the way in and its colour
 // on the way out.
-template <int kLoads>  // 16-B loads per lane: 64 * kLoads >= 12 * count
-__device__ __forceinline__ void sh_colour_of_entries(float4* __restrict__ mine, const float* __restrict__ shs,
-                                                     size_t group_first, const uint8_t* __restrict__ owner,
-                                                     int first_entry, int count, int lane, int degree,
-                                                     const float* campos)
-{
-    // all loads are issued before the first LDS write, so they are in flight together; slots past the last
-    // entry re-read that entry (same value, same address)
-    float4 v[kLoads];
-    int dst[kLoads];
-#pragma unroll
-    for (int it = 0; it < kLoads; ++it) {
-        const int q4 = it * 64 + lane;
-        const int e = min(q4 / 12, count - 1), m = q4 % 12;
-        const float4* __restrict__ block =
-            reinterpret_cast<const float4*>(shs + (group_first + owner[first_entry + e]) * 48);
-        {  // (read once per frame: a streaming load, which leaves the cache to the records the blend gathers)
-            typedef float f4v __attribute__((ext_vector_type(4)));
-            const f4v t = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(block) + m);
-            v[it] = make_float4(t.x, t.y, t.z, t.w);
-        }
-        dst[it] = e * (kShStride / 4) + m;
-    }
-#pragma unroll
-    for (int it = 0; it < kLoads; ++it) mine[dst[it]] = v[it];
-    wave_lds_sync();
-    if (lane < count) {
-        float* __restrict__ row = reinterpret_cast<float*>(mine) + lane * kShStride;
-        float b[16], rgb[3] = {0.f, 0.f, 0.f};
-        sh_basis(degree, row[48] - campos[0], row[49] - campos[1], row[50] - campos[2], b);
-        sh_accumulate<0, 16>((degree + 1) * (degree + 1), row, b, rgb);
-        sh_finish(rgb);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) row[48 + c] = rgb[c];
-    }
-}
-
-// sh_colour_of_entries over the split storage of the stored parameters: the first coefficient (12 B per Gaussian) is
+//
+// kSplit: the split storage of the stored parameters.  The first coefficient (12 B per Gaussian) is
 // read by the entry's own lane, the other fifteen (45 floats per Gaussian, dword-aligned) with 16-B loads all the
 // same: a Gaussian's row starts (row & 3) floats behind a 16-B boundary and always spans twelve aligned 16-B chunks.
 // The chunks land in the staging row as they are, so the coefficients of entry e start at float (row & 3) of its
 // row; with the rows' stride of 52 floats consecutive Gaussians then sit an odd number of banks apart.  `n_floats`:
 // 45 P.  The last chunk of the last row may reach past the array: it is pulled back inside, and that row's last
 // floats are fetched by its own lane.
-template <int kLoads>
-__device__ __forceinline__ void sh_colour_of_split_entries(float4* __restrict__ mine, const float* __restrict__ dc,
-                                                           const float* __restrict__ rest, size_t n_floats,
-                                                           size_t group_first, const uint8_t* __restrict__ owner,
-                                                           int first_entry, int count, int lane, int degree,
-                                                           const float* campos)
-{
-    float4 v[kLoads];
-    int dst[kLoads];
-    const size_t last_chunk = n_floats / 4 - 1;  // (a row alone is eleven chunks)
-#pragma unroll
-    for (int it = 0; it < kLoads; ++it) {
-        const int q4 = it * 64 + lane;
-        const int e = min(q4 / 12, count - 1), m = q4 % 12;
-        const size_t first = (group_first + owner[first_entry + e]) * 45;
-        typedef float f4v __attribute__((ext_vector_type(4)));
-        const size_t chunk = min(first / 4 + m, last_chunk);
-        const f4v t = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(rest) + chunk);
-        v[it] = make_float4(t.x, t.y, t.z, t.w);
-        dst[it] = e * (kShStride / 4) + m;
-    }
-    const size_t row = group_first + owner[first_entry + min(lane, count - 1)];
+//
+// fetch() and colour() are apart so that the caller has work to do while the blocks travel.
+constexpr int kShLoads = 12;  // 16-B loads per lane for 64 blocks
+template <bool kSplit>
+struct ShEntries {
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    f4v v[kShLoads];
     float first_coeff[3];
+    size_t row, last_chunk;
+
+    // all loads are in flight together; slots past the last entry re-read that entry (same value, same address)
+    __device__ __forceinline__ void fetch(const float* __restrict__ shs, const float* __restrict__ rest, size_t n_floats,
+                                          size_t group_first, const uint8_t* __restrict__ owner, int first_entry, int count,
+                                          int lane)
+    {
+        last_chunk = n_floats / 4 - 1;  // (kSplit: a row alone is eleven chunks)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) first_coeff[c] = __builtin_nontemporal_load(&dc[3 * row + c]);
+        for (int it = 0; it < kShLoads; ++it) {
+            if (it * 64 >= 12 * count) break;  // uniform: fewer survivors, fewer loads
+            const int q4 = it * 64 + lane;
+            const int e = min(q4 / 12, count - 1), m = q4 % 12;
+            const size_t i = group_first + owner[first_entry + e];
+            // (read once per frame: a streaming load, which leaves the cache to the records the blend gathers)
+            if (kSplit)
+                v[it] = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(rest) + min(i * 45 / 4 + m, last_chunk));
+            else
+                v[it] = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(shs + i * 48) + m);
+        }
+        row = group_first + owner[first_entry + min(lane, count - 1)];
+        if (kSplit)
 #pragma unroll
-    for (int it = 0; it < kLoads; ++it) mine[dst[it]] = v[it];
-    wave_lds_sync();
-    if (lane < count) {
+            for (int c = 0; c < 3; ++c) first_coeff[c] = __builtin_nontemporal_load(&shs[3 * row + c]);
+    }
+
+    __device__ __forceinline__ void colour(float4* __restrict__ mine, const float* __restrict__ rest, int count, int lane, int degree,
+                                           const float* campos)
+    {
+#pragma unroll
+        for (int it = 0; it < kShLoads; ++it) {
+            if (it * 64 >= 12 * count) break;
+            const int q4 = it * 64 + lane;
+            mine[min(q4 / 12, count - 1) * (kShStride / 4) + q4 % 12] = make_float4(v[it].x, v[it].y, v[it].z, v[it].w);
+        }
+        wave_lds_sync();
+        if (lane >= count) return;
         float* __restrict__ slot = reinterpret_cast<float*>(mine) + lane * kShStride;
-        float* __restrict__ coeffs = slot + (int)(row & 3);
-        if ((row + 1) * 45 > 4 * (last_chunk + 1))  // the array's last row, where its length is no multiple of four
+        float* __restrict__ coeffs = slot + (kSplit ? (int)(row & 3) : 0);
+        if (kSplit && (row + 1) * 45 > 4 * (last_chunk + 1))  // the array's last row, where its length is no multiple of four
             for (int k = (int)(4 * (last_chunk + 1) - row * 45); k < 45; ++k) coeffs[k] = rest[row * 45 + k];
         float b[16], rgb[3] = {0.f, 0.f, 0.f};
         sh_basis(degree, slot[48] - campos[0], slot[49] - campos[1], slot[50] - campos[2], b);
         const int terms = (degree + 1) * (degree + 1);
-        sh_accumulate<0, 1>(terms, first_coeff, b, rgb);
-        sh_accumulate<1, 15>(terms, coeffs, b, rgb);
+        if (kSplit) {
+            sh_accumulate<0, 1>(terms, first_coeff, b, rgb);
+            sh_accumulate<1, 15>(terms, coeffs, b, rgb);
+        } else {
+            sh_accumulate<0, 16>(terms, coeffs, b, rgb);
+        }
         sh_finish(rgb);
 #pragma unroll
         for (int c = 0; c < 3; ++c) slot[48 + c] = rgb[c];
     }
-}
+};
 
 // Octree-GS level-of-detail test of one anchor, in the reference's order of fp32 operations
 // (octreegs_encoding.py:251-264).
@@ -220,6 +204,39 @@ __device__ __forceinline__ bool lod_keeps(const gs355_anchor_lod& l, float log2_
     return level <= r;
 }
 
+// The word of the tiles a splat is blended in (TileRegion), from its tile rectangle and its reach.  Rows of a masked region
+// are evaluated here, once per Gaussian, so that the kernels that count and place the pairs only walk bits; larger regions
+// leave that to the wavefronts that expand them.  A row costs some 30 vector instructions and splats of small scenes have
+// one to three of them, in a kernel that waits for memory: 6M Gaussians at 1080p 304 -> 306 us while the SH blocks are on
+// their way (317 ahead of them), 1M large splats 57 -> 59.  What it saves (6M / 1M / 20M Gaussians, the last at 4K):
+// scatter 123 -> 97 / 102 -> 73 / 322 -> 260 us, sort 117 -> 83 / 115 -> 63 / 197 -> 160, blend 323 -> 292 / 164 -> 145 /
+// 785 -> 706, blend backward 1025 -> 870 (6M).
+__device__ __forceinline__ uint64_t tile_region(const Rect q, float px, float py, float qx, float qy, float qz, float ex, float ey)
+{
+    const uint64_t whole = (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
+    if (!(ex < INFINITY)) return whole;
+    if (ex < 0.0f) return 0;
+    const float x = px - (float)(q.x0 * kTile), y = py - (float)(q.y0 * kTile);
+    int c0, c1, r0, r1;
+    TileSpans::tiles_of(x - ex, x + ex, q.x1 - q.x0, c0, c1);
+    TileSpans::tiles_of(y - ey, y + ey, q.y1 - q.y0, r0, r1);
+    const int w = c1 - c0, h = r1 - r0;
+    if (w <= 0 || h <= 0) return 0;
+    const int x0 = q.x0 + c0, y0 = q.y0 + r0;
+    const uint64_t corner = (uint64_t)x0 | ((uint64_t)y0 << 16);
+    if (w > kMaskWidth || w * h > kMaskTiles)
+        return corner | ((uint64_t)((x0 + w) | 0x8000) << 32) | ((uint64_t)(y0 + h) << 48);
+    const TileSpans spans(px, py, qx, qy, qz, ex, ey, x0, y0);
+    uint32_t mask = 0u;
+    for (int r = 0; r < h; ++r) {
+        int first, end;
+        spans.columns(r, w, first, end);
+        mask |= (((1u << end) - 1u) & ~((1u << first) - 1u)) << (r * w);
+    }
+    if (mask == 0u) return 0;
+    return corner | ((uint64_t)(mask | ((uint32_t)(w - 1) << 28) | 0x80000000u) << 32);
+}
+
 // kStored: g holds the vanilla model's stored parameters, activated here (the activated copies would cost a pass over
 // memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
 // front of a kernel of 0.3 ms).
@@ -229,6 +246,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
                                                          uint32_t* __restrict__ tiles_touched,
                                                          uint64_t* __restrict__ rects,
                                                          uint32_t* __restrict__ depth_bits,
+                                                         uint2* __restrict__ wave_totals,
                                                          int32_t* __restrict__ radii)
 {
     // staging area for the 16-coefficient SH blocks of each wavefront's 64 Gaussians
@@ -238,14 +256,16 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     __shared__ int s_alive[4];
 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = i < effective_count(f, g.P);
+    const int P = effective_count(f, g.P);
+    if ((int)(blockIdx.x * blockDim.x) >= P) return;  // (uniform; the capacity behind a device-side count)
+    const bool valid = i < P;
     const float* __restrict__ V = f.viewmatrix;
     const float* __restrict__ M = f.projmatrix;
 
     // ---- geometry: cull, covariance, EWA projection, conic, radius, tile rectangle ----
     int radius = 0;
     uint32_t touched = 0;
-    uint64_t rect_packed = 0;  // x0 | y0 << 16 | x1 << 32 | y1 << 48, zero when culled
+    Rect rect = {0, 0, 0, 0};
     float x = 0.f, y = 0.f, z = 0.f, vz = 0.f, px = 0.f, py = 0.f, ca = 0.f, cc = 0.f, qx = 0.f, qy = 0.f, qz = 0.f;
     // Every per-Gaussian geometry input is requested up front, before the cull
     // decides whether it is needed: one memory latency instead of a chain of
@@ -336,7 +356,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
 
         radius = rad;
         touched = (uint32_t)area;
-        rect_packed = (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
+        rect = q;
         qx = cc * det_inv;
         qy = -cb * det_inv;
         qz = ca * det_inv;
@@ -347,12 +367,45 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         if (valid && fx.visible) fx.visible[i] = radius > 0 ? 1 : 0;
         return;
     }
-    if (valid) {
-        __builtin_nontemporal_store(touched, &tiles_touched[i]);  // (read by the classic scan and the backward pass only)
-        rects[i] = rect_packed;
-    }
     const bool alive = radius > 0;
     if (kStored && alive) opacity = logistic(opacity);
+    {  // the wavefront's keys and survivors: what the frame's key count is made of
+        uint32_t keys = touched;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) keys += __shfl_down(keys, d, 64);
+        const uint32_t visible = (uint32_t)__popcll(__ballot(alive));
+        if ((threadIdx.x & 63) == 0 && valid) wave_totals[i >> 6] = make_uint2(keys, visible);
+    }
+
+    // Reach of the splat, for the culling of tiles (below) and of the blend's pixel blocks: half-extents
+    // (ex, ey) of the axis-aligned box around the region where alpha can reach
+    // 1/255, i.e. where 0.5 d^T Q d <= ln(255 * opacity).  The box is enlarged
+    // by more than the rounding error of the blend's fp32 evaluation of the
+    // exponent (bounded below by `noise`), so a pixel block outside the box is
+    // certain to take the blend's `alpha < 1/255` branch on all of its pixels.
+    // +inf = never cull (large or ill-conditioned splats), -inf = never visible.
+    float ex = 0.f, ey = 0.f;
+    auto reach_and_region = [&]() {
+        uint64_t region = 0;
+        if (alive) {
+            const float reach = (float)radius + 24.0f;  // |d| over every pixel of every touched tile
+            const float noise = 2.4e-7f * (fabsf(qx) + fabsf(qy) + fabsf(qz)) * reach * reach;
+            if (opacity != opacity || !(noise < 0.02f)) {
+                ex = ey = INFINITY;
+            } else if (!(opacity * 255.0f * 1.0001f >= 1.0f)) {
+                ex = ey = -INFINITY;
+            } else {
+                const float tau = fmaxf(__logf(opacity * 255.0f), 0.0f) * 1.001f + 0.05f;
+                ex = sqrtf(2.0f * tau * ca) * 1.001f + 0.01f;
+                ey = sqrtf(2.0f * tau * cc) * 1.001f + 0.01f;
+            }
+            region = tile_region(rect, px, py, qx, qy, qz, f.tile_reach ? ex : INFINITY, ey);
+        }
+        if (valid) {
+            __builtin_nontemporal_store(touched, &tiles_touched[i]);  // (read by the classic scan only)
+            rects[i] = region;
+        }
+    };
 
     // ---- colour ----
     float rgb[3] = {0.f, 0.f, 0.f};
@@ -362,6 +415,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
             rgb[1] = g.colors_precomp[3 * (size_t)i + 1];
             rgb[2] = g.colors_precomp[3 * (size_t)i + 2];
         }
+        reach_and_region();
     } else {
         // Full 192-B blocks: the survivors of the workgroup are packed (in order) and each wavefront fetches the
         // SH blocks of 64 of them with coalesced loads through LDS, so the memory system sees dense wavefronts
@@ -389,71 +443,37 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
                 my_row[50] = z;
             }
             __syncthreads();
-            // each wavefront takes a quarter of the packed survivors (entry e sits in row e of the staging area)
-            const int share = (total + 3) / 4, first_entry = wave * share;
-            if (first_entry < total) {
-                float4* __restrict__ rows = s_sh + first_entry * (kShStride / 4);
-                const size_t group_first = (size_t)blockIdx.x * blockDim.x;
-                const int count = min(share, total - first_entry);
-                if (kStored) {
-                    const size_t n_floats = (size_t)g.P * 45;
-                    if (count <= 16)
-                        sh_colour_of_split_entries<3>(rows, g.shs, par.rest, n_floats, group_first, s_owner, first_entry, count,
-                                                      lane, f.sh_degree, f.campos);
-                    else if (count <= 32)
-                        sh_colour_of_split_entries<6>(rows, g.shs, par.rest, n_floats, group_first, s_owner, first_entry, count,
-                                                      lane, f.sh_degree, f.campos);
-                    else
-                        sh_colour_of_split_entries<12>(rows, g.shs, par.rest, n_floats, group_first, s_owner, first_entry,
-                                                       count, lane, f.sh_degree, f.campos);
-                } else if (count <= 16)  // uniform: fewer survivors, fewer load rounds
-                    sh_colour_of_entries<3>(rows, g.shs, group_first, s_owner, first_entry, count, lane, f.sh_degree, f.campos);
-                else if (count <= 32)
-                    sh_colour_of_entries<6>(rows, g.shs, group_first, s_owner, first_entry, count, lane, f.sh_degree, f.campos);
-                else
-                    sh_colour_of_entries<12>(rows, g.shs, group_first, s_owner, first_entry, count, lane, f.sh_degree, f.campos);
-            }
+            // each wavefront takes a quarter of the packed survivors (entry e sits in row e of the staging area), and finds
+            // its own Gaussians' tiles while their blocks are on the way
+            const int share = (total + 3) / 4, first_entry = wave * share, count = min(share, total - first_entry);
+            float4* __restrict__ rows = s_sh + first_entry * (kShStride / 4);
+            ShEntries<kStored> entries;
+            if (count > 0)
+                entries.fetch(g.shs, par.rest, (size_t)g.P * 45, (size_t)blockIdx.x * blockDim.x, s_owner, first_entry, count, lane);
+            reach_and_region();
+            if (count > 0) entries.colour(rows, par.rest, count, lane, f.sh_degree, f.campos);
             __syncthreads();
             if (alive) {
 #pragma unroll
                 for (int c = 0; c < 3; ++c) rgb[c] = my_row[48 + c];
             }
-        } else if (alive) {
-            float b[16];
-            sh_basis(f.sh_degree, x - f.campos[0], y - f.campos[1], z - f.campos[2], b);
-            const int terms = (f.sh_degree + 1) * (f.sh_degree + 1);
-            if (kStored) {
-                sh_accumulate<0, 1>(terms, g.shs + (size_t)i * 3, b, rgb);
-                sh_accumulate<1, 15>(terms, par.rest + (size_t)i * (f.sh_coeffs - 1) * 3, b, rgb);
-            } else {
-                sh_accumulate<0, 16>(terms, g.shs + (size_t)i * f.sh_coeffs * 3, b, rgb);
+        } else {
+            reach_and_region();
+            if (alive) {
+                float b[16];
+                sh_basis(f.sh_degree, x - f.campos[0], y - f.campos[1], z - f.campos[2], b);
+                const int terms = (f.sh_degree + 1) * (f.sh_degree + 1);
+                if (kStored) {
+                    sh_accumulate<0, 1>(terms, g.shs + (size_t)i * 3, b, rgb);
+                    sh_accumulate<1, 15>(terms, par.rest + (size_t)i * (f.sh_coeffs - 1) * 3, b, rgb);
+                } else {
+                    sh_accumulate<0, 16>(terms, g.shs + (size_t)i * f.sh_coeffs * 3, b, rgb);
+                }
+                sh_finish(rgb);
             }
-            sh_finish(rgb);
         }
     }
     if (!alive) return;
-
-    // Reach of the splat for the blend stage's per-block culling: half-extents
-    // (ex, ey) of the axis-aligned box around the region where alpha can reach
-    // 1/255, i.e. where 0.5 d^T Q d <= ln(255 * opacity).  The box is enlarged
-    // by more than the rounding error of the blend's fp32 evaluation of the
-    // exponent (bounded below by `noise`), so a pixel block outside the box is
-    // certain to take the blend's `alpha < 1/255` branch on all of its pixels.
-    // +inf = never cull (large or ill-conditioned splats), -inf = never visible.
-    float ex, ey;
-    {
-        const float reach = (float)radius + 24.0f;  // |d| over every pixel of every touched tile
-        const float noise = 2.4e-7f * (fabsf(qx) + fabsf(qy) + fabsf(qz)) * reach * reach;
-        if (opacity != opacity || !(noise < 0.02f)) {
-            ex = ey = INFINITY;
-        } else if (!(opacity * 255.0f * 1.0001f >= 1.0f)) {
-            ex = ey = -INFINITY;
-        } else {
-            const float tau = fmaxf(__logf(opacity * 255.0f), 0.0f) * 1.001f + 0.05f;
-            ex = sqrtf(2.0f * tau * ca) * 1.001f + 0.01f;
-            ey = sqrtf(2.0f * tau * cc) * 1.001f + 0.01f;
-        }
-    }
 
     float4* __restrict__ rec = reinterpret_cast<float4*>(records + (size_t)i * kRecordFloats);
     rec[0] = make_float4(px, py, qx, qy);
@@ -469,7 +489,8 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
                                                         const int32_t* __restrict__ radii,
                                                         const uint32_t* __restrict__ offsets,
                                                         const gs355_header* __restrict__ header,
-                                                        uint64_t* __restrict__ keys, uint32_t* __restrict__ values)
+                                                        uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
+                                                        uint64_t* __restrict__ rects)
 {
     __shared__ uint32_t s_end[256];    // inclusive offset of each Gaussian of the group
     __shared__ uint32_t s_depth[256];  // depth bits
@@ -493,6 +514,9 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
             s_y0[t] = q.y0;
             s_w[t] = q.x1 - q.x0;
             s_depth[t] = __float_as_uint(rec[9]);
+            // (the keys of these stages are those of whole rectangles, whatever region the preprocess left: the backward
+            // pass finds a key's gradient record through it)
+            rects[i] = (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
         }
     }
     s_end[t] = end_i;  // threads past P repeat `begin`, harmless: never selected
@@ -521,20 +545,21 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
 }  // namespace
 
 int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
-                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, int32_t* radii, hipStream_t s)
+                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, uint2* wave_totals, int32_t* radii,
+                      hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
     const dim3 block(256), grid((g.P + 255) / 256);
     const FilterArgs none;
     if (radii_only)
         hipLaunchKernelGGL((preprocess_kernel<true, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
-                           tiles_touched, rects, depth_bits, radii);
+                           tiles_touched, rects, depth_bits, wave_totals, radii);
     else if (par)
         hipLaunchKernelGGL((preprocess_kernel<false, true>), grid, block, 0, s, f, g, *par, none, records, tiles_touched,
-                           rects, depth_bits, radii);
+                           rects, depth_bits, wave_totals, radii);
     else
         hipLaunchKernelGGL((preprocess_kernel<false, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
-                           tiles_touched, rects, depth_bits, radii);
+                           tiles_touched, rects, depth_bits, wave_totals, radii);
     GS355_CHECK_LAUNCH("preprocess");
     return GS355_OK;
 }
@@ -544,7 +569,7 @@ int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const Fil
     if (g.P == 0) return GS355_OK;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((g.P + 255) / 256), dim3(256), 0, s, f, g, ParameterArgs(), x, (float*)nullptr,
-                           (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, radii);
+                           (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, (uint2*)nullptr, radii);
     };
     if (x.stored)
         launch(preprocess_kernel<true, true>);
@@ -555,12 +580,12 @@ int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const Fil
 }
 
 int launch_duplicate(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii,
-                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values,
+                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values, uint64_t* rects,
                      hipStream_t s)
 {
     if (P == 0) return GS355_OK;
     hipLaunchKernelGGL(duplicate_kernel, dim3((P + 255) / 256), dim3(256), 0, s, f, P, records, radii, offsets,
-                       header, keys, values);
+                       header, keys, values, rects);
     GS355_CHECK_LAUNCH("duplicate");
     return GS355_OK;
 }

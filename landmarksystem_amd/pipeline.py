@@ -65,7 +65,8 @@ class Workspace:
         self.frames = 0
         self.overflows = 0
         self.sort_mispredictions = 0  # frames with buckets in a sorter size class that was expected empty
-        self.last_num_keys = 0  # of the latest frame rendered over this workspace
+        self.last_num_keys = 0  # of the latest frame rendered over this workspace: (tile, Gaussian) keys of whole rectangles
+        self.last_num_pairs = 0  # ... and those of them that were sorted and blended
         self.sort_class_idle = [0, 0, 0]  # consecutive frames that left each larger sorter size class empty
         self.sort_class_wait = [4, 4, 4]  # ... and how many of them it takes before the class's launch is left out
 
@@ -349,10 +350,10 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
     if ws.key_capacity == 0:
         ws.key_capacity = max(1 << 20, 4 * inputs.P)
     if not classic and inputs.tiles <= _lib.MAX_FAST_TILES and inputs.P <= _lib.MAX_FAST_GAUSSIANS:
-        front = _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_COUNT
+        front = _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_REACH | _lib.STAGE_TILE_COUNT
         back = _lib.STAGE_TILE_SCATTER | _lib.STAGE_TILESORT | _lib.STAGE_BLEND
         # the scatter variant that suited the previous frame of this workspace (either is correct for any frame)
-        back |= (_lib.STAGE_TILE_SCATTER_TWO_LEVEL if ws.last_num_keys >= _lib.TWO_LEVEL_MIN_KEYS
+        back |= (_lib.STAGE_TILE_SCATTER_TWO_LEVEL if ws.last_num_pairs >= _lib.TWO_LEVEL_MIN_KEYS
                  else _lib.STAGE_TILE_SCATTER_ONE_LEVEL)
         # no launch for a sorter size class that the last few frames left empty (a hint: the library sorts the
         # buckets of such a class all the same, but far slower than the launch costs, so a class that turns up
@@ -375,6 +376,7 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
                                 C.byref(out.c), front | back, stream))
         total, overflow = header.num_keys_total, header.overflow
         out.num_keys = ws.last_num_keys = total
+        ws.last_num_pairs = header.num_keys
         out.num_visible = header.num_visible
         ws.frames += 1
         counts = tuple(header.sort_class_count)

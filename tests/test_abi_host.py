@@ -543,3 +543,17 @@ def test_static_count_rejects_more_anchors_than_its_array_covers():
     an.anchor = an.feat = an.offset = an.scaling = an.visible_mask = an.campos = 0x1000
     rc = lib.gs355_decode_count_static(C.byref(d), C.byref(an), 0x1000, 0x1000, None)  # rejected before any HIP call
     assert rc == _lib.GS355_ENOSPC and b"at most" in lib.gs355_last_error()
+
+
+def test_tile_reach_is_for_the_bucketed_stages():
+    lib = _lib.load()
+    frame, g, out = _frame(), _gauss(), _lib.Outputs()
+    out.image = out.radii = 0x1000
+
+    def run(mask):
+        return lib.gs355_run(C.byref(frame), C.byref(g), 0x1000, 1024, 100, C.byref(out), mask, None)
+
+    for classic in (_lib.STAGE_SCAN, _lib.STAGE_DUPLICATE, _lib.STAGE_SORT, _lib.STAGE_RANGES, _lib.STAGE_ALL):
+        assert "whole rectangles" in _err(_lib.GS355_EINVAL, run, _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_REACH | classic)
+    assert "no known stage" in _err(_lib.GS355_EINVAL, run, _lib.STAGE_TILE_REACH)
+    assert "needed" in _err(_lib.GS355_ENOSPC, run, _lib.PIPELINE_FAST | _lib.STAGE_TILE_REACH)
