@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
             const TileReach reach(quad_lane<0>(v.x), quad_lane<0>(v.y), quad_lane<0>(v.z), quad_lane<0>(v.w),
                                   quad_lane<1>(v.x), quad_lane<2>(v.z), quad_lane<2>(v.w), (float)(tile_x * kTile),
                                   (float)(tile_y * kTile));
-            const float row_mask = __uint_as_float(reach.row((float)part) << (4 * part));
+            const float row_mask = __uint_as_float(reach.unless_infinite(reach.row((float)part), 0xFu) << (4 * part));
             const uint32_t mask = __float_as_uint(quad_lane<0>(row_mask)) | __float_as_uint(quad_lane<1>(row_mask)) |
                                   __float_as_uint(quad_lane<2>(row_mask)) | __float_as_uint(quad_lane<3>(row_mask));
             if (part == 0) {

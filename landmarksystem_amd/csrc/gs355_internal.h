@@ -117,8 +117,7 @@ __device__ __forceinline__ float pair_exponent(float dx, float dy, float hx, flo
 // backward blend): blend 198 -> 161 us (1M large splats, 1080p), 361 -> 334 us (6M), 969 -> 903 us (20M, 4K), 304 -> 290 us
 // (500k anchors).
 struct TileReach {
-    float rho, across, scale, left, right, t_first, t_step, t_span;
-    bool never, always;
+    float rho, across, scale, left, right, t_first, t_step, t_span, reach;
 
     __device__ __forceinline__ TileReach(float px, float py, float conic_x, float conic_y, float conic_z, float reach_x,
                                          float reach_y, float tile_x0, float tile_y0)
@@ -135,8 +134,13 @@ struct TileReach {
         right = __builtin_fmaf(0.25f, x + slack, 1.0f);
         left = __builtin_fmaf(0.25f, x - slack, 0.2499f);
         scale = 0.25f * reach_x;
-        never = reach_x < 0.0f;
-        always = !(reach_x < __builtin_inff());
+        reach = reach_x;
+    }
+
+    // Rows as they come from row(), for a reach that is a number; +inf reaches `all`, -inf nothing.
+    __device__ __forceinline__ uint32_t unless_infinite(uint32_t mask, uint32_t all) const
+    {
+        return reach < 0.0f ? 0u : reach < __builtin_inff() ? mask : all;
     }
 
     __device__ __forceinline__ uint32_t row(float b) const
@@ -148,10 +152,15 @@ struct TileReach {
         const float hi = __builtin_fmaf(scale, __builtin_fmaf(rho, up, across * half_up), right);
         const float lo = __builtin_fmaf(scale, __builtin_fmaf(rho, down, -(across * half_down)), left);
         const uint32_t n1 = (uint32_t)__builtin_amdgcn_fmed3f(hi, 0.0f, 4.0f), n0 = (uint32_t)__builtin_amdgcn_fmed3f(lo, 0.0f, 4.0f);
-        const uint32_t columns = ((1u << n1) - 1u) & ~((1u << n0) - 1u);
-        return never ? 0u : always ? 0xFu : columns;
+        return ((1u << n1) - 1u) & ~((1u << n0) - 1u);
     }
 };
+
+// A splat whose |rho| is below this has no pixel with an exponent above zero.  The two square terms of the exponent outweigh
+// the mixed one by at least 1 - |rho| of their sum, and pair_exponent's five roundings are off by less than 2^-21 = 4.8e-7
+// of it (rho itself by 4e-7): the exponent comes out negative, or zero at the splat's centre.  The blends test for exponents
+// above zero only where a staged record is beyond it (axes of more than 400:1 on the screen) or not a number.
+constexpr float kDefinite = 0.99999f;
 
 // The columns of tiles that the splat's alpha >= 1/255 ellipse can reach, for one row of tiles at a time: TileReach's span
 // with tiles in the place of blocks (the same formula, and the same slack).  Rows and columns count from tile (x0, y0).
