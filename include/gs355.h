@@ -127,7 +127,7 @@ typedef struct gs355_header {
 typedef struct gs355_layout {
     size_t header;        /* gs355_header */
     size_t records;       /* f32[P][12]: px, py, conic_x, conic_y, conic_z, opacity, r, g, b, depth, reach_x, reach_y */
-    size_t tiles_touched; /* u32[P] */
+    size_t tiles_touched; /* u32[P]    tiles of the whole rectangle (with GS355_STAGE_TILE_REACH written by the scan only) */
     size_t rects;         /* u64[P]    tiles the Gaussian is blended in, zero when there are none: its tile rectangle
                            * (u16 x0, y0, x1, y1), or with GS355_STAGE_TILE_REACH a part of it (TileRegion in
                            * gs355_internal.h) */
@@ -145,7 +145,8 @@ typedef struct gs355_layout {
                            * u32[ceil(tiles/16)+1], the work list of the scatter's second level, and
                            * u32[ceil(tiles/64)], buckets per larger sorter size class in each block of 64 tiles */
     size_t bin_visible;   /* {u64, u32, u32}[slices]  keys and visible Gaussians of each slice's share of what follows,
-                           * {u32, u32}[ceil(P/64)]   keys and visible Gaussians per 64 Gaussians */
+                           * {u32, u32}[ceil(P/64)]   keys and visible Gaussians per 64 Gaussians,
+                           * u8[P]                    channels of a colour from SH coefficients that are above zero (bits) */
     size_t tile_lists;    /* u32[8+4*tiles]  counts, work counters and lists of the buckets of each larger sorter size class */
     size_t total_bytes;
     int32_t unsorted_buffer; /* which keys/values buffer the duplicate stage writes (0) */
@@ -194,7 +195,7 @@ enum {
      * that its alpha >= 1/255 ellipse reaches.  The blend and the backward pass would take the `alpha < 1/255` branch for
      * every pixel of the other tiles, so images and gradients are the same bits; sorted keys, values and ranges are those
      * of the remaining keys.  num_keys_total, and with it the overflow of a capacity, still count whole rectangles.
-     * Refused together with a classic stage.  No effect beyond 32767 tiles along an axis. */
+     * Refused together with a classic stage (in later calls the scan goes back to whole rectangles).  No effect beyond 32767 tiles along an axis. */
     GS355_STAGE_TILE_REACH = 65536,
     GS355_PIPELINE_FAST = 1 | 128 | 512 | 256 | 32
 };

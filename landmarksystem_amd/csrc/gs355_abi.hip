@@ -94,7 +94,7 @@ int make_layout(int32_t P, int64_t n_cap, int32_t W, int32_t H, gs355_layout* L)
     L->ranges = take(tiles * 2 * sizeof(uint32_t));
     L->bin_matrix = take((tiles <= (size_t)kBinMaxTilesWide ? bin_matrix_words(tiles) : 0) * sizeof(uint32_t));
     L->tile_base = take((2 * tiles + 3 * ((tiles + 63) / 64) + (tiles + kCoarseTiles - 1) / kCoarseTiles + 1) * sizeof(uint32_t));
-    L->bin_visible = take((size_t)kBinMaxGroups * sizeof(SliceTotals) + wave_totals_count(P) * sizeof(uint2));
+    L->bin_visible = take((size_t)kBinMaxGroups * sizeof(SliceTotals) + wave_totals_count(P) * sizeof(uint2) + p);
     L->tile_lists = take((kListHeader + 4 * tiles) * sizeof(uint32_t));
     L->total_bytes = off;
     L->sort_bits = 32 + ceil_log2((uint32_t)tiles);
@@ -280,6 +280,7 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
     auto* tile_base = reinterpret_cast<uint32_t*>(ws + L.tile_base);
     auto* slice_totals = reinterpret_cast<SliceTotals*>(ws + L.bin_visible);
     auto* wave_totals = reinterpret_cast<uint2*>(slice_totals + kBinMaxGroups);
+    auto* lit = reinterpret_cast<uint8_t*>(wave_totals + wave_totals_count(g->P));
     auto* tile_lists = reinterpret_cast<uint32_t*>(ws + L.tile_lists);
     hipStream_t s = static_cast<hipStream_t>(stream);
     FrameArgs fa = make_args(frame);
@@ -288,13 +289,15 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
     const uint32_t cap = (uint32_t)n_cap;
 
     if (stage_mask & GS355_STAGE_PREPROCESS)
-        if ((rc = launch_preprocess(fa, *g, par, false, records, touched, rects, depth_bits, wave_totals, out->radii, s))) return rc;
-    if (stage_mask & GS355_STAGE_SCAN)
+        if ((rc = launch_preprocess(fa, *g, par, false, records, touched, rects, depth_bits, wave_totals, lit, out->radii, s))) return rc;
+    if (stage_mask & GS355_STAGE_SCAN) {
+        if ((rc = launch_whole_rectangles(fa, g->P, records, out->radii, touched, rects, s))) return rc;
         if ((rc = launch_scan_offsets(touched, out->radii, g->P, g->P_device, offsets, scan_tmp, header,
                                       static_cast<gs355_header*>(out->header_copy), cap, s)))
             return rc;
+    }
     if (stage_mask & GS355_STAGE_DUPLICATE)
-        if ((rc = launch_duplicate(fa, g->P, records, out->radii, offsets, header, keys[0], vals[0], rects, s))) return rc;
+        if ((rc = launch_duplicate(fa, g->P, records, out->radii, offsets, header, keys[0], vals[0], s))) return rc;
     if (stage_mask & GS355_STAGE_SORT)
         if ((rc = launch_sort(header, cap, L.sort_passes, keys[0], keys[1], vals[0], vals[1], hist, scan_tmp, s)))
             return rc;
@@ -402,7 +405,7 @@ int gs355_visible_filter(const gs355_frame* frame, const gs355_gaussians* g, int
     if (g->P > 0 && !radii) return set_error(GS355_EINVAL, "radii is NULL");
     if (g->P_device) return set_error(GS355_EINVAL, "visible_filter does not take a device-side Gaussian count");
     const FrameArgs fa = make_args(frame);
-    return launch_preprocess(fa, *g, nullptr, true, nullptr, nullptr, nullptr, nullptr, nullptr, radii, static_cast<hipStream_t>(stream));
+    return launch_preprocess(fa, *g, nullptr, true, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, radii, static_cast<hipStream_t>(stream));
 }
 
 namespace {
@@ -473,7 +476,9 @@ static int render_backward(const gs355_frame* frame, const gs355_gaussians* g, c
                                   reinterpret_cast<const uint32_t*>(ws + L.ranges),
                                   reinterpret_cast<const uint32_t*>(ws + L.values[L.sorted_buffer]),
                                   reinterpret_cast<const float*>(ws + L.records),
-                                  reinterpret_cast<const uint64_t*>(ws + L.rects), *in,
+                                  reinterpret_cast<const uint64_t*>(ws + L.rects),
+                                  reinterpret_cast<const uint8_t*>(ws + L.bin_visible + (size_t)kBinMaxGroups * sizeof(SliceTotals) +
+                                                                   wave_totals_count(g->P) * sizeof(uint2)), *in,
                                   reinterpret_cast<uint2*>(sc + B.record_slots),
                                   reinterpret_cast<uint32_t*>(sc + B.next_slot),
                                   reinterpret_cast<float*>(sc + B.key_grads), *grads, par, static_cast<hipStream_t>(stream));

@@ -633,6 +633,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
                                                                   const float* __restrict__ records,
                                                                   const uint64_t* __restrict__ rects,
                                                                   const RecordSlots* __restrict__ slots,
+                                                                  const uint8_t* __restrict__ lit,
                                                                   const float* __restrict__ key_grads,
                                                                   gs355_gradients out, ParameterArgs par, bool summed)
 {
@@ -686,7 +687,8 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
     }
     // the Gaussian's own inputs are requested before its records are waited for, too
     float in_mean[3] = {0.f, 0.f, 0.f}, in_scale[3] = {0.f, 0.f, 0.f}, in_rot[4] = {0.f, 0.f, 0.f, 0.f};
-    float in_opacity = 0.f, in_rgb[3] = {0.f, 0.f, 0.f};
+    float in_opacity = 0.f;
+    uint32_t in_lit = 0u;
     if (alive) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) in_mean[k] = g.means3D[3 * si + k];
@@ -697,9 +699,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
             for (int k = 0; k < 4; ++k) in_rot[k] = g.rotations[4 * si + k];
         }
         if (kStored) in_opacity = g.opacities[si];
-        if (g.shs)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) in_rgb[c] = records[si * kRecordFloats + 6 + c];
+        if (g.shs) in_lit = lit[si];
     }
     float4 A0, A1, A2;
     sum_records(key_grads, run, region, f.plain_regions, records, si, mine + kPartialsAt, A0, A1, A2);
@@ -870,10 +870,9 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
             ny = diry * inv_len;
             nz = dirz * inv_len;
             K = (f.sh_degree + 1) * (f.sh_degree + 1);
-            // the forward pass clamped the colour at zero: a zero in the record means no gradient
-            gcol[0] = in_rgb[0] > 0.0f ? dcol[0] : 0.0f;
-            gcol[1] = in_rgb[1] > 0.0f ? dcol[1] : 0.0f;
-            gcol[2] = in_rgb[2] > 0.0f ? dcol[2] : 0.0f;
+            // the forward pass clamped the colour at zero: a channel at zero gets no gradient
+#pragma unroll
+            for (int c = 0; c < 3; ++c) gcol[c] = ((in_lit >> c) & 1u) != 0u ? dcol[c] : 0.0f;
         }
     }
 
@@ -1012,7 +1011,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
 
 int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const gs355_header* header,
                            const uint32_t* ranges, const uint32_t* values, const float* records,
-                           const uint64_t* rects, const gs355_backward_inputs& in, uint2* record_slots, uint32_t* next_slot,
+                           const uint64_t* rects, const uint8_t* lit, const gs355_backward_inputs& in, uint2* record_slots, uint32_t* next_slot,
                            float* key_grads, const gs355_gradients& out, const ParameterArgs* par, hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
@@ -1042,7 +1041,7 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
         GS355_CHECK_LAUNCH("record sums");
     }
     auto launch = [&](auto kernel, const ParameterArgs& p) {
-        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, rects, slots, key_grads, out, p,
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, rects, slots, lit, key_grads, out, p,
                            summed);
     };
     if (par) {

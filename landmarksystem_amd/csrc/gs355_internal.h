@@ -269,13 +269,15 @@ constexpr float kAlphaCut = -7.99435329f;  // bits 0xc0ffd1be
 // stage launchers (each returns a gs355_status)
 // `par` (may be NULL): g holds stored parameters
 int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
-                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, uint2* wave_totals, int32_t* radii,
-                      hipStream_t s);
+                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, uint2* wave_totals, uint8_t* lit,
+                      int32_t* radii, hipStream_t s);
 int launch_scan_offsets(const uint32_t* tiles_touched, const int32_t* radii, int32_t P, const uint32_t* p_device,
                         uint32_t* offsets, uint32_t* scan_tmp, gs355_header* header, gs355_header* header_copy, uint32_t n_cap, hipStream_t s);
 int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const FilterArgs& x, int32_t* radii, hipStream_t s);
+int launch_whole_rectangles(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii, uint32_t* tiles_touched,
+                            uint64_t* rects, hipStream_t s);
 int launch_duplicate(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii,
-                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values, uint64_t* rects,
+                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values,
                      hipStream_t s);
 int launch_sort(const gs355_header* header, uint32_t n_cap, int passes, uint64_t* keys0, uint64_t* keys1,
                 uint32_t* vals0, uint32_t* vals1, uint32_t* hist, uint32_t* scan_tmp, hipStream_t s);
@@ -286,7 +288,7 @@ int launch_blend(const FrameArgs& f, const gs355_header* header, const uint32_t*
 
 int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const gs355_header* header,
                            const uint32_t* ranges, const uint32_t* values, const float* records,
-                           const uint64_t* rects, const gs355_backward_inputs& in, uint2* record_slots, uint32_t* next_slot,
+                           const uint64_t* rects, const uint8_t* lit, const gs355_backward_inputs& in, uint2* record_slots, uint32_t* next_slot,
                            float* key_grads, const gs355_gradients& out, const ParameterArgs* par, hipStream_t s);
 
 // Activations of the stored parameters, each with the framework's own elementwise rounding (the caller is compiled

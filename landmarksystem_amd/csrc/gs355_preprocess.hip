@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
                                                          uint32_t* __restrict__ tiles_touched,
                                                          uint64_t* __restrict__ rects,
                                                          uint32_t* __restrict__ depth_bits,
-                                                         uint2* __restrict__ wave_totals,
+                                                         uint2* __restrict__ wave_totals, uint8_t* __restrict__ lit,
                                                          int32_t* __restrict__ radii)
 {
     // staging area for the 16-coefficient SH blocks of each wavefront's 64 Gaussians
@@ -402,7 +402,8 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
             region = tile_region(rect, px, py, qx, qy, qz, f.tile_reach ? ex : INFINITY, ey);
         }
         if (valid) {
-            __builtin_nontemporal_store(touched, &tiles_touched[i]);  // (read by the classic scan only)
+            // (the classic scan's input, which that makes by itself where it was left out: 4 of 16 B per Gaussian)
+            if (!f.tile_reach) __builtin_nontemporal_store(touched, &tiles_touched[i]);
             rects[i] = region;
         }
     };
@@ -473,6 +474,10 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
             }
         }
     }
+    // Which channels are above zero is all that the backward pass wants of a colour (zero: clamped, no gradient): a byte
+    // instead of 12 of the record's 48, whose cache lines it would read from end to end (preprocess backward of 6M
+    // Gaussians 780 -> 723 us, for 2 us here, which the tile counts left out above give back).
+    if (valid && (kStored || !g.colors_precomp)) lit[i] = (uint8_t)((rgb[0] > 0.0f) | ((rgb[1] > 0.0f) << 1) | ((rgb[2] > 0.0f) << 2));
     if (!alive) return;
 
     float4* __restrict__ rec = reinterpret_cast<float4*>(records + (size_t)i * kRecordFloats);
@@ -482,6 +487,21 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     depth_bits[i] = __float_as_uint(vz);
 }
 
+// Before the classic stages, whose keys are those of whole rectangles: every Gaussian's rectangle and its tiles, whatever
+// region the preprocess left (the backward pass finds a key's gradient record through it).
+__global__ __launch_bounds__(256) void whole_rectangles_kernel(FrameArgs f, int32_t P, const float* __restrict__ records,
+                                                               const int32_t* __restrict__ radii,
+                                                               uint32_t* __restrict__ tiles_touched, uint64_t* __restrict__ rects)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= effective_count(f, P)) return;
+    const int rad = radii[i];
+    Rect q = {0, 0, 0, 0};
+    if (rad > 0) q = tile_rect(records[(size_t)i * kRecordFloats], records[(size_t)i * kRecordFloats + 1], rad, f.grid_x, f.grid_y);
+    tiles_touched[i] = (uint32_t)((q.x1 - q.x0) * (q.y1 - q.y0));
+    rects[i] = (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
+}
+
 // One workgroup expands the keys of 256 consecutive Gaussians.  Output slots
 // are walked by consecutive lanes (coalesced stores); each slot finds its
 // source Gaussian by binary search over the group's offsets held in LDS.
@@ -489,8 +509,7 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
                                                         const int32_t* __restrict__ radii,
                                                         const uint32_t* __restrict__ offsets,
                                                         const gs355_header* __restrict__ header,
-                                                        uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-                                                        uint64_t* __restrict__ rects)
+                                                        uint64_t* __restrict__ keys, uint32_t* __restrict__ values)
 {
     __shared__ uint32_t s_end[256];    // inclusive offset of each Gaussian of the group
     __shared__ uint32_t s_depth[256];  // depth bits
@@ -514,9 +533,6 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
             s_y0[t] = q.y0;
             s_w[t] = q.x1 - q.x0;
             s_depth[t] = __float_as_uint(rec[9]);
-            // (the keys of these stages are those of whole rectangles, whatever region the preprocess left: the backward
-            // pass finds a key's gradient record through it)
-            rects[i] = (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
         }
     }
     s_end[t] = end_i;  // threads past P repeat `begin`, harmless: never selected
@@ -545,21 +561,21 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
 }  // namespace
 
 int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
-                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, uint2* wave_totals, int32_t* radii,
-                      hipStream_t s)
+                      uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, uint2* wave_totals, uint8_t* lit,
+                      int32_t* radii, hipStream_t s)
 {
     if (g.P == 0) return GS355_OK;
     const dim3 block(256), grid((g.P + 255) / 256);
     const FilterArgs none;
     if (radii_only)
         hipLaunchKernelGGL((preprocess_kernel<true, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
-                           tiles_touched, rects, depth_bits, wave_totals, radii);
+                           tiles_touched, rects, depth_bits, wave_totals, lit, radii);
     else if (par)
         hipLaunchKernelGGL((preprocess_kernel<false, true>), grid, block, 0, s, f, g, *par, none, records, tiles_touched,
-                           rects, depth_bits, wave_totals, radii);
+                           rects, depth_bits, wave_totals, lit, radii);
     else
         hipLaunchKernelGGL((preprocess_kernel<false, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
-                           tiles_touched, rects, depth_bits, wave_totals, radii);
+                           tiles_touched, rects, depth_bits, wave_totals, lit, radii);
     GS355_CHECK_LAUNCH("preprocess");
     return GS355_OK;
 }
@@ -569,7 +585,7 @@ int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const Fil
     if (g.P == 0) return GS355_OK;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((g.P + 255) / 256), dim3(256), 0, s, f, g, ParameterArgs(), x, (float*)nullptr,
-                           (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, (uint2*)nullptr, radii);
+                           (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, (uint2*)nullptr, (uint8_t*)nullptr, radii);
     };
     if (x.stored)
         launch(preprocess_kernel<true, true>);
@@ -579,13 +595,22 @@ int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const Fil
     return GS355_OK;
 }
 
+int launch_whole_rectangles(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii, uint32_t* tiles_touched,
+                            uint64_t* rects, hipStream_t s)
+{
+    if (P == 0) return GS355_OK;
+    hipLaunchKernelGGL(whole_rectangles_kernel, dim3((P + 255) / 256), dim3(256), 0, s, f, P, records, radii, tiles_touched, rects);
+    GS355_CHECK_LAUNCH("whole rectangles");
+    return GS355_OK;
+}
+
 int launch_duplicate(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii,
-                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values, uint64_t* rects,
+                     const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values,
                      hipStream_t s)
 {
     if (P == 0) return GS355_OK;
     hipLaunchKernelGGL(duplicate_kernel, dim3((P + 255) / 256), dim3(256), 0, s, f, P, records, radii, offsets,
-                       header, keys, values, rects);
+                       header, keys, values);
     GS355_CHECK_LAUNCH("duplicate");
     return GS355_OK;
 }
