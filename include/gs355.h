@@ -328,8 +328,8 @@ typedef struct gs355_gradients {
     float *cov3D_precomp;  /* [P,6] */
 } gs355_gradients;
 
-/* Bytes of scratch gs355_render_backward needs for P Gaussians and a key capacity of n_cap: one 48-byte
- * gradient record per key, and the index of each Gaussian's first record. */
+/* Bytes of scratch gs355_render_backward needs for P Gaussians and a key capacity of n_cap: a gradient
+ * record of at most 48 bytes per key, and the index of each Gaussian's first record. */
 GS355_API int gs355_backward_scratch_bytes(int32_t P, int64_t n_cap, size_t *bytes);
 
 /* frame, g, workspace, workspace_bytes, n_cap: exactly what the forward call (gs355_render, or gs355_run through

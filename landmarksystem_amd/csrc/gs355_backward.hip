@@ -11,9 +11,9 @@
 //                    known from the forward outputs), dL/dalpha_i = T_i f_i - (R - P_i) / (1 - alpha_i): no
 //                    division by a transmittance and no second, reversed walk.  Per-pair contributions are summed
 //                    over the 16 pixels of a block four list entries at a time, added to the wavefront's own sums of
-//                    the staged Gaussians in LDS (no atomics), and written once per batch of 64 as one 48-byte
-//                    record per (tile, Gaussian) key.  No global atomics (they cost more than the rest of the
-//                    kernel): the records of a Gaussian are consecutive, in the order its tile region is
+//                    the staged Gaussians in LDS (no atomics), and written once per batch of 64 as one 36-byte
+//                    record (48 with a depth gradient) per (tile, Gaussian) key.  No global atomics (they cost
+//                    more than the rest of the kernel): the records of a Gaussian are consecutive, in the order its tile region is
 //                    walked, and are summed in that order, so gradients are identical from run to run.
 //   sum_large        (scenes of up to 262144 Gaussians) the records of Gaussians of many tiles, summed by many lanes
 //   preprocess_backward  per Gaussian: conic -> 2-D covariance -> Jacobian / 3-D covariance -> scale, rotation,
@@ -28,7 +28,34 @@ namespace gs355 {
 
 namespace {
 
-constexpr int kKeyFloats = GS355_KEY_GRAD_FLOATS;  // per-key record: dpx, dpy, dconic xyz, dopacity, drgb, ddepth, 2 unused
+// Per-key record, three parts of N floats: (dpx, dpy, dconic x), (dconic y, dconic z, dopacity), (dr, dg, db), or where a
+// gradient arrives for the depth plane (dpx, dpy, dconic x, dconic y), (dconic z, dopacity, dr, dg), (db, ddepth, 0, 0).
+// 36 bytes in the place of 48 where the depth has none: preprocess backward of 6M Gaussians 724 -> 707 us, of 550k decoded
+// ones 57 -> 54, record sums of 100k large splats 40 -> 38.
+template <bool kDepth>
+constexpr int kPartFloats = kDepth ? 4 : 3;
+static_assert(3 * kPartFloats<true> == GS355_KEY_GRAD_FLOATS, "the scratch holds a record of the larger kind per key");
+template <int N>
+struct RecordPart {
+    float v[N];
+    static __device__ __forceinline__ RecordPart load(const float* __restrict__ p)
+    {
+        RecordPart r;
+#pragma unroll
+        for (int k = 0; k < N; ++k) r.v[k] = p[k];
+        return r;
+    }
+    __device__ __forceinline__ void store(float* __restrict__ p) const
+    {
+#pragma unroll
+        for (int k = 0; k < N; ++k) p[k] = v[k];
+    }
+    __device__ __forceinline__ void add(const RecordPart& o)
+    {
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = v[k] + o.v[k];
+    }
+};
 
 // Where a Gaussian's records lie: those of its tile region (TileRegion), by tile number, from some first slot on.  The blend
 // needs the slot of one tile (tx, ty) per key: base + ty * width + tx with base = first - y0 * width - x0 (modulo 2^32),
@@ -201,13 +228,17 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     for (int k = tid; k < 4 * (kBatch + 1) * 5; k += 256) (&s_sum[0][0][0])[k] = make_float2(0.f, 0.f);
 
     uint32_t base = lo;
+    // of this batch's Gaussian; requested one batch ahead (6M Gaussians 874 -> 861 us; the records themselves ahead, too, cost
+    // a wavefront per SIMD: 870)
+    uint32_t index = lo + staged < hi ? values[lo + staged] : 0u;
     for (; base < hi; base += kBatch) {
         const uint64_t live = __ballot(T > 0.0f);
         const bool wave_done = live == 0ull;
         if (lane == 0) s_wave_done[wave] = wave_done ? 1u : 0u;
         const int count = (int)min((uint32_t)kBatch, hi - base);
         if (staged < count) {
-            const uint32_t g = values[base + staged];
+            const uint32_t g = index;
+            if (base + kBatch + staged < hi) index = values[base + kBatch + staged];
             float4 v = reinterpret_cast<const float4*>(records + (size_t)g * kRecordFloats)[min(part, 2)];
             if (part == 3) {
                 const RecordSlots at = slots[g];
@@ -374,25 +405,37 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
         const float green = quad_lane<2>(m.y), blue = quad_lane<3>(m.y), depth = quad_lane<1>(l);
         if (staged < count && part < 3) {
             const float hx = s_a[staged].z, ny = s_a[staged].w, hz = s_b[staged].x;
-            float4 v;
+            RecordPart<kPartFloats<kDepth>> v;
             // d power / d centre = -(conic_x dx + conic_y dy, conic_z dy + conic_y dx), with conic_x = -2 hx etc.
-            if (part == 0)
-                v = make_float4(2.0f * hx * m.y + ny * my, 2.0f * hz * my + ny * m.y, -0.5f * l, -mxy);
-            else if (part == 1)
-                // M = sum of opacity * dL/dopacity over the tile's pixels (zero, not 0 * inf, for a Gaussian that never
-                // blended)
-                v = make_float4(-0.5f * m.y, M != 0.0f ? M * __builtin_amdgcn_exp2f(-s_b[staged].y) : 0.0f, red, green);
-            else
-                v = make_float4(blue, kDepth ? depth : 0.0f, 0.f, 0.f);
-            reinterpret_cast<float4*>(key_grads + (size_t)s_slot[staged] * kKeyFloats)[part] = v;
+            // M = sum of opacity * dL/dopacity over the tile's pixels (zero, not 0 * inf, for a Gaussian that never
+            // blended)
+            if (part == 0) {
+                v.v[0] = 2.0f * hx * m.y + ny * my;
+                v.v[1] = 2.0f * hz * my + ny * m.y;
+                v.v[2] = -0.5f * l;
+                if (kDepth) v.v[3] = -mxy;
+            } else if (part == 1) {
+                const float d_opacity = M != 0.0f ? M * __builtin_amdgcn_exp2f(-s_b[staged].y) : 0.0f;
+                v.v[0] = kDepth ? -0.5f * m.y : -mxy;
+                v.v[1] = kDepth ? d_opacity : -0.5f * m.y;
+                v.v[2] = kDepth ? red : d_opacity;
+                if (kDepth) v.v[3] = green;
+            } else {
+                v.v[0] = kDepth ? blue : red;
+                v.v[1] = kDepth ? depth : green;
+                v.v[2] = kDepth ? 0.0f : blue;
+                if (kDepth) v.v[3] = 0.0f;
+            }
+            v.store(key_grads + ((size_t)s_slot[staged] * 3 + part) * kPartFloats<kDepth>);
         }
     }
     // keys the tile never reached (every pixel finished before them) contribute nothing: every record is written
     for (uint32_t j = base + tid; j < hi; j += 256) {
         const RecordSlots at = slots[values[j]];
         const uint32_t slot = at.base + (uint32_t)tile_y * at.width + (uint32_t)tile_x;
-        float4* __restrict__ dst = reinterpret_cast<float4*>(key_grads + (size_t)slot * kKeyFloats);
-        dst[0] = dst[1] = dst[2] = make_float4(0.f, 0.f, 0.f, 0.f);
+        float* __restrict__ dst = key_grads + (size_t)slot * 3 * kPartFloats<kDepth>;
+#pragma unroll
+        for (int k = 0; k < 3 * kPartFloats<kDepth>; ++k) dst[k] = 0.0f;
     }
 }
 
@@ -442,8 +485,8 @@ constexpr int kShStride = 52;  // floats per Gaussian in the SH staging area (16
 // Up to kSerialRecords of them are added by the Gaussian's own lane, four requested at a time (indices past the last
 // one re-read it and are not added).  A Gaussian of more keys would keep its whole wavefront waiting for one lane's
 // chain of requests (a splat of an early training step covers hundreds of tiles: 245 us of kernel for 100k Gaussians,
-// 112 with this), so those are served by all lanes, four Gaussians at a time: sixteen lanes take one, three per record
-// (48 bytes), five records side by side and four such rounds in flight, and the partial sums meet in LDS.
+// 112 with this), so those are served by all lanes, four Gaussians at a time: sixteen lanes take one, three per
+// record, five records side by side and four such rounds in flight, and the partial sums meet in LDS.
 constexpr uint32_t kSerialRecords = 8;
 // Scenes of few Gaussians leave most of the chip idle even so (a wavefront per 64 Gaussians): up to this many, a kernel
 // of its own gives every Gaussian of more than kSerialRecords keys a wavefront and leaves the sum in its first slot
@@ -461,36 +504,35 @@ __device__ __forceinline__ TileSpans spans_of(const TileRegion& q, const float* 
     return s;
 }
 
-__device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-
+template <int N>
 __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads, const RecordRun run, uint64_t region, bool plain,
-                                            const float* __restrict__ splats, size_t index, float4* __restrict__ partial, float4& A0, float4& A1, float4& A2)
+                                            const float* __restrict__ splats, size_t index, float4* __restrict__ partial,
+                                            RecordPart<N> A[3])
 {
+    typedef RecordPart<N> Part;
     const int lane = threadIdx.x & 63, group = lane >> 4, sub = lane & 15;
-    const float4* __restrict__ records = reinterpret_cast<const float4*>(key_grads);
-    A0 = A1 = A2 = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) A[q] = Part{};
     const uint32_t n = run.n;
     const bool serial = !summed_ahead(run);
     if (serial) {
-        const float4* __restrict__ rec = records + (size_t)run.first * (kKeyFloats / 4);
+        const float* __restrict__ rec = key_grads + (size_t)run.first * (3 * N);
         const uint32_t keys = run.keys();
         uint32_t left = run.masked ? run.mask : (1u << n) - 1u, last = 0;
         for (uint32_t k0 = 0; k0 < keys; k0 += 4) {
-            float4 r[4][3];
+            Part r[4][3];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 last = left != 0u ? (uint32_t)__builtin_ctz(left) : last;
                 left &= left - 1u;  // (0 stays 0)
-                const size_t k = last;
 #pragma unroll
-                for (int q = 0; q < 3; ++q) r[u][q] = rec[3 * k + q];
+                for (int q = 0; q < 3; ++q) r[u][q] = Part::load(rec + (3u * last + (uint32_t)q) * N);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 if (k0 + (uint32_t)u < keys) {
-                    A0 = add4(A0, r[u][0]);
-                    A1 = add4(A1, r[u][1]);
-                    A2 = add4(A2, r[u][2]);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) A[q].add(r[u][q]);
                 }
             }
         }
@@ -517,27 +559,25 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
             q.place((int)k, row, col);
             return q.holds((int)k, row, col, spans);
         };
-        const float4* __restrict__ rec = records + (size_t)first_of * (kKeyFloats / 4) + part;
-        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        const float* __restrict__ rec = key_grads + ((size_t)first_of * 3 + part) * N;
+        Part sum = {};
         for (uint32_t k0 = (uint32_t)slot; k0 < n_mine; k0 += 20) {
-            float4 r[4];
+            Part r[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) r[u] = rec[3 * (size_t)min(k0 + 5u * (uint32_t)u, n_mine - 1)];
+            for (int u = 0; u < 4; ++u) r[u] = Part::load(rec + 3 * N * (size_t)min(k0 + 5u * (uint32_t)u, n_mine - 1));
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                if (held(k0 + 5u * (uint32_t)u)) sum = add4(sum, r[u]);
+                if (held(k0 + 5u * (uint32_t)u)) sum.add(r[u]);
         }
-        if (sub < 15) partial[15 * group + sub] = sum;
+        if (sub < 15) sum.store(reinterpret_cast<float*>(partial + 15 * group + sub));
         wave_lds_sync();
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             if (lane != lane_of[g]) continue;
 #pragma unroll
-            for (int k = 0; k < 5; ++k) {
-                A0 = add4(A0, partial[15 * g + 3 * k]);
-                A1 = add4(A1, partial[15 * g + 3 * k + 1]);
-                A2 = add4(A2, partial[15 * g + 3 * k + 2]);
-            }
+            for (int k = 0; k < 5; ++k)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) A[p].add(Part::load(reinterpret_cast<const float*>(partial + 15 * g + 3 * k + p)));
         }
         wave_lds_sync();
     }
@@ -549,6 +589,7 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
 // waited for its rectangle and then for its records, 47 us for 100k Gaussians of some 20 records each; then 35 (18 was what
 // reading them took).  Regions leave out half of those records and the others are looked up in a span: 40.
 constexpr int kSumPerWave = 8;
+template <int N>
 __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const int32_t* __restrict__ radii,
                                                         const float* __restrict__ splats,
                                                         const uint64_t* __restrict__ rects,
@@ -563,7 +604,8 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const
     uint32_t left = (uint32_t)__ballot(lane < kSumPerWave && i0 + lane < P && radius > 0 && summed_ahead(run));
     if (left == 0u) return;
     const int slot = lane / 3, part = lane % 3;
-    float4* const all = reinterpret_cast<float4*>(key_grads) + part;
+    typedef RecordPart<N> Part;
+    float* const all = key_grads + part * N;
     uint32_t first = 0, n = 0, k0 = 0;  // the current step: records k0 .. k0 + 47 of the n from `first`
     int from = 0, from1 = 0;            // its Gaussian's lane, the next step's
     auto next = [&](uint32_t& f, uint32_t& m) {
@@ -573,20 +615,20 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const
         f = (uint32_t)__builtin_amdgcn_readlane((int)run.first, l);
         m = (uint32_t)__builtin_amdgcn_readlane((int)run.n, l);
     };
-    auto request = [&](uint32_t f, uint32_t m, uint32_t k, float4 r[3]) {
+    auto request = [&](uint32_t f, uint32_t m, uint32_t k, Part r[3]) {
 #pragma unroll
         for (int u = 0; u < 3; ++u)
-            r[u] = all[((size_t)f + min(k + (uint32_t)slot + 16u * (uint32_t)u, m - 1)) * (kKeyFloats / 4)];
+            r[u] = Part::load(all + ((size_t)f + min(k + (uint32_t)slot + 16u * (uint32_t)u, m - 1)) * (3 * N));
     };
     next(first, n);
     from = from1;
-    float4 r[3], sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    Part r[3], sum = {};
     request(first, n, k0, r);
     for (;;) {  // (uniform; ends with the last Gaussian's last step)
         const bool last = k0 + 48u >= n;
         const bool more = !last || left != 0u;
         uint32_t first1 = first, n1 = n, k1 = k0 + 48u;
-        float4 r1[3] = {};
+        Part r1[3] = {};
         if (last && more) {
             next(first1, n1);
             k1 = 0;
@@ -602,18 +644,19 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const
             if (slot >= 16 || k >= n) continue;
             int row, col;
             q.place((int)k, row, col);
-            if (q.holds((int)k, row, col, spans)) sum = add4(sum, r[u]);
+            if (q.holds((int)k, row, col, spans)) sum.add(r[u]);
         }
         if (last) {
 #pragma unroll
             for (int d = 24; d >= 3; d >>= 1) {
-                const float4 other = make_float4(__shfl_down(sum.x, d, 64), __shfl_down(sum.y, d, 64),
-                                                 __shfl_down(sum.z, d, 64), __shfl_down(sum.w, d, 64));
-                sum = add4(sum, other);  // (lanes past the last slot hold zeros; sums other than the first slot's are not used)
+                Part other;
+#pragma unroll
+                for (int k = 0; k < N; ++k) other.v[k] = __shfl_down(sum.v[k], d, 64);
+                sum.add(other);  // (lanes past the last slot hold zeros; sums other than the first slot's are not used)
             }
             // (into the slot of the region's first record; a mask's first tile may be past number 0)
-            if (slot == 0) all[(size_t)first * (kKeyFloats / 4)] = sum;
-            sum = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (slot == 0) sum.store(all + (size_t)first * (3 * N));
+            sum = Part{};
         }
         if (!more) break;
         first = first1, n = n1, k0 = k1, from = from1;
@@ -627,7 +670,7 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const
 // vanilla model's stored parameters, and the gradients are theirs (activations' derivatives included); the rows of the
 // SH coefficients behind the first are then staged back to back, 3 (M - 1) floats each, as they lie in memory: a
 // wavefront's 64 rows start on a 256-B boundary whatever their length.
-template <int kMode, bool kStored>
+template <int kMode, bool kStored, bool kDepth>
 __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kernel(FrameArgs f, gs355_gaussians g,
                                                                   const int32_t* __restrict__ radii,
                                                                   const float* __restrict__ records,
@@ -701,15 +744,19 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
         if (kStored) in_opacity = g.opacities[si];
         if (g.shs) in_lit = lit[si];
     }
-    float4 A0, A1, A2;
-    sum_records(key_grads, run, region, f.plain_regions, records, si, mine + kPartialsAt, A0, A1, A2);
+    constexpr int N = kPartFloats<kDepth>;
+    RecordPart<N> A[3];
+    sum_records<N>(key_grads, run, region, f.plain_regions, records, si, mine + kPartialsAt, A);
     if (alive) {
         const float* __restrict__ V = f.viewmatrix;
         const float* __restrict__ Pm = f.projmatrix;
-        const float g_px = A0.x, g_py = A0.y, gA = A0.z, gB = A0.w, gC = A1.x;
-        dop = A1.y;
-        dcol[0] = A1.z; dcol[1] = A1.w; dcol[2] = A2.x;
-        const float g_depth = A2.y;
+        const float g_px = A[0].v[0], g_py = A[0].v[1], gA = A[0].v[2];
+        const float gB = kDepth ? A[0].v[N - 1] : A[1].v[0], gC = kDepth ? A[1].v[0] : A[1].v[1];
+        dop = kDepth ? A[1].v[1] : A[1].v[2];
+        dcol[0] = kDepth ? A[1].v[2] : A[2].v[0];
+        dcol[1] = kDepth ? A[1].v[N - 1] : A[2].v[1];
+        dcol[2] = kDepth ? A[2].v[0] : A[2].v[2];
+        const float g_depth = kDepth ? A[2].v[1] : 0.0f;
         const float x = in_mean[0], y = in_mean[1], z = in_mean[2];
 
         // ---- pixel position ----
@@ -1035,31 +1082,34 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
                         (out.shs == nullptr || (reinterpret_cast<uintptr_t>(out.shs) & 15u) == 0);
     const dim3 grid((g.P + 255) / 256), block(256);
     const bool summed = g.P <= kSumAheadMax;
-    if (summed) {
-        hipLaunchKernelGGL(sum_large_kernel, dim3((g.P + 4 * kSumPerWave - 1) / (4 * kSumPerWave)), dim3(256), 0, s, g.P,
-                           (bool)f.plain_regions, in.radii, records, rects, slots, key_grads);
-        GS355_CHECK_LAUNCH("record sums");
-    }
-    auto launch = [&](auto kernel, const ParameterArgs& p) {
-        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, rects, slots, lit, key_grads, out, p,
-                           summed);
+    auto finish = [&](auto with_depth) {
+        constexpr bool kDepth = with_depth.value;
+        if (summed) {
+            hipLaunchKernelGGL(sum_large_kernel<kPartFloats<kDepth>>, dim3((g.P + 4 * kSumPerWave - 1) / (4 * kSumPerWave)), dim3(256),
+                               0, s, g.P, (bool)f.plain_regions, in.radii, records, rects, slots, key_grads);
+            GS355_CHECK_LAUNCH("record sums");
+        }
+        auto launch = [&](auto kernel, const ParameterArgs& p) {
+            hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, rects, slots, lit, key_grads, out, p, summed);
+        };
+        if (par) {
+            if ((reinterpret_cast<uintptr_t>(par->rest) & 15u) != 0 || (reinterpret_cast<uintptr_t>(par->d_rest) & 15u) != 0)
+                launch(preprocess_backward_kernel<0, true, kDepth>, *par);
+            else if (f.sh_degree == 0)
+                launch(preprocess_backward_kernel<1, true, kDepth>, *par);
+            else
+                launch(preprocess_backward_kernel<2, true, kDepth>, *par);
+        } else if (!staged) {
+            launch(preprocess_backward_kernel<0, false, kDepth>, ParameterArgs());
+        } else if (f.sh_degree == 0) {
+            launch(preprocess_backward_kernel<1, false, kDepth>, ParameterArgs());
+        } else {
+            launch(preprocess_backward_kernel<2, false, kDepth>, ParameterArgs());
+        }
+        GS355_CHECK_LAUNCH("preprocess backward");
+        return (int)GS355_OK;
     };
-    if (par) {
-        if ((reinterpret_cast<uintptr_t>(par->rest) & 15u) != 0 || (reinterpret_cast<uintptr_t>(par->d_rest) & 15u) != 0)
-            launch(preprocess_backward_kernel<0, true>, *par);
-        else if (f.sh_degree == 0)
-            launch(preprocess_backward_kernel<1, true>, *par);
-        else
-            launch(preprocess_backward_kernel<2, true>, *par);
-    } else if (!staged) {
-        launch(preprocess_backward_kernel<0, false>, ParameterArgs());
-    } else if (f.sh_degree == 0) {
-        launch(preprocess_backward_kernel<1, false>, ParameterArgs());
-    } else {
-        launch(preprocess_backward_kernel<2, false>, ParameterArgs());
-    }
-    GS355_CHECK_LAUNCH("preprocess backward");
-    return GS355_OK;
+    return in.dL_ddepth ? finish(std::true_type{}) : finish(std::false_type{});
 }
 
 }  // namespace gs355
