@@ -583,11 +583,13 @@ __device__ __forceinline__ void sum_records(const float* __restrict__ key_grads,
     }
 }
 
-// Sixteen records side by side, three lanes each, three such rounds per step; the first record is overwritten once all
-// of them have been read (its new value depends on every one).  A wavefront takes eight Gaussians and requests the next
-// step, of the same Gaussian or the next, before it adds the current one: with one Gaussian a wavefront, every one of them
-// waited for its rectangle and then for its records, 47 us for 100k Gaussians of some 20 records each; then 35 (18 was what
-// reading them took).  Regions leave out half of those records and the others are looked up in a span: 40.
+// A wavefront takes eight Gaussians, a step 64 tile numbers of one: a lane each finds those that the region holds, and the
+// held records are read sixteen side by side, three lanes each, up to four such rounds.  The next step, of the same Gaussian
+// or the next, is requested before the current one is added.  The first record is overwritten once all of them have been
+// read (its new value depends on every one).
+// What bounds it is the instructions per tile number: with the three lanes of a record each asking for its tile number, a
+// record that the region leaves out took its turn like the others, and 100k Gaussians of some 20 records each took 39 us; with
+// one question per tile number and only held records in the rounds, 26.
 constexpr int kSumPerWave = 8;
 template <int N>
 __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const int32_t* __restrict__ radii,
@@ -595,57 +597,74 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const
                                                         const uint64_t* __restrict__ rects,
                                                         const RecordSlots* __restrict__ slots, float* key_grads)
 {
-    const int lane = threadIdx.x & 63;
-    const int i0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * kSumPerWave);
+    __shared__ uint8_t s_held[4][2][64];  // tile numbers (from the step's first) of a step's records, this step's and the next's
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + wave) * kSumPerWave);
     const int i = min(i0 + (lane & (kSumPerWave - 1)), P - 1);
     const int32_t radius = radii[i];
     const uint64_t region = rects[i];
-    const RecordRun run = record_run(slots[i], TileRegion(region, plain));
+    const TileRegion own(region, plain);
+    const RecordRun run = record_run(slots[i], own);
     uint32_t left = (uint32_t)__ballot(lane < kSumPerWave && i0 + lane < P && radius > 0 && summed_ahead(run));
     if (left == 0u) return;
+    const TileSpans own_spans = spans_of(own, splats, (size_t)i);
     const int slot = lane / 3, part = lane % 3;
     typedef RecordPart<N> Part;
     float* const all = key_grads + part * N;
-    uint32_t first = 0, n = 0, k0 = 0;  // the current step: records k0 .. k0 + 47 of the n from `first`
-    int from = 0, from1 = 0;            // its Gaussian's lane, the next step's
-    auto next = [&](uint32_t& f, uint32_t& m) {
+    // the Gaussian whose records are requested next: slots first .. first + n - 1, and the step's first tile number
+    uint32_t first = 0, n = 0, e0 = 0;
+    TileRegion q(0ull, plain);
+    TileSpans spans;
+    auto next = [&]() {
         const int l = __builtin_ctz(left);
-        from1 = l;
         left &= left - 1u;
-        f = (uint32_t)__builtin_amdgcn_readlane((int)run.first, l);
-        m = (uint32_t)__builtin_amdgcn_readlane((int)run.n, l);
+        first = (uint32_t)__builtin_amdgcn_readlane((int)run.first, l);
+        n = (uint32_t)__builtin_amdgcn_readlane((int)run.n, l);
+        e0 = 0;
+        q = TileRegion((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)region, l) |
+                           ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(region >> 32), l) << 32),
+                       plain);  // (uniform, and so are its spans)
+        auto of_lane = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+        spans.rho = of_lane(own_spans.rho), spans.across = of_lane(own_spans.across), spans.slack = of_lane(own_spans.slack);
+        spans.rx = of_lane(own_spans.rx), spans.x = of_lane(own_spans.x), spans.y = of_lane(own_spans.y);
+        spans.inv_y = of_lane(own_spans.inv_y);
     };
-    auto request = [&](uint32_t f, uint32_t m, uint32_t k, Part r[3]) {
-#pragma unroll
-        for (int u = 0; u < 3; ++u)
-            r[u] = Part::load(all + ((size_t)f + min(k + (uint32_t)slot + 16u * (uint32_t)u, m - 1)) * (3 * N));
-    };
-    next(first, n);
-    from = from1;
-    Part r[3], sum = {};
-    request(first, n, k0, r);
-    for (;;) {  // (uniform; ends with the last Gaussian's last step)
-        const bool last = k0 + 48u >= n;
-        const bool more = !last || left != 0u;
-        uint32_t first1 = first, n1 = n, k1 = k0 + 48u;
-        Part r1[3] = {};
-        if (last && more) {
-            next(first1, n1);
-            k1 = 0;
-        }
-        if (more) request(first1, n1, k1, r1);
-        const TileRegion q((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)region, from) |
-                               ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(region >> 32), from) << 32),
-                           plain);  // (uniform, and so are its spans)
-        const TileSpans spans = spans_of(q, splats, (size_t)(i0 + from));
-#pragma unroll
-        for (int u = 0; u < 3; ++u) {
-            const uint32_t k = k0 + (uint32_t)slot + 16u * (uint32_t)u;
-            if (slot >= 16 || k >= n) continue;
+    // (the loads stand behind no branch, so that the compiler knows how many are under way; what they read past the last
+    // record is not added)
+    auto request = [&](uint8_t* held, Part r[4]) {
+        const uint32_t e = e0 + (uint32_t)lane;
+        bool holds = e < n;
+        if (holds) {
             int row, col;
-            q.place((int)k, row, col);
-            if (q.holds((int)k, row, col, spans)) sum.add(r[u]);
+            q.place((int)e, row, col);
+            holds = q.holds((int)e, row, col, spans);
         }
+        const uint64_t m = __ballot(holds);
+        if (holds) held[lanes_below_in(m)] = (uint8_t)lane;
+        wave_lds_sync();
+        const int count = __popcll(m);
+        const uint8_t* const mine = held + min(slot, 15);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t at = slot + 16 * u < count ? mine[16 * u] : 0u;
+            r[u] = Part::load(all + ((size_t)first + e0 + at) * (3 * N));
+        }
+        return count;
+    };
+    next();
+    Part r[4], sum = {};
+    int count = request(s_held[wave][0], r);
+    for (int buffer = 1;; buffer ^= 1) {  // (uniform; ends with the last Gaussian's last step)
+        const uint32_t first0 = first;
+        const bool last = e0 + 64u >= n;
+        const bool more = !last || left != 0u;
+        if (!last) e0 += 64u;
+        else if (more) next();
+        Part r1[4];
+        const int count1 = request(s_held[wave][buffer], r1);  // (behind the last step: once more, and not used)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (slot < 16 && slot + 16 * u < count) sum.add(r[u]);
         if (last) {
 #pragma unroll
             for (int d = 24; d >= 3; d >>= 1) {
@@ -655,13 +674,13 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const
                 sum.add(other);  // (lanes past the last slot hold zeros; sums other than the first slot's are not used)
             }
             // (into the slot of the region's first record; a mask's first tile may be past number 0)
-            if (slot == 0) sum.store(all + (size_t)first * (3 * N));
+            if (slot == 0) sum.store(all + (size_t)first0 * (3 * N));
             sum = Part{};
         }
         if (!more) break;
-        first = first1, n = n1, k0 = k1, from = from1;
+        count = count1;
 #pragma unroll
-        for (int u = 0; u < 3; ++u) r[u] = r1[u];
+        for (int u = 0; u < 4; ++u) r[u] = r1[u];
     }
 }
 

@@ -123,8 +123,10 @@ def test_gradients_do_not_change(gpu_device, make):
     for name in a:
         x, y = a[name].double(), b[name].double()
         assert torch.isfinite(x).all() and float(x.abs().max()) > 0
-        # fp32 sums of up to a few thousand terms in two orders
-        assert float((x - y).norm()) <= 1e-6 * float(x.norm()), name
+        # Sums in two orders.  sum_large_kernel adds n terms in sixteen lanes and those in a tree: of the first scene's 273
+        # tiles, 18 terms in a lane and four levels, so at most 21 roundings of 2^-24 in a term's way in either order, 2.5e-6
+        # of the terms; the gradients are linear in the sums.  (The others: more tiles, shorter sums.)
+        assert float((x - y).norm()) <= 2.5e-6 * float(x.norm()), name
         assert float((x - y).abs().max()) <= 1e-5 * float(x.abs().max()), name
 
 
