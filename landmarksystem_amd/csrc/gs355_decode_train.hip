@@ -26,7 +26,7 @@
 //
 // As torch operations the backward pass alone was some thirty launches of skinny matrix products, index and reduction
 // kernels.  A training step at 200k anchors with ten offsets, most of them visible, at 1080p: 3.48 ms with the statements
-// in both directions, 1.50 with these kernels (two runs of one side differ by 7 %).
+// in both directions, 1.50 with these kernels when they were written, 1.18 now, the rasterizer included.
 #include "gs355_internal.h"
 
 namespace gs355 {
@@ -77,16 +77,44 @@ __device__ __forceinline__ int head_of(int o, int n) { return o < n ? 0 : o < 8 
 __device__ __forceinline__ int head_base(int j, int n) { return j == 0 ? 0 : j == 1 ? n : 8 * n; }
 __device__ __forceinline__ int head_outputs(int j, int n) { return j == 0 ? n : j == 1 ? 7 * n : 3 * n; }
 
+// By a workgroup of 256: every thread requests all of its floats before it waits for the first (one after the other, a branch
+// around each, they took 20 us).
 __device__ __forceinline__ void load_parameters(HeadParameters& s, const TrainArgs& d)
 {
-    const int threads = blockDim.x;
-    for (int i = threadIdx.x; i < 3 * 32 * kW0Stride; i += threads) {
-        const int j = i / (32 * kW0Stride), r = i % (32 * kW0Stride) / kW0Stride, c = i % kW0Stride;
-        s.w0[j][r * kW0Stride + c] = c < d.in_dim[j] ? d.w0[j][r * d.in_dim[j] + c] : 0.0f;
+    constexpr int kThreads = 256, kEach0 = (32 * 36 + kThreads - 1) / kThreads, kEach1 = (kFeat * 7 * kMaxOffsets + kThreads - 1) / kThreads;
+    const int tid = threadIdx.x;
+    auto from = [](const float* p, int count) {  // zeros past the last of the floats
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, 4 * count, 0x00020000);
+    };
+    float v0[3][kEach0], v1[3][kEach1];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const auto w0 = from(d.w0[j], 32 * d.in_dim[j]), w1 = from(d.w1[j], kFeat * head_outputs(j, d.n));
+#pragma unroll
+        for (int k = 0; k < kEach0; ++k)
+            v0[j][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(w0, 4 * tid, 4 * kThreads * k, 0));
+#pragma unroll
+        for (int k = 0; k < (j == 0 ? 2 : j == 1 ? kEach1 : 4); ++k)
+            v1[j][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(w1, 4 * tid, 4 * kThreads * k, 0));
     }
-    for (int i = threadIdx.x; i < kRows * kW1Stride; i += threads) {
-        const int o = i / kW1Stride, c = i % kW1Stride, j = head_of(o, d.n);
-        s.w1[i] = o < 11 * d.n && c < kFeat ? d.w1[j][(o - head_base(j, d.n)) * kFeat + c] : 0.0f;
+    static_assert(kFeat * kMaxOffsets <= 2 * kThreads && kFeat * 3 * kMaxOffsets <= 4 * kThreads, "");
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int w = d.in_dim[j], inv_w = (65536 + w - 1) / w;  // e / w == (e * inv_w) >> 16 for e < 32 w, w = 35 or 36
+#pragma unroll
+        for (int k = 0; k < kEach0; ++k) {
+            const int e = k * kThreads + tid, r = (e * inv_w) >> 16;
+            if (e < 32 * w) s.w0[j][r * kW0Stride + e - r * w] = v0[j][k];
+        }
+        if (tid < 32) {
+            if (w < 36) s.w0[j][tid * kW0Stride + 35] = 0.0f;
+            s.w0[j][tid * kW0Stride + 36] = 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < (j == 0 ? 2 : j == 1 ? kEach1 : 4); ++k) {
+            const int e = k * kThreads + tid;
+            if (e < kFeat * head_outputs(j, d.n)) s.w1[(head_base(j, d.n) + e / kFeat) * kW1Stride + e % kFeat] = v1[j][k];
+        }
     }
 }
 
@@ -482,85 +510,135 @@ __global__ __launch_bounds__(256) void train_items_kernel(TrainArgs d, const uin
 constexpr int kBackwardWaves = 4;      // one per SIMD: 176 registers of weight gradients and as many again
 constexpr int kBackwardMaxGroups = 256;
 constexpr int kTilePre = kGroup * 11 * kMaxOffsets;  // floats of a tile's pre-activation gradients
+constexpr int kHiddenStride = 36;      // of a row of hidden units in LDS (16-B reads of 32 rows at one unit on distinct banks)
+// LDS of a wavefront: pre-activation gradients head by head as in memory, input rows, one head's hidden units by row, and
+// their gradients
+constexpr int kWaveIn = kTilePre, kWaveHidden = kWaveIn + kGroup * 36, kWaveUnit = kWaveHidden + kGroup * kHiddenStride;
+constexpr int kWaveFloats = kWaveUnit + kGroup * kW1Stride;
 
-// `count` floats from memory to LDS, both 16-B aligned, without passing through registers; the last few of a count that is
-// no multiple of four are copied one by one.
-__device__ __forceinline__ void copy_to_lds(const float* src, float* dst, int count, int lane)
+// A run of kFloat4s * 64 float4 (or fewer) on its way through a wavefront's registers.
+template <int kFloat4s>
+struct InFlight {
+    floatx4 v[kFloat4s];
+    // The whole fours of `count` floats (both uniform): buffer loads, whose descriptor holds the address and gives zeros past
+    // the last of them, so that no lane needs an address of its own.  No rows, no request, but no branch either: behind one
+    // the compiler no longer knows how many loads are under way, and waits for all of them.
+    __device__ __forceinline__ void request(const float* src, int count, int lane)
+    {
+        const auto from = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), 0, 4 * (count & ~3), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < kFloat4s; ++i)
+            v[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(from, 16 * lane, 1024 * i, 0));
+    }
+    __device__ __forceinline__ void store(float* dst, int space, int lane) const
+    {
+#pragma unroll
+        for (int i = 0; i < kFloat4s; ++i)
+            if (64 * i + lane < space / 4) reinterpret_cast<floatx4*>(dst)[64 * i + lane] = v[i];
+    }
+};
+// The floats behind the last whole four of `count` (the last tile's rows may end in between).
+__device__ __forceinline__ void copy_rest(const float* __restrict__ src, float* dst, int count, int lane)
 {
-    typedef __attribute__((address_space(1))) const void global_void;
-    typedef __attribute__((address_space(3))) void lds_void;
-    for (int i = 0; i < count / 4; i += 64)  // uniform
-        if (i + lane < count / 4)            // (lane l of a copy writes float4 l behind the uniform LDS address)
-            __builtin_amdgcn_global_load_lds((global_void*)(src + 4 * (i + lane)), (lds_void*)(dst + 4 * i), 16, 0, 0);
     if (lane < (count & 3)) dst[(count & ~3) + lane] = src[(count & ~3) + lane];
 }
 
 // A wavefront keeps all 11 blocks of 32 x 32 weight gradients in registers, so there is one wavefront per SIMD and a
-// workgroup per compute unit, each with its own quarter of the LDS for the tile's rows; tiles come from memory straight to
-// LDS.  146 us at 200k anchors (37 us of matrix instructions; the rest is the wait for a tile's rows, which one wavefront
-// per SIMD does not hide).
+// workgroup per compute unit, each with its own quarter of the LDS for the tile's rows.  Nothing else hides the wait for a
+// tile's rows: the next tile's are requested, into registers, as soon as this one's have gone to LDS, and arrive while it is
+// worked on (copies straight to LDS make every later read of LDS wait for them).  86 us at 200k anchors: 37 us of matrix instructions, some 11 us for a tile's 7.4 us of them, since the operands of the next are read from
+// LDS while one runs, and not earlier; 8 us for the weights, 4 for adding up the gradients, and a last round of tiles in a
+// third of the wavefronts.  Rows requested when they are needed, weights one after the other, the last tile's rows too, and
+// gradients added by one wavefront after the other: 145.
 // kAnchor: the anchors' own gradient is wanted (the layers are then also walked back to view direction and distance).
-// kOffsets: offsets per anchor, or 0 (d.n).  Ten, the decoder's default, has its loops unrolled; with the count a variable
-// the compiler spills 16 registers (33 with kAnchor), and the kernel takes 185 us at ten offsets instead of 146 (206 and 162
-// with kAnchor; 200k anchors).  Any other count takes the variable one: 166 us at eight offsets (unrolled 134), 137 at four
-// (111), 175 at nine (whose odd counts an unrolled loop would have to guard).  A copy of the kernel for each of them would
-// take 25 to 32 us off a training step of more than a millisecond; only the default has one.
+// kOffsets: offsets per anchor, or 0 (d.n).  Ten, the decoder's default, has its loops unrolled and requests rows ahead; with
+// the count a variable there are no registers for that (400 bytes per lane were spilled), and the rows are requested together
+// when they are needed.  At 200k anchors 89 us (105 with kAnchor) with ten offsets; with the variable count 123 (141) at
+// eight and 98 (114) at four.
 template <bool kAnchor, int kOffsets>
 __global__ __launch_bounds__(64 * kBackwardWaves) void train_layers_kernel(
     TrainArgs d, const uint32_t* __restrict__ rows, const float* __restrict__ d_op, const float* __restrict__ d_cov,
     const float* __restrict__ d_col, gs355_decode_gradients out, float* __restrict__ partials)
 {
-    __shared__ HeadParameters s;
-    __shared__ __align__(16) float s_pre[kBackwardWaves][kTilePre];       // gradients of the pre-activations, head by head as in memory
-    __shared__ __align__(16) float s_in[kBackwardWaves][kGroup * 36];     // input rows
-    __shared__ __align__(16) float s_hidden[kBackwardWaves][kGroup * 32];  // one head's hidden units, by row
-    __shared__ float s_unit[kBackwardWaves][kGroup * kW1Stride];          // ... and their gradients
-    load_parameters(s, d);
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
-    const int n = kOffsets ? kOffsets : d.n, outputs = 11 * n;
+    // the parameters, then the wavefronts' parts; at the end the wavefronts' weight gradients, one after the other
+    __shared__ __align__(16) float s_all[kGradFloats + kBackwardWaves * kWaveFloats];
+    static_assert(kGradFloats % 4 == 0 && kWaveFloats % 4 == 0 && kBackwardWaves * kGradFloats <= kGradFloats + kBackwardWaves * kWaveFloats, "");
+    HeadParameters& s = *reinterpret_cast<HeadParameters*>(s_all);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
+    const int n = kOffsets ? kOffsets : d.n;
     const int width = d.with_dist ? 36 : 35;
     const float* const input_rows = d.with_dist ? d.with_dist : d.without;
-    float* const pre = s_pre[wave];
-    float* const input = s_in[wave];
-    float* const hidden = s_hidden[wave];
-    float* const unit = s_unit[wave];
+    // a tile's rows on their way
+    InFlight<(kGroup * kMaxOffsets / 4 + 63) / 64> fly_op;
+    InFlight<(kGroup * 7 * kMaxOffsets / 4 + 63) / 64> fly_cov;
+    InFlight<(kGroup * 3 * kMaxOffsets / 4 + 63) / 64> fly_col;
+    InFlight<(kGroup * 36 / 4 + 63) / 64> fly_in;
+    InFlight<kGroup * kFeat / 4 / 64> fly_hidden;  // one head's
+    constexpr bool kAhead = kOffsets != 0;         // (with loops of unknown length there are no registers for them)
+    const uint32_t stride = gridDim.x * kBackwardWaves;
+    auto rows_of = [&](uint32_t tile) { return (int)min(d.V - min(tile * kGroup, d.V), (uint32_t)kGroup); };
+    auto request_rows = [&](uint32_t tile) {
+        const size_t row0 = (size_t)tile * kGroup;
+        const int count = rows_of(tile);
+        fly_op.request(d_op + row0 * n, count * n, lane);
+        fly_cov.request(d_cov + row0 * 7 * n, count * 7 * n, lane);
+        fly_col.request(d_col + row0 * 3 * n, count * 3 * n, lane);
+        fly_in.request(input_rows + row0 * width, count * width, lane);
+    };
+    auto request_hidden = [&](int j, uint32_t tile) {
+        fly_hidden.request(d.hidden[j] + (size_t)tile * kGroup * kFeat, rows_of(tile) * kFeat, lane);
+    };
+    const uint32_t first_tile = blockIdx.x * kBackwardWaves + wave;
+    if (kAhead) {
+        request_rows(first_tile);
+        request_hidden(0, first_tile);
+    }
+    static_assert(kBackwardWaves == 4, "");
+    load_parameters(s, d);
+    __syncthreads();
 
     floatx16 grad1[5] = {}, grad0[6] = {};  // dW1: opacity | covariance x 3 | colour; dW0: features, extras + bias per head
-    float bias1[2] = {0.f, 0.f};            // db1 of outputs lane and 64 + lane
+    float bias1[5] = {};                    // db1 of the rows of grad1, the even and the odd rows' in either half of the lanes
     const uint32_t tiles = (d.V + kGroup - 1) / kGroup;
-    for (uint32_t tile = blockIdx.x * kBackwardWaves + wave; tile < tiles; tile += gridDim.x * kBackwardWaves) {
+    for (uint32_t tile = first_tile; tile < tiles; tile += stride) {
         const uint32_t row0 = tile * kGroup, r = min(row0 + (uint32_t)col, d.V - 1);
         const bool live = row0 + (uint32_t)col < d.V;
-        const int tile_rows = (int)min((uint32_t)kGroup, d.V - row0);
-        if (tile_rows < kGroup) {  // (rows that do not exist: zeros)
-            for (int i = lane; i < kGroup * outputs; i += 64) pre[i] = 0.0f;
-            for (int i = lane; i < kGroup * width; i += 64) input[i] = 0.0f;
-            for (int i = lane; i < kGroup * kFeat; i += 64) hidden[i] = 0.0f;
-            wave_lds_sync();
+        const int tile_rows = rows_of(tile);  // uniform
+        // (an offset that the compiler does not know: it would keep dozens of addresses in registers over the tiles)
+        int from = 0;
+        asm volatile("" : "+s"(from));
+        float* const pre = s_all + kGradFloats + wave * kWaveFloats + from;
+        float* const input = pre + kWaveIn;
+        float* const hidden = pre + kWaveHidden;
+        float* const unit = pre + kWaveUnit;
+        const uint32_t target = d.compact_feat ? r : rows[r];  // the row of the features' gradient
+        if (!kAhead) request_rows(tile);
+        fly_op.store(pre, kGroup * n, lane);
+        fly_cov.store(pre + kGroup * n, kGroup * 7 * n, lane);
+        fly_col.store(pre + kGroup * 8 * n, kGroup * 3 * n, lane);
+        fly_in.store(input, kGroup * width, lane);
+        if (tile_rows < kGroup) {
+            copy_rest(d_op + (size_t)row0 * n, pre, tile_rows * n, lane);
+            copy_rest(d_cov + (size_t)row0 * 7 * n, pre + kGroup * n, tile_rows * 7 * n, lane);
+            copy_rest(d_col + (size_t)row0 * 3 * n, pre + kGroup * 8 * n, tile_rows * 3 * n, lane);
+            copy_rest(input_rows + (size_t)row0 * width, input, tile_rows * width, lane);
         }
-        copy_to_lds(d_op + (size_t)row0 * n, pre, tile_rows * n, lane);
-        copy_to_lds(d_cov + (size_t)row0 * 7 * n, pre + kGroup * n, tile_rows * 7 * n, lane);
-        copy_to_lds(d_col + (size_t)row0 * 3 * n, pre + kGroup * 8 * n, tile_rows * 3 * n, lane);
-        copy_to_lds(input_rows + (size_t)row0 * width, input, tile_rows * width, lane);
-        copy_to_lds(d.hidden[0] + (size_t)row0 * kFeat, hidden, tile_rows * kFeat, lane);
+        if (kAhead) request_rows(tile + stride);
         floatx16 d_feat = {}, d_extra = {};
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const int base = head_base(j, n), count = head_outputs(j, n);
-            float relu[16];  // the hidden units of this lane's row, in accumulator order (only their sign is used)
+            if (!kAhead) request_hidden(j, tile);
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const float4 v = reinterpret_cast<const float4*>(d.hidden[j] + (size_t)r * kFeat)[2 * b + half];
-                relu[4 * b] = v.x, relu[4 * b + 1] = v.y, relu[4 * b + 2] = v.z, relu[4 * b + 3] = v.w;
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies have landed
+            for (int i = 0; i < kGroup * kFeat / 4 / 64; ++i)  // the lane's float4 of row 8 i + lane / 8
+                *reinterpret_cast<floatx4*>(hidden + (8 * i + (lane >> 3)) * kHiddenStride + 4 * (lane & 7)) = fly_hidden.v[i];
+            if (kAhead) request_hidden(j < 2 ? j + 1 : 0, j < 2 ? tile : tile + stride);
             wave_lds_sync();
             // the head's gradients: row stride `count`, conflict-free for the counts of ten offsets (twice an odd number)
             const float* const g = pre + kGroup * base;
             floatx16 dh = {};
             {
-                const float* const w1 = s.w1 + base * kW1Stride + col;  // transposed: this lane's hidden unit
+                const float* const w1 = s.w1 + base * kW1Stride + col + from;  // transposed: this lane's hidden unit
                 const int steps = (count + 1) / 2;
                 constexpr int kUnroll = kOffsets ? 35 : 1;
 #pragma unroll kUnroll
@@ -571,33 +649,30 @@ __global__ __launch_bounds__(64 * kBackwardWaves) void train_layers_kernel(
                 }
             }
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                dh[v] = relu[v] > 0.0f ? dh[v] : 0.0f;
-                unit[col * kW1Stride + unit_of(v, half)] = dh[v];
+            for (int b = 0; b < 4; ++b) {  // the hidden units of this lane's row, in accumulator order (only their sign is used)
+                const floatx4 relu = *reinterpret_cast<const floatx4*>(hidden + col * kHiddenStride + 4 * (2 * b + half));
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    dh[4 * b + t] = relu[t] > 0.0f ? dh[4 * b + t] : 0.0f;
+                    unit[col * kW1Stride + unit_of(4 * b + t, half)] = dh[4 * b + t];
+                }
             }
             // dW1 and db1: products over the tile's rows
 #pragma unroll
             for (int q = 0; q < (j == 1 ? 3 : 1); ++q) {
                 if (32 * q >= count) break;  // uniform
                 const int o = min(32 * q + col, count - 1);  // (rows past the head's last output are not used)
-                floatx16& acc = grad1[j == 0 ? 0 : j == 1 ? 1 + q : 4];
+                const int at = j == 0 ? 0 : j == 1 ? 1 + q : 4;
 #pragma unroll
-                for (int k = 0; k < 16; ++k)
-                    acc = mfma(g[(2 * k + half) * count + o], hidden[(2 * k + half) * kFeat + col], acc);
-            }
-            {
-                const int o0 = lane - base, o1 = 64 + lane - base;
-                if (o0 >= 0 && o0 < count)
-#pragma unroll 8
-                    for (int k = 0; k < kGroup; ++k) bias1[0] += g[k * count + o0];
-                if (o1 >= 0 && o1 < count)
-#pragma unroll 8
-                    for (int k = 0; k < kGroup; ++k) bias1[1] += g[k * count + o1];
+                for (int k = 0; k < 16; ++k) {
+                    const float left = g[(2 * k + half) * count + o];
+                    grad1[at] = mfma(left, hidden[(2 * k + half) * kHiddenStride + col], grad1[at]);
+                    bias1[at] += left;
+                }
             }
             wave_lds_sync();
-            if (j < 2) copy_to_lds(d.hidden[j + 1] + (size_t)row0 * kFeat, hidden, tile_rows * kFeat, lane);
             // back to the inputs, and dW0
-            const float* const w0 = s.w0[j];
+            const float* const w0 = s.w0[j] + from;
 #pragma unroll
             for (int v = 0; v < 16; ++v) d_feat = mfma(w0[unit_of(v, half) * kW0Stride + col], dh[v], d_feat);
             if (kAnchor) {
@@ -617,7 +692,7 @@ __global__ __launch_bounds__(64 * kBackwardWaves) void train_layers_kernel(
             wave_lds_sync();
         }
         if (live && out.feat) {
-            float4* const dst = reinterpret_cast<float4*>(out.feat + (d.compact_feat ? (size_t)r : (size_t)rows[r]) * kFeat);
+            float4* const dst = reinterpret_cast<float4*>(out.feat + (size_t)target * kFeat);
 #pragma unroll
             for (int b = 0; b < 4; ++b)
                 dst[2 * b + half] = make_float4(d_feat[4 * b], d_feat[4 * b + 1], d_feat[4 * b + 2], d_feat[4 * b + 3]);
@@ -634,40 +709,40 @@ __global__ __launch_bounds__(64 * kBackwardWaves) void train_layers_kernel(
         }
     }
 
-    // ---- the workgroup's weight gradients, its wavefronts one after the other, over the parameters' LDS ----
+    // ---- the wavefronts' weight gradients side by side in LDS (what is no gradient is not read), then their sums in order ----
     __syncthreads();
-    float* const sums0 = s.w0[0];
-    float* const sums1 = s.w1;
-    for (int i = threadIdx.x; i < 3 * 32 * kW0Stride; i += blockDim.x) sums0[i] = 0.0f;
-    for (int i = threadIdx.x; i < kRows * kW1Stride; i += blockDim.x) sums1[i] = 0.0f;
-    for (int w = 0; w < kBackwardWaves; ++w) {
-        __syncthreads();
-        if (wave != w) continue;
+    float* const mine = s_all + wave * kGradFloats;
+    float* const mine1 = mine + 3 * 32 * kW0Stride;
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int base = head_base(j, n), count = head_outputs(j, n);
+    for (int j = 0; j < 3; ++j) {
+        const int base = head_base(j, n), count = head_outputs(j, n);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            float* const dst = mine + j * 32 * kW0Stride + unit_of(v, half) * kW0Stride;
+            dst[col] = grad0[2 * j][v];
+            if (col < width - 32) dst[32 + col] = grad0[2 * j + 1][v];
+            else if (col == width - 32) dst[36] = grad0[2 * j + 1][v];  // (the bias keeps its column)
+            else if (col == 4) dst[35] = 0.0f;  // (no rows at all, and so no input rows that would tell their width)
+        }
+#pragma unroll
+        for (int q = 0; q < (j == 1 ? 3 : 1); ++q)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                float* const dst = s.w0[j] + unit_of(v, half) * kW0Stride;
-                dst[col] += grad0[2 * j][v];
-                if (col < width - 32) dst[32 + col] += grad0[2 * j + 1][v];
-                else if (col == width - 32) dst[36] += grad0[2 * j + 1][v];  // (the bias keeps its column)
+                const int o = 32 * q + unit_of(v, half);
+                if (o < count) mine1[(base + o) * kW1Stride + col] = grad1[j == 0 ? 0 : j == 1 ? 1 + q : 4][v];
             }
 #pragma unroll
-            for (int q = 0; q < (j == 1 ? 3 : 1); ++q)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int o = 32 * q + unit_of(v, half);
-                    if (o < count) sums1[(base + o) * kW1Stride + col] += grad1[j == 0 ? 0 : j == 1 ? 1 + q : 4][v];
-                }
+        for (int q = 0; q < (j == 1 ? 3 : 1); ++q) {
+            const float part = bias1[j == 0 ? 0 : j == 1 ? 1 + q : 4], sum = part + __shfl_xor(part, 32, 64);
+            if (half == 0 && 32 * q + col < count) mine1[(base + 32 * q + col) * kW1Stride + 32] = sum;
         }
-        if (lane < outputs) sums1[lane * kW1Stride + 32] += bias1[0];
-        if (64 + lane < outputs) sums1[(64 + lane) * kW1Stride + 32] += bias1[1];
     }
     __syncthreads();
     float* const to = partials + (size_t)blockIdx.x * kGradFloats;
-    for (int i = threadIdx.x; i < 3 * 32 * kW0Stride; i += blockDim.x) to[i] = sums0[i];
-    for (int i = threadIdx.x; i < kRows * kW1Stride; i += blockDim.x) to[3 * 32 * kW0Stride + i] = sums1[i];
+    static_assert(kBackwardWaves == 4, "");
+#pragma unroll 4
+    for (int i = threadIdx.x; i < kGradFloats; i += 64 * kBackwardWaves)
+        to[i] = ((s_all[i] + s_all[kGradFloats + i]) + s_all[2 * kGradFloats + i]) + s_all[3 * kGradFloats + i];
 }
 
 // Sixty-four elements of the weight gradients per workgroup, the workgroups' contributions split over 16 wavefronts.

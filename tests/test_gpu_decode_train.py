@@ -76,6 +76,15 @@ def test_decode_and_gradients(gpu_device, A, n, visible, dist, level, bank):
         _close(a.grad, b.grad, name)
 
 
+@pytest.mark.parametrize("A,n,dist", [
+    (34_001, 3, (False, False, False)), (33_025, 10, (False, False, False)), (70_003, 10, (True, False, True)),
+    (32_769, 9, (True, True, True))])
+def test_several_tiles_per_wavefront(gpu_device, A, n, dist):
+    """The layers' backward pass requests a tile's rows while it works on the one before (more than 32768 rows), and the last
+    tile's end between whole fours of floats."""
+    test_decode_and_gradients(gpu_device, A, n, 1.0, dist, False, False)
+
+
 @pytest.mark.parametrize("how", ["save_on_cpu", "checkpoint"])
 @pytest.mark.parametrize("bank", [False, True])
 def test_gradients_under_saved_tensor_hooks(gpu_device, how, bank):
