@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void train_inputs_kernel(TrainArgs d, const ui
 // 4 q + r) becomes the second's right operand by two lane exchanges per pair of registers.  Outputs pass through LDS so
 // that they leave in 16-byte stores (a row of 70 is not a multiple of that).
 // Six library products, three activations and a counting pass took 250 us at 200k anchors (176k of them visible, ten
-// offsets); this takes 66 us for the 170 MB it moves.
+// offsets); this takes 59 us for the 170 MB it moves.
 // The rows are as many as the device-side count of visible anchors says, `visible_rows`: nothing is read back before the
 // number of kept offsets is.
 constexpr int kHeadBlocks = 8;                           // of 16 outputs: opacity 1, covariance up to 5, colour up to 2
@@ -232,7 +232,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 {
     __shared__ float s_b0[3][32];
     __shared__ float s_b1[kHeadBlocks * 16];
-    __shared__ __align__(16) float s_out[4][kHeadOut];
+    // the weights on their way to registers, then the outputs of each wavefront's 16 rows
+    __shared__ __align__(16) float s_all[kGradFloats > 4 * kHeadOut ? kGradFloats : 4 * kHeadOut];
+    HeadParameters& s_parameters = *reinterpret_cast<HeadParameters*>(s_all);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, quarter = lane >> 4, col = lane & 15;
     const int n = d.n;
     const uint32_t groups = (d.V + kGroup - 1) / kGroup;  // that have a place in `totals`
@@ -246,6 +248,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         s_b1[i] = o < head_outputs(j, n) ? d.b1[j][o] : 0.0f;
     }
     auto input_of = [&](int step) { return step < 8 ? 8 * (step / 2) + 2 * quarter + (step & 1) : 32 + quarter; };
+    // (by way of LDS: a lane's own 118 loads from 64 places each took 15 to 20 us)
+    load_parameters(s_parameters, d);
+    __syncthreads();
     float w0[3][2][9], w1[kHeadBlocks][8];  // lane (quarter, column i): unit 16 block + i, input_of(step)
 #pragma unroll
     for (int j = 0; j < 3; ++j)
@@ -254,16 +259,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int k = 0; k < 9; ++k) {
                 const int in = input_of(k);
-                w0[j][h][k] = in < d.in_dim[j] ? d.w0[j][(16 * h + col) * d.in_dim[j] + in] : 0.0f;
+                w0[j][h][k] = s_parameters.w0[j][(16 * h + col) * kW0Stride + in];  // (zero past the head's inputs)
             }
 #pragma unroll
     for (int blk = 0; blk < kHeadBlocks; ++blk) {
         const int j = block_head(blk), o = block_first(blk) + col;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) w1[blk][k] = o < head_outputs(j, n) ? d.w1[j][o * kFeat + input_of(k)] : 0.0f;
+        for (int k = 0; k < 8; ++k)
+            w1[blk][k] = o < head_outputs(j, n) ? s_parameters.w1[(head_base(j, n) + o) * kW1Stride + input_of(k)] : 0.0f;
     }
     __syncthreads();
-    float* const out = s_out[wave];
+    float* const out = s_all + wave * kHeadOut;
     for (uint32_t tile = blockIdx.x * 4 + wave; tile < groups; tile += gridDim.x * 4) {
         const uint32_t row0 = tile * kGroup;
         if (row0 >= V) {  // (the scan goes over all places)
@@ -354,80 +360,70 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// The items (row, offset) of a group of 32 rows, row-major (the output order), two per thread of a workgroup of 256: the
-// first output slots of the workgroup's four wavefronts in either round.
-struct GroupItems {
+// The items (row, offset) of a group of 32 rows, row-major (the output order), one per thread of a workgroup of 32 n rounded
+// up to wavefronts.  (Two rounds of 256 threads, the second mostly empty: emit 59 us, items 57; one round: 51 and 53.)
+constexpr int kItemThreads = kGroup * kMaxOffsets;
+static_assert(kItemThreads % 64 == 0, "");
+int item_threads(int n) { return (kGroup * n + 63) / 64 * 64; }
+struct GroupItem {
     int count;             // of the group
-    uint32_t slot[2];      // this thread's, were its item kept
-    bool kept[2];
-    float pre[2];          // opacity pre-activations
+    uint32_t slot;         // this thread's, were its item kept
+    bool kept;
+    float pre;             // opacity pre-activation
 };
-__device__ __forceinline__ void group_items(const TrainArgs& d, uint32_t group, uint32_t first_slot, GroupItems& g)
+__device__ __forceinline__ GroupItem group_item(const TrainArgs& d, uint32_t group, uint32_t first_slot)
 {
-    __shared__ uint32_t s_kept[2][4];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ uint32_t s_kept[kItemThreads / 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, it = threadIdx.x;
     const size_t row0 = (size_t)group * kGroup;
+    GroupItem g;
     g.count = (int)min((size_t)kGroup, (size_t)d.V - row0) * d.n;
-    uint64_t mask[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int it = 256 * i + (int)threadIdx.x;
-        g.pre[i] = d.pre[0][row0 * d.n + min(it, g.count - 1)];
-        g.kept[i] = it < g.count && g.pre[i] > 0.0f;
-        mask[i] = __ballot(g.kept[i]);
-        if (lane == 0) s_kept[i][wave] = (uint32_t)__popcll(mask[i]);
-    }
+    g.pre = d.pre[0][row0 * d.n + min(it, g.count - 1)];
+    g.kept = it < g.count && g.pre > 0.0f;
+    const uint64_t mask = __ballot(g.kept);
+    if (lane == 0) s_kept[wave] = (uint32_t)__popcll(mask);
     __syncthreads();
-    uint32_t slot = first_slot;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        for (int w = 0; w < 4; ++w) {
-            if (w == wave) g.slot[i] = slot + lanes_below_in(mask[i]);
-            slot += s_kept[i][w];
-        }
-    }
+    g.slot = first_slot + lanes_below_in(mask);
+    for (int w = 0; w < wave; ++w) g.slot += s_kept[w];
+    return g;
 }
 
-// One workgroup per group, an item per thread and round.  Memory-bound: some 130 MB at 200k anchors in 54 us.
-__global__ __launch_bounds__(256) void train_emit_kernel(TrainArgs d, const uint2* __restrict__ base, uint32_t capacity,
+// Memory-bound: some 130 MB at 200k anchors.
+__global__ __launch_bounds__(kItemThreads) void train_emit_kernel(TrainArgs d, const uint2* __restrict__ base, uint32_t capacity,
                                                          gs355_decoded out, const uint32_t* __restrict__ rows)
 {
     const int n = d.n, inv_n = (65536 + n - 1) / n;  // item / n == (item * inv_n) >> 16 for item < 32 n
     const size_t row0 = (size_t)blockIdx.x * kGroup;
-    GroupItems g;
-    group_items(d, blockIdx.x, base[blockIdx.x].x, g);
+    const GroupItem g = group_item(d, blockIdx.x, base[blockIdx.x].x);
+    const int it = threadIdx.x;
+    if (it >= g.count) return;
+    const int rl = (it * inv_n) >> 16, m = it - rl * n;
+    const size_t item = row0 * n + it, pos = g.slot;
+    const float t = tanhf(g.pre);
+    out.neural_opacity[item] = t;
+    out.mask[item] = g.kept ? 1 : 0;
+    if (!g.kept || pos >= capacity) return;  // (the second cannot happen: capacity comes from the count pass)
+    const size_t a = rows[row0 + rl];
+    const float* __restrict__ c7 = d.pre[1] + 7 * item;
+    const float* __restrict__ c3 = d.pre[2] + 3 * item;
+    out.opacity[pos] = t;
+    const float q[4] = {c7[3], c7[4], c7[5], c7[6]};
+    const float norm = quaternion_norm(q);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int it = 256 * i + (int)threadIdx.x;
-        if (it >= g.count) continue;
-        const int rl = (it * inv_n) >> 16, m = it - rl * n;
-        const size_t item = row0 * n + it, pos = g.slot[i];
-        const float t = tanhf(g.pre[i]);
-        out.neural_opacity[item] = t;
-        out.mask[item] = g.kept[i] ? 1 : 0;
-        if (!g.kept[i] || pos >= capacity) continue;  // (the second cannot happen: capacity comes from the count pass)
-        const size_t a = rows[row0 + rl];
-        const float* __restrict__ c7 = d.pre[1] + 7 * item;
-        const float* __restrict__ c3 = d.pre[2] + 3 * item;
-        out.opacity[pos] = t;
-        const float q[4] = {c7[3], c7[4], c7[5], c7[6]};
-        const float norm = quaternion_norm(q);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            out.color[3 * pos + k] = logistic(c3[k]);
-            out.scaling[3 * pos + k] = d.scaling[6 * a + 3 + k] * logistic(c7[k]);
-            out.xyz[3 * pos + k] = d.anchor[3 * a + k] + d.offset[(a * n + m) * 3 + k] * d.scaling[6 * a + k];
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) out.rot[4 * pos + k] = q[k] / norm;
+    for (int k = 0; k < 3; ++k) {
+        out.color[3 * pos + k] = logistic(c3[k]);
+        out.scaling[3 * pos + k] = d.scaling[6 * a + 3 + k] * logistic(c7[k]);
+        out.xyz[3 * pos + k] = d.anchor[3 * a + k] + d.offset[(a * n + m) * 3 + k] * d.scaling[6 * a + k];
     }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) out.rot[4 * pos + k] = q[k] / norm;
 }
 
 // Cotangents of the outputs to those of the pre-activations (`d_pre`, shaped as d.pre), and what does not go through the
 // heads: gradients of offsets and scales, and the anchors' part through the Gaussians' positions.  A row's sums over its
-// offsets are taken in their order from LDS.  Memory-bound: some 210 MB at 200k anchors in 57 us (inside the kernel below,
-// a wavefront at a time, it was most of 389 us).
-__global__ __launch_bounds__(256) void train_items_kernel(TrainArgs d, const uint2* __restrict__ base,
+// offsets are taken in their order from LDS.  Memory-bound: some 210 MB at 200k anchors (inside the
+// kernel below, a wavefront at a time, it was most of 389 us).
+__global__ __launch_bounds__(kItemThreads) void train_items_kernel(TrainArgs d, const uint2* __restrict__ base,
                                                           const uint32_t* __restrict__ rows, gs355_decode_cotangents g,
                                                           gs355_decode_gradients out, float* __restrict__ d_op,
                                                           float* __restrict__ d_cov, float* __restrict__ d_col)
@@ -435,18 +431,15 @@ __global__ __launch_bounds__(256) void train_items_kernel(TrainArgs d, const uin
     __shared__ float s_part[kGroup * kMaxOffsets][9];  // an item's share of d scaling (6) and d anchor (3)
     const int n = d.n, inv_n = (65536 + n - 1) / n;
     const size_t row0 = (size_t)blockIdx.x * kGroup;
-    GroupItems items;
-    group_items(d, blockIdx.x, base[blockIdx.x].x, items);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int it = 256 * i + (int)threadIdx.x;
-        if (it >= items.count) continue;
+    const GroupItem items = group_item(d, blockIdx.x, base[blockIdx.x].x);
+    const int it = threadIdx.x;
+    if (it < items.count) {
         const int rl = (it * inv_n) >> 16, m = it - rl * n;
-        const size_t item = row0 * n + it, pos = items.slot[i], a = rows[row0 + rl];
+        const size_t item = row0 * n + it, pos = items.slot, a = rows[row0 + rl];
         float dt = g.neural_opacity ? g.neural_opacity[item] : 0.0f;
         float c7[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, c3[3] = {0.f, 0.f, 0.f}, d_off[3] = {0.f, 0.f, 0.f};
         float part[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (items.kept[i]) {
+        if (items.kept) {
             if (g.opacity) dt += g.opacity[pos];
             float sc[6];
 #pragma unroll
@@ -483,7 +476,7 @@ __global__ __launch_bounds__(256) void train_items_kernel(TrainArgs d, const uin
 #pragma unroll
             for (int k = 0; k < 4; ++k) c7[3 + k] = d_q[k];
         }
-        const float t = tanhf(items.pre[i]);
+        const float t = tanhf(items.pre);
         // (fused: close to saturation t * t rounded by itself would be wrong by a good part of the difference)
         d_op[item] = dt * __builtin_fmaf(-t, t, 1.0f);
 #pragma unroll
@@ -497,7 +490,7 @@ __global__ __launch_bounds__(256) void train_items_kernel(TrainArgs d, const uin
         for (int k = 0; k < 9; ++k) s_part[it][k] = part[k];
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < 9 * (items.count / n); k += 256) {
+    for (int k = threadIdx.x; k < 9 * (items.count / n); k += (int)blockDim.x) {
         const int rl = k / 9, c = k % 9;
         float sum = 0.0f;
         for (int m = 0; m < n; ++m) sum += s_part[rl * n + m][c];
@@ -938,7 +931,7 @@ int gs355_decode_train(const gs355_decoder* dec, const gs355_anchors* an, const 
             if (!out->neural_opacity || !out->mask ||
                 (capacity > 0 && (!out->xyz || !out->color || !out->opacity || !out->scaling || !out->rot)))
                 return set_error(GS355_EINVAL, "decoded outputs must all be non-NULL");
-            hipLaunchKernelGGL(train_emit_kernel, dim3(groups), dim3(256), 0, s, a, base, (uint32_t)capacity, *out, list);
+            hipLaunchKernelGGL(train_emit_kernel, dim3(groups), dim3(item_threads(a.n)), 0, s, a, base, (uint32_t)capacity, *out, list);
             GS355_CHECK_LAUNCH("decode train: emit");
             return GS355_OK;
         default: return set_error(GS355_EINVAL, "phase must be one of GS355_TRAIN_* (got 0x%x)", phase);
@@ -974,7 +967,7 @@ int gs355_decode_train_backward(const gs355_decoder* dec, const gs355_anchors* a
     for (int j = 0; j < 3; ++j) d_pre[j] = reinterpret_cast<float*>(sc + S.d_pre[j]);
     float* partials = reinterpret_cast<float*>(sc + S.partials);
     if (a.V > 0) {
-        hipLaunchKernelGGL(train_items_kernel, dim3((a.V + kGroup - 1) / kGroup), dim3(256), 0, s, a, base, list, *cotangents,
+        hipLaunchKernelGGL(train_items_kernel, dim3((a.V + kGroup - 1) / kGroup), dim3(item_threads(a.n)), 0, s, a, base, list, *cotangents,
                            *grads, d_pre[0], d_pre[1], d_pre[2]);
         GS355_CHECK_LAUNCH("decode train: items");
     }
