@@ -131,28 +131,17 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
         s_keys = 0;
         s_nqueue = 0;
     }
-    __syncthreads();
-    {  // this workgroup's share of the preprocess's totals (any split serves: the layout adds the shares up)
-        const int per = (n_totals + (int)gridDim.x - 1) / (int)gridDim.x, end = min(n_totals, (c + 1) * per);
-        unsigned long long keys = 0;
-        uint32_t visible = 0;
-        for (int k = c * per + tid; k < end; k += kBinThreads) {
-            const uint2 v = wave_totals[k];
-            keys += v.x;
-            visible += v.y;
-        }
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            keys += __shfl_down(keys, d, 64);
-            visible += __shfl_down(visible, d, 64);
-        }
-        if ((tid & 63) == 0 && visible) {
-            atomicAdd(&s_keys, keys);
-            atomicAdd(&s_visible, visible);
-        }
-    }
+    // the workgroup's share of the preprocess's totals (any split serves: the layout adds the shares up), requested here and
+    // added up behind the tiles
+    const int share = (n_totals + (int)gridDim.x - 1) / (int)gridDim.x, share_end = min(n_totals, (c + 1) * share);
+    const int share_first = c * share + tid;
+    const uint2 total = share_first < share_end ? wave_totals[share_first] : make_uint2(0u, 0u);
     const int g_begin = min(P, c * per_group);
     const int g_end = min(P, g_begin + per_group);
+    // a slice of few Gaussians: several lanes each, and a single round
+    const int lanes = lanes_per_gaussian(per_group), only = g_begin + tid / lanes;
+    const uint64_t only_rect = lanes > 1 && only < g_end ? rects[only] : 0ull;
+    __syncthreads();
     auto add = [&](int t) { atomicAdd(&s_count[kWide ? t >> kCoarseShift : t], 1u); };
     // large rectangles: one per wavefront at a time, 64 tiles per step (the sixteen wavefronts work on sixteen
     // rectangles side by side; the whole workgroup on one rectangle left most of its threads idle)
@@ -173,22 +162,18 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
         }
     };
 
-    const int lanes = lanes_per_gaussian(per_group);
-    if (lanes > 1) {  // (uniform; a single round)
-        if (tid == 0) s_nqueue = 0;
-        __syncthreads();
-        const int i = g_begin + tid / lanes, sub = tid % lanes;
-        if (i < g_end) {
-            const TileRegion q(rects[i], f.plain_regions);
+    if (lanes > 1) {  // (uniform)
+        const int sub = tid % lanes;
+        if (only < g_end) {
+            const TileRegion q(only_rect, f.plain_regions);
             if (q.area > kInlineTiles * lanes) {
-                if (sub == 0) s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
+                if (sub == 0) s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)only;
             } else {
-                walk_region(q, records + (size_t)i * kRecordFloats, sub, lanes, f.grid_x, add);
+                walk_region(q, records + (size_t)only * kRecordFloats, sub, lanes, f.grid_x, add);
             }
         }
         __syncthreads();
         walk_queue();
-        __syncthreads();
     } else {
         // a thread's Gaussians of a round: their rectangles are requested together, and those of the next round before
         // this round's are walked (a slice is a dozen rounds or more, each otherwise a memory latency plus its walk)
@@ -231,6 +216,24 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
             __syncthreads();
             walk_queue();
             __syncthreads();
+        }
+    }
+    if (share_first - (tid & 63) < share_end) {  // (uniform)
+        unsigned long long keys = total.x;
+        uint32_t visible = total.y;
+        for (int k = share_first + kBinThreads; k < share_end; k += kBinThreads) {
+            const uint2 v = wave_totals[k];
+            keys += v.x;
+            visible += v.y;
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            keys += __shfl_down(keys, d, 64);
+            visible += __shfl_down(visible, d, 64);
+        }
+        if ((tid & 63) == 0) {
+            atomicAdd(&s_keys, keys);
+            atomicAdd(&s_visible, visible);
         }
     }
     __syncthreads();
