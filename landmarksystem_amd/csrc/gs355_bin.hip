@@ -1009,27 +1009,6 @@ __device__ __forceinline__ void write_sorted(const Buf cur, uint32_t n, uint32_t
 }
 
 // ---------------------------------------------------------------------------
-// Lane exchanges inside the vector unit (no LDS): sums, minima and maxima over a wavefront.
-template <int kCtrl, int kRows>
-__device__ __forceinline__ uint32_t dpp(uint32_t absent, uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)absent, (int)v, kCtrl, kRows, 0xf, false);
-}
-template <typename Op>
-__device__ __forceinline__ uint32_t wave_scan(uint32_t v, uint32_t neutral, Op op)  // inclusive
-{
-    v = op(v, dpp<0x111, 0xf>(neutral, v));  // row_shr 1, 2, 4, 8
-    v = op(v, dpp<0x112, 0xf>(neutral, v));
-    v = op(v, dpp<0x114, 0xf>(neutral, v));
-    v = op(v, dpp<0x118, 0xf>(neutral, v));
-    v = op(v, dpp<0x142, 0xa>(neutral, v));  // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
-    return op(v, dpp<0x143, 0xc>(neutral, v));
-}
-__device__ __forceinline__ uint32_t wave_sum_scan(uint32_t v)
-{
-    return wave_scan(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
-}
-
 // In-LDS bucket sorter: kT threads, up to kT * kR pairs, kR of them held in each thread's registers.
 // The counting sort keeps the bucket in LDS once, as 64-bit pairs.  The radix passes it falls back to keep it as depth bits
 // and index (8 B per pair) plus two 16-bit permutations that ping-pong between passes (4 B per pair), every pass ranking

@@ -371,8 +371,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     if (kStored && alive) opacity = logistic(opacity);
     {  // the wavefront's keys and survivors: what the frame's key count is made of
         uint32_t keys = touched;
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) keys += __shfl_down(keys, d, 64);
+        keys = (uint32_t)__builtin_amdgcn_readlane((int)wave_sum_scan(keys), 63);
         const uint32_t visible = (uint32_t)__popcll(__ballot(alive));
         if ((threadIdx.x & 63) == 0 && valid) wave_totals[i >> 6] = make_uint2(keys, visible);
     }
