@@ -219,20 +219,17 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
         }
     }
     if (share_first - (tid & 63) < share_end) {  // (uniform)
-        unsigned long long keys = total.x;
+        uint64_t keys = total.x;
         uint32_t visible = total.y;
         for (int k = share_first + kBinThreads; k < share_end; k += kBinThreads) {
             const uint2 v = wave_totals[k];
             keys += v.x;
             visible += v.y;
         }
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            keys += __shfl_down(keys, d, 64);
-            visible += __shfl_down(visible, d, 64);
-        }
+        keys = wave_sum(keys);
+        visible = wave_sum(visible);
         if ((tid & 63) == 0) {
-            atomicAdd(&s_keys, keys);
+            atomicAdd(&s_keys, (unsigned long long)keys);
             atomicAdd(&s_visible, visible);
         }
     }
@@ -638,9 +635,7 @@ __global__ __launch_bounds__(64 * kPrefixParts) void slice_prefix_kernel(uint32_
     }
     if (part == 0) {
         if (live) totals[t] = total;
-        uint64_t sum64 = live ? total : 0u;  // the 64 tiles of this workgroup are one block of the layout's scan
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) sum64 += __shfl_down(sum64, d, 64);
+        const uint64_t sum64 = wave_sum((uint64_t)(live ? total : 0u));  // the 64 tiles of this workgroup are one block of the layout's scan
         if (lane == 0) block_sums[blockIdx.x] = sum64;
         if (block_classes) {  // columns are tiles: how many of the 64 fall in each larger sorter size class, a byte each
             const uint32_t v = live ? total : 0u;
@@ -713,15 +708,14 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
                 keys += v.keys;
             }
         }
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            before += __shfl_down(before, d, 64);
-            total += __shfl_down(total, d, 64);
-            vis += __shfl_down(vis, d, 64);
-            keys += __shfl_down(keys, d, 64);
-            class_before += __shfl_down(class_before, d, 64);
-            class_total += __shfl_down(class_total, d, 64);
-        }
+        before = wave_sum(before);
+        total = wave_sum(total);
+        vis = wave_sum(vis);
+        keys = wave_sum(keys);
+        // (three counts of 21 bits: two of them, and the third)
+        auto sum_classes = [](uint64_t v) { return ((uint64_t)wave_sum((uint32_t)(v >> 42)) << 42) + wave_sum((uint64_t)(v & ((1ull << 42) - 1ull))); };
+        class_before = sum_classes(class_before);
+        class_total = sum_classes(class_total);
         if (lane == 0) {
             s_before[wave] = before;
             s_total[wave] = total;
@@ -784,13 +778,8 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
     const uint32_t t = block * 64u + (uint32_t)lane;
     const bool live = t < tiles;
     const uint32_t v = live ? totals[t] : 0u;
-    uint32_t inc = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t up = __shfl_up(inc, d, 64);
-        if (lane >= d) inc += up;
-    }
     if (block * 64u >= tiles) return;  // (uniform per wavefront)
+    const uint32_t inc = wave_sum_scan(v);
     const uint32_t first = (uint32_t)base + inc - v;
     if (live) tile_base[t] = first;
     if (!kTiles) return;

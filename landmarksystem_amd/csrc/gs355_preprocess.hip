@@ -370,8 +370,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     const bool alive = radius > 0;
     if (kStored && alive) opacity = logistic(opacity);
     {  // the wavefront's keys and survivors: what the frame's key count is made of
-        uint32_t keys = touched;
-        keys = (uint32_t)__builtin_amdgcn_readlane((int)wave_sum_scan(keys), 63);
+        const uint32_t keys = wave_sum(touched);
         const uint32_t visible = (uint32_t)__popcll(__ballot(alive));
         if ((threadIdx.x & 63) == 0 && valid) wave_totals[i >> 6] = make_uint2(keys, visible);
     }
