@@ -316,12 +316,17 @@ __device__ __forceinline__ uint32_t dpp(uint32_t absent, uint32_t v)
     return (uint32_t)__builtin_amdgcn_update_dpp((int)absent, (int)v, kCtrl, kRows, 0xf, false);
 }
 template <typename Op>
-__device__ __forceinline__ uint32_t wave_scan(uint32_t v, uint32_t neutral, Op op)  // inclusive
+__device__ __forceinline__ uint32_t row_scan(uint32_t v, uint32_t neutral, Op op)  // inclusive, over each row of sixteen lanes
 {
     v = op(v, dpp<0x111, 0xf>(neutral, v));  // row_shr 1, 2, 4, 8
     v = op(v, dpp<0x112, 0xf>(neutral, v));
     v = op(v, dpp<0x114, 0xf>(neutral, v));
-    v = op(v, dpp<0x118, 0xf>(neutral, v));
+    return op(v, dpp<0x118, 0xf>(neutral, v));
+}
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, uint32_t neutral, Op op)  // inclusive
+{
+    v = row_scan(v, neutral, op);
     v = op(v, dpp<0x142, 0xa>(neutral, v));  // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
     return op(v, dpp<0x143, 0xc>(neutral, v));
 }
