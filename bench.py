@@ -134,7 +134,7 @@ def stage_breakdown(torch, pipeline, _lib, inp, n_cap, steps):
     class_counts = ((words[2] >> 32) & 0xFFFFFFFF, words[3] & 0xFFFFFFFF, (words[3] >> 32) & 0xFFFFFFFF)
     skip = sum(m for m, c in zip(_lib.STAGE_TILESORT_SKIP, class_counts) if c == 0)
     fast = [("preprocess", front), ("tile_count", _lib.STAGE_TILE_COUNT),
-            ("tile_scatter", _lib.STAGE_TILE_SCATTER), ("tile_sort", _lib.STAGE_TILESORT | skip),
+            ("tile_scatter", _lib.STAGE_TILE_SCATTER), ("tile_sort", _lib.STAGE_TILESORT | _lib.STAGE_TILESORT_VALUES | skip),
             ("blend", _lib.STAGE_BLEND)]
     classic = [("scan", _lib.STAGE_SCAN), ("duplicate", _lib.STAGE_DUPLICATE), ("sort", _lib.STAGE_SORT),
                ("ranges", _lib.STAGE_RANGES)]

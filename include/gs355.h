@@ -197,6 +197,9 @@ enum {
      * of the remaining keys.  num_keys_total, and with it the overflow of a capacity, still count whole rectangles.
      * Refused together with a classic stage (in later calls the scan goes back to whole rectangles).  No effect beyond 32767 tiles along an axis. */
     GS355_STAGE_TILE_REACH = 65536,
+    /* Modifier of TILESORT: the sorted values only.  No later stage reads the sorted keys, eight of the twelve bytes that the
+     * sort writes per key; their buffer is left as it is (its contents are then undefined). */
+    GS355_STAGE_TILESORT_VALUES = 131072,
     GS355_PIPELINE_FAST = 1 | 128 | 512 | 256 | 32
 };
 

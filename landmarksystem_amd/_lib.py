@@ -22,6 +22,7 @@ STAGE_TILE_SCATTER_ONE_LEVEL = 2048  # choose by the key count (which launches b
 TWO_LEVEL_MIN_KEYS = 6 << 20         # the device's own threshold
 STAGE_TILESORT_SKIP = (4096, 8192, 16384)  # modifiers of STAGE_TILESORT: do not launch that size class's sorter
 STAGE_TILE_REACH = 65536  # modifier of STAGE_PREPROCESS: keys only for the tiles that a Gaussian's alpha >= 1/255 ellipse reaches
+STAGE_TILESORT_VALUES = 131072  # modifier of STAGE_TILESORT: the sorted values only (no later stage reads the sorted keys)
 PIPELINE_FAST = STAGE_PREPROCESS | STAGE_TILE_COUNT | STAGE_TILE_SCATTER | STAGE_TILESORT | STAGE_BLEND
 MAX_FAST_TILES = 36000 * 16  # limits of the tile-bucketed stages (the classic stages have neither)
 MAX_FAST_GAUSSIANS = 1 << 28

@@ -30,10 +30,11 @@ constexpr size_t kAlign = 256;
 constexpr uint32_t kKnownStages = GS355_STAGE_ALL | GS355_STAGE_BLEND_PLAIN | GS355_STAGE_TILE_COUNT | GS355_STAGE_TILESORT | GS355_STAGE_TILE_SCATTER |
                                   GS355_STAGE_TILE_SCATTER_TWO_LEVEL | GS355_STAGE_TILE_SCATTER_ONE_LEVEL |
                                   GS355_STAGE_TILESORT_SKIP_1 | GS355_STAGE_TILESORT_SKIP_2 | GS355_STAGE_TILESORT_SKIP_3 |
-                                  GS355_STAGE_TILE_REACH;
+                                  GS355_STAGE_TILE_REACH | GS355_STAGE_TILESORT_VALUES;
 constexpr uint32_t kScatterModifiers = GS355_STAGE_TILE_SCATTER_TWO_LEVEL | GS355_STAGE_TILE_SCATTER_ONE_LEVEL;
 constexpr uint32_t kStageModifiers =
-    kScatterModifiers | GS355_STAGE_TILESORT_SKIP_1 | GS355_STAGE_TILESORT_SKIP_2 | GS355_STAGE_TILESORT_SKIP_3 | GS355_STAGE_TILE_REACH;
+    kScatterModifiers | GS355_STAGE_TILESORT_SKIP_1 | GS355_STAGE_TILESORT_SKIP_2 | GS355_STAGE_TILESORT_SKIP_3 | GS355_STAGE_TILE_REACH |
+    GS355_STAGE_TILESORT_VALUES;
 constexpr int64_t kMaxKeys = (1ll << 32) - 1 - kSortTile;  // key slots are indexed with u32
 
 size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
@@ -324,7 +325,7 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
             return rc;
     if (stage_mask & GS355_STAGE_TILESORT)
         if ((rc = launch_tile_sort(header, tiles, ranges, tile_lists, buckets, keys[L.sorted_buffer],
-                                   vals[L.sorted_buffer],
+                                   vals[L.sorted_buffer], (stage_mask & GS355_STAGE_TILESORT_VALUES) == 0,
                                    ((stage_mask & GS355_STAGE_TILESORT_SKIP_1) ? 1u : 0u) |
                                        ((stage_mask & GS355_STAGE_TILESORT_SKIP_2) ? 2u : 0u) |
                                        ((stage_mask & GS355_STAGE_TILESORT_SKIP_3) ? 4u : 0u),

@@ -402,7 +402,7 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
 // lists: u32[kListHeader + 4 * tiles]: the four class counts, four spare words, the four lists
 constexpr int kListHeader = 8;
 int launch_tile_sort(const gs355_header* header, int tiles, const uint32_t* ranges, uint32_t* lists,
-                     uint64_t* buckets, uint64_t* out_keys, uint32_t* out_vals, uint32_t skip_classes, hipStream_t s);
+                     uint64_t* buckets, uint64_t* out_keys, uint32_t* out_vals, bool keys_too, uint32_t skip_classes, hipStream_t s);
 
 // anchor decode: argument checks, and the exclusive prefix of per-run (kept offsets, visible anchors) with the totals
 int check_decoder(const gs355_decoder* dec, const gs355_anchors* an);

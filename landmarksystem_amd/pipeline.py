@@ -351,7 +351,7 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
         ws.key_capacity = max(1 << 20, 4 * inputs.P)
     if not classic and inputs.tiles <= _lib.MAX_FAST_TILES and inputs.P <= _lib.MAX_FAST_GAUSSIANS:
         front = _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_REACH | _lib.STAGE_TILE_COUNT
-        back = _lib.STAGE_TILE_SCATTER | _lib.STAGE_TILESORT | _lib.STAGE_BLEND
+        back = _lib.STAGE_TILE_SCATTER | _lib.STAGE_TILESORT | _lib.STAGE_TILESORT_VALUES | _lib.STAGE_BLEND
         # the scatter variant that suited the previous frame of this workspace (either is correct for any frame)
         back |= (_lib.STAGE_TILE_SCATTER_TWO_LEVEL if ws.last_num_pairs >= _lib.TWO_LEVEL_MIN_KEYS
                  else _lib.STAGE_TILE_SCATTER_ONE_LEVEL)

@@ -556,4 +556,5 @@ def test_tile_reach_is_for_the_bucketed_stages():
     for classic in (_lib.STAGE_SCAN, _lib.STAGE_DUPLICATE, _lib.STAGE_SORT, _lib.STAGE_RANGES, _lib.STAGE_ALL):
         assert "whole rectangles" in _err(_lib.GS355_EINVAL, run, _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_REACH | classic)
     assert "no known stage" in _err(_lib.GS355_EINVAL, run, _lib.STAGE_TILE_REACH)
+    assert "no known stage" in _err(_lib.GS355_EINVAL, run, _lib.STAGE_TILESORT_VALUES)
     assert "needed" in _err(_lib.GS355_ENOSPC, run, _lib.PIPELINE_FAST | _lib.STAGE_TILE_REACH)
