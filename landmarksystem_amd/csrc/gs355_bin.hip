@@ -1158,7 +1158,7 @@ struct LdsSorter {
     // monotonically and a coarse bin's end is a whole number, so the map stays monotone.
     // The pairs wait in registers, and pass through LDS three times as they are (to their bin, to its ranking readers, to
     // their place): ten LDS accesses per pair.  Kept in LDS as separate words behind a permutation they took twenty (6M
-    // Gaussians, 1080p, 13.4M pairs: the four classes 17 + 51 + 80 + 20 us, now 15 + 36 + 61 + 11).
+    // Gaussians, 1080p, 13.4M pairs: the four classes 17 + 51 + 80 + 20 us, so 15 + 36 + 61 + 11).
     // Returns false when some bin is too full for this to pay (nothing but the counters has then been written): the caller
     // runs the radix passes.
     static constexpr uint32_t kMaxBin = 256;
