@@ -240,7 +240,10 @@ __device__ __forceinline__ uint64_t tile_region(const Rect q, float px, float py
 // kStored: g holds the vanilla model's stored parameters, activated here (the activated copies would cost a pass over
 // memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
 // front of a kernel of 0.3 ms).
-template <bool kRadiiOnly, bool kStored>
+// kPacked: SH blocks of 16 coefficients at 16-byte boundaries, fetched by way of LDS.  The 53 KB of that leave three wavefronts
+// per SIMD, so calls without such blocks (colours given, or of another size) run a kernel without it, at eight: 1.5M decoded
+// Gaussians 100 -> 76 us, 600k 32.5 -> 24.5, 160k 13.8 -> 12.4.
+template <bool kRadiiOnly, bool kStored, bool kPacked>
 __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaussians g, ParameterArgs par, FilterArgs fx,
                                                          float* __restrict__ records,
                                                          uint32_t* __restrict__ tiles_touched,
@@ -250,9 +253,9 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
                                                          int32_t* __restrict__ radii)
 {
     // staging area for the 16-coefficient SH blocks of each wavefront's 64 Gaussians
-    __shared__ float4 s_sh[kRadiiOnly ? 1 : 4 * 64 * kShStride / 4];
+    __shared__ float4 s_sh[kPacked ? 4 * 64 * kShStride / 4 : 1];
     // the workgroup's surviving Gaussians, packed in order: position within the workgroup; survivors per wavefront
-    __shared__ uint8_t s_owner[kRadiiOnly ? 1 : 256];
+    __shared__ uint8_t s_owner[kPacked ? 256 : 1];
     __shared__ int s_alive[4];
 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -421,7 +424,9 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         // however many Gaussians were culled.  Other block sizes: every survivor fetches its own block.  Same
         // values and the same order of additions either way.
         const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        const bool packed = f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(kStored ? par.rest : g.shs) & 15u) == 0;  // uniform
+        // (uniform, and true wherever kPacked is; with the branches below left out of that variant the compiler orders its
+        // loads otherwise: 6M Gaussians 308 -> 325 us)
+        const bool packed = kPacked && f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(kStored ? par.rest : g.shs) & 15u) == 0;
         if (packed) {
             const uint64_t m = __ballot(alive);
             if (lane == 0) s_alive[wave] = __popcll(m);
@@ -565,15 +570,17 @@ int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const Parame
     if (g.P == 0) return GS355_OK;
     const dim3 block(256), grid((g.P + 255) / 256);
     const FilterArgs none;
-    if (radii_only)
-        hipLaunchKernelGGL((preprocess_kernel<true, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
-                           tiles_touched, rects, depth_bits, wave_totals, lit, radii);
-    else if (par)
-        hipLaunchKernelGGL((preprocess_kernel<false, true>), grid, block, 0, s, f, g, *par, none, records, tiles_touched,
-                           rects, depth_bits, wave_totals, lit, radii);
-    else
-        hipLaunchKernelGGL((preprocess_kernel<false, false>), grid, block, 0, s, f, g, ParameterArgs(), none, records,
-                           tiles_touched, rects, depth_bits, wave_totals, lit, radii);
+    const bool packed = f.sh_coeffs == 16 && (par || !g.colors_precomp) &&
+                        (reinterpret_cast<uintptr_t>(par ? par->rest : g.shs) & 15u) == 0;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, par ? *par : ParameterArgs(), none, records, tiles_touched, rects,
+                           depth_bits, wave_totals, lit, radii);
+    };
+    if (radii_only) launch(preprocess_kernel<true, false, false>);
+    else if (par && packed) launch(preprocess_kernel<false, true, true>);
+    else if (par) launch(preprocess_kernel<false, true, false>);
+    else if (packed) launch(preprocess_kernel<false, false, true>);
+    else launch(preprocess_kernel<false, false, false>);
     GS355_CHECK_LAUNCH("preprocess");
     return GS355_OK;
 }
@@ -586,9 +593,9 @@ int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const Fil
                            (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, (uint2*)nullptr, (uint8_t*)nullptr, radii);
     };
     if (x.stored)
-        launch(preprocess_kernel<true, true>);
+        launch(preprocess_kernel<true, true, false>);
     else
-        launch(preprocess_kernel<true, false>);
+        launch(preprocess_kernel<true, false, false>);
     GS355_CHECK_LAUNCH("anchor filter");
     return GS355_OK;
 }

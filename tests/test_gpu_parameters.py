@@ -132,3 +132,23 @@ def test_frame_call_reports_an_overflow_and_is_repeated(gpu_device, stored):
     assert call(want.num_keys) == (1, 0, want.num_keys, want.num_visible)
     for a, b in ((out.image, want.image), (out.depth, want.depth), (out.alpha, want.alpha), (out.radii, want.radii)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("P", [1, 255, 257, 5000])
+def test_coefficient_blocks_off_their_boundary(gpu_device, P):
+    """Blocks of 16 coefficients at 16-byte boundaries travel through LDS, others are read by their own lanes, in a kernel
+    without that room: the same sums in the same order."""
+    scene = scenes.tiny_scene(P=P, width=331, height=203, sh_degree=3, seed=P % 97)
+    settings = settings_for(scene, gpu_device)
+    d = scene.to(gpu_device)
+    room = torch.empty(P * 48 + 4, device=gpu_device)
+    outs = []
+    for first in (0, 1):
+        shs = room[first:first + P * 48].view(P, 16, 3)
+        shs.copy_(d.shs)
+        assert shs.data_ptr() % 16 == 4 * first
+        inp = pipeline.FrameInputs(settings, d.means3D, opacities=d.opacities, shs=shs, scales=d.scales, rotations=d.rotations)
+        out = pipeline.render(inp, ws=pipeline.Workspace(gpu_device))
+        outs.append((out.image.clone(), out.depth.clone(), out.radii.clone()))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
