@@ -46,7 +46,7 @@ COUNTER_TRAFFIC = {
     # profiles/bench_c3_6M_1080p_valu_counters.txt
     "blend_issued_flops": 6.69e9,
     "blend_issued_flops_source": "profiles/bench_c3_6M_1080p_valu_counters.txt",
-    "blend_valu_busy": 1.052,  # (matrix instructions count as issued and run beside the vector ones)
+    "blend_valu_busy": 1.062,  # (matrix instructions count as issued and run beside the vector ones)
 }
 
 # Same for `--config 5`: HBM bytes per launch of the two decode kernels (count + emit)
