@@ -71,8 +71,8 @@ __global__ __launch_bounds__(256) void ranges_kernel(const gs355_header* __restr
 // The lists' walk (walk_lists) evaluates the four entries of a round side by
 // side, without a branch: T never grows, so one test behind the round finds
 // the pixels that finish in it, and the round is then repeated entry by entry
-// from its alphas; and a batch whose records are all finite and `definite`
-// (kDefinite) needs no test for exponents above zero.  A branch per entry and
+// from its alphas; and a batch whose records are all finite and definite()
+// needs no test for exponents above zero.  A branch per entry and
 // test held up the issue of the next entry's instructions, above all with one
 // wavefront per SIMD: blend of 10k Gaussians at 256x256 20.4 -> 15.7 us, 1M
 // large splats at 1080p 145 -> 134, 6M 292 -> 276, 20M at 4K 706 -> 676.
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
 #pragma unroll
                 for (int b = 3; b >= 0; --b) mask = (mask << 4) | reach.row((float)b);
                 mask = reach.unless_infinite(mask, 0xFFFFu);
-                ordinary = fabsf(reach.rho) < kDefinite;
+                ordinary = definite(r0.z, reach.rho);
             }
             s_b[tid] = make_float4(-0.5f * r1.x, log2o, __uint_as_float(mask), 0.f);
             s_c[tid] = make_float4(r1.z, r1.w, r2.x, r2.y);

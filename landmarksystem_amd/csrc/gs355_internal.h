@@ -156,11 +156,16 @@ struct TileReach {
     }
 };
 
-// A splat whose |rho| is below this has no pixel with an exponent above zero.  The two square terms of the exponent outweigh
-// the mixed one by at least 1 - |rho| of their sum, and pair_exponent's five roundings are off by less than 2^-21 = 4.8e-7
-// of it (rho itself by 4e-7): the exponent comes out negative, or zero at the splat's centre.  The blends test for exponents
-// above zero only where a staged record is beyond it (axes of more than 400:1 on the screen) or not a number.
+// A splat whose conic is positive and whose |rho| is below kDefinite has no pixel with an exponent above zero.  The two square
+// terms of the exponent outweigh the mixed one by at least 1 - |rho| of their sum, and pair_exponent's five roundings are off
+// by less than 2^-21 = 4.8e-7 of it (rho itself by 4e-7): the exponent comes out negative, or zero at the splat's centre.
+// rho alone does not tell: it is that of a negative definite conic as well, which a caller's covariance can lead to (minus 0.3
+// to 0.6 square pixels, before the low-pass) and whose exponents are above zero everywhere else.  Conics of mixed signs give
+// |rho| = 1, as do products of the diagonal that are zero or not a number; finite conics of accepted splats stay below 2^50
+// (entries of a 2D covariance that are not zero are 2^-25 or more), so that the product does not overflow.  The blends test for exponents above
+// zero only where a staged record is not definite (axes of more than 400:1 on the screen, most often).
 constexpr float kDefinite = 0.99999f;
+__device__ __forceinline__ bool definite(float conic_x, float rho) { return conic_x > 0.0f && fabsf(rho) < kDefinite; }
 
 // The columns of tiles that the splat's alpha >= 1/255 ellipse can reach, for one row of tiles at a time: TileReach's span
 // with tiles in the place of blocks (the same formula, and the same slack).  Rows and columns count from tile (x0, y0).

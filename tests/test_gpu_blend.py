@@ -6,7 +6,8 @@ import pytest
 import torch
 
 from landmarksystem_amd import _lib, pipeline, scenes
-from tests.helpers import settings_for
+from oracle import c_oracle as co
+from tests.helpers import oracle_frame, oracle_gaussians, settings_for
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +50,40 @@ def test_colours_that_are_not_finite_stay_with_their_pixels(gpu_device, value):
     assert 0 < int(touched.sum()) < touched.numel()
     assert torch.equal(~torch.isfinite(images[2]), touched)
     assert torch.equal(images[2][~touched], images[0][~touched])
+
+
+def _run(scene, device, ws, mask, **kw):
+    inp = pipeline.FrameInputs(settings_for(scene, device), scene.means3D.to(device), opacities=scene.opacities.to(device), **kw)
+    out = pipeline.FrameOutputs(inp)
+    n_cap = 8_000_000
+    ws.ensure(inp.P, n_cap, inp.width, inp.height)
+    lay = pipeline.run_stages(inp, out, ws, n_cap, mask)
+    records = ws.view(lay, "records", inp.P, 0, inp.tiles)[out.radii > 0]
+    return inp, out, records.double()
+
+
+@pytest.mark.parametrize("others", [0, 300])
+def test_covariances_that_are_negative_on_the_screen_are_rejected(gpu_device, others):
+    """A negative definite conic has an exponent above zero everywhere but at its centre, and next to no correlation: it must
+    not pass for an ellipse.  Alone, and in batches with ordinary splats."""
+    scene = scenes.tiny_scene(P=400, width=133, height=75, sh_degree=0, seed=11)
+    matrix = scene.camera.world_view_transform
+    depth = scene.means3D @ matrix[:3, 2] + matrix[3, 2]
+    focal = scene.camera.width / (2.0 * math.tan(scene.camera.FovX * 0.5))
+    # minus 0.31 to 0.55 square pixels before the low-pass adds its 0.3
+    pixels = 0.31 + 0.24 * torch.rand(400, generator=torch.Generator().manual_seed(4))
+    cov = torch.zeros(400, 6)
+    cov[:, [0, 3, 5]] = -(pixels * (depth / focal) ** 2)[:, None]
+    cov[:others, [0, 3, 5]] = 0.02
+    scene.opacities[:] = 0.9
+    ws = pipeline.Workspace(gpu_device)
+    kw = dict(shs=scene.shs.to(gpu_device), cov3D_precomp=cov.to(gpu_device))
+    inp, out, records = _run(scene, gpu_device, ws, _lib.PIPELINE_FAST, **kw)
+    qx, qy, qz = records[:, 2], records[:, 3], records[:, 4]
+    assert int(((qx < 0) & (qx * qz > 4 * qy * qy)).sum()) >= 20
+    images = [out.image.clone(), out.depth.clone(), out.alpha.clone()]
+    pipeline.run_stages(inp, out, ws, 8_000_000, _lib.STAGE_BLEND_PLAIN)
+    for a, b in zip(images, (out.image, out.depth, out.alpha)):
+        assert torch.equal(a, b)
+    ref = co.render(oracle_frame(scene), oracle_gaussians(scene, cov3D_precomp=cov.numpy()))
+    assert float((images[2].cpu() - torch.from_numpy(ref["alpha"])).abs().max()) < 1e-4
