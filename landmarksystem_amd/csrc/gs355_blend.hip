@@ -71,11 +71,17 @@ __global__ __launch_bounds__(256) void ranges_kernel(const gs355_header* __restr
 // The lists' walk (walk_lists) evaluates the four entries of a round side by
 // side, without a branch: T never grows, so one test behind the round finds
 // the pixels that finish in it, and the round is then repeated entry by entry
-// from its alphas; and a batch whose records are all finite and definite()
-// needs no test for exponents above zero.  A branch per entry and
+// from its alphas; and a batch whose records are all definite() needs no test
+// for exponents above zero.  A branch per entry and
 // test held up the issue of the next entry's instructions, above all with one
 // wavefront per SIMD: blend of 10k Gaussians at 256x256 20.4 -> 15.7 us, 1M
 // large splats at 1080p 145 -> 134, 6M 292 -> 276, 20M at 4K 706 -> 676.
+// Batches with a record that is not definite make that test for each entry,
+// behind one branch per round that all lanes take alike (within 1 % of no
+// branch for the others, where a second copy of the walk spills registers and
+// the test for every batch costs up to 5 %).  One long needle is staged by many
+// tiles, and a walk entry by entry took such a scene from 151 to 203 us; this
+// one to 157.
 //
 // The accumulation itself, four channels times w, is one matrix instruction of
 // sixteen 4x4x1 products: the four lanes of a quad hold w of four consecutive
@@ -99,7 +105,7 @@ struct PixelState {
     f32x4 sums;
 };
 
-// One entry by itself: batches that are not ordinary, and the verification variant.
+// One entry by itself: batches with channels that are not finite, and the verification variant.
 // a = px, py, hx, ny;  b = hz, log2(opacity);  c = this lane's channel of (r, g, b, depth).  kPlain: every channel of the
 // batch's records is finite.  Otherwise a pixel that rejects a Gaussian must not meet its channels even with w = 0.
 template <bool kCutOnExponent, bool kPlain>
@@ -165,7 +171,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
     __shared__ float4 s_a[kBatch + 1];  // px, py, -conic_x / 2, -conic_y          (+ the null record)
     __shared__ float4 s_b[kBatch + 1];  // -conic_z / 2, log2(opacity), mask of the blocks it can reach, unused
     __shared__ float4 s_c[kBatch + 1];  // r, g, b, depth
-    __shared__ uint32_t s_wave_state[4];  // bit 0: all pixels of the wavefront finished; 1: it staged a record that is not ordinary
+    __shared__ uint32_t s_wave_state[4];  // bit 0: all pixels of the wavefront finished; it staged 1: a channel that is not finite, 2: a record that is not definite
     // per wavefront and 4x4 block: byte offsets of the staged records of the Gaussians that can reach the block
     __shared__ __align__(8) ListEntry s_list[kCull ? 4 : 1][4][kListWords];
 
@@ -201,20 +207,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
                       *reinterpret_cast<const float*>(rec_c + entry + channel)};
     };
     // the four lane groups walk their lists side by side, four entries per round
-    auto walk_lists = [&](uint32_t quads) {
+    auto walk_lists = [&](bool all_definite, uint32_t quads) {
         const uint2* __restrict__ mine = reinterpret_cast<const uint2*>(s_list[wave][group]);
         uint2 next = mine[0];  // read ahead by one round (rounds past the end are never used)
         for (uint32_t left = quads; left != 0u; --left) {
             const Staged e[4] = {fetch(next.x & 0xFFFFu), fetch(next.x >> 16), fetch(next.y & 0xFFFFu), fetch(next.y >> 16)};
             next = *++mine;
-            float alpha[4], w[4], T = p.T;
+            float power[4], t[4], alpha[4], w[4], T = p.T;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const float dx = e[q].a.x - pxf, dy = e[q].a.y - pyf;
-                const float power = pair_exponent(dx, dy, e[q].a.z, e[q].a.w, e[q].b.x);
-                const float t = __builtin_fmaf(power, 1.4426950408889634f, e[q].b.y);
-                alpha[q] = fminf(0.99f, __builtin_amdgcn_exp2f(t < kAlphaCut ? -__builtin_inff() : t));
+                power[q] = pair_exponent(dx, dy, e[q].a.z, e[q].a.w, e[q].b.x);
+                t[q] = __builtin_fmaf(power[q], 1.4426950408889634f, e[q].b.y);
             }
+            if (!all_definite) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) t[q] = power[q] > 0.0f ? -__builtin_inff() : t[q];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) alpha[q] = fminf(0.99f, __builtin_amdgcn_exp2f(t[q] < kAlphaCut ? -__builtin_inff() : t[q]));
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 w[q] = alpha[q] * T;
@@ -259,7 +270,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
     for (uint32_t base = lo; base < hi; base += kBatch) {
         const uint64_t live = __ballot(p.T > 0.0f);  // lanes whose pixel is still accumulating
         const bool wave_done = live == 0ull;
-        bool ordinary = true;
+        bool finite = true, is_definite = true;
         const uint32_t j = base + tid;
         if (j < hi) {
             const uint32_t g = values[j];
@@ -274,21 +285,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
 #pragma unroll
                 for (int b = 3; b >= 0; --b) mask = (mask << 4) | reach.row((float)b);
                 mask = reach.unless_infinite(mask, 0xFFFFu);
-                ordinary = definite(r0.z, reach.rho);
+                is_definite = definite(r0.z, reach.rho);
             }
             s_b[tid] = make_float4(-0.5f * r1.x, log2o, __uint_as_float(mask), 0.f);
             s_c[tid] = make_float4(r1.z, r1.w, r2.x, r2.y);
             // (the sum of the magnitudes overflows only where one of them is beyond 2^125: then the careful way is right too)
-            ordinary = ordinary && fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < __builtin_inff();
+            finite = fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < __builtin_inff();
         } else if (kCull) {
             s_b[tid].z = 0.0f;  // (no record: reaches no block)
         }
-        const bool all_ordinary = __ballot(!ordinary) == 0ull;
-        if (lane == 0) s_wave_state[wave] = (wave_done ? 1u : 0u) | (all_ordinary ? 0u : 2u);
+        const bool all_finite = __ballot(!finite) == 0ull, all_definite = __ballot(!is_definite) == 0ull;
+        if (lane == 0) s_wave_state[wave] = (wave_done ? 1u : 0u) | (all_finite ? 0u : 2u) | (all_definite ? 0u : 4u);
         __syncthreads();
         const uint32_t w0 = s_wave_state[0], w1 = s_wave_state[1], w2 = s_wave_state[2], w3 = s_wave_state[3];
         if ((w0 & w1 & w2 & w3 & 1u) != 0u) break;
-        const bool plain = __builtin_amdgcn_readfirstlane((int)((w0 | w1 | w2 | w3) & 2u)) == 0;
+        const int unusual = __builtin_amdgcn_readfirstlane((int)((w0 | w1 | w2 | w3) & 6u));
         const int count = (int)min((uint32_t)kBatch, hi - base);
         if (!wave_done) {
             if (kCull) {
@@ -320,10 +331,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
                         s_list[wave][b][at] = (ListEntry)kNullEntry;
                 // a wavefront's LDS operations execute in order: its list writes precede the reads below
                 wave_lds_sync();
-                if (plain) walk_lists(quads);
+                if ((unusual & 2) == 0) walk_lists(unusual == 0, quads);
                 else walk_lists_carefully(quads);
             } else {
-                if (plain) walk_all(std::true_type{}, count);
+                if (unusual == 0) walk_all(std::true_type{}, count);
                 else walk_all(std::false_type{}, count);
             }
         }

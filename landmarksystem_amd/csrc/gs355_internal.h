@@ -162,8 +162,8 @@ struct TileReach {
 // rho alone does not tell: it is that of a negative definite conic as well, which a caller's covariance can lead to (minus 0.3
 // to 0.6 square pixels, before the low-pass) and whose exponents are above zero everywhere else.  Conics of mixed signs give
 // |rho| = 1, as do products of the diagonal that are zero or not a number; finite conics of accepted splats stay below 2^50
-// (entries of a 2D covariance that are not zero are 2^-25 or more), so that the product does not overflow.  The blends test for exponents above
-// zero only where a staged record is not definite (axes of more than 400:1 on the screen, most often).
+// (entries of a 2D covariance that are not zero are 2^-25 or more), so that the product does not overflow.  The forward blend tests for exponents
+// above zero only in batches with a record that is not definite (axes of more than 400:1 on the screen, most often).
 constexpr float kDefinite = 0.99999f;
 __device__ __forceinline__ bool definite(float conic_x, float rho) { return conic_x > 0.0f && fabsf(rho) < kDefinite; }
 

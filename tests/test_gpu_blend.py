@@ -87,3 +87,46 @@ def test_covariances_that_are_negative_on_the_screen_are_rejected(gpu_device, ot
         assert torch.equal(a, b)
     ref = co.render(oracle_frame(scene), oracle_gaussians(scene, cov3D_precomp=cov.numpy()))
     assert float((images[2].cpu() - torch.from_numpy(ref["alpha"])).abs().max()) < 1e-4
+
+
+def _needles(thin, others=100_000, needles=40):
+    """Faint splats of some tiles each, and needles across the image: 300 px long and 0.5 px (thin) or 3 px wide, on a diagonal, so that their
+    correlation on the screen is beyond 0.99999 or short of it.  Either kind has so large an extent that its reach is not
+    computed: the tiles and blocks that evaluate them are the same for both."""
+    scene = scenes.tiny_scene(P=others + needles, width=1280, height=720, sh_degree=0, seed=5, log_scale_mean=-3.5, spread=1.6)
+    angle = math.radians(20.0)
+    scene.means3D[-needles:] = torch.randn(needles, 3, generator=torch.Generator().manual_seed(1)) * 0.4
+    scene.scales[-needles:] = torch.tensor([0.8, 1e-5 if thin else 8e-3, 1e-5 if thin else 8e-3])
+    scene.rotations[-needles:] = torch.tensor([math.cos(angle), 0.0, 0.0, math.sin(angle)])
+    scene.opacities[:] = 0.02
+    return scene
+
+
+def test_thin_needles_do_not_slow_their_batches(gpu_device):
+    """A needle may have pixels with an exponent above zero, but its batches are still blended four entries side by side:
+    one comparison more per entry.  (Entry by entry the thin ones took 1.34 times as long as the wide ones; with the comparison
+    1.02 times.)"""
+    ms, ws = {}, pipeline.Workspace(gpu_device)
+    for thin in (False, True):
+        scene = _needles(thin)
+        kw = dict(shs=scene.shs.to(gpu_device), scales=scene.scales.to(gpu_device), rotations=scene.rotations.to(gpu_device))
+        inp, out, records = _run(scene, gpu_device, ws, _lib.PIPELINE_FAST, **kw)
+        rho = records[:, 3].abs() / (records[:, 2] * records[:, 4]).sqrt()
+        beyond = int((rho >= 0.99999).sum())
+        assert beyond >= 30 if thin else beyond == 0
+        assert int(torch.isinf(records[:, 10]).sum()) >= 30
+        times = []
+        for _ in range(12):
+            start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            pipeline.run_stages(inp, out, ws, 8_000_000, _lib.STAGE_BLEND)
+            stop.record()
+            stop.synchronize()
+            times.append(start.elapsed_time(stop))
+        ms[thin] = sorted(times)[2]
+        images = [out.image.clone(), out.depth.clone(), out.alpha.clone()]
+        pipeline.run_stages(inp, out, ws, 8_000_000, _lib.STAGE_BLEND_PLAIN)
+        for a, b in zip(images, (out.image, out.depth, out.alpha)):
+            assert torch.equal(a, b)
+    print("blend with needles: %.1f us wide, %.1f us thin" % (1e3 * ms[False], 1e3 * ms[True]))
+    assert ms[True] < 1.15 * ms[False]
