@@ -136,8 +136,9 @@ def stage_breakdown(torch, pipeline, _lib, inp, n_cap, steps):
     fast = [("preprocess", front), ("tile_count", _lib.STAGE_TILE_COUNT),
             ("tile_scatter", _lib.STAGE_TILE_SCATTER), ("tile_sort", _lib.STAGE_TILESORT | _lib.STAGE_TILESORT_VALUES | skip),
             ("blend", _lib.STAGE_BLEND)]
-    classic = [("scan", _lib.STAGE_SCAN), ("duplicate", _lib.STAGE_DUPLICATE), ("sort", _lib.STAGE_SORT),
-               ("ranges", _lib.STAGE_RANGES)]
+    # (behind a preprocess without the modifier, as that path has it: after one with it the scan makes rectangles whole first)
+    classic = [("preprocess_whole", _lib.STAGE_PREPROCESS), ("scan", _lib.STAGE_SCAN),
+               ("duplicate", _lib.STAGE_DUPLICATE), ("sort", _lib.STAGE_SORT), ("ranges", _lib.STAGE_RANGES)]
     ms = time_stages(torch, pipeline, inp, out, ws, n_cap, fast, steps)
     ms.update(time_stages(torch, pipeline, inp, out, ws, n_cap, classic, max(3, steps // 4)))
     lay = _lib.workspace_layout(inp.P, n_cap, inp.width, inp.height)

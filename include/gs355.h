@@ -119,7 +119,9 @@ typedef struct gs355_header {
      * caller needs to choose GS355_STAGE_TILESORT_SKIP_* for the next frame. */
     uint32_t sort_class_count[3];
     uint32_t ready;          /* set to 1 in a header copy, after everything else in it (in the workspace: not used) */
-    uint32_t reserved[7];
+    uint32_t parts;          /* preprocess stage: 1 if `rects` holds parts of tile rectangles (GS355_STAGE_TILE_REACH), else 0
+                              * (in the workspace only) */
+    uint32_t reserved[6];
 } gs355_header;
 
 /* Byte offsets of every array inside the caller's workspace (each 256-byte

@@ -85,7 +85,8 @@ class Header(C.Structure):
         ("num_visible", C.c_uint32),
         ("sort_class_count", C.c_uint32 * 3),
         ("ready", C.c_uint32),
-        ("reserved", C.c_uint32 * 7),
+        ("parts", C.c_uint32),
+        ("reserved", C.c_uint32 * 6),
     ]
 
 

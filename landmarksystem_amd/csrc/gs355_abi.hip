@@ -202,6 +202,7 @@ FrameArgs make_args(const gs355_frame* f)
     a.p_device = nullptr;
     a.plain_regions = a.grid_x > 32767 || a.grid_y > 32767;
     a.tile_reach = 0;
+    a.parts = nullptr;
     return a;
 }
 
@@ -287,16 +288,15 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
     FrameArgs fa = make_args(frame);
     fa.p_device = g->P_device;
     fa.tile_reach = (stage_mask & GS355_STAGE_TILE_REACH) && !fa.plain_regions;
+    fa.parts = &header->parts;
     const uint32_t cap = (uint32_t)n_cap;
 
     if (stage_mask & GS355_STAGE_PREPROCESS)
         if ((rc = launch_preprocess(fa, *g, par, false, records, touched, rects, depth_bits, wave_totals, lit, out->radii, s))) return rc;
-    if (stage_mask & GS355_STAGE_SCAN) {
-        if ((rc = launch_whole_rectangles(fa, g->P, records, out->radii, touched, rects, s))) return rc;
-        if ((rc = launch_scan_offsets(touched, out->radii, g->P, g->P_device, offsets, scan_tmp, header,
+    if (stage_mask & GS355_STAGE_SCAN)
+        if ((rc = launch_scan_offsets(fa, g->P, records, out->radii, touched, rects, offsets, scan_tmp, header,
                                       static_cast<gs355_header*>(out->header_copy), cap, s)))
             return rc;
-    }
     if (stage_mask & GS355_STAGE_DUPLICATE)
         if ((rc = launch_duplicate(fa, g->P, records, out->radii, offsets, header, keys[0], vals[0], s))) return rc;
     if (stage_mask & GS355_STAGE_SORT)

@@ -36,6 +36,7 @@ struct FrameArgs {  // by-value kernel argument
     const uint32_t* p_device;  // optional device-side number of Gaussians (gs355_gaussians.P_device)
     int32_t plain_regions;  // the grid is too large for flags in the tile regions' words (TileRegion)
     int32_t tile_reach;     // preprocess: a Gaussian's region is the tiles its alpha >= 1/255 ellipse reaches
+    uint32_t* parts;        // preprocess: the workspace header's word for that
 };
 
 // Number of Gaussians a kernel processes: the host's P, or the device-side count when there is one.
@@ -90,6 +91,12 @@ __device__ __forceinline__ Rect tile_rect(float px, float py, int radius, int gr
     q.x1 = tile_clamp((px + r + 15.0f) / 16.0f, grid_x);
     q.y1 = tile_clamp((py + r + 15.0f) / 16.0f, grid_y);
     return q;
+}
+
+// the rectangle as a Gaussian's tiles (TileRegion)
+__device__ __forceinline__ uint64_t whole_region(const Rect q)
+{
+    return (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
 }
 
 // Exponent of one (pixel, Gaussian) pair,  hx dx^2 + ny dx dy + hz dy^2  with hx = -conic_x / 2, ny = -conic_y,
@@ -276,11 +283,10 @@ constexpr float kAlphaCut = -7.99435329f;  // bits 0xc0ffd1be
 int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
                       uint32_t* tiles_touched, uint64_t* rects, uint32_t* depth_bits, uint2* wave_totals, uint8_t* lit,
                       int32_t* radii, hipStream_t s);
-int launch_scan_offsets(const uint32_t* tiles_touched, const int32_t* radii, int32_t P, const uint32_t* p_device,
-                        uint32_t* offsets, uint32_t* scan_tmp, gs355_header* header, gs355_header* header_copy, uint32_t n_cap, hipStream_t s);
+int launch_scan_offsets(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii, uint32_t* tiles_touched,
+                        uint64_t* rects, uint32_t* offsets, uint32_t* scan_tmp, gs355_header* header, gs355_header* header_copy,
+                        uint32_t n_cap, hipStream_t s);
 int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const FilterArgs& x, int32_t* radii, hipStream_t s);
-int launch_whole_rectangles(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii, uint32_t* tiles_touched,
-                            uint64_t* rects, hipStream_t s);
 int launch_duplicate(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii,
                      const uint32_t* offsets, const gs355_header* header, uint64_t* keys, uint32_t* values,
                      hipStream_t s);

@@ -213,7 +213,7 @@ __device__ __forceinline__ bool lod_keeps(const gs355_anchor_lod& l, float log2_
 // 785 -> 706, blend backward 1025 -> 870 (6M).
 __device__ __forceinline__ uint64_t tile_region(const Rect q, float px, float py, float qx, float qy, float qz, float ex, float ey)
 {
-    const uint64_t whole = (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
+    const uint64_t whole = whole_region(q);
     if (!(ex < INFINITY)) return whole;
     if (ex < 0.0f) return 0;
     const float x = px - (float)(q.x0 * kTile), y = py - (float)(q.y0 * kTile);
@@ -375,7 +375,10 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     {  // the wavefront's keys and survivors: what the frame's key count is made of
         const uint32_t keys = wave_sum(touched);
         const uint32_t visible = (uint32_t)__popcll(__ballot(alive));
-        if ((threadIdx.x & 63) == 0 && valid) wave_totals[i >> 6] = make_uint2(keys, visible);
+        if ((threadIdx.x & 63) == 0 && valid) {
+            wave_totals[i >> 6] = make_uint2(keys, visible);
+            if (i == 0) *f.parts = (uint32_t)f.tile_reach;
+        }
     }
 
     // Reach of the splat, for the culling of tiles (below) and of the blend's pixel blocks: half-extents
@@ -490,21 +493,6 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     depth_bits[i] = __float_as_uint(vz);
 }
 
-// Before the classic stages, whose keys are those of whole rectangles: every Gaussian's rectangle and its tiles, whatever
-// region the preprocess left (the backward pass finds a key's gradient record through it).
-__global__ __launch_bounds__(256) void whole_rectangles_kernel(FrameArgs f, int32_t P, const float* __restrict__ records,
-                                                               const int32_t* __restrict__ radii,
-                                                               uint32_t* __restrict__ tiles_touched, uint64_t* __restrict__ rects)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= effective_count(f, P)) return;
-    const int rad = radii[i];
-    Rect q = {0, 0, 0, 0};
-    if (rad > 0) q = tile_rect(records[(size_t)i * kRecordFloats], records[(size_t)i * kRecordFloats + 1], rad, f.grid_x, f.grid_y);
-    tiles_touched[i] = (uint32_t)((q.x1 - q.x0) * (q.y1 - q.y0));
-    rects[i] = (uint64_t)q.x0 | ((uint64_t)q.y0 << 16) | ((uint64_t)q.x1 << 32) | ((uint64_t)q.y1 << 48);
-}
-
 // One workgroup expands the keys of 256 consecutive Gaussians.  Output slots
 // are walked by consecutive lanes (coalesced stores); each slot finds its
 // source Gaussian by binary search over the group's offsets held in LDS.
@@ -597,15 +585,6 @@ int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const Fil
     else
         launch(preprocess_kernel<true, false, false>);
     GS355_CHECK_LAUNCH("anchor filter");
-    return GS355_OK;
-}
-
-int launch_whole_rectangles(const FrameArgs& f, int32_t P, const float* records, const int32_t* radii, uint32_t* tiles_touched,
-                            uint64_t* rects, hipStream_t s)
-{
-    if (P == 0) return GS355_OK;
-    hipLaunchKernelGGL(whole_rectangles_kernel, dim3((P + 255) / 256), dim3(256), 0, s, f, P, records, radii, tiles_touched, rects);
-    GS355_CHECK_LAUNCH("whole rectangles");
     return GS355_OK;
 }
 

@@ -145,3 +145,34 @@ def test_classic_stages_after_it(gpu_device):
     b = pipeline.render_backward(got["inp"], got["out"], got["ws"].buffer, cot)
     for name in a:
         assert torch.equal(a[name], b[name]), name
+
+
+def test_the_scan_remakes_rectangles_only_where_they_were_cut(gpu_device):
+    """Whole rectangles are read as the preprocess left them, in the same call or a later one: what has been put in their place
+    is still there afterwards.  Parts of them are made whole, once."""
+    scene = mixed_scene(5000, 200, 120, 6)
+    d = scene.to(gpu_device)
+    inp = pipeline.FrameInputs(settings_for(scene, gpu_device), d.means3D, opacities=d.opacities, shs=d.shs, scales=d.scales,
+                               rotations=d.rotations)
+    out, ws, n_cap = pipeline.FrameOutputs(inp), pipeline.Workspace(gpu_device), 2_000_000
+    lay = ws.ensure(inp.P, n_cap, inp.width, inp.height)
+    ws.buffer.fill_(0xA5)
+    rects = ws.buffer[lay.rects:lay.rects + 8 * inp.P].view(torch.int64)
+
+    def words(*masks):
+        for mask in masks:
+            pipeline.run_stages(inp, out, ws, n_cap, mask)
+        return rects.clone(), ws.view(lay, "offsets", inp.P, 0, inp.tiles).clone()
+
+    whole, offsets = words(_lib.STAGE_PREPROCESS | _lib.STAGE_SCAN)
+    mark = 0x0001000100000000  # (one tile, at the corner)
+    rects.fill_(mark)
+    got = words(_lib.STAGE_SCAN)
+    assert bool((got[0] == mark).all()) and torch.equal(got[1], offsets)
+    parts, _ = words(_lib.STAGE_PREPROCESS | _lib.STAGE_TILE_REACH)
+    assert int((parts != whole).sum()) > 1000
+    got = words(_lib.STAGE_SCAN)
+    assert torch.equal(got[0], whole) and torch.equal(got[1], offsets)
+    rects.fill_(mark)
+    got = words(_lib.STAGE_SCAN)
+    assert bool((got[0] == mark).all()) and torch.equal(got[1], offsets)
