@@ -241,7 +241,7 @@ __device__ __forceinline__ uint64_t tile_region(const Rect q, float px, float py
 // memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
 // front of a kernel of 0.3 ms).
 // kPacked: SH blocks of 16 coefficients at 16-byte boundaries, fetched by way of LDS.  The 53 KB of that leave three wavefronts
-// per SIMD, so calls without such blocks (colours given, or of another size) run a kernel without it, at eight: 1.5M decoded
+// per SIMD, so calls without such blocks (colours given, or blocks of another size) run a kernel without it, at eight: 1.5M decoded
 // Gaussians 100 -> 76 us, 600k 32.5 -> 24.5, 160k 13.8 -> 12.4.
 template <bool kRadiiOnly, bool kStored, bool kPacked>
 __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaussians g, ParameterArgs par, FilterArgs fx,
@@ -264,15 +264,25 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     const bool valid = i < P;
     const float* __restrict__ V = f.viewmatrix;
     const float* __restrict__ M = f.projmatrix;
+    // Read here, ahead of the kernel's stores, so that it goes through the scalar cache: behind them the compiler reads it
+    // with vector loads, one more latency between the SH blocks and the colours (6M Gaussians 304 -> 316 us).
+    float campos[3] = {0.f, 0.f, 0.f};
+    if (kPacked) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) campos[k] = f.campos[k];
+    }
 
     // ---- geometry: cull, covariance, EWA projection, conic, radius, tile rectangle ----
     int radius = 0;
     uint32_t touched = 0;
     Rect rect = {0, 0, 0, 0};
     float x = 0.f, y = 0.f, z = 0.f, vz = 0.f, px = 0.f, py = 0.f, ca = 0.f, cc = 0.f, qx = 0.f, qy = 0.f, qz = 0.f;
-    // Every per-Gaussian geometry input is requested up front, before the cull
-    // decides whether it is needed: one memory latency instead of a chain of
-    // dependent ones (culled Gaussians cost 28 to 32 B of extra reads).
+    // Every per-Gaussian geometry input is requested before the cull decides
+    // whether it is needed, instead of a chain of dependent latencies (culled
+    // Gaussians cost 28 to 32 B of extra reads).  With the branch for given
+    // covariances the mean arrives before the others are requested; compiled
+    // apart, without that wait, the frame of 6M Gaussians stays as it is and the
+    // radii-only kernel goes from 57.8 to 61 us.
     float cov[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, scale[3] = {0.f, 0.f, 0.f}, quat[4] = {0.f, 0.f, 0.f, 0.f};
     float opacity = 0.f;
     bool gated = false;  // anchor outside the level-of-detail mask (anchor prefilter only)
@@ -414,7 +424,8 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
 
     // ---- colour ----
     float rgb[3] = {0.f, 0.f, 0.f};
-    if (!kStored && g.colors_precomp) {
+    const bool given = !kStored && !kPacked && g.colors_precomp != nullptr;
+    if (given) {
         if (alive) {
             rgb[0] = g.colors_precomp[3 * (size_t)i];
             rgb[1] = g.colors_precomp[3 * (size_t)i + 1];
@@ -426,11 +437,8 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         // SH blocks of 64 of them with coalesced loads through LDS, so the memory system sees dense wavefronts
         // however many Gaussians were culled.  Other block sizes: every survivor fetches its own block.  Same
         // values and the same order of additions either way.
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        // (uniform, and true wherever kPacked is; with the branches below left out of that variant the compiler orders its
-        // loads otherwise: 6M Gaussians 308 -> 325 us)
-        const bool packed = kPacked && f.sh_coeffs == 16 && (reinterpret_cast<uintptr_t>(kStored ? par.rest : g.shs) & 15u) == 0;
-        if (packed) {
+        if constexpr (kPacked) {
+            const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
             const uint64_t m = __ballot(alive);
             if (lane == 0) s_alive[wave] = __popcll(m);
             __syncthreads();
@@ -454,11 +462,15 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
             // its own Gaussians' tiles while their blocks are on the way
             const int share = (total + 3) / 4, first_entry = wave * share, count = min(share, total - first_entry);
             float4* __restrict__ rows = s_sh + first_entry * (kShStride / 4);
+            // The opacity has to be there before the blocks are requested: the number of loads behind it then depends on the
+            // number of survivors, so that waiting for it would be waiting for all of them, ahead of the work that is to hide
+            // them (6M Gaussians 304 -> 326 us).
+            if (!kStored) asm volatile("" : "+v"(opacity));
             ShEntries<kStored> entries;
             if (count > 0)
                 entries.fetch(g.shs, par.rest, (size_t)g.P * 45, (size_t)blockIdx.x * blockDim.x, s_owner, first_entry, count, lane);
             reach_and_region();
-            if (count > 0) entries.colour(rows, par.rest, count, lane, f.sh_degree, f.campos);
+            if (count > 0) entries.colour(rows, par.rest, count, lane, f.sh_degree, campos);
             __syncthreads();
             if (alive) {
 #pragma unroll
@@ -483,7 +495,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     // Which channels are above zero is all that the backward pass wants of a colour (zero: clamped, no gradient): a byte
     // instead of 12 of the record's 48, whose cache lines it would read from end to end (preprocess backward of 6M
     // Gaussians 780 -> 723 us, for 2 us here, which the tile counts left out above give back).
-    if (valid && (kStored || !g.colors_precomp)) lit[i] = (uint8_t)((rgb[0] > 0.0f) | ((rgb[1] > 0.0f) << 1) | ((rgb[2] > 0.0f) << 2));
+    if (valid && !given) lit[i] = (uint8_t)((rgb[0] > 0.0f) | ((rgb[1] > 0.0f) << 1) | ((rgb[2] > 0.0f) << 2));
     if (!alive) return;
 
     float4* __restrict__ rec = reinterpret_cast<float4*>(records + (size_t)i * kRecordFloats);
