@@ -329,9 +329,10 @@ def cpu_pair_stats(scene, cam=None, colors_precomp=None, sh_degree=None, keep_fr
 def parity_leg(torch, pipeline, inp, ref):
     """The `parity` object: one frame through the product path (pipeline.render over a workspace of its own) against
     the frame the C checker rendered from the same inputs: radii and key count bit for bit; image, depth and alpha as
-    measured errors.  The product path makes keys only for the tiles that a splat reaches, so every sorted key and value
-    and the tile ranges are compared, bit for bit, on the same stages run over whole rectangles, whose image has to be the
-    product path's."""
+    measured errors.  The product path makes keys only for the tiles that a splat reaches and leaves them sorted by tile,
+    depth and index as values and tile ranges: they have to be the checker's sorted keys and values without the pairs left
+    out.  Every sorted key and value and the tile ranges are then compared, bit for bit, on the same stages run over whole
+    rectangles, whose image has to be the product path's."""
     import numpy as np
 
     from landmarksystem_amd import _lib
@@ -346,6 +347,12 @@ def parity_leg(torch, pipeline, inp, ref):
              "num_keys": bool(n == ref["num_keys"])}
     got = dict(image=out.image.cpu().numpy(), depth=out.depth.cpu().numpy(), alpha=out.alpha.cpu().numpy())
     if n == ref["num_keys"]:
+        ranges = take("ranges", np.uint32).astype(np.int64)
+        tile = np.repeat(np.arange(inp.tiles, dtype=np.int64), ranges[:, 1] - ranges[:, 0])
+        pairs = (tile << 32) | take("sorted_values", np.uint32)[:len(tile)].astype(np.int64)
+        whole = ((ref["sorted_keys"] >> np.uint64(32)).astype(np.int64) << 32) | ref["sorted_values"].astype(np.int64)
+        exact["reached_pairs_in_order"] = bool(len(pairs) == ws.last_num_pairs and
+                                               np.array_equal(whole[np.isin(whole, pairs)], pairs))
         pipeline.run_stages(inp, out, ws, out.key_capacity, _lib.PIPELINE_FAST)
         torch.cuda.synchronize()
         exact["image_of_whole_rectangles"] = bool(np.array_equal(out.image.cpu().numpy(), got["image"]))
