@@ -397,14 +397,16 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     // by more than the rounding error of the blend's fp32 evaluation of the
     // exponent (bounded below by `noise`), so a pixel block outside the box is
     // certain to take the blend's `alpha < 1/255` branch on all of its pixels.
-    // +inf = never cull (large or ill-conditioned splats), -inf = never visible.
+    // +inf = never cull (large or ill-conditioned splats; conics that are not
+    // positive definite, to which a caller's covariances can lead: those have
+    // no such box), -inf = never visible.
     float ex = 0.f, ey = 0.f;
     auto reach_and_region = [&]() {
         uint64_t region = 0;
         if (alive) {
             const float reach = (float)radius + 24.0f;  // |d| over every pixel of every touched tile
             const float noise = 2.4e-7f * (fabsf(qx) + fabsf(qy) + fabsf(qz)) * reach * reach;
-            if (opacity != opacity || !(noise < 0.02f)) {
+            if (opacity != opacity || !(noise < 0.02f) || !(qx > 0.0f && qz > 0.0f)) {
                 ex = ey = INFINITY;
             } else if (!(opacity * 255.0f * 1.0001f >= 1.0f)) {
                 ex = ey = -INFINITY;

@@ -7,7 +7,7 @@ import torch
 
 from landmarksystem_amd import _lib, pipeline, scenes
 from oracle import c_oracle as co
-from tests.helpers import oracle_frame, oracle_gaussians, settings_for
+from tests.helpers import check_images, oracle_frame, oracle_gaussians, settings_for
 
 pytestmark = pytest.mark.gpu
 
@@ -87,6 +87,38 @@ def test_covariances_that_are_negative_on_the_screen_are_rejected(gpu_device, ot
         assert torch.equal(a, b)
     ref = co.render(oracle_frame(scene), oracle_gaussians(scene, cov3D_precomp=cov.numpy()))
     assert float((images[2].cpu() - torch.from_numpy(ref["alpha"])).abs().max()) < 1e-4
+
+
+@pytest.mark.parametrize("others", [0, 300])
+def test_indefinite_covariances_are_blended_wherever_they_reach(gpu_device, others):
+    """A conic of mixed signs has no ellipse outside of which nothing is blended: its alpha stays up along two lines.  No tile
+    and no block may be left out for it."""
+    g = torch.Generator().manual_seed(9)
+    scene = scenes.tiny_scene(P=400, width=133, height=75, sh_degree=0, seed=12)
+    matrix = scene.camera.world_view_transform
+    depth = scene.means3D @ matrix[:3, 2] + matrix[3, 2]
+    focal = scene.camera.width / (2.0 * math.tan(scene.camera.FovX * 0.5))
+    axes = torch.linalg.qr(torch.randn(400, 3, 3, generator=g))[0]
+    sizes = (2.0 + 6.0 * torch.rand(400, 3, generator=g)) ** 2 * torch.tensor([1.0, 1.0, -1.0]) * (depth / focal)[:, None] ** 2
+    full = (axes * sizes[:, None, :]) @ axes.transpose(1, 2).contiguous()
+    cov = torch.stack([full[:, i, j] for i, j in ((0, 0), (0, 1), (0, 2), (1, 1), (1, 2), (2, 2))], dim=1).contiguous()
+    cov[:others] = torch.tensor([0.02, 0.0, 0.0, 0.02, 0.0, 0.02])
+    scene.opacities[:] = 0.3
+    ws = pipeline.Workspace(gpu_device)
+    kw = dict(shs=scene.shs.to(gpu_device), cov3D_precomp=cov.to(gpu_device))
+    images = []
+    for reach in (_lib.STAGE_TILE_REACH, 0):
+        inp, out, records = _run(scene, gpu_device, ws, _lib.PIPELINE_FAST | reach, **kw)
+        images.append([out.image.clone(), out.depth.clone(), out.alpha.clone()])
+    qx, qy, qz = records[:, 2], records[:, 3], records[:, 4]
+    assert int((qx * qz < qy * qy).sum()) >= 30
+    pipeline.run_stages(inp, out, ws, 8_000_000, _lib.STAGE_BLEND_PLAIN)
+    ref = co.render(oracle_frame(scene), oracle_gaussians(scene, cov3D_precomp=cov.numpy()))
+    for planes in images:
+        for a, b in zip(planes, (out.image, out.depth, out.alpha)):
+            assert torch.equal(a, b)
+    check_images(dict(image=out.image.cpu().numpy(), depth=out.depth.cpu().numpy(), alpha=out.alpha.cpu().numpy()), ref,
+                 "indefinite covariances")
 
 
 def _needles(thin, others=100_000, needles=40):
