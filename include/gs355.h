@@ -195,9 +195,10 @@ enum {
     GS355_STAGE_TILESORT_SKIP_3 = 16384,
     /* Modifier of PREPROCESS, for the tile-bucketed stages: a Gaussian gets keys only for those tiles of its rectangle
      * that its alpha >= 1/255 ellipse reaches.  The blend and the backward pass would take the `alpha < 1/255` branch for
-     * every pixel of the other tiles, so images and gradients are the same bits; sorted keys, values and ranges are those
-     * of the remaining keys.  num_keys_total, and with it the overflow of a capacity, still count whole rectangles.
-     * Refused together with a classic stage (in later calls the scan goes back to whole rectangles).  No effect beyond 32767 tiles along an axis. */
+     * every pixel of the other tiles, so images are the same bits and gradients sums of the same numbers (those of large
+     * splats in another order); sorted keys, values and ranges are those of the remaining keys.  num_keys_total, and with
+     * it the overflow of a capacity, still count whole rectangles.  Refused together with a classic stage (in later calls
+     * the scan goes back to whole rectangles).  No effect beyond 32767 tiles along an axis. */
     GS355_STAGE_TILE_REACH = 65536,
     /* Modifier of TILESORT: the sorted values only.  No later stage reads the sorted keys, eight of the twelve bytes that the
      * sort writes per key; their buffer is left as it is (its contents are then undefined). */

@@ -160,8 +160,9 @@ __device__ __forceinline__ float add_halves(float a, float b)
 //     row ends with the totals of its own two or three.
 // Reducing each step by itself with lane exchanges took 53 vector instructions per step, more than the gradient
 // arithmetic; this takes about 20.  Blend backward at 6M Gaussians / 1080p: 1.34 -> 1.25 ms, 622M -> 491M vector
-// instructions, LDS pipe 73 -> 37 % busy (493M and 38 % with the check for sums that are not finite, 0.4 % of a step).  Larger matrix instructions do not pay for the sums (1.45 ms): fp32 ones
-// occupy the SIMD like the vector instructions they replace.
+// instructions, LDS pipe 73 -> 37 % busy (493M and 38 % with the check for sums that are not finite, 0.4 % of a
+// step).  Larger matrix instructions do not pay for the sums (1.45 ms): fp32 ones occupy the SIMD like the vector
+// instructions they replace.
 // kDepth: a gradient arrives for the depth plane.
 template <bool kDepth>
 __global__ __launch_bounds__(256) void blend_backward_kernel(

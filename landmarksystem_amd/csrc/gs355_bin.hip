@@ -51,7 +51,8 @@ __device__ __forceinline__ int lanes_per_gaussian(int per_group)
 
 // A share of a region's tiles for each of `lanes` lanes (a power of two), this one the `sub`-th; `record`: the Gaussian's.
 // Of a region with spans a lane takes whole rows, or several lanes one where there are more lanes than rows: a row's span
-// costs some 30 instructions, too many to evaluate for every tile (100k large splats: count 24.3, scatter 27.0 us by tile, 12.2 and 18.0 by row).
+// costs some 30 instructions, too many to evaluate for every tile (100k large splats: count 24.3, scatter 27.0 us by tile,
+// 12.2 and 18.0 by row).
 template <typename Visit>
 __device__ __forceinline__ void walk_region(const TileRegion& q, const float* __restrict__ record, int sub, int lanes, int grid_x,
                                             Visit visit)
@@ -652,15 +653,16 @@ __global__ __launch_bounds__(64 * kPrefixParts) void slice_prefix_kernel(uint32_
 // Layout of the buckets from the tiles' totals: one wavefront per block of 64 tiles, four per workgroup.  Every
 // workgroup adds up the block totals itself (a few hundred words, at most 9000): those before its own blocks give its
 // first slot, all of them the number of pairs; the slices' totals are the frame's key count, which decides overflow before
-// anything is published — so no workgroup waits for another and no separate scan pass is launched.  Workgroup 0 also writes the frame header and
-// the work list of the scatter's second level: chunk_base[b] = chunks of kFineChunk pairs in the coarse bins before
-// b, chunk_base[bins] = all (`bin_pairs`, the pairs per bin, may be the same array).  With kTiles the wavefronts
-// publish tile bases, the scatter's cursors, the ranges and the lists of buckets too large for the small sorter;
-// without, the columns are coarse bins and only their bases are written.  Where the buckets per size class were counted
+// anything is published — so no workgroup waits for another and no separate scan pass is launched.  Workgroup 0 also
+// writes the frame header and the work list of the scatter's second level: chunk_base[b] = chunks of kFineChunk pairs in
+// the coarse bins before b, chunk_base[bins] = all (`bin_pairs`, the pairs per bin, may be the same array).  With
+// kTiles the wavefronts publish tile bases, the scatter's cursors, the ranges and the lists of buckets too large for the
+// small sorter; without, the columns are coarse bins and only their bases are written.  Where the buckets per size class were counted
 // by block (`block_classes`, a byte per class), a block's places in the lists follow from the blocks before it, as its
 // slots do; else they are requested from the lists' counters (`lists[0..3]` cleared by an earlier kernel), which costs
-// three dependent round trips to memory (9.1 us at 1080p against 5.1).  `totals` and `tile_base` may be the same array.  `header_known`: second layout of a frame (by tile,
-// after the one by coarse bin): the header stands, and nothing is done on overflow.
+// three dependent round trips to memory (9.1 us at 1080p against 5.1).  `totals` and `tile_base` may be the same array.
+// `header_known`: second layout of a frame (by tile, after the one by coarse bin): the header stands, and nothing is done
+// on overflow.
 template <bool kTiles>
 __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* totals, uint32_t tiles,
                                                            const uint64_t* __restrict__ block_sums, uint32_t n_blocks,

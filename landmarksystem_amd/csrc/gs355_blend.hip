@@ -171,7 +171,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
     __shared__ float4 s_a[kBatch + 1];  // px, py, -conic_x / 2, -conic_y          (+ the null record)
     __shared__ float4 s_b[kBatch + 1];  // -conic_z / 2, log2(opacity), mask of the blocks it can reach, unused
     __shared__ float4 s_c[kBatch + 1];  // r, g, b, depth
-    __shared__ uint32_t s_wave_state[4];  // bit 0: all pixels of the wavefront finished; it staged 1: a channel that is not finite, 2: a record that is not definite
+    // bit 0: all pixels of the wavefront finished; it staged 1: a channel that is not finite, 2: a record that is not definite
+    __shared__ uint32_t s_wave_state[4];
     // per wavefront and 4x4 block: byte offsets of the staged records of the Gaussians that can reach the block
     __shared__ __align__(8) ListEntry s_list[kCull ? 4 : 1][4][kListWords];
 

@@ -227,7 +227,8 @@ __device__ __forceinline__ void swap_lane_rows(float& a, float& b)
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_heads_kernel(
-    TrainArgs d, const uint32_t* __restrict__ visible_rows, uint32_t* __restrict__ visible_out, float* __restrict__ hidden0, float* __restrict__ hidden1, float* __restrict__ hidden2,
+    TrainArgs d, const uint32_t* __restrict__ visible_rows, uint32_t* __restrict__ visible_out, float* __restrict__ hidden0,
+    float* __restrict__ hidden1, float* __restrict__ hidden2,
     float* __restrict__ pre0, float* __restrict__ pre1, float* __restrict__ pre2, uint2* __restrict__ totals)
 {
     __shared__ float s_b0[3][32];
@@ -539,15 +540,16 @@ __device__ __forceinline__ void copy_rest(const float* __restrict__ src, float* 
 // A wavefront keeps all 11 blocks of 32 x 32 weight gradients in registers, so there is one wavefront per SIMD and a
 // workgroup per compute unit, each with its own quarter of the LDS for the tile's rows.  Nothing else hides the wait for a
 // tile's rows: the next tile's are requested, into registers, as soon as this one's have gone to LDS, and arrive while it is
-// worked on (copies straight to LDS make every later read of LDS wait for them).  86 us at 200k anchors: 37 us of matrix instructions, some 11 us for a tile's 7.4 us of them, since the operands of the next are read from
-// LDS while one runs, and not earlier; 8 us for the weights, 4 for adding up the gradients, and a last round of tiles in a
-// third of the wavefronts.  Rows requested when they are needed, weights one after the other, the last tile's rows too, and
-// gradients added by one wavefront after the other: 145.
+// worked on (copies straight to LDS make every later read of LDS wait for them).  200k anchors, 176k of them visible, ten
+// offsets: 86 to 88 us.  37 us of that are matrix instructions.  A tile takes some 11 us, of which its matrix instructions
+// are 7.4: the operands of the next one are read from LDS while one runs, and not earlier.  8 us go to the weights and 4 to
+// adding up the gradients, and the last round of tiles fills a third of the wavefronts.  Rows requested when they are needed,
+// weights one after the other, the last tile's rows too, and gradients added by one wavefront after the other: 145.
 // kAnchor: the anchors' own gradient is wanted (the layers are then also walked back to view direction and distance).
 // kOffsets: offsets per anchor, or 0 (d.n).  Ten, the decoder's default, has its loops unrolled and requests rows ahead; with
 // the count a variable there are no registers for that (400 bytes per lane were spilled), and the rows are requested together
-// when they are needed.  At 200k anchors 89 us (105 with kAnchor) with ten offsets; with the variable count 123 (141) at
-// eight and 98 (114) at four.
+// when they are needed.  The same anchors: 88 us (105 with kAnchor) with ten offsets; with the variable count 123 (141) at
+// eight and 98 (116) at four.
 template <bool kAnchor, int kOffsets>
 __global__ __launch_bounds__(64 * kBackwardWaves) void train_layers_kernel(
     TrainArgs d, const uint32_t* __restrict__ rows, const float* __restrict__ d_op, const float* __restrict__ d_cov,
