@@ -59,7 +59,20 @@ def _run(scene, device, ws, mask, **kw):
     ws.ensure(inp.P, n_cap, inp.width, inp.height)
     lay = pipeline.run_stages(inp, out, ws, n_cap, mask)
     records = ws.view(lay, "records", inp.P, 0, inp.tiles)[out.radii > 0]
+    out.key_capacity = n_cap
     return inp, out, records.double()
+
+
+def _check_gradients(scene, ws, inp, out, ref, cov):
+    """The backward pass takes the decisions that the frame took: gradients of a weighted image sum against the oracle's, without
+    the pixels that hold a decision within rounding of its threshold.  (fp32 sums: 1e-4 of the largest, as the smoke test.)"""
+    weights = torch.randn(3, inp.height, inp.width, generator=torch.Generator().manual_seed(6))
+    weights[:, torch.from_numpy(ref["fragile"].reshape(inp.height, inp.width) > 0)] = 0.0
+    got = pipeline.render_backward(inp, out, ws.buffer, weights.to(inp.device), want=("opacities", "shs"))
+    want = co.render_backward(oracle_frame(scene), oracle_gaussians(scene, cov3D_precomp=cov.numpy()), ref, weights.numpy())
+    for name, grad in got.items():
+        expected = torch.from_numpy(want[name]).reshape(grad.shape)
+        assert float((grad.cpu().double() - expected).abs().max()) <= 1e-4 * float(expected.abs().max()), name
 
 
 @pytest.mark.parametrize("others", [0, 300])
@@ -87,6 +100,8 @@ def test_covariances_that_are_negative_on_the_screen_are_rejected(gpu_device, ot
         assert torch.equal(a, b)
     ref = co.render(oracle_frame(scene), oracle_gaussians(scene, cov3D_precomp=cov.numpy()))
     assert float((images[2].cpu() - torch.from_numpy(ref["alpha"])).abs().max()) < 1e-4
+    if others:
+        _check_gradients(scene, ws, inp, out, ref, cov)
 
 
 @pytest.mark.parametrize("others", [0, 300])
@@ -119,6 +134,7 @@ def test_indefinite_covariances_are_blended_wherever_they_reach(gpu_device, othe
             assert torch.equal(a, b)
     check_images(dict(image=out.image.cpu().numpy(), depth=out.depth.cpu().numpy(), alpha=out.alpha.cpu().numpy()), ref,
                  "indefinite covariances")
+    _check_gradients(scene, ws, inp, out, ref, cov)
 
 
 def _needles(thin, others=100_000, needles=40):
@@ -137,7 +153,7 @@ def _needles(thin, others=100_000, needles=40):
 def test_thin_needles_do_not_slow_their_batches(gpu_device):
     """A needle may have pixels with an exponent above zero, but its batches are still blended four entries side by side:
     one comparison more per entry.  (Entry by entry the thin ones took 1.34 times as long as the wide ones; with the comparison
-    1.02 times.)"""
+    1.02 to 1.05 times.)"""
     ms, ws = {}, pipeline.Workspace(gpu_device)
     for thin in (False, True):
         scene = _needles(thin)
@@ -161,4 +177,4 @@ def test_thin_needles_do_not_slow_their_batches(gpu_device):
         for a, b in zip(images, (out.image, out.depth, out.alpha)):
             assert torch.equal(a, b)
     print("blend with needles: %.1f us wide, %.1f us thin" % (1e3 * ms[False], 1e3 * ms[True]))
-    assert ms[True] < 1.15 * ms[False]
+    assert ms[True] < 1.2 * ms[False]
