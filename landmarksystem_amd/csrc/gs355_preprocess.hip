@@ -107,31 +107,36 @@ __device__ __forceinline__ void sh_finish(float res[3])
     }
 }
 
-// SH blocks (16 coefficients, 192 B) are staged through LDS; the stride keeps the 16-B reads of the 64 lanes on
-// distinct banks (stride = 4 mod 8 floats).
-constexpr int kShStride = 52;  // floats per Gaussian in the staging area
-
-// One wavefront fetches the SH blocks of up to 64 Gaussians with coalesced 16-B loads (twelve lanes per block)
-// and each lane then evaluates the colour of its own entry from LDS.  `owner[e]` is the position of entry e's
+// One wavefront fetches the SH blocks of up to 64 Gaussians with coalesced 16-B loads (twelve lanes per block of sixteen
+// coefficients) and each lane then evaluates the colour of its own entry from LDS.  `owner[e]` is the position of entry e's
 // Gaussian within the workgroup's 256 (entries are the workgroup's surviving Gaussians, packed in order), so the
 // loads touch survivors' blocks only, however few of the 256 survived.  A row of the staging area holds an
-// entry's 48 coefficients and, in its 4 floats of padding, the Gaussian's position on the way in and its colour
-// on the way out.
+// entry's coefficients and, behind them, the Gaussian's position on the way in and its colour on the way out.
 //
-// kSplit: the split storage of the stored parameters.  The first coefficient (12 B per Gaussian) is
-// read by the entry's own lane, the other fifteen (45 floats per Gaussian, dword-aligned) with 16-B loads all the
-// same: a Gaussian's row starts (row & 3) floats behind a 16-B boundary and always spans twelve aligned 16-B chunks.
-// The chunks land in the staging row as they are, so the coefficients of entry e start at float (row & 3) of its
-// row; with the rows' stride of 52 floats consecutive Gaussians then sit an odd number of banks apart.  `n_floats`:
-// 45 P.  The last chunk of the last row may reach past the array: it is pulled back inside, and that row's last
-// floats are fetched by its own lane.
+// kCoeffs: coefficients per Gaussian, 4, 9 or 16 (degrees 1 to 3).  kSplit: the split storage of the stored parameters,
+// whose first coefficient (12 B per Gaussian) is read by the entry's own lane, and the others as a row of their own.
+// Rows of a multiple of four floats are 16-B chunks as they are.  The others (27 floats of nine coefficients; 45 and 9
+// behind a first one) are dword-aligned and read with 16-B loads all the same: a Gaussian's row starts up to three floats
+// behind a 16-B boundary, (row * kRow) & 3, and spans kChunks aligned chunks.  They land in the staging row as they are,
+// so that the coefficients of entry e start at that float of its row.  `n_floats`: kRow P.  The last chunk of the last row
+// may reach past the array: it is pulled back inside, and that row's last floats are fetched by its own lane.
+//
+// What it is for: a lane that reads its own block asks for a cache line per dword, and 64 lanes' blocks of 108 B are more
+// lines than the L1 keeps until their next dword.  3M Gaussians at 1080p: nine coefficients 216 -> 113 us, four 94 -> 81
+// (sixteen: 152); stored parameters 207 -> 121 and 97 -> 87.
 //
 // fetch() and colour() are apart so that the caller has work to do while the blocks travel.
-constexpr int kShLoads = 12;  // 16-B loads per lane for 64 blocks
-template <bool kSplit>
+template <bool kSplit, int kCoeffs>
 struct ShEntries {
+    static constexpr int kRow = 3 * (kSplit ? kCoeffs - 1 : kCoeffs);  // floats per Gaussian
+    static constexpr bool kWhole = kRow % 4 == 0;
+    static constexpr int kChunks = kWhole ? kRow / 4 : (kRow + 6) / 4;  // 16-B loads per row, and per lane for 64 rows
+    static constexpr int kBeside = 4 * kChunks;  // floats before the position / colour
+    // floats per row of the staging area: 4 modulo 8 keeps the 16-B reads of the 64 lanes on distinct banks
+    static constexpr int kStride = 4 * (kChunks + 1 + kChunks % 2);
+
     typedef float f4v __attribute__((ext_vector_type(4)));
-    f4v v[kShLoads];
+    f4v v[kChunks];
     float first_coeff[3];
     size_t row, last_chunk;
 
@@ -140,18 +145,19 @@ struct ShEntries {
                                           size_t group_first, const uint8_t* __restrict__ owner, int first_entry, int count,
                                           int lane)
     {
-        last_chunk = n_floats / 4 - 1;  // (kSplit: a row alone is eleven chunks)
+        last_chunk = n_floats / 4 - 1;  // (one row alone is two chunks or more)
+        const f4v* __restrict__ chunks = reinterpret_cast<const f4v*>(kSplit ? rest : shs);
 #pragma unroll
-        for (int it = 0; it < kShLoads; ++it) {
-            if (it * 64 >= 12 * count) break;  // uniform: fewer survivors, fewer loads
+        for (int it = 0; it < kChunks; ++it) {
+            if (it * 64 >= kChunks * count) break;  // uniform: fewer survivors, fewer loads
             const int q4 = it * 64 + lane;
-            const int e = min(q4 / 12, count - 1), m = q4 % 12;
+            const int e = min(q4 / kChunks, count - 1), m = q4 % kChunks;
             const size_t i = group_first + owner[first_entry + e];
             // (read once per frame: a streaming load, which leaves the cache to the records the blend gathers)
-            if (kSplit)
-                v[it] = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(rest) + min(i * 45 / 4 + m, last_chunk));
+            if (kWhole)
+                v[it] = __builtin_nontemporal_load(chunks + i * (kRow / 4) + m);
             else
-                v[it] = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(shs + i * 48) + m);
+                v[it] = __builtin_nontemporal_load(chunks + min(i * kRow / 4 + m, last_chunk));
         }
         row = group_first + owner[first_entry + min(lane, count - 1)];
         if (kSplit)
@@ -159,33 +165,33 @@ struct ShEntries {
             for (int c = 0; c < 3; ++c) first_coeff[c] = __builtin_nontemporal_load(&shs[3 * row + c]);
     }
 
-    __device__ __forceinline__ void colour(float4* __restrict__ mine, const float* __restrict__ rest, int count, int lane, int degree,
-                                           const float* campos)
+    __device__ __forceinline__ void colour(float4* __restrict__ mine, const float* __restrict__ shs, const float* __restrict__ rest,
+                                           int count, int lane, int degree, const float* campos)
     {
 #pragma unroll
-        for (int it = 0; it < kShLoads; ++it) {
-            if (it * 64 >= 12 * count) break;
+        for (int it = 0; it < kChunks; ++it) {
+            if (it * 64 >= kChunks * count) break;
             const int q4 = it * 64 + lane;
-            mine[min(q4 / 12, count - 1) * (kShStride / 4) + q4 % 12] = make_float4(v[it].x, v[it].y, v[it].z, v[it].w);
+            mine[min(q4 / kChunks, count - 1) * (kStride / 4) + q4 % kChunks] = make_float4(v[it].x, v[it].y, v[it].z, v[it].w);
         }
         wave_lds_sync();
         if (lane >= count) return;
-        float* __restrict__ slot = reinterpret_cast<float*>(mine) + lane * kShStride;
-        float* __restrict__ coeffs = slot + (kSplit ? (int)(row & 3) : 0);
-        if (kSplit && (row + 1) * 45 > 4 * (last_chunk + 1))  // the array's last row, where its length is no multiple of four
-            for (int k = (int)(4 * (last_chunk + 1) - row * 45); k < 45; ++k) coeffs[k] = rest[row * 45 + k];
+        float* __restrict__ slot = reinterpret_cast<float*>(mine) + lane * kStride;
+        float* __restrict__ coeffs = slot + (kWhole ? 0 : (int)((uint32_t)row * (uint32_t)kRow & 3u));
+        if (!kWhole && (row + 1) * kRow > 4 * (last_chunk + 1))  // the array's last row, where its length is no multiple of four
+            for (int k = (int)(4 * (last_chunk + 1) - row * kRow); k < kRow; ++k) coeffs[k] = (kSplit ? rest : shs)[row * kRow + k];
         float b[16], rgb[3] = {0.f, 0.f, 0.f};
-        sh_basis(degree, slot[48] - campos[0], slot[49] - campos[1], slot[50] - campos[2], b);
+        sh_basis(degree, slot[kBeside] - campos[0], slot[kBeside + 1] - campos[1], slot[kBeside + 2] - campos[2], b);
         const int terms = (degree + 1) * (degree + 1);
         if (kSplit) {
             sh_accumulate<0, 1>(terms, first_coeff, b, rgb);
-            sh_accumulate<1, 15>(terms, coeffs, b, rgb);
+            sh_accumulate<1, kCoeffs - 1>(terms, coeffs, b, rgb);
         } else {
-            sh_accumulate<0, 16>(terms, coeffs, b, rgb);
+            sh_accumulate<0, kCoeffs>(terms, coeffs, b, rgb);
         }
         sh_finish(rgb);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) slot[48 + c] = rgb[c];
+        for (int c = 0; c < 3; ++c) slot[kBeside + c] = rgb[c];
     }
 };
 
@@ -240,10 +246,10 @@ __device__ __forceinline__ uint64_t tile_region(const Rect q, float px, float py
 // kStored: g holds the vanilla model's stored parameters, activated here (the activated copies would cost a pass over
 // memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
 // front of a kernel of 0.3 ms).
-// kPacked: SH blocks of 16 coefficients at 16-byte boundaries, fetched by way of LDS.  The 53 KB of that leave three wavefronts
-// per SIMD, so calls without such blocks (colours given, or blocks of another size) run a kernel without it, at eight: 1.5M decoded
-// Gaussians 100 -> 76 us, 600k 32.5 -> 24.5, 160k 13.8 -> 12.4.
-template <bool kRadiiOnly, bool kStored, bool kPacked>
+// kPacked: coefficients of SH blocks that are fetched by way of LDS (ShEntries), 0: none.  The 20 to 53 KB of that leave seven to
+// three wavefronts per SIMD, so calls without such blocks (colours given, or blocks of another size) run a kernel without it, at
+// eight: 1.5M decoded Gaussians 100 -> 76 us, 600k 32.5 -> 24.5, 160k 13.8 -> 12.4.
+template <bool kRadiiOnly, bool kStored, int kPacked>
 __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaussians g, ParameterArgs par, FilterArgs fx,
                                                          float* __restrict__ records,
                                                          uint32_t* __restrict__ tiles_touched,
@@ -252,8 +258,9 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
                                                          uint2* __restrict__ wave_totals, uint8_t* __restrict__ lit,
                                                          int32_t* __restrict__ radii)
 {
-    // staging area for the 16-coefficient SH blocks of each wavefront's 64 Gaussians
-    __shared__ float4 s_sh[kPacked ? 4 * 64 * kShStride / 4 : 1];
+    typedef ShEntries<kStored, kPacked ? kPacked : 16> Entries;
+    // staging area for the SH blocks of each wavefront's 64 Gaussians
+    __shared__ float4 s_sh[kPacked ? 4 * 64 * Entries::kStride / 4 : 1];
     // the workgroup's surviving Gaussians, packed in order: position within the workgroup; survivors per wavefront
     __shared__ uint8_t s_owner[kPacked ? 256 : 1];
     __shared__ int s_alive[4];
@@ -435,7 +442,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         }
         reach_and_region();
     } else {
-        // Full 192-B blocks: the survivors of the workgroup are packed (in order) and each wavefront fetches the
+        // Blocks of 4, 9 or 16 coefficients: the survivors of the workgroup are packed (in order) and each wavefront fetches the
         // SH blocks of 64 of them with coalesced loads through LDS, so the memory system sees dense wavefronts
         // however many Gaussians were culled.  Other block sizes: every survivor fetches its own block.  Same
         // values and the same order of additions either way.
@@ -452,31 +459,31 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
             }
             // packed entry e lives in row e of the staging area
             float* __restrict__ my_row = reinterpret_cast<float*>(s_sh) +
-                                         (before + __popcll(m & ((1ull << lane) - 1ull))) * kShStride;
+                                         (before + __popcll(m & ((1ull << lane) - 1ull))) * Entries::kStride;
             if (alive) {
                 s_owner[before + __popcll(m & ((1ull << lane) - 1ull))] = (uint8_t)threadIdx.x;
-                my_row[48] = x;
-                my_row[49] = y;
-                my_row[50] = z;
+                my_row[Entries::kBeside] = x;
+                my_row[Entries::kBeside + 1] = y;
+                my_row[Entries::kBeside + 2] = z;
             }
             __syncthreads();
             // each wavefront takes a quarter of the packed survivors (entry e sits in row e of the staging area), and finds
             // its own Gaussians' tiles while their blocks are on the way
             const int share = (total + 3) / 4, first_entry = wave * share, count = min(share, total - first_entry);
-            float4* __restrict__ rows = s_sh + first_entry * (kShStride / 4);
+            float4* __restrict__ rows = s_sh + first_entry * (Entries::kStride / 4);
             // The opacity has to be there before the blocks are requested: the number of loads behind it then depends on the
             // number of survivors, so that waiting for it would be waiting for all of them, ahead of the work that is to hide
             // them (6M Gaussians 304 -> 326 us).
             if (!kStored) asm volatile("" : "+v"(opacity));
-            ShEntries<kStored> entries;
+            Entries entries;
             if (count > 0)
-                entries.fetch(g.shs, par.rest, (size_t)g.P * 45, (size_t)blockIdx.x * blockDim.x, s_owner, first_entry, count, lane);
+                entries.fetch(g.shs, par.rest, (size_t)g.P * Entries::kRow, (size_t)blockIdx.x * blockDim.x, s_owner, first_entry, count, lane);
             reach_and_region();
-            if (count > 0) entries.colour(rows, par.rest, count, lane, f.sh_degree, campos);
+            if (count > 0) entries.colour(rows, g.shs, par.rest, count, lane, f.sh_degree, campos);
             __syncthreads();
             if (alive) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) rgb[c] = my_row[48 + c];
+                for (int c = 0; c < 3; ++c) rgb[c] = my_row[Entries::kBeside + c];
             }
         } else {
             reach_and_region();
@@ -572,17 +579,18 @@ int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const Parame
     if (g.P == 0) return GS355_OK;
     const dim3 block(256), grid((g.P + 255) / 256);
     const FilterArgs none;
-    const bool packed = f.sh_coeffs == 16 && (par || !g.colors_precomp) &&
-                        (reinterpret_cast<uintptr_t>(par ? par->rest : g.shs) & 15u) == 0;
+    // (any other number of coefficients, and blocks off the 16-byte boundaries of ordinary allocations: a lane per block)
+    const bool aligned = (par || !g.colors_precomp) && (reinterpret_cast<uintptr_t>(par ? par->rest : g.shs) & 15u) == 0;
+    const int packed = aligned ? f.sh_coeffs : 0;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, par ? *par : ParameterArgs(), none, records, tiles_touched, rects,
                            depth_bits, wave_totals, lit, radii);
     };
-    if (radii_only) launch(preprocess_kernel<true, false, false>);
-    else if (par && packed) launch(preprocess_kernel<false, true, true>);
-    else if (par) launch(preprocess_kernel<false, true, false>);
-    else if (packed) launch(preprocess_kernel<false, false, true>);
-    else launch(preprocess_kernel<false, false, false>);
+    if (radii_only) launch(preprocess_kernel<true, false, 0>);
+    else if (packed == 16) launch(par ? preprocess_kernel<false, true, 16> : preprocess_kernel<false, false, 16>);
+    else if (packed == 9) launch(par ? preprocess_kernel<false, true, 9> : preprocess_kernel<false, false, 9>);
+    else if (packed == 4) launch(par ? preprocess_kernel<false, true, 4> : preprocess_kernel<false, false, 4>);
+    else launch(par ? preprocess_kernel<false, true, 0> : preprocess_kernel<false, false, 0>);
     GS355_CHECK_LAUNCH("preprocess");
     return GS355_OK;
 }
@@ -595,9 +603,9 @@ int launch_anchor_filter(const FrameArgs& f, const gs355_gaussians& g, const Fil
                            (uint32_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr, (uint2*)nullptr, (uint8_t*)nullptr, radii);
     };
     if (x.stored)
-        launch(preprocess_kernel<true, true, false>);
+        launch(preprocess_kernel<true, true, 0>);
     else
-        launch(preprocess_kernel<true, false, false>);
+        launch(preprocess_kernel<true, false, 0>);
     GS355_CHECK_LAUNCH("anchor filter");
     return GS355_OK;
 }
