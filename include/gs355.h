@@ -133,7 +133,7 @@ typedef struct gs355_layout {
     size_t rects;         /* u64[P]    tiles the Gaussian is blended in, zero when there are none: its tile rectangle
                            * (u16 x0, y0, x1, y1), or with GS355_STAGE_TILE_REACH a part of it (TileRegion in
                            * gs355_internal.h) */
-    size_t depth_bits;    /* u32[P]    view depth as raw bits (written for survivors only) */
+    size_t depth_bits;    /* u32[P]    view depth as raw bits (of the others: anything) */
     size_t offsets;       /* u32[P]   inclusive prefix sum of tiles_touched */
     size_t scan_tmp;      /* u32[...] block sums of the scans */
     size_t keys[2];       /* u64[n_cap] x 2 (ping-pong) */

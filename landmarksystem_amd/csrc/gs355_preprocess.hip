@@ -243,6 +243,10 @@ __device__ __forceinline__ uint64_t tile_region(const Rect q, float px, float py
     return corner | ((uint64_t)(mask | ((uint32_t)(w - 1) << 28) | 0x80000000u) << 32);
 }
 
+// Scenes from which on a wavefront's records leave as whole lines: at half a million the way through LDS costs what it saves
+// (colours given: 500k 14.8 us by lane, 15.0 by line; 1M 25.8 and 23.4; 130k 7.1 and 7.3).
+constexpr int kRecordLinesFrom = 1 << 19;
+
 // kStored: g holds the vanilla model's stored parameters, activated here (the activated copies would cost a pass over
 // memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
 // front of a kernel of 0.3 ms).
@@ -261,6 +265,8 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     typedef ShEntries<kStored, kPacked ? kPacked : 16> Entries;
     // staging area for the SH blocks of each wavefront's 64 Gaussians
     __shared__ float4 s_sh[kPacked ? 4 * 64 * Entries::kStride / 4 : 1];
+    // the records of each wavefront on their way out, where there are no rows to take their place
+    __shared__ float4 s_records[kRadiiOnly || kPacked ? 1 : 4 * 64 * 3];
     // the workgroup's surviving Gaussians, packed in order: position within the workgroup; survivors per wavefront
     __shared__ uint8_t s_owner[kPacked ? 256 : 1];
     __shared__ int s_alive[4];
@@ -433,6 +439,10 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
 
     // ---- colour ----
     float rgb[3] = {0.f, 0.f, 0.f};
+    const uint64_t alive_lanes = __ballot(alive);
+    // LDS of this wavefront alone, for its records: where there are rows, of what those leave, or over those that have been read
+    float4* out_rows = kPacked ? s_sh : s_records + (threadIdx.x >> 6) * 64 * 3;
+    bool room = P >= kRecordLinesFrom;
     const bool given = !kStored && !kPacked && g.colors_precomp != nullptr;
     if (given) {
         if (alive) {
@@ -448,7 +458,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         // values and the same order of additions either way.
         if constexpr (kPacked) {
             const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-            const uint64_t m = __ballot(alive);
+            const uint64_t m = alive_lanes;
             if (lane == 0) s_alive[wave] = __popcll(m);
             __syncthreads();
             int before = 0, total = 0;
@@ -485,6 +495,11 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
 #pragma unroll
                 for (int c = 0; c < 3; ++c) rgb[c] = my_row[Entries::kBeside + c];
             }
+            // (behind all survivors' rows, or over this wavefront's own)
+            constexpr int kRow4 = Entries::kStride / 4, kOutRows = (64 * 3 + kRow4 - 1) / kRow4;
+            const bool behind = total + 4 * kOutRows <= 256;
+            out_rows = s_sh + (behind ? total + wave * kOutRows : before) * kRow4;
+            room = room && (behind || __popcll(m) >= kOutRows);
         } else {
             reach_and_region();
             if (alive) {
@@ -505,13 +520,34 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
     // instead of 12 of the record's 48, whose cache lines it would read from end to end (preprocess backward of 6M
     // Gaussians 780 -> 723 us, for 2 us here, which the tile counts left out above give back).
     if (valid && !given) lit[i] = (uint8_t)((rgb[0] > 0.0f) | ((rgb[1] > 0.0f) << 1) | ((rgb[2] > 0.0f) << 2));
-    if (!alive) return;
-
-    float4* __restrict__ rec = reinterpret_cast<float4*>(records + (size_t)i * kRecordFloats);
-    rec[0] = make_float4(px, py, qx, qy);
-    rec[1] = make_float4(qz, opacity, rgb[0], rgb[1]);
-    rec[2] = make_float4(rgb[2], vz, ex, ey);
-    depth_bits[i] = __float_as_uint(vz);
+    const float4 r0 = make_float4(px, py, qx, qy), r1 = make_float4(qz, opacity, rgb[0], rgb[1]), r2 = make_float4(rgb[2], vz, ex, ey);
+    if (valid) depth_bits[i] = __float_as_uint(vz);
+    if (room) {
+        // A wavefront's records leave as whole lines, those of 64 B that hold some of a survivor's record: what else is in
+        // them is nobody's.  A lane that stores its own record makes three requests of 16 B, each of which takes a CU's path
+        // to the L2 as long as one of 64, and where neighbours were culled, lines that are written in parts.  20M Gaussians of
+        // which 57 / 44 / 24 % survive: 1184 / 1039 / 751 -> 1031 / 910 / 715 us (degree 0, 44 %: 666 -> 488), 6M of which
+        // 88 % do 380 -> 328, their stored parameters 393 -> 347 (the kernel by itself, again and again; within frames 305 ->
+        // 287 and 356 -> 301), 3.9M decoded Gaussians 78 -> 62.
+        const int lane = threadIdx.x & 63;
+        wave_lds_sync();
+        out_rows[3 * lane] = r0;
+        out_rows[3 * lane + 1] = r1;
+        out_rows[3 * lane + 2] = r2;
+        wave_lds_sync();
+        float4* __restrict__ dst = reinterpret_cast<float4*>(records + (size_t)(i - lane) * kRecordFloats);
+        const int end = 3 * min(64, P - (i - lane));
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int at = 64 * k + lane;
+            if (at < end && ((alive_lanes >> ((at & ~3) / 3)) & 3ull) != 0ull) dst[at] = out_rows[at];
+        }
+    } else if (alive) {
+        float4* __restrict__ rec = reinterpret_cast<float4*>(records + (size_t)i * kRecordFloats);
+        rec[0] = r0;
+        rec[1] = r1;
+        rec[2] = r2;
+    }
 }
 
 // One workgroup expands the keys of 256 consecutive Gaussians.  Output slots
@@ -579,9 +615,11 @@ int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const Parame
     if (g.P == 0) return GS355_OK;
     const dim3 block(256), grid((g.P + 255) / 256);
     const FilterArgs none;
-    // (any other number of coefficients, and blocks off the 16-byte boundaries of ordinary allocations: a lane per block)
+    // Any other number of coefficients, and blocks off the 16-byte boundaries of ordinary allocations: a lane per block.  So are
+    // small blocks of small scenes, whose lines the caches keep: four coefficients 17.7 us at 500k and 32.6 at 1M by lane, 18.7 and
+    // 29.6 by way of LDS; nine 10.0 at 130k and 16.4 at 250k by lane, 10.3 and 13.7.
     const bool aligned = (par || !g.colors_precomp) && (reinterpret_cast<uintptr_t>(par ? par->rest : g.shs) & 15u) == 0;
-    const int packed = aligned ? f.sh_coeffs : 0;
+    const int packed = aligned && g.P >= (f.sh_coeffs == 4 ? 1 << 19 : f.sh_coeffs == 9 ? 1 << 17 : 0) ? f.sh_coeffs : 0;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, par ? *par : ParameterArgs(), none, records, tiles_touched, rects,
                            depth_bits, wave_totals, lit, radii);
