@@ -145,7 +145,8 @@ typedef struct gs355_layout {
     size_t tile_base;     /* u32[2][tiles]   first slot of each tile's bucket; its next free slot during the scatter;
                            * then u64[ceil(tiles/64)], the first slot of each block of 64 tiles, and
                            * u32[ceil(tiles/16)+1], the work list of the scatter's second level, and
-                           * u32[ceil(tiles/64)], buckets per larger sorter size class in each block of 64 tiles */
+                           * u32[ceil(tiles/64)], buckets per larger sorter size class in each block of 64 tiles, and
+                           * u32[tiles], pairs per tile */
     size_t bin_visible;   /* {u64, u32, u32}[slices]  keys and visible Gaussians of each slice's share of what follows,
                            * {u32, u32}[ceil(P/64)]   keys and visible Gaussians per 64 Gaussians,
                            * u8[P]                    channels of a colour from SH coefficients that are above zero (bits) */
@@ -172,7 +173,8 @@ enum {
     /* Tile-bucketed equivalent of SCAN + DUPLICATE + SORT + RANGES: same sorted keys, values, ranges and
      * header, far less memory traffic.
      *   TILE_COUNT    pairs per (slice of Gaussians, tile) in LDS-private counters; prefix over slices; tile
-     *                 bases = ranges; header (key count, overflow, visible count).  Beyond 36000 tiles the
+     *                 bases = ranges; header (key count, overflow, visible count); where TILE_SCATTER follows in the same call, its
+     *                 launch makes bases, ranges and header.  Beyond 36000 tiles the
      *                 slices count per bin of 16 consecutive tiles, and ranges follow with TILE_SCATTER.
      *   TILE_SCATTER  (depth bits << 32 | index) pairs into their tile's bucket: straight for frames of fewer
      *                 than 6 * 2^20 pairs, through bins of 16 consecutive tiles beyond (decided on the device;

@@ -94,7 +94,7 @@ int make_layout(int32_t P, int64_t n_cap, int32_t W, int32_t H, gs355_layout* L)
     L->sort_hist = take(hist_words * sizeof(uint32_t));
     L->ranges = take(tiles * 2 * sizeof(uint32_t));
     L->bin_matrix = take((tiles <= (size_t)kBinMaxTilesWide ? bin_matrix_words(tiles) : 0) * sizeof(uint32_t));
-    L->tile_base = take((2 * tiles + 3 * ((tiles + 63) / 64) + (tiles + kCoarseTiles - 1) / kCoarseTiles + 1) * sizeof(uint32_t));
+    L->tile_base = take((3 * tiles + 3 * ((tiles + 63) / 64) + (tiles + kCoarseTiles - 1) / kCoarseTiles + 1) * sizeof(uint32_t));
     L->bin_visible = take((size_t)kBinMaxGroups * sizeof(SliceTotals) + wave_totals_count(P) * sizeof(uint2) + p);
     L->tile_lists = take((kListHeader + 4 * tiles) * sizeof(uint32_t));
     L->total_bytes = off;
@@ -307,11 +307,14 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
     // tile-bucketed path: buckets live in the buffer the sorted keys do not use
     const int tiles = fa.grid_x * fa.grid_y;
     uint64_t* buckets = keys[1 - L.sorted_buffer];
+    // a scatter that follows in the same call makes the layout, and the header, itself (not from counts per coarse bin)
+    const bool in_scatter = (stage_mask & GS355_STAGE_TILE_COUNT) && (stage_mask & GS355_STAGE_TILE_SCATTER) && tiles <= kBinMaxTiles;
+    const ScatterLayout make = {slice_totals, static_cast<gs355_header*>(out->header_copy)};
     if (stage_mask & GS355_STAGE_TILE_COUNT) {
         if ((rc = launch_tile_count(fa, g->P, rects, records, wave_totals, bin_matrix, slice_totals, s))) return rc;
         if ((rc = launch_tile_layout(g->P, bin_matrix, slice_totals, tiles, cap, header,
                                      static_cast<gs355_header*>(out->header_copy), tile_base, ranges, tile_lists,
-                                     s)))
+                                     in_scatter, s)))
             return rc;
     }
     if (stage_mask & GS355_STAGE_TILE_SCATTER)
@@ -321,7 +324,7 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
                                       (stage_mask & GS355_STAGE_TILE_SCATTER_TWO_LEVEL)   ? 2
                                       : (stage_mask & GS355_STAGE_TILE_SCATTER_ONE_LEVEL) ? 1
                                                                                           : 0,
-                                      s)))
+                                      in_scatter ? &make : nullptr, s)))
             return rc;
     if (stage_mask & GS355_STAGE_TILESORT)
         if ((rc = launch_tile_sort(header, tiles, ranges, tile_lists, buckets, keys[L.sorted_buffer],
@@ -373,18 +376,15 @@ int gs355_render_frame(const gs355_frame* frame, const gs355_gaussians* g, int32
     ParameterArgs par;
     par.rest = features_rest;
     const ParameterArgs* p = stored_parameters ? &par : nullptr;
-    // Both halves are checked before the first one is enqueued: from then on a store to the header is on its way, and a call
+    // All of it is checked before the first stage is enqueued: from then on a store to the header is on its way, and a call
     // that returned ahead of it would have it land in the next call's header, which would pass for that frame's.
     gs355_layout L;
     int rc = check_stages(frame, g, p, workspace, workspace_bytes, n_cap, out, stage_mask, &L);
     if (rc) return rc;
-    gs355_outputs later = *out;
-    later.header_copy = nullptr;
     volatile gs355_header* header = static_cast<volatile gs355_header*>(out->header_copy);
     header->ready = 0u;
     __atomic_thread_fence(__ATOMIC_SEQ_CST);
-    rc = enqueue_stages(frame, g, p, workspace, L, n_cap, out, stage_mask & kFront, stream);
-    if (!rc) rc = enqueue_stages(frame, g, p, workspace, L, n_cap, &later, stage_mask & ~kFront, stream);
+    rc = enqueue_stages(frame, g, p, workspace, L, n_cap, out, stage_mask, stream);
     if (rc) {  // (a launch failed: what was enqueued before it ends first, for the same reason)
         (void)hipStreamSynchronize(static_cast<hipStream_t>(stream));
         return rc;

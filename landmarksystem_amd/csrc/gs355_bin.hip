@@ -258,6 +258,161 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
 // launched and each returns at once when the other one applies.
 constexpr uint32_t kTwoLevelMinKeys = 6u << 20;
 
+// Layout of the buckets inside the scatter (frames whose scatter follows the slice prefix in one call; tile_publish_kernel
+// does the same in a launch of its own).  Every workgroup needs all tile bases anyway, and has them from the tiles' totals
+// for two scans of a wavefront per 64 tiles; a block of 64 tiles is published (cursors, ranges, size-class lists) by one
+// workgroup, the header by the first and the second level's work list by the last.  A launch of 256 threads for 256 tiles
+// takes 4.4 us, most of it start and end.  Frames of 10k Gaussians at 256x256 47.5 -> 45.3 us, 130k 89.3 -> 85.4, 1M large
+// splats 336 -> 329 and 6M 782 -> 773 at 1080p, 20M at 4K 1610 -> 1584 (with the first rectangles requested ahead of it, which is
+// 2 us of the 130k frame).
+struct LayoutArgs {
+    const uint32_t* totals;       // [tiles]; NULL: the layout is there already
+    const uint64_t* block_sums;   // [ceil(tiles / 64)]
+    const uint32_t* block_classes;
+    const SliceTotals* slice_totals;
+    uint32_t n_cap;
+    gs355_header* header;
+    gs355_header* header_copy;
+    uint32_t* ranges;
+    uint32_t* lists;
+    uint32_t* chunk_base;  // pairs per coarse bin, turned into chunks before each bin; NULL: no second level follows
+};
+
+// The frame's header from sums over all blocks and slices (one thread).  `in_class`: buckets per larger size class, or NULL.
+__device__ __forceinline__ void write_header(gs355_header* header, gs355_header* header_copy, uint64_t keys, uint32_t total,
+                                             bool overflow, uint32_t n_cap, uint32_t visible, const uint32_t* in_class)
+{
+    for (int k = 0; k < (header_copy ? 2 : 1); ++k) {
+        gs355_header* const h = k ? header_copy : header;
+        h->num_keys_total = keys;
+        h->num_keys = overflow ? n_cap : total;
+        h->overflow = overflow ? 1u : 0u;
+        h->num_visible = visible;
+        for (int c = 0; c < 3; ++c) h->sort_class_count[c] = in_class ? in_class[c] : 0xFFFFFFFFu;
+    }
+    if (header_copy) mark_ready(header_copy);
+}
+
+// A bucket's larger size class, or -1 (too small for the lists, or beyond the LDS sorters: sorted by its own workgroup of
+// the class-0 kernel).
+__device__ __forceinline__ int size_class(uint32_t n)
+{
+    if (n > (uint32_t)kTileSortCap[3]) return -1;
+    if (n > (uint32_t)kTileSortCap[2]) return 2;
+    if (n > (uint32_t)kTileSortCap[1]) return 1;
+    return n > (uint32_t)kTileSortCap[0] ? 0 : -1;
+}
+
+constexpr uint32_t chunks_of(uint32_t pairs);
+
+// Fills s_bin with this slice's first slot in each column and publishes the layout; returns the number of pairs, or
+// 0xFFFFFFFF for a frame that overflowed.  `scratch`: 4096 words of LDS, free again behind the next barrier.  `row`: what
+// earlier slices put into each tile.
+template <int kShift>
+__device__ __forceinline__ uint32_t lay_out(const LayoutArgs& a, int T, uint32_t* __restrict__ tile_base,
+                                            const uint32_t* __restrict__ row, uint32_t* __restrict__ s_bin,
+                                            uint32_t* __restrict__ scratch)
+{
+    static_assert((kBinMaxTiles + 63) / 64 <= kBinThreads && kBinMaxTiles < (1 << 16), "a block per thread, 16 bits a class");
+    static_assert(kBinMaxGroups <= kBinThreads, "a slice per thread");
+    constexpr int kWavesHere = kBinThreads / 64;
+    uint32_t* const s_block = scratch;                    // pairs before each block of 64 tiles
+    uint32_t* const s_classes = scratch + kBinThreads;    // buckets of classes 0 and 1 before it (16 bits each)
+    uint32_t* const s_class2 = scratch + 2 * kBinThreads;
+    uint32_t* const s_waves = scratch + 3 * kBinThreads;  // per wavefront: these three, visible Gaussians, keys
+    constexpr int kSums = 6;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int n_blocks = (T + 63) / 64;
+    // (the first block's values are under way while the sums are made)
+    const int t_first = wave * 64 + lane;
+    uint32_t next_total = t_first < T ? a.totals[t_first] : 0u, next_before = t_first < T ? row[t_first] : 0u;
+    const uint32_t pairs = tid < n_blocks ? (uint32_t)a.block_sums[tid] : 0u;  // (beyond 2^32 pairs the frame overflows)
+    const uint32_t word = tid < n_blocks ? a.block_classes[tid] : 0u;
+    SliceTotals slice = {0ull, 0u, 0u};
+    if (tid < (int)gridDim.x) slice = a.slice_totals[tid];
+    const uint32_t two = (word & 0xFFu) | ((word & 0xFF00u) << 8), third = (word >> 16) & 0xFFu;
+    const uint32_t pairs_inc = wave_sum_scan(pairs), two_inc = wave_sum_scan(two), third_inc = wave_sum_scan(third);
+    // (keys below 2^50, as two sums: 24 bits and the rest)
+    const uint32_t sums[kSums] = {pairs_inc, two_inc, third_inc, wave_sum_scan(slice.visible),
+                                  wave_sum_scan((uint32_t)slice.keys & 0xFFFFFFu), wave_sum_scan((uint32_t)(slice.keys >> 24))};
+    if (lane == 63) {
+#pragma unroll
+        for (int k = 0; k < kSums; ++k) s_waves[kWavesHere * k + wave] = sums[k];
+    }
+    __syncthreads();
+    uint32_t before[3], all[kSums];  // over the wavefronts, a lane each
+#pragma unroll
+    for (int k = 0; k < kSums; ++k) {
+        static_assert(kWavesHere == 16, "a row of lanes");
+        const uint32_t inc = row_scan(s_waves[kWavesHere * k + (lane & 15)], 0u, [](uint32_t x, uint32_t y) { return x + y; });
+        all[k] = (uint32_t)__builtin_amdgcn_readlane((int)inc, 15);
+        if (k < 3) before[k] = wave ? (uint32_t)__builtin_amdgcn_readlane((int)inc, wave - 1) : 0u;
+    }
+    const uint64_t keys = ((uint64_t)all[5] << 24) + all[4];  // of whole rectangles: at least the pairs
+    if (tid < n_blocks) {
+        s_block[tid] = before[0] + pairs_inc - pairs;
+        s_classes[tid] = before[1] + two_inc - two;
+        s_class2[tid] = before[2] + third_inc - third;
+    }
+    const bool overflow = keys > (uint64_t)a.n_cap;
+    if (blockIdx.x == 0 && tid == 0) {
+        const uint32_t in_class[3] = {all[1] & 0xFFFFu, all[1] >> 16, all[2]};
+        write_header(a.header, a.header_copy, keys, all[0], overflow, a.n_cap, all[3], in_class);
+        for (int c = 0; c < 3; ++c) a.lists[c] = in_class[c];
+    }
+    if (overflow) return 0xFFFFFFFFu;  // later stages do nothing either
+    __syncthreads();
+    for (int b = wave; b < n_blocks; b += kWavesHere) {  // (uniform per wavefront)
+        const int t = b * 64 + lane, t_next = t + kBinThreads;
+        const uint32_t v = next_total, earlier = next_before;
+        if (b + kWavesHere < n_blocks) {
+            next_total = t_next < T ? a.totals[t_next] : 0u;
+            next_before = t_next < T ? row[t_next] : 0u;
+        }
+        const uint32_t end = s_block[b] + wave_sum_scan(v), first = end - v;
+        if (kShift == 0) {
+            if (t < T) s_bin[t] = first + earlier;
+        } else {  // a column is a row of sixteen lanes
+            static_assert(kShift == 0 || kCoarseTiles == 16, "a row of lanes");
+            auto add = [](uint32_t x, uint32_t y) { return x + y; };
+            const uint32_t start = end - row_scan(v, 0u, add), sum = row_scan(earlier, 0u, add);  // (in the row's last lane)
+            if ((lane & 15) == 15 && (t & ~15) < T) s_bin[t >> kCoarseShift] = start + sum;
+        }
+        if ((uint32_t)b % gridDim.x != blockIdx.x) continue;
+        if (t < T) {
+            tile_base[t] = first;
+            tile_base[T + t] = first;  // the bucket's next free slot during the second level
+            a.ranges[2 * t] = v ? first : 0u;
+            a.ranges[2 * t + 1] = v ? end : 0u;
+        }
+        const int cls = size_class(v);
+        const uint32_t at[3] = {s_classes[b] & 0xFFFFu, s_classes[b] >> 16, s_class2[b]};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const uint64_t m = __ballot(cls == c);
+            if (cls == c) a.lists[kListHeader + (size_t)c * T + lanes_below_in(m, at[c])] = (uint32_t)t;
+        }
+    }
+    if (a.chunk_base && blockIdx.x == gridDim.x - 1) {
+        const int bins = (T + kCoarseTiles - 1) >> kCoarseShift, per_thread = (bins + kBinThreads - 1) / kBinThreads;
+        const int q0 = min(tid * per_thread, bins), q1 = min(q0 + per_thread, bins);
+        uint32_t chunks = 0;
+        for (int q = q0; q < q1; ++q) chunks += chunks_of(a.chunk_base[q]);
+        const uint32_t inc = wave_sum_scan(chunks);
+        if (lane == 63) s_waves[kSums * kWavesHere + wave] = inc;
+        __syncthreads();
+        uint32_t run = inc - chunks;
+        for (int w = 0; w < wave; ++w) run += s_waves[kSums * kWavesHere + w];
+        for (int q = q0; q < q1; ++q) {  // (each element is read before it is overwritten, by its own thread)
+            const uint32_t n = chunks_of(a.chunk_base[q]);
+            a.chunk_base[q] = run;
+            run += n;
+        }
+        if (tid == kBinThreads - 1) a.chunk_base[bins] = run;
+    }
+    return all[0];
+}
+
 // The walk of the counting kernel with one cursor per column: a coarse bin (kShift = kCoarseShift) or a tile
 // (kShift = 0, straight into the buckets).  The tiles of one rectangle row are consecutive, so a row takes one slot
 // request per coarse bin it crosses instead of one per tile.  Runs only when min_keys <= pairs of the frame <
@@ -269,39 +424,65 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
                                                               const uint64_t* __restrict__ rects,
                                                               const float* __restrict__ records,
                                                               const uint32_t* __restrict__ depth_bits,
-                                                              const gs355_header* __restrict__ header,
+                                                              const gs355_header* header,
                                                               uint32_t min_keys, uint32_t max_keys,
                                                               const uint32_t* __restrict__ matrix,
-                                                              const uint32_t* __restrict__ bases,
-                                                              uint64_t* __restrict__ dst)
+                                                              uint32_t* bases,
+                                                              uint64_t* __restrict__ dst, LayoutArgs layout)
 {
     static_assert(!kWide || kShift > 0, "beyond kBinMaxTiles tiles only coarse bins fit in LDS");
     extern __shared__ uint32_t s_bin[];  // [columns] next free slot of this slice in each column
     __shared__ uint32_t s_queue[kBinItems * kBinThreads];
     __shared__ uint32_t s_nqueue;
 
-    if (header->overflow || header->num_keys < min_keys || header->num_keys >= max_keys) return;
-    if (f.p_device) {
-        P = effective_count(f, P);
-        per_group = slice_size(P, (int)gridDim.x);
-    }
     constexpr int kSpan = 1 << kShift;
     const int T = f.grid_x * f.grid_y, bins = (T + kSpan - 1) >> kShift;
     const int tid = threadIdx.x, c = blockIdx.x, wave = tid >> 6, lane = tid & 63;
     // a column's first slot for this slice: the column's base (kWide: bases[b]; else the base of its first tile)
     // plus what the earlier slices put into it (the matrix holds that per bin when kWide, else per tile)
     const uint32_t* __restrict__ row = matrix + (size_t)c * (kWide ? bins : T);
-    for (int b = tid; b < bins; b += kBinThreads)
-        s_bin[b] = kWide ? bases[b] + row[b] : kShift ? bases[b << kShift] : bases[b] + row[b];
-    if (!kWide && kShift) {
-        __syncthreads();
-        for (int t = tid; t < T; t += kBinThreads) {
-            const uint32_t before = row[t];
-            if (before) atomicAdd(&s_bin[t >> kShift], before);
-        }
+    if (f.p_device) {
+        P = effective_count(f, P);
+        per_group = slice_size(P, (int)gridDim.x);
     }
     const int g_begin = min(P, c * per_group);
     const int g_end = min(P, g_begin + per_group);
+    // the first round's rectangles and depths, under way while the layout is made
+    const int lanes = lanes_per_gaussian(per_group);
+    uint64_t rr[kBinItems] = {};
+    uint32_t depths[kBinItems] = {};
+    auto request = [&](int first) {
+#pragma unroll
+        for (int u = 0; u < kBinItems; ++u) {
+            const int i = min(first + u * kBinThreads + tid, g_end - 1);
+            rr[u] = rects[i];
+            depths[u] = depth_bits[i];
+        }
+    };
+    if (g_begin < g_end) {  // (uniform)
+        if (lanes > 1) {
+            const int i = min(g_begin + tid / lanes, g_end - 1);
+            rr[0] = rects[i];
+            depths[0] = depth_bits[i];
+        } else {
+            request(g_begin);
+        }
+    }
+    if (!kWide && layout.totals) {  // (uniform)
+        const uint32_t keys = lay_out<kShift>(layout, T, bases, row, s_bin, s_queue);
+        if (keys == 0xFFFFFFFFu || keys < min_keys || keys >= max_keys) return;
+    } else {
+        if (header->overflow || header->num_keys < min_keys || header->num_keys >= max_keys) return;
+        for (int b = tid; b < bins; b += kBinThreads)
+            s_bin[b] = kWide ? bases[b] + row[b] : kShift ? bases[b << kShift] : bases[b] + row[b];
+        if (!kWide && kShift) {
+            __syncthreads();
+            for (int t = tid; t < T; t += kBinThreads) {
+                const uint32_t before = row[t];
+                if (before) atomicAdd(&s_bin[t >> kShift], before);
+            }
+        }
+    }
     // the tiles [ta, tb) of one rectangle row, cut where they cross into the next column
     auto emit_row = [&](int ta, int tb, uint64_t payload) {
         while (ta < tb) {
@@ -342,14 +523,13 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
             walk_region(q, record, lane, 64, f.grid_x, [&](int t) { emit_tile(t, payload); });
         }
     };
-    const int lanes = lanes_per_gaussian(per_group);
     if (lanes > 1) {  // (uniform; a single round, as in the count)
         if (tid == 0) s_nqueue = 0;
         __syncthreads();
         const int i = g_begin + tid / lanes, sub = tid % lanes;
         if (i < g_end) {
-            const TileRegion q(rects[i], f.plain_regions);
-            const uint64_t payload = payload_of(depth_bits[i], (uint32_t)i);
+            const TileRegion q(rr[0], f.plain_regions);
+            const uint64_t payload = payload_of(depths[0], (uint32_t)i);
             if (q.area > kInlineTiles * lanes) {
                 if (sub == 0) s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
             } else {
@@ -365,14 +545,8 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
     for (int first = g_begin; first < g_end; first += kBinItems * kBinThreads) {
         if (tid == 0) s_nqueue = 0;
         __syncthreads();
-        uint64_t rr[kBinItems];
-        uint32_t dd[kBinItems];
-#pragma unroll
-        for (int u = 0; u < kBinItems; ++u) {
-            const int i = min(first + u * kBinThreads + tid, g_end - 1);
-            rr[u] = rects[i];
-            dd[u] = depth_bits[i];
-        }
+        // (requested a round ahead, as in the count, they are awaited together with the stores in between: 6M Gaussians +6 us)
+        if (first != g_begin) request(first);
 #pragma unroll
         for (int u = 0; u < kBinItems; ++u) {
             const int i = first + u * kBinThreads + tid;
@@ -381,7 +555,7 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
                 if (q.area > (q.spans ? 0 : kInlineTiles)) {
                     s_queue[atomicAdd(&s_nqueue, 1u)] = (uint32_t)i;
                 } else {
-                    const uint64_t payload = payload_of(dd[u], (uint32_t)i);
+                    const uint64_t payload = payload_of(depths[u], (uint32_t)i);
                     walk_rows(q, f.grid_x, [&](int ta, int tb) { emit_row(ta, tb, payload); });
                 }
             }
@@ -404,6 +578,7 @@ constexpr int kFineThreads = 256;
 constexpr int kFineWaves = kFineThreads / 64;
 constexpr int kFineItems = 8;                             // pairs per thread and chunk
 constexpr int kFineChunk = kFineThreads * kFineItems;  // 2048 pairs = 16 KB of LDS
+constexpr uint32_t chunks_of(uint32_t pairs) { return (pairs + (uint32_t)kFineChunk - 1u) / (uint32_t)kFineChunk; }
 constexpr int kFineGrid = 8192;                          // a chunk per workgroup at 6M Gaussians / 1080p, a few each at 4K
 
 // A workgroup's run of chunks.  next() gives the following chunk's bin, first pair and pair count.
@@ -728,23 +903,12 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
     const uint64_t keys = (s_keys[0] + s_keys[1]) + (s_keys[2] + s_keys[3]);  // of whole rectangles: at least `total`
     const bool overflow = keys > (uint64_t)n_cap;
     if (blockIdx.x == 0 && threadIdx.x == 0 && !header_known) {
-        header->num_keys_total = keys;
-        header->num_keys = overflow ? n_cap : (uint32_t)total;
-        header->overflow = overflow ? 1u : 0u;
-        header->num_visible = (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]);
-        const bool counted = block_classes != nullptr;
-        const uint64_t in_class = (s_class_total[0] + s_class_total[1]) + (s_class_total[2] + s_class_total[3]);
-        for (int c = 0; c < 3; ++c) header->sort_class_count[c] = counted ? class_count(in_class, c) : 0xFFFFFFFFu;
-        if (counted && kTiles)
-            for (int c = 0; c < 3; ++c) lists[c] = class_count(in_class, c);
-        if (header_copy) {
-            header_copy->num_keys_total = keys;
-            header_copy->num_keys = overflow ? n_cap : (uint32_t)total;
-            header_copy->overflow = overflow ? 1u : 0u;
-            header_copy->num_visible = (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]);
-            for (int c = 0; c < 3; ++c) header_copy->sort_class_count[c] = counted ? class_count(in_class, c) : 0xFFFFFFFFu;
-            mark_ready(header_copy);
-        }
+        const uint64_t packed = (s_class_total[0] + s_class_total[1]) + (s_class_total[2] + s_class_total[3]);
+        const uint32_t in_class[3] = {class_count(packed, 0), class_count(packed, 1), class_count(packed, 2)};
+        write_header(header, header_copy, keys, (uint32_t)total, overflow, n_cap, (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]),
+                     block_classes ? in_class : nullptr);
+        if (block_classes && kTiles)
+            for (int c = 0; c < 3; ++c) lists[c] = in_class[c];
     }
     if (overflow) return;  // later stages do nothing either
 
@@ -752,7 +916,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         const int per_thread = (bins + 255) / 256;
         const int q0 = min((int)threadIdx.x * per_thread, bins), q1 = min(q0 + per_thread, bins);
         uint32_t chunks = 0;
-        for (int q = q0; q < q1; ++q) chunks += (bin_pairs[q] + (uint32_t)kFineChunk - 1u) / (uint32_t)kFineChunk;
+        for (int q = q0; q < q1; ++q) chunks += chunks_of(bin_pairs[q]);
         uint32_t cinc = chunks;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
@@ -764,7 +928,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         uint32_t run = cinc - chunks;
         for (int w = 0; w < wave; ++w) run += s_chunks[w];
         for (int q = q0; q < q1; ++q) {  // (each element is read before it is overwritten, by its own thread)
-            const uint32_t n = (bin_pairs[q] + (uint32_t)kFineChunk - 1u) / (uint32_t)kFineChunk;
+            const uint32_t n = chunks_of(bin_pairs[q]);
             chunk_base[q] = run;
             run += n;
         }
@@ -788,11 +952,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
     }
     // buckets beyond the smallest sorter's capacity go on the list of their size class (order within a list is free;
     // without counts by block, one request per wavefront and class)
-    int cls = -1;
-    if (v > (uint32_t)kTileSortCap[3]) cls = -1;  // beyond the LDS sorters: sorted by its own workgroup of the class-0 kernel
-    else if (v > (uint32_t)kTileSortCap[2]) cls = 2;
-    else if (v > (uint32_t)kTileSortCap[1]) cls = 1;
-    else if (v > (uint32_t)kTileSortCap[0]) cls = 0;
+    const int cls = size_class(v);
     uint64_t class_first = 0;
     if (block_classes) {
         class_first = (s_class_before[0] + s_class_before[1]) + (s_class_before[2] + s_class_before[3]);
@@ -1500,11 +1660,15 @@ static int allow_large_lds()
 }
 
 static inline int coarse_bins(int tiles) { return (tiles + kCoarseTiles - 1) >> kCoarseShift; }
-// the tile_base array: u32[2][tiles], u64[blocks of 64 tiles], u32[coarse bins + 1] chunk bases
+// the tile_base array: u32[2][tiles], u64[blocks of 64 tiles], u32[coarse bins + 1] chunk bases, u32[blocks] size classes,
+// u32[tiles] pairs per tile (up to kBinMaxTiles tiles)
+static inline uint64_t* block_totals(uint32_t* tile_base, int tiles) { return reinterpret_cast<uint64_t*>(tile_base + 2 * (size_t)tiles); }
 static inline uint32_t* chunk_bases(uint32_t* tile_base, int tiles)
 {
     return tile_base + 2 * (size_t)tiles + 2 * (size_t)((tiles + 63) / 64);
 }
+static inline uint32_t* class_counts(uint32_t* tile_base, int tiles) { return chunk_bases(tile_base, tiles) + coarse_bins(tiles) + 1; }
+static inline uint32_t* tile_totals(uint32_t* tile_base, int tiles) { return class_counts(tile_base, tiles) + (tiles + 63) / 64; }
 
 int launch_tile_count(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint2* wave_totals,
                       uint32_t* matrix, SliceTotals* slice_totals, hipStream_t s)
@@ -1544,22 +1708,26 @@ static int launch_layout(const uint32_t* totals, uint32_t* bases, int columns, c
 
 // Up to kBinMaxTiles tiles: everything the later stages need (tile bases, cursors, ranges, size-class lists,
 // header).  Beyond: the header and the coarse bins' bases (in tile_cursor[0, bins)); the per-tile layout follows
-// in launch_tile_scatter once the pairs of each bin can be counted by tile.
+// in launch_tile_scatter once the pairs of each bin can be counted by tile.  `in_scatter`: the scatter follows in the same
+// call and publishes the layout itself (ScatterLayout), where there is one counter per tile.
 int launch_tile_layout(int32_t P, uint32_t* matrix, const SliceTotals* slice_totals, int tiles, uint32_t n_cap,
-                       gs355_header* header, gs355_header* header_copy, uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, hipStream_t s)
+                       gs355_header* header, gs355_header* header_copy, uint32_t* tile_base, uint32_t* ranges, uint32_t* lists,
+                       bool in_scatter, hipStream_t s)
 {
     int per_group;
     const int groups = bin_groups(P, &per_group);
-    uint64_t* blocks = reinterpret_cast<uint64_t*>(tile_base + 2 * (size_t)tiles);
+    uint64_t* blocks = block_totals(tile_base, tiles);
     const int bins = coarse_bins(tiles);
     uint32_t* chunk_base = chunk_bases(tile_base, tiles);
-    uint32_t* block_classes = chunk_base + bins + 1;  // [ceil(tiles / 64)]
     if (tiles <= kBinMaxTiles) {
+        uint32_t* block_classes = class_counts(tile_base, tiles);
+        uint32_t* totals = tile_totals(tile_base, tiles);
         // (the pairs of each coarse bin go to chunk_base, which the block scan turns into chunk bases in place)
         hipLaunchKernelGGL(slice_prefix_kernel, dim3((tiles + 63) / 64), dim3(64 * kPrefixParts), 0, s, matrix, groups, tiles,
-                           tile_base, blocks, chunk_base, block_classes, lists);
+                           totals, blocks, chunk_base, block_classes, lists);
         GS355_CHECK_LAUNCH("bin: slice prefix");
-        return launch_layout<true>(tile_base, tile_base, tiles, blocks, slice_totals, groups, n_cap, header, header_copy, false, ranges,
+        if (in_scatter) return GS355_OK;
+        return launch_layout<true>(totals, tile_base, tiles, blocks, slice_totals, groups, n_cap, header, header_copy, false, ranges,
                                    lists, chunk_base, bins, chunk_base, block_classes, s);
     }
     // (both in the cursor half of tile_base, which the tile-level layout of launch_tile_scatter overwrites later)
@@ -1575,7 +1743,7 @@ int launch_tile_layout(int32_t P, uint32_t* matrix, const SliceTotals* slice_tot
 int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint32_t* depth_bits,
                         gs355_header* header, const uint32_t* matrix, uint32_t n_cap,
                         uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, uint64_t* buckets, uint64_t* coarse,
-                        int levels, hipStream_t s)
+                        int levels, const ScatterLayout* make, hipStream_t s)
 {
     int per_group;
     const int groups = bin_groups(P, &per_group);
@@ -1587,24 +1755,29 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
     uint32_t min_keys = 0;  // pairs from which the two levels run
     bool fine = true;
     if (T <= kBinMaxTiles) {
+        LayoutArgs layout = {};  // (the first launch makes it)
+        if (make)
+            layout = {tile_totals(tile_base, T), block_totals(tile_base, T), class_counts(tile_base, T), make->slice_totals, n_cap,
+                      header, make->header_copy, ranges, lists, levels != 1 ? chunk_bases(tile_base, T) : nullptr};
         if (levels != 2) {
             min_keys = levels == 1 ? UINT32_MAX : kTwoLevelMinKeys;
             hipLaunchKernelGGL((scatter_kernel<0, false>), dim3(groups), dim3(kBinThreads), (size_t)T * sizeof(uint32_t), s,
-                               f, P, per_group, rects, records, depth_bits, header, 0u, min_keys, matrix, tile_base, buckets);
+                               f, P, per_group, rects, records, depth_bits, header, 0u, min_keys, matrix, tile_base, buckets, layout);
             GS355_CHECK_LAUNCH("bin: scatter");
+            layout.totals = nullptr;
         }
         fine = levels != 1;
         if (fine) {
             hipLaunchKernelGGL((scatter_kernel<kCoarseShift, false>), dim3(groups), dim3(kBinThreads), coarse_lds, s, f, P,
-                               per_group, rects, records, depth_bits, header, min_keys, UINT32_MAX, matrix, tile_base, coarse);
+                               per_group, rects, records, depth_bits, header, min_keys, UINT32_MAX, matrix, tile_base, coarse, layout);
             GS355_CHECK_LAUNCH("bin: coarse scatter");
         }
     } else {
-        const uint32_t* bin_base = tile_cursor;  // (replaced by the tiles' cursors once the coarse level is done)
+        uint32_t* bin_base = tile_cursor;  // (replaced by the tiles' cursors once the coarse level is done)
         hipLaunchKernelGGL((scatter_kernel<kCoarseShift, true>), dim3(groups), dim3(kBinThreads), coarse_lds, s, f, P,
-                           per_group, rects, records, depth_bits, header, 0u, UINT32_MAX, matrix, bin_base, coarse);
+                           per_group, rects, records, depth_bits, header, 0u, UINT32_MAX, matrix, bin_base, coarse, LayoutArgs{});
         GS355_CHECK_LAUNCH("bin: coarse scatter");
-        uint64_t* blocks = reinterpret_cast<uint64_t*>(tile_base + 2 * (size_t)T);
+        uint64_t* blocks = block_totals(tile_base, T);
         if ((rc = launch_fill_u32(tile_base, (size_t)T, 0u, s))) return rc;
         if ((rc = launch_fill_u32(reinterpret_cast<uint32_t*>(blocks), 2 * (size_t)((T + 63) / 64), 0u, s))) return rc;
         hipLaunchKernelGGL(fine_count_kernel, dim3(kFineGrid), dim3(kFineThreads), 0, s, header, bin_base, bins, T,

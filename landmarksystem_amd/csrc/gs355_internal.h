@@ -389,7 +389,8 @@ inline size_t bin_matrix_words(size_t tiles)
     return (size_t)kBinMaxGroups * columns;
 }
 // tile_base: u32[2][tiles] (bases, then the scatter's cursors), then u64[ceil(tiles / 64)] (bases of blocks of 64 tiles),
-// then u32[coarse bins + 1] (chunks of the second scatter level before each bin).  Beyond kBinMaxTiles tiles launch_tile_layout
+// then u32[coarse bins + 1] (chunks of the second scatter level before each bin), u32[ceil(tiles / 64)] (buckets per larger
+// sorter size class) and u32[tiles] (pairs per tile).  Beyond kBinMaxTiles tiles launch_tile_layout
 // publishes the header and the coarse bins' bases only; ranges, lists and tile bases follow in launch_tile_scatter.
 // per slice, and before it per 64 Gaussians (the preprocess's wavefronts): keys of the whole rectangles, Gaussians with a
 // radius.  The frame's key count and its overflow go by the whole rectangles, so that a capacity that suffices for them
@@ -402,14 +403,20 @@ inline size_t wave_totals_count(int32_t P) { return ((size_t)P + 63) / 64; }
 int launch_tile_count(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint2* wave_totals,
                       uint32_t* matrix, SliceTotals* slice_totals, hipStream_t s);
 int launch_tile_layout(int32_t P, uint32_t* matrix, const SliceTotals* slice_totals, int tiles, uint32_t n_cap,
-                       gs355_header* header, gs355_header* header_copy, uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, hipStream_t s);
+                       gs355_header* header, gs355_header* header_copy, uint32_t* tile_base, uint32_t* ranges, uint32_t* lists,
+                       bool in_scatter, hipStream_t s);
+// What a scatter that makes the layout itself (after launch_tile_layout with `in_scatter`) needs besides its own arguments.
+struct ScatterLayout {
+    const SliceTotals* slice_totals;
+    gs355_header* header_copy;
+};
 // `coarse`: a second buffer of the buckets' size (first level of the two-level scatter).  `levels`: 1 or 2 = that
 // scatter whatever the frame holds, 0 = chosen on the device by the key count (both variants are launched); images
-// beyond kBinMaxTiles tiles always take two levels
+// beyond kBinMaxTiles tiles always take two levels.  `make`: NULL, or the layout is made on the way (up to kBinMaxTiles tiles)
 int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint32_t* depth_bits,
                         gs355_header* header, const uint32_t* matrix, uint32_t n_cap,
                         uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, uint64_t* buckets, uint64_t* coarse,
-                        int levels, hipStream_t s);
+                        int levels, const ScatterLayout* make, hipStream_t s);
 // lists: u32[kListHeader + 4 * tiles]: the four class counts, four spare words, the four lists
 constexpr int kListHeader = 8;
 int launch_tile_sort(const gs355_header* header, int tiles, const uint32_t* ranges, uint32_t* lists,

@@ -2,8 +2,10 @@
 the numbers of lanes and with rectangles on both sides of the queue's threshold, against the classic stages' arrays."""
 import numpy as np
 import pytest
+import torch
 
-from landmarksystem_amd import _lib, scenes
+from landmarksystem_amd import _lib, pipeline, scenes
+from tests.helpers import settings_for
 from tests.test_gpu_parity import crowded_scene, run_all_stages, run_fast_path
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +42,51 @@ def test_sorted_values_without_their_keys(gpu_device, make, skip):
     got = run_fast_path(scene, gpu_device, modifiers=skip | _lib.STAGE_TILESORT_VALUES)
     for name in ("ranges", "sorted_values", "image", "depth", "alpha"):
         np.testing.assert_array_equal(got[name], want[name], err_msg=name)
+
+
+@pytest.mark.parametrize("width,height,P,log_scale", [
+    (16, 16, 70, 0.0), (16 * 63, 16, 3000, -2.0), (16 * 64, 16, 3000, -2.0), (16 * 65, 16, 3000, -2.0), (1000, 700, 9000, -2.5),
+    (16 * 1023, 16, 20_000, -2.5), (4096, 2304, 40_000, -5.0), (16 * 360, 1600, 40_000, -5.0)])
+@pytest.mark.parametrize("levels", [0, _lib.STAGE_TILE_SCATTER_ONE_LEVEL, _lib.STAGE_TILE_SCATTER_TWO_LEVEL])
+def test_layout_made_by_the_scatter(gpu_device, width, height, P, log_scale, levels):
+    """Tile count and scatter in one call, where the scatter makes the layout, against one call each: at the edges of the
+    layout's blocks of 64 tiles and of a workgroup's sixteen of them, up to the 36000 tiles of the LDS counters; and for a
+    capacity one key short."""
+    scene = scenes.tiny_scene(P=P, width=width, height=height, sh_degree=0, seed=3, log_scale_mean=log_scale)
+    inp = pipeline.FrameInputs(settings_for(scene, gpu_device), scene.means3D.to(gpu_device), shs=scene.shs.to(gpu_device),
+                               opacities=scene.opacities.to(gpu_device), scales=scene.scales.to(gpu_device),
+                               rotations=scene.rotations.to(gpu_device))
+    tiles = inp.tiles
+
+    def frame(joint, n_cap):
+        out, ws = pipeline.FrameOutputs(inp), pipeline.Workspace(gpu_device)
+        lay = ws.ensure(P, n_cap, width, height)
+        ws.buffer.fill_(0xA5)
+        if joint:
+            masks = (_lib.STAGE_PREPROCESS, _lib.STAGE_TILE_COUNT | _lib.STAGE_TILE_SCATTER | levels)
+        else:
+            masks = (_lib.STAGE_PREPROCESS, _lib.STAGE_TILE_COUNT, _lib.STAGE_TILE_SCATTER | levels)
+        for mask in masks + (_lib.STAGE_TILESORT,):
+            pipeline.run_stages(inp, out, ws, n_cap, mask)
+        torch.cuda.synchronize()
+        raw = ws.buffer.cpu().numpy()
+        header = raw[lay.header:lay.header + 32].view(np.uint32)
+        lists = raw[lay.tile_lists:lay.tile_lists + 4 * (8 + 4 * tiles)].view(np.uint32)
+        got = {"header": header}
+        if header[3] == 0:
+            n = int(header[2])
+            got["ranges"] = raw[lay.ranges:lay.ranges + 8 * tiles].view(np.uint32)
+            got["keys"] = ws.view(lay, "sorted_keys", P, n, tiles).cpu().numpy()
+            got["values"] = ws.view(lay, "sorted_values", P, n, tiles).cpu().numpy()
+            got["counts"] = lists[:3]
+            for c in range(3):
+                got["list %d" % c] = np.sort(lists[8 + c * tiles:][:lists[c]])
+        return got
+
+    total = int(frame(False, 1 << 25)["header"][0])
+    assert 0 < total < 1 << 25
+    for n_cap in (total, total - 1):
+        want, got = frame(False, n_cap), frame(True, n_cap)
+        assert want["header"][3] == (n_cap < total) and want.keys() == got.keys()
+        for name in want:
+            np.testing.assert_array_equal(got[name], want[name], err_msg=name)
