@@ -64,12 +64,15 @@ struct DecodeArgs {
     const float* b0[3];
     const float* w1[3];
     const float* b1[3];
-    // one-call decode (gs355_decode): the count pass leaves per-run totals behind, a one-workgroup scan turns
+    // one-call decode (gs355_decode): the count pass leaves per-run totals behind, a one-workgroup scan (or the emit pass) turns
     // them into run bases, and the emit pass (which recomputes the opacity head: matrix instructions are cheap
     // here, registers and memory requests are not) places its Gaussians from those instead of per-anchor offsets
     uint2* run_totals;       // [runs] (kept offsets, visible anchors) per run of anchors, or NULL
     uint2* run_tiles;        // [runs] kept offsets of the run before each of its four tiles, 16 bits each (with run_totals)
     const uint2* run_base;   // [runs] exclusive prefix of run_totals, or NULL
+    int scan_here;           // the emit pass makes that prefix itself (runs <= kScanStripes * its workgroups), and the sums:
+    uint32_t* num_emitted;   // of the kept offsets, or NULL
+    uint32_t* num_visible;   // of the visible anchors, or NULL
     float* neural_opacity;   // [A_vis * n] tanh of every pre-activation, in visible-anchor order, or NULL
     uint8_t* kept_mask;      // [A_vis * n] pre-activation > 0, or NULL
 };
@@ -429,6 +432,11 @@ __global__ __launch_bounds__(64 * kCountWaves, 4) void decode_count_kernel(Decod
 // 84 us; a million anchors behind a level-of-detail mask 59 -> 38 us; 60k anchors, where a wavefront has one tile, 31 -> 15.
 constexpr int kEmitWaves = 12;
 constexpr int kEmitCap = 256;  // workgroups: one per CU
+// Up to this many runs per workgroup the emit pass adds up the runs' totals itself: a workgroup's k-th run needs the runs of
+// the stripes before (gridDim.x runs each) and those before it in its own.  62 KB per workgroup at a million anchors, read
+// while the weights are, in the place of a launch of one workgroup of 3 to 5 us: frames of 60k anchors 116 -> 113 us, of a
+// million behind a level-of-detail mask 203 -> 200.6, of 500k 371 -> 369.
+constexpr int kScanStripes = 32;
 constexpr int kRowWords = 72;  // an anchor's words: first opacity, colour, offset scale, position; then covariance
 constexpr int kRowColour = 16, kRowExtra = 48;
 
@@ -459,9 +467,25 @@ __global__ __launch_bounds__(64 * kEmitWaves, 3) void decode_emit_kernel(DecodeA
     __shared__ float s_bias[256];
     __shared__ half8_t s_hi[kAllFrags];
     __shared__ half8_t s_lo[kWLo ? kAllFrags : 1];
+    __shared__ uint4 s_stripe[kScanStripes];  // (kept offsets, visible anchors) of a stripe of runs, and of those before this workgroup's
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
     const int n = d.n;
     const int runs = (d.A + kRun - 1) / kRun;
+    if (d.scan_here) {
+        static_assert(kEmitCap <= 4 * 64, "four runs of a stripe per lane");
+        for (int k = wave; k * (int)gridDim.x < runs; k += kEmitWaves) {
+            uint2 all = make_uint2(0u, 0u), before = make_uint2(0u, 0u);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int at = 64 * u + lane, r = k * (int)gridDim.x + at;
+                const uint2 v = at < (int)gridDim.x && r < runs ? d.run_totals[r] : make_uint2(0u, 0u);
+                all = make_uint2(all.x + v.x, all.y + v.y);
+                if (at < (int)blockIdx.x) before = make_uint2(before.x + v.x, before.y + v.y);
+            }
+            const uint4 sums = make_uint4(wave_sum(all.x), wave_sum(all.y), wave_sum(before.x), wave_sum(before.y));
+            if (lane == 0) s_stripe[k] = sums;
+        }
+    }
     stage_biases(d, s_bias, 64 * kEmitWaves);
     for (int f = wave; f < 19; f += kEmitWaves) {
         const int head = f < 5 ? 0 : f < 14 ? 1 : 2;
@@ -478,10 +502,19 @@ __global__ __launch_bounds__(64 * kEmitWaves, 3) void decode_emit_kernel(DecodeA
         const int my_run = first_run + lane * (int)gridDim.x;
         uint32_t tiles = my_run < runs ? kRunTiles : 0;  // two-call decode: the visible anchors are not known here
         uint2 run_base = make_uint2(0u, 0u), run_tiles = make_uint2(0u, 0u);
-        if (d.run_base && my_run < runs) {
+        if (!offsets && my_run < runs) {
             tiles = (d.run_totals[my_run].y + 31u) >> 5;
-            run_base = d.run_base[my_run];
             run_tiles = d.run_tiles[my_run];
+            if (!d.scan_here) run_base = d.run_base[my_run];
+        }
+        if (d.scan_here) {  // (one round: a lane per stripe)
+            const uint4 v = my_run < runs ? s_stripe[lane] : make_uint4(0u, 0u, 0u, 0u);
+            const uint32_t x = wave_sum_scan(v.x), y = wave_sum_scan(v.y);
+            run_base = make_uint2(x - v.x + v.z, y - v.y + v.w);
+            if (blockIdx.x == 0 && wave == 0 && lane == 63) {
+                if (d.num_emitted) *d.num_emitted = x;
+                if (d.num_visible) *d.num_visible = y;
+            }
         }
         uint32_t upto = tiles;
 #pragma unroll
@@ -927,6 +960,9 @@ static int fill_args(const gs355_decoder* dec, const gs355_anchors* an, bool all
     a.run_totals = nullptr;
     a.run_tiles = nullptr;
     a.run_base = nullptr;
+    a.scan_here = 0;
+    a.num_emitted = nullptr;
+    a.num_visible = nullptr;
     a.neural_opacity = nullptr;
     a.kept_mask = nullptr;
     *out = a;
@@ -1145,6 +1181,8 @@ int gs355_decode(const gs355_decoder* dec, const gs355_anchors* an, int64_t capa
     uint2* run_base = reinterpret_cast<uint2*>(ws + L.run_base);
     a.run_totals = reinterpret_cast<uint2*>(ws + L.run_totals);
     a.run_tiles = reinterpret_cast<uint2*>(ws + L.run_tiles);
+    const bool emits = do_emit && (capacity > 0 || out->neural_opacity || out->mask);
+    a.scan_here = do_count && emits && runs <= (uint32_t)(kScanStripes * kEmitCap);
     if (do_count) {
         if (bank) {
             BankArgs b;
@@ -1165,11 +1203,12 @@ int gs355_decode(const gs355_decoder* dec, const gs355_anchors* an, int64_t capa
         }
         launch_count(s, a, nullptr);
         GS355_CHECK_LAUNCH("decode: count");
-        if ((rc = launch_run_scan(a.run_totals, run_base, runs, out->count, out->num_visible, s))) return rc;
+        if (!a.scan_here && (rc = launch_run_scan(a.run_totals, run_base, runs, out->count, out->num_visible, s))) return rc;
     }
-    if (!do_emit) return GS355_OK;
-    if (capacity == 0 && !out->neural_opacity && !out->mask) return GS355_OK;
+    if (!emits) return GS355_OK;
     a.run_base = run_base;
+    a.num_emitted = out->count;
+    a.num_visible = out->num_visible;
     a.neural_opacity = out->neural_opacity;
     a.kept_mask = out->mask;
     launch_emit(s, a, nullptr, (uint32_t)capacity, *out);

@@ -371,3 +371,28 @@ def test_a_copy_of_a_decoder_that_has_decoded(gpu_device):
         for twin in (copy.deepcopy(dec), pickle.loads(pickle.dumps(dec))):
             for a, b in zip(twin(*call)[:5], want):
                 assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("A,frac", [(1, 1.0), (128, 0.9), (129, 1.0), (32_768, 0.5), (32_769, 0.02), (70_001, 0.6), (1_048_576, 0.1),
+                                    (1_048_577, 0.1)])
+def test_decode_that_scans_its_runs_by_itself(gpu_device, A, frac):
+    """One call for counting and emitting, where the emit pass makes the prefix over the runs of anchors, against a call each
+    (the prefix in a launch of its own; beyond 2^20 anchors in both): the same counts and Gaussians bit for bit, at the edges of
+    a run, of a run per workgroup and of the largest prefix."""
+    sc = scenes.config5(A=A)
+    dec = build_decoder(sc, gpu_device)
+    g = torch.Generator().manual_seed(A)
+    vis = torch.rand(A, generator=g) < frac
+    vis[A - 1] = True
+    t = [x.to(gpu_device).contiguous() for x in (sc.camera.camera_center, sc.anchor, sc.anchor_feat, sc.offset, sc.scaling)]
+    vis = vis.to(gpu_device)
+    res = dec.decode_on_device(*t, vis, want_training_outputs=True)
+    want = dec(*t, vis)
+    G, a_vis = dec.read_counts(res)
+    assert (G, a_vis) == (want[0].shape[0], int(vis.sum()))
+    for name, a, b in zip(("xyz", "color", "opacity", "scaling", "rot"), (res.xyz, res.color, res.opacity, res.scaling, res.rot), want):
+        assert torch.equal(a[:G], b), name
+    with torch.no_grad():
+        every = dec.train()(*t, vis)
+    for name, a, b in zip(("neural_opacity", "mask"), (res.neural_opacity, res.mask), every[5:]):
+        assert torch.equal(a.reshape(-1)[:10 * a_vis], b.reshape(-1)), name
