@@ -374,11 +374,11 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
 #pragma unroll
                     for (int b = 0; b < 4; ++b) {  // (two blocks may hold the same entry)
                         if ((any & (kBlockLanes << (4 * b))) == 0ull) continue;  // (uniform: nothing blended in the block)
-                        if (group == b) {
+                        if (group == b) {  // (rows 2 and 3 hold what rows 0 and 1 do for the last pair: one exchange with LDS, not two)
                             const float2 v = sums[row];
                             const float l = *last;
                             sums[row] = make_float2(v.x + sum_a, v.y + sum_b);
-                            if (row < 2) *last = l + sum_c;
+                            *last = l + sum_c;
                         }
                         wave_lds_sync();
                     }
