@@ -121,7 +121,8 @@ typedef struct gs355_header {
     uint32_t ready;          /* set to 1 in a header copy, after everything else in it (in the workspace: not used) */
     uint32_t parts;          /* preprocess stage: 1 if `rects` holds parts of tile rectangles (GS355_STAGE_TILE_REACH), else 0
                               * (in the workspace only) */
-    uint32_t reserved[6];
+    uint32_t ordered;        /* tile-sort stage: 1 once it has put the tiles in the order the blends take them (in the workspace only) */
+    uint32_t reserved[5];
 } gs355_header;
 
 /* Byte offsets of every array inside the caller's workspace (each 256-byte
@@ -150,7 +151,8 @@ typedef struct gs355_layout {
     size_t bin_visible;   /* {u64, u32, u32}[slices]  keys and visible Gaussians of each slice's share of what follows,
                            * {u32, u32}[ceil(P/64)]   keys and visible Gaussians per 64 Gaussians,
                            * u8[P]                    channels of a colour from SH coefficients that are above zero (bits) */
-    size_t tile_lists;    /* u32[8+4*tiles]  counts, work counters and lists of the buckets of each larger sorter size class */
+    size_t tile_lists;    /* u32[8+4*tiles]  counts, work counters and lists of the buckets of each larger sorter size class,
+                           * {u32 tile, first, last, 0}[tiles]  the tiles by the length of their lists (257 to 36000 tiles) */
     size_t total_bytes;
     int32_t unsorted_buffer; /* which keys/values buffer the duplicate stage writes (0) */
     int32_t sorted_buffer;   /* which buffer holds the sorted pairs after the sort stage */

@@ -86,7 +86,8 @@ class Header(C.Structure):
         ("sort_class_count", C.c_uint32 * 3),
         ("ready", C.c_uint32),
         ("parts", C.c_uint32),
-        ("reserved", C.c_uint32 * 6),
+        ("ordered", C.c_uint32),
+        ("reserved", C.c_uint32 * 5),
     ]
 
 

@@ -96,7 +96,7 @@ int make_layout(int32_t P, int64_t n_cap, int32_t W, int32_t H, gs355_layout* L)
     L->bin_matrix = take((tiles <= (size_t)kBinMaxTilesWide ? bin_matrix_words(tiles) : 0) * sizeof(uint32_t));
     L->tile_base = take((3 * tiles + 3 * ((tiles + 63) / 64) + (tiles + kCoarseTiles - 1) / kCoarseTiles + 1) * sizeof(uint32_t));
     L->bin_visible = take((size_t)kBinMaxGroups * sizeof(SliceTotals) + wave_totals_count(P) * sizeof(uint2) + p);
-    L->tile_lists = take((kListHeader + 4 * tiles) * sizeof(uint32_t));
+    L->tile_lists = take((kListHeader + 8 * tiles) * sizeof(uint32_t));
     L->total_bytes = off;
     L->sort_bits = 32 + ceil_log2((uint32_t)tiles);
     L->sort_passes = (L->sort_bits + kRadixBits - 1) / kRadixBits;
@@ -335,7 +335,7 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
                                    s)))
             return rc;
     if (stage_mask & (GS355_STAGE_BLEND | GS355_STAGE_BLEND_PLAIN))
-        if ((rc = launch_blend(fa, header, ranges, vals[L.sorted_buffer], records, out->image, out->depth, out->alpha,
+        if ((rc = launch_blend(fa, header, ranges, tile_order(tile_lists, tiles), vals[L.sorted_buffer], records, out->image, out->depth, out->alpha,
                                (stage_mask & GS355_STAGE_BLEND) != 0, s)))
             return rc;
     return GS355_OK;
@@ -473,8 +473,10 @@ static int render_backward(const gs355_frame* frame, const gs355_gaussians* g, c
                          g->P, (long long)n_cap);
     const char* ws = static_cast<const char*>(workspace);
     char* sc = static_cast<char*>(scratch);
-    return launch_render_backward(make_args(frame), *g, reinterpret_cast<const gs355_header*>(ws + L.header),
+    const FrameArgs fa = make_args(frame);
+    return launch_render_backward(fa, *g, reinterpret_cast<const gs355_header*>(ws + L.header),
                                   reinterpret_cast<const uint32_t*>(ws + L.ranges),
+                                  tile_order(reinterpret_cast<const uint32_t*>(ws + L.tile_lists), fa.grid_x * fa.grid_y),
                                   reinterpret_cast<const uint32_t*>(ws + L.values[L.sorted_buffer]),
                                   reinterpret_cast<const float*>(ws + L.records),
                                   reinterpret_cast<const uint64_t*>(ws + L.rects),

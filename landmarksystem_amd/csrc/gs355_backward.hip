@@ -166,7 +166,7 @@ __device__ __forceinline__ float add_halves(float a, float b)
 // kDepth: a gradient arrives for the depth plane.
 template <bool kDepth>
 __global__ __launch_bounds__(256) void blend_backward_kernel(
-    FrameArgs f, const gs355_header* __restrict__ header, const uint32_t* __restrict__ ranges,
+    FrameArgs f, const gs355_header* __restrict__ header, const uint32_t* __restrict__ ranges, const uint4* __restrict__ order,
     const uint32_t* __restrict__ values, const float* __restrict__ records, const float* __restrict__ image,
     const float* __restrict__ out_depth, const float* __restrict__ out_alpha, const float* __restrict__ g_image,
     const float* __restrict__ g_depth, const float* __restrict__ g_alpha, const RecordSlots* __restrict__ slots,
@@ -188,7 +188,8 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     __shared__ __align__(4) uint8_t s_list[4][4][kBatch + 8];
 
     if (header->overflow) return;
-    const int tile = blockIdx.x;
+    const BlendTile list(header, ranges, order);
+    const int tile = (int)list.tile;
     const int tile_x = tile % f.grid_x, tile_y = tile / f.grid_x;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int row = lane >> 4, group = (lane >> 2) & 3, sub = lane & 3;
@@ -221,7 +222,7 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     // staging: thread 4 k + part brings part `part` of the batch's Gaussian k (part 3: the slot of its record), and later
     // writes a third of its record
     const int staged = tid >> 2, part = tid & 3;
-    const uint32_t lo = ranges[2 * tile], hi = ranges[2 * tile + 1];
+    const uint32_t lo = list.lo, hi = list.hi;
     float T = inside ? 1.0f : -1.0f, prefix = 0.0f;
     if (tid < 3)
         (tid == 0 ? s_a : tid == 1 ? s_b : s_c)[kBatch] = make_float4(0.f, tid == 1 ? -__builtin_inff() : 0.f, 0.f, 0.f);
@@ -1077,7 +1078,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
 }  // namespace
 
 int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const gs355_header* header,
-                           const uint32_t* ranges, const uint32_t* values, const float* records,
+                           const uint32_t* ranges, const uint4* order, const uint32_t* values, const float* records,
                            const uint64_t* rects, const uint8_t* lit, const gs355_backward_inputs& in, uint2* record_slots, uint32_t* next_slot,
                            float* key_grads, const gs355_gradients& out, const ParameterArgs* par, hipStream_t s)
 {
@@ -1090,7 +1091,7 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
     GS355_CHECK_LAUNCH("record slots");
     const int tiles = f.grid_x * f.grid_y;
     auto blend = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(tiles), dim3(256), 0, s, f, header, ranges, values, records, in.image, in.depth,
+        hipLaunchKernelGGL(kernel, dim3(tiles), dim3(256), 0, s, f, header, ranges, order, values, records, in.image, in.depth,
                            in.alpha, in.dL_dimage, in.dL_ddepth, in.dL_dalpha, slots, key_grads);
     };
     if (in.dL_ddepth)

@@ -164,6 +164,7 @@ constexpr int kListWords = kBatch + 8;  // entries per list: a batch, padded to 
 template <bool kCull>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) void blend_kernel(FrameArgs f, const gs355_header* __restrict__ header,
                                                     const uint32_t* __restrict__ ranges,
+                                                    const uint4* __restrict__ order,
                                                     const uint32_t* __restrict__ values,
                                                     const float* __restrict__ records, float* __restrict__ image,
                                                     float* __restrict__ out_depth, float* __restrict__ out_alpha)
@@ -177,7 +178,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
     __shared__ __align__(8) ListEntry s_list[kCull ? 4 : 1][4][kListWords];
 
     if (header->overflow) return;
-    const int tile = blockIdx.x;
+    const BlendTile list(header, ranges, order);
+    const int tile = (int)list.tile;
     const int tile_x = tile % f.grid_x, tile_y = tile / f.grid_x;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int group = lane >> 4, sub = lane & 15;  // 4x4 block within the quadrant, pixel within the block
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
     const float pxf = (float)px, pyf = (float)py;
     const int first_bit = 8 * (wave >> 1) + 2 * (wave & 1);  // the quadrant's first block in a record's block mask
 
-    const uint32_t lo = ranges[2 * tile], hi = ranges[2 * tile + 1];
+    const uint32_t lo = list.lo, hi = list.hi;
     PixelState p = {inside ? 1.0f : 0.0f, inside ? 0.0001f : -1.0f, 1.0f, {0.f, 0.f, 0.f, 0.f}};
     if (tid == 0) {  // the null record: zero conic and log2(opacity) = -inf give alpha = 0
         s_a[kBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -388,15 +390,15 @@ int launch_ranges(const gs355_header* header, uint32_t n_cap, const uint64_t* ke
     return GS355_OK;
 }
 
-int launch_blend(const FrameArgs& f, const gs355_header* header, const uint32_t* ranges, const uint32_t* values,
+int launch_blend(const FrameArgs& f, const gs355_header* header, const uint32_t* ranges, const uint4* order, const uint32_t* values,
                  const float* records, float* image, float* depth, float* alpha, bool cull, hipStream_t s)
 {
     const int tiles = f.grid_x * f.grid_y;
     if (cull)
-        hipLaunchKernelGGL(blend_kernel<true>, dim3(tiles), dim3(256), 0, s, f, header, ranges, values, records, image,
+        hipLaunchKernelGGL(blend_kernel<true>, dim3(tiles), dim3(256), 0, s, f, header, ranges, order, values, records, image,
                            depth, alpha);
     else
-        hipLaunchKernelGGL(blend_kernel<false>, dim3(tiles), dim3(256), 0, s, f, header, ranges, values, records, image,
+        hipLaunchKernelGGL(blend_kernel<false>, dim3(tiles), dim3(256), 0, s, f, header, ranges, order, values, records, image,
                            depth, alpha);
     GS355_CHECK_LAUNCH("blend");
     return GS355_OK;

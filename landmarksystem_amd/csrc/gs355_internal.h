@@ -294,11 +294,12 @@ int launch_sort(const gs355_header* header, uint32_t n_cap, int passes, uint64_t
                 uint32_t* vals0, uint32_t* vals1, uint32_t* hist, uint32_t* scan_tmp, hipStream_t s);
 int launch_ranges(const gs355_header* header, uint32_t n_cap, const uint64_t* keys, uint32_t* ranges, int tiles,
                   hipStream_t s);
-int launch_blend(const FrameArgs& f, const gs355_header* header, const uint32_t* ranges, const uint32_t* values, const float* records,
-                 float* image, float* depth, float* alpha, bool cull, hipStream_t s);
+// `order`: the tiles in the tile sort's order where header->ordered says so
+int launch_blend(const FrameArgs& f, const gs355_header* header, const uint32_t* ranges, const uint4* order, const uint32_t* values,
+                 const float* records, float* image, float* depth, float* alpha, bool cull, hipStream_t s);
 
 int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const gs355_header* header,
-                           const uint32_t* ranges, const uint32_t* values, const float* records,
+                           const uint32_t* ranges, const uint4* order, const uint32_t* values, const float* records,
                            const uint64_t* rects, const uint8_t* lit, const gs355_backward_inputs& in, uint2* record_slots, uint32_t* next_slot,
                            float* key_grads, const gs355_gradients& out, const ParameterArgs* par, hipStream_t s);
 
@@ -417,9 +418,28 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
                         gs355_header* header, const uint32_t* matrix, uint32_t n_cap,
                         uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, uint64_t* buckets, uint64_t* coarse,
                         int levels, const ScatterLayout* make, hipStream_t s);
-// lists: u32[kListHeader + 4 * tiles]: the four class counts, four spare words, the four lists
+// lists: u32[kListHeader + 8 * tiles]: the four class counts, four spare words, the four lists, then {u32 tile, first, last, 0}
+// [tiles], the tiles by the length of their lists
 constexpr int kListHeader = 8;
-int launch_tile_sort(const gs355_header* header, int tiles, const uint32_t* ranges, uint32_t* lists,
+inline uint4* tile_order(uint32_t* lists, int tiles) { return reinterpret_cast<uint4*>(lists + kListHeader + 4 * (size_t)tiles); }
+inline const uint4* tile_order(const uint32_t* lists, int tiles) { return tile_order(const_cast<uint32_t*>(lists), tiles); }
+// The tile of a blend's workgroup and its list.
+struct BlendTile {
+    uint32_t tile, lo, hi;
+    __device__ __forceinline__ BlendTile(const gs355_header* __restrict__ header, const uint32_t* __restrict__ ranges,
+                                         const uint4* __restrict__ order)
+    {
+        // (all three requested together: one latency)
+        const uint32_t b = blockIdx.x;
+        const uint4 o = order[b];
+        const uint2 r = reinterpret_cast<const uint2*>(ranges)[b];
+        const bool ordered = header->ordered != 0u;
+        tile = ordered ? o.x : b;
+        lo = ordered ? o.y : r.x;
+        hi = ordered ? o.z : r.y;
+    }
+};
+int launch_tile_sort(gs355_header* header, int tiles, const uint32_t* ranges, uint32_t* lists,
                      uint64_t* buckets, uint64_t* out_keys, uint32_t* out_vals, bool keys_too, uint32_t skip_classes, hipStream_t s);
 
 // anchor decode: argument checks, and the exclusive prefix of per-run (kept offsets, visible anchors) with the totals

@@ -161,6 +161,7 @@ __global__ __launch_bounds__(256) void scan_sums_kernel(uint64_t* __restrict__ s
             header->num_visible = s_vis[0] + s_vis[1] + s_vis[2] + s_vis[3];
             header->sort_class_count[0] = header->sort_class_count[1] = header->sort_class_count[2] = 0xFFFFFFFFu;
             header->parts = 0u;  // (whole rectangles from here on)
+            header->ordered = 0u;
             if (header_copy) {
                 header_copy->num_keys_total = total;
                 header_copy->num_keys = total > n_cap ? n_cap : (uint32_t)total;

@@ -90,3 +90,45 @@ def test_layout_made_by_the_scatter(gpu_device, width, height, P, log_scale, lev
         assert want["header"][3] == (n_cap < total) and want.keys() == got.keys()
         for name in want:
             np.testing.assert_array_equal(got[name], want[name], err_msg=name)
+
+
+@pytest.mark.parametrize("width,height,P,log_scale", [
+    (256, 256, 900, -1.0), (16 * 257, 16, 3000, -3.0), (512, 256, 2000, -2.0), (513, 256, 2000, -2.0), (1000, 700, 9000, -2.5),
+    (16 * 360, 1600, 30_000, -5.0), (16 * 361, 1600, 30_000, -5.0)])
+def test_tiles_in_the_order_of_their_lists(gpu_device, width, height, P, log_scale):
+    """The tile sort's order of the tiles: each of them once, with its range, no later than a list of more than 1/16 less; made
+    for 257 to 36000 tiles; the same image with and without it; and forgotten when a new frame's header is written."""
+    scene = scenes.tiny_scene(P=P, width=width, height=height, sh_degree=0, seed=5, log_scale_mean=log_scale)
+    inp = pipeline.FrameInputs(settings_for(scene, gpu_device), scene.means3D.to(gpu_device), shs=scene.shs.to(gpu_device),
+                               opacities=scene.opacities.to(gpu_device), scales=scene.scales.to(gpu_device),
+                               rotations=scene.rotations.to(gpu_device))
+    out, ws, tiles, n_cap = pipeline.FrameOutputs(inp), pipeline.Workspace(gpu_device), inp.tiles, 1 << 24
+    lay = ws.ensure(P, n_cap, width, height)
+    ws.buffer.fill_(0xA5)
+    run = lambda mask: pipeline.run_stages(inp, out, ws, n_cap, mask)  # noqa: E731
+    word = lambda: ws.buffer[lay.header + 40:lay.header + 44].view(torch.int32)  # noqa: E731
+    run(_lib.STAGE_PREPROCESS)
+    run(_lib.STAGE_TILE_COUNT | _lib.STAGE_TILE_SCATTER)
+    assert int(word()) == 0
+    run(_lib.STAGE_TILESORT | _lib.STAGE_BLEND)
+    made = 257 <= tiles <= 36000
+    assert int(word()) == made
+    image = out.image.clone()
+    if made:
+        at = lay.tile_lists + 4 * (8 + 4 * tiles)
+        order = ws.buffer[at:at + 16 * tiles].view(torch.int32).view(tiles, 4).cpu().numpy()
+        ranges = ws.view(lay, "ranges", P, 0, tiles).cpu().numpy()
+        assert (np.sort(order[:, 0]) == np.arange(tiles)).all()
+        np.testing.assert_array_equal(order[:, 1:3], ranges[order[:, 0]])
+        n = (order[:, 2] - order[:, 1]).astype(np.int64)
+        assert n.max() > 0 and (np.minimum.accumulate(n) * 17 >= n * 16).all()
+        word().zero_()
+        out.image.zero_()
+        run(_lib.STAGE_BLEND)
+        assert torch.equal(out.image, image)
+        word().fill_(1)
+    run(_lib.STAGE_TILE_COUNT)
+    assert int(word()) == 0
+    word().fill_(1)
+    run(_lib.STAGE_SCAN)
+    assert int(word()) == 0
