@@ -6,7 +6,7 @@
 // Blending: one 256-thread workgroup per 16x16 pixel tile, each of its four
 // wavefronts owning an 8x8 pixel quadrant, each group of 16 lanes a 4x4 block
 // of it.  The tile's depth-sorted Gaussians are staged through LDS in batches
-// of 256 records (48 B each, rescaled while staging so that the per-pixel
+// of 252 records (48 B each, rescaled while staging so that the per-pixel
 // arithmetic needs no constant multiplies); every 4x4 block gets its own list
 // of the staged Gaussians that can reach it, and the four lane groups of a
 // wavefront walk their lists side by side, four entries per round, so one
@@ -145,9 +145,13 @@ __device__ __forceinline__ void blend_one(PixelState& p, float pxf, float pyf, c
 }
 
 using ListEntry = uint16_t;
-constexpr int kBatch = 256;            // records staged per round
+// Records staged per round: so many that eight workgroups fit into a CU's LDS, with at most 64 registers eight wavefronts per
+// SIMD in the place of seven (256, and room behind the lists for one round more).  Blend of 1M large splats at 1080p 133.5 ->
+// 129.5 us, of 6M 288 -> 283, octree frame 47.8 -> 45.3; with the next batch's indices requested a batch ahead (a latency less
+// per batch: 10k Gaussians, a wavefront per SIMD, 16.1 -> 15.6) and the lists padded by their own lane groups side by side.
+constexpr int kBatch = 252;
 constexpr uint32_t kNullEntry = kBatch * 16;  // list entry of the null record (opacity 0: rejected by every pixel)
-constexpr int kListWords = kBatch + 8;  // entries per list: a batch, padded to a multiple of four, one round read ahead
+constexpr int kListWords = kBatch + 4;  // entries per list: a batch, padded to a multiple of four, one round read ahead
 
 // kCull: staging a record also finds which of the tile's sixteen 4x4 blocks its
 // alpha >= 1/255 ellipse can reach (TileReach), and each wavefront appends the
@@ -162,7 +166,7 @@ constexpr int kListWords = kBatch + 8;  // entries per list: a batch, padded to 
 // of four, so the walk needs no per-entry length test and reads four entries at
 // a time.
 template <bool kCull>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) void blend_kernel(FrameArgs f, const gs355_header* __restrict__ header,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void blend_kernel(FrameArgs f, const gs355_header* __restrict__ header,
                                                     const uint32_t* __restrict__ ranges,
                                                     const uint4* __restrict__ order,
                                                     const uint32_t* __restrict__ values,
@@ -270,13 +274,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
         }
     };
 
+    // this thread's Gaussian of the batch, requested one batch ahead
+    uint32_t index = lo + tid < hi ? values[lo + tid] : 0u;
     for (uint32_t base = lo; base < hi; base += kBatch) {
         const uint64_t live = __ballot(p.T > 0.0f);  // lanes whose pixel is still accumulating
         const bool wave_done = live == 0ull;
         bool finite = true, is_definite = true;
         const uint32_t j = base + tid;
-        if (j < hi) {
-            const uint32_t g = values[j];
+        if (tid < kBatch && j < hi) {
+            const uint32_t g = index;
+            if (j + kBatch < hi) index = values[j + kBatch];
             const float4* __restrict__ rec = reinterpret_cast<const float4*>(records + (size_t)g * kRecordFloats);
             const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
             // a negative opacity gives a negative alpha, which every pixel rejects: log2(0) = -inf does the same
@@ -294,8 +301,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
             s_c[tid] = make_float4(r1.z, r1.w, r2.x, r2.y);
             // (the sum of the magnitudes overflows only where one of them is beyond 2^125: then the careful way is right too)
             finite = fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < __builtin_inff();
-        } else if (kCull) {
-            s_b[tid].z = 0.0f;  // (no record: reaches no block)
         }
         const bool all_finite = __ballot(!finite) == 0ull, all_definite = __ballot(!is_definite) == 0ull;
         if (lane == 0) s_wave_state[wave] = (wave_done ? 1u : 0u) | (all_finite ? 0u : 2u) | (all_definite ? 0u : 4u);
@@ -312,7 +317,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
                 // the hardware's masked bit count.
                 for (int chunk = 0; chunk < count; chunk += 64) {
                     const int k = chunk + lane;
-                    const uint32_t reached = __float_as_uint(s_b[k].z) >> first_bit;
+                    const uint32_t reached = k < count ? __float_as_uint(s_b[k].z) >> first_bit : 0u;
 #pragma unroll
                     for (int b = 0; b < 4; ++b) {
                         // a block whose 16 pixels have all finished gets no entries (its lane group idles through
@@ -327,11 +332,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
                 const uint32_t longest = (uint32_t)__builtin_amdgcn_readfirstlane(
                     (int)max(max(len[0], len[1]), max(len[2], len[3])));
                 const uint32_t quads = (longest + 3u) / 4u;
-                // pad every list with the null record up to the common length
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    for (uint32_t at = len[b] + (uint32_t)lane; at < quads * 4u; at += 64u)
-                        s_list[wave][b][at] = (ListEntry)kNullEntry;
+                // every lane group pads its list with the null record up to the common length
+                uint32_t mine = len[0];
+                mine = group == 1 ? len[1] : mine;
+                mine = group == 2 ? len[2] : mine;
+                mine = group == 3 ? len[3] : mine;
+                for (uint32_t at = mine + (uint32_t)sub; at < quads * 4u; at += 16u)
+                    s_list[wave][group][at] = (ListEntry)kNullEntry;
                 // a wavefront's LDS operations execute in order: its list writes precede the reads below
                 wave_lds_sync();
                 if ((unusual & 2) == 0) walk_lists(unusual == 0, quads);

@@ -8,6 +8,7 @@ import torch
 from landmarksystem_amd import _lib, pipeline, scenes
 from oracle import c_oracle as co
 from tests.helpers import check_images, oracle_frame, oracle_gaussians, settings_for
+from tests.test_gpu_parity import crowded_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -178,3 +179,17 @@ def test_thin_needles_do_not_slow_their_batches(gpu_device):
             assert torch.equal(a, b)
     print("blend with needles: %.1f us wide, %.1f us thin" % (1e3 * ms[False], 1e3 * ms[True]))
     assert ms[True] < 1.2 * ms[False]
+
+
+@pytest.mark.parametrize("P", [1, 3, 63, 64, 65, 251, 252, 253, 256, 504, 505, 757])
+def test_lists_at_the_edges_of_a_batch(gpu_device, P):
+    """Every Gaussian in every tile: lists of a batch of 252 records and around it, of one and two of its chunks of 64."""
+    scene = crowded_scene(P, width=48, height=33)
+    ws = pipeline.Workspace(gpu_device)
+    inp, out = _render(scene, gpu_device, ws)
+    culled = [out.image.clone(), out.depth.clone(), out.alpha.clone()]
+    got = dict(image=out.image.cpu().numpy(), depth=out.depth.cpu().numpy(), alpha=out.alpha.cpu().numpy())
+    pipeline.run_stages(inp, out, ws, ws.key_capacity, _lib.STAGE_BLEND_PLAIN)
+    for a, b in zip(culled, (out.image, out.depth, out.alpha)):
+        assert torch.equal(a, b)
+    check_images(got, co.render(oracle_frame(scene), oracle_gaussians(scene)), "lists of %d" % P, max_fragile_frac=0.5)
