@@ -284,9 +284,12 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
             const uint32_t longest = (uint32_t)__builtin_amdgcn_readfirstlane(
                 (int)max(max(len[0], len[1]), max(len[2], len[3])));
             const uint32_t quads = (longest + 3u) / 4u;
-#pragma unroll
-            for (int b = 0; b < 4; ++b)  // padded with the null record to the common length
-                if (len[b] + (uint32_t)lane < quads * 4u) s_list[wave][b][len[b] + (uint32_t)lane] = (uint8_t)kBatch;
+            // every block's lanes pad its list with the null record up to the common length
+            uint32_t own = len[0];
+            own = group == 1 ? len[1] : own;
+            own = group == 2 ? len[2] : own;
+            own = group == 3 ? len[3] : own;
+            for (uint32_t at = own + (uint32_t)(4 * row + sub); at < quads * 4u; at += 16u) s_list[wave][group][at] = (uint8_t)kBatch;
             wave_lds_sync();
             const uint32_t* __restrict__ mine = reinterpret_cast<const uint32_t*>(s_list[wave][group]);
             uint32_t next = mine[0];  // read ahead by one round (rounds past the end are never used)
