@@ -1533,6 +1533,114 @@ struct LdsSorter {
     }
 };
 
+// The counting sort of LdsSorter by one wavefront, for buckets of up to 256 pairs: no barriers, and four times as many buckets
+// side by side.  (A workgroup of four wavefronts per bucket waits at ten barriers however few pairs there are.)  It has no
+// radix passes to fall back to: depths that share a bin rank themselves among all of it, which for 256 equal depths are 64
+// steps.  8160 tiles of 145 pairs: 18.8 -> 13.8 us, 4056 of 93: 10.8 -> 9.4, 2170 of 243: 9.7 -> 8.6; frames of larger buckets
+// unchanged.  For up to 512 pairs (eight per lane): 16.3, 11.1 and 10.0, and 500k anchors' tiles 24.8 -> 29.1.  Sorted by the
+// wavefronts of the workgroups that the larger buckets have, one of four: slower than without (octree frame 206 -> 212).
+struct WaveSorter {
+    static constexpr int kR = 4, kCap = 64 * kR, kB = kCap;  // pairs per lane, pairs, fine bins
+    static constexpr int kCoarse = 64;
+    static constexpr int kWords = 2 * (kCap + 4) + kB + 4 + 2 * kCoarse;
+
+    uint64_t* pairs;  // [kCap + 4]
+    uint32_t* count;  // [kB + 4]
+    uint32_t* coarse;  // [kCoarse]; float2 [kCoarse] over the same words
+
+    __device__ explicit WaveSorter(uint32_t* lds)
+        : pairs(reinterpret_cast<uint64_t*>(lds)), count(lds + 2 * (kCap + 4)), coarse(lds + 2 * (kCap + 4) + kB + 4)
+    {
+    }
+
+    __device__ __forceinline__ void run(uint32_t tile, uint32_t lo, uint32_t n, const uint64_t* __restrict__ buckets, bool keys_too,
+                                        uint64_t* __restrict__ out_keys, uint32_t* __restrict__ out_vals) const
+    {
+        const uint32_t lane = threadIdx.x & 63u;
+        if (n == 0u || n > (uint32_t)kCap) return;  // (uniform)
+        uint64_t v[kR];
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r) v[r] = r * 64u + lane < n ? __builtin_nontemporal_load(&buckets[lo + r * 64u + lane]) : 0ull;  // (read once)
+        reinterpret_cast<uint4*>(count)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        coarse[lane] = 0u;
+        uint32_t dmin = 0xFFFFFFFFu, dmax = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r) {
+            if (r * 64u + lane < n) {
+                dmin = min(dmin, (uint32_t)(v[r] >> 32));
+                dmax = max(dmax, (uint32_t)(v[r] >> 32));
+            }
+        }
+        dmin = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(dmin, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return min(a, b); }), 63);
+        dmax = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(dmax, 0u, [](uint32_t a, uint32_t b) { return max(a, b); }), 63);
+        wave_lds_sync();
+        const float scale = (float)kCoarse / ((float)(dmax - dmin) + 1.0f);
+        float at[kR];
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r) {
+            at[r] = fminf((float)((uint32_t)(v[r] >> 32) - dmin) * scale, (float)kCoarse - 0.00001f);
+            if (r * 64u + lane < n) atomicAdd(&coarse[(uint32_t)at[r]], 1u);
+        }
+        wave_lds_sync();
+        const uint32_t own = coarse[lane], inc = wave_sum_scan(own);
+        wave_lds_sync();
+        float2* const line = reinterpret_cast<float2*>(coarse);
+        line[lane] = make_float2((float)(inc - own), (float)own);
+        wave_lds_sync();
+        uint32_t bin[kR], slot[kR];
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r) {
+            bin[r] = slot[r] = 0;
+            if (r * 64u + lane < n) {
+                const float2 l = line[(uint32_t)at[r]];
+                const float pos = __builtin_fmaf(__builtin_amdgcn_fractf(at[r]), l.y, l.x);  // in [0, n]
+                bin[r] = min((uint32_t)pos, (uint32_t)kB - 1u);
+                slot[r] = atomicAdd(&count[bin[r]], 1u);
+            }
+        }
+        wave_lds_sync();
+        const uint4 mine = reinterpret_cast<const uint4*>(count)[lane];  // (a lane owns four consecutive bins)
+        const uint32_t c = (mine.x + mine.y) + (mine.z + mine.w);
+        const uint32_t first = wave_sum_scan(c) - c, f1 = first + mine.x, f2 = f1 + mine.y;
+        wave_lds_sync();
+        reinterpret_cast<uint4*>(count)[lane] = make_uint4(first, f1, f2, f2 + mine.z);
+        if (lane == 0) count[kB] = n;
+        if (lane < 4) pairs[n + lane] = ~0ull;
+        wave_lds_sync();
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r)
+            if (r * 64u + lane < n) pairs[count[bin[r]] + slot[r]] = v[r];
+        wave_lds_sync();
+        // (as LdsSorter: what follows the bin is larger than all of its members)
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r) {
+            if (r * 64u + lane < n) {
+                const uint32_t begin = count[bin[r]], end = count[bin[r] + 1];
+                uint32_t rank = begin;
+                for (uint32_t q = begin; q < end; q += 4) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) rank += pairs[q + k] < v[r] ? 1u : 0u;
+                }
+                slot[r] = rank;
+            }
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r)
+            if (r * 64u + lane < n) pairs[slot[r]] = v[r];
+        wave_lds_sync();
+#pragma unroll
+        for (uint32_t r = 0; r < kR; ++r) {
+            const uint32_t j = r * 64u + lane;
+            if (j < n) {
+                const uint64_t p = pairs[j];
+                if (keys_too) __builtin_nontemporal_store(((uint64_t)tile << 32) | (p >> 32), &out_keys[lo + j]);
+                out_vals[lo + j] = (uint32_t)p;
+            }
+        }
+    }
+};
+
 // Tiles in the order of their lists' lengths, longest first, as (tile, first, last, 0).  The blends' workgroups nearly all start at
 // once in frames of a few thousand tiles, and the compute unit with the longest lists decides; in larger frames the last ones to
 // start do.  2170 tiles: blend 47.1 -> 44.7 us, 1734: backward blend 100.5 -> 96.1; 8160 tiles, 6M Gaussians: 276.9 -> 272.6 and
@@ -1599,8 +1707,9 @@ __device__ __forceinline__ void order_tiles(const uint32_t* __restrict__ ranges,
 // sorted whatever the caller expected.
 //
 // The first workgroup is none of the tiles': it orders them by the length of their lists for the blends (order_tiles), beside
-// the sorts.
-template <int kT, int kR>
+// the sorts.  kByWave: behind the workgroups with a tile each come some with a wavefront per tile, four consecutive ones, for the
+// buckets of up to 256 pairs, which the others leave.
+template <int kT, int kR, bool kByWave>
 __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header,
                                                             const uint32_t* __restrict__ ranges,
                                                             uint64_t* __restrict__ buckets,
@@ -1617,8 +1726,18 @@ __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header
         return;
     }
     static_assert((256 + kWaves * 256 + 8) * sizeof(uint32_t) <= LdsSorter<kT, kR>::kBytes, "scratch of the global passes");
-    const uint32_t tile = blockIdx.x - (order ? 1u : 0u);
+    const uint32_t block = blockIdx.x - (order ? 1u : 0u);
+    if (kByWave && block >= tiles) {
+        static_assert(!kByWave || WaveSorter::kWords * (kT / 64) * sizeof(uint32_t) <= LdsSorter<kT, kR>::kBytes, "a sorter per wavefront");
+        const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), tile = (block - tiles) * (kT / 64) + wave;
+        if (tile >= tiles) return;
+        const uint2 r = reinterpret_cast<const uint2*>(ranges)[tile];
+        WaveSorter(s_dyn + wave * WaveSorter::kWords).run(tile, r.x, r.y - r.x, buckets, keys_too, out_keys, out_vals);
+        return;
+    }
+    const uint32_t tile = block;
     const uint32_t lo = ranges[2 * tile], n = ranges[2 * tile + 1] - lo;
+    if (kByWave && n <= (uint32_t)WaveSorter::kCap) return;
     bool through_global = n > (uint32_t)kTileSortCap[3];
     if (skip_classes != 0u && n > (uint32_t)LdsSorter<kT, kR>::kCap && !through_global) {
         const int cls = n <= (uint32_t)kTileSortCap[1] ? 0 : n <= (uint32_t)kTileSortCap[2] ? 1 : 2;
@@ -1721,7 +1840,7 @@ static int allow_large_lds()
         (e = raise_lds_limit(scatter_kernel<0, false>, bin_bytes)) != hipSuccess ||
         (e = raise_lds_limit(scatter_kernel<kCoarseShift, true>, bin_bytes)) != hipSuccess ||
         (e = raise_lds_limit(tile_sort_list_1024x5_kernel, LdsSorter<1024, 5>::kBytes)) != hipSuccess ||
-        (e = raise_lds_limit(tile_sort_each_kernel<1024, 5>, LdsSorter<1024, 5>::kBytes)) != hipSuccess ||
+        (e = raise_lds_limit(tile_sort_each_kernel<1024, 5, false>, LdsSorter<1024, 5>::kBytes)) != hipSuccess ||
         (e = raise_lds_limit(tile_sort_list_kernel<1024, 10, true>, LdsSorter<1024, 10>::kBytes)) != hipSuccess)
         return set_error(GS355_EHIP, "LDS limit of the binning / tile sort kernels: %s", hipGetErrorString(e));
     done[dev].store(1, std::memory_order_release);  // racing threads set the same values
@@ -1884,12 +2003,12 @@ int launch_tile_sort(gs355_header* header, int tiles, const uint32_t* ranges, ui
     const uint32_t* list0 = lists + kListHeader;
     const bool one_launch = tiles <= kOneLaunchTiles;
     uint4* order = tiles >= kOrderMinTiles && tiles <= kOrderMaxTiles ? tile_order(lists, tiles) : nullptr;
-    const dim3 grid(tiles + (order ? 1 : 0));
+    const int each = tiles + (order ? 1 : 0);
     if (one_launch)
-        hipLaunchKernelGGL((tile_sort_each_kernel<1024, 5>), grid, dim3(1024), S2::kBytes, s, header, ranges, buckets,
+        hipLaunchKernelGGL((tile_sort_each_kernel<1024, 5, false>), dim3(each), dim3(1024), S2::kBytes, s, header, ranges, buckets,
                            out_keys, out_vals, keys_too, skip_classes, order, (uint32_t)tiles);
     else
-        hipLaunchKernelGGL((tile_sort_each_kernel<256, 4>), grid, dim3(256), S0::kBytes, s, header, ranges, buckets,
+        hipLaunchKernelGGL((tile_sort_each_kernel<256, 4, true>), dim3(each + (tiles + 3) / 4), dim3(256), S0::kBytes, s, header, ranges, buckets,
                            out_keys, out_vals, keys_too, skip_classes, order, (uint32_t)tiles);
     GS355_CHECK_LAUNCH("tile sort: class 0");
     // A launch per larger class, a workgroup per tile: those past the end of the class's list leave at once, which

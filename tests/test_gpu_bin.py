@@ -132,3 +132,17 @@ def test_tiles_in_the_order_of_their_lists(gpu_device, width, height, P, log_sca
     word().fill_(1)
     run(_lib.STAGE_SCAN)
     assert int(word()) == 0
+
+
+@pytest.mark.parametrize("P,duplicates", [(1, 0), (2, 1), (63, 0), (64, 30), (65, 0), (200, 100), (255, 0), (256, 128), (257, 0)])
+@pytest.mark.parametrize("one_depth", [False, True])
+def test_buckets_that_a_wavefront_sorts(gpu_device, P, duplicates, one_depth):
+    """Every Gaussian in each of 625 tiles: buckets of up to 256 pairs, and one more, with equal depths among them or nothing else."""
+    scene = crowded_scene(P, width=400, height=400, duplicates=duplicates)
+    if one_depth:
+        scene.means3D[:] = scene.means3D[0].clone()
+    want = run_all_stages(scene, gpu_device)
+    for modifiers in (0, _lib.STAGE_TILESORT_VALUES):
+        got = run_fast_path(scene, gpu_device, modifiers=modifiers)
+        for name in ("ranges", "sorted_keys", "sorted_values")[::2 if modifiers else 1]:
+            np.testing.assert_array_equal(got[name], want[name], err_msg="%d %s" % (P, name))
