@@ -246,6 +246,11 @@ __device__ __forceinline__ uint64_t tile_region(const Rect q, float px, float py
 // Scenes from which on a wavefront's records leave as whole lines: at half a million the way through LDS costs what it saves
 // (colours given: 500k 14.8 us by lane, 15.0 by line; 1M 25.8 and 23.4; 130k 7.1 and 7.3).
 constexpr int kRecordLinesFrom = 1 << 19;
+// Scenes from which on those lines are streamed: 100 MB of records, of which the L2 keeps little for the blend whatever this kernel
+// does, while what the binning reads next stays.  Preprocess within frames: 6M 299 -> 285 us, 20M at 4K 819 -> 764, stored
+// parameters 311 -> 285, and the count and scatter of 20M 89 + 204 -> 82 + 196; frames of 4.5M Gaussians 2.4 % (a slab), 6.5 (a
+// ball) and 0.7 (a part of a scene) quicker, of 3.3M 1.7, 3.6 and 0.4, of 2M 0.4, 0.2 and -0.1, of 1M 0.5, 0.1 and 0.
+constexpr int kRecordsStreamedFrom = 1 << 21;
 
 // kStored: g holds the vanilla model's stored parameters, activated here (the activated copies would cost a pass over
 // memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
@@ -537,10 +542,16 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         wave_lds_sync();
         float4* __restrict__ dst = reinterpret_cast<float4*>(records + (size_t)(i - lane) * kRecordFloats);
         const int end = 3 * min(64, P - (i - lane));
+        const bool streamed = P >= kRecordsStreamedFrom;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const int at = 64 * k + lane;
-            if (at < end && ((alive_lanes >> ((at & ~3) / 3)) & 3ull) != 0ull) dst[at] = out_rows[at];
+            if (at < end && ((alive_lanes >> ((at & ~3) / 3)) & 3ull) != 0ull) {
+                typedef float f32x4 __attribute__((ext_vector_type(4)));
+                const float4 v = out_rows[at];
+                if (streamed) __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4*>(dst + at));
+                else dst[at] = v;
+            }
         }
     } else if (alive) {
         float4* __restrict__ rec = reinterpret_cast<float4*>(records + (size_t)i * kRecordFloats);

@@ -64,3 +64,19 @@ def test_records_that_leave_by_the_line(gpu_device, degree, spread):
         records.append(rows[keep].clone())
     assert records[0].shape[0] > 10
     assert torch.equal(records[0], records[1]) and torch.equal(records[0], records[2])
+
+
+@pytest.mark.parametrize("degree,spread", [(0, 1.0), (3, 6.0)])
+def test_records_that_are_streamed(gpu_device, degree, spread):
+    """The same Gaussians in a scene of 2^21 and in one of one fewer: the same records."""
+    P = 1 << 21
+    scene = scenes.tiny_scene(P=P, width=150, height=97, sh_degree=degree, spread=spread, seed=degree)
+    records = []
+    for n in (P, P - 1):
+        d = [t[:n].contiguous().to(gpu_device) for t in (scene.means3D, scene.opacities, scene.shs, scene.scales, scene.rotations)]
+        inp = pipeline.FrameInputs(settings_for(scene, gpu_device), d[0], opacities=d[1], shs=d[2], scales=d[3], rotations=d[4])
+        out, ws = pipeline.FrameOutputs(inp), pipeline.Workspace(gpu_device)
+        lay = pipeline.run_stages(inp, out, ws, 1 << 10, _lib.STAGE_PREPROCESS)
+        rows = ws.view(lay, "records", n, 0, inp.tiles).view(torch.int32)
+        records.append(rows[:P - 1][out.radii[:P - 1] > 0].clone())
+    assert records[0].shape[0] > 1000 and torch.equal(records[0], records[1])
