@@ -307,8 +307,10 @@ __device__ __forceinline__ int size_class(uint32_t n)
 constexpr uint32_t chunks_of(uint32_t pairs);
 
 // Fills s_bin with this slice's first slot in each column and publishes the layout; returns the number of pairs, or
-// 0xFFFFFFFF for a frame that overflowed.  `scratch`: 4096 words of LDS, free again behind the next barrier.  `row`: what
-// earlier slices put into each tile.
+// 0xFFFFFFFF for a frame that overflowed.  `scratch`: kLayoutWords words of LDS, free again behind the next barrier.  `row`:
+// what earlier slices put into each tile.
+constexpr int kLayoutWords = 4 * kBinThreads;
+
 template <int kShift>
 __device__ __forceinline__ uint32_t lay_out(const LayoutArgs& a, int T, uint32_t* __restrict__ tile_base,
                                             const uint32_t* __restrict__ row, uint32_t* __restrict__ s_bin,
@@ -322,6 +324,7 @@ __device__ __forceinline__ uint32_t lay_out(const LayoutArgs& a, int T, uint32_t
     uint32_t* const s_class2 = scratch + 2 * kBinThreads;
     uint32_t* const s_waves = scratch + 3 * kBinThreads;  // per wavefront: these three, visible Gaussians, keys
     constexpr int kSums = 6;
+    static_assert(3 * kBinThreads + (kSums + 1) * kWavesHere <= kLayoutWords, "and the chunks' sums");
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int n_blocks = (T + 63) / 64;
     // (the first block's values are under way while the sums are made)
@@ -434,6 +437,7 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
     static_assert(!kWide || kShift > 0, "beyond kBinMaxTiles tiles only coarse bins fit in LDS");
     extern __shared__ uint32_t s_bin[];  // [columns] next free slot of this slice in each column
     __shared__ uint32_t s_queue[kBinItems * kBinThreads];
+    static_assert(kBinItems * kBinThreads >= kLayoutWords, "the layout is made in the queue's memory");
     __shared__ uint32_t s_nqueue;
 
     constexpr int kSpan = 1 << kShift;
