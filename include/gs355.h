@@ -122,7 +122,9 @@ typedef struct gs355_header {
     uint32_t parts;          /* preprocess stage: 1 if `rects` holds parts of tile rectangles (GS355_STAGE_TILE_REACH), else 0
                               * (in the workspace only) */
     uint32_t ordered;        /* tile-sort stage: 1 once it has put the tiles in the order the blends take them (in the workspace only) */
-    uint32_t reserved[5];
+    uint32_t sort_beyond_count; /* tile-count stage, as sort_class_count: buckets of more than 10240 pairs.  They are sorted by the
+                              * launch of the largest class, so GS355_STAGE_TILESORT_SKIP_3 suits frames without any of either */
+    uint32_t reserved[4];
 } gs355_header;
 
 /* Byte offsets of every array inside the caller's workspace (each 256-byte
@@ -191,8 +193,8 @@ enum {
     GS355_STAGE_TILE_SCATTER_TWO_LEVEL = 1024, /* modifier of TILE_SCATTER: through the bins whatever the key count */
     GS355_STAGE_TILE_SCATTER_ONE_LEVEL = 2048, /* modifier of TILE_SCATTER: straight into the buckets (ignored beyond 36000 tiles) */
     /* Modifiers of TILESORT: do not launch the sorter of the 2nd / 3rd / 4th size class (1025..2048, 2049..5120,
-     * 5121..10240 pairs per bucket).  A launch over an empty class costs 4-6 us, and most frames leave one or more
-     * classes empty (header.sort_class_count of the previous frame is a good predictor).  A hint, not a promise:
+     * 5121 and more pairs per bucket).  A launch over an empty class costs 4-6 us, and most frames leave one or more
+     * classes empty (header.sort_class_count and sort_beyond_count of the previous frame are good predictors).  A hint, not a promise:
      * buckets of a skipped class are still sorted, one workgroup each through global memory -- same result, slower. */
     GS355_STAGE_TILESORT_SKIP_1 = 4096,
     GS355_STAGE_TILESORT_SKIP_2 = 8192,

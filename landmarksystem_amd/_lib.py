@@ -87,7 +87,8 @@ class Header(C.Structure):
         ("ready", C.c_uint32),
         ("parts", C.c_uint32),
         ("ordered", C.c_uint32),
-        ("reserved", C.c_uint32 * 5),
+        ("sort_beyond_count", C.c_uint32),
+        ("reserved", C.c_uint32 * 4),
     ]
 
 

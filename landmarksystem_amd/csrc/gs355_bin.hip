@@ -9,8 +9,8 @@
 // their tile's bucket (in one level, or through coarse bins of 16 tiles when
 // the frame holds many pairs).  What remains is an independent sort of each
 // bucket by its low word, done by one workgroup per tile entirely in LDS (up
-// to 10240 pairs in the 160 KB of a CU; larger buckets run radix passes
-// through global memory).  Bucket order after the scatter is arbitrary, so
+// to 10240 pairs in the 160 KB of a CU; larger buckets are split into such
+// pieces first).  Bucket order after the scatter is arbitrary, so
 // pairs are ordered by (depth bits, Gaussian index): exactly the order a
 // stable sort of the emission-ordered keys produces.
 //
@@ -278,9 +278,11 @@ struct LayoutArgs {
     uint32_t* chunk_base;  // pairs per coarse bin, turned into chunks before each bin; NULL: no second level follows
 };
 
-// The frame's header from sums over all blocks and slices (one thread).  `in_class`: buckets per larger size class, or NULL.
+// The frame's header from sums over all blocks and slices (one thread).  `in_class`: buckets on the lists of the larger size
+// classes, or NULL; `beyond`: those of the last that are larger than the LDS.
 __device__ __forceinline__ void write_header(gs355_header* header, gs355_header* header_copy, uint64_t keys, uint32_t total,
-                                             bool overflow, uint32_t n_cap, uint32_t visible, const uint32_t* in_class)
+                                             bool overflow, uint32_t n_cap, uint32_t visible, const uint32_t* in_class,
+                                             uint32_t beyond)
 {
     for (int k = 0; k < (header_copy ? 2 : 1); ++k) {
         gs355_header* const h = k ? header_copy : header;
@@ -288,18 +290,17 @@ __device__ __forceinline__ void write_header(gs355_header* header, gs355_header*
         h->num_keys = overflow ? n_cap : total;
         h->overflow = overflow ? 1u : 0u;
         h->num_visible = visible;
-        for (int c = 0; c < 3; ++c) h->sort_class_count[c] = in_class ? in_class[c] : 0xFFFFFFFFu;
+        for (int c = 0; c < 3; ++c) h->sort_class_count[c] = in_class ? in_class[c] - (c == 2 ? beyond : 0u) : 0xFFFFFFFFu;
+        h->sort_beyond_count = in_class ? beyond : 0xFFFFFFFFu;
         h->ordered = 0u;  // (until the tile sort has made the order)
     }
     if (header_copy) mark_ready(header_copy);
 }
 
-// A bucket's larger size class, or -1 (too small for the lists, or beyond the LDS sorters: sorted by its own workgroup of
-// the class-0 kernel).
+// A bucket's larger size class, or -1 (too small for the lists).
 __device__ __forceinline__ int size_class(uint32_t n)
 {
-    if (n > (uint32_t)kTileSortCap[3]) return -1;
-    if (n > (uint32_t)kTileSortCap[2]) return 2;
+    if (n > (uint32_t)kTileSortCap[2]) return 2;  // (and what is larger than the LDS)
     if (n > (uint32_t)kTileSortCap[1]) return 1;
     return n > (uint32_t)kTileSortCap[0] ? 0 : -1;
 }
@@ -334,7 +335,8 @@ __device__ __forceinline__ uint32_t lay_out(const LayoutArgs& a, int T, uint32_t
     const uint32_t word = tid < n_blocks ? a.block_classes[tid] : 0u;
     SliceTotals slice = {0ull, 0u, 0u};
     if (tid < (int)gridDim.x) slice = a.slice_totals[tid];
-    const uint32_t two = (word & 0xFFu) | ((word & 0xFF00u) << 8), third = (word >> 16) & 0xFFu;
+    // (16 bits each: classes 0 and 1; class 2 and those of it beyond the LDS)
+    const uint32_t two = (word & 0xFFu) | ((word & 0xFF00u) << 8), third = ((word >> 16) & 0xFFu) | ((word >> 24) << 16);
     const uint32_t pairs_inc = wave_sum_scan(pairs), two_inc = wave_sum_scan(two), third_inc = wave_sum_scan(third);
     // (keys below 2^50, as two sums: 24 bits and the rest)
     const uint32_t sums[kSums] = {pairs_inc, two_inc, third_inc, wave_sum_scan(slice.visible),
@@ -356,12 +358,12 @@ __device__ __forceinline__ uint32_t lay_out(const LayoutArgs& a, int T, uint32_t
     if (tid < n_blocks) {
         s_block[tid] = before[0] + pairs_inc - pairs;
         s_classes[tid] = before[1] + two_inc - two;
-        s_class2[tid] = before[2] + third_inc - third;
+        s_class2[tid] = (before[2] + third_inc - third) & 0xFFFFu;
     }
     const bool overflow = keys > (uint64_t)a.n_cap;
     if (blockIdx.x == 0 && tid == 0) {
-        const uint32_t in_class[3] = {all[1] & 0xFFFFu, all[1] >> 16, all[2]};
-        write_header(a.header, a.header_copy, keys, all[0], overflow, a.n_cap, all[3], in_class);
+        const uint32_t in_class[3] = {all[1] & 0xFFFFu, all[1] >> 16, all[2] & 0xFFFFu};
+        write_header(a.header, a.header_copy, keys, all[0], overflow, a.n_cap, all[3], in_class, all[2] >> 16);
         for (int c = 0; c < 3; ++c) a.lists[c] = in_class[c];
     }
     if (overflow) return 0xFFFFFFFFu;  // later stages do nothing either
@@ -818,8 +820,9 @@ __global__ __launch_bounds__(64 * kPrefixParts) void slice_prefix_kernel(uint32_
             const uint32_t v = live ? total : 0u;
             const uint32_t n1 = (uint32_t)__popcll(__ballot(v > (uint32_t)kTileSortCap[0] && v <= (uint32_t)kTileSortCap[1]));
             const uint32_t n2 = (uint32_t)__popcll(__ballot(v > (uint32_t)kTileSortCap[1] && v <= (uint32_t)kTileSortCap[2]));
-            const uint32_t n3 = (uint32_t)__popcll(__ballot(v > (uint32_t)kTileSortCap[2] && v <= (uint32_t)kTileSortCap[3]));
-            if (lane == 0) block_classes[blockIdx.x] = n1 | (n2 << 8) | (n3 << 16);
+            const uint32_t n3 = (uint32_t)__popcll(__ballot(v > (uint32_t)kTileSortCap[2]));
+            const uint32_t beyond = (uint32_t)__popcll(__ballot(v > (uint32_t)kTileSortCap[3]));  // (of them)
+            if (lane == 0) block_classes[blockIdx.x] = n1 | (n2 << 8) | (n3 << 16) | (beyond << 24);
         }
         if (bin_sums) {  // columns are tiles: the pairs of each coarse bin (kCoarseTiles consecutive tiles)
             uint32_t bin = live ? total : 0u;
@@ -857,12 +860,13 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
     __shared__ uint64_t s_before[4], s_total[4], s_class_before[4], s_class_total[4], s_keys[4];
     __shared__ uint32_t s_vis[4], s_chunks[4];
     if (header_known && header->overflow) return;
-    // counts of the three classes, 21 bits each
+    // counts of the three classes and of what is beyond the LDS, 16 bits each
+    static_assert(kBinMaxTiles < (1 << 16), "(columns that are tiles)");
     auto classes_of = [&](uint32_t b) {
         const uint32_t w = block_classes[b];
-        return (uint64_t)(w & 0xFFu) | ((uint64_t)((w >> 8) & 0xFFu) << 21) | ((uint64_t)((w >> 16) & 0xFFu) << 42);
+        return (uint64_t)((w & 0xFFu) | ((w & 0xFF00u) << 8)) | ((uint64_t)(((w >> 16) & 0xFFu) | ((w >> 24) << 16)) << 32);
     };
-    auto class_count = [](uint64_t packed, int c) { return (uint32_t)(packed >> (21 * c)) & 0x1FFFFFu; };
+    auto class_count = [](uint64_t packed, int c) { return (uint32_t)(packed >> (16 * c)) & 0xFFFFu; };
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t first_block = blockIdx.x * 4u, block = first_block + (uint32_t)wave;
     {
@@ -890,8 +894,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         total = wave_sum(total);
         vis = wave_sum(vis);
         keys = wave_sum(keys);
-        // (three counts of 21 bits: two of them, and the third)
-        auto sum_classes = [](uint64_t v) { return ((uint64_t)wave_sum((uint32_t)(v >> 42)) << 42) + wave_sum((uint64_t)(v & ((1ull << 42) - 1ull))); };
+        auto sum_classes = [](uint64_t v) { return ((uint64_t)wave_sum((uint32_t)(v >> 32)) << 32) | wave_sum((uint32_t)v); };
         class_before = sum_classes(class_before);
         class_total = sum_classes(class_total);
         if (lane == 0) {
@@ -911,7 +914,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
         const uint64_t packed = (s_class_total[0] + s_class_total[1]) + (s_class_total[2] + s_class_total[3]);
         const uint32_t in_class[3] = {class_count(packed, 0), class_count(packed, 1), class_count(packed, 2)};
         write_header(header, header_copy, keys, (uint32_t)total, overflow, n_cap, (s_vis[0] + s_vis[1]) + (s_vis[2] + s_vis[3]),
-                     block_classes ? in_class : nullptr);
+                     block_classes ? in_class : nullptr, class_count(packed, 3));
         if (block_classes && kTiles)
             for (int c = 0; c < 3; ++c) lists[c] = in_class[c];
     }
@@ -977,10 +980,7 @@ __global__ __launch_bounds__(256) void tile_publish_kernel(const uint32_t* total
     }
 }
 
-constexpr int kThreads = 256;
-constexpr int kWaves = 4;
-constexpr int kRounds = 4;                      // 64-key rounds per wave per chunk
-constexpr int kChunk = kWaves * kRounds * 64;  // 1024 pairs ranked per iteration
+constexpr int kRounds = 4;  // 64-key rounds per wavefront and step of a radix pass
 
 // ---------------------------------------------------------------------------
 // Storage of a bucket during sorting: two words per pair.
@@ -1015,21 +1015,23 @@ struct GlobalPairs {
 
 struct SortScratch {
     uint32_t* hist;           // [256] digit totals, then running digit bases
-    uint32_t (*cnt)[256];     // [kWaves][256] per-wave digit counts of the current chunk
+    uint32_t (*cnt)[256];     // [kT / 64][256] per-wave digit counts of the current chunk
     uint32_t* flags;          // [8] small flags / partial sums
 };
 
 // One stable 8-bit LSD pass over n pairs, digit taken from the depth word
 // (by_depth) or the index word.  Returns false (and moves nothing) when every
 // pair has the same digit.
-template <typename Src, typename Dst>
+template <int kT, typename Src, typename Dst>
 __device__ __forceinline__ bool radix_pass(const Src src, const Dst dst, uint32_t n, int shift, bool by_depth, const SortScratch sc)
 {
+    constexpr int kWaves = kT / 64, kChunk = kWaves * kRounds * 64;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    sc.hist[tid] = 0;
+    const bool digit = kT == 256 || tid < 256;  // (uniform per wavefront) a thread per digit
+    if (digit) sc.hist[tid] = 0;
     if (tid < 8) sc.flags[tid] = 0;
     __syncthreads();
-    for (uint32_t j = tid; j < n; j += kThreads) {
+    for (uint32_t j = tid; j < n; j += kT) {
         uint32_t kd, ki;
         src.load(j, kd, ki);
         atomicAdd(&sc.hist[((by_depth ? kd : ki) >> shift) & 255u], 1u);
@@ -1037,19 +1039,21 @@ __device__ __forceinline__ bool radix_pass(const Src src, const Dst dst, uint32_
     __syncthreads();
     {
         // exclusive scan of the 256 digit totals; detect the single-digit case
-        const uint32_t h = sc.hist[tid];
+        const uint32_t h = digit ? sc.hist[tid] : 0u;
         uint32_t inc = h;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const uint32_t up = __shfl_up(inc, d, 64);
             if (lane >= d) inc += up;
         }
-        if (lane == 63) sc.flags[wave] = inc;
+        if (digit && lane == 63) sc.flags[wave] = inc;
         if (h == n) sc.flags[4] = 1;
         __syncthreads();
-        uint32_t off = 0;
-        for (int w = 0; w < wave; ++w) off += sc.flags[w];
-        sc.hist[tid] = off + inc - h;
+        if (digit) {
+            uint32_t off = 0;
+            for (int w = 0; w < wave; ++w) off += sc.flags[w];
+            sc.hist[tid] = off + inc - h;
+        }
         const bool single = sc.flags[4] != 0;
         __syncthreads();
         if (single) return false;
@@ -1057,7 +1061,7 @@ __device__ __forceinline__ bool radix_pass(const Src src, const Dst dst, uint32_
     const uint64_t lanes_below = (1ull << lane) - 1ull;
     for (uint32_t c0 = 0; c0 < n; c0 += kChunk) {
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) sc.cnt[w][tid] = 0;
+        for (int w = 0; w < kWaves; w += kT / 256) (&sc.cnt[w][0])[tid] = 0;
         __syncthreads();
         uint32_t kd[kRounds], ki[kRounds], rank[kRounds];
 #pragma unroll
@@ -1085,7 +1089,7 @@ __device__ __forceinline__ bool radix_pass(const Src src, const Dst dst, uint32_
             rank[r] = pre + below;
         }
         __syncthreads();
-        {
+        if (digit) {
             uint32_t run = sc.hist[tid];
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
@@ -1111,14 +1115,14 @@ __device__ __forceinline__ bool radix_pass(const Src src, const Dst dst, uint32_
 
 // Sort n pairs held in buffer A (B is scratch of the same size) by
 // (depth bits, index).  Returns true if the result is in B.
-template <typename Buf>
+template <int kT, typename Buf>
 __device__ __forceinline__ bool sort_pairs(const Buf A, const Buf B, uint32_t n, const SortScratch sc)
 {
     bool in_b = false;
     // depth passes; pairs of one tile rarely share depth bits, so the index
     // word is only brought in when a tie is actually present
     for (int pass = 0; pass < 4; ++pass) {
-        const bool moved = in_b ? radix_pass(B, A, n, pass * 8, true, sc) : radix_pass(A, B, n, pass * 8, true, sc);
+        const bool moved = in_b ? radix_pass<kT>(B, A, n, pass * 8, true, sc) : radix_pass<kT>(A, B, n, pass * 8, true, sc);
         if (moved) in_b = !in_b;
     }
     {
@@ -1126,7 +1130,7 @@ __device__ __forceinline__ bool sort_pairs(const Buf A, const Buf B, uint32_t n,
         if (threadIdx.x == 0) sc.flags[5] = 0;
         __syncthreads();
         bool tie = false;
-        for (uint32_t j = threadIdx.x; j + 1 < n; j += kThreads) {
+        for (uint32_t j = threadIdx.x; j + 1 < n; j += kT) {
             uint32_t d0, i0, d1, i1;
             cur.load(j, d0, i0);
             cur.load(j + 1, d1, i1);
@@ -1142,17 +1146,17 @@ __device__ __forceinline__ bool sort_pairs(const Buf A, const Buf B, uint32_t n,
     for (int pass = 0; pass < 8; ++pass) {
         const bool by_depth = pass >= 4;
         const int shift = (pass & 3) * 8;
-        const bool moved = in_b ? radix_pass(B, A, n, shift, by_depth, sc) : radix_pass(A, B, n, shift, by_depth, sc);
+        const bool moved = in_b ? radix_pass<kT>(B, A, n, shift, by_depth, sc) : radix_pass<kT>(A, B, n, shift, by_depth, sc);
         if (moved) in_b = !in_b;
     }
     return in_b;
 }
 
-template <typename Buf>
+template <int kT, typename Buf>
 __device__ __forceinline__ void write_sorted(const Buf cur, uint32_t n, uint32_t tile, bool keys_too, uint64_t* out_keys,
                                              uint32_t* out_vals)
 {
-    for (uint32_t j = threadIdx.x; j < n; j += kThreads) {
+    for (uint32_t j = threadIdx.x; j < n; j += kT) {
         uint32_t kd, ki;
         cur.load(j, kd, ki);
         if (keys_too) out_keys[j] = ((uint64_t)tile << 32) | (uint64_t)kd;
@@ -1703,12 +1707,10 @@ __device__ __forceinline__ void order_tiles(const uint32_t* __restrict__ ranges,
     each([&](uint32_t t, uint2 r) { order[atomicAdd(&bins[bin_of(r.y - r.x)], 1u)] = make_uint4(t, r.x, r.y, 0u); });
 }
 
-// Smallest size class: one workgroup per tile; tiles with larger buckets leave at once, except those beyond the
-// capacity of the largest LDS sorter, which are sorted here by radix passes through global memory, ping-ponging
-// between the bucket and the tile's slice of the output keys (their scratch lies over the LDS sorter's area).
-// `skip_classes` (bit c: the sorter of larger class c is not launched for this frame, the caller expecting no bucket
-// of that size): such a bucket, should there be one after all, takes the global-memory route too, so every bucket is
-// sorted whatever the caller expected.
+// Smallest size class: one workgroup per tile; tiles with larger buckets leave at once.  `skip_classes` (bit c: the sorter of
+// larger class c is not launched for this frame, the caller expecting no bucket of that size): such a bucket, should there be
+// one after all, is sorted here by radix passes through global memory, ping-ponging between the bucket and the tile's slice
+// of the output keys (their scratch lies over the LDS sorter's area), so every bucket is sorted whatever the caller expected.
 //
 // The first workgroup is none of the tiles': it orders them by the length of their lists for the blends (order_tiles), beside
 // the sorts.  kByWave: behind the workgroups with a tile each come some with a wavefront per tile, four consecutive ones, for the
@@ -1729,7 +1731,8 @@ __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header
         if (threadIdx.x == 0) header->ordered = 1u;
         return;
     }
-    static_assert((256 + kWaves * 256 + 8) * sizeof(uint32_t) <= LdsSorter<kT, kR>::kBytes, "scratch of the global passes");
+    constexpr int kThreads = 256;  // of a bucket that goes through global memory
+    static_assert((256 + kThreads / 64 * 256 + 8) * sizeof(uint32_t) <= LdsSorter<kT, kR>::kBytes, "scratch of the global passes");
     const uint32_t block = blockIdx.x - (order ? 1u : 0u);
     if (kByWave && block >= tiles) {
         static_assert(!kByWave || WaveSorter::kWords * (kT / 64) * sizeof(uint32_t) <= LdsSorter<kT, kR>::kBytes, "a sorter per wavefront");
@@ -1742,18 +1745,18 @@ __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header
     const uint32_t tile = block;
     const uint32_t lo = ranges[2 * tile], n = ranges[2 * tile + 1] - lo;
     if (kByWave && n <= (uint32_t)WaveSorter::kCap) return;
-    bool through_global = n > (uint32_t)kTileSortCap[3];
-    if (skip_classes != 0u && n > (uint32_t)LdsSorter<kT, kR>::kCap && !through_global) {
+    bool through_global = false;
+    if (skip_classes != 0u && n > (uint32_t)LdsSorter<kT, kR>::kCap) {
         const int cls = n <= (uint32_t)kTileSortCap[1] ? 0 : n <= (uint32_t)kTileSortCap[2] ? 1 : 2;
         through_global = (skip_classes >> cls) & 1u;
     }
     if (through_global) {  // (uniform over the workgroup; passes of kThreads threads)
         if (threadIdx.x >= kThreads) return;
-        const SortScratch sc = {s_dyn, reinterpret_cast<uint32_t(*)[256]>(s_dyn + 256), s_dyn + 256 + kWaves * 256};
+        const SortScratch sc = {s_dyn, reinterpret_cast<uint32_t(*)[256]>(s_dyn + 256), s_dyn + 256 + kThreads / 64 * 256};
         const GlobalPairs A = {buckets + lo}, B = {out_keys + lo};
-        const bool in_b = sort_pairs(A, B, n, sc);
+        const bool in_b = sort_pairs<kThreads>(A, B, n, sc);
         // when the result sits in the output slice itself, each element is rewritten in place by the thread that read it
-        write_sorted(in_b ? B : A, n, tile, keys_too, out_keys + lo, out_vals + lo);
+        write_sorted<kThreads>(in_b ? B : A, n, tile, keys_too, out_keys + lo, out_vals + lo);
         return;
     }
     const LdsSorter<kT, kR> sorter(s_dyn);
@@ -1765,9 +1768,8 @@ __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header
 // once: the hardware's own dispatch hands out the buckets.  (Persistent workgroups that fetched their work from a
 // counter spent 8-14 us per bucket on dependent requests -- counter, list entry, range, pairs -- whatever the
 // bucket held, requesting the next bucket inside the current sort did not hide them, and even a plain strided loop
-// around the sort costs a sixth of the kernel's time in registers kept alive across it.)  kStrided: a launch
-// smaller than the list, for the class whose workgroups fill a CU each.
-template <int kT, int kR, bool kStrided>
+// around the sort costs a sixth of the kernel's time in registers kept alive across it.)
+template <int kT, int kR>
 __device__ __forceinline__ void tile_sort_list_body(const gs355_header* __restrict__ header,
                                                     const uint32_t* __restrict__ ranges,
                                                     const uint32_t* __restrict__ list,
@@ -1778,12 +1780,7 @@ __device__ __forceinline__ void tile_sort_list_body(const gs355_header* __restri
 {
     if (header->overflow) return;
     const LdsSorter<kT, kR> sorter(lds);
-    const uint32_t count = *list_count;
-    if (kStrided) {
-        for (uint32_t k = blockIdx.x; k < count; k += gridDim.x) sorter.run(list[k], ranges, buckets, keys_too, out_keys, out_vals);
-    } else if (blockIdx.x < count) {
-        sorter.run(list[blockIdx.x], ranges, buckets, keys_too, out_keys, out_vals);
-    }
+    if (blockIdx.x < *list_count) sorter.run(list[blockIdx.x], ranges, buckets, keys_too, out_keys, out_vals);
 }
 
 // 1024 threads x 5 rounds, held to 64 VGPRs so that two workgroups share a CU
@@ -1793,20 +1790,155 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     uint32_t* __restrict__ out_vals)
 {
     extern __shared__ uint32_t s_dyn[];
-    tile_sort_list_body<1024, 5, false>(header, ranges, list, list_count, buckets, keys_too, out_keys, out_vals, s_dyn);
+    tile_sort_list_body<1024, 5>(header, ranges, list, list_count, buckets, keys_too, out_keys, out_vals, s_dyn);
 }
 
-template <int kT, int kR, bool kStrided>
-__global__ __launch_bounds__(kT) void tile_sort_list_kernel(const gs355_header* __restrict__ header,
-                                                            const uint32_t* __restrict__ ranges,
-                                                            const uint32_t* __restrict__ list,
-                                                            const uint32_t* __restrict__ list_count,
-                                                            const uint64_t* __restrict__ buckets, bool keys_too,
-                                                            uint64_t* __restrict__ out_keys,
-                                                            uint32_t* __restrict__ out_vals)
+__global__ __launch_bounds__(512) void tile_sort_list_512x4_kernel(
+    const gs355_header* __restrict__ header, const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ list,
+    const uint32_t* __restrict__ list_count, const uint64_t* __restrict__ buckets, bool keys_too, uint64_t* __restrict__ out_keys,
+    uint32_t* __restrict__ out_vals)
 {
     extern __shared__ uint32_t s_dyn[];
-    tile_sort_list_body<kT, kR, kStrided>(header, ranges, list, list_count, buckets, keys_too, out_keys, out_vals, s_dyn);
+    tile_sort_list_body<512, 4>(header, ranges, list, list_count, buckets, keys_too, out_keys, out_vals, s_dyn);
+}
+
+// The largest class, 5121 pairs and more: a workgroup of it fills a CU, so the launch is the chip's size and strides over the
+// list.  A bucket beyond the LDS sorter's capacity is written to the tile's slice of the output keys first, ordered by kBins
+// bins of its depth range (one count, one move: the bins' cursors are in LDS), and is then sorted piece by piece, a piece being
+// as many whole bins as the LDS sorter holds.  A single bin of more pairs than that (equal depths, or nearly) goes through
+// global memory by radix passes, between the output keys and the bucket.  Three reads of the pairs and a write, where radix
+// passes by 256 threads took eight reads, four writes and a step of four barriers per 1024 pairs of each.  6M Gaussians at 979x546
+// (tiles of up to 12k pairs among 2170): 383 -> 103 us with the smallest class's kernel, which sorted them; at 400x300 (475 tiles
+// of 14k): 2158 -> 299.
+struct LargeSorter {
+    using Piece = LdsSorter<1024, 10>;
+    static constexpr int kT = 1024, kBins = 4096, kWaves = kT / 64, kAhead = 4;
+    static constexpr size_t kBytes = Piece::kBytes + kBins * sizeof(uint32_t);
+    static_assert(kBins == 4 * kT && kBins == 64 * 64, "four bins a thread; a lane for each 64 of them");
+    static_assert(Piece::kBytes % 16 == 0 && kBytes <= 160 * 1024, "in the CU's LDS");
+    static_assert((256 + kWaves * 256 + 8) * sizeof(uint32_t) <= Piece::kBytes, "scratch of the global passes");
+
+    uint32_t* lds;
+    uint32_t* first;  // [kBins] pairs in the bins before each
+
+    __device__ explicit LargeSorter(uint32_t* s) : lds(s), first(s + Piece::kBytes / sizeof(uint32_t)) {}
+
+    // calls f(pair) for this thread's pairs of the n at `from`, kAhead of them requested together
+    template <typename F>
+    static __device__ __forceinline__ void each(const uint64_t* from, uint32_t n, F f)
+    {
+        for (uint32_t j0 = threadIdx.x; j0 < n; j0 += kAhead * kT) {
+            uint64_t v[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) v[u] = from[min(j0 + (uint32_t)u * kT, n - 1u)];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u)
+                if (j0 + (uint32_t)u * kT < n) f(v[u]);
+        }
+    }
+
+    // Moves the n pairs of `from` to `to`, ordered by bin, and fills `first`; begins and ends with a barrier.
+    __device__ __forceinline__ void split(const uint64_t* from, uint64_t* to, uint32_t n) const
+    {
+        uint32_t* const cursor = lds;  // [kBins]
+        uint32_t* const sums = lds + kBins;  // [2 * kWaves]
+        const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+        uint32_t dmin = 0xFFFFFFFFu, dmax = 0;
+        each(from, n, [&](uint64_t v) {
+            dmin = min(dmin, (uint32_t)(v >> 32));
+            dmax = max(dmax, (uint32_t)(v >> 32));
+        });
+        dmin = wave_scan(dmin, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return min(a, b); });
+        dmax = wave_scan(dmax, 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
+        __syncthreads();
+        reinterpret_cast<uint4*>(cursor)[tid] = make_uint4(0u, 0u, 0u, 0u);
+        if (lane == 63) {
+            sums[wave] = dmin;
+            sums[kWaves + wave] = dmax;
+        }
+        __syncthreads();
+        dmin = 0xFFFFFFFFu;
+        dmax = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            dmin = min(dmin, sums[w]);
+            dmax = max(dmax, sums[kWaves + w]);
+        }
+        // (conversion and multiplication round monotonically)
+        const float scale = (float)kBins / ((float)(dmax - dmin) + 1.0f);
+        auto bin_of = [&](uint64_t v) { return min((uint32_t)((float)((uint32_t)(v >> 32) - dmin) * scale), (uint32_t)kBins - 1u); };
+        each(from, n, [&](uint64_t v) { atomicAdd(&cursor[bin_of(v)], 1u); });
+        __syncthreads();
+        const uint4 mine = reinterpret_cast<const uint4*>(cursor)[tid];
+        const uint32_t c = (mine.x + mine.y) + (mine.z + mine.w), inc = wave_sum_scan(c);
+        if (lane == 63) sums[wave] = inc;
+        __syncthreads();
+        uint32_t f0 = inc - c;
+        for (int w = 0; w < wave; ++w) f0 += sums[w];
+        const uint32_t f1 = f0 + mine.x, f2 = f1 + mine.y;
+        const uint4 firsts = make_uint4(f0, f1, f2, f2 + mine.z);
+        reinterpret_cast<uint4*>(cursor)[tid] = firsts;
+        reinterpret_cast<uint4*>(first)[tid] = firsts;
+        __syncthreads();
+        each(from, n, [&](uint64_t v) { to[atomicAdd(&cursor[bin_of(v)], 1u)] = v; });
+        __syncthreads();
+    }
+
+    // Where the piece that starts at `pos` (a bin's first pair, pos < n) ends: behind as many bins as the LDS sorter holds,
+    // at least one.
+    __device__ __forceinline__ uint32_t piece_end(uint32_t pos, uint32_t n) const
+    {
+        const uint32_t limit = pos + (uint32_t)Piece::kCap;
+        if (n <= limit) return n;
+        const int lane = threadIdx.x & 63;
+        // the last bin that starts at or before the limit: its 64 bins first (the bins' first pairs do not decrease, the first is 0)
+        const int row = __popcll(__ballot(first[lane * 64] <= limit)) - 1;
+        const uint32_t v = first[row * 64 + lane];
+        const int col = __popcll(__ballot(v <= limit)) - 1;
+        const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)v, col);
+        if (end > pos) return end;
+        const int next = row * 64 + col + 1;  // (the bin itself is larger)
+        return next < kBins ? first[next] : n;
+    }
+
+    __device__ __forceinline__ void run(uint32_t tile, const uint32_t* ranges, uint64_t* buckets, bool keys_too, uint64_t* out_keys,
+                                        uint32_t* out_vals) const
+    {
+        const Piece sorter(lds);
+        const uint32_t lo = ranges[2 * tile], n = ranges[2 * tile + 1] - lo;
+        const bool whole = n <= (uint32_t)Piece::kCap;
+        if (!whole) split(buckets + lo, out_keys + lo, n);
+        const uint64_t* const from = whole ? buckets : out_keys;
+        for (uint32_t pos = 0, end; pos < n; pos = end) {  // (uniform, for all its barriers)
+            end = (uint32_t)__builtin_amdgcn_readfirstlane((int)(whole ? n : piece_end(pos, n)));
+            if (end - pos <= (uint32_t)Piece::kCap) {
+                Piece::Fetched f;
+                f.tile = tile;
+                f.lo = lo + pos;
+                f.n = end - pos;
+                sorter.fetch_pairs(f, from);
+                sorter.sort_fetched(f, keys_too, out_keys, out_vals);
+            } else {
+                const SortScratch sc = {lds, reinterpret_cast<uint32_t(*)[256]>(lds + 256), lds + 256 + kWaves * 256};
+                const GlobalPairs A = {out_keys + lo + pos}, B = {buckets + lo + pos};
+                const bool in_b = sort_pairs<kT>(A, B, end - pos, sc);
+                // (what is rewritten in place is rewritten by the thread that read it)
+                write_sorted<kT>(in_b ? B : A, end - pos, tile, keys_too, out_keys + lo + pos, out_vals + lo + pos);
+                __syncthreads();
+            }
+        }
+    }
+};
+
+__global__ __launch_bounds__(LargeSorter::kT) void tile_sort_large_kernel(const gs355_header* header, const uint32_t* ranges,
+                                                                          const uint32_t* list, const uint32_t* list_count,
+                                                                          uint64_t* buckets, bool keys_too, uint64_t* out_keys,
+                                                                          uint32_t* out_vals)
+{
+    extern __shared__ uint32_t s_dyn[];
+    if (header->overflow) return;
+    const uint32_t count = *list_count;
+    for (uint32_t k = blockIdx.x; k < count; k += gridDim.x) LargeSorter(s_dyn).run(list[k], ranges, buckets, keys_too, out_keys, out_vals);
 }
 
 }  // namespace
@@ -1845,7 +1977,7 @@ static int allow_large_lds()
         (e = raise_lds_limit(scatter_kernel<kCoarseShift, true>, bin_bytes)) != hipSuccess ||
         (e = raise_lds_limit(tile_sort_list_1024x5_kernel, LdsSorter<1024, 5>::kBytes)) != hipSuccess ||
         (e = raise_lds_limit(tile_sort_each_kernel<1024, 5, false>, LdsSorter<1024, 5>::kBytes)) != hipSuccess ||
-        (e = raise_lds_limit(tile_sort_list_kernel<1024, 10, true>, LdsSorter<1024, 10>::kBytes)) != hipSuccess)
+        (e = raise_lds_limit(tile_sort_large_kernel, LargeSorter::kBytes)) != hipSuccess)
         return set_error(GS355_EHIP, "LDS limit of the binning / tile sort kernels: %s", hipGetErrorString(e));
     done[dev].store(1, std::memory_order_release);  // racing threads set the same values
     return GS355_OK;
@@ -1999,7 +2131,7 @@ int launch_tile_sort(gs355_header* header, int tiles, const uint32_t* ranges, ui
     using S0 = LdsSorter<256, 4>;    // <= 1024 pairs, one workgroup per tile
     using S1 = LdsSorter<512, 4>;    // <= 2048
     using S2 = LdsSorter<1024, 5>;   // <= 5120
-    using S3 = LdsSorter<1024, 10>;  // <= 10240
+    using S3 = LargeSorter::Piece;   // <= 10240, and larger ones in pieces
     static_assert(S0::kCap == kTileSortCap[0] && S1::kCap == kTileSortCap[1] && S2::kCap == kTileSortCap[2] &&
                       S3::kCap == kTileSortCap[3], "size classes out of step with the layout kernel");
     int rc;
@@ -2020,7 +2152,7 @@ int launch_tile_sort(gs355_header* header, int tiles, const uint32_t* ranges, ui
     // largest class is the exception: a workgroup of it fills a CU, so its launch is the chip's size and strides.
     // (skip_classes: bit c set = the caller expects list c to be empty; the kernel above has sorted what is on it)
     if (!(skip_classes & 1u) && !one_launch) {
-        hipLaunchKernelGGL((tile_sort_list_kernel<512, 4, false>), dim3(tiles), dim3(512), S1::kBytes, s, header, ranges,
+        hipLaunchKernelGGL(tile_sort_list_512x4_kernel, dim3(tiles), dim3(512), S1::kBytes, s, header, ranges,
                            list0, lists + 0, buckets, keys_too, out_keys, out_vals);
         GS355_CHECK_LAUNCH("tile sort: class 1");
     }
@@ -2030,7 +2162,7 @@ int launch_tile_sort(gs355_header* header, int tiles, const uint32_t* ranges, ui
         GS355_CHECK_LAUNCH("tile sort: class 2");
     }
     if (!(skip_classes & 4u)) {
-        hipLaunchKernelGGL((tile_sort_list_kernel<1024, 10, true>), dim3(tiles < 256 ? tiles : 256), dim3(1024), S3::kBytes,
+        hipLaunchKernelGGL(tile_sort_large_kernel, dim3(tiles < 256 ? tiles : 256), dim3(LargeSorter::kT), LargeSorter::kBytes,
                            s, header, ranges, list0 + 2 * (size_t)tiles, lists + 2, buckets, keys_too, out_keys, out_vals);
         GS355_CHECK_LAUNCH("tile sort: class 3");
     }

@@ -160,6 +160,7 @@ __global__ __launch_bounds__(256) void scan_sums_kernel(uint64_t* __restrict__ s
             header->overflow = total > n_cap ? 1u : 0u;
             header->num_visible = s_vis[0] + s_vis[1] + s_vis[2] + s_vis[3];
             header->sort_class_count[0] = header->sort_class_count[1] = header->sort_class_count[2] = 0xFFFFFFFFu;
+            header->sort_beyond_count = 0xFFFFFFFFu;
             header->parts = 0u;  // (whole rectangles from here on)
             header->ordered = 0u;
             if (header_copy) {
@@ -169,6 +170,7 @@ __global__ __launch_bounds__(256) void scan_sums_kernel(uint64_t* __restrict__ s
                 header_copy->num_visible = s_vis[0] + s_vis[1] + s_vis[2] + s_vis[3];
                 header_copy->sort_class_count[0] = header_copy->sort_class_count[1] = header_copy->sort_class_count[2] =
                     0xFFFFFFFFu;
+                header_copy->sort_beyond_count = 0xFFFFFFFFu;
                 mark_ready(header_copy);
             }
         }

@@ -379,7 +379,8 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
         ws.last_num_pairs = header.num_keys
         out.num_visible = header.num_visible
         ws.frames += 1
-        counts = tuple(header.sort_class_count)
+        counts = list(header.sort_class_count)
+        counts[2] += header.sort_beyond_count  # (sorted by the same launch)
         ws.sort_class_idle = [0 if n else i + 1 for n, i in zip(counts, ws.sort_class_idle)]  # (0xFFFFFFFF: not counted)
         wrong = [c for c in skipped if counts[c] != 0]
         if wrong and not overflow:

@@ -146,3 +146,31 @@ def test_buckets_that_a_wavefront_sorts(gpu_device, P, duplicates, one_depth):
         got = run_fast_path(scene, gpu_device, modifiers=modifiers)
         for name in ("ranges", "sorted_keys", "sorted_values")[::2 if modifiers else 1]:
             np.testing.assert_array_equal(got[name], want[name], err_msg="%d %s" % (P, name))
+
+
+@pytest.mark.parametrize("P,equal", [(10240, 0), (10241, 0), (10241, 10241), (20500, 3000), (24000, 12000), (31000, 31000)])
+@pytest.mark.parametrize("side", [32, 400])
+def test_buckets_beyond_the_lds(gpu_device, P, equal, side):
+    """Every Gaussian in each of 4 or 625 tiles: one piece, several, equal depths among them, and more of those in one bin than
+    the LDS sorter holds (alone, and between other bins)."""
+    scene = crowded_scene(P, width=side, height=side)
+    if equal:
+        scene.means3D[::P // equal][:equal] = scene.means3D[0].clone()
+    want = run_all_stages(scene, gpu_device)
+    assert (want["ranges"][:, 1] - want["ranges"][:, 0]).max() == P
+    for modifiers in (0, _lib.STAGE_TILESORT_VALUES):
+        got = run_fast_path(scene, gpu_device, modifiers=modifiers)
+        for name in ("ranges", "sorted_keys", "sorted_values")[::2 if modifiers else 1]:
+            np.testing.assert_array_equal(got[name], want[name], err_msg="%d %s" % (P, name))
+    # their launch is not left out where the frames before held only such buckets
+    scene.opacities[:] = 0.05
+    inputs = pipeline.FrameInputs(settings_for(scene, gpu_device), scene.means3D.to(gpu_device),
+                                  opacities=scene.opacities.to(gpu_device), shs=scene.shs.to(gpu_device),
+                                  scales=scene.scales.to(gpu_device), rotations=scene.rotations.to(gpu_device))
+    ws = pipeline.Workspace(gpu_device)
+    for _ in range(6):
+        pipeline.render(inputs, ws=ws)
+    header = ws.header
+    assert P < 12_000 or side > 32 or header.sort_beyond_count > 0
+    assert (ws.sort_class_idle[2] == 0) == (header.sort_class_count[2] + header.sort_beyond_count > 0)
+    assert ws.sort_mispredictions == 0
