@@ -253,10 +253,9 @@ __global__ __launch_bounds__(kBinThreads) void tile_count_kernel(FrameArgs f, in
 // tile_base[16 b] plus the sum of the slice prefixes of the bin's tiles.  A
 // coarse pair carries the tile's position within its bin in the low four bits
 // of the index word.  The two launches of the second level cost some 40 us
-// whatever the frame holds, so frames below kTwoLevelMinKeys pairs scatter in
-// one level; the key count is only known on the device, so both variants are
-// launched and each returns at once when the other one applies.
-constexpr uint32_t kTwoLevelMinKeys = 6u << 20;
+// whatever the frame holds, so frames of few pairs (two_level_from) scatter
+// in one level; the key count is only known on the device, so both variants
+// are launched and each returns at once when the other one applies.
 
 // Layout of the buckets inside the scatter (frames whose scatter follows the slice prefix in one call; tile_publish_kernel
 // does the same in a launch of its own).  Every workgroup needs all tile bases anyway, and has them from the tiles' totals
@@ -2067,7 +2066,7 @@ int launch_tile_layout(int32_t P, uint32_t* matrix, const SliceTotals* slice_tot
 int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint32_t* depth_bits,
                         gs355_header* header, const uint32_t* matrix, uint32_t n_cap,
                         uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, uint64_t* buckets, uint64_t* coarse,
-                        int levels, const ScatterLayout* make, hipStream_t s)
+                        int levels, uint32_t two_from, const ScatterLayout* make, hipStream_t s)
 {
     int per_group;
     const int groups = bin_groups(P, &per_group);
@@ -2084,7 +2083,7 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
             layout = {tile_totals(tile_base, T), block_totals(tile_base, T), class_counts(tile_base, T), make->slice_totals, n_cap,
                       header, make->header_copy, ranges, lists, levels != 1 ? chunk_bases(tile_base, T) : nullptr};
         if (levels != 2) {
-            min_keys = levels == 1 ? UINT32_MAX : kTwoLevelMinKeys;
+            min_keys = levels == 1 ? UINT32_MAX : two_from;
             hipLaunchKernelGGL((scatter_kernel<0, false>), dim3(groups), dim3(kBinThreads), (size_t)T * sizeof(uint32_t), s,
                                f, P, per_group, rects, records, depth_bits, header, 0u, min_keys, matrix, tile_base, buckets, layout);
             GS355_CHECK_LAUNCH("bin: scatter");

@@ -411,13 +411,18 @@ struct ScatterLayout {
     const SliceTotals* slice_totals;
     gs355_header* header_copy;
 };
+// Pairs from which a frame scatters in two levels.  Whole frames, two levels against one: given scenes, in random order, 1.04 of
+// the time at 1.0M pairs, 1.02 at 1.7M, 1.00 at 2.8M, 0.99 at 3.2M, 0.96 at 5.9M, 0.94 at 9.8M.  Decoded Gaussians follow their
+// anchors, runs of neighbours whose pairs the L2 merges by itself: 1.05 at 1.7M, 1.03 at 7.0M, 1.02 at 9.4M (more not measured).
+// Gaussians with colours of their own may have been either.
+inline uint32_t two_level_from(bool decoded, bool own_colours) { return (decoded ? 12u : own_colours ? 6u : 3u) << 20; }
 // `coarse`: a second buffer of the buckets' size (first level of the two-level scatter).  `levels`: 1 or 2 = that
-// scatter whatever the frame holds, 0 = chosen on the device by the key count (both variants are launched); images
+// scatter whatever the frame holds, 0 = chosen on the device by the key count against `two_from` (both variants are launched); images
 // beyond kBinMaxTiles tiles always take two levels.  `make`: NULL, or the layout is made on the way (up to kBinMaxTiles tiles)
 int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, const float* records, const uint32_t* depth_bits,
                         gs355_header* header, const uint32_t* matrix, uint32_t n_cap,
                         uint32_t* tile_base, uint32_t* ranges, uint32_t* lists, uint64_t* buckets, uint64_t* coarse,
-                        int levels, const ScatterLayout* make, hipStream_t s);
+                        int levels, uint32_t two_from, const ScatterLayout* make, hipStream_t s);
 // lists: u32[kListHeader + 8 * tiles]: the four class counts, four spare words, the four lists, then {u32 tile, first, last, 0}
 // [tiles], the tiles by the length of their lists
 constexpr int kListHeader = 8;

@@ -174,3 +174,24 @@ def test_buckets_beyond_the_lds(gpu_device, P, equal, side):
     assert P < 12_000 or side > 32 or header.sort_beyond_count > 0
     assert (ws.sort_class_idle[2] == 0) == (header.sort_class_count[2] + header.sort_beyond_count > 0)
     assert ws.sort_mispredictions == 0
+
+
+@pytest.mark.parametrize("form", ["shs", "colours", "count"])
+def test_frames_between_the_scatters_thresholds(gpu_device, form):
+    """3 to 6 Mi pairs: the first frame of a workspace scatters in one level, the second as its pairs and the Gaussians' form say."""
+    scene = crowded_scene(8500, width=400, height=400)
+    scene.opacities[:] = 0.05
+    scene.scales[:] = scene.scales.clamp(min=1.5)
+    at = lambda x: x.to(gpu_device)
+    colour = dict(shs=at(scene.shs)) if form == "shs" else dict(colors_precomp=at(scene.shs[:, 0].contiguous()).abs())
+    if form == "count":
+        colour["count"] = torch.tensor([scene.P], dtype=torch.int32, device=gpu_device)
+    inputs = pipeline.FrameInputs(settings_for(scene, gpu_device), at(scene.means3D), opacities=at(scene.opacities),
+                                  scales=at(scene.scales), rotations=at(scene.rotations), **colour)
+    ws = pipeline.Workspace(gpu_device)
+    first = pipeline.render(inputs, ws=ws)
+    assert 3 << 20 < ws.last_num_pairs < 6 << 20, ws.last_num_pairs
+    for _ in range(2):
+        again = pipeline.render(inputs, ws=ws)
+        for name in ("image", "depth", "alpha"):
+            assert torch.equal(getattr(again, name), getattr(first, name)), name
