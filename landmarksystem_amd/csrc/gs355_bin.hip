@@ -1803,15 +1803,19 @@ __global__ __launch_bounds__(512) void tile_sort_list_512x4_kernel(
 
 // The largest class, 5121 pairs and more: a workgroup of it fills a CU, so the launch is the chip's size and strides over the
 // list.  A bucket beyond the LDS sorter's capacity is written to the tile's slice of the output keys first, ordered by kBins
-// bins of its depth range (one count, one move: the bins' cursors are in LDS), and is then sorted piece by piece, a piece being
-// as many whole bins as the LDS sorter holds.  A single bin of more pairs than that (equal depths, or nearly) goes through
-// global memory by radix passes, between the output keys and the bucket.  Three reads of the pairs and a write, where radix
-// passes by 256 threads took eight reads, four writes and a step of four barriers per 1024 pairs of each.  6M Gaussians at 979x546
-// (tiles of up to 12k pairs among 2170): 383 -> 103 us with the smallest class's kernel, which sorted them; at 400x300 (475 tiles
-// of 14k): 2158 -> 299.
+// bins of its depths (their range, two counts and a move: the bins' cursors are in LDS), and then goes through LDS piece by
+// piece, as many whole bins as fit, where each pair ranks itself among its bin's.  Buckets with a bin of more than kMaxBin pairs
+// sort the pieces as LDS sorters do, and a single bin that none holds (equal depths, or nearly) goes through global memory by
+// radix passes, between the output keys and the bucket.  Radix passes by 256 threads took eight reads, four writes and a step of
+// four barriers per 1024 pairs of each: 6M Gaussians at 979x546 (tiles of up to 12k pairs among 2170) 383 -> 90 us with the smallest
+// class's kernel, which sorted them; at 400x300 (475 tiles of 14k) 2158 -> 260.  (Bins of equal width and every piece through the LDS
+// sorter: 103 and 299.  Buckets of up to 16k pairs held in LDS and registers throughout: 111 and 288, the registers spill.)
 struct LargeSorter {
     using Piece = LdsSorter<1024, 10>;
     static constexpr int kT = 1024, kBins = 4096, kWaves = kT / 64, kAhead = 4;
+    static constexpr int kLine = 2 * Piece::kCap + 8;  // words before the map's lines (behind a piece's pairs and four more)
+    static constexpr uint32_t kMaxBin = 128;
+    static_assert(kBins + 2 * kWaves <= kLine && (kLine + 512) * sizeof(uint32_t) <= Piece::kBytes && kLine % 2 == 0, "apart");
     static constexpr size_t kBytes = Piece::kBytes + kBins * sizeof(uint32_t);
     static_assert(kBins == 4 * kT && kBins == 64 * 64, "four bins a thread; a lane for each 64 of them");
     static_assert(Piece::kBytes % 16 == 0 && kBytes <= 160 * 1024, "in the CU's LDS");
@@ -1836,11 +1840,28 @@ struct LargeSorter {
         }
     }
 
-    // Moves the n pairs of `from` to `to`, ordered by bin, and fills `first`; begins and ends with a barrier.
-    __device__ __forceinline__ void split(const uint64_t* from, uint64_t* to, uint32_t n) const
+    // The map of depths onto bins, as in LdsSorter::counting_sort: 256 coarse bins give a pair's likely position, which is
+    // scaled to the fine bins.  (Positions below 2^24 are exact where coarse bins meet.)
+    struct Map {
+        const float2* line;  // [256] pairs before each coarse bin and in it
+        uint32_t dmin;
+        float scale, to_bin;
+        __device__ __forceinline__ float at(uint64_t v) const { return fminf((float)((uint32_t)(v >> 32) - dmin) * scale, 255.99998f); }
+        __device__ __forceinline__ uint32_t bin(uint64_t v) const
+        {
+            const float a = at(v);
+            const float2 l = line[(uint32_t)a];
+            return min((uint32_t)(__builtin_fmaf(__builtin_amdgcn_fractf(a), l.y, l.x) * to_bin), (uint32_t)kBins - 1u);
+        }
+    };
+
+    // Moves the n < 2^24 pairs of `from` to `to`, ordered by bin, and fills `first` and the map; returns the pairs of the fullest
+    // bin.  Begins and ends with a barrier.
+    __device__ __forceinline__ uint32_t split(const uint64_t* from, uint64_t* to, uint32_t n, Map& map) const
     {
         uint32_t* const cursor = lds;  // [kBins]
         uint32_t* const sums = lds + kBins;  // [2 * kWaves]
+        uint32_t* const coarse = lds + kLine;  // [256], then the map's lines
         const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
         uint32_t dmin = 0xFFFFFFFFu, dmax = 0;
         each(from, n, [&](uint64_t v) {
@@ -1851,6 +1872,7 @@ struct LargeSorter {
         dmax = wave_scan(dmax, 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
         __syncthreads();
         reinterpret_cast<uint4*>(cursor)[tid] = make_uint4(0u, 0u, 0u, 0u);
+        if (tid < 256) coarse[tid] = 0u;
         if (lane == 63) {
             sums[wave] = dmin;
             sums[kWaves + wave] = dmax;
@@ -1863,23 +1885,78 @@ struct LargeSorter {
             dmin = min(dmin, sums[w]);
             dmax = max(dmax, sums[kWaves + w]);
         }
-        // (conversion and multiplication round monotonically)
-        const float scale = (float)kBins / ((float)(dmax - dmin) + 1.0f);
-        auto bin_of = [&](uint64_t v) { return min((uint32_t)((float)((uint32_t)(v >> 32) - dmin) * scale), (uint32_t)kBins - 1u); };
-        each(from, n, [&](uint64_t v) { atomicAdd(&cursor[bin_of(v)], 1u); });
+        map.line = reinterpret_cast<const float2*>(coarse);
+        map.dmin = dmin;
+        map.scale = 256.0f / ((float)(dmax - dmin) + 1.0f);
+        map.to_bin = (float)kBins / (float)n;
+        each(from, n, [&](uint64_t v) { atomicAdd(&coarse[(uint32_t)map.at(v)], 1u); });
+        __syncthreads();
+        uint32_t own = 0, upto = 0;
+        if (tid < 256) {  // (wavefronts 0..3)
+            own = coarse[tid];
+            upto = wave_sum_scan(own);
+            if (lane == 63) sums[wave] = upto;
+        }
+        __syncthreads();
+        if (tid < 256) {
+            uint32_t before = upto - own;
+            for (int w = 0; w < wave; ++w) before += sums[w];
+            reinterpret_cast<float2*>(coarse)[tid] = make_float2((float)before, (float)own);
+        }
+        __syncthreads();
+        each(from, n, [&](uint64_t v) { atomicAdd(&cursor[map.bin(v)], 1u); });
         __syncthreads();
         const uint4 mine = reinterpret_cast<const uint4*>(cursor)[tid];
         const uint32_t c = (mine.x + mine.y) + (mine.z + mine.w), inc = wave_sum_scan(c);
-        if (lane == 63) sums[wave] = inc;
+        const uint32_t most = wave_scan(max(max(mine.x, mine.y), max(mine.z, mine.w)), 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
+        if (lane == 63) {
+            sums[wave] = inc;
+            sums[kWaves + wave] = most;
+        }
         __syncthreads();
-        uint32_t f0 = inc - c;
+        uint32_t f0 = inc - c, fullest = 0;
         for (int w = 0; w < wave; ++w) f0 += sums[w];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) fullest = max(fullest, sums[kWaves + w]);
         const uint32_t f1 = f0 + mine.x, f2 = f1 + mine.y;
         const uint4 firsts = make_uint4(f0, f1, f2, f2 + mine.z);
         reinterpret_cast<uint4*>(cursor)[tid] = firsts;
         reinterpret_cast<uint4*>(first)[tid] = firsts;
         __syncthreads();
-        each(from, n, [&](uint64_t v) { to[atomicAdd(&cursor[bin_of(v)], 1u)] = v; });
+        each(from, n, [&](uint64_t v) { to[atomicAdd(&cursor[map.bin(v)], 1u)] = v; });
+        __syncthreads();
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)fullest);
+    }
+
+    // Writes out the piece [pos, end) of a bucket of n pairs that lie ordered by bin: a pair ranks itself among its bin's, four at a
+    // time (what follows a bin is larger than all of it).  Ends with a barrier.
+    __device__ __forceinline__ void rank_piece(uint32_t tile, uint32_t lo, uint32_t n, uint32_t pos, uint32_t end, const Map& map, bool keys_too,
+                                               uint64_t* out_keys, uint32_t* out_vals) const
+    {
+        uint64_t* const pairs = reinterpret_cast<uint64_t*>(lds);  // [kCap + 4]
+        const uint32_t count = end - pos;
+        constexpr int kR = Piece::kCap / kT;
+        uint64_t v[kR];
+#pragma unroll
+        for (int r = 0; r < kR; ++r) v[r] = out_keys[lo + pos + min((uint32_t)(r * kT) + threadIdx.x, count - 1u)];
+#pragma unroll
+        for (int r = 0; r < kR; ++r)
+            if ((uint32_t)(r * kT) + threadIdx.x < count) pairs[r * kT + threadIdx.x] = v[r];
+        if (threadIdx.x < 4) pairs[count + threadIdx.x] = ~0ull;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kR; ++r) {
+            if ((uint32_t)(r * kT) + threadIdx.x >= count) continue;
+            const uint32_t bin = map.bin(v[r]), stop = (bin + 1u < (uint32_t)kBins ? first[bin + 1u] : n) - pos;
+            uint32_t rank = first[bin] - pos;
+            for (uint32_t q = rank; q < stop; q += 4) {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) rank += pairs[q + k] < v[r] ? 1u : 0u;
+            }
+            rank += lo + pos;
+            if (keys_too) out_keys[rank] = ((uint64_t)tile << 32) | (v[r] >> 32);
+            out_vals[rank] = (uint32_t)v[r];
+        }
         __syncthreads();
     }
 
@@ -1906,11 +1983,17 @@ struct LargeSorter {
         const Piece sorter(lds);
         const uint32_t lo = ranges[2 * tile], n = ranges[2 * tile + 1] - lo;
         const bool whole = n <= (uint32_t)Piece::kCap;
-        if (!whole) split(buckets + lo, out_keys + lo, n);
+        const bool any_order = n >= (1u << 24);
+        Map map;
+        uint32_t fullest = 0;
+        if (!whole && !any_order) fullest = split(buckets + lo, out_keys + lo, n, map);
+        const bool ranked = !whole && !any_order && fullest <= kMaxBin;
         const uint64_t* const from = whole ? buckets : out_keys;
         for (uint32_t pos = 0, end; pos < n; pos = end) {  // (uniform, for all its barriers)
-            end = (uint32_t)__builtin_amdgcn_readfirstlane((int)(whole ? n : piece_end(pos, n)));
-            if (end - pos <= (uint32_t)Piece::kCap) {
+            end = (uint32_t)__builtin_amdgcn_readfirstlane((int)(whole || any_order ? n : piece_end(pos, n)));
+            if (ranked) {
+                rank_piece(tile, lo, n, pos, end, map, keys_too, out_keys, out_vals);
+            } else if (end - pos <= (uint32_t)Piece::kCap) {
                 Piece::Fetched f;
                 f.tile = tile;
                 f.lo = lo + pos;
@@ -1919,7 +2002,7 @@ struct LargeSorter {
                 sorter.sort_fetched(f, keys_too, out_keys, out_vals);
             } else {
                 const SortScratch sc = {lds, reinterpret_cast<uint32_t(*)[256]>(lds + 256), lds + 256 + kWaves * 256};
-                const GlobalPairs A = {out_keys + lo + pos}, B = {buckets + lo + pos};
+                const GlobalPairs A = {(any_order ? buckets : out_keys) + lo + pos}, B = {(any_order ? out_keys : buckets) + lo + pos};
                 const bool in_b = sort_pairs<kT>(A, B, end - pos, sc);
                 // (what is rewritten in place is rewritten by the thread that read it)
                 write_sorted<kT>(in_b ? B : A, end - pos, tile, keys_too, out_keys + lo + pos, out_vals + lo + pos);

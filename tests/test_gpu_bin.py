@@ -148,7 +148,7 @@ def test_buckets_that_a_wavefront_sorts(gpu_device, P, duplicates, one_depth):
             np.testing.assert_array_equal(got[name], want[name], err_msg="%d %s" % (P, name))
 
 
-@pytest.mark.parametrize("P,equal", [(10240, 0), (10241, 0), (10241, 10241), (20500, 3000), (24000, 12000), (31000, 31000)])
+@pytest.mark.parametrize("P,equal", [(10240, 0), (10241, 0), (10241, 10241), (16384, 100), (16385, 100), (20500, 3000), (31000, 100), (24000, 12000), (31000, 31000)])
 @pytest.mark.parametrize("side", [32, 400])
 def test_buckets_beyond_the_lds(gpu_device, P, equal, side):
     """Every Gaussian in each of 4 or 625 tiles: one piece, several, equal depths among them, and more of those in one bin than
