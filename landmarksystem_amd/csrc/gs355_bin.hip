@@ -1792,13 +1792,17 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     tile_sort_list_body<1024, 5>(header, ranges, list, list_count, buckets, keys_too, out_keys, out_vals, s_dyn);
 }
 
-__global__ __launch_bounds__(512) void tile_sort_list_512x4_kernel(
-    const gs355_header* __restrict__ header, const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ list,
-    const uint32_t* __restrict__ list_count, const uint64_t* __restrict__ buckets, bool keys_too, uint64_t* __restrict__ out_keys,
-    uint32_t* __restrict__ out_vals)
+template <int kT, int kR>
+__global__ __launch_bounds__(kT) void tile_sort_list_kernel(const gs355_header* __restrict__ header,
+                                                            const uint32_t* __restrict__ ranges,
+                                                            const uint32_t* __restrict__ list,
+                                                            const uint32_t* __restrict__ list_count,
+                                                            const uint64_t* __restrict__ buckets, bool keys_too,
+                                                            uint64_t* __restrict__ out_keys,
+                                                            uint32_t* __restrict__ out_vals)
 {
     extern __shared__ uint32_t s_dyn[];
-    tile_sort_list_body<512, 4>(header, ranges, list, list_count, buckets, keys_too, out_keys, out_vals, s_dyn);
+    tile_sort_list_body<kT, kR>(header, ranges, list, list_count, buckets, keys_too, out_keys, out_vals, s_dyn);
 }
 
 // The largest class, 5121 pairs and more: a workgroup of it fills a CU, so the launch is the chip's size and strides over the
@@ -2234,7 +2238,7 @@ int launch_tile_sort(gs355_header* header, int tiles, const uint32_t* ranges, ui
     // largest class is the exception: a workgroup of it fills a CU, so its launch is the chip's size and strides.
     // (skip_classes: bit c set = the caller expects list c to be empty; the kernel above has sorted what is on it)
     if (!(skip_classes & 1u) && !one_launch) {
-        hipLaunchKernelGGL(tile_sort_list_512x4_kernel, dim3(tiles), dim3(512), S1::kBytes, s, header, ranges,
+        hipLaunchKernelGGL((tile_sort_list_kernel<512, 4>), dim3(tiles), dim3(512), S1::kBytes, s, header, ranges,
                            list0, lists + 0, buckets, keys_too, out_keys, out_vals);
         GS355_CHECK_LAUNCH("tile sort: class 1");
     }
