@@ -40,20 +40,20 @@ MFMA_F16_PEAK_TFLOPS = 2500.0
 COUNTER_TRAFFIC = {
     "source": "profiles/bench_c3_6M_1080p_hbm_traffic.txt",
     "workload": "configs[2]",
-    "bytes": {"blend": 1376.4e6, "preprocess": 1693.5e6, "keys_sort_ranges": 572.5e6},
+    "bytes": {"blend": 1466.7e6, "preprocess": 1712.7e6, "keys_sort_ranges": 577.1e6},
     # fp32 flops the blend kernel issues per launch in vector instructions (64 lanes x (2 FMA + MUL + ADD) wavefront
     # instructions; the four channels' accumulation is a matrix instruction and not among them), from
     # profiles/bench_c3_6M_1080p_valu_counters.txt
-    "blend_issued_flops": 6.69e9,
+    "blend_issued_flops": 6.70e9,
     "blend_issued_flops_source": "profiles/bench_c3_6M_1080p_valu_counters.txt",
-    "blend_valu_busy": 1.057,  # (matrix instructions count as issued and run beside the vector ones)
+    "blend_valu_busy": 1.138,  # (matrix instructions count as issued and run beside the vector ones)
 }
 
 # Same for `--config 5`: HBM bytes per launch of the two decode kernels (count + emit)
 COUNTER_TRAFFIC_C5 = {
     "source": "profiles/bench_c5_scaffold_500k_hbm_traffic.txt",
     "workload": "configs[4]",
-    "bytes": {"decode": 244.4e6},
+    "bytes": {"decode": 244.3e6},
 }
 
 
