@@ -574,7 +574,7 @@ __global__ __launch_bounds__(kBinThreads) void scatter_kernel(FrameArgs f, int32
 
 // Second level: the pairs of a coarse bin (contiguous) go to the buckets of the bin's tiles, a chunk of kFineChunk pairs
 // at a time.  Chunks never cross a bin; chunk_base[b] = chunks of the bins before b, chunk_base[bins] = all of them
-// (tile_publish_kernel).  The kFineGrid workgroups take equal, contiguous runs of chunks, so every workgroup has work
+// (made with the layout).  The kFineGrid workgroups take equal, contiguous runs of chunks, so every workgroup has work
 // however the pairs are spread over the bins, and a bin of many pairs is shared by many workgroups.  A chunk is split
 // by tile inside LDS first (wave-level ranking by the four tile bits, a scan over the per-wave counts), the
 // workgroup reserves a run of slots per bucket with one global atomic each, and consecutive lanes then store
@@ -1762,7 +1762,7 @@ __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header
     sorter.run(tile, ranges, buckets, keys_too, out_keys, out_vals);
 }
 
-// Larger size classes: one workgroup per entry of the class list made by tile_publish_kernel.  The number of
+// Larger size classes: one workgroup per entry of the class list made with the layout.  The number of
 // entries is only known on the device, so a launch has a workgroup per tile and those past the list's end leave at
 // once: the hardware's own dispatch hands out the buckets.  (Persistent workgroups that fetched their work from a
 // counter spent 8-14 us per bucket on dependent requests -- counter, list entry, range, pairs -- whatever the
