@@ -444,11 +444,12 @@ GS355_API int gs355_decode_emit(const gs355_decoder *dec, const gs355_anchors *a
                       const gs355_decoded *out, void *stream);
 
 /* The whole decode with nothing read back: count phase (feature bank, opacity head, kept offsets per run of
- * anchors, a one-workgroup scan over the runs) and emit phase.  The outputs have room for `capacity` Gaussians
+ * anchors) and emit phase; the prefix over the runs is the count phase's where that is alone, else the emit phase's.  The outputs have room for `capacity` Gaussians
  * (n_offsets per anchor always suffices); G stays on the device in out->count, where gs355_gaussians.P_device of
  * the rasterizer can read it.  Gaussians beyond `capacity` are not written.  `phases`: both for one call; or the
  * count phase alone (only out->count / out->num_visible are written), then -- after the caller has read G and
- * sized its outputs -- the emit phase with the same decoder, anchors and workspace, untouched in between.  With a
+ * sized its outputs -- the emit phase with the same decoder, anchors and workspace, untouched in between.  The emit
+ * phase may be repeated, also behind a call of both phases whose capacity turned out too small.  With a
  * feature bank the mixed features of the visible anchors go through the workspace.  gs355_decode_count / _emit
  * above do not support the feature bank. */
 enum { GS355_DECODE_COUNT = 1, GS355_DECODE_EMIT = 2, GS355_DECODE_ALL = 3 };

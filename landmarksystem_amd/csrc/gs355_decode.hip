@@ -69,8 +69,8 @@ struct DecodeArgs {
     // here, registers and memory requests are not) places its Gaussians from those instead of per-anchor offsets
     uint2* run_totals;       // [runs] (kept offsets, visible anchors) per run of anchors, or NULL
     uint2* run_tiles;        // [runs] kept offsets of the run before each of its four tiles, 16 bits each (with run_totals)
-    const uint2* run_base;   // [runs] exclusive prefix of run_totals, or NULL
-    int scan_here;           // the emit pass makes that prefix itself (runs <= kScanStripes * its workgroups), and the sums:
+    uint2* run_base;         // [runs] exclusive prefix of run_totals, or NULL
+    int scan_here;           // the emit pass makes that prefix itself (runs <= kScanStripes * its workgroups), for a later one too, and the sums:
     uint32_t* num_emitted;   // of the kept offsets, or NULL
     uint32_t* num_visible;   // of the visible anchors, or NULL
     float* neural_opacity;   // [A_vis * n] tanh of every pre-activation, in visible-anchor order, or NULL
@@ -511,6 +511,7 @@ __global__ __launch_bounds__(64 * kEmitWaves, 3) void decode_emit_kernel(DecodeA
             const uint4 v = my_run < runs ? s_stripe[lane] : make_uint4(0u, 0u, 0u, 0u);
             const uint32_t x = wave_sum_scan(v.x), y = wave_sum_scan(v.y);
             run_base = make_uint2(x - v.x + v.z, y - v.y + v.w);
+            if (wave == 0 && my_run < runs) d.run_base[my_run] = run_base;  // (for an emit phase that is repeated, with more room)
             if (blockIdx.x == 0 && wave == 0 && lane == 63) {
                 if (d.num_emitted) *d.num_emitted = x;
                 if (d.num_visible) *d.num_visible = y;

@@ -1,13 +1,14 @@
 """GPU parity of the MFMA anchor decode (through gs355_decode_count / _emit)
 against the fp32 torch-CPU oracle of AnchorDecoder.forward."""
 import copy
+import ctypes as C
 import pickle
 
 import numpy as np
 import pytest
 import torch
 
-from landmarksystem_amd import scenes
+from landmarksystem_amd import _lib, scenes
 from landmarksystem_amd.anchor_decoder import FusedAnchorDecoder
 from oracle import anchor_oracle as ao
 
@@ -396,3 +397,41 @@ def test_decode_that_scans_its_runs_by_itself(gpu_device, A, frac):
         every = dec.train()(*t, vis)
     for name, a, b in zip(("neural_opacity", "mask"), (res.neural_opacity, res.mask), every[5:]):
         assert torch.equal(a.reshape(-1)[:10 * a_vis], b.reshape(-1)), name
+
+
+@pytest.mark.parametrize("A", [1, 129, 32_769, 70_001])
+def test_emit_again_behind_both_phases(gpu_device, A):
+    """Both phases in one call with too little room, then the emit phase alone with enough over the same workspace: what the count
+    phase and the emit phase by themselves give, the by-products of training included, and nothing outside of them."""
+    sc = scenes.config5(A=A)
+    dec = build_decoder(sc, gpu_device)
+    vis = torch.rand(A, generator=torch.Generator().manual_seed(A)) < 0.6
+    vis[A - 1] = True
+    t = [x.to(gpu_device).contiguous() for x in (sc.camera.camera_center, sc.anchor, sc.anchor_feat, sc.offset, sc.scaling)]
+    _, _, struct, an, keep = dec._marshal(*t, vis.to(gpu_device), None)  # (`keep`: the tensors that `an` points into)
+    widths = dict(xyz=3, color=3, opacity=1, scaling=3, rot=4)
+
+    def run(ws, capacity, phases):
+        guard = 1024  # rows behind the outputs that stay as they are
+        out = {k: torch.full((capacity + guard, w), -7.0, device=gpu_device) for k, w in widths.items()}
+        out["neural_opacity"] = torch.full((10 * A + guard,), -7.0, device=gpu_device)
+        out["mask"] = torch.full((10 * A + guard,), 7, dtype=torch.uint8, device=gpu_device)
+        count = torch.zeros(2, dtype=torch.int32, device=gpu_device)
+        o = _lib.Decoded(**{k: v.data_ptr() for k, v in out.items()}, count=count.data_ptr(), num_visible=count.data_ptr() + 4)
+        _lib.check(_lib.load().gs355_decode(C.byref(struct), C.byref(an), capacity, C.byref(o), ws.data_ptr(), ws.numel(), phases,
+                                            torch.cuda.current_stream().cuda_stream))
+        return out, count.tolist()
+
+    need = C.c_size_t()
+    _lib.check(_lib.load().gs355_decode_workspace_bytes(A, 10, 0, C.byref(need)))
+    spaces = [torch.full((need.value,), 0xA5, dtype=torch.uint8, device=gpu_device) for _ in range(2)]
+    G, a_vis = run(spaces[0], 0, _lib.DECODE_COUNT)[1]
+    assert G > 0 and a_vis == int(vis.sum())
+    want, _ = run(spaces[0], G, _lib.DECODE_EMIT)
+    some, counts = run(spaces[1], G // 2, _lib.DECODE_ALL)
+    assert counts == [G, a_vis]
+    got, _ = run(spaces[1], G, _lib.DECODE_EMIT)
+    for name in want:
+        assert torch.equal(got[name], want[name]), name
+    for name in widths:
+        assert torch.equal(some[name][:G // 2], want[name][:G // 2]) and bool((some[name][G // 2:] == -7.0).all()), name
