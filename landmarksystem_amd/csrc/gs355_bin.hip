@@ -274,7 +274,7 @@ struct LayoutArgs {
     gs355_header* header_copy;
     uint32_t* ranges;
     uint32_t* lists;
-    uint32_t* chunk_base;  // pairs per coarse bin, turned into chunks before each bin; NULL: no second level follows
+    uint32_t* chunk_base;  // pairs per coarse bin, turned into chunks before each bin (for a second level in a later call too)
 };
 
 // The frame's header from sums over all blocks and slices (one thread).  `in_class`: buckets on the lists of the larger size
@@ -330,6 +330,14 @@ __device__ __forceinline__ uint32_t lay_out(const LayoutArgs& a, int T, uint32_t
     // (the first block's values are under way while the sums are made)
     const int t_first = wave * 64 + lane;
     uint32_t next_total = t_first < T ? a.totals[t_first] : 0u, next_before = t_first < T ? row[t_first] : 0u;
+    const int bins = (T + kCoarseTiles - 1) >> kCoarseShift;
+    constexpr int kBinsEach = ((kBinMaxTiles >> kCoarseShift) + kBinThreads) / kBinThreads;  // coarse bins per thread of the last workgroup
+    const bool last = blockIdx.x == gridDim.x - 1;
+    uint32_t bin_chunks[kBinsEach] = {};
+    if (last)
+#pragma unroll
+        for (int k = 0; k < kBinsEach; ++k)
+            if (kBinsEach * tid + k < bins) bin_chunks[k] = chunks_of(a.chunk_base[kBinsEach * tid + k]);
     const uint32_t pairs = tid < n_blocks ? (uint32_t)a.block_sums[tid] : 0u;  // (beyond 2^32 pairs the frame overflows)
     const uint32_t word = tid < n_blocks ? a.block_classes[tid] : 0u;
     SliceTotals slice = {0ull, 0u, 0u};
@@ -398,20 +406,19 @@ __device__ __forceinline__ uint32_t lay_out(const LayoutArgs& a, int T, uint32_t
             if (cls == c) a.lists[kListHeader + (size_t)c * T + lanes_below_in(m, at[c])] = (uint32_t)t;
         }
     }
-    if (a.chunk_base && blockIdx.x == gridDim.x - 1) {
-        const int bins = (T + kCoarseTiles - 1) >> kCoarseShift, per_thread = (bins + kBinThreads - 1) / kBinThreads;
-        const int q0 = min(tid * per_thread, bins), q1 = min(q0 + per_thread, bins);
+    if (last) {  // (each element was read by the thread that overwrites it)
         uint32_t chunks = 0;
-        for (int q = q0; q < q1; ++q) chunks += chunks_of(a.chunk_base[q]);
+#pragma unroll
+        for (int k = 0; k < kBinsEach; ++k) chunks += bin_chunks[k];
         const uint32_t inc = wave_sum_scan(chunks);
         if (lane == 63) s_waves[kSums * kWavesHere + wave] = inc;
         __syncthreads();
         uint32_t run = inc - chunks;
         for (int w = 0; w < wave; ++w) run += s_waves[kSums * kWavesHere + w];
-        for (int q = q0; q < q1; ++q) {  // (each element is read before it is overwritten, by its own thread)
-            const uint32_t n = chunks_of(a.chunk_base[q]);
-            a.chunk_base[q] = run;
-            run += n;
+#pragma unroll
+        for (int k = 0; k < kBinsEach; ++k) {
+            if (kBinsEach * tid + k < bins) a.chunk_base[kBinsEach * tid + k] = run;
+            run += bin_chunks[k];
         }
         if (tid == kBinThreads - 1) a.chunk_base[bins] = run;
     }
@@ -2168,7 +2175,7 @@ int launch_tile_scatter(const FrameArgs& f, int32_t P, const uint64_t* rects, co
         LayoutArgs layout = {};  // (the first launch makes it)
         if (make)
             layout = {tile_totals(tile_base, T), block_totals(tile_base, T), class_counts(tile_base, T), make->slice_totals, n_cap,
-                      header, make->header_copy, ranges, lists, levels != 1 ? chunk_bases(tile_base, T) : nullptr};
+                      header, make->header_copy, ranges, lists, chunk_bases(tile_base, T)};
         if (levels != 2) {
             min_keys = levels == 1 ? UINT32_MAX : two_from;
             hipLaunchKernelGGL((scatter_kernel<0, false>), dim3(groups), dim3(kBinThreads), (size_t)T * sizeof(uint32_t), s,

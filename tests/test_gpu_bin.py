@@ -93,6 +93,36 @@ def test_layout_made_by_the_scatter(gpu_device, width, height, P, log_scale, lev
 
 
 @pytest.mark.parametrize("width,height,P,log_scale", [
+    (16, 16, 70, 0.0), (16 * 65, 16, 3000, -2.0), (1000, 700, 9000, -2.5), (16 * 1023, 16, 20_000, -2.5), (16 * 360, 1600, 40_000, -5.0)])
+def test_scattered_again_in_two_levels(gpu_device, width, height, P, log_scale):
+    """Tile count and scatter in one level in one call, then the scatter by itself in two: the work list of its second level (bins of
+    16 tiles, as many as 2250) is there, and the pairs end where they did."""
+    scene = scenes.tiny_scene(P=P, width=width, height=height, sh_degree=0, seed=4, log_scale_mean=log_scale)
+    inp = pipeline.FrameInputs(settings_for(scene, gpu_device), scene.means3D.to(gpu_device), shs=scene.shs.to(gpu_device),
+                               opacities=scene.opacities.to(gpu_device), scales=scene.scales.to(gpu_device),
+                               rotations=scene.rotations.to(gpu_device))
+    out, ws, tiles, n_cap = pipeline.FrameOutputs(inp), pipeline.Workspace(gpu_device), inp.tiles, 1 << 24
+    lay = ws.ensure(P, n_cap, width, height)
+    ws.buffer.fill_(0x0)
+    run = lambda mask: pipeline.run_stages(inp, out, ws, n_cap, mask)  # noqa: E731
+    run(_lib.STAGE_PREPROCESS)
+    run(_lib.STAGE_TILE_COUNT | _lib.STAGE_TILE_SCATTER | _lib.STAGE_TILE_SCATTER_ONE_LEVEL)
+    at = lay.tile_base + 4 * (2 * tiles + 2 * ((tiles + 63) // 64))
+    bins = (tiles + 15) // 16
+    chunks = ws.buffer[at:at + 4 * (bins + 1)].view(torch.int32).cpu().numpy()
+    ranges = ws.view(lay, "ranges", P, 0, tiles).cpu().numpy()
+    n = np.pad(ranges[:, 1] - ranges[:, 0], (0, 16 * bins - tiles)).reshape(bins, 16).sum(1)
+    np.testing.assert_array_equal(chunks, np.concatenate([[0], np.cumsum((n + 2047) // 2048)]))
+    assert n.sum() > 0
+    run(_lib.STAGE_TILESORT)
+    want = [ws.view(lay, name, P, int(n.sum()), tiles).clone() for name in ("sorted_keys", "sorted_values")]
+    run(_lib.STAGE_TILE_SCATTER | _lib.STAGE_TILE_SCATTER_TWO_LEVEL)
+    run(_lib.STAGE_TILESORT)
+    for a, name in zip(want, ("sorted_keys", "sorted_values")):
+        assert torch.equal(ws.view(lay, name, P, int(n.sum()), tiles), a), name
+
+
+@pytest.mark.parametrize("width,height,P,log_scale", [
     (256, 256, 900, -1.0), (16 * 257, 16, 3000, -3.0), (512, 256, 2000, -2.0), (513, 256, 2000, -2.0), (1000, 700, 9000, -2.5),
     (16 * 360, 1600, 30_000, -5.0), (16 * 361, 1600, 30_000, -5.0)])
 def test_tiles_in_the_order_of_their_lists(gpu_device, width, height, P, log_scale):
