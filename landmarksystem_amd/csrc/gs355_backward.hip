@@ -444,14 +444,32 @@ __global__ __launch_bounds__(256) void blend_backward_kernel(
     }
 }
 
-// The preprocess's backward pass reads its inputs once and writes gradients that nothing reads soon: streaming accesses leave the
-// L2 to the records, which lanes pick out of lines a part at a time (streamed as well, they take the kernel to 1059 us).  6M
-// Gaussians from stored parameters: stores 706 -> 674 us, the coefficients' copies 668, the other inputs 660; and the next
-// frame's preprocess, which finds more of its lines unwritten, 326 -> 312.
-__device__ __forceinline__ void stream(float4* p, const float4 v)
+// The preprocess's backward pass reads its inputs once and writes gradients that nothing reads before the pass has ended.  In large
+// scenes streaming accesses (kStreamed) leave the L2 to the records, which lanes pick out of lines a part at a time (streamed as
+// well, they take the kernel to 1059 us).  6M Gaussians from stored parameters: stores 706 -> 674 us, the coefficients' copies 668,
+// the other inputs 660; and the next frame's preprocess, which finds more of its lines unwritten, 326 -> 312.
+// Smaller scenes' parameters and gradients are in the caches when the optimizer reads both next: Adam's step alone, behind a pass
+// with ordinary and with streaming accesses, 30k Gaussians of sixteen coefficients 98 and 104 us, 100k of nine 87 and 108, of one
+// 84 and 104.  Pass and step: 100k of nine 457 to 468 and 475 to 483 us, 150k of sixteen 482 and 473, 270k 629 and 631, 400k 760
+// and 750, 1M 1191 and 1146.
+constexpr int kStreamedFrom = 1 << 17;
+template <bool kStreamed>
+__device__ __forceinline__ void put(float4* p, const float4 v)
 {
     const f32x4 x = {v.x, v.y, v.z, v.w};
-    __builtin_nontemporal_store(x, reinterpret_cast<f32x4*>(p));
+    if (kStreamed) __builtin_nontemporal_store(x, reinterpret_cast<f32x4*>(p));
+    else *p = v;
+}
+template <bool kStreamed>
+__device__ __forceinline__ void put(float* p, float v)
+{
+    if (kStreamed) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+template <bool kStreamed>
+__device__ __forceinline__ float get(const float* p)
+{
+    return kStreamed ? __builtin_nontemporal_load(p) : *p;
 }
 constexpr float kShC0 = 0.28209479177387814f;
 constexpr float kShC1 = 0.4886025119029199f;
@@ -703,7 +721,7 @@ __global__ __launch_bounds__(256) void sum_large_kernel(int P, bool plain, const
 // vanilla model's stored parameters, and the gradients are theirs (activations' derivatives included); the rows of the
 // SH coefficients behind the first are then staged back to back, 3 (M - 1) floats each, as they lie in memory: a
 // wavefront's 64 rows start on a 256-B boundary whatever their length.
-template <int kMode, bool kStored, bool kDepth>
+template <int kMode, bool kStored, bool kDepth, bool kStreamed>
 __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kernel(FrameArgs f, gs355_gaussians g,
                                                                   const int32_t* __restrict__ radii,
                                                                   const float* __restrict__ records,
@@ -754,12 +772,12 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
     if (fetch_sh && kStored) {
         typedef __attribute__((address_space(1))) const void global_void;
         typedef __attribute__((address_space(3))) void lds_void;
-        constexpr int kStreaming = 2;  // (the copy's cache policy: nontemporal)
+        constexpr int kPolicy = kStreamed ? 2 : 0;  // (of the copies: nontemporal, or as ordinary loads)
         const float4* src = reinterpret_cast<const float4*>(par.rest + run_first);
 #pragma unroll
         for (int it = 0; it < 12; ++it)
             if (it * 64 + lane < run4)  // (lane l of a copy writes float4 l behind the uniform LDS address)
-                __builtin_amdgcn_global_load_lds((global_void*)(src + it * 64 + lane), (lds_void*)(mine + it * 64), 16, 0, kStreaming);
+                __builtin_amdgcn_global_load_lds((global_void*)(src + it * 64 + lane), (lds_void*)(mine + it * 64), 16, 0, kPolicy);
         if (lane < run_tail) tail = par.rest[run_first + 4 * run4 + lane];
     }
     // the Gaussian's own inputs are requested before its records are waited for, too
@@ -768,14 +786,14 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
     uint32_t in_lit = 0u;
     if (alive) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) in_mean[k] = __builtin_nontemporal_load(&g.means3D[3 * si + k]);
+        for (int k = 0; k < 3; ++k) in_mean[k] = get<kStreamed>(&g.means3D[3 * si + k]);
         if (kStored || !g.cov3D_precomp) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) in_scale[k] = __builtin_nontemporal_load(&g.scales[3 * si + k]);
+            for (int k = 0; k < 3; ++k) in_scale[k] = get<kStreamed>(&g.scales[3 * si + k]);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) in_rot[k] = __builtin_nontemporal_load(&g.rotations[4 * si + k]);
+            for (int k = 0; k < 4; ++k) in_rot[k] = get<kStreamed>(&g.rotations[4 * si + k]);
         }
-        if (kStored) in_opacity = __builtin_nontemporal_load(&g.opacities[si]);
+        if (kStored) in_opacity = get<kStreamed>(&g.opacities[si]);
         if (g.shs) in_lit = lit[si];
     }
     constexpr int N = kPartFloats<kDepth>;
@@ -1006,7 +1024,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
         if (kStored) {
             if (out.shs && valid)
 #pragma unroll
-                for (int c = 0; c < 3; ++c) __builtin_nontemporal_store(alive ? b[0] * gcol[c] : 0.0f, &out.shs[3 * si + c]);
+                for (int c = 0; c < 3; ++c) put<kStreamed>(&out.shs[3 * si + c], alive ? b[0] * gcol[c] : 0.0f);
             if (par.d_rest && staged) {
                 wave_lds_sync();  // rows were read above
 #pragma unroll
@@ -1021,7 +1039,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
                 float4* __restrict__ dst = reinterpret_cast<float4*>(par.d_rest + run_first);
 #pragma unroll
                 for (int it = 0; it < 12; ++it)
-                    if (it * 64 + lane < run4) stream(&dst[it * 64 + lane], mine[it * 64 + lane]);
+                    if (it * 64 + lane < run4) put<kStreamed>(&dst[it * 64 + lane], mine[it * 64 + lane]);
                 if (lane < run_tail) par.d_rest[run_first + 4 * run4 + lane] = reinterpret_cast<float*>(mine)[4 * run4 + lane];
             } else if (par.d_rest && valid) {
 #pragma unroll
@@ -1048,7 +1066,7 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
                 for (int it = 0; it < 12; ++it) {
                     const int q4 = it * 64 + lane;
                     const int e = q4 / 12, m = q4 % 12;
-                    if (e < count) stream(reinterpret_cast<float4*>(out.shs + (wave_first + e) * 48) + m, mine[e * (kShStride / 4) + m]);
+                    if (e < count) put<kStreamed>(reinterpret_cast<float4*>(out.shs + (wave_first + e) * 48) + m, mine[e * (kShStride / 4) + m]);
                 }
             } else if (valid) {
                 float* __restrict__ o = out.shs + si * M * 3;
@@ -1069,23 +1087,23 @@ __global__ __launch_bounds__(256, kStored ? 3 : 1) void preprocess_backward_kern
 
     if (out.means3D)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) __builtin_nontemporal_store(dmean[k], &out.means3D[3 * si + k]);
+        for (int k = 0; k < 3; ++k) put<kStreamed>(&out.means3D[3 * si + k], dmean[k]);
     if (out.means2D)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) __builtin_nontemporal_store(d2[k], &out.means2D[3 * si + k]);
-    if (out.opacities) __builtin_nontemporal_store(dop, &out.opacities[i]);
+        for (int k = 0; k < 3; ++k) put<kStreamed>(&out.means2D[3 * si + k], d2[k]);
+    if (out.opacities) put<kStreamed>(&out.opacities[i], dop);
     if (out.colors_precomp)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) __builtin_nontemporal_store(dcol[k], &out.colors_precomp[3 * si + k]);
+        for (int k = 0; k < 3; ++k) put<kStreamed>(&out.colors_precomp[3 * si + k], dcol[k]);
     if (out.scales)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) __builtin_nontemporal_store(dscale[k], &out.scales[3 * si + k]);
+        for (int k = 0; k < 3; ++k) put<kStreamed>(&out.scales[3 * si + k], dscale[k]);
     if (out.rotations)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) __builtin_nontemporal_store(drot[k], &out.rotations[4 * si + k]);
+        for (int k = 0; k < 4; ++k) put<kStreamed>(&out.rotations[4 * si + k], drot[k]);
     if (out.cov3D_precomp)
 #pragma unroll
-        for (int k = 0; k < 6; ++k) __builtin_nontemporal_store(dcov[k], &out.cov3D_precomp[6 * si + k]);
+        for (int k = 0; k < 6; ++k) put<kStreamed>(&out.cov3D_precomp[6 * si + k], dcov[k]);
 }
 
 }  // namespace
@@ -1126,20 +1144,25 @@ int launch_render_backward(const FrameArgs& f, const gs355_gaussians& g, const g
         auto launch = [&](auto kernel, const ParameterArgs& p) {
             hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, in.radii, records, rects, slots, lit, key_grads, out, p, summed);
         };
-        if (par) {
-            if ((reinterpret_cast<uintptr_t>(par->rest) & 15u) != 0 || (reinterpret_cast<uintptr_t>(par->d_rest) & 15u) != 0)
-                launch(preprocess_backward_kernel<0, true, kDepth>, *par);
-            else if (f.sh_degree == 0)
-                launch(preprocess_backward_kernel<1, true, kDepth>, *par);
-            else
-                launch(preprocess_backward_kernel<2, true, kDepth>, *par);
-        } else if (!staged) {
-            launch(preprocess_backward_kernel<0, false, kDepth>, ParameterArgs());
-        } else if (f.sh_degree == 0) {
-            launch(preprocess_backward_kernel<1, false, kDepth>, ParameterArgs());
-        } else {
-            launch(preprocess_backward_kernel<2, false, kDepth>, ParameterArgs());
-        }
+        auto pass = [&](auto streamed) {
+            constexpr bool kStreamed = streamed.value;
+            if (par) {
+                if ((reinterpret_cast<uintptr_t>(par->rest) & 15u) != 0 || (reinterpret_cast<uintptr_t>(par->d_rest) & 15u) != 0)
+                    launch(preprocess_backward_kernel<0, true, kDepth, kStreamed>, *par);
+                else if (f.sh_degree == 0)
+                    launch(preprocess_backward_kernel<1, true, kDepth, kStreamed>, *par);
+                else
+                    launch(preprocess_backward_kernel<2, true, kDepth, kStreamed>, *par);
+            } else if (!staged) {
+                launch(preprocess_backward_kernel<0, false, kDepth, kStreamed>, ParameterArgs());
+            } else if (f.sh_degree == 0) {
+                launch(preprocess_backward_kernel<1, false, kDepth, kStreamed>, ParameterArgs());
+            } else {
+                launch(preprocess_backward_kernel<2, false, kDepth, kStreamed>, ParameterArgs());
+            }
+        };
+        if (g.P >= kStreamedFrom) pass(std::true_type{});
+        else pass(std::false_type{});
         GS355_CHECK_LAUNCH("preprocess backward");
         return (int)GS355_OK;
     };
