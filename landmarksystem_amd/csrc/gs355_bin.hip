@@ -1659,11 +1659,15 @@ struct WaveSorter {
 // once in frames of a few thousand tiles, and the compute unit with the longest lists decides; in larger frames the last ones to
 // start do.  2170 tiles: blend 47.1 -> 44.7 us, 1734: backward blend 100.5 -> 96.1; 8160 tiles, 6M Gaussians: 276.9 -> 272.6 and
 // 844.7 -> 830.1, although neighbouring tiles no longer find each other's records in the L2.  One workgroup beside the sorts
-// makes it in their time (the sorts of 2170 tiles 9.1 -> 9.5 us; as a launch of its own it took 9 to 33 us, more than it gave).
+// makes it, in 9 us for 8160 tiles, 16 for 14400 and 32 for 32400 (nearly all empty: 58, they share a bin), so it is made where
+// the sorts take as long, from kOrderMinPairs pairs per tile on average (the sorts of 2170 tiles 9.1 -> 9.5 us with it).  With fewer it was the
+// launch's length and the blends gained nothing: at 3840x2160 frames of 17, 14k, 582k and 2.2M pairs 126, 120, 155 and 249 us with it, 84,
+// 94, 143 and 237 without; at 1920x1080 of 19, 30k and 500k pairs 48, 51 and 76, and 39, 48 and 73.
 // Lengths are taken to a sixteenth of a power of two; the order within one of those steps is free.
 constexpr int kOrderBins = 512;        // sixteen steps for each of 32 powers of two
 constexpr int kOrderMinTiles = 257;    // up to a tile per compute unit there is nothing to order
 constexpr int kOrderMaxTiles = kBinMaxTiles;
+constexpr uint32_t kOrderMinPairs = 128;  // per tile
 
 template <int kT>
 __device__ __forceinline__ void order_tiles(const uint32_t* __restrict__ ranges, uint32_t tiles, uint4* __restrict__ order,
@@ -1718,8 +1722,8 @@ __device__ __forceinline__ void order_tiles(const uint32_t* __restrict__ ranges,
 // one after all, is sorted here by radix passes through global memory, ping-ponging between the bucket and the tile's slice
 // of the output keys (their scratch lies over the LDS sorter's area), so every bucket is sorted whatever the caller expected.
 //
-// The first workgroup is none of the tiles': it orders them by the length of their lists for the blends (order_tiles), beside
-// the sorts.  kByWave: behind the workgroups with a tile each come some with a wavefront per tile, four consecutive ones, for the
+// The first workgroup is none of the tiles': in frames of many pairs it orders them by the length of their lists for the blends
+// (order_tiles), beside the sorts.  kByWave: behind the workgroups with a tile each come some with a wavefront per tile, four consecutive ones, for the
 // buckets of up to 256 pairs, which the others leave.
 template <int kT, int kR, bool kByWave>
 __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header,
@@ -1733,6 +1737,7 @@ __global__ __launch_bounds__(kT) void tile_sort_each_kernel(gs355_header* header
     if (header->overflow) return;
     if (order && blockIdx.x == 0) {
         static_assert((kOrderBins + kT / 64) * sizeof(uint32_t) <= LdsSorter<kT, kR>::kBytes, "bins and sums");
+        if (header->num_keys < kOrderMinPairs * tiles) return;
         order_tiles<kT>(ranges, tiles, order, s_dyn);
         if (threadIdx.x == 0) header->ordered = 1u;
         return;

@@ -123,11 +123,12 @@ def test_scattered_again_in_two_levels(gpu_device, width, height, P, log_scale):
 
 
 @pytest.mark.parametrize("width,height,P,log_scale", [
-    (256, 256, 900, -1.0), (16 * 257, 16, 3000, -3.0), (512, 256, 2000, -2.0), (513, 256, 2000, -2.0), (1000, 700, 9000, -2.5),
-    (16 * 360, 1600, 30_000, -5.0), (16 * 361, 1600, 30_000, -5.0)])
+    (256, 256, 900, -1.0), (16 * 257, 16, 3000, -1.5), (512, 256, 2000, -2.0), (513, 256, 2000, -2.0), (1000, 700, 9000, -2.5),
+    (1000, 700, 9000, -5.0), (16 * 360, 1600, 4000, -2.5), (16 * 360, 1600, 30_000, -5.0), (16 * 361, 1600, 4000, -2.5)])
 def test_tiles_in_the_order_of_their_lists(gpu_device, width, height, P, log_scale):
     """The tile sort's order of the tiles: each of them once, with its range, no later than a list of more than 1/16 less; made
-    for 257 to 36000 tiles; the same image with and without it; and forgotten when a new frame's header is written."""
+    for 257 to 36000 tiles of 128 pairs or more on average; the same image with and without it; and forgotten when a new frame's
+    header is written."""
     scene = scenes.tiny_scene(P=P, width=width, height=height, sh_degree=0, seed=5, log_scale_mean=log_scale)
     inp = pipeline.FrameInputs(settings_for(scene, gpu_device), scene.means3D.to(gpu_device), shs=scene.shs.to(gpu_device),
                                opacities=scene.opacities.to(gpu_device), scales=scene.scales.to(gpu_device),
@@ -141,7 +142,9 @@ def test_tiles_in_the_order_of_their_lists(gpu_device, width, height, P, log_sca
     run(_lib.STAGE_TILE_COUNT | _lib.STAGE_TILE_SCATTER)
     assert int(word()) == 0
     run(_lib.STAGE_TILESORT | _lib.STAGE_BLEND)
-    made = 257 <= tiles <= 36000
+    pairs = int(ws.view(lay, "header", P, 0, tiles)[1].item()) & 0xFFFFFFFF
+    assert pairs > 0 and (pairs >= 128 * tiles) == (log_scale > -5.0)
+    made = 257 <= tiles <= 36000 and log_scale > -5.0
     assert int(word()) == made
     image = out.image.clone()
     if made:
