@@ -113,17 +113,16 @@ __device__ __forceinline__ void sh_finish(float res[3])
 // loads touch survivors' blocks only, however few of the 256 survived.  A row of the staging area holds an
 // entry's coefficients and, behind them, the Gaussian's position on the way in and its colour on the way out.
 //
-// kCoeffs: coefficients per Gaussian, 4, 9 or 16 (degrees 1 to 3).  kSplit: the split storage of the stored parameters,
+// kCoeffs: coefficients per Gaussian, 4, 9 or 16 (degrees 1 to 3).  kSplit: the split storage of the stored parameters (9 or 16),
 // whose first coefficient (12 B per Gaussian) is read by the entry's own lane, and the others as a row of their own.
-// Rows of a multiple of four floats are 16-B chunks as they are.  The others (27 floats of nine coefficients; 45 and 9
-// behind a first one) are dword-aligned and read with 16-B loads all the same: a Gaussian's row starts up to three floats
+// Rows of a multiple of four floats are 16-B chunks as they are.  The others (27 floats of nine coefficients, 45 behind a
+// first one) are dword-aligned and read with 16-B loads all the same: a Gaussian's row starts up to three floats
 // behind a 16-B boundary, (row * kRow) & 3, and spans kChunks aligned chunks.  They land in the staging row as they are,
 // so that the coefficients of entry e start at that float of its row.  `n_floats`: kRow P.  The last chunk of the last row
 // may reach past the array: it is pulled back inside, and that row's last floats are fetched by its own lane.
 //
 // What it is for: a lane that reads its own block asks for a cache line per dword, and 64 lanes' blocks of 108 B are more
-// lines than the L1 keeps until their next dword.  3M Gaussians at 1080p: nine coefficients 216 -> 113 us, four 94 -> 81
-// (sixteen: 152); stored parameters 207 -> 121 and 97 -> 87.
+// lines than the L1 keeps until their next dword (staged_blocks).
 //
 // fetch() and colour() are apart so that the caller has work to do while the blocks travel.
 template <bool kSplit, int kCoeffs>
@@ -256,7 +255,7 @@ constexpr int kRecordsStreamedFrom = 1 << 21;
 // memory each, and joining the SH coefficients one over 192 B per Gaussian: at 6M Gaussians 1.3 ms of such passes in
 // front of a kernel of 0.3 ms).
 // kPacked: coefficients of SH blocks that are fetched by way of LDS (ShEntries), 0: none.  The 20 to 53 KB of that leave seven to
-// three wavefronts per SIMD, so calls without such blocks (colours given, or blocks of another size) run a kernel without it, at
+// three wavefronts per SIMD, so calls whose blocks go by lane (staged_blocks), and those with colours given, run a kernel without it, at
 // eight: 1.5M decoded Gaussians 100 -> 76 us, 600k 32.5 -> 24.5, 160k 13.8 -> 12.4.
 template <bool kRadiiOnly, bool kStored, int kPacked>
 __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaussians g, ParameterArgs par, FilterArgs fx,
@@ -457,10 +456,9 @@ __global__ __launch_bounds__(256) void preprocess_kernel(FrameArgs f, gs355_gaus
         }
         reach_and_region();
     } else {
-        // Blocks of 4, 9 or 16 coefficients: the survivors of the workgroup are packed (in order) and each wavefront fetches the
-        // SH blocks of 64 of them with coalesced loads through LDS, so the memory system sees dense wavefronts
-        // however many Gaussians were culled.  Other block sizes: every survivor fetches its own block.  Same
-        // values and the same order of additions either way.
+        // kPacked: the survivors of the workgroup are packed (in order) and each wavefront fetches the SH blocks of 64 of
+        // them with coalesced loads through LDS, so the memory system sees dense wavefronts however many Gaussians were
+        // culled.  Else every survivor fetches its own block.  Same values and the same order of additions either way.
         if constexpr (kPacked) {
             const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
             const uint64_t m = alive_lanes;
@@ -617,6 +615,25 @@ __global__ __launch_bounds__(256) void duplicate_kernel(FrameArgs f, int32_t P, 
     }
 }
 
+// Whether SH blocks travel through LDS (ShEntries) or each lane reads its own.  Staged, a block is fetched whole, by three to seven
+// wavefronts per SIMD; a lane fetches what the active degree needs, at eight.  So it takes a degree that needs all or most of
+// the block, and a scene whose blocks the caches do not keep between a lane's dwords.  By way of LDS and by lane, us at 1080p
+// with 88 % of the Gaussians on the screen:
+//   16 coefficients, degree 3   131k 11.2 14.7, 800k 46 154, 6M 288 879         degree 2   131k 11.1 10.9, 300k 21 26, 6M 280 458
+//   9, degree 2                 131k 10.0 9.4, 200k 13.2 14.5, 6M 215 391       stored     200k 14.5 13.6, 300k 17.4 17.7, 6M 210 340
+//   4, degree 1                 524k 20.3 18.1, 800k 26.6 26.8, 6M 151 169      stored     524k 23.0 19.5, 2M 61 55, 6M 171 165
+//   16, degree 1                800k 45 34, 6M 278 267                          stored     800k 49 35, 6M 292 289
+//   16, degree 0                800k 45 29, 6M 279 233                          stored     800k 49 26, 6M 292 136
+//   9, degree 1                 300k 17.5 14.6, 1.2M 48 46, 6M 211 250          stored     300k 17.0 14.9, 1.2M 47 42, 6M 208 227
+//   9, degree 0                 300k 17.0 12.7, 1.2M 47 39, 6M 207 212          stored     300k 16.5 13.2, 1.2M 46 33, 6M 207 139
+// (with 16 % on the screen nine coefficients at degree 1, 4M and 12M: 108 80 and 310 246)
+bool staged_blocks(int coeffs, int degree, bool stored, int32_t P)
+{
+    if (coeffs == 16) return degree >= 2;
+    if (coeffs == 9) return degree >= 2 && P >= (stored ? 4 << 16 : 3 << 16);
+    return coeffs == 4 && degree >= 1 && !stored && P >= 3 << 18;
+}
+
 }  // namespace
 
 int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const ParameterArgs* par, bool radii_only, float* records,
@@ -626,11 +643,9 @@ int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const Parame
     if (g.P == 0) return GS355_OK;
     const dim3 block(256), grid((g.P + 255) / 256);
     const FilterArgs none;
-    // Any other number of coefficients, and blocks off the 16-byte boundaries of ordinary allocations: a lane per block.  So are
-    // small blocks of small scenes, whose lines the caches keep: four coefficients 17.7 us at 500k and 32.6 at 1M by lane, 18.7 and
-    // 29.6 by way of LDS; nine 10.0 at 130k and 16.4 at 250k by lane, 10.3 and 13.7.
+    // (any other number of coefficients, and blocks off the 16-byte boundaries of ordinary allocations: a lane per block)
     const bool aligned = (par || !g.colors_precomp) && (reinterpret_cast<uintptr_t>(par ? par->rest : g.shs) & 15u) == 0;
-    const int packed = aligned && g.P >= (f.sh_coeffs == 4 ? 1 << 19 : f.sh_coeffs == 9 ? 1 << 17 : 0) ? f.sh_coeffs : 0;
+    const int packed = aligned && staged_blocks(f.sh_coeffs, f.sh_degree, par != nullptr, g.P) ? f.sh_coeffs : 0;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, block, 0, s, f, g, par ? *par : ParameterArgs(), none, records, tiles_touched, rects,
                            depth_bits, wave_totals, lit, radii);
@@ -638,7 +653,7 @@ int launch_preprocess(const FrameArgs& f, const gs355_gaussians& g, const Parame
     if (radii_only) launch(preprocess_kernel<true, false, 0>);
     else if (packed == 16) launch(par ? preprocess_kernel<false, true, 16> : preprocess_kernel<false, false, 16>);
     else if (packed == 9) launch(par ? preprocess_kernel<false, true, 9> : preprocess_kernel<false, false, 9>);
-    else if (packed == 4) launch(par ? preprocess_kernel<false, true, 4> : preprocess_kernel<false, false, 4>);
+    else if (packed == 4) launch(preprocess_kernel<false, false, 4>);
     else launch(par ? preprocess_kernel<false, true, 0> : preprocess_kernel<false, false, 0>);
     GS355_CHECK_LAUNCH("preprocess");
     return GS355_OK;

@@ -25,14 +25,16 @@ def _frame(scene, device, shs, rest, scales, rotations, opacities, active):
     return records.view(torch.int32), out.radii.clone()
 
 
-# Rows of 9, 12, 24, 27, 45 and 48 floats, whose last one ends on every remainder of a 16-byte chunk, in scenes of as many Gaussians
-# as it takes (four coefficients: 2^19, nine: 2^17); one survivor, all, and workgroups of which few survive.
-@pytest.mark.parametrize("stored", [False, True])
-@pytest.mark.parametrize("degree,P,active,spread", [
-    (1, 1 << 19, 1, 1.0), (1, (1 << 19) + 1, 1, 6.0), (1, (1 << 19) + 2, 0, 3.0), (1, (1 << 19) + 63, 1, 1.0),
-    (2, 1 << 17, 2, 1.0), (2, (1 << 17) + 1, 1, 6.0), (2, (1 << 17) + 2, 0, 3.0), (2, (1 << 17) + 67, 2, 1.0),
-    (3, 1, 3, 0.1), (3, 2, 3, 0.1), (3, 3, 1, 0.1), (3, 63, 2, 1.0), (3, 258, 3, 6.0), (3, 5000, 0, 3.0)])
-def test_blocks_through_lds_give_the_same_colours(gpu_device, stored, degree, P, active, spread):
+# Rows of 12, 24, 27, 45 and 48 floats, whose last one ends on every remainder of a 16-byte chunk, in scenes of as many Gaussians
+# and at the degrees that it takes (four coefficients: not stored, 3 2^18, degree 1; nine: 2^18, degree 2; sixteen: degree 2); one
+# survivor, all, and workgroups of which few survive.
+@pytest.mark.parametrize("degree,P,active,spread,stored", [
+    (1, 3 << 18, 1, 1.0, False), (1, (3 << 18) + 1, 1, 6.0, False), (1, (3 << 18) + 63, 1, 3.0, False),
+    (2, 1 << 18, 2, 1.0, False), (2, (1 << 18) + 1, 2, 6.0, False), (2, (1 << 18) + 2, 2, 3.0, False), (2, (1 << 18) + 67, 2, 1.0, False),
+    (2, 1 << 18, 2, 1.0, True), (2, (1 << 18) + 1, 2, 6.0, True), (2, (1 << 18) + 2, 2, 3.0, True), (2, (1 << 18) + 67, 2, 1.0, True),
+    (3, 1, 3, 0.1, False), (3, 2, 3, 0.1, False), (3, 3, 2, 0.1, False), (3, 63, 2, 1.0, False), (3, 258, 3, 6.0, False), (3, 5000, 2, 3.0, False),
+    (3, 1, 3, 0.1, True), (3, 2, 3, 0.1, True), (3, 3, 2, 0.1, True), (3, 63, 2, 1.0, True), (3, 258, 3, 6.0, True), (3, 5000, 2, 3.0, True)])
+def test_blocks_through_lds_give_the_same_colours(gpu_device, degree, P, active, spread, stored):
     scene = scenes.tiny_scene(P=P, width=150, height=97, sh_degree=degree, spread=spread, seed=P)
     scales, opacities = scene.scales.to(gpu_device), scene.opacities.to(gpu_device)
     shs, rest = scene.shs.to(gpu_device), None
@@ -80,3 +82,34 @@ def test_records_that_are_streamed(gpu_device, degree, spread):
         rows = ws.view(lay, "records", n, 0, inp.tiles).view(torch.int32)
         records.append(rows[:P - 1][out.radii[:P - 1] > 0].clone())
     assert records[0].shape[0] > 1000 and torch.equal(records[0], records[1])
+
+
+@pytest.mark.parametrize("coeffs,active,P,stored", [(9, 0, 200_000, False), (9, 0, 200_000, True), (9, 1, 200_000, True), (9, 0, 1_000_000, True),
+                                                    (4, 1, 600_000, True), (16, 0, 1_000_000, False), (16, 1, 300_000, True)])
+def test_blocks_that_a_degree_does_not_need_are_not_fetched(gpu_device, coeffs, active, P, stored):
+    """The preprocess at less than the stored degree, or over small blocks of small scenes, against the same by a lane per block (blocks
+    fetched whole: 1.15 to 1.9 times as long)."""
+    scene = scenes.config3(P=P)
+    shs, scales, opacities, rest = scene.shs[:, :coeffs].contiguous().to(gpu_device), scene.scales.to(gpu_device), scene.opacities.to(gpu_device), None
+    if stored:
+        scales, opacities = scales.log(), torch.logit(opacities)
+        shs, rest = shs[:, :1].contiguous(), shs[:, 1:].contiguous()
+    runs = []
+    for off in (False, True):
+        pick = _off_boundary if off else (lambda t: t)
+        inp = pipeline.FrameInputs(settings_for(scene, gpu_device, sh_degree=active), scene.means3D.to(gpu_device), opacities=opacities,
+                                   shs=shs if stored else pick(shs), scales=scales, rotations=scene.rotations.to(gpu_device),
+                                   features_rest=pick(rest) if stored else None)
+        runs.append((inp, pipeline.FrameOutputs(inp), pipeline.Workspace(gpu_device)))
+    best = [1e9, 1e9]
+    for k in range(12):
+        start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        torch.cuda._sleep(400_000)  # (the host is ahead when the first of them begins)
+        start.record()
+        for _ in range(20):
+            pipeline.run_stages(*runs[k % 2], 1 << 10, _lib.STAGE_PREPROCESS)
+        stop.record()
+        torch.cuda.synchronize()
+        best[k % 2] = min(best[k % 2], start.elapsed_time(stop) / 20)
+    print("preprocess: %.1f us, %.1f us by lane" % (1e3 * best[0], 1e3 * best[1]))
+    assert best[0] < 1.1 * best[1]
