@@ -181,7 +181,7 @@ enum {
      *                 launch makes bases, ranges and header.  Beyond 36000 tiles the
      *                 slices count per bin of 16 consecutive tiles, and ranges follow with TILE_SCATTER.
      *   TILE_SCATTER  (depth bits << 32 | index) pairs into their tile's bucket: straight for frames of fewer
-     *                 than 6 * 2^20 pairs, through bins of 16 consecutive tiles beyond (decided on the device;
+     *                 than 6 * 2^20 pairs (12 * 2^20 with gs355_gaussians.P_device), through bins of 16 consecutive tiles beyond (decided on the device;
      *                 always beyond 36000 tiles).  The decision costs the launch of the variant that then does
      *                 nothing; a caller that knows the size of its frames (say from the previous frame's header)
      *                 names the variant with one of the modifiers below.  Either variant is correct for any frame.

@@ -19,8 +19,8 @@ STAGE_BLEND_PLAIN = 64
 STAGE_TILE_COUNT, STAGE_TILESORT, STAGE_TILE_SCATTER = 128, 256, 512
 STAGE_TILE_SCATTER_TWO_LEVEL = 1024  # modifiers of STAGE_TILE_SCATTER: name the variant instead of letting the device
 STAGE_TILE_SCATTER_ONE_LEVEL = 2048  # choose by the key count (which launches both)
-# the device's own thresholds: Gaussians with a count on the device (decoded), with colours of their own, others
-TWO_LEVEL_FROM_DECODED, TWO_LEVEL_FROM_COLOURS, TWO_LEVEL_FROM = 12 << 20, 6 << 20, 3 << 20
+# the device's own thresholds: Gaussians with a count on the device (decoded), others
+TWO_LEVEL_FROM_DECODED, TWO_LEVEL_FROM = 12 << 20, 6 << 20
 STAGE_TILESORT_SKIP = (4096, 8192, 16384)  # modifiers of STAGE_TILESORT: do not launch that size class's sorter
 STAGE_TILE_REACH = 65536  # modifier of STAGE_PREPROCESS: keys only for the tiles that a Gaussian's alpha >= 1/255 ellipse reaches
 STAGE_TILESORT_VALUES = 131072  # modifier of STAGE_TILESORT: the sorted values only (no later stage reads the sorted keys)

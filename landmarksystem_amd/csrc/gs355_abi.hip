@@ -324,7 +324,7 @@ static int enqueue_stages(const gs355_frame* frame, const gs355_gaussians* g, co
                                       (stage_mask & GS355_STAGE_TILE_SCATTER_TWO_LEVEL)   ? 2
                                       : (stage_mask & GS355_STAGE_TILE_SCATTER_ONE_LEVEL) ? 1
                                                                                           : 0,
-                                      two_level_from(g->P_device != nullptr, g->colors_precomp != nullptr), in_scatter ? &make : nullptr, s)))
+                                      two_level_from(g->P_device != nullptr), in_scatter ? &make : nullptr, s)))
             return rc;
     if (stage_mask & GS355_STAGE_TILESORT)
         if ((rc = launch_tile_sort(header, tiles, ranges, tile_lists, buckets, keys[L.sorted_buffer],

@@ -411,11 +411,12 @@ struct ScatterLayout {
     const SliceTotals* slice_totals;
     gs355_header* header_copy;
 };
-// Pairs from which a frame scatters in two levels.  Whole frames, two levels against one: given scenes, in random order, 1.04 of
-// the time at 1.0M pairs, 1.02 at 1.7M, 1.00 at 2.8M, 0.99 at 3.2M, 0.96 at 5.9M, 0.94 at 9.8M.  Decoded Gaussians follow their
-// anchors, runs of neighbours whose pairs the L2 merges by itself: 1.05 at 1.7M, 1.03 at 7.0M, 1.02 at 9.4M (more not measured).
-// Gaussians with colours of their own may have been either.
-inline uint32_t two_level_from(bool decoded, bool own_colours) { return (decoded ? 12u : own_colours ? 6u : 3u) << 20; }
+// Pairs from which a frame scatters in two levels.  What decides is the order that the Gaussians are stored in, which the call does
+// not say.  Whole frames at 1080p, two levels against one: slabs in random order 0.96 of the time at 3.7 to 5.7 Mi pairs, 0.94 at 7.6,
+// 0.93 at 9.5; in Morton order, whose runs of neighbours the L2 merges by itself, 1.04 at all of these, in blocks of 20 m 1.03.  The
+// line lies between.  Decoded Gaussians follow their anchors: 1.05 at 1.7 Mi pairs, 1.03 at 7.0, 1.02 at 9.4 (more not measured);
+// where the caller has read their number they arrive as given ones.
+inline uint32_t two_level_from(bool decoded) { return (decoded ? 12u : 6u) << 20; }
 // `coarse`: a second buffer of the buckets' size (first level of the two-level scatter).  `levels`: 1 or 2 = that
 // scatter whatever the frame holds, 0 = chosen on the device by the key count against `two_from` (both variants are launched); images
 // beyond kBinMaxTiles tiles always take two levels.  `make`: NULL, or the layout is made on the way (up to kBinMaxTiles tiles)

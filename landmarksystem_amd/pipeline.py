@@ -353,8 +353,7 @@ def render(inputs: FrameInputs, want_depth: bool = True, want_alpha: bool = True
         front = _lib.STAGE_PREPROCESS | _lib.STAGE_TILE_REACH | _lib.STAGE_TILE_COUNT
         back = _lib.STAGE_TILE_SCATTER | _lib.STAGE_TILESORT | _lib.STAGE_TILESORT_VALUES | _lib.STAGE_BLEND
         # the scatter variant that suited the previous frame of this workspace (either is correct for any frame)
-        two_from = (_lib.TWO_LEVEL_FROM_DECODED if inputs.count is not None
-                    else _lib.TWO_LEVEL_FROM_COLOURS if inputs.colors_precomp is not None else _lib.TWO_LEVEL_FROM)
+        two_from = _lib.TWO_LEVEL_FROM if inputs.count is None else _lib.TWO_LEVEL_FROM_DECODED
         back |= (_lib.STAGE_TILE_SCATTER_TWO_LEVEL if ws.last_num_pairs >= two_from
                  else _lib.STAGE_TILE_SCATTER_ONE_LEVEL)
         # no launch for a sorter size class that the last few frames left empty (a hint: the library sorts the

@@ -558,3 +558,10 @@ def test_tile_reach_is_for_the_bucketed_stages():
     assert "no known stage" in _err(_lib.GS355_EINVAL, run, _lib.STAGE_TILE_REACH)
     assert "no known stage" in _err(_lib.GS355_EINVAL, run, _lib.STAGE_TILESORT_VALUES)
     assert "needed" in _err(_lib.GS355_ENOSPC, run, _lib.PIPELINE_FAST | _lib.STAGE_TILE_REACH)
+
+
+def test_the_drivers_scatter_thresholds_are_the_librarys():
+    """The pairs from which pipeline.render names the two-level scatter against those from which the library chooses it by itself."""
+    with open(os.path.join(ROOT, "landmarksystem_amd", "csrc", "gs355_internal.h")) as f:
+        rule = re.search(r"two_level_from\(bool decoded\) \{ return \(decoded \? (\d+)u : (\d+)u\) << 20; \}", f.read())
+    assert (_lib.TWO_LEVEL_FROM_DECODED, _lib.TWO_LEVEL_FROM) == (int(rule.group(1)) << 20, int(rule.group(2)) << 20)

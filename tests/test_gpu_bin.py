@@ -209,10 +209,12 @@ def test_buckets_beyond_the_lds(gpu_device, P, equal, side):
     assert ws.sort_mispredictions == 0
 
 
+@pytest.mark.parametrize("P,pairs", [(8500, (3, 6)), (13_000, (6, 12)), (24_000, (12, 18))])
 @pytest.mark.parametrize("form", ["shs", "colours", "count"])
-def test_frames_between_the_scatters_thresholds(gpu_device, form):
-    """3 to 6 Mi pairs: the first frame of a workspace scatters in one level, the second as its pairs and the Gaussians' form say."""
-    scene = crowded_scene(8500, width=400, height=400)
+def test_frames_between_the_scatters_thresholds(gpu_device, monkeypatch, form, P, pairs):
+    """3 to 6, 6 to 12 and more Mi pairs: the first frame of a workspace scatters in one level, the second as its pairs and the
+    Gaussians' form say, and the images are the same."""
+    scene = crowded_scene(P, width=400, height=400)
     scene.opacities[:] = 0.05
     scene.scales[:] = scene.scales.clamp(min=1.5)
     at = lambda x: x.to(gpu_device)
@@ -221,10 +223,21 @@ def test_frames_between_the_scatters_thresholds(gpu_device, form):
         colour["count"] = torch.tensor([scene.P], dtype=torch.int32, device=gpu_device)
     inputs = pipeline.FrameInputs(settings_for(scene, gpu_device), at(scene.means3D), opacities=at(scene.opacities),
                                   scales=at(scene.scales), rotations=at(scene.rotations), **colour)
-    ws = pipeline.Workspace(gpu_device)
+    ws, named = pipeline.Workspace(gpu_device), []
+    render_frame = _lib.load().gs355_render_frame
+
+    def watched(*args):
+        named.append(args[-2] & (_lib.STAGE_TILE_SCATTER_ONE_LEVEL | _lib.STAGE_TILE_SCATTER_TWO_LEVEL))
+        return render_frame(*args)
+
+    monkeypatch.setattr(_lib.load(), "gs355_render_frame", watched)
     first = pipeline.render(inputs, ws=ws)
-    assert 3 << 20 < ws.last_num_pairs < 6 << 20, ws.last_num_pairs
+    assert pairs[0] << 20 <= ws.last_num_pairs < pairs[1] << 20, ws.last_num_pairs
+    assert set(named) == {_lib.STAGE_TILE_SCATTER_ONE_LEVEL}
+    two = pairs[0] >= (12 if form == "count" else 6)
     for _ in range(2):
+        named.clear()
         again = pipeline.render(inputs, ws=ws)
+        assert named == [_lib.STAGE_TILE_SCATTER_TWO_LEVEL if two else _lib.STAGE_TILE_SCATTER_ONE_LEVEL]
         for name in ("image", "depth", "alpha"):
             assert torch.equal(getattr(again, name), getattr(first, name)), name
