@@ -45,13 +45,13 @@ def test_sorted_values_without_their_keys(gpu_device, make, skip):
 
 
 @pytest.mark.parametrize("width,height,P,log_scale", [
-    (16, 16, 70, 0.0), (16 * 63, 16, 3000, -2.0), (16 * 64, 16, 3000, -2.0), (16 * 65, 16, 3000, -2.0), (1000, 700, 9000, -2.5),
+    (16, 16, 70, 0.0), (48, 16, 12_000, 0.5), (16 * 63, 16, 3000, -2.0), (16 * 64, 16, 3000, -2.0), (16 * 65, 16, 3000, -2.0), (1000, 700, 9000, -2.5),
     (16 * 1023, 16, 20_000, -2.5), (4096, 2304, 40_000, -5.0), (16 * 360, 1600, 40_000, -5.0)])
 @pytest.mark.parametrize("levels", [0, _lib.STAGE_TILE_SCATTER_ONE_LEVEL, _lib.STAGE_TILE_SCATTER_TWO_LEVEL])
 def test_layout_made_by_the_scatter(gpu_device, width, height, P, log_scale, levels):
     """Tile count and scatter in one call, where the scatter makes the layout, against one call each: at the edges of the
-    layout's blocks of 64 tiles and of a workgroup's sixteen of them, up to the 36000 tiles of the LDS counters; and for a
-    capacity one key short."""
+    layout's blocks of 64 tiles and of a workgroup's sixteen of them, up to the 36000 tiles of the LDS counters; with buckets
+    beyond 10240 pairs; and for a capacity one key short."""
     scene = scenes.tiny_scene(P=P, width=width, height=height, sh_degree=0, seed=3, log_scale_mean=log_scale)
     inp = pipeline.FrameInputs(settings_for(scene, gpu_device), scene.means3D.to(gpu_device), shs=scene.shs.to(gpu_device),
                                opacities=scene.opacities.to(gpu_device), scales=scene.scales.to(gpu_device),
@@ -70,7 +70,7 @@ def test_layout_made_by_the_scatter(gpu_device, width, height, P, log_scale, lev
             pipeline.run_stages(inp, out, ws, n_cap, mask)
         torch.cuda.synchronize()
         raw = ws.buffer.cpu().numpy()
-        header = raw[lay.header:lay.header + 32].view(np.uint32)
+        header = raw[lay.header:lay.header + 48].view(np.uint32)  # (up to sort_beyond_count)
         lists = raw[lay.tile_lists:lay.tile_lists + 4 * (8 + 4 * tiles)].view(np.uint32)
         got = {"header": header}
         if header[3] == 0:
@@ -79,6 +79,9 @@ def test_layout_made_by_the_scatter(gpu_device, width, height, P, log_scale, lev
             got["keys"] = ws.view(lay, "sorted_keys", P, n, tiles).cpu().numpy()
             got["values"] = ws.view(lay, "sorted_values", P, n, tiles).cpu().numpy()
             got["counts"] = lists[:3]
+            n = got["ranges"].reshape(tiles, 2)
+            beyond = (n[:, 1] - n[:, 0] > 10240).sum() if tiles <= 36000 else 0xFFFFFFFF  # (not counted)
+            assert header[11] == beyond and (P != 12_000 or beyond == 3)
             for c in range(3):
                 got["list %d" % c] = np.sort(lists[8 + c * tiles:][:lists[c]])
         return got
@@ -207,6 +210,25 @@ def test_buckets_beyond_the_lds(gpu_device, P, equal, side):
     assert P < 12_000 or side > 32 or header.sort_beyond_count > 0
     assert (ws.sort_class_idle[2] == 0) == (header.sort_class_count[2] + header.sort_beyond_count > 0)
     assert ws.sort_mispredictions == 0
+
+
+@pytest.mark.parametrize("P", [(1 << 24) - 1, 1 << 24])
+def test_buckets_of_all_that_a_float_counts(gpu_device, P):
+    """One tile of 2^24 pairs, which radix passes through global memory sort, and one of a pair fewer, which is the largest that
+    is split by depth: ordered by depth, and by index where depths are equal."""
+    scene = crowded_scene(P, width=16, height=16)
+    inp = pipeline.FrameInputs(settings_for(scene, gpu_device), *(t.to(gpu_device) for t in (scene.means3D, scene.opacities, scene.shs)),
+                               scales=scene.scales.to(gpu_device), rotations=scene.rotations.to(gpu_device))
+    out, ws = pipeline.FrameOutputs(inp), pipeline.Workspace(gpu_device)
+    for mask in (_lib.STAGE_PREPROCESS, _lib.STAGE_TILE_COUNT | _lib.STAGE_TILE_SCATTER, _lib.STAGE_TILESORT):
+        lay = pipeline.run_stages(inp, out, ws, P, mask)
+    assert ws.view(lay, "ranges", P, P, 1).tolist() == [[0, P]]
+    depth, index = ws.view(lay, "sorted_keys", P, P, 1), ws.view(lay, "sorted_values", P, P, 1).long()
+    assert bool((depth >> 32 == 0).all())
+    own = ws.buffer[lay.depth_bits:lay.depth_bits + 4 * P].view(torch.int32)
+    assert torch.equal(own[index].long(), depth)
+    step = depth.diff()
+    assert bool(((step > 0) | ((step == 0) & (index.diff() > 0))).all())
 
 
 @pytest.mark.parametrize("P,pairs", [(8500, (3, 6)), (13_000, (6, 12)), (24_000, (12, 18))])
