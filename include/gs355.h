@@ -115,15 +115,16 @@ typedef struct gs355_header {
     uint32_t overflow;       /* 1 if num_keys_total > key capacity (the frame must be redone with more) */
     uint32_t num_visible;    /* Gaussians with radius > 0 */
     /* Tile-count stage, images of at most 36000 tiles: buckets in each of the three larger sorter size classes
-     * (1025..2048, 2049..5120, 5121..10240 pairs); 0xFFFFFFFF = not counted (scan stage, larger images).  What a
-     * caller needs to choose GS355_STAGE_TILESORT_SKIP_* for the next frame. */
+     * (1025..2048, 2049..5120, 5121..10240 pairs); 0xFFFFFFFF = not counted (scan stage, larger images).  With
+     * sort_beyond_count, what a caller needs to choose GS355_STAGE_TILESORT_SKIP_* for the next frame. */
     uint32_t sort_class_count[3];
     uint32_t ready;          /* set to 1 in a header copy, after everything else in it (in the workspace: not used) */
     uint32_t parts;          /* preprocess stage: 1 if `rects` holds parts of tile rectangles (GS355_STAGE_TILE_REACH), else 0
                               * (in the workspace only) */
     uint32_t ordered;        /* tile-sort stage: 1 once it has put the tiles in the order the blends take them (in the workspace only) */
     uint32_t sort_beyond_count; /* tile-count stage, as sort_class_count: buckets of more than 10240 pairs.  They are sorted by the
-                              * launch of the largest class, so GS355_STAGE_TILESORT_SKIP_3 suits frames without any of either */
+                              * launch of the largest class: GS355_STAGE_TILESORT_SKIP_3 suits frames where sort_class_count[2] and
+                              * this are both zero */
     uint32_t reserved[4];
 } gs355_header;
 

@@ -738,7 +738,7 @@ __global__ __launch_bounds__(kFineThreads) void fine_count_kernel(const gs355_he
                                                                   uint32_t* __restrict__ list_counts)
 {
     __shared__ uint32_t s_count[kCoarseTiles];
-    if (blockIdx.x == 0 && threadIdx.x < 4) list_counts[threadIdx.x] = 0u;  // filled by tile_publish_kernel
+    if (blockIdx.x == 0 && threadIdx.x < 4) list_counts[threadIdx.x] = 0u;  // filled with the layout
     if (header->overflow) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t num_keys = header->num_keys;
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(64 * kPrefixParts) void slice_prefix_kernel(uint32_
                                                                          uint32_t* __restrict__ list_counts)
 {
     __shared__ uint32_t s_part[kPrefixParts][64];
-    if (blockIdx.x == 0 && threadIdx.x < 4) list_counts[threadIdx.x] = 0u;  // filled by tile_publish_kernel
+    if (blockIdx.x == 0 && threadIdx.x < 4) list_counts[threadIdx.x] = 0u;  // filled with the layout
     const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
     const int t = blockIdx.x * 64 + lane;
     const int per = (groups + kPrefixParts - 1) / kPrefixParts;  // <= kPrefixRows

@@ -435,7 +435,7 @@ constexpr int kEmitCap = 256;  // workgroups: one per CU
 // Up to this many runs per workgroup the emit pass adds up the runs' totals itself: a workgroup's k-th run needs the runs of
 // the stripes before (gridDim.x runs each) and those before it in its own.  62 KB per workgroup at a million anchors, read
 // while the weights are, in the place of a launch of one workgroup of 3 to 5 us: frames of 60k anchors 116 -> 113 us, of a
-// million behind a level-of-detail mask 203 -> 200.6, of 500k 371 -> 369.
+// million behind a level-of-detail mask 203 -> 200.6, of 500k 371 -> 369.  The bases go to the workspace all the same (8 B per run).
 constexpr int kScanStripes = 32;
 constexpr int kRowWords = 72;  // an anchor's words: first opacity, colour, offset scale, position; then covariance
 constexpr int kRowColour = 16, kRowExtra = 48;

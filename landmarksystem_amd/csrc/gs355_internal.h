@@ -17,7 +17,7 @@ constexpr int kSortTile = kSortThreads * kSortItems;
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
 
-// tile-bucketed sort: buckets up to kTileSortCap[3] pairs are sorted in LDS; larger ones go through global memory
+// tile-bucketed sort: buckets up to kTileSortCap[3] pairs are sorted in LDS; larger ones are split into such pieces first
 constexpr int kTileSortCap[4] = {1024, 2048, 5120, 10240};  // in-LDS sorter size classes (pairs per bucket)
 
 // scan geometry: 256 threads x 16 items per workgroup
