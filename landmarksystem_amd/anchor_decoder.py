@@ -35,6 +35,7 @@ module.  The rasterizer behind it differentiates in HIP.
 import ctypes as C
 import functools
 import threading
+import weakref
 from collections import OrderedDict
 from typing import NamedTuple, Optional
 
@@ -360,7 +361,7 @@ class FusedAnchorDecoder(nn.Module):
         # different streams may be in flight together): "workspace" of gs355_decode, "block" of reused outputs
         self._per_stream = OrderedDict()
         self._marshalled = None  # (key, gs355_decoder struct, the tensors it points at)
-        self._feat_checked = None  # (identity of the last feature tensor, whether fp16 holds it exactly)
+        self._feat_checked = None  # (the last feature tensor, its state, whether fp16 holds it exactly)
 
     def __getstate__(self):
         """What a copy or a pickle takes along: not the buffers of past calls and the records of pointers into them."""
@@ -456,11 +457,13 @@ class FusedAnchorDecoder(nn.Module):
         dec = self._decoder_struct(dev)
         # features that fp16 cannot hold exactly (fp32-trained checkpoints) go through the matrix cores as hi + lo
         # pairs; checked once per feature tensor, not per frame
-        feat_key = (id(anchor_feat), anchor_feat._version, anchor_feat.data_ptr(), tuple(anchor_feat.shape))
-        if self._feat_checked is None or self._feat_checked[0] != feat_key:
+        # (a weak reference: another tensor may have the identity and the address of one that is gone)
+        feat_key = (anchor_feat._version, anchor_feat.data_ptr(), tuple(anchor_feat.shape))
+        checked = self._feat_checked
+        if checked is None or checked[0]() is not anchor_feat or checked[1] != feat_key:
             f32 = tensors[1]
-            self._feat_checked = (feat_key, bool(torch.equal(f32.half().float(), f32)))
-        dec.fp32_features = 0 if self._feat_checked[1] else 1
+            checked = self._feat_checked = (weakref.ref(anchor_feat), feat_key, bool(torch.equal(f32.half().float(), f32)))
+        dec.fp32_features = 0 if checked[2] else 1
         kept = self._kept(dev)
         if kept.get("anchors") != A:
             need = C.c_size_t()

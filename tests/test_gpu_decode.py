@@ -435,3 +435,28 @@ def test_emit_again_behind_both_phases(gpu_device, A):
         assert torch.equal(got[name], want[name]), name
     for name in widths:
         assert torch.equal(some[name][:G // 2], want[name][:G // 2]) and bool((some[name][G // 2:] == -7.0).all()), name
+
+
+def test_features_in_the_place_of_others_that_are_gone(gpu_device):
+    """Features that fp16 does not hold, in a tensor that got the address and the identity of one whose features it did: decoded as a
+    decoder decodes them that has seen no others."""
+    sc = scenes.config5(A=1000)
+    dec = build_decoder(sc, gpu_device)
+    t = [x.to(gpu_device).contiguous() for x in (sc.camera.camera_center, sc.anchor, sc.offset, sc.scaling)]
+    exact = sc.anchor_feat.to(gpu_device)
+    general = exact + 1e-4 * torch.randn(exact.shape, generator=torch.Generator().manual_seed(1)).to(gpu_device)
+    call = lambda d, feat: d(t[0], t[1], feat, t[2], t[3])[:5]  # noqa: E731
+    want = call(build_decoder(sc, gpu_device), general)
+    assert not torch.equal(call(dec, exact)[1], want[1])
+    same = 0
+    for _ in range(20):
+        feat = exact.clone()
+        call(dec, feat)
+        was = (id(feat), feat.data_ptr())
+        del feat
+        feat = general.clone()
+        same += was == (id(feat), feat.data_ptr())
+        for a, b in zip(call(dec, feat), want):
+            assert torch.equal(a, b)
+        del feat
+    print("%d of 20 took the place" % same)
